@@ -11,6 +11,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmta_hip.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 
 # dtype codes of include/mta_hip.h
 MTA_F32, MTA_BF16, MTA_F16 = 0, 1, 2
@@ -60,6 +61,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 class MTALibraryError(RuntimeError):
@@ -81,6 +83,20 @@ def load() -> ctypes.CDLL:
         fn.restype, fn.argtypes = res, args
     _lib = lib
     return lib
+
+
+def host():
+    """The native host path of the modules (csrc/host/mta_host.cpp), loaded on first use."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise MTALibraryError(f"{HOST_PATH} is missing or does not load ({e}): build it with "
+                                  "`python -m multitokenatention_triton_amd.build`. There is no fallback path.") from e
+        _host = module
+    return _host
 
 
 def strerror(code: int) -> str:

@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import _lib, ops
 
 
 class TritonAttention(torch.autograd.Function):
@@ -56,4 +56,9 @@ class TritonConvAttention(nn.Module):
             self.weight[:, self.kernel_size[0] // 2, self.kernel_size[1] // 2] = 1.0
 
     def forward(self, Q, K, V, causal, softmax_scale):
-        return TritonAttention.apply(Q, K, V, self.weight, causal, softmax_scale)
+        weight = self.weight
+        if torch.is_grad_enabled() and (Q.requires_grad or K.requires_grad or V.requires_grad or weight.requires_grad):
+            return TritonAttention.apply(Q, K, V, weight, causal, softmax_scale)
+        # (nothing to differentiate: no row statistic is written)
+        assert weight.size(0) == Q.size(1)
+        return _lib.host().conv_attn(Q, K, V, weight, causal, softmax_scale), None

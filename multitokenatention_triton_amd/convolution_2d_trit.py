@@ -12,35 +12,22 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib
 
 
 class Conv2dTritonFunction(torch.autograd.Function):
-    """apply(input (N,C,H,W), weight (C,R,S), causal) -> (N,C,H,W), same dtype as input.
+    """apply(input (N,C,H,W), weight (C,R,S), causal) -> (N,C,H,W), same dtype as input, differentiable: forward and backward
+    (convolution_2d_trit.py:300-378) are one native autograd node (csrc/host/mta_host.cpp).
 
     Two optional flags for callers that know who reads the results (both only matter when ``causal``):
     ``fill_upper=False`` -- the output is only read on and below the diagonal; ``grad_fill_upper=False`` -- so is the
     input gradient that backward returns.  What lies above the diagonal is then left unwritten."""
 
     @staticmethod
-    def forward(ctx, input, weight, causal, fill_upper=True, grad_fill_upper=True):
-        ctx.save_for_backward(input, weight)
-        ctx.causal = causal
-        ctx.grad_fill_upper = grad_fill_upper
-        return ops.conv2d_causal(input, weight, causal, fill_upper=fill_upper)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        """convolution_2d_trit.py:336-378.  The reference returns the weight gradient in fp64 and lets autograd
-        cast it; here it is accumulated in fp32 and cast to the weight's dtype."""
-        input, weight = ctx.saved_tensors
-        grad_input = grad_weight = None
-        if ctx.needs_input_grad[0]:
-            grad_input = ops.conv2d_bwd_input(grad_output, weight, ctx.causal, fill_upper=ctx.grad_fill_upper)
-        if ctx.needs_input_grad[1]:
-            grad_weight = ops.conv2d_bwd_weight(input, grad_output.to(input.dtype), tuple(weight.shape[1:]),
-                                                ctx.causal).to(weight.dtype)
-        return grad_input, grad_weight, None, None, None
+    def apply(input, weight, causal, fill_upper=True, grad_fill_upper=True):
+        # same check and message as convolution_2d_trit.py:306
+        assert input.size(1) == weight.size(0), "This implementation assumes depthwise convolution (C_in == C_out)"
+        return _lib.host().conv2d_apply(input, weight, causal, fill_upper, grad_fill_upper)
 
 
 class Conv2dTriton(nn.Module):

@@ -1,0 +1,465 @@
+// Native host path of the modules: one call per forward, one autograd node per module.
+//
+// At the lengths where a kernel takes a few microseconds the host is what bounds a call: an MTA forward of three kernels
+// spent 84 us in Python (argument checks, a device context, a ctypes call and an allocation per stage) and a training step
+// 530 us (seven autograd nodes with a Python frame each way).  The routes therefore live here, over the operators of
+// ops.hpp; the Python modules keep parameters, masks and the rarely taken routes.
+#include <torch/extension.h>
+
+#include "ops.hpp"
+
+namespace py = pybind11;
+
+namespace mta_host {
+namespace {
+
+// largest mixing group the one-pass mix/softmax/mix kernel keeps in registers, and what its matrix-core variant takes
+constexpr int64_t FUSED_MAX_GROUP = 8, FUSED_MFMA_GROUP = 16, FUSED_MFMA_MAX_KEYS = 4096;
+
+bool no_row_lists()
+{
+    const char *e = getenv("MTA_MIX16_NO_ROW_LISTS");
+    return e && !strcmp(e, "1");
+}
+
+// whether mix -> softmax (-> mix) over mixing groups of `group` heads runs as one kernel
+bool one_pass_group(int64_t group, at::ScalarType t, int64_t n_keys, const OptTensor &w1, const OptTensor &w2)
+{
+    if (group <= FUSED_MAX_GROUP) return true;
+    return group == FUSED_MFMA_GROUP && (t == at::kBFloat16 || t == at::kHalf) && n_keys % 8 == 0 && n_keys <= FUSED_MFMA_MAX_KEYS &&
+           (!w1 || w1->scalar_type() == t) && (!w2 || w2->scalar_type() == t);
+}
+
+// the matrix-core variant for groups of 16 takes a key bias or a band mask in its row-list form only
+bool masks_ok(int64_t group, bool masked) { return !masked || group <= FUSED_MAX_GROUP || (group == FUSED_MFMA_GROUP && !no_row_lists()); }
+
+int64_t lcm(int64_t a, int64_t b)
+{
+    int64_t x = a, y = b;
+    while (y) { const int64_t t = x % y; x = y; y = t; }
+    return a / x * b;
+}
+
+// 1/sqrt(D) as the reference forms it: in fp32
+double score_scale(const Tensor &q) { return (double)(1.0f / std::sqrt((float)q.size(-1))); }
+
+// the optional observer of the modules: called with a stage's name right before it is enqueued
+struct Mark {
+    const py::object &hook;
+    void operator()(const char *stage) const
+    {
+        if (!hook.is_none()) hook(stage);
+    }
+};
+
+// (B,H,S,D) seen as (B,S,H,D), without a view relation that autograd would track
+Tensor heads_last(const Tensor &o)
+{
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return o.transpose(1, 2);
+}
+
+// int32 (B,S): p + 1 for the rows p that see no key, 0 for the others (mta_band_zero_fwd then clears those rows)
+Tensor empty_row_ends(const Tensor &empty_rows)
+{
+    const Tensor rows = at::arange(1, empty_rows.size(-1) + 1, empty_rows.options().dtype(at::kInt));
+    return at::where(empty_rows, rows.unsqueeze(0), at::zeros({}, rows.options())).contiguous();
+}
+
+struct Structure {
+    bool pre_identity, post_conv_identity, post_identity;
+    int64_t pre_group, post_group;   // 0 = dense
+};
+
+// ---- inference -------------------------------------------------------------------------------------------------------
+// The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
+// hides (-inf) are zeroed, so that their scores enter the pre-softmax conv as 0, and their V rows too where a post-softmax
+// conv that is not the identity writes into their columns.  `first`: int32 (B,S), a band mask (row p sees the keys
+// first[p] .. p), applied to the scores inside the first kernel and as -inf inside the softmax kernel, and behind a
+// post-softmax conv that is not the identity the hidden stretch of every row is zeroed again; the caller has checked that
+// the first kernel exists.  `empty_rows`: bool (B,S), the rows of the band that see no key (first[p] = p + 1): the softmax
+// leaves NaN in them, which the reference replaces by zeros ahead of its post-softmax conv
+// (mta_attention_triton.py:81) - here those rows of the probabilities are cleared ahead of a post-softmax conv that is not
+// the identity, and their rows of the output, where nothing else would, at the end.
+Tensor forward_inference(const Tensor &q, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
+                         const Tensor &w_post, bool causal, bool pre_identity, int64_t pre_group, bool post_conv_identity, bool post_identity,
+                         int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows, bool planes,
+                         double dropout, const py::object &hook)
+{
+    at::NoGradGuard no_grad;
+    const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
+    const Mark mark{hook};
+    Tensor k = k_, v = v_;
+    if (key_bias) {
+        const Tensor hidden = key_bias->eq(-INFINITY).unsqueeze(1).unsqueeze(-1);
+        k = k.masked_fill(hidden, 0);
+        if (!post_conv_identity) v = v.masked_fill(hidden, 0);
+    }
+    const double scale = score_scale(q);
+    const int64_t heads = w_pre.size(0), n_keys = k.size(-2);
+    const OptTensor w1 = pre_identity ? OptTensor() : OptTensor(w_pre), w2 = post_identity ? OptTensor() : OptTensor(w_post);
+    const int64_t g_pre = pre_identity ? 1 : pre_group ? pre_group : heads, g_post = post_identity ? 1 : post_group ? post_group : heads;
+    const int64_t g_both = lcm(g_pre, g_post);
+    const bool masked = key_bias || first;
+    const auto dtype = q.scalar_type();
+    const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, masked);
+    // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
+    const bool own_pv = q.size(-2) == n_keys && dtype == v.scalar_type() && causal_pv_supported(dtype, q.size(-2), v.size(-1));
+    const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
+
+    // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
+    // in the triangular layout (what lies on and below the diagonal only, the rows a workgroup of the softmax stage reads
+    // side by side): half the footprint, and every stage streams memory in longer runs.
+    if (!planes && causal && one_pass && own_pv && dropout <= 0 && (g_both == 2 || g_both == 4 || g_both == 8 || g_both == 16) && bias_vectors &&
+        tri_route_supported(q, k, conv_w, g_both, w1, w2, first.has_value(), false, key_bias.has_value())) {
+        mark("qk_conv");
+        Tensor scores = qk_conv_tri(q, k, conv_w, scale, g_both, first);
+        mark("mix_softmax_mix");
+        scores = headmix_softmax_tri(scores, w1, w2, q.size(0), heads, n_keys, g_both, first, false, key_bias);
+        mark("pv");
+        Tensor out = causal_pv_tri(scores, v, g_both, first);
+        if (empty_rows) out.masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
+        mark("end");
+        return out.transpose(1, 2);
+    }
+
+    Tensor scores;
+    // (dense groups of 16 heads ahead of a post-softmax conv: the first score tensor still travels in the triangular layout,
+    // the softmax stage hands the conv (B,H,S,S) planes)
+    const bool tri_first = !planes && causal && !one_pass && g_pre == 16 && masks_ok(16, masked) && w1 &&
+                           !(post_conv_identity && !w2 && !own_pv) &&
+                           tri_route_supported(q, k, conv_w, 16, w1, OptTensor(), first.has_value(), true, key_bias.has_value());
+    if (tri_first) {
+        mark("qk_conv");
+        scores = qk_conv_tri(q, k, conv_w, scale, 16, first);
+    } else if (qk_conv_supported(q, k, conv_w)) {
+        mark("qk_conv");
+        scores = qk_conv(q, k, conv_w, causal, scale, false, first);
+    } else {
+        TORCH_CHECK(!first, "the band mask needs the one-kernel first stage");
+        mark("qk");
+        scores = at::matmul(q, k.transpose(2, 3));
+        mark("conv_pre");
+        scores = conv2d(scores, conv_w, causal, scale, true);
+    }
+
+    if (one_pass) {
+        mark("mix_softmax_mix");
+        scores = headmix_softmax(scores, w1, w2, causal, g_both, !own_pv, key_bias, first);
+    } else {
+        const bool fill = post_conv_identity && !w2 && !own_pv;
+        if (tri_first) {
+            mark("mix_softmax");
+            scores = headmix_softmax_tri(scores, w1, OptTensor(), q.size(0), heads, n_keys, g_pre, first, true, key_bias);
+        } else if (one_pass_group(g_pre, dtype, n_keys, w1, OptTensor()) && masks_ok(g_pre, masked)) {
+            mark("mix_softmax");
+            scores = headmix_softmax(scores, w1, OptTensor(), causal, g_pre, fill, key_bias, first);
+        } else {
+            mark("mix_pre");   // (the softmax kernel that follows never reads above the diagonal)
+            scores = headmix(scores, w_pre, causal, 0.0, g_pre, false);
+            mark("softmax");
+            scores = headmix_softmax(scores, OptTensor(), OptTensor(), causal, 0, fill, key_bias, first);
+        }
+        if (empty_rows && !post_conv_identity) band_zero_(scores, empty_row_ends(*empty_rows));
+        // conv and mix in one pass, the conv result never written: taken where it measures at least as fast as the two
+        // kernels (mixing groups of up to 4 heads and the sizes with a vector-staged instance; dense groups of 16).  Under a
+        // band mask the conv's result is zeroed at the hidden positions ahead of the mixing: two kernels.
+        const int64_t r = post_conv_w.size(1), s = post_conv_w.size(2);
+        const bool mix16 = g_post == 16 && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
+                           post_conv_w.scalar_type() == scores.scalar_type() && w_post.scalar_type() == scores.scalar_type() && n_keys % 8 == 0;
+        const bool small_groups = g_post <= 4 && ((r == 3 && s == 3) || (r == 7 && s == 7));
+        OptTensor done;
+        if (!first && !post_conv_identity && w2 && (small_groups || mix16)) {
+            mark("conv_mix_post");
+            done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
+        }
+        if (done) {
+            scores = *done;
+        } else {
+            // neither our head mixing nor our P V reads above the diagonal: whoever feeds them need not write there
+            if (!post_conv_identity) {
+                mark("conv_post");
+                scores = conv2d(scores, post_conv_w, causal, std::nullopt, !w2 && !own_pv);
+                // (the conv has spread probability into columns the rows do not see: mta_attention_triton.py:82-83)
+                if (first) band_zero_(scores, *first);
+            }
+            if (w2) {
+                mark("mix_post");
+                scores = headmix(scores, w_post, causal, 0.0, g_post, !own_pv);
+            }
+        }
+    }
+    if (dropout > 0) scores = at::dropout(scores, dropout, true);
+    mark("pv");
+    OptTensor out = own_pv ? causal_pv(scores, v, causal, first) : OptTensor();
+    if (!out) out = at::matmul(scores, v);
+    if (empty_rows) out->masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
+    mark("end");
+    return out->transpose(1, 2);
+}
+
+// ---- training ----------------------------------------------------------------------------------------------------------
+// round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it: the scores kernel with factor 1
+// and the pass-through tap as 3x3 kernel, which copies its input exactly.  Nothing where that kernel does not apply.
+// `first`: a band mask, zeros ahead of a row's first visible key (the kernel does not visit the key blocks no row of a query
+// block sees: the hidden stretch of every row is cleared afterwards).
+OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
+{
+    if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !is16(a)) return std::nullopt;
+    Tensor w = at::zeros({a.size(1), 3, 3}, a.options());
+    w.select(1, 2).select(1, 1).fill_(1.0);
+    if (!qk_conv_supported(a, b, w)) return std::nullopt;
+    Tensor out = qk_conv(a, b, w, true, 1.0, false, first);
+    if (first) band_zero_(out, *first);
+    return out;
+}
+
+struct TrainOptions {
+    bool causal, pre_causal, post_causal;
+    double pre_fill, post_fill;
+    int64_t pre_group, post_group;   // 0 = dense (the weight gradient is then dense too)
+    double dropout;
+    OptTensor first;       // int32 (B,S), a band mask
+    OptTensor key_bias;    // fp32 (B,S); the caller has zeroed the K and V rows of the keys it hides
+    OptTensor empty_rows;  // bool (B,S), the rows of the band that see no key: their probabilities are cleared
+};
+
+// The reference's operator sequence (mta_attention_triton.py:68-92) as one differentiable function.  Between two stages
+// nothing reads above the diagonal when causal (the kernels never do, in either direction), so nothing is written there,
+// except what goes into a library GEMM.
+struct MtaTraining : torch::autograd::Function<MtaTraining> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &conv_w,
+                          const Tensor &w_pre, const Tensor &post_conv_w, const Tensor &w_post, const TrainOptions *opt, const Mark *mark_)
+    {
+        const TrainOptions &o = *opt;
+        const Mark &mark = *mark_;
+        const double scale = score_scale(q);
+        const bool fill = !o.causal;
+        Tensor raw, x;   // raw scores (kept where the first stage is two operators), conv result
+        if (qk_conv_supported(q, k, conv_w)) {
+            mark("qk_conv");
+            x = qk_conv(q, k, conv_w, o.causal, scale, false, o.first);
+            // The kernel leaves the key blocks that no row of a query block sees unwritten.  The softmax stage does not read
+            // a row's hidden stretch, but its weight gradient multiplies what is stored there by a gradient that is 0: the
+            // stretch is cleared, so that the product is 0 too.
+            if (o.first) band_zero_(x, *o.first);
+        } else {
+            TORCH_CHECK(!o.first, "the band mask needs the one-kernel first stage");
+            mark("qk");
+            raw = at::matmul(q, k.transpose(2, 3));
+            mark("conv_pre");
+            x = conv2d(raw, conv_w, o.causal, scale, false);
+        }
+        const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
+        Tensor p;
+        if (one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, o.key_bias || o.first)) {
+            mark("mix_softmax");
+            p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
+        } else {
+            mark("mix_pre");
+            const Tensor m = headmix(x, w_pre, o.pre_causal, fill ? o.pre_fill : 0.0, o.pre_group, fill);
+            mark("softmax");
+            p = headmix_softmax(m, OptTensor(), OptTensor(), o.causal, 0, fill, o.key_bias, o.first);
+        }
+        if (o.empty_rows) band_zero_(p, empty_row_ends(*o.empty_rows));
+        mark("conv_post");
+        Tensor c = conv2d(p, post_conv_w, o.causal, std::nullopt, fill);
+        if (o.first) band_zero_(c, *o.first);
+        mark("mix_post");
+        // the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
+        const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && v.size(-2) == n_keys &&
+                              c.size(-2) == c.size(-1) && causal_pv_supported(v.scalar_type(), c.size(-1), v.size(-1));
+        TORCH_CHECK(!o.first || lower_pv, "the band mask needs the lower-triangle products");
+        Tensor m = headmix(c, w_post, o.post_causal, lower_pv ? 0.0 : o.post_fill, o.post_group, !lower_pv), keep;
+        if (o.dropout > 0) std::tie(m, keep) = at::native_dropout(m, o.dropout, true);
+        mark("pv");
+        Tensor out = lower_pv ? *causal_pv(m, v, true, o.first) : at::matmul(m, v);
+        mark("end");
+        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, o.first ? *o.first : Tensor()});
+        ctx->saved_data["causal"] = o.causal;
+        ctx->saved_data["pre_causal"] = o.pre_causal;
+        ctx->saved_data["post_causal"] = o.post_causal;
+        ctx->saved_data["pre_group"] = o.pre_group;
+        ctx->saved_data["post_group"] = o.post_group;
+        ctx->saved_data["dropout"] = o.dropout;
+        ctx->saved_data["lower_pv"] = lower_pv;
+        return heads_last(out);
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &conv_w = saved[3], &w_pre = saved[4], &post_conv_w = saved[5],
+                     &w_post = saved[6], &x = saved[8], &p = saved[9], &c = saved[10], &m = saved[11], &keep = saved[12];
+        Tensor raw = saved[7];
+        const OptTensor first = saved[13].defined() ? OptTensor(saved[13]) : OptTensor();
+        const bool causal = ctx->saved_data["causal"].toBool(), pre_causal = ctx->saved_data["pre_causal"].toBool(),
+                   post_causal = ctx->saved_data["post_causal"].toBool(), lower_pv = ctx->saved_data["lower_pv"].toBool();
+        const int64_t pre_group = ctx->saved_data["pre_group"].toInt(), post_group = ctx->saved_data["post_group"].toInt();
+        const double dropout = ctx->saved_data["dropout"].toDouble(), scale = score_scale(q);
+        const bool fill = !causal;
+        const c10::OptionalDeviceGuard guard(q.device());
+        bool need[7];
+        for (int i = 0; i < 7; ++i) need[i] = ctx->needs_input_grad(i);
+        const bool need_qk = need[0] || need[1], need_x = need_qk || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
+        torch::autograd::variable_list out(9);
+
+        const Tensor go = grads[0].transpose(1, 2).contiguous();
+        if (need[2]) {
+            const OptTensor dv = lower_pv ? causal_ptx(m, go, true) : OptTensor();
+            out[2] = dv ? *dv : at::matmul(m.transpose(2, 3), go);
+        }
+        if (!need_c && !need[6]) return out;
+        const OptTensor lower_dm = lower_pv ? lower_scores(go, v, first) : OptTensor();
+        TORCH_CHECK(lower_dm || !first);
+        Tensor dm = lower_dm ? *lower_dm : at::matmul(go, v.transpose(2, 3));
+        if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
+        dm = dm.to(c.scalar_type());
+        if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
+        if (!need_c) return out;
+        const Tensor dc = headmix_bwd_input(dm, w_post, post_causal, post_group, fill);
+        if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
+        if (!need_p) return out;
+        const Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, fill);
+        // (the head mixing's gradient kernels never read above the diagonal when causal)
+        const Tensor ds = softmax_bwd(p, dp, causal, false);
+        if (need[4]) out[4] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
+        if (!need_x) return out;
+        const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, fill);
+        if (need_qk) {
+            const bool lower = causal && q.sizes() == k.sizes() && causal_pv_supported(q.scalar_type(), k.size(-2), q.size(-1));
+            const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
+            if (first) band_zero_(g, *first);
+            if (need[0]) {
+                const OptTensor dq = lower ? causal_pv(g, k, true, OptTensor()) : OptTensor();
+                out[0] = (dq ? *dq : at::matmul(g, k)).mul(scale);
+            }
+            if (need[1]) {
+                const OptTensor dk = lower ? causal_ptx(g, q, true) : OptTensor();
+                out[1] = (dk ? *dk : at::matmul(g.transpose(2, 3), q)).mul(scale);
+            }
+        }
+        if (need[3]) {
+            if (!raw.defined()) {   // (the kernel gradient reads its first argument on and below the diagonal only)
+                const OptTensor lower_raw = causal ? lower_scores(q, k, first) : OptTensor();
+                TORCH_CHECK(lower_raw || !first);
+                raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
+            }
+            out[3] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale);
+        }
+        return out;
+    }
+};
+
+Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
+                        const Tensor &w_post, bool causal, bool pre_causal, bool post_causal, double pre_fill, double post_fill,
+                        int64_t pre_group, int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows,
+                        double dropout, const py::object &hook)
+{
+    const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
+    TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout, first, key_bias, empty_rows};
+    const Mark mark{hook};
+    Tensor kk = k, vv = v;
+    if (key_bias) {   // (the hidden keys' K and V rows receive no gradient, as in the reference, whose masked_fill / where cut it)
+        const Tensor hidden = key_bias->eq(-INFINITY).unsqueeze(1).unsqueeze(-1);
+        kk = k.masked_fill(hidden, 0);
+        vv = v.masked_fill(hidden, 0);
+    }
+    return MtaTraining::apply(q, kk, vv, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);
+}
+
+// ---- the two operators ---------------------------------------------------------------------------------------------
+struct Conv2d : torch::autograd::Function<Conv2d> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &w, bool causal, bool fill_upper, bool grad_fill_upper)
+    {
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["causal"] = causal;
+        ctx->saved_data["grad_fill_upper"] = grad_fill_upper;
+        return conv2d(x, w, causal, std::nullopt, fill_upper);
+    }
+    // convolution_2d_trit.py:336-378.  The reference returns the weight gradient in fp64 and lets autograd cast it; here it
+    // is accumulated in fp32 and cast to the weight's dtype.
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const c10::OptionalDeviceGuard guard(saved[0].device());
+        const bool causal = ctx->saved_data["causal"].toBool();
+        torch::autograd::variable_list out(5);
+        const Tensor dy = on_gpu(grads[0], "grad_output");
+        if (ctx->needs_input_grad(0)) out[0] = conv2d_bwd_input(dy, saved[1], causal, ctx->saved_data["grad_fill_upper"].toBool());
+        if (ctx->needs_input_grad(1)) out[1] = conv2d_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, 1.0);
+        return out;
+    }
+};
+
+struct HeadMix : torch::autograd::Function<HeadMix> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &w, bool causal, double fill, int64_t group,
+                          bool fill_upper, bool grad_fill_upper)
+    {
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["causal"] = causal;
+        ctx->saved_data["group"] = group;
+        ctx->saved_data["grad_fill_upper"] = grad_fill_upper;
+        return headmix(x, w, causal, fill_upper || !causal ? fill : 0.0, group, fill_upper);
+    }
+    // triton_linear_head.py:322-370.  Above the diagonal the input gradient is 0 (the reference leaves torch.empty_like
+    // memory there); the weight gradient is accumulated in fp32 and cast.
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const c10::OptionalDeviceGuard guard(saved[0].device());
+        const bool causal = ctx->saved_data["causal"].toBool();
+        const int64_t group = ctx->saved_data["group"].toInt();
+        torch::autograd::variable_list out(7);
+        const Tensor dy = on_gpu(grads[0], "grad_output");
+        if (ctx->needs_input_grad(0)) out[0] = headmix_bwd_input(dy, saved[1], causal, group, ctx->saved_data["grad_fill_upper"].toBool());
+        if (ctx->needs_input_grad(1)) out[1] = headmix_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, group);
+        return out;
+    }
+};
+
+bool wants_grad(const Tensor &a, const Tensor &b) { return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad()); }
+
+Tensor conv2d_apply(const Tensor &x, const Tensor &w, bool causal, bool fill_upper, bool grad_fill_upper)
+{
+    const c10::OptionalDeviceGuard guard(x.is_cuda() ? std::optional<c10::Device>(x.device()) : std::nullopt);
+    if (!wants_grad(x, w)) return conv2d(x, w, causal, std::nullopt, fill_upper);
+    return Conv2d::apply(x, w, causal, fill_upper, grad_fill_upper);
+}
+
+Tensor headmix_apply(const Tensor &x, const Tensor &w, bool causal, double fill, int64_t group, bool fill_upper, bool grad_fill_upper)
+{
+    const c10::OptionalDeviceGuard guard(x.is_cuda() ? std::optional<c10::Device>(x.device()) : std::nullopt);
+    if (!wants_grad(x, w)) return headmix(x, w, causal, fill_upper || !causal ? fill : 0.0, group, fill_upper);
+    return HeadMix::apply(x, w, causal, fill, group, fill_upper, grad_fill_upper);
+}
+
+// O = softmax(mask(conv(mask0(Q K^T))) * scale) V, without the row statistic a backward pass would keep
+Tensor conv_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &w_, bool causal, std::optional<double> softmax_scale)
+{
+    const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), v = on_gpu(v_, "V"), w = on_gpu(w_, "W");
+    TORCH_CHECK_VALUE(q.dim() == 4 && q.sizes() == k.sizes() && q.sizes() == v.sizes(), "Q, K, V must share a (B,H,S,D) shape, got ", q.sizes(),
+                      ", ", k.sizes(), ", ", v.sizes());
+    TORCH_CHECK_TYPE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "Q, K, V must share a dtype");
+    TORCH_CHECK(w.dim() == 3 && w.size(0) == q.size(1), "CHANNEL_DIM == NUM_HEADS");
+    const c10::OptionalDeviceGuard guard(q.device());
+    Tensor o = at::empty(q.sizes(), q.options());
+    const double scale = softmax_scale ? *softmax_scale : 1.0 / std::sqrt((double)q.size(3));
+    check(mta_conv_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(w), out_ptr(o), q.size(0), q.size(1), q.size(2), q.size(3), (int)w.size(1), (int)w.size(2),
+                            causal, (float)scale, code(q, "Q"), code(w, "W"), stream_of(q)),
+          "mta_conv_attn_fwd");
+    return o;
+}
+
+}  // namespace
+}  // namespace mta_host
+
+PYBIND11_MODULE(_host, m)
+{
+    using namespace mta_host;
+    m.def("forward_inference", &forward_inference);
+    m.def("forward_training", &forward_training);
+    m.def("conv2d_apply", &conv2d_apply);
+    m.def("headmix_apply", &headmix_apply);
+    m.def("conv_attn", &conv_attn);
+}

@@ -1,0 +1,283 @@
+// Tensor-level operators over the C ABI for the native routes: torch supplies device memory and the stream, the checks are
+// the ones the kernels rely on, every computation is a call into libmta_hip.so.
+#pragma once
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cmath>
+#include <optional>
+
+#include "../../../include/mta_hip.h"
+
+namespace mta_host {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+inline int code(const Tensor &t, const char *what)
+{
+    switch (t.scalar_type()) {
+    case at::kFloat: return MTA_F32;
+    case at::kBFloat16: return MTA_BF16;
+    case at::kHalf: return MTA_F16;
+    default: C10_THROW_ERROR(TypeError, c10::str(what, ": dtype ", t.scalar_type(), " is not supported (float32, bfloat16, float16)"));
+    }
+}
+
+inline bool is16(const Tensor &t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
+
+inline Tensor on_gpu(const Tensor &t, const char *what)
+{
+    TORCH_CHECK(t.is_cuda(), what, " lives on ", t.device(), ": the MTA kernels only run on an AMD GPU (there is no CPU path)");
+    return t.is_contiguous() ? t : t.contiguous();
+}
+
+inline void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// 0 = ok; negative = argument rejected (ValueError); positive = HIP error (RuntimeError)
+inline void check(int rc, const char *what)
+{
+    if (rc == 0) return;
+    TORCH_CHECK_VALUE(rc > 0, what, ": ", mta_strerror(rc), " (code ", rc, ")");
+    TORCH_CHECK(false, what, ": ", mta_strerror(rc), " (code ", rc, ")");
+}
+
+inline const void *ptr(const Tensor &t) { return t.const_data_ptr(); }
+inline const void *ptr(const OptTensor &t) { return t ? t->const_data_ptr() : nullptr; }
+inline void *out_ptr(const Tensor &t) { return t.mutable_data_ptr(); }
+
+// the `causal` argument of the conv / head-mixing entry points
+inline int causal_mode(bool causal, bool fill_upper) { return !causal ? 0 : fill_upper ? 1 : MTA_CAUSAL_LOWER_ONLY; }
+
+inline int64_t tri_row_offset(int64_t p)
+{
+    const int64_t a = p >> 6;
+    return 2048 * a * (a + 1) + (p & 63) * 64 * (a + 1);
+}
+
+inline Tensor conv2d(const Tensor &x_, const Tensor &w_, bool causal, std::optional<double> in_scale, bool fill_upper)
+{
+    const Tensor x = on_gpu(x_, "input"), w = on_gpu(w_, "weight");
+    TORCH_CHECK_VALUE(x.dim() == 4 && w.dim() == 3, "expected input (N,C,H,W) and weight (C,R,S), got ", x.sizes(), " and ", w.sizes());
+    TORCH_CHECK(x.size(1) == w.size(0), "This implementation assumes depthwise convolution (C_in == C_out)");
+    Tensor y = at::empty(x.sizes(), x.options());
+    const int64_t n = x.size(0), c = x.size(1), h = x.size(2), wd = x.size(3);
+    const int r = (int)w.size(1), s = (int)w.size(2), ic = code(x, "input"), wc = code(w, "weight");
+    int rc;
+    if (in_scale)
+        rc = mta_conv2d_scaled_fwd(ptr(x), ptr(w), out_ptr(y), n, c, h, wd, r, s, causal_mode(causal, fill_upper), (float)*in_scale, ic, wc, stream_of(x));
+    else
+        rc = mta_conv2d_fwd(ptr(x), ptr(w), out_ptr(y), n, c, h, wd, r, s, causal_mode(causal, fill_upper), ic, wc, stream_of(x));
+    check(rc, "mta_conv2d_fwd");
+    return y;
+}
+
+inline Tensor conv2d_bwd_input(const Tensor &dy_, const Tensor &w_, bool causal, bool fill_upper)
+{
+    const Tensor dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    Tensor dx = at::empty(dy.sizes(), dy.options());
+    check(mta_conv2d_bwd_input(ptr(dy), ptr(w), out_ptr(dx), dy.size(0), dy.size(1), dy.size(2), dy.size(3), (int)w.size(1), (int)w.size(2),
+                               causal_mode(causal, fill_upper), code(dy, "grad_output"), code(w, "weight"), stream_of(dy)),
+          "mta_conv2d_bwd_input");
+    return dx;
+}
+
+// the gradient of a (C,R,S) kernel, times `scale`, in the dtype of `like`
+inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tensor &like, bool causal, double scale)
+{
+    const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output");
+    TORCH_CHECK_VALUE(x.sizes() == dy.sizes() && x.scalar_type() == dy.scalar_type(), "input and grad_output must share shape and dtype");
+    const int64_t n = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3);
+    const int r = (int)like.size(1), s = (int)like.size(2);
+    Tensor dw = at::empty({c, r, s}, x.options().dtype(at::kFloat));
+    const int64_t bytes = std::max<int64_t>(mta_conv2d_bwd_weight_workspace(n, c, h, w, r, s), 16);
+    Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+    check(mta_conv2d_bwd_weight(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, h, w, r, s, causal, code(x, "input"), stream_of(x)),
+          "mta_conv2d_bwd_weight");
+    if (scale != 1.0) dw.mul_(scale);
+    return dw.to(like.scalar_type());
+}
+
+inline Tensor headmix(const Tensor &x_, const Tensor &w_, bool causal, double fill, int64_t group, bool fill_upper)
+{
+    const Tensor x = on_gpu(x_, "input"), w = on_gpu(w_, "weight");
+    TORCH_CHECK_VALUE(x.dim() == 4, "expected input (N,C,P,Q), got ", x.sizes());
+    TORCH_CHECK(w.dim() == 2 && w.size(0) == w.size(1), "Weight must be square matrix, got ", w.sizes());
+    TORCH_CHECK(x.size(1) == w.size(0), "Channel dimension ", x.size(1), " must match weight dimension ", w.size(0));
+    Tensor y = at::empty(x.sizes(), x.options());
+    check(mta_headmix_fwd(ptr(x), ptr(w), out_ptr(y), x.size(0), x.size(1), x.size(2), x.size(3), (int)group, causal_mode(causal, fill_upper),
+                          (float)fill, code(x, "input"), code(w, "weight"), stream_of(x)),
+          "mta_headmix_fwd");
+    return y;
+}
+
+inline Tensor headmix_bwd_input(const Tensor &dy_, const Tensor &w_, bool causal, int64_t group, bool fill_upper)
+{
+    const Tensor dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    Tensor dx = at::empty(dy.sizes(), dy.options());
+    check(mta_headmix_bwd_input(ptr(dy), ptr(w), out_ptr(dx), dy.size(0), dy.size(1), dy.size(2), dy.size(3), (int)group,
+                                causal_mode(causal, fill_upper), code(dy, "grad_output"), code(w, "weight"), stream_of(dy)),
+          "mta_headmix_bwd_input");
+    return dx;
+}
+
+// the gradient of a (C,C) head weight in the dtype of `like`; group > 0: confined to the diagonal blocks
+inline Tensor headmix_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tensor &like, bool causal, int64_t group)
+{
+    const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output");
+    TORCH_CHECK_VALUE(x.sizes() == dy.sizes() && x.scalar_type() == dy.scalar_type(), "input and grad_output must share shape and dtype");
+    const int64_t n = x.size(0), c = x.size(1), p = x.size(2), q = x.size(3);
+    const int64_t bytes = mta_headmix_bwd_weight_workspace(n, c, p, q);
+    TORCH_CHECK_VALUE(bytes > 0, "mta_headmix_bwd_weight: no kernel for ", c, " heads (at most 128)");
+    Tensor dw = at::empty({c, c}, x.options().dtype(at::kFloat)), ws = at::empty({std::max<int64_t>(bytes, 16)}, x.options().dtype(at::kByte));
+    check(mta_headmix_bwd_weight(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, causal, code(x, "input"), stream_of(x)),
+          "mta_headmix_bwd_weight");
+    if (group > 0) {
+        const Tensor blk = at::arange(c, x.options().dtype(at::kLong)).floor_divide(group);
+        dw.mul_(blk.unsqueeze(1).eq(blk.unsqueeze(0)));
+    }
+    return dw.to(like.scalar_type());
+}
+
+inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTensor &w2, bool causal, int64_t group, bool fill_upper,
+                              const OptTensor &key_bias, const OptTensor &first)
+{
+    const Tensor x = on_gpu(x_, "input");
+    TORCH_CHECK_VALUE(x.dim() == 4, "expected input (N,C,P,Q), got ", x.sizes());
+    OptTensor a, b;
+    if (w1) a = on_gpu(*w1, "weight");
+    if (w2) b = on_gpu(*w2, "weight");
+    TORCH_CHECK_TYPE(!a || !b || a->scalar_type() == b->scalar_type(), "w1 and w2 must share a dtype");
+    const int wc = a ? code(*a, "weight") : b ? code(*b, "weight") : MTA_F32;
+    Tensor y = at::empty(x.sizes(), x.options());
+    check(mta_headmix_softmax_band_fwd(ptr(x), ptr(a), ptr(b), ptr(key_bias), ptr(first), out_ptr(y), x.size(0), x.size(1), x.size(2), x.size(3),
+                                       (int)group, causal, fill_upper, code(x, "input"), wc, stream_of(x)),
+          "mta_headmix_softmax_band_fwd");
+    return y;
+}
+
+inline Tensor softmax_bwd(const Tensor &p_, const Tensor &dp_, bool causal, bool fill_upper)
+{
+    const Tensor p = on_gpu(p_, "probabilities"), dp = on_gpu(dp_, "grad_output");
+    Tensor dx = at::empty(p.sizes(), p.options());
+    check(mta_softmax_bwd(ptr(p), ptr(dp), out_ptr(dx), p.size(0), p.size(1), p.size(2), p.size(3), causal, fill_upper, code(p, "probabilities"),
+                          stream_of(p)),
+          "mta_softmax_bwd");
+    return dx;
+}
+
+// nothing (nullopt) when the library has no kernel for the combination
+inline OptTensor conv2d_headmix(const Tensor &x_, const Tensor &wc_, const Tensor &wm_, bool causal, int64_t group, bool fill_upper)
+{
+    const Tensor x = on_gpu(x_, "input"), wc = on_gpu(wc_, "conv weight"), wm = on_gpu(wm_, "mix weight");
+    Tensor y = at::empty(x.sizes(), x.options());
+    const int rc = mta_conv2d_headmix_fwd(ptr(x), ptr(wc), ptr(wm), out_ptr(y), x.size(0), x.size(1), x.size(2), x.size(3), (int)wc.size(1),
+                                          (int)wc.size(2), (int)group, causal, fill_upper, code(x, "input"), code(wc, "weight"),
+                                          code(wm, "weight"), stream_of(x));
+    if (rc == MTA_ERR_UNSUPPORTED) return std::nullopt;
+    check(rc, "mta_conv2d_headmix_fwd");
+    return y;
+}
+
+inline bool qk_conv_supported(const Tensor &q, const Tensor &k, const Tensor &w)
+{
+    if (q.dim() != 4 || q.sizes() != k.sizes() || q.scalar_type() != k.scalar_type() || w.dim() != 3 || !is16(q) ||
+        w.scalar_type() != q.scalar_type())
+        return false;
+    return mta_qk_conv_supported(q.size(2), q.size(3), (int)w.size(1), (int)w.size(2), code(q, "Q"), code(w, "W")) != 0;
+}
+
+inline bool causal_pv_supported(at::ScalarType t, int64_t s, int64_t d)
+{
+    return (t == at::kBFloat16 || t == at::kHalf) && (d == 64 || d == 128) && s % 8 == 0;
+}
+
+// scale * conv(mask0(Q K^T)) as a (B,H,S,S) tensor; the caller has asked qk_conv_supported
+inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool causal, double scale, bool fill_upper, const OptTensor &first)
+{
+    const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
+    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    Tensor y = at::empty({b, h, s, s}, q.options());
+    const int r = (int)w.size(1), sk = (int)w.size(2), ic = code(q, "Q"), wc = code(w, "W");
+    const int rc = first ? mta_qk_conv_band_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, r, sk, (float)scale, fill_upper, ic, wc, stream_of(q))
+                         : mta_qk_conv_fwd(ptr(q), ptr(k), ptr(w), out_ptr(y), b, h, s, d, r, sk, causal, (float)scale, fill_upper, ic, wc, stream_of(q));
+    check(rc, "mta_qk_conv_fwd");
+    return y;
+}
+
+inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first)
+{
+    const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
+    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), v.size(2), v.size(3))) return std::nullopt;
+    Tensor o = at::empty(v.sizes(), v.options());
+    check(mta_causal_pv_band_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), causal, code(p, "P"), stream_of(p)),
+          "mta_causal_pv_fwd");
+    return o;
+}
+
+inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal)
+{
+    const Tensor p = on_gpu(p_, "P"), x = on_gpu(x_, "X");
+    if (p.scalar_type() != x.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), x.size(2), x.size(3))) return std::nullopt;
+    Tensor o = at::empty(x.sizes(), x.options());
+    check(mta_causal_ptx_fwd(ptr(p), ptr(x), out_ptr(o), x.size(0), x.size(1), x.size(2), x.size(3), causal, code(p, "P"), stream_of(p)),
+          "mta_causal_ptx_fwd");
+    return o;
+}
+
+inline void band_zero_(const Tensor &x, const Tensor &first)
+{
+    check(mta_band_zero_fwd(out_ptr(x), ptr(first), x.size(0), x.size(1), x.size(2), code(x, "input"), stream_of(x)), "mta_band_zero_fwd");
+}
+
+// whether the triangular-layout kernels exist (host-side questions to the library)
+inline bool tri_route_supported(const Tensor &q, const Tensor &k, const Tensor &conv_w, int64_t group, const OptTensor &w1, const OptTensor &w2,
+                                bool band, bool out_planes, bool key_bias)
+{
+    if (!qk_conv_supported(q, k, conv_w) || (!w1 && !w2)) return false;
+    for (const OptTensor *w : {&w1, &w2})
+        if (*w && ((*w)->scalar_type() != q.scalar_type() || reinterpret_cast<uintptr_t>(ptr(*w)) % 4)) return false;
+    const int64_t h = q.size(1), s = q.size(2);
+    if (h % group || group * tri_row_offset(s) >= (int64_t(1) << 31) || !causal_pv_supported(q.scalar_type(), s, q.size(3))) return false;
+    const int c = code(q, "Q");
+    return mta_headmix_softmax_tri_supported(h, s, (int)group, out_planes, c, c, w1.has_value(), w2.has_value(), band, key_bias) != 0;
+}
+
+inline Tensor qk_conv_tri(const Tensor &q_, const Tensor &k_, const Tensor &w_, double scale, int64_t group, const OptTensor &first)
+{
+    const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
+    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    Tensor y = at::empty({b * h * tri_row_offset(s)}, q.options());
+    check(mta_qk_conv_tri_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, (int)w.size(1), (int)w.size(2), (float)scale, (int)group,
+                              code(q, "Q"), code(w, "W"), stream_of(q)),
+          "mta_qk_conv_tri_fwd");
+    return y;
+}
+
+inline Tensor headmix_softmax_tri(const Tensor &x, const OptTensor &w1, const OptTensor &w2, int64_t n, int64_t c, int64_t s, int64_t group,
+                                  const OptTensor &first, bool out_planes, const OptTensor &key_bias)
+{
+    OptTensor a, b;
+    if (w1) a = on_gpu(*w1, "weight");
+    if (w2) b = on_gpu(*w2, "weight");
+    Tensor y = out_planes ? at::empty({n, c, s, s}, x.options()) : at::empty(x.sizes(), x.options());
+    const int ic = code(x, "input");
+    check(mta_headmix_softmax_tri_fwd(ptr(x), ptr(a), ptr(b), ptr(key_bias), ptr(first), out_ptr(y), n, c, s, (int)group, out_planes, ic, ic,
+                                      stream_of(x)),
+          "mta_headmix_softmax_tri_fwd");
+    return y;
+}
+
+inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, const OptTensor &first)
+{
+    const Tensor v = on_gpu(v_, "V");
+    Tensor o = at::empty(v.sizes(), v.options());
+    check(mta_causal_pv_tri_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), (int)group, code(p, "P"),
+                                stream_of(p)),
+          "mta_causal_pv_tri_fwd");
+    return o;
+}
+
+}  // namespace mta_host

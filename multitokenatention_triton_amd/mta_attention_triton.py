@@ -73,30 +73,9 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 from .convolution_2d_trit import Conv2dTriton, Conv2dTritonFunction
 from .triton_linear_head import TritonLinearHead, TritonLinearHeadFunction
-
-# largest mixing group the one-pass mix/softmax/mix kernel keeps in registers ...
-_FUSED_MAX_GROUP = 8
-# ... and the group size its matrix-core variant takes (16-bit data, rows of up to _FUSED_MFMA_MAX_KEYS keys)
-_FUSED_MFMA_GROUP = 16
-_FUSED_MFMA_MAX_KEYS = 4096
-
-
-def _one_pass_group(group: int, scores_dtype, n_keys: int, *weights) -> bool:
-    """Whether mix -> softmax (-> mix) over mixing groups of ``group`` heads runs as one kernel."""
-    if group <= _FUSED_MAX_GROUP:
-        return True
-    return (group == _FUSED_MFMA_GROUP and scores_dtype in (torch.bfloat16, torch.float16)
-            and n_keys % 8 == 0 and n_keys <= _FUSED_MFMA_MAX_KEYS
-            and all(w is None or w.dtype == scores_dtype for w in weights))
-# where the one-pass post-softmax conv + head mixing kernel is used (see forward)
-_CONV_MIX_MAX_GROUP = 4
-_CONV_MIX_SIZES = ((3, 3), (7, 7))
-# ... and for dense groups of 16 heads at 16-bit dtypes (conv and mixing both on the matrix cores)
-_CONV_MIX16_SIZES = ((3, 3), (5, 5), (7, 7))
-
 
 _IDENTITY_KERNELS = {}
 
@@ -124,37 +103,32 @@ def _lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torc
 
 
 class _ProbsTimesValues(torch.autograd.Function):
-    """P V of the training route (mta_attention_triton.py:89).  When ``lower`` (causal: the producer of P wrote nothing
-    above the diagonal, and the head mixing's gradient kernels, which take dP from here, read nothing there) all three
-    products touch the lower triangle of their (B,H,S,S) operand only: forward ``mta_causal_pv_fwd``, dV = P^T dO
+    """P V of the mask-pass training route (mta_attention_triton.py:89).  When ``lower`` (causal: the producer of P wrote
+    nothing above the diagonal, and the head mixing's gradient kernels, which take dP from here, read nothing there) all
+    three products touch the lower triangle of their (B,H,S,S) operand only: forward ``mta_causal_pv_fwd``, dV = P^T dO
     ``mta_causal_ptx_fwd``, dP = dO V^T ``_lower_scores``.  Where those kernels do not apply (fp32, ragged lengths, other
     head sizes) the caller has filled P and the library GEMMs run."""
 
     @staticmethod
-    def forward(ctx, p, v, lower, first_visible=None):
-        # (first_visible: a band mask, P is 0 ahead of every row's first visible key; needs ``lower``.  The gradient with
-        # respect to P is then formed inside the band only: 0 at the hidden positions, where the reference's
-        # ``torch.where(mask == -inf, 0.0, scores)`` cuts it)
-        assert first_visible is None or lower
-        ctx.save_for_backward(p, v, first_visible)
+    def forward(ctx, p, v, lower):
+        ctx.save_for_backward(p, v)
         ctx.lower = lower
-        out = ops.causal_pv(p, v, True, first_visible=first_visible) if lower else None
+        out = ops.causal_pv(p, v, True) if lower else None
         return out if out is not None else torch.matmul(p, v)
 
     @staticmethod
     def backward(ctx, grad_output):
-        p, v, first_visible = ctx.saved_tensors
+        p, v = ctx.saved_tensors
         dp = dv = None
         if ctx.needs_input_grad[0]:
-            dp = _lower_scores(grad_output, v, first_visible) if ctx.lower else None
+            dp = _lower_scores(grad_output, v) if ctx.lower else None
             if dp is None:
-                assert first_visible is None
                 dp = torch.matmul(grad_output, v.transpose(2, 3))
         if ctx.needs_input_grad[1]:
             dv = ops.causal_ptx(p, grad_output.contiguous(), True) if ctx.lower else None
             if dv is None:
                 dv = torch.matmul(p.transpose(2, 3), grad_output)
-        return dp, dv, None, None
+        return dp, dv, None
 
 
 def _lower_products_supported(x: torch.Tensor, s_keys: int) -> bool:
@@ -163,52 +137,25 @@ def _lower_products_supported(x: torch.Tensor, s_keys: int) -> bool:
 
 
 class _ScaledScoresConv(torch.autograd.Function):
-    """conv(round(Q K^T) * scale) for the training route (mta_attention_triton.py:69-73).  Forward: the inference
-    route's one kernel (``mta_qk_conv_fwd``, the raw scores never reach memory) where it exists; otherwise the library
-    GEMM, then ``mta_conv2d_scaled_fwd``, which applies the factor (and the rounding to the score dtype that the
-    reference's separate multiplication performs) on the way into the conv.  Backward: the conv's input gradient ``g``
-    goes through the two products dQ = G K and dK = G^T Q and the factor is applied to their (B,H,S,D) results - under
-    the causal rule with ``mta_causal_pv_fwd`` and ``mta_causal_ptx_fwd``, which read the lower triangle of ``g`` only (it
-    is then not written above the diagonal either), else with the library GEMMs; the kernel gradient is taken against
-    the raw scores -- kept by the second forward, recomputed with one product after the first, which so saves a
-    (B,H,S,S) activation -- and scaled afterwards.  Neither direction spends a pass over a (B,H,S,S) tensor on the
-    factor."""
+    """conv(mask0(round(Q K^T)) * scale) for training under a mask of arbitrary content
+    (mta_attention_triton.py:69-73): the raw scores are written, the hidden ones zeroed in place (``mask_planes``, uint8
+    (1|B, 1|H, S, S)) and kept for the kernel gradient; ``mta_conv2d_scaled_fwd`` applies the factor (and the rounding to
+    the score dtype that the reference's separate multiplication performs) on the way into the conv.  Backward: the conv's
+    input gradient ``g``, zeroed at the same positions, goes through the two products dQ = G K and dK = G^T Q and the factor
+    is applied to their (B,H,S,D) results - under the causal rule with ``mta_causal_pv_fwd`` and ``mta_causal_ptx_fwd``,
+    which read the lower triangle of ``g`` only (it is then not written above the diagonal either), else with the library
+    GEMMs; the kernel gradient is taken against the raw scores and scaled afterwards."""
 
     @staticmethod
-    def forward(ctx, xq, xk, weight, scale, causal, mark, first_visible=None, mask_planes=None):
-        # (first_visible: a band mask, applied to the scores ahead of the conv (mta_attention_triton.py:72-73) inside the
-        # one kernel, which the caller has checked exists; backward: the conv's input gradient is zeroed at the hidden
-        # positions, the raw scores for the kernel gradient are recomputed inside the band)
-        # (mask_planes: uint8 (1|B, 1|H, S, S), a mask of arbitrary content: the raw scores are written, the hidden ones
-        # zeroed in place, and kept for the kernel gradient; backward zeroes the conv's input gradient at the same positions)
-        ctx.scale, ctx.causal, ctx.first_visible, ctx.mask_planes = scale, causal, first_visible, mask_planes
-        if mask_planes is not None:
-            assert first_visible is None
-            mark("qk")
-            raw = _lower_scores(xq, xk) if causal else None
-            if raw is None:
-                raw = torch.matmul(xq, xk.transpose(2, 3))
-            mark("mask")
-            if ops.mask_fill(raw, mask_planes, False, causal, out=raw) is None:
-                raise RuntimeError("mask planes need a number of keys that is a multiple of 8")
-            mark("conv_pre")
-            ctx.save_for_backward(xq, xk, weight, raw)
-            return ops.conv2d_causal(raw, weight, causal, in_scale=scale, fill_upper=False)
-        # (the stage that follows, head mixing or mixing + softmax, never reads above the diagonal)
-        if ops.qk_conv_supported(xq, xk, weight):
-            mark("qk_conv")
-            out = ops.qk_conv(xq, xk, weight, causal, scale, fill_upper=False, first_visible=first_visible)
-            if out is not None and first_visible is not None:
-                # The kernel leaves the key blocks that no row of a query block sees unwritten.  The softmax stage does not
-                # read a row's hidden stretch, but its weight gradient multiplies what is stored there by a gradient that
-                # is 0: the stretch is cleared, so that the product is 0 too.
-                out = ops.band_zero_(out, first_visible)
-            if out is not None:
-                ctx.save_for_backward(xq, xk, weight, None)
-                return out
-        assert first_visible is None, "the band mask needs the one-kernel first stage"
+    def forward(ctx, xq, xk, weight, scale, causal, mark, mask_planes):
+        ctx.scale, ctx.causal, ctx.mask_planes = scale, causal, mask_planes
         mark("qk")
-        raw = torch.matmul(xq, xk.transpose(2, 3))
+        raw = _lower_scores(xq, xk) if causal else None
+        if raw is None:
+            raw = torch.matmul(xq, xk.transpose(2, 3))
+        mark("mask")
+        if ops.mask_fill(raw, mask_planes, False, causal, out=raw) is None:
+            raise RuntimeError("mask planes need a number of keys that is a multiple of 8")
         mark("conv_pre")
         ctx.save_for_backward(xq, xk, weight, raw)
         return ops.conv2d_causal(raw, weight, causal, in_scale=scale, fill_upper=False)
@@ -220,33 +167,15 @@ class _ScaledScoresConv(torch.autograd.Function):
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
             lower = ctx.causal and xq.shape == xk.shape and _lower_products_supported(xq, xk.size(-2))
             g = ops.conv2d_bwd_input(grad_output, weight, ctx.causal, fill_upper=not lower)
-            if ctx.first_visible is not None:
-                assert lower
-                if ops.band_zero_(g, ctx.first_visible) is None:
-                    raise RuntimeError("band masks need 16-bit scores of a length that is a multiple of 8")
-            if ctx.mask_planes is not None:
-                ops.mask_fill(g, ctx.mask_planes, False, lower, out=g)
+            ops.mask_fill(g, ctx.mask_planes, False, lower, out=g)
             if ctx.needs_input_grad[0]:
-                dq = ops.causal_pv(g, xk, True) if lower else None
-                if dq is None:
-                    assert not lower
-                    dq = torch.matmul(g, xk)
-                dq = dq * ctx.scale
+                dq = (ops.causal_pv(g, xk, True) if lower else torch.matmul(g, xk)) * ctx.scale
             if ctx.needs_input_grad[1]:
-                dk = ops.causal_ptx(g, xq, True) if lower else None
-                if dk is None:
-                    assert not lower
-                    dk = torch.matmul(g.transpose(2, 3), xq)
-                dk = dk * ctx.scale
+                dk = (ops.causal_ptx(g, xq, True) if lower else torch.matmul(g.transpose(2, 3), xq)) * ctx.scale
         if ctx.needs_input_grad[2]:
-            if raw is None:  # (the kernel gradient reads its first argument on and below the diagonal only)
-                raw = _lower_scores(xq, xk, ctx.first_visible) if ctx.causal else None
-                if raw is None:
-                    assert ctx.first_visible is None
-                    raw = torch.matmul(xq, xk.transpose(2, 3))
             dw = ops.conv2d_bwd_weight(raw, grad_output.to(raw.dtype), tuple(weight.shape[1:]), ctx.causal)
             dw = (dw * ctx.scale).to(weight.dtype)
-        return dq, dk, dw, None, None, None, None, None
+        return dq, dk, dw, None, None, None, None
 
 
 class _MaskFill(torch.autograd.Function):
@@ -290,70 +219,36 @@ class _MaskAdd(torch.autograd.Function):
         return grad_output, None, None
 
 
-class _BandZero(torch.autograd.Function):
-    """x[b,h,p,q] = 0 for q < first_visible[b,p], in place: what ``torch.where(mask == -inf, 0.0, scores)`` behind the
-    post-softmax conv does under a band mask (mta_attention_triton.py:82-83).  Its gradient would be the same zeroing;
-    here the gradient that arrives is zero at those positions already - the gradient with respect to the probabilities
-    is formed inside the band only (``_ProbsTimesValues``) and what lies between, dropout and head mixing, acts per
-    position - so it is handed on as it is."""
+class _Softmax(torch.autograd.Function):
+    """Row softmax over the keys for the mask-pass training route (mta_attention_triton.py:79), one kernel: computed in fp32
+    and stored in the score dtype, as ``F.softmax(scores.float()).type_as(scores)`` leaves it.  ``zero_planes``: uint8
+    visibility planes of a mask under which some row sees nothing - that row's NaN becomes zeros, as behind the reference's
+    masked_fill ahead of its post-softmax conv, and the stored probabilities give it a zero gradient.  Backward: from the
+    stored probabilities (``mta_softmax_bwd``)."""
 
     @staticmethod
-    def forward(ctx, x, first_visible):
-        if ops.band_zero_(x, first_visible) is None:
-            raise RuntimeError("band masks need 16-bit scores of a length that is a multiple of 8")
-        ctx.mark_dirty(x)
-        return x
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        return grad_output, None
-
-
-class _MixSoftmax(torch.autograd.Function):
-    """softmax(mix(x, weight)) over the keys for the training route (mta_attention_triton.py:75-79), one kernel
-    (``mta_headmix_softmax_fwd``; ``weight=None``: the softmax alone).  The probabilities are computed in fp32 from the
-    mixed scores rounded to the score dtype and stored in it, as ``F.softmax(scores.float()).type_as(scores)`` leaves
-    them.  Backward: the softmax gradient from the stored probabilities (``mta_softmax_bwd``), then the head mixing's
-    two gradient kernels."""
-
-    @staticmethod
-    def forward(ctx, x, weight, causal, group_size, fill_upper=True, grad_fill_upper=True, key_bias=None,
-                first_visible=None, zero_planes=None):
-        # (key_bias: fp32 (B,Sk) added to the mixed scores, 0 or -inf per key; first_visible: int32 (B,S), a band mask.
-        # Constants: the gradient is the softmax's own, taken from the stored probabilities, which are 0 at what is hidden)
-        p = ops.headmix_softmax(x, weight, None, causal, group_size=group_size if weight is not None else None,
-                                fill_upper=fill_upper, key_bias=key_bias, first_visible=first_visible)
+    def forward(ctx, x, causal, fill_upper, zero_planes):
+        p = ops.headmix_softmax(x, None, None, causal, fill_upper=fill_upper)
         if zero_planes is not None:
-            # (a mask under which some row sees nothing: that row's NaN becomes zeros, as behind the reference's masked_fill
-            # ahead of its post-softmax conv - and the stored probabilities give it a zero gradient.  Either the mask's uint8
-            # visibility planes, or for a band mask an int32 (B,S) array that is p + 1 for such a row p and 0 elsewhere)
-            if zero_planes.dtype == torch.int32:
-                if ops.band_zero_(p, zero_planes) is None:
-                    raise RuntimeError("band masks need 16-bit scores of a length that is a multiple of 8")
-            else:
-                ops.mask_fill(p, zero_planes, False, causal, out=p)
-        ctx.save_for_backward(x if weight is not None else None, weight, p)
-        ctx.causal, ctx.group_size, ctx.grad_fill_upper = causal, group_size, grad_fill_upper
+            ops.mask_fill(p, zero_planes, False, causal, out=p)
+        ctx.save_for_backward(p)
+        ctx.causal, ctx.fill_upper = causal, fill_upper
         return p
 
     @staticmethod
     def backward(ctx, grad_output):
-        x, weight, p = ctx.saved_tensors
-        # the head mixing's gradient kernels never read above the diagonal; whoever takes the gradient we return might
-        ds = ops.softmax_bwd(p, grad_output.to(p.dtype), ctx.causal,
-                             fill_upper=weight is None and ctx.grad_fill_upper)
-        if weight is None:
-            return ds, None, None, None, None, None, None, None, None
-        dx = dw = None
-        if ctx.needs_input_grad[0]:
-            dx = ops.headmix_bwd_input(ds, weight, ctx.causal, ctx.group_size, fill_upper=ctx.grad_fill_upper)
-        if ctx.needs_input_grad[1]:
-            dw = ops.headmix_bwd_weight(x, ds, ctx.causal)
-            if ctx.group_size:
-                blk = torch.arange(weight.shape[0], device=weight.device) // ctx.group_size
-                dw = dw * (blk[:, None] == blk[None, :])
-            dw = dw.to(weight.dtype)
-        return dx, dw, None, None, None, None, None, None, None
+        p, = ctx.saved_tensors
+        return ops.softmax_bwd(p, grad_output.to(p.dtype), ctx.causal, fill_upper=ctx.fill_upper), None, None, None
+
+
+def _weight_of(module) -> torch.Tensor:
+    weight = module._parameters.get("weight")
+    return weight if weight is not None else module.weight   # (a parametrised weight is an attribute)
+
+
+def _wants_grad(xq, xk, xv, weights) -> bool:
+    return torch.is_grad_enabled() and (xq.requires_grad or xk.requires_grad or xv.requires_grad
+                                        or any(w.requires_grad for w in weights))
 
 
 @dataclass
@@ -427,227 +322,63 @@ class MTAAttentionTriton(nn.Module):
 
     def forward(self, xq, xk, xv, mask, chunk_start_ids):
         assert chunk_start_ids is None, "MTAAttentionTriton does not support chunked attention"
-        wants_grad = torch.is_grad_enabled() and (xq.requires_grad or xk.requires_grad or xv.requires_grad
-                                                  or any(p.requires_grad for p in self.parameters()))
         if self.use_mask:
-            return self._forward_with_mask(xq, xk, xv, mask, wants_grad)
-        if wants_grad:
-            return self._forward_stagewise(xq, xk, xv)
-        return self._forward_fused(xq, xk, xv)
+            return self._forward_with_mask(xq, xk, xv, mask)
+        return self._forward_native(xq, xk, xv)
 
-    def _forward_fused(self, xq, xk, xv, key_bias=None, first_visible=None, empty_rows=None):
-        """Inference route (module docstring).  ``key_bias``: fp32 (B,Sk), added to the mixed scores ahead of the
-        softmax -- the caller has zeroed the K and V rows of the keys it hides.  ``first_visible``: int32 (B,S), a band
-        mask (row p sees the keys first_visible[p] .. p): applied to the scores inside the first kernel and as -inf
-        inside the softmax kernel, and behind a post-softmax conv that is not the identity the hidden stretch of every row
-        is zeroed again; the caller has checked that the first kernel exists.  ``empty_rows``: bool (B,S) or None, the
-        rows of the band that see no key (first_visible[p] = p + 1).  Their scores enter the conv as 0 like any hidden
-        score; the softmax leaves NaN in them, which the reference replaces by zeros ahead of its post-softmax conv
-        (mta_attention_triton.py:81): here those rows of the probabilities are cleared ahead of a post-softmax conv
-        that is not the identity, and their rows of the output, where nothing else would, at the end."""
-        head_dim = xq.size(-1)
-        # the reference multiplies by rsqrt(tensor(head_dim)), an fp32 scalar (mta_attention_triton.py:69-71)
-        scale = float(torch.rsqrt(torch.tensor(float(head_dim))))
+    def _weights(self):
+        """The four weights, in the order of the stages (looked up in the submodules' parameter tables: attribute access on
+        a module is a microsecond each)."""
+        modules = self._modules
+        return (_weight_of(modules["mta_conv_triton"]), _weight_of(modules["wpsm_triton"]),
+                _weight_of(modules["mta_conv_after_sm_triton"]), _weight_of(modules["wposm_triton"]))
+
+    def _forward_native(self, xq, xk, xv, key_bias=None, first_visible=None, empty_rows=None):
+        """Both routes of the module docstring in native code (csrc/host/mta_host.cpp).  ``key_bias``: fp32 (B,Sk), added to
+        the mixed scores ahead of the softmax; the K and V rows of the keys it hides count as zeros.  ``first_visible``:
+        int32 (B,S), a band mask (row p sees the keys first_visible[p] .. p); the caller has checked that the first kernel
+        exists.  ``empty_rows``: bool (B,S) or None, the rows of the band that see no key (first_visible[p] = p + 1)."""
+        weights = self._weights()
+        host = _lib.host()
+        dropout = self.dropout if self.training else 0.0
+        if _wants_grad(xq, xk, xv, weights):
+            pre, post = self._modules["wpsm_triton"], self._modules["wposm_triton"]
+            return host.forward_training(xq, xk, xv, *weights, self.causal, pre.causal, post.causal, pre.output_value, post.output_value,
+                                         pre.group_size or 0, post.group_size or 0, key_bias, first_visible, empty_rows, dropout,
+                                         self._stage_hook)
         st = self._current_structure()
-        w_pre, w_post = self.wpsm_triton.weight, self.wposm_triton.weight
-        g_pre = st.pre_head_group or self.n_heads
-        g_post = st.post_head_group or self.n_heads
-        w1 = None if st.pre_head_identity else w_pre
-        w2 = None if st.post_head_identity else w_post
-        if w1 is None:
-            g_pre = 1
-        if w2 is None:
-            g_post = 1
-        post_conv_identity = st.post_conv_identity
-        n_keys = xk.size(-2)
-        g_both = _lcm(g_pre, g_post)
-        # (the matrix-core variant for groups of 16 takes a key bias or a band mask in its row-list form only)
-        row_plain = key_bias is None and first_visible is None
-        masks_ok = lambda group: row_plain or group <= _FUSED_MAX_GROUP or (
-            group == _FUSED_MFMA_GROUP and os.environ.get("MTA_MIX16_NO_ROW_LISTS") != "1")
-        one_pass = post_conv_identity and _one_pass_group(g_both, xq.dtype, n_keys, w1, w2) and masks_ok(g_both)
-        # the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
-        own_pv = (xq.size(-2) == xk.size(-2) and xq.dtype == xv.dtype
-                  and ops.causal_pv_supported(xq.dtype, xq.size(-2), xv.size(-1)))
+        return host.forward_inference(xq, xk, xv, *weights, self.causal, st.pre_head_identity, st.pre_head_group or 0, st.post_conv_identity,
+                                      st.post_head_identity, st.post_head_group or 0, key_bias, first_visible, empty_rows,
+                                      self.score_layout == "planes", dropout, self._stage_hook)
 
-        # Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they
-        # travel in the triangular layout (what lies on and below the diagonal only, the rows a workgroup of the softmax
-        # stage reads side by side): half the footprint, and every stage streams memory in longer runs.
-        if (self.score_layout != "planes" and self.causal and one_pass and own_pv
-                and not (self.training and self.dropout > 0) and g_both in (2, 4, 8, 16)
-                and (key_bias is None or (key_bias.is_contiguous() and key_bias.data_ptr() % 16 == 0))
-                and ops.tri_route_supported(xq, xk, self.mta_conv_triton.weight, g_both, w1, w2, first_visible is not None,
-                                            key_bias=key_bias is not None)):
-            self._mark("qk_conv")
-            scores = ops.qk_conv_tri(xq, xk, self.mta_conv_triton.weight, scale, g_both, first_visible=first_visible)
-            self._mark("mix_softmax_mix")
-            scores = ops.headmix_softmax_tri(scores, w1, w2, xq.size(0), self.n_heads, n_keys, g_both,
-                                             first_visible=first_visible, key_bias=key_bias)
-            self._mark("pv")
-            output = ops.causal_pv_tri(scores, xv, g_both, first_visible=first_visible)
-            if empty_rows is not None:
-                output.masked_fill_(empty_rows[:, None, :, None], 0)
-            self._mark("end")
-            return output.transpose(1, 2)
-
-        # QK^T -> *1/sqrt(d) -> conv: one kernel when it exists for this dtype / size, else GEMM + conv
-        scores = None
-        # (dense groups of 16 heads ahead of a post-softmax conv: the first score tensor still travels in the triangular
-        # layout, the softmax stage hands the conv (B,H,S,S) planes)
-        tri_first = (self.score_layout != "planes" and self.causal and not one_pass and g_pre == 16 and masks_ok(16)
-                     and w1 is not None and not (post_conv_identity and w2 is None and not own_pv)
-                     and (key_bias is None or key_bias.is_contiguous())
-                     and ops.tri_route_supported(xq, xk, self.mta_conv_triton.weight, 16, w1, None, first_visible is not None,
-                                                 out_planes=True, key_bias=key_bias is not None))
-        if tri_first:
-            self._mark("qk_conv")
-            scores = ops.qk_conv_tri(xq, xk, self.mta_conv_triton.weight, scale, 16, first_visible=first_visible)
-        elif ops.qk_conv_supported(xq, xk, self.mta_conv_triton.weight):
-            self._mark("qk_conv")
-            scores = ops.qk_conv(xq, xk, self.mta_conv_triton.weight, self.causal, scale, fill_upper=False,
-                                 first_visible=first_visible)
-        if scores is None:
-            assert first_visible is None, "the band mask needs the one-kernel first stage"
-            self._mark("qk")
-            scores = torch.matmul(xq, xk.transpose(2, 3))
-            self._mark("conv_pre")
-            scores = ops.conv2d_causal(scores, self.mta_conv_triton.weight, self.causal, in_scale=scale)
-
-        if one_pass:
-            self._mark("mix_softmax_mix")
-            scores = ops.headmix_softmax(scores, w1, w2, self.causal, group_size=g_both,
-                                         fill_upper=not own_pv, key_bias=key_bias, first_visible=first_visible)
-        else:
-            if tri_first:
-                self._mark("mix_softmax")
-                scores = ops.headmix_softmax_tri(scores, w1, None, xq.size(0), self.n_heads, n_keys, g_pre, out_planes=True,
-                                                 first_visible=first_visible, key_bias=key_bias)
-            elif _one_pass_group(g_pre, xq.dtype, n_keys, w1) and masks_ok(g_pre):
-                self._mark("mix_softmax")
-                scores = ops.headmix_softmax(scores, w1, None, self.causal, group_size=g_pre, key_bias=key_bias,
-                                             first_visible=first_visible,
-                                             fill_upper=post_conv_identity and w2 is None and not own_pv)
-            else:
-                self._mark("mix_pre")
-                fill = float("-inf") if self.causal else 0.0
-                # (the softmax kernel that follows never reads above the diagonal)
-                scores = ops.headmix(scores, w_pre, self.causal, fill, group_size=g_pre, fill_upper=False)
-                self._mark("softmax")
-                scores = ops.headmix_softmax(scores, None, None, self.causal, key_bias=key_bias,
-                                             first_visible=first_visible,
-                                             fill_upper=post_conv_identity and w2 is None and not own_pv)
-            if empty_rows is not None and not post_conv_identity:
-                # (the rows that see nothing, NaN out of the softmax: zeros into the conv, whole rows up to the diagonal)
-                rows_all = torch.arange(1, n_keys + 1, device=empty_rows.device, dtype=torch.int32)
-                if ops.band_zero_(scores, torch.where(empty_rows, rows_all[None, :], 0).to(torch.int32)) is None:
-                    raise RuntimeError("band masks need 16-bit scores of a length that is a multiple of 8")
-            done = None
-            # conv and mix in one pass, the conv result never written: taken where it measures at least as fast as the
-            # two kernels (mixing groups of up to 4 heads, kernel sizes with a vector-staged instance: 3x3, 7x7)
-            ks = tuple(self.mta_conv_after_sm_triton.weight.shape[1:])
-            conv_w = self.mta_conv_after_sm_triton.weight
-            mix16 = (g_post == 16 and ks in _CONV_MIX16_SIZES and scores.dtype in (torch.bfloat16, torch.float16)
-                     and conv_w.dtype == scores.dtype and w_post.dtype == scores.dtype and n_keys % 8 == 0)
-            # (under a band mask the conv's result is zeroed at the hidden positions ahead of the mixing, as the reference
-            # does: two kernels with that step between them)
-            if first_visible is None and not post_conv_identity and w2 is not None and (
-                    (g_post <= _CONV_MIX_MAX_GROUP and ks in _CONV_MIX_SIZES) or mix16):
-                self._mark("conv_mix_post")
-                done = ops.conv2d_headmix(scores, self.mta_conv_after_sm_triton.weight, w_post, self.causal,
-                                          group_size=g_post, fill_upper=not own_pv)
-            if done is not None:
-                scores = done
-            else:
-                # neither our head mixing nor our P V reads above the diagonal: whoever feeds them need not write there
-                if not post_conv_identity:
-                    self._mark("conv_post")
-                    scores = ops.conv2d_causal(scores, self.mta_conv_after_sm_triton.weight, self.causal,
-                                               fill_upper=w2 is None and not own_pv)
-                    if first_visible is not None:
-                        # the conv has spread probability into columns the rows do not see
-                        # (mta_attention_triton.py:82-83: torch.where(mask == -inf, 0.0, scores))
-                        if ops.band_zero_(scores, first_visible) is None:
-                            raise RuntimeError("band masks need 16-bit scores of a length that is a multiple of 8")
-                if w2 is not None:
-                    self._mark("mix_post")
-                    scores = ops.headmix(scores, w_post, self.causal, 0.0, group_size=g_post, fill_upper=not own_pv)
-
-        scores = F.dropout(scores, p=self.dropout, training=self.training)
-        self._mark("pv")
-        output = ops.causal_pv(scores, xv, self.causal, first_visible=first_visible) if own_pv else None
-        if output is None:
-            output = torch.matmul(scores, xv)
-        if empty_rows is not None:
-            output.masked_fill_(empty_rows[:, None, :, None], 0)
-        self._mark("end")
-        return output.transpose(1, 2)
-
-    def _forward_stagewise(self, xq, xk, xv, key_bias=None, first_visible=None, mask_planes=None, mask_additive=None,
-                           mask_empty_rows=False, band_empty_rows=None):
-        """The reference's own sequence of operators (mta_attention_triton.py:68-92), each differentiable: taken
-        whenever a gradient may be asked for.  No weight structure is assumed here, so every entry of the four
-        weights receives its gradient.
-
-        ``key_bias`` (fp32 (B,Sk), 0 / -inf per key, or finite values of a 2-D additive mask): "causal rule + hidden
-        keys" under use_mask (mta_attention_triton.py:72-73, 77, 81-83).  The K and V rows of the hidden keys are zeroed
-        (differentiably: those rows receive no gradient, as in the reference, whose masked_fill / where cut it): the
-        scores of their columns then enter the pre-softmax conv as 0, the bias hides them from the softmax, and what the
-        post-softmax conv writes into their columns meets zero V rows - and receives a zero gradient from them.
-
-        ``first_visible`` (int32 (B,S)): a band mask, row p sees the keys first_visible[p] .. p.  Applied where the
-        reference applies the mask tensor: to the scores ahead of the pre-softmax conv (inside the scores kernel), as
-        -inf inside the softmax kernel, and as zeros behind the post-softmax conv; the caller has checked that the
-        kernels this needs exist (``_band_training_supported``).
-
-        ``mask_planes`` (uint8 (1|B, 1|H, S, S), non-zero = attend): a 0 / -inf mask of arbitrary content.  The three
-        elementwise mask steps of the reference run as in-place passes between the operators (``_MaskFill``, and inside
-        ``_ScaledScoresConv``); head mixing and softmax run as two kernels, the mask goes between them."""
-        if key_bias is not None:
-            hidden = (key_bias == float("-inf"))[:, None, :, None]
-            xk = xk.masked_fill(hidden, 0)
-            xv = xv.masked_fill(hidden, 0)
+    def _forward_stagewise_planes(self, xq, xk, xv, mask_planes, mask_additive=None, mask_empty_rows=False):
+        """Training under a mask of arbitrary content: the reference's own sequence of operators
+        (mta_attention_triton.py:68-92), each differentiable.  ``mask_planes`` (uint8 (1|B, 1|H, S, S), non-zero = attend);
+        the three elementwise mask steps of the reference run as in-place passes between the operators (``_MaskFill``, and
+        inside ``_ScaledScoresConv``); head mixing and softmax run as two kernels, the mask goes between them.
+        ``mask_additive``: finite values besides 0, the mask in the scores' dtype is added.  No weight structure is assumed
+        here, so every entry of the four weights receives its gradient."""
         scale = float(torch.rsqrt(torch.tensor(float(xq.size(-1)))))
-        scores = _ScaledScoresConv.apply(xq, xk, self.mta_conv_triton.weight, scale, self.causal, self._mark,
-                                         first_visible, mask_planes)
-        group = self.wpsm_triton.group_size
-        w_pre = self.wpsm_triton.weight
+        scores = _ScaledScoresConv.apply(xq, xk, self.mta_conv_triton.weight, scale, self.causal, self._mark, mask_planes)
         # Between two of these stages nothing reads above the diagonal (causal kernels never do, in either direction),
         # so nothing is written there: only the last stage's output, which torch's GEMM reads in full, and the score
         # gradient that goes into torch's GEMMs (inside _ScaledScoresConv) are filled.
         lower = not self.causal   # value of the fill flags: False (leave alone) when causal
-        # (band_empty_rows: bool (B,S), the rows of the band mask that see no key: their probabilities are cleared)
-        zero_rows = mask_planes if mask_empty_rows else None
-        if band_empty_rows is not None:
-            rows_all = torch.arange(1, xk.size(-2) + 1, device=xq.device, dtype=torch.int32)
-            zero_rows = torch.where(band_empty_rows, rows_all[None, :], 0).to(torch.int32).contiguous()
-        g_eff = group or self.n_heads
-        # (the matrix-core variant for groups of 16 takes a key bias in its row-list form only)
-        bias_ok = (key_bias is None and first_visible is None) or g_eff <= _FUSED_MAX_GROUP or (
-            g_eff == _FUSED_MFMA_GROUP and os.environ.get("MTA_MIX16_NO_ROW_LISTS") != "1")
-        if _one_pass_group(g_eff, scores.dtype, xk.size(-2), w_pre) and bias_ok and mask_planes is None:
-            self._mark("mix_softmax")
-            scores = _MixSoftmax.apply(scores, w_pre, self.causal, group, lower, lower, key_bias, first_visible, zero_rows)
+        pre, post = self.wpsm_triton, self.wposm_triton
+        self._mark("mix_pre")
+        scores = TritonLinearHeadFunction.apply(scores, pre.weight, pre.causal, pre.output_value, pre.group_size, lower, lower)
+        self._mark("mask")
+        if mask_additive is None:
+            scores = _MaskFill.apply(scores, mask_planes, True, self.causal)
         else:
-            self._mark("mix_pre")
-            scores = TritonLinearHeadFunction.apply(scores, w_pre, self.wpsm_triton.causal, self.wpsm_triton.output_value,
-                                                    group, lower, lower)
-            if mask_planes is not None:
-                self._mark("mask")
-                if mask_additive is None:
-                    scores = _MaskFill.apply(scores, mask_planes, True, self.causal)
-                else:   # (finite values besides 0: the mask in the scores' dtype is added)
-                    scores = _MaskAdd.apply(scores, mask_additive, self.causal)
-            self._mark("softmax")
-            scores = _MixSoftmax.apply(scores, None, self.causal, None, lower, lower, key_bias, first_visible, zero_rows)
+            scores = _MaskAdd.apply(scores, mask_additive, self.causal)
+        self._mark("softmax")
+        scores = _Softmax.apply(scores, self.causal, lower, mask_planes if mask_empty_rows else None)
         self._mark("conv_post")
         scores = Conv2dTritonFunction.apply(scores, self.mta_conv_after_sm_triton.weight, self.causal, lower, lower)
-        if first_visible is not None:
-            scores = _BandZero.apply(scores, first_visible)
-        if mask_planes is not None:
-            self._mark("mask")
-            scores = _MaskFill.apply(scores, mask_planes, False, self.causal)
+        self._mark("mask")
+        scores = _MaskFill.apply(scores, mask_planes, False, self.causal)
         self._mark("mix_post")
-        post = self.wposm_triton
         # the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
         lower_pv = (self.causal and post.causal and scores.dtype == xv.dtype
                     and _lower_products_supported(xv, scores.size(-1)) and scores.size(-2) == scores.size(-1))
@@ -657,8 +388,7 @@ class MTAAttentionTriton(nn.Module):
         self._mark("pv")
         # (the gradient with respect to the probabilities goes back into the head mixing's gradient kernels, through the
         # dropout's elementwise mask at most: nothing there reads above the diagonal when causal)
-        assert first_visible is None or lower_pv
-        output = _ProbsTimesValues.apply(scores, xv, lower_pv, first_visible)
+        output = _ProbsTimesValues.apply(scores, xv, lower_pv)
         self._mark("end")
         return output.transpose(1, 2)
 
@@ -707,7 +437,7 @@ class MTAAttentionTriton(nn.Module):
         self._declared = WeightStructure()
         self.weight_structure = "dense"
 
-    def _forward_with_mask(self, xq, xk, xv, mask, wants_grad=True):
+    def _forward_with_mask(self, xq, xk, xv, mask):
         """use_mask=True: an explicit additive mask tensor drives the masking (mta_attention_triton.py:63-64,
         77-83, 96-98); the kernels still apply their own causal rule when ``causal`` is set.
 
@@ -722,17 +452,15 @@ class MTAAttentionTriton(nn.Module):
         8 is read as a byte per position by three mask passes between the single-stage kernels; what is left takes the
         reference's own steps, at the end of this function."""
         if self.causal and xq.size(-2) == xk.size(-2):
-            # (with a gradient wanted: the same masks through the differentiable operators)
-            hidden_keys = self._forward_stagewise_hidden_keys if wants_grad else self._forward_hidden_keys
             if not isinstance(mask, torch.Tensor):
-                return self._forward_stagewise(xq, xk, xv) if wants_grad else self._forward_fused(xq, xk, xv)
+                return self._forward_native(xq, xk, xv)
             if mask.dim() == 2 and xq.size(0) == 1:
                 assert mask.size(0) == xq.size(0)
                 if mask.dtype == torch.bool:
                     bias = torch.where(mask, 0.0, float("-inf")).to(torch.float32)
                 else:
                     bias = mask.type(xq.dtype).to(torch.float32)   # the reference adds it in the I/O dtype
-                return hidden_keys(xq, xk, xv, bias.contiguous())
+                return self._forward_native(xq, xk, xv, key_bias=bias.contiguous())
             # a 4-D mask, the same for all heads, of one of two forms goes into the kernels without a (B,H,S,S) tensor:
             # "causal rule + hidden keys" per batch entry (key padding: a key bias and zeroed K and V rows, as for the
             # 2-D mask above) and "row p sees the keys first[p] .. p" (sliding windows, packed documents: one int32 per
@@ -740,21 +468,16 @@ class MTAAttentionTriton(nn.Module):
             if mask.dim() == 4:
                 kind, what = self._structured_mask(mask, xq.size(0), xq.size(-2))
                 if kind == "keys":
-                    return hidden_keys(xq, xk, xv, what)
-                if kind == "band" and ops.qk_conv_supported(xq, xk, self.mta_conv_triton.weight):
-                    empty_rows = self._band_empty_rows(mask)
-                    if not wants_grad:
-                        return self._forward_fused(xq, xk, xv, first_visible=what, empty_rows=empty_rows)
-                    if self._band_training_supported(xq, xk, xv):
-                        return self._forward_stagewise(xq, xk, xv, first_visible=what, band_empty_rows=empty_rows)
+                    return self._forward_native(xq, xk, xv, key_bias=what)
+                if (kind == "band" and ops.qk_conv_supported(xq, xk, self.mta_conv_triton.weight)
+                        and (not _wants_grad(xq, xk, xv, self._weights()) or self._band_training_supported(xq, xk, xv))):
+                    return self._forward_native(xq, xk, xv, first_visible=what, empty_rows=self._band_empty_rows(mask))
         elif (not self.causal and isinstance(mask, torch.Tensor) and mask.dim() == 4 and xq.size(-2) == xk.size(-2)):
             # no causal rule and a mask that hides the same keys from every row (key padding of an encoder batch): the same
             # key bias and zeroed K and V rows, through the kernels' non-causal form
             kind, what = self._structured_mask(mask, xq.size(0), xq.size(-2))
             if kind == "keys":
-                if wants_grad:
-                    return self._forward_stagewise(xq, xk, xv, key_bias=what)
-                return self._forward_hidden_keys(xq, xk, xv, what)
+                return self._forward_native(xq, xk, xv, key_bias=what)
         if (isinstance(mask, torch.Tensor) and mask.dim() == 4 and xq.size(-2) == xk.size(-2) and xk.size(-2) % 8 == 0):
             planes, additive, empty_rows = self._mask_planes(mask, xq.size(0), xq.size(-2))
             if additive is not None:   # (the reference adds the mask in the scores' dtype)
@@ -762,9 +485,8 @@ class MTAAttentionTriton(nn.Module):
                 if additive.data_ptr() % 16 != 0:
                     planes = None
             if planes is not None:
-                if wants_grad:
-                    return self._forward_stagewise(xq, xk, xv, mask_planes=planes, mask_additive=additive,
-                                                   mask_empty_rows=empty_rows)
+                if _wants_grad(xq, xk, xv, self._weights()):
+                    return self._forward_stagewise_planes(xq, xk, xv, planes, additive, empty_rows)
                 return self._forward_mask_planes(xq, xk, xv, planes, additive, empty_rows)
         mask = self._update_mask(mask=mask, bsz=xq.size(0), xq=xq, xk_size=xk.size(-2))
         scale = float(torch.rsqrt(torch.tensor(float(xq.size(-1)))))  # a host scalar: the product stays one vectorised pass
@@ -849,19 +571,6 @@ class MTAAttentionTriton(nn.Module):
                 and _lower_products_supported(xq, s)
                 and all(w.dtype == xq.dtype for w in (self.mta_conv_triton.weight, self.mta_conv_after_sm_triton.weight,
                                                       self.wpsm_triton.weight, self.wposm_triton.weight)))
-
-    def _forward_stagewise_hidden_keys(self, xq, xk, xv, bias):
-        return self._forward_stagewise(xq, xk, xv, key_bias=bias)
-
-    def _forward_hidden_keys(self, xq, xk, xv, bias):
-        """The fused route under "causal rule + one additive value per (batch entry, key)" (``bias``: fp32 (B,S)).  The K
-        rows of hidden keys (-inf) are zeroed: their scores then enter the pre-softmax conv as 0.  Their probabilities
-        are 0; a post-softmax conv that is not the identity writes into their columns all the same, which the reference
-        zeroes again - here those columns meet zeroed V rows instead."""
-        hidden = (bias == float("-inf"))[:, None, :, None]
-        if not self._current_structure().post_conv_identity:
-            xv = xv.masked_fill(hidden, 0)
-        return self._forward_fused(xq, xk.masked_fill(hidden, 0), xv, key_bias=bias)
 
     def _structured_mask(self, mask, bsz: int, s: int):
         """What a 4-D ``mask`` (bool with True = attend, or additive with 0 / -inf; one plane for all heads) amounts to
@@ -1012,11 +721,6 @@ class MTAAttentionTriton(nn.Module):
             if hasattr(mta_attention, "wposm"):
                 self.wposm_triton.weight.copy_(mta_attention.wposm.weight.data)
         self.assume_dense_weights()
-
-
-def _lcm(a: int, b: int) -> int:
-    import math
-    return a * b // math.gcd(a, b)
 
 
 __all__ = ["MTAAttentionTriton", "MTAConfig", "WeightStructure"]

@@ -13,41 +13,23 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from . import ops
+from . import _lib
 
 
 class TritonLinearHeadFunction(torch.autograd.Function):
-    """apply(input (N,C,P,Q), weight (C,C), causal=True, output_value=0.0[, group_size]).
+    """apply(input (N,C,P,Q), weight (C,C), causal=True, output_value=0.0[, group_size]), differentiable: forward and
+    backward (triton_linear_head.py:281-370) are one native autograd node (csrc/host/mta_host.cpp).
 
     Two optional flags for callers that know who reads the results (both only matter when ``causal``):
     ``fill_upper=False`` -- the output is only read on and below the diagonal; ``grad_fill_upper=False`` -- so is the
     input gradient that backward returns.  What lies above the diagonal is then left unwritten."""
 
     @staticmethod
-    def forward(ctx, input, weight, causal=True, output_value=0.0, group_size=None, fill_upper=True,
-                grad_fill_upper=True):
-        ctx.save_for_backward(input, weight)
-        ctx.causal = causal
-        ctx.group_size = group_size
-        ctx.grad_fill_upper = grad_fill_upper
-        return ops.headmix(input, weight, causal, output_value, group_size, fill_upper=fill_upper)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        """triton_linear_head.py:322-370.  Above the diagonal the input gradient is 0 (the reference leaves
-        ``torch.empty_like`` memory there); the weight gradient is accumulated in fp32 and cast."""
-        input, weight = ctx.saved_tensors
-        grad_input = grad_weight = None
-        if ctx.needs_input_grad[0]:
-            grad_input = ops.headmix_bwd_input(grad_output, weight, ctx.causal, ctx.group_size,
-                                               fill_upper=ctx.grad_fill_upper)
-        if ctx.needs_input_grad[1]:
-            grad_weight = ops.headmix_bwd_weight(input, grad_output.to(input.dtype), ctx.causal)
-            if ctx.group_size:
-                blk = torch.arange(weight.shape[0], device=weight.device) // ctx.group_size
-                grad_weight = grad_weight * (blk[:, None] == blk[None, :])
-            grad_weight = grad_weight.to(weight.dtype)
-        return grad_input, grad_weight, None, None, None, None, None
+    def apply(input, weight, causal=True, output_value=0.0, group_size=None, fill_upper=True, grad_fill_upper=True):
+        # same checks and messages as triton_linear_head.py:286-290
+        assert weight.size(0) == weight.size(-1), f"Weight must be square matrix, got {weight.shape}"
+        assert input.size(1) == weight.size(0), f"Channel dimension {input.size(1)} must match weight dimension {weight.size(0)}"
+        return _lib.host().headmix_apply(input, weight, causal, output_value, group_size or 0, fill_upper, grad_fill_upper)
 
 
 class TritonLinearHead(nn.Module):
