@@ -1,0 +1,28 @@
+// The 16-bit kernels of the fused conv-attention path by I/O type; returns 1 when no instance covers the kernel size (the
+// caller then uses the general kernel).  scores_only: stop after the conv (o = the score tensor; band_lo, tri_gl and
+// fill_upper belong to it), else the attention output (lse may be NULL).
+#pragma once
+
+#include "common.hpp"
+
+namespace mta {
+struct conv_attn_args {
+    const void *q, *k, *v, *w;
+    void *o;
+    float *lse;
+    int64_t B, H, S, D;
+    int R, Sk, causal;
+    float scale;
+    int fill_upper;
+    const int *band_lo;   // scores only: first visible key per row, or NULL
+    int tri_gl;           // scores only: > 0 = triangular layout, groups of that many heads
+    bool scores_only;
+    hipStream_t st;
+};
+int conv_attn_mfma_bf16(const conv_attn_args &a);
+int conv_attn_mfma_f16(const conv_attn_args &a);
+inline int conv_attn_mfma_dispatch(int io_dtype, const conv_attn_args &a)
+{
+    return io_dtype == MTA_BF16 ? conv_attn_mfma_bf16(a) : io_dtype == MTA_F16 ? conv_attn_mfma_f16(a) : 1;
+}
+}  // namespace mta

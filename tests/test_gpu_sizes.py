@@ -1,0 +1,50 @@
+"""GPU parity at the sizes where a kernel's tiling can go wrong - remainders, edges of tiles, the smallest of a range - for
+kernel variants that a rule on sizes or types chooses.  Against the CPU oracle; tolerances as in test_gpu_attention.py for
+module outputs (fp32 rtol 1e-4 / atol 1e-5, 16-bit atol 2e-2), derived where the test says so."""
+import pytest
+import torch
+
+from oracle import mta_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def tol(dtype):
+    return dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=0.0, atol=2e-2)
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    import multitokenatention_triton_amd as m
+    return m
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype,r,sk", [(torch.bfloat16, 3, 5), (torch.float16, 7, 9), (torch.bfloat16, 11, 15),
+                                        *[(torch.float32, *k) for k in ((3, 3), (3, 5), (5, 5), (5, 7), (6, 11), (7, 7), (7, 9), (11, 15))]])
+def test_conv_attention_kernel_sizes(pkg, dtype, r, sk, d, causal):
+    """Every compile-time kernel size of the fused kernels: one row, one key block, edges of the 118- to 128-row query
+    blocks and 64-key blocks."""
+    for s in (1, 63, 121, 130, 257):
+        print(f"conv_attention {dtype} {r}x{sk} d={d} s={s} causal={causal}", flush=True)
+        q, k, v = O.seeded_qkv(1, 2, s, d, dtype, seed=43)
+        w = O.seeded_conv_weight(2, r, sk, 0.05, dtype)
+        want = O.conv_attention_forward(q, k, v, w, causal, None)
+        got = pkg.ops.conv_attn_fwd(q.cuda(), k.cuda(), v.cuda(), w.cuda(), causal, None).cpu()
+        torch.testing.assert_close(got.float(), want.float(), **tol(dtype))
+
+
+@pytest.mark.parametrize("dtype,r,sk", [(torch.bfloat16, 3, 5), (torch.float16, 7, 9)])
+def test_qk_conv_kernel_sizes(pkg, dtype, r, sk):
+    """The scores stage at the same sizes; bound as in test_qk_conv_parity: two 16-bit roundings of scores of magnitude
+    sqrt(d)*|w|, i.e. 2 ulp + atol."""
+    for s, d in ((8, 64), (120, 128), (264, 64), (1032, 128)):
+        print(f"qk_conv {dtype} {r}x{sk} d={d} s={s}", flush=True)
+        q, k, _ = O.seeded_qkv(1, 2, s, d, dtype, seed=7)
+        w = O.seeded_conv_weight(2, r, sk, 0.05, dtype)
+        scale = float(torch.rsqrt(torch.tensor(float(d))))
+        want = O.depthwise_conv(torch.tril(torch.matmul(q, k.transpose(2, 3)) * torch.rsqrt(torch.tensor(d))), w, True)
+        got = pkg.ops.qk_conv(q.cuda(), k.cuda(), w.cuda(), True, scale).cpu()
+        ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+        torch.testing.assert_close(got.float(), want.float(), rtol=2 * ulp, atol=2e-2)
