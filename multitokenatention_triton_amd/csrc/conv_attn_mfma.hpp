@@ -49,8 +49,25 @@ constexpr int QK_OCC = 3;     // wavefronts per SIMD the scores-only kernel is c
 constexpr int QK_CHUNK = 32;  // key blocks per work item of the scores-only kernel when no item table is built
 // with an item table: long and short items (key blocks), and the share of a query block's key range that goes into short
 // ones (MTA_QK_CHUNK_LONG / MTA_QK_CHUNK_SHORT / MTA_QK_SHORT_PERCENT in the environment override them, for comparisons)
-// (measured at B2 H16 S4096 D128: 32/32/0 237 us, 16/16/0 231, 64/16/50 238, 48/24/50 228, 52/26/50 227, 48/24/35 243)
-constexpr int QK_CHUNK_LONG = 48, QK_CHUNK_SHORT = 24, QK_SHORT_PERCENT = 50;
+// (long items measured at B2 H16 S4096 D128: 32/32/0 237 us, 16/16/0 231, 64/16/50 238, 48/24/50 228, 52/26/50 227, 48/24/35 243)
+constexpr int QK_SHORT_PERCENT = 50;
+constexpr int ITEM_TABLE_MAX = 768;
+struct qk_chunks { int big, small; };
+// How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 24000 on the grid
+// runs in several rounds whatever the length and 48/24 keeps the rebuilt columns few; below, items as short as it takes to
+// have two or three per CU, down to one key block, win although each rebuilds one key block's worth of columns: the grid is
+// otherwise a fraction of the chip, each workgroup walking its keys alone.  Measured (us, with 48/24 -> with this rule):
+// B1 H8 S256 D64 3x3 (80 blocks) 13.3 -> 7.6; B1 H16 S512 D128 5x5 (448) 23.3 -> 11.5; B2 H16 S512 D64 6x11 (896) 22.6 -> 13.4;
+// B4 H16 S512 (1792) 26.3 -> 22.0; B1 H8 S2048 D64 (2450) 48.9 -> 23.9; B1 H16 S2048 D128 7x7 (4900) 60.4 -> 40.8;
+// B1 H16 S4096 D128 7x7 (18900) 140 -> 133.
+inline qk_chunks qk_chunk_rule(int64_t blocks, int64_t head_blocks, int nqb)
+{
+    if (blocks >= 24000) return {48, 24};
+    if (blocks < 600) return {1, 1};
+    int small = (int)std::min<int64_t>(std::max<int64_t>((blocks + 400) / 800, 1), 8);
+    while (head_blocks / small + 2 * nqb > ITEM_TABLE_MAX && small < 24) small *= 2;   // (the table holds one head's items)
+    return {2 * small, small};
+}
 constexpr int F_SLD = 80;  // score-tile row stride (elements): exactly the retained columns + one key block.  A wider
                            // row costs the scores-only kernel its third workgroup per CU, and with this one a fragment
                            // read (16 consecutive rows x 64 bytes) is free of bank conflicts as it is: the LDS serves
@@ -171,7 +188,6 @@ template <int R, int SK, int NW> struct fused_geom {
 // The chunks need not be equal: the first part of a query block's key range goes into long items (one extra key block
 // per item rebuilds the retained score columns, and an item costs a few microseconds to set up), the rest into short
 // ones, which are started last and even out the end of the grid.
-constexpr int ITEM_TABLE_MAX = 768;
 struct item_table {
     int n;
     uint32_t e[ITEM_TABLE_MAX];  // query block (11 bits) | first key block << 11 (11 bits) | key blocks << 22
@@ -793,9 +809,16 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
         static thread_local uint32_t items[ITEM_TABLE_MAX];
         static thread_local int lens[ITEM_TABLE_MAX];
         // long chunks for the first part of a query block's key range, short ones for the last QK_SHORT_SHARE of it
-        static const int big = [] { const char *e = getenv("MTA_QK_CHUNK_LONG"); return e ? atoi(e) : QK_CHUNK_LONG; }();
-        static const int small = [] { const char *e = getenv("MTA_QK_CHUNK_SHORT"); return e ? atoi(e) : QK_CHUNK_SHORT; }();
+        static const int env_big = [] { const char *e = getenv("MTA_QK_CHUNK_LONG"); return e ? atoi(e) : 0; }();
+        static const int env_small = [] { const char *e = getenv("MTA_QK_CHUNK_SHORT"); return e ? atoi(e) : 0; }();
         static const int share = [] { const char *e = getenv("MTA_QK_SHORT_PERCENT"); return e ? atoi(e) : QK_SHORT_PERCENT; }();
+        int64_t head_blocks = 0;
+        for (int qb = 0; qb < nqb; ++qb) {
+            const int64_t ql = std::min<int64_t>((int64_t)qb * G::BQ + G::BQ - 1, S - 1);
+            head_blocks += (causal ? ql / F_BK : (S - 1) / F_BK) + 1;
+        }
+        const qk_chunks cut = qk_chunk_rule(B * H * head_blocks, head_blocks, nqb);
+        const int big = env_big ? env_big : cut.big, small = env_small ? env_small : cut.small;
         int n = 0;
         bool ok = big >= 1 && small >= 1 && big <= MAXLEN && small <= MAXLEN && share >= 0 && share <= 100;
         for (int qb = 0; qb < nqb && ok; ++qb) {
