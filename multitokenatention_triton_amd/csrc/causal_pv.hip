@@ -243,6 +243,274 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
   }
 }
 
+// ---- small grids ----------------------------------------------------------------------------------------------------
+// The two products with 32 output rows per workgroup, whose four wavefronts take every fourth 32-row step of the contraction
+// each, on operands of their own in LDS (no barrier in the loop), and add their sums up at the end.  With 128 rows per
+// wavefront group a short sequence is a few dozen workgroups that each walk their keys alone; this is 8 times as many with a
+// quarter of the steps.  The price is that a V (X) block serves 32 rows instead of 128, so long sequences of many heads,
+// whose grids fill the chip anyway, keep the kernels above and below (narrow_grid()).
+constexpr int RB = 2, N_ROWS = 16 * RB;   // 16-row blocks, output rows per workgroup (64 rows: the sums leave too few registers)
+constexpr int N_STEP = 32;                // contraction rows per step
+// the sums of the four wavefronts, added in their order: wavefront w takes 16-wide blocks w, w+4, ... of the head dim
+template <typename T, int D, typename STORE>
+__device__ __forceinline__ void narrow_reduce(T *a, T *b, const f32x4 (&oacc)[RB][D / 16], int wave, int lane, STORE &&store)
+{
+    constexpr int DB = D / 16, PART = RB * DB * 64;   // 16-byte vectors of one wavefront's sums: half a buffer
+    static_assert((size_t)PART * 16 * 2 <= (size_t)4 * N_STEP * D * sizeof(T), "two wavefronts' sums fit a buffer");
+    f32x4 *const part[4] = {reinterpret_cast<f32x4 *>(a), reinterpret_cast<f32x4 *>(a) + PART, reinterpret_cast<f32x4 *>(b),
+                            reinterpret_cast<f32x4 *>(b) + PART};
+    __syncthreads();   // nobody reads operands any more
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) part[wave][(rb * DB + db) * 64 + lane] = oacc[rb][db];
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int i = 0; i < DB / 4; ++i) {
+            const int db = i * 4 + wave, at = (rb * DB + db) * 64 + lane;
+            store(rb, db, ((part[0][at] + part[1][at]) + part[2][at]) + part[3][at]);
+        }
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
+                                                                  int causal, int nrb, int64_t total_wg, int64_t per_xcd,
+                                                                  const int *__restrict__ band_lo, int H, int tri_gl)
+{
+    constexpr int CPR = D / 8, TILE = N_STEP * D, ROUNDS = TILE / 8 / 64, DB = D / 16;
+    __shared__ __align__(16) T v_a_all[4 * TILE];
+    __shared__ __align__(16) T v_b_all[4 * TILE];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    T *const v_a = v_a_all + wave * TILE;
+    T *const v_b = v_b_all + wave * TILE;
+    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (lid >= total_wg) return;
+    const int64_t bh = lid / nrb;
+    const int q0 = (nrb - 1 - (int)(lid % nrb)) * N_ROWS;   // longest rows first
+    const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
+    const T *Vp = V + bh * (int64_t)S * D;
+    T *Op = O + bh * (int64_t)S * D;
+
+    auto issue_v = [&](int j, T *dst) {   // keys past the sequence re-read the last one: their probabilities are masked
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            const int slot = r * 64 + lane, row = slot / CPR, c = (slot % CPR) ^ v_swizzle<D>(row);
+            int vr = j * N_STEP + row;
+            vr = vr >= S ? S - 1 : vr;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Vp + (int64_t)vr * D + c * 8), (lds_void_t *)(dst + r * 64 * 8), 16, 0, 0);
+        }
+    };
+    int prow[RB];
+    const T *prow_ptr[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        prow[rb] = q0 + rb * 16 + ln;
+        const int pc = prow[rb] < S ? prow[rb] : S - 1;
+        prow_ptr[rb] = tri_gl > 0 ? Pp + tri_gl * tri_rowoff(pc) + (int)(bh % tri_gl) * tri_rowlen(pc) + kg * 8
+                                  : Pp + (int64_t)pc * S + kg * 8;
+    }
+    auto load_p = [&](int j, frag8<T> (&pf)[RB]) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int key = j * N_STEP + kg * 8;
+            const bool ok = key < S && !(causal && key > prow[rb]);
+            pf[rb] = *reinterpret_cast<const frag8<T> *>(prow_ptr[rb] + (ok ? j * N_STEP : -kg * 8));
+        }
+    };
+    const int q_last = (q0 + N_ROWS - 1 < S - 1) ? q0 + N_ROWS - 1 : S - 1;
+    const int j_end = causal ? q_last / N_STEP : (S - 1) / N_STEP;
+    int j0 = 0;
+    if (band_lo) {   // the steps ahead of the first key any of these rows sees hold zeros
+        const int fr = q0 + (lane & 31);
+        int f = fr < S ? band_lo[(bh / H) * (int64_t)S + fr] : S;
+#pragma unroll
+        for (int off = N_ROWS / 2; off > 0; off >>= 1) {
+            const int o = __shfl_xor(f, off);
+            f = o < f ? o : f;
+        }
+        f = __builtin_amdgcn_readfirstlane(f);
+        j0 = (f > 0 ? f : 0) / N_STEP;
+        if (j0 > j_end) j0 = j_end;
+    }
+    // this wavefront's steps: j = wave (mod 4), by the step's own number (what a band mask skips leaves every sum as it is)
+    const int jw = j0 + ((wave - j0) & 3);
+    f32x4 oacc[RB][DB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[rb][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    frag8<T> p_a[RB], p_b[RB];
+    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pcur)[RB], frag8<T> (&pnext)[RB]) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);   // this wavefront's V block and P fragments have arrived
+        asm volatile("" ::: "memory");
+        if (j + 4 <= j_end) {
+            issue_v(j + 4, Vn);
+            load_p(j + 4, pnext);
+        }
+        frag8<T> pf[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int key0 = j * N_STEP + kg * 8;
+            pf[rb] = pcur[rb];
+            const int lim = causal ? (prow[rb] < S - 1 ? prow[rb] : S - 1) : S - 1;
+            if (key0 + 7 > lim) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    if (key0 + t > lim) pf[rb].v[t] = from_float<T>(0.0f);
+            }
+        }
+        auto load_vf = [&](int db, frag8<T> &dst) {
+            const int key_a = kg * 8 + (ln >> 2), key_b = key_a + 4, ch = db * 2 + ((ln & 3) >> 1), sub = (ln & 1) * 4;
+            const T *pa = Vb + key_a * D + ((ch ^ v_swizzle<D>(key_a)) * 8) + sub;
+            const T *pb = Vb + key_b * D + ((ch ^ v_swizzle<D>(key_b)) * 8) + sub;
+            struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pa),
+                                           __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pb)};
+            dst = __builtin_bit_cast(frag8<T>, both);
+        };
+        frag8<T> vf[2];
+        load_vf(0, vf[0]);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            if (db + 1 < DB) load_vf(db + 1, vf[(db + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) mma16(oacc[rb][db], vf[db & 1], pf[rb]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (jw <= j_end) {
+        issue_v(jw, v_a);
+        load_p(jw, p_a);
+        for (int j = jw;;) {
+            step(j, v_a, v_b, p_a, p_b);
+            if ((j += 4) > j_end) break;
+            step(j, v_b, v_a, p_b, p_a);
+            if ((j += 4) > j_end) break;
+        }
+    }
+    narrow_reduce<T, D>(v_a_all, v_b_all, oacc, wave, lane, [&](int rb, int db, const f32x4 &sum) {
+        if (prow[rb] >= S) return;
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v]);
+        *reinterpret_cast<quad *>(Op + (int64_t)prow[rb] * D + db * 16 + kg * 4) = out;
+    });
+}
+
+// swizzle of a P tile of 32 keys (4 chunks per row): the transpose read serves rows 0..3 and 8..11 (+4, +16) together, and
+// rows 8 apart share banks
+__device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1); }
+
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
+                                                                   int causal, int nkb, int64_t total_wg, int64_t per_xcd)
+{
+    constexpr int XC = D / 8, XT = N_STEP * D, PCH = N_ROWS / 8, XR = XT / 8 / 64, PT = N_STEP * N_ROWS, PR = PT / 8 / 64, DB = D / 16;
+    __shared__ __align__(16) T x_a_all[4 * XT];
+    __shared__ __align__(16) T x_b_all[4 * XT];
+    __shared__ __align__(16) T p_a_all[4 * PT];
+    __shared__ __align__(16) T p_b_all[4 * PT];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    T *const x_a = x_a_all + wave * XT;
+    T *const x_b = x_b_all + wave * XT;
+    T *const p_a = p_a_all + wave * PT;
+    T *const p_b = p_b_all + wave * PT;
+    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (lid >= total_wg) return;
+    const int64_t bh = lid / nkb;
+    const int k0 = (int)(lid % nkb) * N_ROWS;   // under the causal rule the first keys have the most query rows
+    const T *Pp = P + bh * (int64_t)S * S;
+    const T *Xp = X + bh * (int64_t)S * D;
+    T *Op = O + bh * (int64_t)S * D;
+    auto issue = [&](int j, T *xdst, T *pdst) {   // rows past the sequence re-read the last row, keys past it the first chunk
+#pragma unroll
+        for (int r = 0; r < XR; ++r) {
+            const int slot = r * 64 + lane, row = slot / XC, c = (slot % XC) ^ v_swizzle<D>(row);
+            int pr = j * N_STEP + row;
+            pr = pr >= S ? S - 1 : pr;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + (int64_t)pr * D + c * 8), (lds_void_t *)(xdst + r * 64 * 8), 16, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < PR; ++r) {
+            const int slot = r * 64 + lane, row = slot / PCH;
+            int c = (slot % PCH) ^ p_swizzle(row);
+            if (k0 + c * 8 >= S) c = 0;
+            int pr = j * N_STEP + row;
+            pr = pr >= S ? S - 1 : pr;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Pp + (int64_t)pr * S + k0 + c * 8), (lds_void_t *)(pdst + r * 64 * 8), 16, 0, 0);
+        }
+    };
+    auto read_tr = [&](const T *tile, int ld, int sw_a, int sw_b, int blk) {   // rows 8kg + t of a row-major block, column 16*blk + ln
+        const int row_a = kg * 8 + (ln >> 2), row_b = row_a + 4, ch = blk * 2 + ((ln & 3) >> 1), sub = (ln & 1) * 4;
+        const T *pa = tile + row_a * ld + ((ch ^ sw_a) * 8) + sub;
+        const T *pb = tile + row_b * ld + ((ch ^ sw_b) * 8) + sub;
+        struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pa),
+                                       __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pb)};
+        return __builtin_bit_cast(frag8<T>, both);
+    };
+    const int ra = kg * 8 + (ln >> 2);
+    const int xs_a = v_swizzle<D>(ra), xs_b = v_swizzle<D>(ra + 4), ps_a = p_swizzle(ra), ps_b = p_swizzle(ra + 4);
+    int krow[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) krow[rb] = k0 + rb * 16 + ln;
+    const int j_end = (S - 1) / N_STEP, j_start = causal ? k0 / N_STEP : 0;
+    const int jw = j_start + ((wave - j_start) & 3);
+    f32x4 oacc[RB][DB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[rb][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto step = [&](int j, const T *Xb, const T *Pb, T *Xn, T *Pn) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        if (j + 4 <= j_end) issue(j + 4, Xn, Pn);
+        const int pbase = j * N_STEP;
+        const bool edge = pbase + N_STEP > S || (causal && pbase < k0 + N_ROWS - 1);   // (wavefront-uniform)
+        frag8<T> pf[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            pf[rb] = read_tr(Pb, N_ROWS, ps_a, ps_b, rb);
+            if (edge) {   // query rows above the key (causal: P is undefined there) or past the sequence count as 0
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const int p = pbase + kg * 8 + t;
+                    if (p >= S || (causal && p < krow[rb])) pf[rb].v[t] = from_float<T>(0.0f);
+                }
+            }
+        }
+        frag8<T> xf[2];
+        xf[0] = read_tr(Xb, D, xs_a, xs_b, 0);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            if (db + 1 < DB) xf[(db + 1) & 1] = read_tr(Xb, D, xs_a, xs_b, db + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) mma16(oacc[rb][db], xf[db & 1], pf[rb]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (jw <= j_end) {
+        issue(jw, x_a, p_a);
+        for (int j = jw;;) {
+            step(j, x_a, p_a, x_b, p_b);
+            if ((j += 4) > j_end) break;
+            step(j, x_b, p_b, x_a, p_a);
+            if ((j += 4) > j_end) break;
+        }
+    }
+    narrow_reduce<T, D>(x_a_all, x_b_all, oacc, wave, lane, [&](int rb, int db, const f32x4 &sum) {
+        if (krow[rb] >= S) return;
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v]);
+        *reinterpret_cast<quad *>(Op + (int64_t)krow[rb] * D + db * 16 + kg * 4) = out;
+    });
+}
+
 // ---- the transposed product --------------------------------------------------------------------------------------
 // O[k, :] = sum over p of P[p, k] X[p, :], p >= k only when causal: the gradients that the two matrix products of the
 // attention leave on their right-hand operands (dV = P^T dO, dK = G^T Q), whose left factor is only defined - and only
@@ -396,13 +664,41 @@ __global__ __launch_bounds__(P_NT, P_OCC) void causal_ptx_kernel(const T *__rest
   }
 }
 
+// MTA_PV_SPLIT in the environment: 1 / 2 / 3 = always one group / two groups / the narrow kernels (comparison switch)
+int pv_force()
+{
+    static const int force = [] { const char *e = getenv("MTA_PV_SPLIT"); return e ? atoi(e) : 0; }();
+    return force;
+}
+// Whether a product whose wide grid has that many workgroups (pairs of 128-row blocks) runs on the narrow kernels.  The line
+// lies where the two meet (us, wide -> narrow; P V in the triangular layout / P^T X): B1 H16 D128 S512 16.6 -> 6.7 / 17.8 -> 6.6;
+// S1024 24.3 -> 12.8 / 25.3 -> 10.8; S2048 (128 workgroups) 48.8 -> 27.3 / 40.8 -> 24.5; S4096 (256) 95 -> 118 / 77 -> 102;
+// B4 S1024 (256) 33.4 -> 37.5 / 27.7 -> 34.0; D64, half the bytes per V row: B1 H32 S2048 (256) 45.3 -> 36.1 / 30.1 -> 30.9,
+// B1 H16 S4096 (256) 93 -> 88 / 61 -> 70.
+bool narrow_grid(int64_t wide_wg, int most)
+{
+    if (pv_force()) return pv_force() == 3;
+    return wide_wg <= most;
+}
+
 template <typename T, int D>
 int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st)
 {
-    const int nkb = (int)((S + T_KB - 1) / T_KB);
-    const int64_t total_wg = B * H * ((nkb + 1) / 2), per_xcd = (total_wg + 7) / 8;
+    int nkb = (int)((S + T_KB - 1) / T_KB);
+    int64_t total_wg = B * H * ((nkb + 1) / 2);
+    const bool narrow = narrow_grid(total_wg, 192);
+    if (narrow) {
+        nkb = (int)((S + N_ROWS - 1) / N_ROWS);
+        total_wg = B * H * nkb;
+    }
+    const int64_t per_xcd = (total_wg + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
     dim3 grid((unsigned)(per_xcd * 8));
+    if (narrow) {
+        auto kern = causal_ptx_narrow_kernel<T, D>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg, per_xcd);
+        return launch_status();
+    }
     auto kern = causal_ptx_kernel<T, D>;
     hipLaunchKernelGGL(kern, grid, dim3(P_NT), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg,
                        per_xcd);
@@ -413,13 +709,24 @@ template <typename T, int D>
 int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st,
            const int *band_lo = nullptr, int tri_gl = 0)
 {
-    const int nqb = (int)((S + P_BQ - 1) / P_BQ);
-    const int64_t total_wg = B * H * ((nqb + 1) / 2), per_xcd = (total_wg + 7) / 8;
+    int nqb = (int)((S + P_BQ - 1) / P_BQ);
+    int64_t total_wg = B * H * ((nqb + 1) / 2);
+    const bool narrow = narrow_grid(total_wg, D == 64 ? 256 : 192);
+    if (narrow) {
+        nqb = (int)((S + N_ROWS - 1) / N_ROWS);
+        total_wg = B * H * nqb;
+    }
+    const int64_t per_xcd = (total_wg + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
     dim3 grid((unsigned)(per_xcd * 8));
+    if (narrow) {
+        auto kern = causal_pv_narrow_kernel<T, D>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb, total_wg, per_xcd,
+                           band_lo, (int)H, tri_gl);
+        return launch_status();
+    }
     // a grid of at most one workgroup per CU runs the two-group instance (key blocks split between them)
-    static const int force = [] { const char *e = getenv("MTA_PV_SPLIT"); return e ? atoi(e) : 0; }();  // 1 / 2: test switch
-    const bool split = force ? force == 2 : total_wg <= device_cu_count();
+    const bool split = pv_force() ? pv_force() == 2 : total_wg <= device_cu_count();
     if (split) {
         auto kern = causal_pv_kernel<T, D, 2>;
         hipLaunchKernelGGL(kern, grid, dim3(P_NT * 2), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,

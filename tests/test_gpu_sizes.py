@@ -48,3 +48,25 @@ def test_qk_conv_kernel_sizes(pkg, dtype, r, sk):
         got = pkg.ops.qk_conv(q.cuda(), k.cuda(), w.cuda(), True, scale).cpu()
         ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
         torch.testing.assert_close(got.float(), want.float(), rtol=2 * ulp, atol=2e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_narrow_products(pkg, d, dtype):
+    """P V and P^T X on the narrow kernels (small grids): one row, edges of the 32-row blocks and of the steps that the four
+    wavefronts share, NaN above the diagonal.  Against the fp32 product of the same 16-bit values; what differs is the order
+    of at most 264 fp32 sums and one rounding of a result of magnitude at most sqrt(264)."""
+    g = torch.Generator().manual_seed(11)
+    for s in (8, 32, 40, 136, 264):
+        print(f"narrow products {dtype} d={d} s={s}", flush=True)
+        p = torch.randn(2, 3, s, s, generator=g).to(dtype)
+        x = torch.randn(2, 3, s, d, generator=g).to(dtype)
+        low = torch.tril(torch.ones(s, s, dtype=torch.bool))
+        poisoned = p.masked_fill(~low, float("nan")).cuda()
+        lower = p.float().masked_fill(~low, 0.0)
+        ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        for got, want in ((pkg.ops.causal_pv(poisoned, x.cuda(), True), lower @ x.float()),
+                          (pkg.ops.causal_ptx(poisoned, x.cuda(), True), lower.transpose(2, 3) @ x.float()),
+                          (pkg.ops.causal_pv(p.cuda(), x.cuda(), False), p.float() @ x.float()),
+                          (pkg.ops.causal_ptx(p.cuda(), x.cuda(), False), p.float().transpose(2, 3) @ x.float())):
+            torch.testing.assert_close(got.float().cpu(), want, rtol=ulp * 1.01, atol=1e-4)
