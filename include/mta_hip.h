@@ -311,6 +311,12 @@ int mta_conv2d_bwd_weight(const void *x, const void *dy, void *dw, void *workspa
                           int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, int causal, int io_dtype,
                           void *stream);
 
+/* The same with the result times `scale`, rounded once to w_dtype: dw is (C,R,S) of that dtype (the gradient an optimizer
+ * takes for a kernel of that dtype, without an elementwise pass over the fp32 one). */
+int mta_conv2d_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
+                             int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale,
+                             int io_dtype, int w_dtype, void *stream);
+
 /* mta_conv2d_bwd_weight for callers that cannot allocate device memory or pass a workspace (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same kernels
  * and same result; the partial sums live in a 1 MiB array that the library holds statically on each device it runs
@@ -331,6 +337,10 @@ int mta_headmix_bwd_input(const void *dy, const void *w, void *dx, int64_t N, in
 int64_t mta_headmix_bwd_weight_workspace(int64_t N, int64_t C, int64_t P, int64_t Q);
 int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
                            int64_t N, int64_t C, int64_t P, int64_t Q, int causal, int io_dtype, void *stream);
+/* The same rounded once to w_dtype; group_size > 0: 0 outside the diagonal blocks of that size (dw of a weight that is
+ * block diagonal by construction). */
+int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                              int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream);
 
 /* Structure of the small MTA parameters, evaluated on the device (one workgroup, a few microseconds).  The
  * reference has no counterpart: its glue (mta_attention_triton.py:69-89) always runs every stage.  The glue

@@ -7,11 +7,14 @@
 // partial matrix per workgroup in a scratch buffer, a second kernel adds the partials in a fixed order); the
 // reference accumulates with fp32 tl.dot and fp64 atomics (triton_linear_head.py:193-278).
 //
-// 16-bit tensors with C = 16 or 32 take the matrix cores: A = dY (rows = output heads), B = X (columns = input heads),
-// 32 positions per v_mfma_f32_16x16x32.  Which position feeds which contraction slot is free as long as both
-// operands agree; product t of a 128-position chunk takes positions 32t..32t+31, lane (head r, group g) the eight from
-// 32t + 8g on: a wavefront's load instruction covers 64 contiguous bytes of each of 16 heads.
-// Everything else (fp32, other head counts, rows that are not a multiple of 8 keys) takes a generic LDS kernel.
+// Up to 32 heads take the matrix cores: A = dY (rows = output heads), B = X (columns = input heads), positions as the
+// contraction index (v_mfma_f32_16x16x32 for 16-bit data, v_mfma_f32_16x16x4f32 - exact fp32 products, fp32 sums - for
+// fp32).  Which position feeds which contraction slot is free as long as both operands agree: a lane (row r, group g) loads
+// 16 contiguous bytes of a head's row and feeds them as they lie, so that a load instruction covers 64 contiguous bytes per
+// row.  With at most 8 (4) heads the 16 operand rows are two (four) sets of the heads at different positions; the blocks of
+// the product in which the sets meet themselves are the result, added up at the end, the others are dropped.  HBM-bound:
+// B1 H32 S1024 fp32 422 -> @FP32@ us against the generic kernel (one thread per pair of heads over an LDS tile), B1 H8 S256
+// bf16 31 -> @H8@ us.  More heads take that kernel.
 #include "common.hpp"
 #include "mfma.hpp"
 
@@ -19,60 +22,92 @@ namespace {
 using namespace mta;
 
 constexpr int NT = 256;
-// positions per wavefront step of the MFMA kernel: 512 contiguous bytes of every head's row with 16 heads, 256 with 32
-// (registers)
-template <int NB> constexpr int chunk_of() { return NB == 1 ? 256 : 128; }
-
 // Rows are visited in an order that interleaves short and long ones (0, P-1, 1, P-2, ...), so that under the causal
 // mask a pair of consecutive rows always carries P+1 positions.
 __device__ __forceinline__ int interleaved_row(int j, int P) { return (j & 1) ? P - 1 - (j >> 1) : (j >> 1); }
 
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-// One 128-position chunk of one query row: where it starts and where the row's attended positions end.
+// One chunk of one query row: where it starts and where the row's attended positions end.
 struct hm_unit {
     int64_t rowbase;
     int q0, last;
 };
 
-// The chunk's operands of a lane: for product t the eight positions from q0 + 32t + 8g on, of head 16a + r.
-template <int NB> struct hm_operands {
-    u4 dy[NB][chunk_of<NB>() / 32], x[NB][chunk_of<NB>() / 32];
+// How a wavefront reads a chunk of T x heads.  NB blocks of 16 operand rows; SETS sets of 16/SETS heads each per block (one
+// block if more than one set); TT products (16 bit) or groups of four products (fp32) per chunk.
+template <typename T, int NB, int SETS> struct hm_shape {
+    static_assert(SETS == 1 || NB == 1, "sets of heads within one block");
+    static constexpr int V = vec_of<T>::n;             // positions per load
+    static constexpr int TT = (NB == 1 && SETS == 1 && V == 8) ? 8 : 4;
+    static constexpr int STEP = 4 * V * SETS;          // positions per load instruction (and head)
+    static constexpr int CHUNK = STEP * TT;            // positions per chunk
+    static constexpr int HEADS = SETS == 1 ? 16 * NB : 16 / SETS;
 };
 
-template <typename T, int NB>
-__device__ __forceinline__ void hm_load(hm_operands<NB> &o, const T *x, const T *dy, const hm_unit &u, int64_t plane, int r,
-                                        int g)
+// The chunk's operands of a lane: load t the V positions from q0 + STEP*t + V*(g + 4*set) on, of head 16a + (r % heads).
+template <typename T, int NB, int SETS> struct hm_operands {
+    u4 dy[NB][hm_shape<T, NB, SETS>::TT], x[NB][hm_shape<T, NB, SETS>::TT];
+};
+
+// 16 bytes from an address that is aligned to an element only; `total`: elements of the tensor (nothing beyond is read)
+template <typename T> __device__ __forceinline__ u4 load_unaligned(const T *base, int64_t at, int64_t total)
 {
-    const int q = u.q0 + 8 * g;
-    // every load is unconditional: a vector wholly beyond `last` re-reads the row start and is zeroed before use
+    constexpr int V = vec_of<T>::n;
+    u4 v = {0u, 0u, 0u, 0u};
+    if (at + V <= total) {
+        __builtin_memcpy(&v, base + at, 16);
+    } else {
+        T e[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) e[i] = at + i < total ? base[at + i] : from_float<T>(0.0f);
+        __builtin_memcpy(&v, e, 16);
+    }
+    return v;
+}
+
+template <typename T, int NB, int SETS, bool ALIGNED>
+__device__ __forceinline__ void hm_load(hm_operands<T, NB, SETS> &o, const T *x, const T *dy, const hm_unit &u, int64_t plane, int C,
+                                        int r, int g, int64_t total)
+{
+    using G = hm_shape<T, NB, SETS>;
+    const int q = u.q0 + G::V * (g + 4 * (r / (16 / SETS)));
+    // every load is unconditional: a vector wholly beyond `last` re-reads the row start and is zeroed before use; a row of
+    // the operands without a head repeats the last head's (what it leads to is dropped)
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
+        const int h = a * 16 + r % (16 / SETS), hc = h < C ? h : C - 1;
+        const int64_t at = u.rowbase + hc * plane;
+        auto fetch = [&](const T *p, int t) -> u4 {
+            const int qq = (q + G::STEP * t <= u.last) ? q + G::STEP * t : 0;
+            if constexpr (ALIGNED) return *reinterpret_cast<const u4 *>(p + at + qq);
+            else return load_unaligned<T>(p, at + qq, total);
+        };
 #pragma unroll
-        for (int t = 0; t < chunk_of<NB>() / 32; ++t) {
-            const int qq = (q + 32 * t <= u.last) ? q + 32 * t : 0;
-            o.dy[a][t] = *reinterpret_cast<const u4 *>(dy + u.rowbase + (int64_t)(a * 16 + r) * plane + qq);
-        }
+        for (int t = 0; t < G::TT; ++t) o.dy[a][t] = fetch(dy, t);
 #pragma unroll
-        for (int t = 0; t < chunk_of<NB>() / 32; ++t) {
-            const int qq = (q + 32 * t <= u.last) ? q + 32 * t : 0;
-            o.x[a][t] = *reinterpret_cast<const u4 *>(x + u.rowbase + (int64_t)(a * 16 + r) * plane + qq);
-        }
+        for (int t = 0; t < G::TT; ++t) o.x[a][t] = fetch(x, t);
     }
 }
 
-template <typename T, int NB>
-__device__ __forceinline__ void hm_consume(f32x4 (&acc)[NB][NB], hm_operands<NB> &o, const hm_unit &u, int g)
+template <typename T, int NB, int SETS>
+__device__ __forceinline__ void hm_consume(f32x4 (&acc)[NB][NB], hm_operands<T, NB, SETS> &o, const hm_unit &u, int r, int g)
 {
-    if (u.q0 + chunk_of<NB>() - 1 > u.last) {  // the chunk straddles the end of the row: zero what lies beyond it, in both
-                                      // operands (what x holds there need not even be finite)
-        const int q = u.q0 + 8 * g;
+    using G = hm_shape<T, NB, SETS>;
+    if (u.q0 + G::CHUNK - 1 > u.last) {  // the chunk straddles the end of the row: zero what lies beyond it, in both operands
+                                         // (what x holds there need not even be finite)
+        const int q = u.q0 + G::V * (g + 4 * (r / (16 / SETS)));
 #pragma unroll
-        for (int t = 0; t < chunk_of<NB>() / 32; ++t)
+        for (int t = 0; t < G::TT; ++t)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int e = q + 32 * t + 2 * v;
-                const unsigned keep = (e <= u.last ? 0x0000ffffu : 0u) | (e + 1 <= u.last ? 0xffff0000u : 0u);
+                unsigned keep;
+                if constexpr (G::V == 8) {
+                    const int e = q + G::STEP * t + 2 * v;
+                    keep = (e <= u.last ? 0x0000ffffu : 0u) | (e + 1 <= u.last ? 0xffff0000u : 0u);
+                } else {
+                    keep = q + G::STEP * t + v <= u.last ? 0xffffffffu : 0u;
+                }
 #pragma unroll
                 for (int a = 0; a < NB; ++a) {
                     o.dy[a][t][v] &= keep;
@@ -81,22 +116,30 @@ __device__ __forceinline__ void hm_consume(f32x4 (&acc)[NB][NB], hm_operands<NB>
             }
     }
 #pragma unroll
-    for (int t = 0; t < chunk_of<NB>() / 32; ++t)
+    for (int t = 0; t < G::TT; ++t)
 #pragma unroll
         for (int a = 0; a < NB; ++a)
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-                mma16(acc[a][b], __builtin_bit_cast(frag8<T>, o.dy[a][t]), __builtin_bit_cast(frag8<T>, o.x[b][t]));
+            for (int b = 0; b < NB; ++b) {
+                if constexpr (G::V == 8) {
+                    mma16(acc[a][b], __builtin_bit_cast(frag8<T>, o.dy[a][t]), __builtin_bit_cast(frag8<T>, o.x[b][t]));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(o.dy[a][t][v]), __uint_as_float(o.x[b][t][v]), acc[a][b], 0, 0, 0);
+                }
+            }
 }
 
-template <typename T, int NB>  // NB = C / 16
-__global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restrict__ x, const T *__restrict__ dy,
-                                                              float *__restrict__ partial, int N, int P, int Q, int causal)
+template <typename T, int NB, int SETS, bool ALIGNED>
+__global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restrict__ x, const T *__restrict__ dy, float *__restrict__ partial,
+                                                              int N, int C, int P, int Q, int causal)
 {
-    constexpr int C = 16 * NB;
-    __shared__ float red[NT / 64][C * C];
+    using G = hm_shape<T, NB, SETS>;
+    constexpr int LD = 16 * NB;
+    __shared__ float red[NT / 64][LD * LD];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int64_t plane = (int64_t)P * Q;
+    const int64_t plane = (int64_t)P * Q, total = (int64_t)N * C * plane;
     f32x4 acc[NB][NB];
 #pragma unroll
     for (int a = 0; a < NB; ++a)
@@ -104,7 +147,7 @@ __global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restric
         for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     const int64_t rows = (int64_t)N * P;
-    const int64_t nwaves = (int64_t)gridDim.x * (NT / 64), wid = (int64_t)blockIdx.x * (NT / 64) + wave;
+    const int64_t nwaves = (int64_t)gridDim.x * (NT / 64), wid = (int64_t)wave * gridDim.x + blockIdx.x;
     // A wavefront takes pairs of rows (2k, 2k+1) of the interleaved order, k = wid, wid + nwaves, ...; j counts its
     // rows.  The chunks of all its rows form one sequence, and the loads of a chunk are issued before the products of
     // the chunk ahead of it (two operand sets take turns).  (Four wavefronts sharing a row chunk by chunk measured
@@ -121,41 +164,44 @@ __global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restric
         return true;
     };
     auto advance = [&](const hm_unit &u) {
-        q0 += chunk_of<NB>();
+        q0 += G::CHUNK;
         if (q0 > u.last) {
             q0 = 0;
             ++j;
         }
     };
     hm_unit ua, ub;
-    hm_operands<NB> oa, ob;
+    hm_operands<T, NB, SETS> oa, ob;
     bool ha = unit_at(ua);
-    if (ha) hm_load<T, NB>(oa, x, dy, ua, plane, r, g);
+    if (ha) hm_load<T, NB, SETS, ALIGNED>(oa, x, dy, ua, plane, C, r, g, total);
     while (ha) {
         advance(ua);
         const bool hb = unit_at(ub);
         if (!hb) ub = ua;  // nothing follows: fetch the same chunk again, so that the loads in flight never depend on a branch
-        hm_load<T, NB>(ob, x, dy, ub, plane, r, g);
-        hm_consume<T, NB>(acc, oa, ua, g);
+        hm_load<T, NB, SETS, ALIGNED>(ob, x, dy, ub, plane, C, r, g, total);
+        hm_consume<T, NB, SETS>(acc, oa, ua, r, g);
         if (!hb) break;
         advance(ub);
         ha = unit_at(ua);
         if (!ha) ua = ub;
-        hm_load<T, NB>(oa, x, dy, ua, plane, r, g);
-        hm_consume<T, NB>(acc, ob, ub, g);
+        hm_load<T, NB, SETS, ALIGNED>(oa, x, dy, ua, plane, C, r, g, total);
+        hm_consume<T, NB, SETS>(acc, ob, ub, r, g);
     }
-    // acc[a][b][v] = dw[16a + 4g + v][16b + r]
+    // acc[a][b][v] = product of operand rows 16a + 4g + v (dY) and 16b + r (X)
 #pragma unroll
     for (int a = 0; a < NB; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) red[wave][(a * 16 + 4 * g + v) * C + b * 16 + r] = acc[a][b][v];
+            for (int v = 0; v < 4; ++v) red[wave][(a * 16 + 4 * g + v) * LD + b * 16 + r] = acc[a][b][v];
     __syncthreads();
     for (int e = threadIdx.x; e < C * C; e += NT) {
+        const int o = e / C, i = e % C;
         float s = 0.0f;
 #pragma unroll
-        for (int wv = 0; wv < NT / 64; ++wv) s += red[wv][e];
+        for (int wv = 0; wv < NT / 64; ++wv)
+#pragma unroll
+            for (int k = 0; k < SETS; ++k) s += red[wv][(k * (LD / SETS) + o) * LD + k * (LD / SETS) + i];
         partial[(int64_t)blockIdx.x * (C * C) + e] = s;
     }
 }
@@ -206,11 +252,12 @@ __global__ __launch_bounds__(NT) void headmix_bwd_weight_any(const T *__restrict
     for (int pair = tid; pair < CC; pair += NT) partial[(int64_t)blockIdx.x * CC + pair] = sums[pair];
 }
 
-// dw[e] = sum of the partial matrices' entries e, in a fixed order: 64 entries per workgroup, the partial matrices dealt
+// dw[e] = sum of the partial matrices' entries e, in the weight's dtype (group > 0: 0 outside the diagonal blocks), in a fixed order: 64 entries per workgroup, the partial matrices dealt
 // to 16 wavefronts (each adds its share in index order), the 16 sums added in wavefront order
 constexpr int RED_SLICES = 16;
 __global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *__restrict__ partial,
-                                                                   float *__restrict__ dw, int CC, int nparts)
+                                                                   void *__restrict__ dw, int CC, int nparts, int C, int group,
+                                                                   int out_dtype)
 {
     __shared__ float red[RED_SLICES][64];
     const int le = threadIdx.x & 63, sl = threadIdx.x >> 6;
@@ -226,7 +273,10 @@ __global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *
         float t = 0.0f;
 #pragma unroll
         for (int k = 0; k < RED_SLICES; ++k) t += red[k][le];
-        dw[e] = t;
+        if (group > 0 && e / C / group != e % C / group) t = 0.0f;
+        if (out_dtype == MTA_F32) ((float *)dw)[e] = t;
+        else if (out_dtype == MTA_BF16) ((bf16_t *)dw)[e] = from_float<bf16_t>(t);
+        else ((f16_t *)dw)[e] = from_float<f16_t>(t);
     }
 }
 
@@ -250,47 +300,61 @@ extern "C" int64_t mta_headmix_bwd_weight_workspace(int64_t N, int64_t C, int64_
     return (int64_t)num_blocks(N, C, P, Q) * C * C * (int64_t)sizeof(float);
 }
 
-extern "C" int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
-                                      int64_t N, int64_t C, int64_t P, int64_t Q, int causal, int io_dtype, void *stream)
+namespace {
+template <typename T>
+int launch_partials(const T *x, const T *dy, float *partial, int nb, int N, int C, int P, int Q, int causal, hipStream_t st)
+{
+    if (C <= 32) {
+        const bool aligned = Q % vec_of<T>::n == 0 && aligned_to(x, 16) && aligned_to(dy, 16);
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(NT), 0, st, x, dy, partial, N, C, P, Q, causal); };
+#define MTA_HM_CASE(nb_, sets)                                                  \
+    aligned ? go(headmix_bwd_weight_mfma<T, nb_, sets, true>) : go(headmix_bwd_weight_mfma<T, nb_, sets, false>)
+        if (C <= 4) MTA_HM_CASE(1, 4);
+        else if (C <= 8) MTA_HM_CASE(1, 2);
+        else if (C <= 16) MTA_HM_CASE(1, 1);
+        else MTA_HM_CASE(2, 1);
+#undef MTA_HM_CASE
+        return launch_status();
+    }
+    const size_t lds = sizeof(float) * (2 * (size_t)C * (KC + 1) + (size_t)C * C);
+    auto kern = headmix_bwd_weight_any<T>;
+    if (lds > 48 * 1024) {  // per device, so set on every such launch (a cheap host-side call)
+        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(NT), lds, st, x, dy, partial, N, C, P, Q, causal);
+    return launch_status();
+}
+}  // namespace
+
+extern "C" int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                                         int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream)
 {
     if (!x || !dy || !dw || !workspace) return MTA_ERR_NULL;
-    if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
+    if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
     if (N <= 0 || C <= 0 || P <= 0 || Q <= 0 || P > (1 << 24) || Q > (1 << 24) || N * P > 0x7fffffffLL) return MTA_ERR_SHAPE;
     if (C > 128) return MTA_ERR_SHAPE;
-    if (!aligned_to(x, dtype_size(io_dtype)) || !aligned_to(dy, dtype_size(io_dtype)) || !aligned_to(dw, 4) ||
+    if (group_size < 0 || (group_size > 0 && C % group_size != 0)) return MTA_ERR_GROUP;
+    if (!aligned_to(x, dtype_size(io_dtype)) || !aligned_to(dy, dtype_size(io_dtype)) || !aligned_to(dw, dtype_size(w_dtype)) ||
         !aligned_to(workspace, 16))
         return MTA_ERR_ALIGN;
     const int nb = num_blocks(N, C, P, Q);
     if (workspace_bytes < (int64_t)nb * C * C * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
     float *partial = (float *)workspace;
-    const bool mfma_ok = io_dtype != MTA_F32 && (C == 16 || C == 32) && Q % 8 == 0 && aligned_to(x, 16) && aligned_to(dy, 16);
+    int rc = MTA_OK;
     MTA_DISPATCH_IO(io_dtype, {
-        if constexpr (sizeof(io_t) == 2) {
-            if (mfma_ok) {
-                if (C == 16)
-                    hipLaunchKernelGGL((headmix_bwd_weight_mfma<io_t, 1>), dim3(nb), dim3(NT), 0, st, (const io_t *)x,
-                                       (const io_t *)dy, partial, (int)N, (int)P, (int)Q, causal);
-                else
-                    hipLaunchKernelGGL((headmix_bwd_weight_mfma<io_t, 2>), dim3(nb), dim3(NT), 0, st, (const io_t *)x,
-                                       (const io_t *)dy, partial, (int)N, (int)P, (int)Q, causal);
-            }
-        }
-        if (!(sizeof(io_t) == 2 && mfma_ok)) {
-            const size_t lds = sizeof(float) * (2 * (size_t)C * (KC + 1) + (size_t)C * C);
-            auto kern = headmix_bwd_weight_any<io_t>;
-            if (lds > 48 * 1024) {  // per device, so set on every such launch (a cheap host-side call)
-                hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                if (e != hipSuccess) return (int)e;
-            }
-            hipLaunchKernelGGL(kern, dim3(nb), dim3(NT), lds, st, (const io_t *)x,
-                               (const io_t *)dy, partial, (int)N, (int)C, (int)P, (int)Q, causal);
-        }
+        rc = launch_partials<io_t>((const io_t *)x, (const io_t *)dy, partial, nb, (int)N, (int)C, (int)P, (int)Q, causal, st);
     });
-    int rc = launch_status();
     if (rc != MTA_OK) return rc;
     const int CC = (int)(C * C);
-    hipLaunchKernelGGL(reduce_partials, dim3((unsigned)((CC + 63) / 64)), dim3(64 * RED_SLICES), 0, st, partial, (float *)dw,
-                       CC, nb);
+    hipLaunchKernelGGL(reduce_partials, dim3((unsigned)((CC + 63) / 64)), dim3(64 * RED_SLICES), 0, st, partial, dw, CC, nb, (int)C,
+                       group_size, w_dtype);
     return launch_status();
+}
+
+extern "C" int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
+                                      int64_t N, int64_t C, int64_t P, int64_t Q, int causal, int io_dtype, void *stream)
+{
+    return mta_headmix_bwd_weight_as(x, dy, dw, workspace, workspace_bytes, N, C, P, Q, 0, causal, io_dtype, MTA_F32, stream);
 }

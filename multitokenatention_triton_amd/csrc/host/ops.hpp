@@ -91,13 +91,13 @@ inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tenso
     TORCH_CHECK_VALUE(x.sizes() == dy.sizes() && x.scalar_type() == dy.scalar_type(), "input and grad_output must share shape and dtype");
     const int64_t n = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3);
     const int r = (int)like.size(1), s = (int)like.size(2);
-    Tensor dw = at::empty({c, r, s}, x.options().dtype(at::kFloat));
+    Tensor dw = at::empty({c, r, s}, like.options());
     const int64_t bytes = std::max<int64_t>(mta_conv2d_bwd_weight_workspace(n, c, h, w, r, s), 16);
     Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
-    check(mta_conv2d_bwd_weight(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, h, w, r, s, causal, code(x, "input"), stream_of(x)),
+    check(mta_conv2d_bwd_weight_as(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, h, w, r, s, causal, (float)scale, code(x, "input"),
+                                   code(like, "weight"), stream_of(x)),
           "mta_conv2d_bwd_weight");
-    if (scale != 1.0) dw.mul_(scale);
-    return dw.to(like.scalar_type());
+    return dw;
 }
 
 inline Tensor headmix(const Tensor &x_, const Tensor &w_, bool causal, double fill, int64_t group, bool fill_upper)
@@ -131,14 +131,11 @@ inline Tensor headmix_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tens
     const int64_t n = x.size(0), c = x.size(1), p = x.size(2), q = x.size(3);
     const int64_t bytes = mta_headmix_bwd_weight_workspace(n, c, p, q);
     TORCH_CHECK_VALUE(bytes > 0, "mta_headmix_bwd_weight: no kernel for ", c, " heads (at most 128)");
-    Tensor dw = at::empty({c, c}, x.options().dtype(at::kFloat)), ws = at::empty({std::max<int64_t>(bytes, 16)}, x.options().dtype(at::kByte));
-    check(mta_headmix_bwd_weight(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, causal, code(x, "input"), stream_of(x)),
+    Tensor dw = at::empty({c, c}, like.options()), ws = at::empty({std::max<int64_t>(bytes, 16)}, x.options().dtype(at::kByte));
+    check(mta_headmix_bwd_weight_as(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, (int)group, causal, code(x, "input"),
+                                    code(like, "weight"), stream_of(x)),
           "mta_headmix_bwd_weight");
-    if (group > 0) {
-        const Tensor blk = at::arange(c, x.options().dtype(at::kLong)).floor_divide(group);
-        dw.mul_(blk.unsqueeze(1).eq(blk.unsqueeze(0)));
-    }
-    return dw.to(like.scalar_type());
+    return dw;
 }
 
 inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTensor &w2, bool causal, int64_t group, bool fill_upper,

@@ -70,3 +70,23 @@ def test_narrow_products(pkg, d, dtype):
                           (pkg.ops.causal_pv(p.cuda(), x.cuda(), False), p.float() @ x.float()),
                           (pkg.ops.causal_ptx(p.cuda(), x.cuda(), False), p.float().transpose(2, 3) @ x.float())):
             torch.testing.assert_close(got.float().cpu(), want, rtol=ulp * 1.01, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c", [3, 5, 12, 17, 32])
+def test_headmix_weight_gradient_head_counts(pkg, c, dtype):
+    """dW on the matrix cores for head counts that do not fill the operand rows (sets of 4 or 8 heads, blocks of 16), rows of
+    whole 16-byte vectors and ragged ones (whose last vectors reach the end of the tensor), NaN above the diagonal.  Against
+    the double-precision sum of the same values: fp32 sums of n products are off by at most n*2^-24 of the sum of their
+    magnitudes in the worst order, far less in this one; sqrt(n)*2^-22 covers it."""
+    g = torch.Generator().manual_seed(5)
+    for p, q, causal in ((8, 8, True), (33, 65, False), (97, 97, True), (200, 200, True), (64, 1032, False)):
+        print(f"headmix dW c={c} {p}x{q} causal={causal} {dtype}", flush=True)
+        x, dy = (torch.randn(2, c, p, q, generator=g).to(dtype) for _ in range(2))
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        xd, dyd = (t.double().masked_fill(~keep, 0.0) for t in (x, dy))
+        want = torch.einsum("nopq,nipq->oi", dyd, xd)
+        size = torch.einsum("nopq,nipq->oi", dyd.abs(), xd.abs())
+        got = pkg.ops.headmix_bwd_weight(x.masked_fill(~keep, float("nan")).cuda(), dy.masked_fill(~keep, float("nan")).cuda(), causal)
+        bound = (2 * p * q) ** 0.5 * 2.0 ** -22 * size
+        assert ((got.cpu().double() - want).abs() <= bound).all()
