@@ -457,7 +457,7 @@ __global__ __launch_bounds__(NT) void conv2d_bwd_weight_any(const T *__restrict_
 
 // dw[c][t] = scale * sum over the channel's partial kernels, in the weight's dtype: 64 entries per workgroup, the partial
 // kernels dealt to 16 wavefronts (each adds its share in index order), the 16 sums added in wavefront order.  (A thread per
-// entry walking its 64 partial kernels alone took 11 us at 16 channels, 6x11; this takes @RED@.)
+// entry walking its 64 partial kernels alone took 11 us at 16 channels, 6x11; this takes 4.))
 constexpr int RED_SLICES = 16;
 __global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *__restrict__ partial, void *__restrict__ dw, int total,
                                                                    int RS, int bpc, float scale, int out_dtype)

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64 * DM_WAVES, 2) void headmix_dense_wide(const T *
     }
 }
 
-// The same for 16 heads: the contraction of a 16x16x16 product covers the 16 input heads; lane (ln, kg) fetches keys
+// The same for 16 heads (12: B1 S1024 bf16 47 -> 11 us against the kernel for any group): the contraction of a 16x16x16 product covers the 16 input heads; lane (ln, kg) fetches keys
 // 8ln .. 8ln+7 of the heads 4kg .. 4kg+3 (four 16-byte loads), forms the column of key 8ln + j with two byte permutes,
 // and after eight products holds keys 8ln .. 8ln+7 of the output heads 4kg + v.
 typedef short hm_s4 __attribute__((ext_vector_type(4)));
@@ -341,12 +341,12 @@ __device__ __forceinline__ f32x4 hm_mma16(f16_t, hm_u2 a, hm_u2 b)
                                                  f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
 
-template <typename T>
+template <typename T, int HG>
 __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__restrict__ x, const T *__restrict__ w,
                                                                T *__restrict__ y, int C, int P, int Q, int causal,
                                                                float fill, int wt, int qchunks)
 {
-    constexpr int HG = 16;  // heads mixed together
+    static_assert(HG == 12 || HG == 16, "whole groups of four heads");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 15, kg = lane >> 4;
     const int groups = C / HG;
     unsigned b = blockIdx.x;
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
     const int q0 = (qc * DM_WAVES + wave) * DM_KEYS;
     if (q0 >= Q) return;
     const int64_t plane = (int64_t)P * Q;
-    const int64_t base = (n * C + (int64_t)g * HG) * plane + (int64_t)p * Q;  // head g*16, row p, key 0
+    const int64_t base = (n * C + (int64_t)g * HG) * plane + (int64_t)p * Q;  // head g*HG, row p, key 0
     const int last = causal ? (p < Q - 1 ? p : Q - 1) : Q - 1;              // last key that is mixed
     const uint32_t fill2 = pack2<T>(fill, fill);
     typedef unsigned int u4 __attribute__((ext_vector_type(4)));
@@ -368,26 +368,30 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
         if (key < Q && causal != 2) {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                __builtin_nontemporal_store(fv, reinterpret_cast<u4 *>(y + base + (kg * 4 + t) * plane + key));
+                if (HG == 16 || kg * 4 < HG) __builtin_nontemporal_store(fv, reinterpret_cast<u4 *>(y + base + (kg * 4 + t) * plane + key));
         }
         return;
     }
 
-    const T *xp = x + base + (int64_t)(kg * 4) * plane + (key <= last ? key : 0);
+    // (HG = 12: the fourth lane group re-reads the first heads, its weights are 0 and it stores nothing)
+    const int kgc = kg * 4 < HG ? kg : 0;
+    const T *xp = x + base + (int64_t)(kgc * 4) * plane + (key <= last ? key : 0);
     u4 xv[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) xv[t] = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(xp + t * plane));
 
     // w fragment: lane (output head ln, group kg) holds w[o][4kg .. 4kg+3]
     hm_u2 wf;
+    const int lnc = ln < HG ? ln : 0;
     if (!wt) {
-        wf = *reinterpret_cast<const hm_u2 *>(w + (int64_t)(g * HG + ln) * C + g * HG + kg * 4);
+        wf = *reinterpret_cast<const hm_u2 *>(w + (int64_t)(g * HG + lnc) * C + g * HG + kgc * 4);
     } else {  // the transposed matrix: a column of w, gathered element by element (once per wavefront)
         struct alignas(8) quad { T v[4]; } col;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) col.v[t] = w[(int64_t)(g * HG + kg * 4 + t) * C + g * HG + ln];
+        for (int t = 0; t < 4; ++t) col.v[t] = w[(int64_t)(g * HG + kgc * 4 + t) * C + g * HG + lnc];
         wf = __builtin_bit_cast(hm_u2, col);
     }
+    if (HG < 16 && (kg * 4 >= HG || ln >= HG)) wf = hm_u2{0u, 0u};
 
     f32x4 acc[8];
 #pragma unroll
@@ -397,7 +401,7 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
                            __builtin_amdgcn_perm(xv[3][j >> 1], xv[2][j >> 1], sel)};  // heads 4kg .. 4kg+3 of key 8ln + j
         acc[j] = hm_mma16(T{}, wf, col);
     }
-    if (key >= Q || (causal == 2 && key > last)) return;
+    if (key >= Q || (causal == 2 && key > last) || kg * 4 >= HG) return;
     // acc[j][v]: output head 4kg + v, key 8ln + j
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -461,11 +465,12 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
         // 16 or 32 heads mixed densely, 16-bit data and weights of the same dtype: matrix cores
         // (MTA_HEADMIX_NO_MFMA=1 in the environment keeps the vector-ALU kernel, for comparisons)
         static const bool no_mfma = [] { const char *e = getenv("MTA_HEADMIX_NO_MFMA"); return e && e[0] == '1'; }();
-        if (G == 16 && !no_mfma && w_same_dtype && aligned_to(w, 8) && C % 4 == 0) {
+        if ((G == 16 || G == 12) && !no_mfma && w_same_dtype && aligned_to(w, 8) && C % 4 == 0) {
             const int qch = (int)((Q + DM_WAVES * DM_KEYS - 1) / (DM_WAVES * DM_KEYS));
-            const int64_t blocks = N * (C / 16) * P * qch;
+            const int64_t blocks = N * (C / G) * P * qch;
             if (blocks > 0x7fffffffLL) return MTA_ERR_SHAPE;
-            hipLaunchKernelGGL((headmix_dense16<T>), dim3((unsigned)blocks), dim3(64 * DM_WAVES), 0, st, (const T *)x,
+            auto kern = G == 16 ? headmix_dense16<T, 16> : headmix_dense16<T, 12>;
+            hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * DM_WAVES), 0, st, (const T *)x,
                                (const T *)w, (T *)y, (int)C, (int)P, (int)Q, causal, fill, wt, qch);
             return launch_status();
         }
@@ -504,6 +509,7 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
     MTA_HM_CASE(2)
     MTA_HM_CASE(4)
     MTA_HM_CASE(8)
+    MTA_HM_CASE(12)
     MTA_HM_CASE(16)
     MTA_HM_CASE(32)
 #undef MTA_HM_CASE

@@ -90,3 +90,23 @@ def test_headmix_weight_gradient_head_counts(pkg, c, dtype):
         got = pkg.ops.headmix_bwd_weight(x.masked_fill(~keep, float("nan")).cuda(), dy.masked_fill(~keep, float("nan")).cuda(), causal)
         bound = (2 * p * q) ** 0.5 * 2.0 ** -22 * size
         assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_headmix_twelve_heads(pkg, transposed, dtype):
+    """12 heads mixed densely, alone and as two groups of 24 heads, whole vectors and ragged rows, forward and input gradient;
+    one rounding of an fp32 sum of 12 products of magnitude at most 1.5 each (fp32: the order of that sum)."""
+    g = torch.Generator().manual_seed(6)
+    for c, group, p, q, causal in ((12, None, 40, 40, True), (12, None, 33, 1032, False), (24, 12, 72, 72, True), (12, None, 51, 51, True)):
+        print(f"headmix 12 heads c={c} {p}x{q} {dtype}", flush=True)
+        x = torch.randn(2, c, p, q, generator=g).to(dtype)
+        w = (O.block_diag_head_weight(c, 12, 0.3, g, dtype) if group else torch.eye(c) + 0.3 * torch.randn(c, c, generator=g)).to(dtype)
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        m = w.double().t() if transposed else w.double()
+        want = torch.einsum("oi,nipq->nopq", m, x.double().masked_fill(~keep, 0.0))
+        xd = x.masked_fill(~keep, float("nan")).cuda()
+        got = (pkg.ops.headmix_bwd_input(xd, w.cuda(), causal, group_size=group) if transposed
+               else pkg.ops.headmix(xd, w.cuda(), causal, 0.0, group_size=group))
+        ulp = {torch.float32: 2.0 ** -21, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+        torch.testing.assert_close(got.double().cpu(), want.masked_fill(~keep, 0.0), rtol=ulp, atol=1e-5)
