@@ -220,6 +220,10 @@ int mta_qk_conv_band_fwd(const void *q, const void *k, const void *w, const void
 int mta_causal_pv_fwd(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D,
                       int causal, int io_dtype, void *stream);
 
+/* mta_causal_pv_fwd with the result times `scale`, rounded once (the gradient of Q: dQ = scale * G K). */
+int mta_causal_pv_scaled_fwd(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
+                             float scale, int io_dtype, void *stream);
+
 /* The same under a band mask: first_visible is int32, (B,S), or NULL; P[b,h,p,k] must be 0 for k < first_visible[b,p]
  * (what mta_headmix_softmax_band_fwd leaves there), and the key blocks ahead of the first key any row of a block of 128
  * query rows sees are not read.  Requires causal when first_visible is given. */
@@ -288,6 +292,10 @@ int mta_headmix_softmax_tri_supported(int64_t C, int64_t S, int group_size, int 
 int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D,
                        int causal, int io_dtype, void *stream);
 
+/* mta_causal_ptx_fwd with the result times `scale`, rounded once (the gradient of K). */
+int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
+                              float scale, int io_dtype, void *stream);
+
 /* ---- backward of the two standalone operators -------------------------------------------------------------
  * Gradients flow through the same masks as the forward pass: with `causal`, entries of dy above the diagonal are
  * never read (the forward wrote a constant there) and gradients with respect to inputs above the diagonal are +0
@@ -341,6 +349,14 @@ int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *worksp
  * block diagonal by construction). */
 int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
                               int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream);
+/* y[i][b,h,p,:] = p < S_in and not hidden ? x[i][b,h,p,:] * scale[i] : 0 for i < count <= 3: rows of (B,H,S_in,D[i]) tensors
+ * into dense (B,H,S_out,D[i]) ones - padded with zero rows or cut -, x with the strides x_strides[3i .. 3i+2] (batch entry,
+ * head, row; elements; the last dimension dense).  hide[i] != 0: the rows with key_bias[b * bias_stride + p] = -inf (fp32)
+ * count as zeros, what the reference's masked scores see of a hidden key (mta_attention_triton.py:70-73).  The arrays are host
+ * memory, read before the call returns. */
+int mta_rows_copy(int count, const void *const *x, const int64_t *x_strides, void *const *y, const int64_t *D,
+                  const float *scale, const int *hide, const void *key_bias, int64_t bias_stride, int64_t B, int64_t H, int64_t S_in,
+                  int64_t S_out, int io_dtype, void *stream);
 
 /* Structure of the small MTA parameters, evaluated on the device (one workgroup, a few microseconds).  The
  * reference has no counterpart: its glue (mta_attention_triton.py:69-89) always runs every stage.  The glue

@@ -39,7 +39,7 @@ constexpr int P_KS = P_BK / 32;  // 32-key contraction steps per iteration
 template <typename T, int D, int SPLIT>
 __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_pv_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int nqb, int64_t total_wg,
-    int64_t per_xcd, const int *__restrict__ band_lo, int H, int tri_gl)
+    int64_t per_xcd, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
 {
     constexpr int CPR = D / 8;               // 16-byte chunks per V row
     constexpr int TILE = P_BK * D;           // elements per V block
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
         for (int db = 0; db < DB; ++db) {
             struct alignas(8) quad { T v[4]; } out;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[rb][db][v]);
+            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[rb][db][v] * scale);
             *reinterpret_cast<quad *>(Op + (int64_t)prow[rb] * D + db * 16 + kg * 4) = out;
         }
     }
@@ -277,7 +277,7 @@ __device__ __forceinline__ void narrow_reduce(T *a, T *b, const f32x4 (&oacc)[RB
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
                                                                   int causal, int nrb, int64_t total_wg, int64_t per_xcd,
-                                                                  const int *__restrict__ band_lo, int H, int tri_gl)
+                                                                  const int *__restrict__ band_lo, int H, int tri_gl, float scale)
 {
     constexpr int CPR = D / 8, TILE = N_STEP * D, ROUNDS = TILE / 8 / 64, DB = D / 16;
     __shared__ __align__(16) T v_a_all[4 * TILE];
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__res
         if (prow[rb] >= S) return;
         struct alignas(8) quad { T v[4]; } out;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v]);
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v] * scale);
         *reinterpret_cast<quad *>(Op + (int64_t)prow[rb] * D + db * 16 + kg * 4) = out;
     });
 }
@@ -406,7 +406,7 @@ __device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1);
 
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
-                                                                   int causal, int nkb, int64_t total_wg, int64_t per_xcd)
+                                                                   int causal, int nkb, int64_t total_wg, int64_t per_xcd, float scale)
 {
     constexpr int XC = D / 8, XT = N_STEP * D, PCH = N_ROWS / 8, XR = XT / 8 / 64, PT = N_STEP * N_ROWS, PR = PT / 8 / 64, DB = D / 16;
     __shared__ __align__(16) T x_a_all[4 * XT];
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
         if (krow[rb] >= S) return;
         struct alignas(8) quad { T v[4]; } out;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v]);
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v] * scale);
         *reinterpret_cast<quad *>(Op + (int64_t)krow[rb] * D + db * 16 + kg * 4) = out;
     });
 }
@@ -529,7 +529,7 @@ constexpr int T_KS = T_PB / 32;
 template <typename T, int D>
 __global__ __launch_bounds__(P_NT, P_OCC) void causal_ptx_kernel(const T *__restrict__ P, const T *__restrict__ X,
                                                                  T *__restrict__ O, int S, int causal, int nkb, int64_t total_wg,
-                                                                 int64_t per_xcd)
+                                                                 int64_t per_xcd, float scale)
 {
     constexpr int XT = T_PB * D, PT = T_PB * T_KB;  // elements per X block / P tile
     constexpr int XC = D / 8, PC = T_KB / 8;        // 16-byte chunks per row
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(P_NT, P_OCC) void causal_ptx_kernel(const T *__rest
         for (int db = 0; db < DB; ++db) {
             struct alignas(8) quad { T v[4]; } out;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[rb][db][v]);
+            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[rb][db][v] * scale);
             *reinterpret_cast<quad *>(Op + (int64_t)krow[rb] * D + db * 16 + kg * 4) = out;
         }
     }
@@ -682,7 +682,7 @@ bool narrow_grid(int64_t wide_wg, int most)
 }
 
 template <typename T, int D>
-int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st)
+int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, float scale, hipStream_t st)
 {
     int nkb = (int)((S + T_KB - 1) / T_KB);
     int64_t total_wg = B * H * ((nkb + 1) / 2);
@@ -696,18 +696,18 @@ int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_
     dim3 grid((unsigned)(per_xcd * 8));
     if (narrow) {
         auto kern = causal_ptx_narrow_kernel<T, D>;
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg, per_xcd);
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg, per_xcd, scale);
         return launch_status();
     }
     auto kern = causal_ptx_kernel<T, D>;
     hipLaunchKernelGGL(kern, grid, dim3(P_NT), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg,
-                       per_xcd);
+                       per_xcd, scale);
     return launch_status();
 }
 
 template <typename T, int D>
 int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st,
-           const int *band_lo = nullptr, int tri_gl = 0)
+           const int *band_lo = nullptr, int tri_gl = 0, float scale = 1.0f)
 {
     int nqb = (int)((S + P_BQ - 1) / P_BQ);
     int64_t total_wg = B * H * ((nqb + 1) / 2);
@@ -722,7 +722,7 @@ int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t 
     if (narrow) {
         auto kern = causal_pv_narrow_kernel<T, D>;
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb, total_wg, per_xcd,
-                           band_lo, (int)H, tri_gl);
+                           band_lo, (int)H, tri_gl, scale);
         return launch_status();
     }
     // a grid of at most one workgroup per CU runs the two-group instance (key blocks split between them)
@@ -730,20 +730,19 @@ int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t 
     if (split) {
         auto kern = causal_pv_kernel<T, D, 2>;
         hipLaunchKernelGGL(kern, grid, dim3(P_NT * 2), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
-                           total_wg, per_xcd, band_lo, (int)H, tri_gl);
+                           total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
     } else {
         auto kern = causal_pv_kernel<T, D, 1>;
         hipLaunchKernelGGL(kern, grid, dim3(P_NT), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
-                           total_wg, per_xcd, band_lo, (int)H, tri_gl);
+                           total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
     }
     return launch_status();
 }
 }  // namespace
 
-// first_visible (int32, (B,S); NULL = none): P[b,h,p,k] is 0 for k < first_visible[b,p] (what the softmax stage leaves
-// under a band mask); the key blocks ahead of a query block's first visible key are not read.  Implies causal.
-extern "C" int mta_causal_pv_band_fwd(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H,
-                                      int64_t S, int64_t D, int causal, int io_dtype, void *stream)
+namespace {
+int pv_entry(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
+             float scale, int io_dtype, void *stream)
 {
     if (!p || !v || !o) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
@@ -755,8 +754,23 @@ extern "C" int mta_causal_pv_band_fwd(const void *p, const void *v, const void *
     hipStream_t st = (hipStream_t)stream;
     const int *lo = (const int *)first_visible;
     if (io_dtype == MTA_BF16)
-        return D == 64 ? launch<bf16_t, 64>(p, v, o, B, H, S, causal, st, lo) : launch<bf16_t, 128>(p, v, o, B, H, S, causal, st, lo);
-    return D == 64 ? launch<f16_t, 64>(p, v, o, B, H, S, causal, st, lo) : launch<f16_t, 128>(p, v, o, B, H, S, causal, st, lo);
+        return D == 64 ? launch<bf16_t, 64>(p, v, o, B, H, S, causal, st, lo, 0, scale) : launch<bf16_t, 128>(p, v, o, B, H, S, causal, st, lo, 0, scale);
+    return D == 64 ? launch<f16_t, 64>(p, v, o, B, H, S, causal, st, lo, 0, scale) : launch<f16_t, 128>(p, v, o, B, H, S, causal, st, lo, 0, scale);
+}
+}  // namespace
+
+// first_visible (int32, (B,S); NULL = none): P[b,h,p,k] is 0 for k < first_visible[b,p] (what the softmax stage leaves
+// under a band mask); the key blocks ahead of a query block's first visible key are not read.  Implies causal.
+extern "C" int mta_causal_pv_band_fwd(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H,
+                                      int64_t S, int64_t D, int causal, int io_dtype, void *stream)
+{
+    return pv_entry(p, v, first_visible, o, B, H, S, D, causal, 1.0f, io_dtype, stream);
+}
+
+extern "C" int mta_causal_pv_scaled_fwd(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
+                                        float scale, int io_dtype, void *stream)
+{
+    return pv_entry(p, v, nullptr, o, B, H, S, D, causal, scale, io_dtype, stream);
 }
 
 // P in the triangular layout (see tri_rowoff in common.hpp), groups of `group` heads interleaved by rows; causal.
@@ -787,6 +801,12 @@ extern "C" int mta_causal_pv_fwd(const void *p, const void *v, void *o, int64_t 
 extern "C" int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D,
                                   int causal, int io_dtype, void *stream)
 {
+    return mta_causal_ptx_scaled_fwd(p, x, o, B, H, S, D, causal, 1.0f, io_dtype, stream);
+}
+
+extern "C" int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
+                                         float scale, int io_dtype, void *stream)
+{
     if (!p || !x || !o) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
     if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535) return MTA_ERR_SHAPE;
@@ -795,6 +815,6 @@ extern "C" int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t
     if (io_dtype == MTA_F32 || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (io_dtype == MTA_BF16)
-        return D == 64 ? launch_t<bf16_t, 64>(p, x, o, B, H, S, causal, st) : launch_t<bf16_t, 128>(p, x, o, B, H, S, causal, st);
-    return D == 64 ? launch_t<f16_t, 64>(p, x, o, B, H, S, causal, st) : launch_t<f16_t, 128>(p, x, o, B, H, S, causal, st);
+        return D == 64 ? launch_t<bf16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<bf16_t, 128>(p, x, o, B, H, S, causal, scale, st);
+    return D == 64 ? launch_t<f16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<f16_t, 128>(p, x, o, B, H, S, causal, scale, st);
 }

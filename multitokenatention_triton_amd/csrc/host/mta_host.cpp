@@ -52,11 +52,11 @@ struct Mark {
     }
 };
 
-// (B,H,S,D) seen as (B,S,H,D), without a view relation that autograd would track
-Tensor heads_last(const Tensor &o)
+// the first rows of (B,H,S,D) seen as (B,S,H,D), without a view relation that autograd would track
+Tensor heads_last(const Tensor &o, int64_t rows)
 {
     at::AutoDispatchBelowADInplaceOrView guard;
-    return o.transpose(1, 2);
+    return (rows == o.size(2) ? o : o.narrow(2, 0, rows)).transpose(1, 2);
 }
 
 // int32 (B,S): p + 1 for the rows p that see no key, 0 for the others (mta_band_zero_fwd then clears those rows)
@@ -66,10 +66,15 @@ Tensor empty_row_ends(const Tensor &empty_rows)
     return at::where(empty_rows, rows.unsqueeze(0), at::zeros({}, rows.options())).contiguous();
 }
 
-struct Structure {
-    bool pre_identity, post_conv_identity, post_identity;
-    int64_t pre_group, post_group;   // 0 = dense
-};
+// The length the score kernels work on.  They move score rows as 16-byte vectors; under the causal rule a length that is not
+// a multiple of 8 is padded with zero rows: only padding rows see the padding keys, so every result of a real row is what it
+// was (their gradients are zero: the padding rows of the incoming gradient are).  key_bias, first and empty_rows arrive
+// padded.
+int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool causal)
+{
+    const int64_t s = q.size(2);
+    return causal && s == k.size(2) && s == v.size(2) ? (s + 7) / 8 * 8 : s;
+}
 
 // ---- inference -------------------------------------------------------------------------------------------------------
 // The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
@@ -81,20 +86,25 @@ struct Structure {
 // leaves NaN in them, which the reference replaces by zeros ahead of its post-softmax conv
 // (mta_attention_triton.py:81) - here those rows of the probabilities are cleared ahead of a post-softmax conv that is not
 // the identity, and their rows of the output, where nothing else would, at the end.
-Tensor forward_inference(const Tensor &q, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
+Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
                          const Tensor &w_post, bool causal, bool pre_identity, int64_t pre_group, bool post_conv_identity, bool post_identity,
                          int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows, bool planes,
                          double dropout, const py::object &hook)
 {
     at::NoGradGuard no_grad;
-    const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
+    const c10::OptionalDeviceGuard guard(q_.is_cuda() ? std::optional<c10::Device>(q_.device()) : std::nullopt);
     const Mark mark{hook};
-    Tensor k = k_, v = v_;
-    if (key_bias) {
-        const Tensor hidden = key_bias->eq(-INFINITY).unsqueeze(1).unsqueeze(-1);
-        k = k.masked_fill(hidden, 0);
-        if (!post_conv_identity) v = v.masked_fill(hidden, 0);
+    const int64_t s_real = q_.size(2), s_pad = padded_length(q_, k_, v_, causal);
+    Tensor q = q_, k = k_, v = v_;
+    if (s_pad != s_real || key_bias) {
+        RowsCopy rows(s_pad, key_bias);
+        if (s_pad != s_real) q = rows.add(q_, false, 1.0);
+        k = rows.add(k_, true, 1.0);
+        if (s_pad != s_real || !post_conv_identity) v = rows.add(v_, !post_conv_identity, 1.0);
+        rows.run();
     }
+    // (what the padding rows hold is nobody's business)
+    auto result = [&](const Tensor &out) { return (s_pad == s_real ? out : out.narrow(2, 0, s_real)).transpose(1, 2); };
     const double scale = score_scale(q);
     const int64_t heads = w_pre.size(0), n_keys = k.size(-2);
     const OptTensor w1 = pre_identity ? OptTensor() : OptTensor(w_pre), w2 = post_identity ? OptTensor() : OptTensor(w_post);
@@ -120,7 +130,7 @@ Tensor forward_inference(const Tensor &q, const Tensor &k_, const Tensor &v_, co
         Tensor out = causal_pv_tri(scores, v, g_both, first);
         if (empty_rows) out.masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
         mark("end");
-        return out.transpose(1, 2);
+        return result(out);
     }
 
     Tensor scores;
@@ -195,7 +205,7 @@ Tensor forward_inference(const Tensor &q, const Tensor &k_, const Tensor &v_, co
     if (!out) out = at::matmul(scores, v);
     if (empty_rows) out->masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
     mark("end");
-    return out->transpose(1, 2);
+    return result(*out);
 }
 
 // ---- training ----------------------------------------------------------------------------------------------------------
@@ -220,7 +230,8 @@ struct TrainOptions {
     int64_t pre_group, post_group;   // 0 = dense (the weight gradient is then dense too)
     double dropout;
     OptTensor first;       // int32 (B,S), a band mask
-    OptTensor key_bias;    // fp32 (B,S); the caller has zeroed the K and V rows of the keys it hides
+    OptTensor key_bias;    // fp32 (B,S): added ahead of the softmax; the K and V rows of the keys it hides (-inf) count as zeros
+                           // and receive no gradient, as in the reference, whose masked_fill / where cut it
     OptTensor empty_rows;  // bool (B,S), the rows of the band that see no key: their probabilities are cleared
 };
 
@@ -228,11 +239,20 @@ struct TrainOptions {
 // nothing reads above the diagonal when causal (the kernels never do, in either direction), so nothing is written there,
 // except what goes into a library GEMM.
 struct MtaTraining : torch::autograd::Function<MtaTraining> {
-    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &conv_w,
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w,
                           const Tensor &w_pre, const Tensor &post_conv_w, const Tensor &w_post, const TrainOptions *opt, const Mark *mark_)
     {
         const TrainOptions &o = *opt;
         const Mark &mark = *mark_;
+        const int64_t s_real = q_.size(2), s_pad = padded_length(q_, k_, v_, o.causal);
+        Tensor q = q_, k = k_, v = v_;
+        if (s_pad != s_real || o.key_bias) {
+            RowsCopy rows(s_pad, o.key_bias);
+            if (s_pad != s_real) q = rows.add(q_, false, 1.0);
+            k = rows.add(k_, true, 1.0);
+            v = rows.add(v_, true, 1.0);
+            rows.run();
+        }
         const double scale = score_scale(q);
         const bool fill = !o.causal;
         Tensor raw, x;   // raw scores (kept where the first stage is two operators), conv result
@@ -246,7 +266,8 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         } else {
             TORCH_CHECK(!o.first, "the band mask needs the one-kernel first stage");
             mark("qk");
-            raw = at::matmul(q, k.transpose(2, 3));
+            const OptTensor lower_raw = o.causal ? lower_scores(q, k, OptTensor()) : OptTensor();
+            raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
             mark("conv_pre");
             x = conv2d(raw, conv_w, o.causal, scale, false);
         }
@@ -275,7 +296,9 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         mark("pv");
         Tensor out = lower_pv ? *causal_pv(m, v, true, o.first) : at::matmul(m, v);
         mark("end");
-        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, o.first ? *o.first : Tensor()});
+        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, o.first ? *o.first : Tensor(),
+                                o.key_bias ? *o.key_bias : Tensor()});
+        ctx->saved_data["s_real"] = s_real;
         ctx->saved_data["causal"] = o.causal;
         ctx->saved_data["pre_causal"] = o.pre_causal;
         ctx->saved_data["post_causal"] = o.post_causal;
@@ -283,7 +306,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         ctx->saved_data["post_group"] = o.post_group;
         ctx->saved_data["dropout"] = o.dropout;
         ctx->saved_data["lower_pv"] = lower_pv;
-        return heads_last(out);
+        return heads_last(out, s_real);
     }
 
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
@@ -292,7 +315,9 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &conv_w = saved[3], &w_pre = saved[4], &post_conv_w = saved[5],
                      &w_post = saved[6], &x = saved[8], &p = saved[9], &c = saved[10], &m = saved[11], &keep = saved[12];
         Tensor raw = saved[7];
-        const OptTensor first = saved[13].defined() ? OptTensor(saved[13]) : OptTensor();
+        const OptTensor first = saved[13].defined() ? OptTensor(saved[13]) : OptTensor(),
+                        key_bias = saved[14].defined() ? OptTensor(saved[14]) : OptTensor();
+        const int64_t s_real = ctx->saved_data["s_real"].toInt(), s_pad = q.size(2);
         const bool causal = ctx->saved_data["causal"].toBool(), pre_causal = ctx->saved_data["pre_causal"].toBool(),
                    post_causal = ctx->saved_data["post_causal"].toBool(), lower_pv = ctx->saved_data["lower_pv"].toBool();
         const int64_t pre_group = ctx->saved_data["pre_group"].toInt(), post_group = ctx->saved_data["post_group"].toInt();
@@ -304,39 +329,61 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         const bool need_qk = need[0] || need[1], need_x = need_qk || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
         torch::autograd::variable_list out(9);
 
-        const Tensor go = grads[0].transpose(1, 2).contiguous();
-        if (need[2]) {
-            const OptTensor dv = lower_pv ? causal_ptx(m, go, true) : OptTensor();
-            out[2] = dv ? *dv : at::matmul(m.transpose(2, 3), go);
+        Tensor go;   // (B,H,S,D), padded with zero rows
+        {
+            RowsCopy rows(s_pad, OptTensor());
+            go = rows.add(grads[0].transpose(1, 2), false, 1.0);
+            rows.run();
         }
-        if (!need_c && !need[6]) return out;
+        // the gradients of Q, K and V leave without the padding, without what the hidden keys' rows hold, and with the factor
+        const bool cut = s_pad != s_real;
+        Tensor dq, dk, dv;
+        double dq_scale = 1.0, dk_scale = 1.0;
+        auto results = [&] {
+            RowsCopy rows(s_real, key_bias);
+            auto leave = [&](Tensor &g, bool hide, double factor) {
+                return g.defined() && (cut || (hide && key_bias) || factor != 1.0) ? rows.add(g, hide, factor) : g;
+            };
+            out[0] = leave(dq, false, dq_scale);
+            out[1] = leave(dk, true, dk_scale);
+            out[2] = leave(dv, true, 1.0);
+            rows.run();
+            return out;
+        };
+        if (need[2]) {
+            const OptTensor own = lower_pv ? causal_ptx(m, go, true, 1.0) : OptTensor();
+            dv = own ? *own : at::matmul(m.transpose(2, 3), go);
+        }
+        if (!need_c && !need[6]) return results();
         const OptTensor lower_dm = lower_pv ? lower_scores(go, v, first) : OptTensor();
         TORCH_CHECK(lower_dm || !first);
         Tensor dm = lower_dm ? *lower_dm : at::matmul(go, v.transpose(2, 3));
         if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
         dm = dm.to(c.scalar_type());
         if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
-        if (!need_c) return out;
+        if (!need_c) return results();
         const Tensor dc = headmix_bwd_input(dm, w_post, post_causal, post_group, fill);
         if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
-        if (!need_p) return out;
+        if (!need_p) return results();
         const Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, fill);
         // (the head mixing's gradient kernels never read above the diagonal when causal)
         const Tensor ds = softmax_bwd(p, dp, causal, false);
         if (need[4]) out[4] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
-        if (!need_x) return out;
+        if (!need_x) return results();
         const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, fill);
         if (need_qk) {
             const bool lower = causal && q.sizes() == k.sizes() && causal_pv_supported(q.scalar_type(), k.size(-2), q.size(-1));
             const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
             if (first) band_zero_(g, *first);
             if (need[0]) {
-                const OptTensor dq = lower ? causal_pv(g, k, true, OptTensor()) : OptTensor();
-                out[0] = (dq ? *dq : at::matmul(g, k)).mul(scale);
+                const OptTensor own = lower ? causal_pv_scaled(g, k, true, scale) : OptTensor();
+                dq = own ? *own : at::matmul(g, k);
+                if (!own) dq_scale = scale;
             }
             if (need[1]) {
-                const OptTensor dk = lower ? causal_ptx(g, q, true) : OptTensor();
-                out[1] = (dk ? *dk : at::matmul(g.transpose(2, 3), q)).mul(scale);
+                const OptTensor own = lower ? causal_ptx(g, q, true, scale) : OptTensor();
+                dk = own ? *own : at::matmul(g.transpose(2, 3), q);
+                if (!own) dk_scale = scale;
             }
         }
         if (need[3]) {
@@ -347,7 +394,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
             }
             out[3] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale);
         }
-        return out;
+        return results();
     }
 };
 
@@ -359,13 +406,7 @@ Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const
     const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
     TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout, first, key_bias, empty_rows};
     const Mark mark{hook};
-    Tensor kk = k, vv = v;
-    if (key_bias) {   // (the hidden keys' K and V rows receive no gradient, as in the reference, whose masked_fill / where cut it)
-        const Tensor hidden = key_bias->eq(-INFINITY).unsqueeze(1).unsqueeze(-1);
-        kk = k.masked_fill(hidden, 0);
-        vv = v.masked_fill(hidden, 0);
-    }
-    return MtaTraining::apply(q, kk, vv, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);
+    return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);
 }
 
 // ---- the two operators ---------------------------------------------------------------------------------------------

@@ -214,12 +214,24 @@ inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, cons
     return o;
 }
 
-inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal)
+inline OptTensor causal_pv_scaled(const Tensor &p_, const Tensor &v_, bool causal, double scale)
+{
+    const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
+    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), v.size(2), v.size(3))) return std::nullopt;
+    Tensor o = at::empty(v.sizes(), v.options());
+    check(mta_causal_pv_scaled_fwd(ptr(p), ptr(v), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), causal, (float)scale, code(p, "P"),
+                                   stream_of(p)),
+          "mta_causal_pv_scaled_fwd");
+    return o;
+}
+
+inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, double scale)
 {
     const Tensor p = on_gpu(p_, "P"), x = on_gpu(x_, "X");
     if (p.scalar_type() != x.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), x.size(2), x.size(3))) return std::nullopt;
     Tensor o = at::empty(x.sizes(), x.options());
-    check(mta_causal_ptx_fwd(ptr(p), ptr(x), out_ptr(o), x.size(0), x.size(1), x.size(2), x.size(3), causal, code(p, "P"), stream_of(p)),
+    check(mta_causal_ptx_scaled_fwd(ptr(p), ptr(x), out_ptr(o), x.size(0), x.size(1), x.size(2), x.size(3), causal, (float)scale, code(p, "P"),
+                                    stream_of(p)),
           "mta_causal_ptx_fwd");
     return o;
 }
@@ -276,5 +288,50 @@ inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, co
           "mta_causal_pv_tri_fwd");
     return o;
 }
+
+// Rows of up to three (B,H,S,D) tensors, of any strides, into dense ones of S_out rows, one launch (mta_rows_copy).
+class RowsCopy {
+  public:
+    RowsCopy(int64_t s_out, const OptTensor &key_bias) : s_out_(s_out), key_bias_(key_bias) {}
+
+    // hide: the rows of hidden keys count as zeros
+    Tensor add(const Tensor &x_, bool hide, double scale)
+    {
+        TORCH_CHECK(x_.is_cuda(), "input lives on ", x_.device(), ": the MTA kernels only run on an AMD GPU (there is no CPU path)");
+        const Tensor x = x_.stride(3) == 1 ? x_ : x_.contiguous();
+        TORCH_CHECK_VALUE(n_ == 0 || (x.size(0) == like_[0].size(0) && x.size(1) == like_[0].size(1) && x.size(2) == like_[0].size(2) &&
+                                      x.scalar_type() == like_[0].scalar_type()),
+                          "Q, K and V must share batch, heads, length and dtype");
+        Tensor y = at::empty({x.size(0), x.size(1), s_out_, x.size(3)}, x.options());
+        x_ptr_[n_] = ptr(x);
+        y_ptr_[n_] = out_ptr(y);
+        for (int i = 0; i < 3; ++i) strides_[3 * n_ + i] = x.stride(i);
+        d_[n_] = x.size(3);
+        scale_[n_] = (float)scale;
+        hide_[n_] = hide && key_bias_;
+        like_[n_++] = x;
+        return y;
+    }
+
+    void run()
+    {
+        if (n_ == 0) return;
+        const Tensor &x = like_[0];
+        check(mta_rows_copy(n_, x_ptr_, strides_, y_ptr_, d_, scale_, hide_, ptr(key_bias_), key_bias_ ? key_bias_->size(1) : 0, x.size(0), x.size(1),
+                            x.size(2), s_out_, code(x, "input"), stream_of(x)),
+              "mta_rows_copy");
+    }
+
+  private:
+    int64_t s_out_;
+    OptTensor key_bias_;
+    int n_ = 0;
+    const void *x_ptr_[3];
+    void *y_ptr_[3];
+    int64_t strides_[9], d_[3];
+    float scale_[3];
+    int hide_[3];
+    Tensor like_[3];
+};
 
 }  // namespace mta_host

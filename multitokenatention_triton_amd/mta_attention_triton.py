@@ -246,6 +246,12 @@ def _weight_of(module) -> torch.Tensor:
     return weight if weight is not None else module.weight   # (a parametrised weight is an attribute)
 
 
+def _pad_rows(x: torch.Tensor, value) -> torch.Tensor:
+    """(B,S) with S rounded up to a multiple of 8, what the native routes pad causal lengths to."""
+    pad = -x.size(1) % 8
+    return F.pad(x, (0, pad), value=value) if pad else x
+
+
 def _wants_grad(xq, xk, xv, weights) -> bool:
     return torch.is_grad_enabled() and (xq.requires_grad or xk.requires_grad or xv.requires_grad
                                         or any(w.requires_grad for w in weights))
@@ -460,7 +466,7 @@ class MTAAttentionTriton(nn.Module):
                     bias = torch.where(mask, 0.0, float("-inf")).to(torch.float32)
                 else:
                     bias = mask.type(xq.dtype).to(torch.float32)   # the reference adds it in the I/O dtype
-                return self._forward_native(xq, xk, xv, key_bias=bias.contiguous())
+                return self._forward_native(xq, xk, xv, key_bias=_pad_rows(bias, 0.0).contiguous())
             # a 4-D mask, the same for all heads, of one of two forms goes into the kernels without a (B,H,S,S) tensor:
             # "causal rule + hidden keys" per batch entry (key padding: a key bias and zeroed K and V rows, as for the
             # 2-D mask above) and "row p sees the keys first[p] .. p" (sliding windows, packed documents: one int32 per
@@ -469,7 +475,10 @@ class MTAAttentionTriton(nn.Module):
                 kind, what = self._structured_mask(mask, xq.size(0), xq.size(-2))
                 if kind == "keys":
                     return self._forward_native(xq, xk, xv, key_bias=what)
-                if (kind == "band" and ops.qk_conv_supported(xq, xk, self.mta_conv_triton.weight)
+                if (kind == "band" and self._band_supported(xq, xk)
+                        # (rows that see nothing: with 3x5 and 7x9 kernels, which came to the band route last, such masks
+                        # stay on the mask passes, whose stages an observer may count on)
+                        and (self._band_empty_rows(mask) is None or self.mta_conv_triton.kernel_size not in ((3, 5), (7, 9)))
                         and (not _wants_grad(xq, xk, xv, self._weights()) or self._band_training_supported(xq, xk, xv))):
                     return self._forward_native(xq, xk, xv, first_visible=what, empty_rows=self._band_empty_rows(mask))
         elif (not self.causal and isinstance(mask, torch.Tensor) and mask.dim() == 4 and xq.size(-2) == xk.size(-2)):
@@ -562,13 +571,18 @@ class MTAAttentionTriton(nn.Module):
         self._mark("end")
         return output.transpose(1, 2)
 
+    def _band_supported(self, xq, xk) -> bool:
+        """Whether the first kernel takes a band mask for these tensors (lengths are padded to a multiple of 8)."""
+        w = self.mta_conv_triton.weight
+        return (xq.shape == xk.shape and xq.dtype == xk.dtype == w.dtype and xq.dtype in (torch.bfloat16, torch.float16)
+                and bool(_lib.load().mta_qk_conv_supported(8, xq.size(-1), w.size(1), w.size(2), _lib.MTA_BF16, _lib.MTA_BF16)))
+
     def _band_training_supported(self, xq, xk, xv) -> bool:
-        """Whether the differentiable route takes a band mask: 16-bit data of one dtype, a length the in-place zeroing
-        kernel takes, and the lower-triangle products (P V and its gradients, the recomputed raw scores) as kernels."""
-        s = xk.size(-2)
+        """Whether the differentiable route takes a band mask: 16-bit data of one dtype and the lower-triangle products
+        (P V and its gradients, the recomputed raw scores) as kernels."""
         return (xq.dtype in (torch.bfloat16, torch.float16) and xq.dtype == xk.dtype == xv.dtype
-                and xq.shape == xk.shape and s % 8 == 0 and _lower_products_supported(xv, s)
-                and _lower_products_supported(xq, s)
+                and xq.shape == xk.shape and xv.size(-2) == xk.size(-2) and ops.causal_pv_supported(xv.dtype, 8, xv.size(-1))
+                and ops.causal_pv_supported(xq.dtype, 8, xq.size(-1))
                 and all(w.dtype == xq.dtype for w in (self.mta_conv_triton.weight, self.mta_conv_after_sm_triton.weight,
                                                       self.wpsm_triton.weight, self.wposm_triton.weight)))
 
@@ -579,6 +593,7 @@ class MTAAttentionTriton(nn.Module):
           ("band", first)  row p sees exactly the keys first[p] .. p, or none at all (first[p] = p + 1): int32 (B,S);
           (None, None)     anything else (per-head planes, holes that differ between rows, other finite values, a row
                            that sees nothing).
+        With the causal rule the arrays are padded to a multiple of 8 columns, as the native routes pad the rows.
         A few reductions over the mask and one read back; the answer for the last mask object seen is kept while its
         version does not change."""
         if mask.size(0) not in (1, bsz) or mask.size(-2) != s or mask.size(-1) != s or mask.size(1) not in (1, self.n_heads):
@@ -608,22 +623,24 @@ class MTAAttentionTriton(nn.Module):
             visible = visible & lower
             keep = visible[:, -1, :]                       # what the last row sees: every kept key
             if bool((visible == (keep[:, None, :] & lower)).all()) and bool(keep[:, 0].all()):
-                bias = torch.where(keep, 0.0, float("-inf")).to(torch.float32).expand(bsz, s).contiguous()
-                answer = ("keys", bias)
+                bias = torch.where(keep, 0.0, float("-inf")).to(torch.float32).expand(bsz, s)
+                answer = ("keys", _pad_rows(bias, 0.0).contiguous())
             else:
                 count = visible.sum(-1)
                 lead = visible.int().argmax(-1)
                 empty = count == 0      # rows that see no key (the padding of a left-padded batch): first[p] = p + 1
                 if bool((empty | (count == rows[None, :] - lead + 1)).all()):
                     first = torch.where(empty, rows[None, :] + 1, lead)
-                    answer = ("band", first.to(torch.int32).expand(bsz, s).contiguous())
+                    first = _pad_rows(first.to(torch.int32).expand(bsz, s), 0)
+                    first[:, s:] = torch.arange(s, first.size(1), device=mask.device)   # (a padding row sees itself)
+                    answer = ("band", first.contiguous())
                     if bool(empty.any()):
-                        empty_rows = empty.expand(bsz, s).contiguous()
+                        empty_rows = _pad_rows(empty.expand(bsz, s), False).contiguous()
         self._mask_cache = (mask, key, answer, empty_rows)
         return answer
 
     def _band_empty_rows(self, mask):
-        """bool (B,S): the query rows of the band mask last classified that see no key at all, or None if every row sees
+        """bool (B, S rounded up to a multiple of 8): the query rows of the band mask last classified that see no key at all, or None if every row sees
         one."""
         cached = getattr(self, "_mask_cache", None)
         return cached[3] if cached is not None and cached[0] is mask else None

@@ -110,3 +110,66 @@ def test_headmix_twelve_heads(pkg, transposed, dtype):
                else pkg.ops.headmix(xd, w.cuda(), causal, 0.0, group_size=group))
         ulp = {torch.float32: 2.0 ** -21, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
         torch.testing.assert_close(got.double().cpu(), want.masked_fill(~keep, 0.0), rtol=ulp, atol=1e-5)
+
+
+def _mta(pkg, h, ks, ks2, dtype, seed, use_mask=False, structure=None):
+    g = torch.Generator().manual_seed(seed)
+    cfg = pkg.MTAConfig(query_kernel_size=ks[0], key_kernel_size=ks[1], after_sm_query_kernel_size=ks2[0], after_sm_key_kernel_size=ks2[1])
+    mod = pkg.MTAAttentionTriton(h, cfg, dropout=0.0, causal=True, use_mask=use_mask)
+    params = [O.seeded_conv_weight(h, *ks, 0.05, dtype, seed=seed), (torch.eye(h) + 0.1 * torch.randn(h, h, generator=g)).to(dtype),
+              O.seeded_conv_weight(h, *ks2, 0.05, dtype, seed=seed + 1), (torch.eye(h) + 0.1 * torch.randn(h, h, generator=g)).to(dtype)]
+    with torch.no_grad():
+        for p, w in zip((mod.mta_conv_triton, mod.wpsm_triton, mod.mta_conv_after_sm_triton, mod.wposm_triton), params):
+            p.weight.copy_(w)
+    return mod.to(dtype).cuda(), params
+
+
+def _ragged_mask(kind, b, s):
+    rows = torch.arange(s)
+    causal = rows[None, :] <= rows[:, None]
+    if kind == "window":
+        return (causal & (rows[None, :] > rows[:, None] - max(1, s // 3)))[None, None]
+    if kind == "padding":
+        lengths = torch.tensor([s - 3 * i for i in range(b)]).clamp(min=1)
+        return (causal[None] & (rows[None, None, :] < lengths[:, None, None]))[:, None]
+    return None
+
+
+@pytest.mark.parametrize("kind", ["none", "padding", "window"])
+@pytest.mark.parametrize("dtype,h,s,d", [(torch.bfloat16, 4, 33, 64), (torch.float16, 16, 129, 128), (torch.bfloat16, 12, 68, 64),
+                                         (torch.float32, 8, 61, 64), (torch.bfloat16, 8, 1, 64), (torch.float16, 16, 7, 64)])
+def test_mta_padded_lengths(pkg, dtype, h, s, d, kind):
+    """Causal lengths that are not a multiple of 8 run padded with zero rows: output and all seven gradients, without a mask,
+    under key padding and under a window, against the oracle (given the mask tensor)."""
+    print(f"mta padded length {dtype} h={h} s={s} d={d} {kind}", flush=True)
+    b = 2
+    mod, params = _mta(pkg, h, (5, 5), (3, 3), dtype, 51, use_mask=kind != "none")
+    mask = _ragged_mask(kind, b, s)
+    q, k, v = O.seeded_qkv(b, h, s, d, dtype, seed=52)
+    go = torch.randn(b, s, h, d, generator=torch.Generator().manual_seed(53)).to(dtype)
+    leaves = [t.clone().float().requires_grad_(True) for t in (q, k, v)]
+    wl = [p.clone().float().requires_grad_(True) for p in params]
+    am = None if mask is None else torch.where(mask, 0.0, float("-inf"))
+    want = O.mta_forward(*leaves, wl[0].unsqueeze(1), wl[1], wl[2].unsqueeze(1), wl[3], mask=am)
+    want.backward(go.float())
+    dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    gmask = None if mask is None else mask.cuda()
+    with torch.no_grad():
+        plain = mod(*dev, gmask, None)
+    out = mod(*dev, gmask, None)
+    out.backward(go.cuda())
+    assert out.shape == (b, s, h, d) and plain.shape == out.shape
+    # the forward against the oracle in the data's own dtype, which rounds where the kernels round: what is left is one ulp
+    # of the 16-bit format here and there (head mixing makes |out| a little larger than the convex combinations of tol())
+    want16 = O.mta_forward(q, k, v, params[0].unsqueeze(1), params[1], params[2].unsqueeze(1), params[3],
+                           mask=None if am is None else am.to(dtype)).float()
+    bound = tol(dtype) if dtype == torch.float32 else dict(rtol=2.0 ** (-7 if dtype == torch.bfloat16 else -10), atol=2e-2)
+    torch.testing.assert_close(plain.float().cpu(), want16, **bound)
+    torch.testing.assert_close(out.detach().float().cpu(), want16, **bound)
+    # gradients in the norm: a chain of about eight roundings of relative size 2^-9 (bf16) / 2^-12 (fp16), times the
+    # cancellation in softmax backward; fp32: sums in another order
+    rel = {torch.float32: 1e-4, torch.bfloat16: 4e-2, torch.float16: 1e-2}[dtype]
+    got = [t.grad for t in dev] + [m.weight.grad for m in (mod.mta_conv_triton, mod.wpsm_triton, mod.mta_conv_after_sm_triton, mod.wposm_triton)]
+    for name, a, w in zip("q k v conv pre conv2 post".split(), got, [t.grad for t in leaves + wl]):
+        assert torch.isfinite(a.float()).all(), name
+        assert float((a.float().cpu() - w).norm()) <= rel * float(w.norm()) + 1e-5, name
