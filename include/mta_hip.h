@@ -296,6 +296,16 @@ int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t B, int64_t
 int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
                               float scale, int io_dtype, void *stream);
 
+/* The three products on the lower triangle for fp32 tensors, D in {64,128}, S % 4 == 0 (MTA_ERR_UNSUPPORTED otherwise), causal:
+ *   mta_lower_scores_f32:  out[p,q] = sum_d a[p,d] b[q,d] for q <= p (QK^T of mta_attention_triton.py:69, and dP = dO V^T);
+ *                          nothing is written above the diagonal beyond the 16-byte vectors that straddle it (zeros)
+ *   mta_causal_pv_f32:     o[p] = scale * sum_{q<=p} p[p,q] v[q]           (P V; dQ)
+ *   mta_causal_ptx_f32:    o[q] = scale * sum_{p>=q} p[p,q] x[p]           (dV, dK)
+ * nothing of p above the diagonal is read. */
+int mta_lower_scores_f32(const void *a, const void *b, void *out, int64_t B, int64_t H, int64_t S, int64_t D, void *stream);
+int mta_causal_pv_f32(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);
+int mta_causal_ptx_f32(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);
+
 /* ---- backward of the two standalone operators -------------------------------------------------------------
  * Gradients flow through the same masks as the forward pass: with `causal`, entries of dy above the diagonal are
  * never read (the forward wrote a constant there) and gradients with respect to inputs above the diagonal are +0

@@ -76,6 +76,29 @@ int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool ca
     return causal && s == k.size(2) && s == v.size(2) ? (s + 7) / 8 * 8 : s;
 }
 
+// round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it: the scores kernel with factor 1
+// and the pass-through tap as 3x3 kernel, which copies its input exactly.  Nothing where that kernel does not apply.
+// `first`: a band mask, zeros ahead of a row's first visible key (the kernel does not visit the key blocks no row of a query
+// block sees: the hidden stretch of every row is cleared afterwards).
+OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
+{
+    if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type()) return std::nullopt;
+    if (a.scalar_type() == at::kFloat) {
+        if (!lower_products_supported(at::kFloat, a.size(2), a.size(3), true) || !a.is_cuda() || first) return std::nullopt;
+        const Tensor x = on_gpu(a, "Q"), y = on_gpu(b, "K");
+        Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
+        check(mta_lower_scores_f32(ptr(x), ptr(y), out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), stream_of(x)), "mta_lower_scores_f32");
+        return out;
+    }
+    if (!is16(a) || !a.is_cuda()) return std::nullopt;
+    Tensor w = at::zeros({a.size(1), 3, 3}, a.options());
+    w.select(1, 2).select(1, 1).fill_(1.0);
+    if (!qk_conv_supported(a, b, w)) return std::nullopt;
+    Tensor out = qk_conv(a, b, w, true, 1.0, false, first);
+    if (first) band_zero_(out, *first);
+    return out;
+}
+
 // ---- inference -------------------------------------------------------------------------------------------------------
 // The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
 // hides (-inf) are zeroed, so that their scores enter the pre-softmax conv as 0, and their V rows too where a post-softmax
@@ -114,7 +137,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const auto dtype = q.scalar_type();
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
-    const bool own_pv = q.size(-2) == n_keys && dtype == v.scalar_type() && causal_pv_supported(dtype, q.size(-2), v.size(-1));
+    const bool own_pv = q.size(-2) == n_keys && dtype == v.scalar_type() && lower_products_supported(dtype, q.size(-2), v.size(-1), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
     // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
@@ -148,9 +171,10 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     } else {
         TORCH_CHECK(!first, "the band mask needs the one-kernel first stage");
         mark("qk");
-        scores = at::matmul(q, k.transpose(2, 3));
-        mark("conv_pre");
-        scores = conv2d(scores, conv_w, causal, scale, true);
+        const OptTensor raw = causal ? lower_scores(q, k, OptTensor()) : OptTensor();
+        scores = raw ? *raw : at::matmul(q, k.transpose(2, 3));
+        mark("conv_pre");   // (the stage that follows never reads above the diagonal)
+        scores = conv2d(scores, conv_w, causal, scale, false);
     }
 
     if (one_pass) {
@@ -201,7 +225,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     }
     if (dropout > 0) scores = at::dropout(scores, dropout, true);
     mark("pv");
-    OptTensor out = own_pv ? causal_pv(scores, v, causal, first) : OptTensor();
+    OptTensor out = own_pv ? causal_pv(scores, v, causal, first, 1.0) : OptTensor();
     if (!out) out = at::matmul(scores, v);
     if (empty_rows) out->masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
     mark("end");
@@ -209,21 +233,6 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
 }
 
 // ---- training ----------------------------------------------------------------------------------------------------------
-// round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it: the scores kernel with factor 1
-// and the pass-through tap as 3x3 kernel, which copies its input exactly.  Nothing where that kernel does not apply.
-// `first`: a band mask, zeros ahead of a row's first visible key (the kernel does not visit the key blocks no row of a query
-// block sees: the hidden stretch of every row is cleared afterwards).
-OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
-{
-    if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !is16(a)) return std::nullopt;
-    Tensor w = at::zeros({a.size(1), 3, 3}, a.options());
-    w.select(1, 2).select(1, 1).fill_(1.0);
-    if (!qk_conv_supported(a, b, w)) return std::nullopt;
-    Tensor out = qk_conv(a, b, w, true, 1.0, false, first);
-    if (first) band_zero_(out, *first);
-    return out;
-}
-
 struct TrainOptions {
     bool causal, pre_causal, post_causal;
     double pre_fill, post_fill;
@@ -289,12 +298,12 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         mark("mix_post");
         // the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
         const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && v.size(-2) == n_keys &&
-                              c.size(-2) == c.size(-1) && causal_pv_supported(v.scalar_type(), c.size(-1), v.size(-1));
+                              c.size(-2) == c.size(-1) && lower_products_supported(v.scalar_type(), c.size(-1), v.size(-1), true);
         TORCH_CHECK(!o.first || lower_pv, "the band mask needs the lower-triangle products");
         Tensor m = headmix(c, w_post, o.post_causal, lower_pv ? 0.0 : o.post_fill, o.post_group, !lower_pv), keep;
         if (o.dropout > 0) std::tie(m, keep) = at::native_dropout(m, o.dropout, true);
         mark("pv");
-        Tensor out = lower_pv ? *causal_pv(m, v, true, o.first) : at::matmul(m, v);
+        Tensor out = lower_pv ? *causal_pv(m, v, true, o.first, 1.0) : at::matmul(m, v);
         mark("end");
         ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, o.first ? *o.first : Tensor(),
                                 o.key_bias ? *o.key_bias : Tensor()});
@@ -372,11 +381,11 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         if (!need_x) return results();
         const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, fill);
         if (need_qk) {
-            const bool lower = causal && q.sizes() == k.sizes() && causal_pv_supported(q.scalar_type(), k.size(-2), q.size(-1));
+            const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), k.size(-2), q.size(-1), true);
             const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
             if (first) band_zero_(g, *first);
             if (need[0]) {
-                const OptTensor own = lower ? causal_pv_scaled(g, k, true, scale) : OptTensor();
+                const OptTensor own = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
                 dq = own ? *own : at::matmul(g, k);
                 if (!own) dq_scale = scale;
             }

@@ -204,35 +204,43 @@ inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool
     return y;
 }
 
-inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first)
+// whether P V and P^T X run as kernels that read (and P's producer need only write) the lower triangle: 16-bit data, which
+// the kernels also take without the causal rule, or fp32 under it
+inline bool lower_products_supported(at::ScalarType t, int64_t s, int64_t d, bool causal)
 {
-    const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
-    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), v.size(2), v.size(3))) return std::nullopt;
-    Tensor o = at::empty(v.sizes(), v.options());
-    check(mta_causal_pv_band_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), causal, code(p, "P"), stream_of(p)),
-          "mta_causal_pv_fwd");
-    return o;
+    return causal_pv_supported(t, s, d) || (t == at::kFloat && causal && (d == 64 || d == 128) && s % 4 == 0 && s <= (1 << 20));
 }
 
-inline OptTensor causal_pv_scaled(const Tensor &p_, const Tensor &v_, bool causal, double scale)
+inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first, double scale)
 {
     const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
-    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), v.size(2), v.size(3))) return std::nullopt;
+    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !lower_products_supported(p.scalar_type(), v.size(2), v.size(3), causal))
+        return std::nullopt;
     Tensor o = at::empty(v.sizes(), v.options());
-    check(mta_causal_pv_scaled_fwd(ptr(p), ptr(v), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), causal, (float)scale, code(p, "P"),
-                                   stream_of(p)),
-          "mta_causal_pv_scaled_fwd");
+    const int64_t b = v.size(0), h = v.size(1), s = v.size(2), d = v.size(3);
+    if (!is16(p)) {
+        TORCH_CHECK(!first);
+        check(mta_causal_pv_f32(ptr(p), ptr(v), out_ptr(o), b, h, s, d, (float)scale, stream_of(p)), "mta_causal_pv_f32");
+    } else if (first) {
+        TORCH_CHECK(scale == 1.0);
+        check(mta_causal_pv_band_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), b, h, s, d, causal, code(p, "P"), stream_of(p)), "mta_causal_pv_fwd");
+    } else {
+        check(mta_causal_pv_scaled_fwd(ptr(p), ptr(v), out_ptr(o), b, h, s, d, causal, (float)scale, code(p, "P"), stream_of(p)), "mta_causal_pv_fwd");
+    }
     return o;
 }
 
 inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, double scale)
 {
     const Tensor p = on_gpu(p_, "P"), x = on_gpu(x_, "X");
-    if (p.scalar_type() != x.scalar_type() || p.size(2) != p.size(3) || !causal_pv_supported(p.scalar_type(), x.size(2), x.size(3))) return std::nullopt;
+    if (p.scalar_type() != x.scalar_type() || p.size(2) != p.size(3) || !lower_products_supported(p.scalar_type(), x.size(2), x.size(3), causal))
+        return std::nullopt;
     Tensor o = at::empty(x.sizes(), x.options());
-    check(mta_causal_ptx_scaled_fwd(ptr(p), ptr(x), out_ptr(o), x.size(0), x.size(1), x.size(2), x.size(3), causal, (float)scale, code(p, "P"),
-                                    stream_of(p)),
-          "mta_causal_ptx_fwd");
+    const int64_t b = x.size(0), h = x.size(1), s = x.size(2), d = x.size(3);
+    if (is16(p))
+        check(mta_causal_ptx_scaled_fwd(ptr(p), ptr(x), out_ptr(o), b, h, s, d, causal, (float)scale, code(p, "P"), stream_of(p)), "mta_causal_ptx_fwd");
+    else
+        check(mta_causal_ptx_f32(ptr(p), ptr(x), out_ptr(o), b, h, s, d, (float)scale, stream_of(p)), "mta_causal_ptx_f32");
     return o;
 }
 

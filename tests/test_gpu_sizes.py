@@ -173,3 +173,34 @@ def test_mta_padded_lengths(pkg, dtype, h, s, d, kind):
     for name, a, w in zip("q k v conv pre conv2 post".split(), got, [t.grad for t in leaves + wl]):
         assert torch.isfinite(a.float()).all(), name
         assert float((a.float().cpu() - w).norm()) <= rel * float(w.norm()) + 1e-5, name
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_fp32_lower_products(pkg, d):
+    """The three fp32 products on the lower triangle: one vector of rows, edges of the tiles (32 / 64 rows, 64 / 128 keys) and
+    of the steps the wavefronts share, NaN above the diagonal.  fp32 sums of n products against double precision: at most
+    sqrt(n) * 2^-22 of the sum of the products' magnitudes."""
+    lib, st = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(12)
+    for s in (4, 32, 36, 64, 100, 128, 196, 260, 516):
+        print(f"fp32 products d={d} s={s}", flush=True)
+        b, h = 2, 3
+        p = torch.randn(b, h, s, s, generator=g)
+        x, y = torch.randn(b, h, s, d, generator=g), torch.randn(b, h, s, d, generator=g)
+        low = torch.tril(torch.ones(s, s, dtype=torch.bool))
+        pd = p.masked_fill(~low, float("nan")).cuda()
+        lower = p.double().masked_fill(~low, 0.0)
+        xd, yd, out = x.cuda(), y.cuda(), torch.full((b, h, s, d), float("nan"), device="cuda")
+
+        def close(got, want, size, n):
+            assert ((got.double().cpu() - want).abs() <= n ** 0.5 * 2.0 ** -22 * size + 1e-30).all()
+
+        assert lib.mta_causal_pv_f32(pd.data_ptr(), xd.data_ptr(), out.data_ptr(), b, h, s, d, 0.5, st) == 0
+        close(out, 0.5 * (lower @ x.double()), 0.5 * (lower.abs() @ x.double().abs()), s)
+        assert lib.mta_causal_ptx_f32(pd.data_ptr(), xd.data_ptr(), out.data_ptr(), b, h, s, d, 0.5, st) == 0
+        close(out, 0.5 * (lower.transpose(2, 3) @ x.double()), 0.5 * (lower.abs().transpose(2, 3) @ x.double().abs()), s)
+        scores = torch.full((b, h, s, s), 7.0, device="cuda")
+        assert lib.mta_lower_scores_f32(xd.data_ptr(), yd.data_ptr(), scores.data_ptr(), b, h, s, d, st) == 0
+        close(scores[..., low.cuda()], (x.double() @ y.double().transpose(2, 3))[..., low], (x.double().abs() @ y.double().abs().transpose(2, 3))[..., low], d)
+        up = scores.cpu()[..., ~low]
+        assert ((up == 7.0) | (up == 0.0)).all()
