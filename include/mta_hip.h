@@ -302,6 +302,11 @@ int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, 
  *   mta_causal_pv_f32:     o[p] = scale * sum_{q<=p} p[p,q] v[q]           (P V; dQ)
  *   mta_causal_ptx_f32:    o[q] = scale * sum_{p>=q} p[p,q] x[p]           (dV, dK)
  * nothing of p above the diagonal is read. */
+/* out = round(a b^T) on and below the diagonal of a (B,H,S,S) tensor: mta_lower_scores_f32 for any I/O dtype (16-bit: S % 8 ==
+ * 0; the scores kernel without its conv).  first_visible (int32 (B,S), 16-bit only, or NULL): the products ahead of a row's
+ * first visible key are 0; key blocks that no row of a block of 128 sees are left unwritten. */
+int mta_lower_scores_fwd(const void *a, const void *b, const void *first_visible, void *out, int64_t B, int64_t H, int64_t S, int64_t D,
+                         int io_dtype, void *stream);
 int mta_lower_scores_f32(const void *a, const void *b, void *out, int64_t B, int64_t H, int64_t S, int64_t D, void *stream);
 int mta_causal_pv_f32(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);
 int mta_causal_ptx_f32(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);

@@ -193,6 +193,8 @@ struct item_table {
     uint32_t e[ITEM_TABLE_MAX];  // query block (11 bits) | first key block << 11 (11 bits) | key blocks << 22
 };
 
+// RAW (scores only, a 1x1 kernel): no conv at all - round(round(Q K^T) * scale) goes from the accumulators to memory: the
+// plain lower-triangle product of the training route (raw scores, dP = dO V^T).  No score tile, no retained columns, no halo.
 // SCORES_ONLY: stop after the conv and write  conv(mask0(scale * Q K^T))  as an (S,S) plane per (batch, head)
 // (`O` is then the score tensor, V is unused).  Only q <= p is written when causal, plus +0 above the
 // diagonal when `fill_upper` is set.
@@ -209,6 +211,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
     using G = fused_geom<R, SK, NW>;
+    constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
     constexpr int F_NT = 64 * NW, F_SR = 32 * NW;
     constexpr int CPR = D / 8;                     // 16-byte chunks per K/V row
     constexpr int TILE = F_BK * D;                 // elements per K or V block
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     __shared__ __align__(16) T B0[TILE];
     __shared__ __align__(16) T B1[TILE];
     __shared__ __align__(16) T B2[SCORES_ONLY ? 8 : TILE];
-    __shared__ __align__(16) T Sc[F_SR * F_SLD];                          // score tile
+    __shared__ __align__(16) T Sc[RAW ? 8 : F_SR * F_SLD];                // score tile
     // zero-padded kernel rows, only needed until the Toeplitz fragments are built: they borrow a buffer that
     // receives its first copy after that (LDS is granted in 1280-byte units; the array's own 648 bytes were the
     // difference between two and three workgroups per CU for the scores-only kernel)
@@ -356,10 +359,11 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         if (j_lo > j_end) return;
     }
     // one key block earlier only fills the retained score columns (before the first one: the right pad, if any)
-    const int j_start = j_lo > 0 ? j_lo - 1 : (G::PWR > 0 ? -1 : 0);
+    const int j_start = RAW ? j_lo : j_lo > 0 ? j_lo - 1 : (G::PWR > 0 ? -1 : 0);
     issue_k(j_start, B0);
     if (!SCORES_ONLY) issue_v(j_start, B1);
 
+    if constexpr (!RAW) {
     // zero the score tile once (columns past HC+BK are read by the last window but never written)
     for (int e = tid; e < F_SR * F_SLD / 8; e += F_NT) {
         pack16<T> z;
@@ -372,6 +376,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         const bool ok = jj >= 0 && jj < SK;
         const T wv = Wt[head * R * SK + (ok ? i * SK + jj : 0)];
         wz[e] = ok ? wv : from_float<T>(0.0f);
+    }
     }
 
     // this lane's two query rows
@@ -408,7 +413,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     // Toeplitz fragments T_i^T: accumulator row m = ln, slots k = 8*kg + t, tap = k - SHIFT - m
     frag8<T> tz[R];
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
+    for (int i = 0; i < (RAW ? 0 : R); ++i) {
         const T *src = wz + i * G::WZ_LD + G::WZ_OFF + kg * 8 - G::SHIFT - ln;
 #pragma unroll
         for (int t = 0; t < 8; ++t) tz[i].v[t] = src[t];
@@ -523,6 +528,12 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                     } else {
                         const u32x2_t s0 = __builtin_amdgcn_permlane16_swap(held[rb][0], lo, false, false);
                         const u32x2_t s1 = __builtin_amdgcn_permlane16_swap(held[rb][1], hi, false, false);
+                        if constexpr (RAW) {
+                            const int kg_o = opaque_lane(kg);
+                            const int col = cbase + (cb - 1 + (kg_o & 1)) * 16 + (kg_o >> 1) * 8, p_ = prow[rb];
+                            if (p_ < S && (PLAIN || (col < S && (!causal || fill_upper || col <= p_))))
+                                *reinterpret_cast<u32x4_t *>(Op + (int64_t)p_ * S + col) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
+                        } else
                         lds_write16_at(wa, (rb * 16 * F_SLD + (cb - 1) * 16) * (int)sizeof(T), u32x4_t{s0[0], s1[0], s0[1], s1[1]});
                     }
                 }
@@ -533,7 +544,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 constexpr int cb = n / KS, ks = n % KS;
                 if constexpr (n + KLD < NSTEP) kissue(std::integral_constant<int, n + KLD>{});
                 // LDS operations younger than read n: the reads issued after it and the score writes issued since
-                constexpr int younger = (n + KLD < NSTEP ? n + KLD : NSTEP - 1) - n + score_writes_between(n > KLD ? n - KLD : 0, n, KS, NCB, LAG);
+                constexpr int younger = (n + KLD < NSTEP ? n + KLD : NSTEP - 1) - n + (RAW ? 0 : score_writes_between(n > KLD ? n - KLD : 0, n, KS, NCB, LAG));
                 lds_wait_upto<(younger < 15 ? younger : 15)>(kring[n % KSLOT]);
                 if constexpr (ks == 0) {
                     sacc[cb & 1][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -549,6 +560,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
             });
             epilogue(std::integral_constant<int, NCB - 1>{});
         }
+        if constexpr (RAW) return;
+        else {
         // score tile complete for everybody.  Only the LDS counter is waited for: a fence would also wait for the
         // copy of the next key block, in flight since the top of the iteration
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -717,6 +730,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 mma16(oacc[1][db], vf[blk & 1], pf[1][ks]);
             }
         }
+        }
     };
     auto plain = [&](int j) {  // (scores-only kernel: a second body per buffer rotation makes the attention kernel spill)
         const int cbase = j * F_BK + G::PWR;
@@ -790,6 +804,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     constexpr int NW = 4;
     constexpr int F_NT = 64 * NW;
     using G = fused_geom<R, SK, NW>;
+    constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
     static_assert(G::fits, "conv window exceeds the 32-key MFMA contraction");
     const int nqb = (int)((S + G::BQ - 1) / G::BQ);
     auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND>;
@@ -830,7 +845,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
                 const int len = j0 < nlong ? std::min(big, nlong - j0) : std::min(small, nk - j0);
                 if (n >= ITEM_TABLE_MAX) { ok = false; break; }
                 // what the kernel visits: one key block earlier rebuilds the retained columns (ahead of the first: the right pad)
-                lens[n] = len + ((j0 > 0 || G::PWR > 0) ? 1 : 0);
+                lens[n] = len + (!RAW && (j0 > 0 || G::PWR > 0) ? 1 : 0);
                 items[n++] = (uint32_t)qb | ((uint32_t)j0 << 11) | ((uint32_t)len << 22);
                 j0 += len;
             }
@@ -865,6 +880,10 @@ int dispatch_mfma(const void *q, const void *k, const void *v, const void *w, vo
                   int tri_gl = 0)
 {
     if constexpr (sizeof(T) == 2) {
+        if constexpr (SCORES_ONLY) {   // no conv (weights are not read)
+            if (R == 1 && Sk == 1)
+                return launch_mfma<T, D, 1, 1, true, BAND>(q, k, v, w, o, lse, B, H, S, causal, scale, fill_upper, st, band_lo, 0);
+        }
 #define MTA_FUSED_CASE(r, s) \
     if (R == r && Sk == s) return launch_mfma<T, D, r, s, SCORES_ONLY, BAND>(q, k, v, w, o, lse, B, H, S, causal, scale, fill_upper, st, band_lo, tri_gl);
         MTA_FUSED_CASE(3, 3)

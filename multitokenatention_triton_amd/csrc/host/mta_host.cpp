@@ -76,25 +76,18 @@ int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool ca
     return causal && s == k.size(2) && s == v.size(2) ? (s + 7) / 8 * 8 : s;
 }
 
-// round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it: the scores kernel with factor 1
-// and the pass-through tap as 3x3 kernel, which copies its input exactly.  Nothing where that kernel does not apply.
+// round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it.  Nothing where there is no kernel.
 // `first`: a band mask, zeros ahead of a row's first visible key (the kernel does not visit the key blocks no row of a query
 // block sees: the hidden stretch of every row is cleared afterwards).
 OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 {
-    if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type()) return std::nullopt;
-    if (a.scalar_type() == at::kFloat) {
-        if (!lower_products_supported(at::kFloat, a.size(2), a.size(3), true) || !a.is_cuda() || first) return std::nullopt;
-        const Tensor x = on_gpu(a, "Q"), y = on_gpu(b, "K");
-        Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
-        check(mta_lower_scores_f32(ptr(x), ptr(y), out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), stream_of(x)), "mta_lower_scores_f32");
-        return out;
-    }
-    if (!is16(a) || !a.is_cuda()) return std::nullopt;
-    Tensor w = at::zeros({a.size(1), 3, 3}, a.options());
-    w.select(1, 2).select(1, 1).fill_(1.0);
-    if (!qk_conv_supported(a, b, w)) return std::nullopt;
-    Tensor out = qk_conv(a, b, w, true, 1.0, false, first);
+    if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !a.is_cuda() ||
+        !lower_products_supported(a.scalar_type(), a.size(2), a.size(3), true) || (first && !is16(a)))
+        return std::nullopt;
+    const Tensor x = on_gpu(a, "Q"), y = on_gpu(b, "K");
+    Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
+    check(mta_lower_scores_fwd(ptr(x), ptr(y), ptr(first), out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
+          "mta_lower_scores_fwd");
     if (first) band_zero_(out, *first);
     return out;
 }

@@ -77,24 +77,13 @@ from . import _lib, ops
 from .convolution_2d_trit import Conv2dTriton, Conv2dTritonFunction
 from .triton_linear_head import TritonLinearHead, TritonLinearHeadFunction
 
-_IDENTITY_KERNELS = {}
-
-
 def _lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it, for consumers that
-    never read there: the scores kernel (``mta_qk_conv_fwd``) with factor 1 and a 3x3 kernel that is the pass-through
-    tap, which copies its input exactly.  Half the output traffic of the library GEMM.  None where that kernel does not
-    apply (fp32, ragged lengths): the caller then takes the GEMM."""
-    if a.shape != b.shape or a.dtype == torch.float32 or a.dtype != b.dtype:
+    never read there (``mta_lower_scores_fwd``): half the output traffic of the library GEMM.  None where that kernel does
+    not apply (ragged lengths, other head sizes): the caller then takes the GEMM."""
+    if a.shape != b.shape or a.dtype != b.dtype:
         return None
-    h = a.size(1)
-    key = (h, a.dtype, a.device)
-    w = _IDENTITY_KERNELS.get(key)
-    if w is None:
-        w = torch.zeros(h, 3, 3, dtype=a.dtype, device=a.device)
-        w[:, 2, 1] = 1.0
-        _IDENTITY_KERNELS[key] = w
-    out = ops.qk_conv(a, b, w, True, 1.0, fill_upper=False, first_visible=first_visible)
+    out = ops.lower_scores(a, b, first_visible)
     if out is not None and first_visible is not None:
         # a band mask: the products ahead of a row's first visible key count as 0.  The kernel does not visit the key
         # blocks that no row of a query block sees: the hidden stretch of every row is cleared afterwards.

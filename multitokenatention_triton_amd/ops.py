@@ -598,6 +598,23 @@ def mask_add(x: torch.Tensor, mask: torch.Tensor, causal: bool, out: Optional[to
     return y
 
 
+def lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """round(a b^T) on and below the diagonal, for a, b (B,H,S,D); see mta_lower_scores_fwd.  Returns ``None`` when
+    unsupported."""
+    a = _device_tensor(a, "Q")
+    b = _device_tensor(b, "K")
+    n, h, s, d = a.shape
+    out = torch.empty((n, h, s, s), dtype=a.dtype, device=a.device)
+    first_visible = _band_arg(first_visible, n, s)
+    with torch.cuda.device(a.device):
+        rc = _lib.load().mta_lower_scores_fwd(a.data_ptr(), b.data_ptr(), first_visible.data_ptr() if first_visible is not None else None,
+                                              out.data_ptr(), n, h, s, d, _code(a, "Q"), _stream(a))
+    if rc in (_lib.MTA_ERR_UNSUPPORTED, -7):
+        return None
+    _lib.check(rc, "mta_lower_scores_fwd")
+    return out
+
+
 def causal_ptx(p: torch.Tensor, x: torch.Tensor, causal: bool) -> Optional[torch.Tensor]:
     """P^T X for P (B,H,S,S), X (B,H,S,D): out[k] = sum_p P[p,k] X[p], over p >= k only when causal (nothing of P above
     the diagonal is read); see mta_causal_ptx_fwd.  Returns ``None`` when unsupported (the caller then uses

@@ -204,3 +204,19 @@ def test_fp32_lower_products(pkg, d):
         close(scores[..., low.cuda()], (x.double() @ y.double().transpose(2, 3))[..., low], (x.double().abs() @ y.double().abs().transpose(2, 3))[..., low], d)
         up = scores.cpu()[..., ~low]
         assert ((up == 7.0) | (up == 0.0)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_lower_scores_without_conv(pkg, d, dtype):
+    """round(a b^T) on and below the diagonal: one vector of rows, edges of the 128-row and 64-key blocks, lengths cut into
+    several work items.  Exact for small integers, whose products and sums fp32 and the 16-bit type (up to 2^8) hold."""
+    g = torch.Generator().manual_seed(13)
+    for s in (8, 64, 72, 128, 200, 264, 1160):
+        print(f"lower scores d={d} s={s} {dtype}", flush=True)
+        a, c = (torch.zeros(1, 2, s, d) for _ in range(2))
+        a[..., :8] = torch.randint(-2, 3, (1, 2, s, 8), generator=g).float()
+        c[..., :8] = torch.randint(-2, 3, (1, 2, s, 8), generator=g).float()
+        got = pkg.ops.lower_scores(a.to(dtype).cuda(), c.to(dtype).cuda()).cpu()
+        low = torch.tril(torch.ones(s, s, dtype=torch.bool))
+        assert torch.equal(got[..., low].float(), (a @ c.transpose(2, 3))[..., low])
