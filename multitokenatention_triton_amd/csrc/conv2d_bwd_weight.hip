@@ -9,7 +9,10 @@
 // reference accumulates in fp64 with atomics, convolution_2d_trit.py:236-295).
 //
 // Work split: the persistent workgroups are divided among the channels; the workgroups of a channel walk that
-// channel's (batch, 32x64 tile) list with a stride.  Tiles wholly above the diagonal are skipped.
+// channel's list of tiles (of strips) with a stride.  Tiles wholly above the diagonal are skipped.
+//
+// fp32, and 16-bit rows that are not whole vectors: row-sliding kernels (conv2d_rows.hpp) for the sizes known at compile
+// time, else 32x64 tiles in LDS (conv2d_bwd_weight_any).
 //
 // 16-bit tensors whose rows are a multiple of 8 keys take the matrix cores (conv2d_bwd_weight_mfma): for a fixed
 // key offset j the sums over q of dy[p,q] * x[p',q+j-pad] for 16 rows p and 16 rows p' are one 16x16 product with the
@@ -19,6 +22,7 @@
 #include <atomic>
 
 #include "common.hpp"
+#include "conv2d_rows.hpp"
 #include "mfma.hpp"
 
 namespace {
@@ -60,91 +64,6 @@ struct split_t { int channel, sub, bpc; };
 __device__ __forceinline__ split_t split_of(int block, int C, int bpc)
 {
     return split_t{block / bpc, block % bpc, bpc};
-}
-
-// Kernel size known at compile time: all R*S sums of a lane live in registers.
-template <typename T, int R, int S>
-__global__ __launch_bounds__(NT) void conv2d_bwd_weight_fixed(const T *__restrict__ x, const T *__restrict__ dy,
-                                                              float *__restrict__ partial, int N, int C, int H, int W,
-                                                              int causal, int tiles_m, int tiles_n, int bpc, int vec_ok)
-{
-    constexpr int LD = TN + S;  // S-1 halo columns + 1 pad
-    __shared__ float tile[(TM + R - 1) * LD];
-    __shared__ float red[NT / 64][R * S];
-    const int tid = threadIdx.x;
-    const split_t sp = split_of(blockIdx.x, C, bpc);
-    const int c = sp.channel;
-    const int tr = tid >> 3, tc = (tid & 7) * 8;
-
-    float acc[R][S];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-        for (int j = 0; j < S; ++j) acc[i][j] = 0.0f;
-
-    const int tiles = tiles_m * tiles_n;
-    const int64_t items = (int64_t)N * tiles;
-    for (int64_t it = sp.sub; it < items; it += sp.bpc) {
-        const int n = (int)(it / tiles), t = (int)(it % tiles);
-        const int tm = t / tiles_n, tn = t % tiles_n;
-        const int p0 = tm * TM, q0 = tn * TN;
-        if (causal && q0 > p0 + TM - 1) continue;  // dy is masked to zero on the whole tile (uniform per workgroup)
-        const int64_t plane = ((int64_t)n * C + c) * H * W;
-        __syncthreads();  // the previous tile's readers are done
-        stage_x<T>(x + plane, tile, LD, H, W, p0, q0, R, S, causal, tid);
-        // this lane's 8 gradient values
-        float g[8];
-        const int p = p0 + tr, q = q0 + tc;
-        if (vec_ok && p < H && q + 8 <= W) {  // eight contiguous values, 16-byte aligned
-            const T *src = dy + plane + (int64_t)p * W + q;
-            T raw[8];
-            if constexpr (sizeof(T) == 2) {
-                *reinterpret_cast<pack16<T> *>(raw) = *reinterpret_cast<const pack16<T> *>(src);
-            } else {
-                *reinterpret_cast<pack16<T> *>(raw) = *reinterpret_cast<const pack16<T> *>(src);
-                *reinterpret_cast<pack16<T> *>(raw + 4) = *reinterpret_cast<const pack16<T> *>(src + 4);
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) g[u] = (causal && q + u > p) ? 0.0f : to_float(raw[u]);
-        } else {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const bool ok = p < H && q + u < W && !(causal && q + u > p);
-                g[u] = ok ? to_float(dy[plane + (int64_t)p * W + q + u]) : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            float win[S + 7];
-            const float *src = tile + (tr + i) * LD + tc;
-#pragma unroll
-            for (int u = 0; u < S + 7; ++u) win[u] = src[u];
-#pragma unroll
-            for (int j = 0; j < S; ++j) {
-                float a = acc[i][j];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) a = fmaf(g[u], win[u + j], a);
-                acc[i][j] = a;
-            }
-        }
-    }
-    // workgroup reduction, once
-    const int wave = tid >> 6, lane = tid & 63;
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-        for (int j = 0; j < S; ++j) {
-            const float s = wave_sum(acc[i][j]);
-            if (lane == 0) red[wave][i * S + j] = s;
-        }
-    __syncthreads();
-    for (int t = tid; t < R * S; t += NT) {
-        float s = 0.0f;
-#pragma unroll
-        for (int wv = 0; wv < NT / 64; ++wv) s += red[wv][t];
-        partial[((int64_t)c * bpc + sp.sub) * (R * S) + t] = s;
-    }
 }
 
 // ---- matrix-core kernel -------------------------------------------------------------------------------------------
@@ -457,7 +376,7 @@ __global__ __launch_bounds__(NT) void conv2d_bwd_weight_any(const T *__restrict_
 
 // dw[c][t] = scale * sum over the channel's partial kernels, in the weight's dtype: 64 entries per workgroup, the partial
 // kernels dealt to 16 wavefronts (each adds its share in index order), the 16 sums added in wavefront order.  (A thread per
-// entry walking its 64 partial kernels alone took 11 us at 16 channels, 6x11; this takes 4.))
+// entry walking its 64 partial kernels alone took 11 us at 16 channels, 6x11; this takes 4.)
 constexpr int RED_SLICES = 16;
 __global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *__restrict__ partial, void *__restrict__ dw, int total,
                                                                    int RS, int bpc, float scale, int out_dtype)
@@ -552,20 +471,7 @@ int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int
 #undef MTA_CONV_CASE
         }
     }
-#define MTA_CONV_CASE(r, s)                                                                                          \
-    if (R == r && S == s) {                                                                                          \
-        hipLaunchKernelGGL((conv2d_bwd_weight_fixed<T, r, s>), grid, dim3(NT), 0, st, (const T *)x, (const T *)dy,    \
-                           partial, (int)N, (int)C, (int)H, (int)W, causal, tiles_m, tiles_n, bpc, vec_ok);           \
-        goto reduce;                                                                                                 \
-    }
-    MTA_CONV_CASE(3, 3)
-    MTA_CONV_CASE(3, 5)
-    MTA_CONV_CASE(5, 5)
-    MTA_CONV_CASE(5, 7)
-    MTA_CONV_CASE(6, 11)
-    MTA_CONV_CASE(7, 7)
-    MTA_CONV_CASE(7, 9)
-#undef MTA_CONV_CASE
+    if (launch_weight_rows<T>(x, dy, partial, bpc, N, C, H, W, R, S, causal, st)) goto reduce;
     {
         const size_t lds = sizeof(float) * ((size_t)(TM + R - 1) * (TN + S) + (size_t)TM * TN + (size_t)R * S);
         auto kern = conv2d_bwd_weight_any<T>;

@@ -8,9 +8,10 @@
 // tiles that lie entirely above the diagonal (they only receive their +0 fill), and
 // applies the causal output rule on store.
 //
-// Two compute paths:
-//   conv2d_valu  fp32 FMAs from an fp32 LDS tile; any I/O and weight dtype; each lane
-//                slides a register window along the key axis (8 outputs per lane).
+// Three compute paths:
+//   conv2d_valu  fp32 FMAs from an fp32 LDS tile (8 outputs per lane); any I/O and weight dtype, any kernel size.
+//   conv2d_rows  fp32 FMAs, sliding down the rows in registers (conv2d_rows.hpp); any I/O and weight dtype, the kernel
+//                sizes known at compile time.
 //   conv2d_mfma  16-bit I/O with weights of the same dtype.  The 6x11 conv costs 66 FMAs
 //                per output, which on the vector ALU takes longer than moving the tensor
 //                through HBM.  Each kernel row is therefore applied as a banded (Toeplitz)
@@ -22,6 +23,7 @@
 //                with ~16x the rate: the kernel becomes HBM-bound.  Products of 16-bit
 //                values are exact in fp32 and accumulation is fp32, as in the VALU path.
 #include "common.hpp"
+#include "conv2d_rows.hpp"
 #include "mfma.hpp"
 #include "strip_common.hpp"
 
@@ -64,14 +66,12 @@ __device__ __forceinline__ void store_row8(T *yp, int64_t W, int H, int p, int q
 //   dx[h,w] = sum_{i,j} w[i,j] * dym[h-i+(R-1), w-j+(S-1)/2]        (dym = dy with q>p read as 0 when causal)
 // which is the same tile computation with the kernel reversed in both axes, the row halo below the tile instead of
 // above it and the key halos swapped; dx is +0 above the diagonal (those inputs were never read).
-template <typename T, int R_T, int S_T, bool BWD>
+template <typename T, bool BWD>
 __global__ __launch_bounds__(NT) void conv2d_valu(const T *__restrict__ x, const void *__restrict__ w,
-                                                  T *__restrict__ y, int C, int H, int W, int R_rt,
-                                                  int S_rt, int causal, float in_scale, int use_scale,
+                                                  T *__restrict__ y, int C, int H, int W, int R,
+                                                  int S, int causal, float in_scale, int use_scale,
                                                   int w_dtype, int tiles_n)
 {
-    const int R = R_T > 0 ? R_T : R_rt;
-    const int S = S_T > 0 ? S_T : S_rt;
     const int pad_h = BWD ? 0 : R - 1, pad_w = BWD ? S - 1 - (S - 1) / 2 : (S - 1) / 2;
     const int LD = V_TN + S;  // S-1 halo columns + 1 pad
     extern __shared__ float smem[];
@@ -114,34 +114,18 @@ __global__ __launch_bounds__(NT) void conv2d_valu(const T *__restrict__ x, const
     }
     __syncthreads();
 
-    if constexpr (R_T > 0 && S_T > 0) {
+    for (int i = 0; i < R; ++i) {
+        const float *src = tile + (tr + i) * LD + tc;
+        for (int j = 0; j < S; ++j) {
+            const float wv = wsm[i * S + j];
 #pragma unroll
-        for (int i = 0; i < R_T; ++i) {
-            float win[S_T + 7];
-            const float *src = tile + (tr + i) * LD + tc;
-#pragma unroll
-            for (int u = 0; u < S_T + 7; ++u) win[u] = src[u];
-#pragma unroll
-            for (int j = 0; j < S_T; ++j) {
-                const float wv = wsm[i * S_T + j];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) acc[u] = fmaf(wv, win[u + j], acc[u]);
-            }
-        }
-    } else {
-        for (int i = 0; i < R; ++i) {
-            const float *src = tile + (tr + i) * LD + tc;
-            for (int j = 0; j < S; ++j) {
-                const float wv = wsm[i * S + j];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) acc[u] = fmaf(wv, src[u + j], acc[u]);
-            }
+            for (int u = 0; u < 8; ++u) acc[u] = fmaf(wv, src[u + j], acc[u]);
         }
     }
     store_row8<T>(yp, W, H, p0 + tr, q0 + tc, acc, causal != 0);
 }
 
-template <typename T, int R_T, int S_T, bool BWD>
+template <typename T, bool BWD>
 int launch_valu(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,
                 int S, int causal, float in_scale, int use_scale, int w_dtype, hipStream_t st)
 {
@@ -150,31 +134,12 @@ int launch_valu(const void *x, const void *w, void *y, int64_t N, int64_t C, int
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)(N * C));
     if (lds > 160 * 1024) return MTA_ERR_KERNEL_SIZE;
     if (lds > 48 * 1024) {  // per device, so set on every such launch (a cheap host-side call)
-        hipError_t e = hipFuncSetAttribute((const void *)conv2d_valu<T, R_T, S_T, BWD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void *)conv2d_valu<T, BWD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL((conv2d_valu<T, R_T, S_T, BWD>), grid, dim3(NT), lds, st, (const T *)x, w, (T *)y, (int)C,
+    hipLaunchKernelGGL((conv2d_valu<T, BWD>), grid, dim3(NT), lds, st, (const T *)x, w, (T *)y, (int)C,
                        (int)H, (int)W, R, S, causal, in_scale, use_scale, w_dtype, tiles_n);
     return launch_status();
-}
-
-template <typename T, bool BWD>
-int dispatch_valu(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,
-                  int S, int causal, float in_scale, int use_scale, int w_dtype, hipStream_t st)
-{
-#define MTA_CONV_CASE(r, s)                                                                               \
-    if (R == r && S == s)                                                                                 \
-        return launch_valu<T, r, s, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);
-    MTA_CONV_CASE(3, 3)
-    MTA_CONV_CASE(3, 5)
-    MTA_CONV_CASE(5, 5)
-    MTA_CONV_CASE(5, 7)
-    MTA_CONV_CASE(6, 11)
-    MTA_CONV_CASE(7, 7)
-    MTA_CONV_CASE(7, 9)
-    MTA_CONV_CASE(11, 15)
-#undef MTA_CONV_CASE
-    return launch_valu<T, 0, 0, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);
 }
 
 // ------------------------------------------------------------------------------------
@@ -753,7 +718,9 @@ int conv2d_entry(const void *x, const void *w, void *y, int64_t N, int64_t C, in
             const int rc = dispatch_mfma<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, st);
             if (rc != 1) return rc;
         }
-        return dispatch_valu<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);
+        const int rc = dispatch_rows<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);
+        if (rc != 1) return rc;
+        return launch_valu<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);
     });
     return MTA_ERR_DTYPE;
 }

@@ -220,3 +220,39 @@ def test_lower_scores_without_conv(pkg, d, dtype):
         got = pkg.ops.lower_scores(a.to(dtype).cuda(), c.to(dtype).cuda()).cpu()
         low = torch.tril(torch.ones(s, s, dtype=torch.bool))
         assert torch.equal(got[..., low].float(), (a @ c.transpose(2, 3))[..., low])
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("r,sk", [(3, 3), (3, 5), (5, 5), (5, 7), (6, 11), (7, 7), (7, 9), (11, 15)])
+def test_row_sliding_conv(pkg, r, sk, dtype, wdtype):
+    """The row-sliding conv kernels, forward / scaled / input gradient / kernel gradient: widths below a window and with every
+    remainder modulo 4, edges of the 64-key and 64- / 128-row wavefront tiles, non-square planes, NaN above the diagonal.
+    Against double precision: R*S (or N*P*Q) fp32 sums, one rounding to the data type (16-bit: also of the scaled input)."""
+    g = torch.Generator().manual_seed(31)
+    io = {torch.float32: 2.0 ** -22, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for p, q, causal in ((4, 4, True), (5, 7, False), (65, 65, True), (66, 70, False), (131, 131, True), (140, 140, True), (33, 259, False)):
+        if dtype == torch.float16 and q % 8 == 0:
+            continue   # (rows of whole vectors: the matrix-core kernels)
+        print(f"rows conv {r}x{sk} {p}x{q} causal={causal} {dtype}/{wdtype}", flush=True)
+        x, dy = (torch.randn(2, 3, p, q, generator=g).to(dtype) for _ in range(2))
+        w = (0.2 * torch.randn(3, r, sk, generator=g)).to(wdtype)
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        xd, dyd = (t.double().masked_fill(~keep, 0.0) for t in (x, dy))
+        xg, dyg = (t.masked_fill(~keep, float("nan")).cuda() for t in (x, dy))
+
+        def conv(a):
+            pad = torch.nn.functional.pad(a, ((sk - 1) // 2, sk - 1 - (sk - 1) // 2, r - 1, 0))
+            return torch.nn.functional.conv2d(pad, w.double().unsqueeze(1), groups=3).masked_fill(~keep, 0.0)
+
+        xa = xd.clone().requires_grad_(True)
+        conv(xa).backward(dyd)
+        wa = w.double().requires_grad_(True)
+        pad = torch.nn.functional.pad(xd, ((sk - 1) // 2, sk - 1 - (sk - 1) // 2, r - 1, 0))
+        torch.nn.functional.conv2d(pad, wa.unsqueeze(1), groups=3).backward(dyd)
+        size = float(r * sk) ** 0.5 * 0.2 * 4          # of a sum of R*S products
+        for got, want in ((pkg.ops.conv2d_causal(xg, w.cuda(), causal), conv(xd)),
+                          (pkg.ops.conv2d_causal(xg, w.cuda(), causal, in_scale=0.125), conv((x.float() * 0.125).to(dtype).double().masked_fill(~keep, 0.0))),
+                          (pkg.ops.conv2d_bwd_input(dyg, w.cuda(), causal), xa.grad.masked_fill(~keep, 0.0))):
+            torch.testing.assert_close(got.double().cpu(), want, rtol=io, atol=size * 2.0 ** -21)
+        dw = pkg.ops.conv2d_bwd_weight(xg, dyg, (r, sk), causal).double().cpu()
+        assert float((dw - wa.grad).abs().max()) <= (2 * p * q) ** 0.5 * 2.0 ** -19 * 16
