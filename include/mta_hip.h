@@ -235,6 +235,8 @@ int mta_causal_pv_band_fwd(const void *p, const void *v, const void *first_visib
  * for a band mask, below the diagonal (above it nothing is touched: the causal kernels on either side neither read nor
  * need it).  16-bit I/O, S % 8 == 0; MTA_ERR_UNSUPPORTED otherwise. */
 int mta_band_zero_fwd(void *x, const void *first_visible, int64_t N, int64_t C, int64_t S, int io_dtype, void *stream);
+/* The same for fp32 data, S % 4 == 0. */
+int mta_band_zero_f32(void *x, const void *first_visible, int64_t N, int64_t C, int64_t S, void *stream);
 
 /* y[n,c,p,q] = visible[n,c,p,q] ? x[n,c,p,q] : (neg_inf ? -inf : 0) for a mask tensor of arbitrary content: the
  * reference's `scores_masked[mask == float("-inf")] = 0` ahead of its two convs, its `scores = scores + mask` ahead of the

@@ -33,6 +33,7 @@ SIGNATURES = {
     "mta_qk_conv_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _f32, _int, _int, _int, _vp]),
     "mta_qk_conv_supported": (_int, [_i64, _i64, _int, _int, _int, _int]),
     "mta_causal_pv_band_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
+    "mta_band_zero_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "mta_band_zero_fwd": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "mta_mask_fill_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _int, _vp]),
     "mta_mask_add_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),

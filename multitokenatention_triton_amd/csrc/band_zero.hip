@@ -11,10 +11,11 @@ using namespace mta;
 typedef unsigned int bz_u4 __attribute__((ext_vector_type(4)));
 constexpr int BZ_NT = 256;
 
-// a workgroup takes BZ_ROWS consecutive rows of one plane, a wavefront a row at a time; 16-bit elements, rows of S
-// elements, S % 8 == 0
+// a workgroup takes BZ_ROWS consecutive rows of one plane, a wavefront a row at a time; rows of S elements of E bytes,
+// whole 16-byte vectors (V elements each)
 constexpr int BZ_ROWS = 32;
-__global__ __launch_bounds__(BZ_NT) void band_zero_kernel(unsigned short *__restrict__ x, const int *__restrict__ first, int C,
+template <int E>
+__global__ __launch_bounds__(BZ_NT) void band_zero_kernel(unsigned char *__restrict__ x, const int *__restrict__ first, int C,
                                                           int S, int blocks_per_plane)
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -22,21 +23,35 @@ __global__ __launch_bounds__(BZ_NT) void band_zero_kernel(unsigned short *__rest
     const int p0 = (int)(blockIdx.x % (unsigned)blocks_per_plane) * BZ_ROWS;
     const int64_t n = plane / (unsigned)C;
     const bz_u4 z = {0u, 0u, 0u, 0u};
+    constexpr int V = 16 / E;
     for (int p = p0 + wave; p < p0 + BZ_ROWS && p < S; p += BZ_NT / 64) {
         int lo = first[n * S + p];
         lo = lo < 0 ? 0 : (lo > p + 1 ? p + 1 : lo);  // (a row that sees nothing: everything up to the diagonal)
-        unsigned short *row = x + ((int64_t)plane * S + p) * S;
-        const int full = lo >> 3;  // whole vectors of 8 hidden keys
-        for (int v = lane; v < full; v += 64) *reinterpret_cast<bz_u4 *>(row + v * 8) = z;
-        const int rest = lo & 7;
+        bz_u4 *row = reinterpret_cast<bz_u4 *>(x + ((int64_t)plane * S + p) * S * E);
+        const int full = lo / V;  // whole vectors of hidden keys
+        for (int v = lane; v < full; v += 64) row[v] = z;
+        const int rest = lo % V;
         if (rest && lane == 0) {
-            bz_u4 t = *reinterpret_cast<const bz_u4 *>(row + full * 8);
+            bz_u4 t = row[full];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (e < rest) t[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
-            *reinterpret_cast<bz_u4 *>(row + full * 8) = t;
+            for (int e = 0; e < V; ++e)
+                if (e < rest) t[e * E / 4] &= E == 4 ? 0u : (e & 1) ? 0x0000ffffu : 0xffff0000u;
+            row[full] = t;
         }
     }
+}
+
+int band_zero(void *x, const void *first_visible, int64_t N, int64_t C, int64_t S, int size, void *stream)
+{
+    if (!x || !first_visible) return MTA_ERR_NULL;
+    if (N <= 0 || C <= 0 || S <= 0 || S > (1 << 24) || N * C * S > 0x7fffffffLL) return MTA_ERR_SHAPE;
+    if (!aligned_to(x, 16) || !aligned_to(first_visible, 4)) return MTA_ERR_ALIGN;
+    if (S * size % 16 != 0) return MTA_ERR_UNSUPPORTED;
+    const int64_t bpp = (S + BZ_ROWS - 1) / BZ_ROWS;
+    auto kern = size == 4 ? band_zero_kernel<4> : band_zero_kernel<2>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(N * C * bpp)), dim3(BZ_NT), 0, (hipStream_t)stream, (unsigned char *)x, (const int *)first_visible,
+                       (int)C, (int)S, (int)bpp);
+    return launch_status();
 }
 }  // namespace
 
@@ -44,11 +59,11 @@ extern "C" int mta_band_zero_fwd(void *x, const void *first_visible, int64_t N, 
 {
     if (!x || !first_visible) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
-    if (N <= 0 || C <= 0 || S <= 0 || S > (1 << 24) || N * C * S > 0x7fffffffLL) return MTA_ERR_SHAPE;
-    if (!aligned_to(x, 16) || !aligned_to(first_visible, 4)) return MTA_ERR_ALIGN;
-    if (io_dtype == MTA_F32 || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
-    const int64_t bpp = (S + BZ_ROWS - 1) / BZ_ROWS;
-    hipLaunchKernelGGL(band_zero_kernel, dim3((unsigned)(N * C * bpp)), dim3(BZ_NT), 0, (hipStream_t)stream,
-                       (unsigned short *)x, (const int *)first_visible, (int)C, (int)S, (int)bpp);
-    return launch_status();
+    if (io_dtype == MTA_F32) return MTA_ERR_UNSUPPORTED;
+    return band_zero(x, first_visible, N, C, S, 2, stream);
+}
+
+extern "C" int mta_band_zero_f32(void *x, const void *first_visible, int64_t N, int64_t C, int64_t S, void *stream)
+{
+    return band_zero(x, first_visible, N, C, S, 4, stream);
 }

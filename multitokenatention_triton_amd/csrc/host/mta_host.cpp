@@ -78,15 +78,15 @@ int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool ca
 
 // round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it.  Nothing where there is no kernel.
 // `first`: a band mask, zeros ahead of a row's first visible key (the kernel does not visit the key blocks no row of a query
-// block sees: the hidden stretch of every row is cleared afterwards).
+// block sees, fp32 visits all: the hidden stretch of every row is cleared afterwards).
 OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 {
     if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !a.is_cuda() ||
-        !lower_products_supported(a.scalar_type(), a.size(2), a.size(3), true) || (first && !is16(a)))
+        !lower_products_supported(a.scalar_type(), a.size(2), a.size(3), true))
         return std::nullopt;
     const Tensor x = on_gpu(a, "Q"), y = on_gpu(b, "K");
     Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
-    check(mta_lower_scores_fwd(ptr(x), ptr(y), ptr(first), out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
+    check(mta_lower_scores_fwd(ptr(x), ptr(y), is16(x) ? ptr(first) : nullptr, out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
           "mta_lower_scores_fwd");
     if (first) band_zero_(out, *first);
     return out;
@@ -96,9 +96,9 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 // The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
 // hides (-inf) are zeroed, so that their scores enter the pre-softmax conv as 0, and their V rows too where a post-softmax
 // conv that is not the identity writes into their columns.  `first`: int32 (B,S), a band mask (row p sees the keys
-// first[p] .. p), applied to the scores inside the first kernel and as -inf inside the softmax kernel, and behind a
+// first[p] .. p), applied to the scores inside the first kernel (where the first stage is two: between them) and as -inf inside the softmax kernel, and behind a
 // post-softmax conv that is not the identity the hidden stretch of every row is zeroed again; the caller has checked that
-// the first kernel exists.  `empty_rows`: bool (B,S), the rows of the band that see no key (first[p] = p + 1): the softmax
+// the first stage exists.  `empty_rows`: bool (B,S), the rows of the band that see no key (first[p] = p + 1): the softmax
 // leaves NaN in them, which the reference replaces by zeros ahead of its post-softmax conv
 // (mta_attention_triton.py:81) - here those rows of the probabilities are cleared ahead of a post-softmax conv that is not
 // the identity, and their rows of the output, where nothing else would, at the end.
@@ -162,9 +162,9 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         mark("qk_conv");
         scores = qk_conv(q, k, conv_w, causal, scale, false, first);
     } else {
-        TORCH_CHECK(!first, "the band mask needs the one-kernel first stage");
         mark("qk");
-        const OptTensor raw = causal ? lower_scores(q, k, OptTensor()) : OptTensor();
+        const OptTensor raw = causal ? lower_scores(q, k, first) : OptTensor();
+        TORCH_CHECK(raw || !first, "the band mask needs the lower-triangle products");
         scores = raw ? *raw : at::matmul(q, k.transpose(2, 3));
         mark("conv_pre");   // (the stage that follows never reads above the diagonal)
         scores = conv2d(scores, conv_w, causal, scale, false);
@@ -266,9 +266,9 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
             // stretch is cleared, so that the product is 0 too.
             if (o.first) band_zero_(x, *o.first);
         } else {
-            TORCH_CHECK(!o.first, "the band mask needs the one-kernel first stage");
             mark("qk");
-            const OptTensor lower_raw = o.causal ? lower_scores(q, k, OptTensor()) : OptTensor();
+            const OptTensor lower_raw = o.causal ? lower_scores(q, k, o.first) : OptTensor();
+            TORCH_CHECK(lower_raw || !o.first, "the band mask needs the lower-triangle products");
             raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
             mark("conv_pre");
             x = conv2d(raw, conv_w, o.causal, scale, false);

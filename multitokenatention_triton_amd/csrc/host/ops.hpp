@@ -218,8 +218,7 @@ inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, cons
         return std::nullopt;
     Tensor o = at::empty(v.sizes(), v.options());
     const int64_t b = v.size(0), h = v.size(1), s = v.size(2), d = v.size(3);
-    if (!is16(p)) {
-        TORCH_CHECK(!first);
+    if (!is16(p)) {   // (the hidden stretch of P holds zeros)
         check(mta_causal_pv_f32(ptr(p), ptr(v), out_ptr(o), b, h, s, d, (float)scale, stream_of(p)), "mta_causal_pv_f32");
     } else if (first) {
         TORCH_CHECK(scale == 1.0);
@@ -246,7 +245,10 @@ inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, dou
 
 inline void band_zero_(const Tensor &x, const Tensor &first)
 {
-    check(mta_band_zero_fwd(out_ptr(x), ptr(first), x.size(0), x.size(1), x.size(2), code(x, "input"), stream_of(x)), "mta_band_zero_fwd");
+    if (is16(x))
+        check(mta_band_zero_fwd(out_ptr(x), ptr(first), x.size(0), x.size(1), x.size(2), code(x, "input"), stream_of(x)), "mta_band_zero_fwd");
+    else
+        check(mta_band_zero_f32(out_ptr(x), ptr(first), x.size(0), x.size(1), x.size(2), stream_of(x)), "mta_band_zero_f32");
 }
 
 // whether the triangular-layout kernels exist (host-side questions to the library)

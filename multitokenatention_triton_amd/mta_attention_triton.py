@@ -125,6 +125,11 @@ def _lower_products_supported(x: torch.Tensor, s_keys: int) -> bool:
     return x.size(-2) == s_keys and ops.causal_pv_supported(x.dtype, s_keys, x.size(-1))
 
 
+def _lower_kernels(x: torch.Tensor) -> bool:
+    """The same question for the native routes, which pad causal lengths to a multiple of 8 and know fp32 as well."""
+    return x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.size(-1) in (64, 128)
+
+
 class _ScaledScoresConv(torch.autograd.Function):
     """conv(mask0(round(Q K^T)) * scale) for training under a mask of arbitrary content
     (mta_attention_triton.py:69-73): the raw scores are written, the hidden ones zeroed in place (``mask_planes``, uint8
@@ -561,19 +566,19 @@ class MTAAttentionTriton(nn.Module):
         return output.transpose(1, 2)
 
     def _band_supported(self, xq, xk) -> bool:
-        """Whether the first kernel takes a band mask for these tensors (lengths are padded to a multiple of 8)."""
+        """Whether the native routes take a band mask for these tensors (lengths are padded to a multiple of 8): inside the
+        first kernel, or between the raw scores and their conv where those are two kernels (fp32, weights of another dtype)."""
         w = self.mta_conv_triton.weight
-        return (xq.shape == xk.shape and xq.dtype == xk.dtype == w.dtype and xq.dtype in (torch.bfloat16, torch.float16)
-                and bool(_lib.load().mta_qk_conv_supported(8, xq.size(-1), w.size(1), w.size(2), _lib.MTA_BF16, _lib.MTA_BF16)))
+        return (xq.shape == xk.shape and xq.dtype == xk.dtype
+                and ((xq.dtype == w.dtype and xq.dtype in (torch.bfloat16, torch.float16)
+                      and bool(_lib.load().mta_qk_conv_supported(8, xq.size(-1), w.size(1), w.size(2), _lib.MTA_BF16, _lib.MTA_BF16)))
+                     or _lower_kernels(xq)))
 
     def _band_training_supported(self, xq, xk, xv) -> bool:
-        """Whether the differentiable route takes a band mask: 16-bit data of one dtype and the lower-triangle products
-        (P V and its gradients, the recomputed raw scores) as kernels."""
-        return (xq.dtype in (torch.bfloat16, torch.float16) and xq.dtype == xk.dtype == xv.dtype
-                and xq.shape == xk.shape and xv.size(-2) == xk.size(-2) and ops.causal_pv_supported(xv.dtype, 8, xv.size(-1))
-                and ops.causal_pv_supported(xq.dtype, 8, xq.size(-1))
-                and all(w.dtype == xq.dtype for w in (self.mta_conv_triton.weight, self.mta_conv_after_sm_triton.weight,
-                                                      self.wpsm_triton.weight, self.wposm_triton.weight)))
+        """Whether the differentiable route takes a band mask: data of one dtype and the lower-triangle products (P V and
+        its gradients, the recomputed raw scores) as kernels."""
+        return (xq.dtype == xk.dtype == xv.dtype and xq.shape == xk.shape and xv.size(-2) == xk.size(-2)
+                and self.wposm_triton.causal and _lower_kernels(xv) and _lower_kernels(xq))
 
     def _structured_mask(self, mask, bsz: int, s: int):
         """What a 4-D ``mask`` (bool with True = attend, or additive with 0 / -inf; one plane for all heads) amounts to

@@ -256,3 +256,49 @@ def test_row_sliding_conv(pkg, r, sk, dtype, wdtype):
             torch.testing.assert_close(got.double().cpu(), want, rtol=io, atol=size * 2.0 ** -21)
         dw = pkg.ops.conv2d_bwd_weight(xg, dyg, (r, sk), causal).double().cpu()
         assert float((dw - wa.grad).abs().max()) <= (2 * p * q) ** 0.5 * 2.0 ** -19 * 16
+
+
+@pytest.mark.parametrize("dtype,wdtype,h,s,d,kernel", [(torch.float32, torch.float32, 4, 65, 64, (5, 5)), (torch.float32, torch.float32, 16, 132, 128, (7, 9)),
+                                                       (torch.bfloat16, torch.float32, 8, 73, 64, (3, 3)), (torch.float16, torch.float32, 12, 200, 128, (6, 11))])
+@pytest.mark.parametrize("kind", ["window", "left"])
+def test_mta_band_mask_two_kernel_first_stage(pkg, dtype, wdtype, h, s, d, kernel, kind):
+    """Band masks where the scores and their conv are two kernels (fp32 data; weights of another dtype): no mask pass over the
+    scores, output and all seven gradients against the oracle given the mask tensor (left: a batch entry whose first rows see
+    nothing, forward only - the reference's gradients are NaN there)."""
+    if kind == "left" and kernel == (7, 9):
+        pytest.skip("rows that see nothing stay on the mask passes with 7x9 kernels")
+    print(f"band mask two kernels {dtype} {wdtype} h={h} s={s} d={d} {kernel} {kind}", flush=True)
+    b = 2
+    mod, params = _mta(pkg, h, kernel, (3, 3), wdtype, 61, use_mask=True)
+    rows = torch.arange(s)
+    causal = rows[None, :] <= rows[:, None]
+    mask = _ragged_mask("window", b, s)
+    if kind == "left":
+        keep = rows[None, :] >= torch.tensor([0, s // 3])[:, None]
+        mask = (keep[:, None, :] & keep[:, :, None] & causal)[:, None]
+    q, k, v = O.seeded_qkv(b, h, s, d, dtype, seed=62)
+    go = torch.randn(b, s, h, d, generator=torch.Generator().manual_seed(63)).to(dtype)
+    leaves = [t.clone().float().requires_grad_(True) for t in (q, k, v)]
+    wl = [p.clone().float().requires_grad_(True) for p in params]
+    want = O.mta_forward(*leaves, wl[0].unsqueeze(1), wl[1], wl[2].unsqueeze(1), wl[3], mask=torch.where(mask, 0.0, float("-inf")).expand(b, h, s, s))
+    dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    stages = []
+    mod._stage_hook = stages.append
+    with torch.no_grad():
+        plain = mod(*dev, mask.cuda(), None)
+    out = mod(*dev, mask.cuda(), None)
+    assert "mask" not in stages and stages.count("pv") == 2, stages
+    # the oracle computes in fp32 throughout: a chain of about six roundings to the data type (2^-9 / 2^-12 each) in the norm
+    rel = {torch.float32: 1e-5, torch.bfloat16: 1.5e-2, torch.float16: 2e-3}[dtype]
+    for got in (plain, out.detach()):
+        assert float((got.float().cpu() - want.detach()).norm()) <= rel * float(want.detach().norm())
+    if kind == "left":
+        assert not out[1, :s // 3].any()
+        return
+    want.backward(go.float())
+    out.backward(go.cuda())
+    rel = {torch.float32: 1e-4, torch.bfloat16: 4e-2, torch.float16: 1e-2}[dtype]   # (as in test_mta_padded_lengths)
+    got = [t.grad for t in dev] + [m.weight.grad for m in (mod.mta_conv_triton, mod.wpsm_triton, mod.mta_conv_after_sm_triton, mod.wposm_triton)]
+    for name, a, w in zip("q k v conv pre conv2 post".split(), got, [t.grad for t in leaves + wl]):
+        assert torch.isfinite(a.float()).all(), name
+        assert float((a.float().cpu() - w).norm()) <= rel * float(w.norm()) + 1e-5, name
