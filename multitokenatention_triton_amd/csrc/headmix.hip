@@ -20,10 +20,12 @@ constexpr int NT = 256;
 
 template <typename T, int VEC> struct alignas(sizeof(T) * VEC) vecN { T v[VEC]; };
 
-// inputs are read once and outputs written once by this kernel: move them as streaming (non-temporal) data
-template <typename V> __device__ __forceinline__ V load_stream(const V *src)
+// Inputs are read once and outputs written once by these kernels.  The outputs are written as streaming (non-temporal) data;
+// the inputs are read so where the tensor is too large for the memory-side cache to still hold what its producer wrote, and
+// as ordinary data where it is not (STREAM, see streams()).
+template <bool STREAM, typename V> __device__ __forceinline__ V load_as(const V *src)
 {
-    if constexpr (sizeof(V) == 16) {
+    if constexpr (STREAM && sizeof(V) == 16) {
         typedef unsigned int u4 __attribute__((ext_vector_type(4)));
         return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const u4 *>(src)));
     }
@@ -60,7 +62,7 @@ __device__ __forceinline__ int rotated_chunk(unsigned &id, unsigned qchunks)
 
 // G heads mixed inside one lane, G known at compile time.  A workgroup covers one query row of one key chunk: on this
 // part the fewer independent streams a wavefront holds, the higher the delivered bandwidth.
-template <typename T, int G, int VEC>
+template <typename T, int G, int VEC, bool STREAM>
 __global__ __launch_bounds__(NT) void headmix_fixed(const T *__restrict__ x, const void *__restrict__ w,
                                                     T *__restrict__ y, int C, int P, int Q, int causal,
                                                     float fill, int w_dtype, int wt, int qchunks)
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(NT) void headmix_fixed(const T *__restrict__ x, con
         const bool live = q < Q && !(causal && q > p);
         const int64_t lb = base - (live ? 0 : q);
 #pragma unroll
-        for (int i = 0; i < G; ++i) xin[i] = load_stream(reinterpret_cast<const V *>(x + lb + i * plane));
+        for (int i = 0; i < G; ++i) xin[i] = load_as<STREAM>(reinterpret_cast<const V *>(x + lb + i * plane));
     }
     for (int t = tid; t < G * G; t += NT) wsm[t] = load_any(w, w_dtype, w_index(g * G + t / G, g * G + t % G, C, wt));
     __syncthreads();
@@ -341,7 +343,7 @@ __device__ __forceinline__ f32x4 hm_mma16(f16_t, hm_u2 a, hm_u2 b)
                                                  f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
 
-template <typename T, int HG>
+template <typename T, int HG, bool STREAM>
 __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__restrict__ x, const T *__restrict__ w,
                                                                T *__restrict__ y, int C, int P, int Q, int causal,
                                                                float fill, int wt, int qchunks)
@@ -373,12 +375,16 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
         return;
     }
 
-    // (HG = 12: the fourth lane group re-reads the first heads, its weights are 0 and it stores nothing)
+    // (HG = 12: the fourth lane group re-reads the first heads, its weights and inputs count as 0 and it stores nothing)
     const int kgc = kg * 4 < HG ? kg : 0;
     const T *xp = x + base + (int64_t)(kgc * 4) * plane + (key <= last ? key : 0);
     u4 xv[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) xv[t] = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(xp + t * plane));
+    for (int t = 0; t < 4; ++t) xv[t] = load_as<STREAM>(reinterpret_cast<const u4 *>(xp + t * plane));
+    if (HG < 16 && kg * 4 >= HG) {   // (0 times an infinity would reach every output head)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) xv[t] = u4{0u, 0u, 0u, 0u};
+    }
 
     // w fragment: lane (output head ln, group kg) holds w[o][4kg .. 4kg+3]
     hm_u2 wf;
@@ -457,10 +463,16 @@ __global__ __launch_bounds__(NT) void headmix_any(const T *__restrict__ x, const
     }
 }
 
+// Whether a tensor is larger than the memory-side cache (256 MB).  Non-temporal loads | ordinary loads, us, bf16 dense 16 heads,
+// the lower triangle of a tensor that the kernel ahead has just written: B2 S1008 (65 MB) 21.4 | 13.7, B1 S2048 (134 MB)
+// 38.7 | 24.6 (cold: 36.5 | 30.3), B1 S4096 (537 MB) 127 | 136.
+inline bool streams(int64_t N, int64_t C, int64_t P, int64_t Q, size_t size) { return N * C * P * Q * (int64_t)size > (256 << 20); }
+
 template <typename T, int VEC>
 int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t P, int64_t Q, int G, int causal,
            float fill, int w_dtype, int wt, bool w_same_dtype, hipStream_t st)
 {
+    const bool stream = VEC > 1 && streams(N, C, P, Q, sizeof(T));
     if constexpr (VEC == 8) {
         // 16 or 32 heads mixed densely, 16-bit data and weights of the same dtype: matrix cores
         // (MTA_HEADMIX_NO_MFMA=1 in the environment keeps the vector-ALU kernel, for comparisons)
@@ -469,7 +481,8 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
             const int qch = (int)((Q + DM_WAVES * DM_KEYS - 1) / (DM_WAVES * DM_KEYS));
             const int64_t blocks = N * (C / G) * P * qch;
             if (blocks > 0x7fffffffLL) return MTA_ERR_SHAPE;
-            auto kern = G == 16 ? headmix_dense16<T, 16> : headmix_dense16<T, 12>;
+            auto kern = G == 16 ? (stream ? headmix_dense16<T, 16, true> : headmix_dense16<T, 16, false>)
+                                : (stream ? headmix_dense16<T, 12, true> : headmix_dense16<T, 12, false>);
             hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * DM_WAVES), 0, st, (const T *)x,
                                (const T *)w, (T *)y, (int)C, (int)P, (int)Q, causal, fill, wt, qch);
             return launch_status();
@@ -501,8 +514,9 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
     if (G == g) {                                                                                              \
         const int64_t blocks = N * (C / G) * P * qchunks;                                                      \
         if (blocks > 0x7fffffffLL) return MTA_ERR_SHAPE;                                                       \
-        hipLaunchKernelGGL((headmix_fixed<T, g, VEC>), dim3((unsigned)blocks), dim3(NT), 0, st, (const T *)x, w, \
-                           (T *)y, (int)C, (int)P, (int)Q, causal, fill, w_dtype, wt, qchunks);                 \
+        auto kern = stream ? headmix_fixed<T, g, VEC, (VEC > 1)> : headmix_fixed<T, g, VEC, false>;            \
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NT), 0, st, (const T *)x, w, (T *)y, (int)C, (int)P, (int)Q, \
+                           causal, fill, w_dtype, wt, qchunks);                                                \
         return launch_status();                                                                                \
     }
     MTA_HM_CASE(1)

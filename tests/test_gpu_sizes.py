@@ -302,3 +302,15 @@ def test_mta_band_mask_two_kernel_first_stage(pkg, dtype, wdtype, h, s, d, kerne
     for name, a, w in zip("q k v conv pre conv2 post".split(), got, [t.grad for t in leaves + wl]):
         assert torch.isfinite(a.float()).all(), name
         assert float((a.float().cpu() - w).norm()) <= rel * float(w.norm()) + 1e-5, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_headmix_twelve_heads_infinity(pkg, dtype):
+    """An infinite score of one head and key: the output heads hold +-inf there (w has no zeros), as the sum of 12 products
+    does - not NaN, which an operand row without a head would make of it (0 * inf)."""
+    g = torch.Generator().manual_seed(8)
+    x, w = torch.randn(1, 12, 16, 16, generator=g).to(dtype), (torch.rand(12, 12, generator=g) + 0.5).to(dtype)
+    x[0, 0, 9, 4] = float("inf")
+    got = pkg.ops.headmix(x.cuda(), w.cuda(), True, 0.0).cpu()
+    assert (got[0, :, 9, 4] == float("inf")).all()
+    assert torch.isfinite(got[0, :, 9, [0, 3, 5]]).all() and torch.isfinite(got[0, :, 8]).all()
