@@ -8,7 +8,7 @@
 // torch's kernel writes out first) reaches memory.  Above the diagonal nothing is read; dx there is +0 (fill_upper) or
 // left alone for a consumer that never reads it.
 //
-// One workgroup per row.  16-bit rows of whole 16-byte vectors up to 8192 keys stay in registers between the sum and
+// One workgroup per row.  Rows of whole 16-byte vectors up to 8192 keys stay in registers between the sum and
 // the result (one read of p and dp); everything else takes two sweeps over the row.
 #include "common.hpp"
 
@@ -32,11 +32,32 @@ __device__ __forceinline__ float block_sum(float v, float *red)
 
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-// NV = 16-byte vectors per thread: rows of up to NV * 2048 keys
-template <typename T, int NV>
-__global__ __launch_bounds__(NT) void softmax_bwd_rows16(const T *__restrict__ p, const T *__restrict__ dp,
-                                                         T *__restrict__ dx, int P, int Q, int causal, int fill_upper)
+// a 16-byte vector as fp32 values, and back
+template <typename T> __device__ __forceinline__ void widen(const u4 &v, float (&f)[vec_of<T>::n])
 {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if constexpr (vec_of<T>::n == 8) unpack2<T>(v[u], f[2 * u], f[2 * u + 1]);
+        else f[u] = __uint_as_float(v[u]);
+    }
+}
+template <typename T> __device__ __forceinline__ u4 narrow(const float (&f)[vec_of<T>::n])
+{
+    u4 v;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if constexpr (vec_of<T>::n == 8) v[u] = pack2<T>(f[2 * u], f[2 * u + 1]);
+        else v[u] = __float_as_uint(f[u]);
+    }
+    return v;
+}
+
+// NV = 16-byte vectors per thread: rows of up to NV * 256 vectors
+template <typename T, int NV>
+__global__ __launch_bounds__(NT) void softmax_bwd_rows(const T *__restrict__ p, const T *__restrict__ dp,
+                                                       T *__restrict__ dx, int P, int Q, int causal, int fill_upper)
+{
+    constexpr int V = vec_of<T>::n;
     __shared__ float red[NT / 64];
     const int64_t row = blockIdx.x;
     const int pr = (int)(row % P);
@@ -49,23 +70,20 @@ __global__ __launch_bounds__(NT) void softmax_bwd_rows16(const T *__restrict__ p
     u4 pv[NV], gv[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int q0 = (v * NT + tid) * 8;
+        const int q0 = (v * NT + tid) * V;
         const int qq = q0 <= last ? q0 : 0;
         pv[v] = *reinterpret_cast<const u4 *>(prow + qq);
         gv[v] = *reinterpret_cast<const u4 *>(grow + qq);
     }
-    float pf[NV][8], gf[NV][8];
+    float pf[NV][V], gf[NV][V];
     float dot = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int q0 = (v * NT + tid) * 8;
+        const int q0 = (v * NT + tid) * V;
+        widen<T>(pv[v], pf[v]);
+        widen<T>(gv[v], gf[v]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            unpack2<T>(pv[v][u], pf[v][2 * u], pf[v][2 * u + 1]);
-            unpack2<T>(gv[v][u], gf[v][2 * u], gf[v][2 * u + 1]);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < V; ++e) {
             const bool in = q0 + e <= last;  // what lies beyond need not even be finite
             pf[v][e] = in ? pf[v][e] : 0.0f;
             gf[v][e] = in ? gf[v][e] : 0.0f;
@@ -75,16 +93,13 @@ __global__ __launch_bounds__(NT) void softmax_bwd_rows16(const T *__restrict__ p
     dot = block_sum(dot, red);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const int q0 = (v * NT + tid) * 8;
+        const int q0 = (v * NT + tid) * V;
         if (q0 >= Q) continue;
         if (q0 > last && !fill_upper) continue;
-        float r[8];
+        float r[V];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r[e] = q0 + e <= last ? pf[v][e] * (gf[v][e] - dot) : 0.0f;  // +0 beyond the row's end
-        u4 out;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) out[u] = pack2<T>(r[2 * u], r[2 * u + 1]);
-        *reinterpret_cast<u4 *>(xrow + q0) = out;
+        for (int e = 0; e < V; ++e) r[e] = q0 + e <= last ? pf[v][e] * (gf[v][e] - dot) : 0.0f;  // +0 beyond the row's end
+        *reinterpret_cast<u4 *>(xrow + q0) = narrow<T>(r);
     }
 }
 
@@ -119,21 +134,18 @@ extern "C" int mta_softmax_bwd(const void *p, const void *dp, void *dx, int64_t 
     if (rows > 0x7fffffffLL) return MTA_ERR_SHAPE;
     if (!aligned_to(p, es) || !aligned_to(dp, es) || !aligned_to(dx, es)) return MTA_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    const bool vec = es == 2 && Q % 8 == 0 && Q <= 8192 && aligned_to(p, 16) && aligned_to(dp, 16) && aligned_to(dx, 16);
     MTA_DISPATCH_IO(io_dtype, {
-        if constexpr (sizeof(io_t) == 2) {
-            if (vec) {
-                if (Q <= 2048)
-                    hipLaunchKernelGGL((softmax_bwd_rows16<io_t, 1>), dim3((unsigned)rows), dim3(NT), 0, st, (const io_t *)p,
-                                       (const io_t *)dp, (io_t *)dx, (int)P, (int)Q, causal, fill_upper);
-                else if (Q <= 4096)
-                    hipLaunchKernelGGL((softmax_bwd_rows16<io_t, 2>), dim3((unsigned)rows), dim3(NT), 0, st, (const io_t *)p,
-                                       (const io_t *)dp, (io_t *)dx, (int)P, (int)Q, causal, fill_upper);
-                else
-                    hipLaunchKernelGGL((softmax_bwd_rows16<io_t, 4>), dim3((unsigned)rows), dim3(NT), 0, st, (const io_t *)p,
-                                       (const io_t *)dp, (io_t *)dx, (int)P, (int)Q, causal, fill_upper);
-                return launch_status();
-            }
+        constexpr int V = vec_of<io_t>::n;
+        if (Q % V == 0 && Q <= 8192 && aligned_to(p, 16) && aligned_to(dp, 16) && aligned_to(dx, 16)) {
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(NT), 0, st, (const io_t *)p, (const io_t *)dp, (io_t *)dx, (int)P, (int)Q,
+                                   causal, fill_upper);
+            };
+            if (Q <= NT * V) go(softmax_bwd_rows<io_t, 1>);
+            else if (Q <= 2 * NT * V) go(softmax_bwd_rows<io_t, 2>);
+            else if (Q <= 4 * NT * V) go(softmax_bwd_rows<io_t, 4>);
+            else go(softmax_bwd_rows<io_t, 32 / V>);
+            return launch_status();
         }
         hipLaunchKernelGGL((softmax_bwd_rows_any<io_t>), dim3((unsigned)rows), dim3(NT), 0, st, (const io_t *)p,
                            (const io_t *)dp, (io_t *)dx, (int)P, (int)Q, causal, fill_upper);

@@ -314,3 +314,18 @@ def test_headmix_twelve_heads_infinity(pkg, dtype):
     got = pkg.ops.headmix(x.cuda(), w.cuda(), True, 0.0).cpu()
     assert (got[0, :, 9, 4] == float("inf")).all()
     assert torch.isfinite(got[0, :, 9, [0, 3, 5]]).all() and torch.isfinite(got[0, :, 8]).all()
+
+
+def test_fp32_softmax_gradient_sizes(pkg):
+    """fp32 rows in registers (up to 8192 keys of whole vectors) and in two sweeps: edges of the instances, NaN above the
+    diagonal.  Against float64: the order of the row's sum of p * dp, sum of |p * dp| at most about 4."""
+    g = torch.Generator().manual_seed(23)
+    for p, q, causal in ((1, 4, True), (68, 68, True), (67, 67, True), (3, 1024, False), (3, 1028, False), (2, 2052, False), (2, 4100, False), (2, 8192, False), (2, 8196, False)):
+        print(f"fp32 softmax gradient {p}x{q} causal={causal}", flush=True)
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        prob = torch.softmax(torch.randn(2, 3, p, q, generator=g).masked_fill(~keep, float("-inf")), -1)
+        dp = torch.randn(2, 3, p, q, generator=g)
+        pd, gd = prob.double(), dp.double().masked_fill(~keep, 0.0)
+        want = pd * (gd - (pd * gd).sum(-1, keepdim=True))
+        got = pkg.ops.softmax_bwd(prob.masked_fill(~keep, float("nan")).cuda(), dp.masked_fill(~keep, float("nan")).cuda(), causal)
+        torch.testing.assert_close(got.double().cpu(), want, rtol=1e-5, atol=2e-6)
