@@ -133,7 +133,7 @@ __device__ __forceinline__ void hm_consume(f32x4 (&acc)[NB][NB], hm_operands<T, 
 
 template <typename T, int NB, int SETS, bool ALIGNED>
 __global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restrict__ x, const T *__restrict__ dy, float *__restrict__ partial,
-                                                              int N, int C, int P, int Q, int causal)
+                                                              int N, int C, int P, int Q, int causal, int slots)
 {
     using G = hm_shape<T, NB, SETS>;
     constexpr int LD = 16 * NB;
@@ -146,42 +146,56 @@ __global__ __launch_bounds__(NT) void headmix_bwd_weight_mfma(const T *__restric
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int64_t rows = (int64_t)N * P;
-    const int64_t nwaves = (int64_t)gridDim.x * (NT / 64), wid = (int64_t)wave * gridDim.x + blockIdx.x;
-    // A wavefront takes pairs of rows (2k, 2k+1) of the interleaved order, k = wid, wid + nwaves, ...; j counts its
-    // rows.  The chunks of all its rows form one sequence, and the loads of a chunk are issued before the products of
-    // the chunk ahead of it (two operand sets take turns).  (Four wavefronts sharing a row chunk by chunk measured
-    // slower: short rows leave most of them without work.)
-    int64_t j = 0;
-    int q0 = 0;
-    auto unit_at = [&](hm_unit &u) -> bool {
-        const int64_t rid = 2 * (wid + (j >> 1) * nwaves) + (j & 1);
-        if (rid >= rows) return false;
-        const int n = (int)(rid / P), p = interleaved_row((int)(rid % P), P);
-        u.last = causal ? (p < Q - 1 ? p : Q - 1) : Q - 1;  // last position of the row that takes part
-        u.rowbase = (int64_t)n * C * plane + (int64_t)p * Q;
-        u.q0 = q0;
-        return true;
-    };
-    auto advance = [&](const hm_unit &u) {
-        q0 += G::CHUNK;
-        if (q0 > u.last) {
-            q0 = 0;
-            ++j;
+    // Rows are taken in pairs (2k, 2k+1) of the interleaved order, a pair's chunks one after the other in `slots` places (the
+    // most a pair has; few are empty), and the places of all pairs are dealt to the wavefronts one by one: wavefront i takes
+    // the places i, i + nwaves, ... - the same number of chunks for each whatever the length, and neighbours read side by side.
+    // The loads of a chunk are issued before the products of the chunk ahead of it (two operand sets take turns).
+    const int64_t rows = (int64_t)N * P, pairs = (rows + 1) / 2;
+    const int nwaves = gridDim.x * (NT / 64), wid = __builtin_amdgcn_readfirstlane(blockIdx.x * (NT / 64) + wave);
+    const int pair_step = nwaves / slots, slot_step = nwaves % slots;
+    int64_t k = wid / slots;
+    int i = wid % slots;
+    auto advance = [&] {
+        k += pair_step;
+        i += slot_step;
+        if (i >= slots) {
+            i -= slots;
+            ++k;
         }
+    };
+    // the chunk of the place at or after (k, i); false where nothing is left
+    auto unit_at = [&](hm_unit &u) -> bool {
+        while (k < pairs) {
+            int c = i;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int64_t rid = 2 * k + half;
+                if (rid >= rows) break;
+                const int n = (int)(rid / P), p = interleaved_row((int)(rid % P), P);
+                u.last = causal ? (p < Q - 1 ? p : Q - 1) : Q - 1;  // last position of the row that takes part
+                if (c * G::CHUNK <= u.last) {
+                    u.rowbase = (int64_t)n * C * plane + (int64_t)p * Q;
+                    u.q0 = c * G::CHUNK;
+                    return true;
+                }
+                c -= u.last / G::CHUNK + 1;
+            }
+            advance();
+        }
+        return false;
     };
     hm_unit ua, ub;
     hm_operands<T, NB, SETS> oa, ob;
     bool ha = unit_at(ua);
     if (ha) hm_load<T, NB, SETS, ALIGNED>(oa, x, dy, ua, plane, C, r, g, total);
     while (ha) {
-        advance(ua);
+        advance();
         const bool hb = unit_at(ub);
         if (!hb) ub = ua;  // nothing follows: fetch the same chunk again, so that the loads in flight never depend on a branch
         hm_load<T, NB, SETS, ALIGNED>(ob, x, dy, ub, plane, C, r, g, total);
         hm_consume<T, NB, SETS>(acc, oa, ua, r, g);
         if (!hb) break;
-        advance(ub);
+        advance();
         ha = unit_at(ua);
         if (!ha) ua = ub;
         hm_load<T, NB, SETS, ALIGNED>(oa, x, dy, ua, plane, C, r, g, total);
@@ -282,12 +296,14 @@ __global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *
 
 constexpr int64_t MAX_WS_BYTES = 8 << 20;  // partial matrices never take more than this
 
-// persistent workgroups (= partial matrices) for a problem
+// Persistent workgroups (= partial matrices) for a problem, at most.  Matrix-core kernels: one per CU, which has 64 to 128 KB
+// of loads in flight; more is slower (256 | 512 | 1024, us: bf16 B1 H16 S1024 10.2 | 11.6 | 13.2, S2048 25.9 | 28.9 | 34.0, B2 H32
+// S2048 112 | 115 | 122, fp32 B1 H32 S1024 27.8 | 34.2 | 40.0).  launch_partials takes fewer where there are fewer chunks.
 inline int num_blocks(int64_t N, int64_t C, int64_t P, int64_t Q)
 {
-    int64_t nb = 1024;
+    int64_t nb = C <= 32 ? 256 : 1024;
     const int64_t pairs = (N * P + 1) / 2;
-    if (nb > pairs) nb = pairs;
+    if (C > 32 && nb > pairs) nb = pairs;
     const int64_t cap = MAX_WS_BYTES / (C * C * (int64_t)sizeof(float));
     if (nb > cap) nb = cap;
     return (int)(nb < 1 ? 1 : nb);
@@ -302,13 +318,20 @@ extern "C" int64_t mta_headmix_bwd_weight_workspace(int64_t N, int64_t C, int64_
 
 namespace {
 template <typename T>
-int launch_partials(const T *x, const T *dy, float *partial, int nb, int N, int C, int P, int Q, int causal, hipStream_t st)
+int launch_partials(const T *x, const T *dy, float *partial, int &nb, int N, int C, int P, int Q, int causal, hipStream_t st)
 {
     if (C <= 32) {
         const bool aligned = Q % vec_of<T>::n == 0 && aligned_to(x, 16) && aligned_to(dy, 16);
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(NT), 0, st, x, dy, partial, N, C, P, Q, causal); };
-#define MTA_HM_CASE(nb_, sets)                                                  \
-    aligned ? go(headmix_bwd_weight_mfma<T, nb_, sets, true>) : go(headmix_bwd_weight_mfma<T, nb_, sets, false>)
+        auto go = [&](auto kern, int chunk) {
+            // the most chunks that the two rows of a pair have: together they hold at most P + 2 attended positions when causal
+            const int full = 2 * ((Q + chunk - 1) / chunk), slots = causal && P / chunk + 2 < full ? P / chunk + 2 : full;
+            const int64_t places = ((int64_t)N * P + 1) / 2 * slots, enough = (places + NT / 64 - 1) / (NT / 64);
+            if (nb > enough) nb = (int)enough;
+            hipLaunchKernelGGL(kern, dim3(nb), dim3(NT), 0, st, x, dy, partial, N, C, P, Q, causal, slots);
+        };
+#define MTA_HM_CASE(nb_, sets)                                                                    \
+    aligned ? go(headmix_bwd_weight_mfma<T, nb_, sets, true>, hm_shape<T, nb_, sets>::CHUNK)      \
+            : go(headmix_bwd_weight_mfma<T, nb_, sets, false>, hm_shape<T, nb_, sets>::CHUNK)
         if (C <= 4) MTA_HM_CASE(1, 4);
         else if (C <= 8) MTA_HM_CASE(1, 2);
         else if (C <= 16) MTA_HM_CASE(1, 1);
@@ -338,7 +361,7 @@ extern "C" int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw
     if (!aligned_to(x, dtype_size(io_dtype)) || !aligned_to(dy, dtype_size(io_dtype)) || !aligned_to(dw, dtype_size(w_dtype)) ||
         !aligned_to(workspace, 16))
         return MTA_ERR_ALIGN;
-    const int nb = num_blocks(N, C, P, Q);
+    int nb = num_blocks(N, C, P, Q);
     if (workspace_bytes < (int64_t)nb * C * C * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
     float *partial = (float *)workspace;
