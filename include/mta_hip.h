@@ -151,6 +151,10 @@ int mta_headmix_softmax_band_fwd(const void *x, const void *w1, const void *w2, 
                                  const void *first_visible, void *y, int64_t N, int64_t C, int64_t P, int64_t Q,
                                  int group_size, int causal, int fill_upper, int io_dtype, int w_dtype, void *stream);
 
+/* Longest row that the entry points above take in one pass over memory for fp32 scores in dense groups of `group_size`
+ * heads (rows of whole 16-byte vectors, 16-byte aligned tensors); 0: no such kernel for this group size. */
+int64_t mta_headmix_softmax_dense_f32_keys(int group_size);
+
 /* Depthwise causal conv followed by head mixing, the conv result never written:
  *   t[h] = round(conv2d(x[h], w_conv[h]))                     as mta_conv2d_fwd
  *   y[o] = round(sum_h w_mix[o,h] t[h])                        as mta_headmix_fwd with fill 0

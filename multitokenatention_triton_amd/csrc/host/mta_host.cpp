@@ -26,12 +26,16 @@ bool no_row_lists()
 bool one_pass_group(int64_t group, at::ScalarType t, int64_t n_keys, const OptTensor &w1, const OptTensor &w2)
 {
     if (group <= FUSED_MAX_GROUP) return true;
+    if (t == at::kFloat) return n_keys % 4 == 0 && n_keys <= mta_headmix_softmax_dense_f32_keys((int)std::min<int64_t>(group, 1 << 20));
     return group == FUSED_MFMA_GROUP && (t == at::kBFloat16 || t == at::kHalf) && n_keys % 8 == 0 && n_keys <= FUSED_MFMA_MAX_KEYS &&
            (!w1 || w1->scalar_type() == t) && (!w2 || w2->scalar_type() == t);
 }
 
-// the matrix-core variant for groups of 16 takes a key bias or a band mask in its row-list form only
-bool masks_ok(int64_t group, bool masked) { return !masked || group <= FUSED_MAX_GROUP || (group == FUSED_MFMA_GROUP && !no_row_lists()); }
+// the 16-bit matrix-core variant for groups of 16 takes a key bias or a band mask in its row-list form only
+bool masks_ok(int64_t group, at::ScalarType t, bool masked)
+{
+    return !masked || group <= FUSED_MAX_GROUP || t == at::kFloat || (group == FUSED_MFMA_GROUP && !no_row_lists());
+}
 
 int64_t lcm(int64_t a, int64_t b)
 {
@@ -128,7 +132,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const int64_t g_both = lcm(g_pre, g_post);
     const bool masked = key_bias || first;
     const auto dtype = q.scalar_type();
-    const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, masked);
+    const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
     const bool own_pv = q.size(-2) == n_keys && dtype == v.scalar_type() && lower_products_supported(dtype, q.size(-2), v.size(-1), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
@@ -152,7 +156,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     Tensor scores;
     // (dense groups of 16 heads ahead of a post-softmax conv: the first score tensor still travels in the triangular layout,
     // the softmax stage hands the conv (B,H,S,S) planes)
-    const bool tri_first = !planes && causal && !one_pass && g_pre == 16 && masks_ok(16, masked) && w1 &&
+    const bool tri_first = !planes && causal && !one_pass && g_pre == 16 && masks_ok(16, dtype, masked) && w1 &&
                            !(post_conv_identity && !w2 && !own_pv) &&
                            tri_route_supported(q, k, conv_w, 16, w1, OptTensor(), first.has_value(), true, key_bias.has_value());
     if (tri_first) {
@@ -178,7 +182,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         if (tri_first) {
             mark("mix_softmax");
             scores = headmix_softmax_tri(scores, w1, OptTensor(), q.size(0), heads, n_keys, g_pre, first, true, key_bias);
-        } else if (one_pass_group(g_pre, dtype, n_keys, w1, OptTensor()) && masks_ok(g_pre, masked)) {
+        } else if (one_pass_group(g_pre, dtype, n_keys, w1, OptTensor()) && masks_ok(g_pre, dtype, masked)) {
             mark("mix_softmax");
             scores = headmix_softmax(scores, w1, OptTensor(), causal, g_pre, fill, key_bias, first);
         } else {
@@ -275,7 +279,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         }
         const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
         Tensor p;
-        if (one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, o.key_bias || o.first)) {
+        if (one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), o.key_bias || o.first)) {
             mark("mix_softmax");
             p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
         } else {

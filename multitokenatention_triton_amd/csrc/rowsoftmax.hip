@@ -23,6 +23,9 @@ namespace mta {
 int mix16_softmax_launch(const void *x, const void *w1, const void *w2, void *y, int64_t N, int64_t C, int64_t P, int64_t Q,
                          int causal, int fill_upper, int io_dtype, int w_dtype, hipStream_t st, int tri_in = 0, int tri_out = 0,
                          const float *key_bias = nullptr, const int *row_lo = nullptr);
+// rowsoftmax_dense_f32.hip: the same pass for fp32 and groups of 9 to 32 heads
+int mix_softmax_dense_f32_launch(const float *x, const void *w1, const void *w2, const float *kb, const int *row_lo, float *y, int64_t N,
+                                 int64_t C, int64_t P, int64_t Q, int HG, int causal, int w_dtype, int fill_upper, hipStream_t st);
 }  // namespace mta
 
 namespace {
@@ -1018,6 +1021,11 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         }
     }
     if (tri_in || tri_out) return MTA_ERR_UNSUPPORTED;  // (only the kernels above know the triangular layout)
+    if constexpr (std::is_same<T, float>::value) {
+        const int rc = mix_softmax_dense_f32_launch((const float *)x, w1, w2, kb_in, row_lo, (float *)y, N, C, P, Q, G, causal,
+                                                    w_dtype, fill_upper, st);
+        if (rc != MTA_ERR_UNSUPPORTED) return rc;
+    }
     if constexpr (sizeof(T) == 2) {
         // no weights, short rows: a wavefront per row (MTA_SOFTMAX_NO_WAVE_ROWS=1 keeps a workgroup per row, for comparisons)
         static const bool no_wave = [] { const char *e_ = getenv("MTA_SOFTMAX_NO_WAVE_ROWS"); return e_ && e_[0] == '1'; }();

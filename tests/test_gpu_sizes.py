@@ -316,6 +316,47 @@ def test_headmix_twelve_heads_infinity(pkg, dtype):
     assert torch.isfinite(got[0, :, 9, [0, 3, 5]]).all() and torch.isfinite(got[0, :, 8]).all()
 
 
+@pytest.mark.parametrize("masked", [None, "bias", "band"])
+@pytest.mark.parametrize("h", [9, 12, 16, 32])
+def test_fp32_dense_mix_softmax_mix(pkg, h, masked):
+    """mix -> softmax -> mix of fp32 scores in dense groups, with either weight, both or a bf16 one: lengths around the edges of
+    the 64-key passes and of every instance, non-causal rows, a key bias that hides keys, a band mask.  Against float64: a
+    score's sum is off by at most h * 2^-24 * 4, which the exponential turns into a relative error of its own size (< 1e-5)."""
+    g = torch.Generator().manual_seed(22)
+    longest = 4096 if h <= 16 else 2048
+    for p, q, causal in ((1, 4, True), (64, 64, True), (132, 132, True), (260, 260, True), (7, 516, False), (3, 1028, False), (2, longest, False)):
+        if masked == "band" and not causal:
+            continue
+        print(f"fp32 dense softmax h={h} {p}x{q} causal={causal} {masked}", flush=True)
+        n, c = (2, 2 * h) if p < 200 else (1, h)
+        x = 2.0 * torch.randn(n, c, p, q, generator=g)
+        keep = (torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)).expand(n, 1, p, q)
+        first, bias = None, None
+        if masked == "band":
+            first = (torch.arange(p).expand(n, p) - torch.tensor([[5], [70]])[:n]).clamp(min=0).to(torch.int32)
+            keep = keep & (torch.arange(q) >= first[:, None, :, None])
+        if masked == "bias":
+            bias = torch.randn(n, q, generator=g)
+            bias[:, q // 2:q // 2 + 2] = float("-inf")
+            bias[:, 0] = 0.5   # (every row sees a key)
+        weights = [torch.block_diag(*[torch.eye(h) + 0.2 * torch.randn(h, h, generator=g) for _ in range(c // h)]) for _ in range(2)]
+        below = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        xd = x.masked_fill(~below, float("nan")).cuda()
+        for one, two, wdtype in ((True, False, torch.float32), (False, True, torch.float32), (True, True, torch.float32), (True, True, torch.bfloat16)):
+            w1, w2 = (w.to(wdtype) if use else None for w, use in zip(weights, (one, two)))
+            s = x.double().masked_fill(~keep, 0.0)
+            if one:
+                s = torch.einsum("oi,nipq->nopq", w1.double(), s)
+            if bias is not None:
+                s = s + bias.double()[:, None, None, :]
+            s = torch.softmax(s.masked_fill(~keep, float("-inf")), -1)
+            if two:
+                s = torch.einsum("oi,nipq->nopq", w2.double(), s)
+            got = pkg.ops.headmix_softmax(xd, None if w1 is None else w1.cuda(), None if w2 is None else w2.cuda(), causal, group_size=h,
+                                          key_bias=None if bias is None else bias.cuda(), first_visible=None if first is None else first.cuda())
+            torch.testing.assert_close(got.double().cpu(), s, rtol=1e-5, atol=1e-6)
+
+
 def test_fp32_softmax_gradient_sizes(pkg):
     """fp32 rows in registers (up to 8192 keys of whole vectors) and in two sweeps: edges of the instances, NaN above the
     diagonal.  Against float64: the order of the row's sum of p * dp, sum of |p * dp| at most about 4."""
