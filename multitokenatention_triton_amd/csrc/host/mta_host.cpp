@@ -37,6 +37,16 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
     return !masked || group <= FUSED_MAX_GROUP || t == at::kFloat || (group == FUSED_MFMA_GROUP && !no_row_lists());
 }
 
+// Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
+// heads at about 20 us each, so that two full rounds of tiles are where it meets the two kernels one after the other (us, one
+// kernel | two, 3x3 / 7x7: B1 S512 25 | 12 / 28 | 14, B1 S1024 27 | 21 / 32 | 26, B2 S1008 39 | 41 / 46 | 49, B1 S1536 49 | 39 / 54 | 47,
+// B1 S2048 54 | 67 / 63 | 80, B4 S1024 51 | 70 / 60 | 83).
+bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only)
+{
+    const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64;
+    return planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk) >= 2 * 512;
+}
+
 int64_t lcm(int64_t a, int64_t b)
 {
     int64_t x = a, y = b;
@@ -196,7 +206,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         // kernels (mixing groups of up to 4 heads and the sizes with a vector-staged instance; dense groups of 16).  Under a
         // band mask the conv's result is zeroed at the hidden positions ahead of the mixing: two kernels.
         const int64_t r = post_conv_w.size(1), s = post_conv_w.size(2);
-        const bool mix16 = g_post == 16 && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
+        const bool mix16 = g_post == 16 && conv_mix16_fills(q.size(0) * (heads / 16), q.size(2), n_keys, causal && own_pv) && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
                            post_conv_w.scalar_type() == scores.scalar_type() && w_post.scalar_type() == scores.scalar_type() && n_keys % 8 == 0;
         const bool small_groups = g_post <= 4 && ((r == 3 && s == 3) || (r == 7 && s == 7));
         OptTensor done;
