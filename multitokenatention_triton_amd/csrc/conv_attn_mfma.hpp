@@ -53,16 +53,16 @@ constexpr int QK_CHUNK = 32;  // key blocks per work item of the scores-only ker
 constexpr int QK_SHORT_PERCENT = 50;
 constexpr int ITEM_TABLE_MAX = 768;
 struct qk_chunks { int big, small; };
-// How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 24000 on the grid
+// How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 16000 on the grid
 // runs in several rounds whatever the length and 48/24 keeps the rebuilt columns few; below, items as short as it takes to
 // have two or three per CU, down to one key block, win although each rebuilds one key block's worth of columns: the grid is
 // otherwise a fraction of the chip, each workgroup walking its keys alone.  Measured (us, with 48/24 -> with this rule):
 // B1 H8 S256 D64 3x3 (80 blocks) 13.3 -> 7.6; B1 H16 S512 D128 5x5 (448) 23.3 -> 11.5; B2 H16 S512 D64 6x11 (896) 22.6 -> 13.4;
-// B4 H16 S512 (1792) 26.3 -> 22.0; B1 H8 S2048 D64 (2450) 48.9 -> 23.9; B1 H16 S2048 D128 7x7 (4900) 60.4 -> 40.8;
-// B1 H16 S4096 D128 7x7 (18900) 140 -> 133.
+// B4 H16 S512 (1792) 26.3 -> 22.0; B1 H8 S2048 D64 (2450) 48.9 -> 23.9; B1 H16 S2048 D128 7x7 (4900) 60.4 -> 40.8.
+// (B1 H16 S4096 D128 7x7, 18900 blocks: 133 instead of 140 launched alone, but the forward it is part of 508.5 instead of 504.1.)
 inline qk_chunks qk_chunk_rule(int64_t blocks, int64_t head_blocks, int nqb)
 {
-    if (blocks >= 24000) return {48, 24};
+    if (blocks >= 16000) return {48, 24};
     if (blocks < 600) return {1, 1};
     int small = (int)std::min<int64_t>(std::max<int64_t>((blocks + 400) / 800, 1), 8);
     while (head_blocks / small + 2 * nqb > ITEM_TABLE_MAX && small < 24) small *= 2;   // (the table holds one head's items)
