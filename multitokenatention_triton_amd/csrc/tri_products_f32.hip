@@ -115,6 +115,86 @@ __global__ __launch_bounds__(256) void lower_scores_f32(const float *__restrict_
     }
 }
 
+// ---- scores of large grids: a workgroup owns 128 query rows x 128 keys, its wavefronts 64 x 64 each ------------------------
+// The kernel above pulls 6 KB through the L1 for every 32 products.  Here slabs of 16 head dims of both operands are copied
+// global -> LDS asynchronously, one slab ahead, and serve all four wavefronts: a third of the bytes per product.  What bounds it
+// now is the fp32 matrix rate (64 more head dims cost 25 us at B1 H32 S1024, 91 TFLOP/s) with the write of the scores behind it.  A slab row is four 16-byte
+// chunks, XOR-swizzled by bits 2 and 3 of the row: the lanes that the LDS serves together (0-7 with 24-31, ...) then cover its
+// banks once.
+constexpr int SL_TILE = 128, SL_D = 16;
+template <int D>
+__global__ __launch_bounds__(256, 3) void lower_scores_f32_slabs(const float *__restrict__ A, const float *__restrict__ Bm, float *__restrict__ C,
+                                                                 int S, int tiles, int64_t total, int64_t per_xcd, int hpx)
+{
+    __shared__ __align__(16) float a_buf[2][SL_TILE * SL_D];
+    __shared__ __align__(16) float b_buf[2][SL_TILE * SL_D];
+    int64_t bh;
+    int tile;
+    if (!place(tiles, total, per_xcd, hpx, bh, tile)) return;
+    int tr = (int)(sqrtf(2.0f * (float)tile + 0.25f) - 0.5f);   // tile row: tr (tr + 1) / 2 tiles lie ahead of it
+    while (tr * (tr + 1) / 2 > tile) --tr;
+    while ((tr + 1) * (tr + 2) / 2 <= tile) ++tr;
+    const int tc = tile - tr * (tr + 1) / 2;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const float *Ap = A + bh * (int64_t)S * D, *Bp = Bm + bh * (int64_t)S * D;
+    // slab s: 128 rows of four chunks, two slots per thread and operand (rows past the sequence re-read the last one)
+    auto issue = [&](int s, int set) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int slot = i * 256 + tid, row = slot >> 2, c = (slot & 3) ^ ((row >> 2) & 3);
+            const int ra = tr * SL_TILE + row < S ? tr * SL_TILE + row : S - 1, rb = tc * SL_TILE + row < S ? tc * SL_TILE + row : S - 1;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Ap + (int64_t)ra * D + SL_D * s + 4 * c), (lds_void_t *)(a_buf[set] + (i * 256 + wave * 64) * 4), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Bp + (int64_t)rb * D + SL_D * s + 4 * c), (lds_void_t *)(b_buf[set] + (i * 256 + wave * 64) * 4), 16, 0, 0);
+        }
+    };
+    const int wp = (wave & 1) * 64, wq = (wave >> 1) * 64, p0 = tr * SL_TILE + wp, q0 = tc * SL_TILE + wq;
+    const bool live = p0 < S && q0 < S && q0 <= p0 + 63;   // (else outside, or wholly above the diagonal)
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[i][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    issue(0, 0);
+#pragma unroll
+    for (int s = 0; s < D / SL_D; ++s) {
+        __builtin_amdgcn_s_waitcnt(0);   // slab s has arrived
+        __syncthreads();                 // for every wavefront; reads of the other buffers are finished
+        if (s + 1 < D / SL_D) issue(s + 1, (s + 1) & 1);
+        if (!live) continue;
+        f32x4 a[4], b[4];
+        const int at = (g ^ ((r >> 2) & 3)) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a[i] = *reinterpret_cast<const f32x4 *>(a_buf[s & 1] + (wp + 16 * i + r) * SL_D + at);
+            b[i] = *reinterpret_cast<const f32x4 *>(b_buf[s & 1] + (wq + 16 * i + r) * SL_D + at);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) mma4(acc[i][k], b[i][t], a[k][t]);
+    }
+    if (!live) return;
+    // acc[i][k][v]: key q0 + 16i + 4g + v of query row p0 + 16k + r
+    float *Cp = C + bh * (int64_t)S * S;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int p = p0 + 16 * k + r;
+        if (p >= S) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int q = q0 + 16 * i + 4 * g;
+            if (q > p) continue;
+            f32x4 o = acc[i][k];
+#pragma unroll
+            for (int v = 1; v < 4; ++v)
+                if (q + v > p) o[v] = 0.0f;
+            *reinterpret_cast<f32x4 *>(Cp + (int64_t)p * S + q) = o;
+        }
+    }
+}
+
 // the sums of a workgroup's four wavefronts, N vectors per lane each, added in wavefront order: wavefront w takes vectors
 // w, w+4, ... ; `part`: 4 * CH * 64 vectors of LDS, CH vectors at a time
 template <int N, int CH, typename GET, typename STORE>
@@ -299,6 +379,11 @@ int check(const void *a, const void *b, const void *c, int64_t B, int64_t H, int
     return MTA_OK;
 }
 
+// Whether the scores run on tiles of 128 x 128 in LDS slabs: from half a workgroup per CU on (us, direct | slabs, D64 / D128:
+// B1 H8 S512, 80 tiles, 6.7 | 9.4 / 9.5 | 13.2; B1 H16 S512, 160, 14.8 | 9.9 / 17.5 | 14.2; B1 H16 S1024, 576, 24.7 | 23.5 / 39.5 | 35.5;
+// B1 H32 S1024, 1152, 40.7 | 38.8 / 69.3 | 63.8; B1 H16 S2048, 2176, 73.2 | 62.5 / 127 | 105).
+bool scores_slabs(int64_t tiles) { return tiles >= 128; }
+
 template <typename K, typename... ARGS>
 int launch(K kern, int64_t bh, int64_t tiles, hipStream_t st, const void *a, const void *b, void *c, int64_t S, ARGS... more)
 {
@@ -314,6 +399,10 @@ extern "C" int mta_lower_scores_f32(const void *a, const void *b, void *out, int
 {
     const int rc = check(a, b, out, B, H, S, D);
     if (rc != MTA_OK) return rc;
+    const int64_t n = (S + SL_TILE - 1) / SL_TILE;
+    if (scores_slabs(B * H * n * (n + 1) / 2))
+        return D == 64 ? launch(lower_scores_f32_slabs<64>, B * H, n * (n + 1) / 2, (hipStream_t)stream, a, b, out, S)
+                       : launch(lower_scores_f32_slabs<128>, B * H, n * (n + 1) / 2, (hipStream_t)stream, a, b, out, S);
     const int64_t tiles = sc_tiles((int)((S + SC_ROWS - 1) / SC_ROWS));
     return D == 64 ? launch(lower_scores_f32<64>, B * H, tiles, (hipStream_t)stream, a, b, out, S)
                    : launch(lower_scores_f32<128>, B * H, tiles, (hipStream_t)stream, a, b, out, S);
