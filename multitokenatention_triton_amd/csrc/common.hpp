@@ -77,7 +77,29 @@ template <> struct vec_of<f16_t> { static constexpr int n = 8; };
 
 template <typename T> struct alignas(16) pack16 { T v[vec_of<T>::n]; };
 
+// A 16-byte vector of a kernel's output.  `stream` (wavefront-uniform): non-temporal, past the caches - for tensors that the
+// kernel behind would not find there anyway; see streams().
+template <typename V> __device__ __forceinline__ void store_out(V *dst, const V &v, bool stream)
+{
+    static_assert(sizeof(V) == 16, "whole vectors");
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    // (the empty statements keep the compiler from merging the two stores into one, an ordinary one, at either end)
+    if (stream) {
+        asm volatile("");
+        __builtin_nontemporal_store(__builtin_bit_cast(u4, v), reinterpret_cast<u4 *>(dst));
+        asm volatile("");
+    } else {
+        *dst = v;
+    }
+}
+
 // ---- host-side helpers --------------------------------------------------------------
+// Whether a (N,C,P,Q) tensor moves as streaming (non-temporal) data: from 128 MB on, of which the memory-side cache (256 MB)
+// holds little by the time the next kernel reads it.  Below, that kernel finds in the caches what this one has written.
+// Ordinary | non-temporal stores in all stages, us: forward bf16 B2 H16 S1001 (64 MB) 98 | 113, fp32 B1 H16 S1024 (64 MB) 192 | 197,
+// training fp16 B1 H16 S2048 (128 MB) 674 | 679; conv training bf16 B2 H16 S2048 (256 MB) 255 | 233, head mixing training
+// B2 H32 S2048 (512 MB) 448 | 424, forward B2 H16 S4096 (1 GB) 604 | 573.
+inline bool streams(int64_t N, int64_t C, int64_t P, int64_t Q, size_t size) { return N * C * P * Q * (int64_t)size > (128 << 20); }
 // ---- the triangular layout of a causal (S,S) score tensor --------------------------------------------------------
 // Only what lies on and below the diagonal is stored.  Row p holds 64*(p/64 + 1) elements (keys 0 .. p and padding up
 // to the next multiple of 64: every row starts on a 128-byte boundary and a 64-key block that holds an attended key is

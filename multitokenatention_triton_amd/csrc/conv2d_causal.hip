@@ -145,9 +145,9 @@ int launch_valu(const void *x, const void *w, void *y, int64_t N, int64_t C, int
 // ------------------------------------------------------------------------------------
 // MFMA (Toeplitz) path
 // ------------------------------------------------------------------------------------
-// The output is written once and not read again by this kernel: non-temporal stores keep it from displacing the input
-// rows that neighbouring strips re-read (halos) in the L2.
-#define MTA_CONV_STORE(ptr, val) __builtin_nontemporal_store((val), (ptr))
+// The output is written once and not read again by this kernel: for large tensors non-temporal stores keep it from displacing
+// the input rows that neighbouring strips re-read (halos) in the L2.
+#define MTA_CONV_STORE(ptr, val) store_out((ptr), (val), STREAM)
 
 constexpr int M_NW = 4;            // wavefronts per workgroup: (16-row block, 128-key half) of the workgroup's strip each
 constexpr int M_WT = 64 * M_NW;    // threads per workgroup
@@ -203,7 +203,7 @@ __device__ __forceinline__ void decode_item(int t, int tiles_n, int tri, int &tm
 
 // +0 over an M_TM x M_TN region, all threads of the workgroup.  FULL: the region lies inside the tensor; the stores are
 // then unconditional (exactly M_TM*M_TN/8/M_WT vector-memory instructions per lane)
-template <typename T, bool FULL = false>
+template <typename T, bool STREAM, bool FULL = false>
 __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int q0, int tid)
 {
     constexpr int VEC = 8, VPRW = M_TN / VEC, RPP = M_WT / VPRW;  // vectors per row, rows per pass
@@ -266,7 +266,7 @@ __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int
 //
 // BWD: the gradient with respect to the input (see conv2d_valu): kernel rows reversed in both axes, the R-1 halo rows
 // below the strip instead of above it.  Key sizes are odd here, so the key halos are the same on both sides.
-template <typename T, int R, int S, bool SCALED, bool BWD>
+template <typename T, int R, int S, bool SCALED, bool BWD, bool STREAM>
 __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
     const T *__restrict__ x, const T *__restrict__ w, T *__restrict__ y, int C, int H, int W, int causal, float in_scale,
     int tiles_n, int ipp, int64_t total, int64_t per_xcd, int nw, int tri)
@@ -541,10 +541,10 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
         if (kind != 0) {
             if (kind == 1) {
                 if (full_out) {
-                    zero_fill_strip<T, true>(yp, H, W, p0, q0, tid);
+                    zero_fill_strip<T, STREAM, true>(yp, H, W, p0, q0, tid);
                     younger = ST;
                 } else {
-                    zero_fill_strip<T>(yp, H, W, p0, q0, tid);
+                    zero_fill_strip<T, STREAM>(yp, H, W, p0, q0, tid);
                     younger = -1;
                 }
             }
@@ -658,15 +658,17 @@ int launch_mfma(const void *x, const void *w, void *y, int64_t N, int64_t C, int
     if (nw < 1) nw = 1;
     if (per_xcd < nw) nw = (int)per_xcd;
     dim3 grid((unsigned)(nw * 8));
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(M_WT), 0, st, (const T *)x, (const T *)w, (T *)y, (int)C, (int)H, (int)W, causal, in_scale,
+                           (int)tiles_n, ipp, total, per_xcd, nw, tri);
+    };
+    const bool stream = streams(N, C, H, W, sizeof(T));
     if constexpr (BWD) {
-        hipLaunchKernelGGL((conv2d_mfma<T, R, S, false, true>), grid, dim3(M_WT), 0, st, (const T *)x, (const T *)w, (T *)y,
-                           (int)C, (int)H, (int)W, causal, in_scale, (int)tiles_n, ipp, total, per_xcd, nw, tri);
+        go(stream ? conv2d_mfma<T, R, S, false, true, true> : conv2d_mfma<T, R, S, false, true, false>);
     } else if (use_scale) {
-        hipLaunchKernelGGL((conv2d_mfma<T, R, S, true, false>), grid, dim3(M_WT), 0, st, (const T *)x, (const T *)w, (T *)y,
-                           (int)C, (int)H, (int)W, causal, in_scale, (int)tiles_n, ipp, total, per_xcd, nw, tri);
+        go(stream ? conv2d_mfma<T, R, S, true, false, true> : conv2d_mfma<T, R, S, true, false, false>);
     } else {
-        hipLaunchKernelGGL((conv2d_mfma<T, R, S, false, false>), grid, dim3(M_WT), 0, st, (const T *)x, (const T *)w, (T *)y,
-                           (int)C, (int)H, (int)W, causal, in_scale, (int)tiles_n, ipp, total, per_xcd, nw, tri);
+        go(stream ? conv2d_mfma<T, R, S, false, false, true> : conv2d_mfma<T, R, S, false, false, false>);
     }
     return launch_status();
 }

@@ -20,9 +20,9 @@ constexpr int NT = 256;
 
 template <typename T, int VEC> struct alignas(sizeof(T) * VEC) vecN { T v[VEC]; };
 
-// Inputs are read once and outputs written once by these kernels.  The outputs are written as streaming (non-temporal) data;
-// the inputs are read so where the tensor is too large for the memory-side cache to still hold what its producer wrote, and
-// as ordinary data where it is not (STREAM, see streams()).
+// Inputs are read once and outputs written once by these kernels: large tensors move as streaming (non-temporal) data, others
+// as ordinary data (STREAM, see streams()).  Non-temporal | ordinary loads, us, bf16 dense 16 heads, the lower triangle of a tensor that
+// the kernel ahead has just written: B2 S1008 (65 MB) 21.4 | 13.7, B1 S2048 (134 MB) 38.7 | 24.6, B1 S4096 (537 MB) 127 | 136.
 template <bool STREAM, typename V> __device__ __forceinline__ V load_as(const V *src)
 {
     if constexpr (STREAM && sizeof(V) == 16) {
@@ -31,14 +31,10 @@ template <bool STREAM, typename V> __device__ __forceinline__ V load_as(const V 
     }
     return *src;
 }
-template <typename V> __device__ __forceinline__ void store_stream(V *dst, const V &v)
+template <bool STREAM, typename V> __device__ __forceinline__ void store_as(V *dst, const V &v)
 {
-    if constexpr (sizeof(V) == 16) {
-        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(__builtin_bit_cast(u4, v), reinterpret_cast<u4 *>(dst));
-        return;
-    }
-    *dst = v;
+    if constexpr (sizeof(V) == 16) store_out(dst, v, STREAM);
+    else *dst = v;
 }
 
 // element (o, i) of the mixing matrix the kernels apply: w[o][i], or w[i][o] when `wt` (the transposed matrix is what
@@ -88,7 +84,7 @@ __global__ __launch_bounds__(NT) void headmix_fixed(const T *__restrict__ x, con
     if (causal && qc * NT * VEC > p) {  // chunk wholly above the diagonal: fill only, nothing read
         if (q < Q && causal != 2) {
 #pragma unroll
-            for (int o = 0; o < G; ++o) store_stream(reinterpret_cast<V *>(y + base + o * plane), fillv);
+            for (int o = 0; o < G; ++o) store_as<STREAM>(reinterpret_cast<V *>(y + base + o * plane), fillv);
         }
         return;
     }
@@ -107,7 +103,7 @@ __global__ __launch_bounds__(NT) void headmix_fixed(const T *__restrict__ x, con
     if (causal && q > p) {
         if (causal != 2) {
 #pragma unroll
-            for (int o = 0; o < G; ++o) store_stream(reinterpret_cast<V *>(y + base + o * plane), fillv);
+            for (int o = 0; o < G; ++o) store_as<STREAM>(reinterpret_cast<V *>(y + base + o * plane), fillv);
         }
         return;
     }
@@ -125,7 +121,7 @@ __global__ __launch_bounds__(NT) void headmix_fixed(const T *__restrict__ x, con
         V out;
 #pragma unroll
         for (int u = 0; u < VEC; ++u) out.v[u] = (causal && q + u > p) ? fill_t : from_float<T>(acc[u]);
-        store_stream(reinterpret_cast<V *>(y + base + o * plane), out);
+        store_as<STREAM>(reinterpret_cast<V *>(y + base + o * plane), out);
     }
 }
 
@@ -370,7 +366,7 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
         if (key < Q && causal != 2) {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                if (HG == 16 || kg * 4 < HG) __builtin_nontemporal_store(fv, reinterpret_cast<u4 *>(y + base + (kg * 4 + t) * plane + key));
+                if (HG == 16 || kg * 4 < HG) store_out(reinterpret_cast<u4 *>(y + base + (kg * 4 + t) * plane + key), fv, STREAM);
         }
         return;
     }
@@ -421,7 +417,7 @@ __global__ __launch_bounds__(64 * DM_WAVES, 4) void headmix_dense16(const T *__r
                 if (key + 2 * u + 1 > last) o[u] = (o[u] & 0x0000ffffu) | (fill2 & 0xffff0000u);
             }
         }
-        __builtin_nontemporal_store(o, reinterpret_cast<u4 *>(y + base + (int64_t)(kg * 4 + v) * plane + key));
+        store_out(reinterpret_cast<u4 *>(y + base + (int64_t)(kg * 4 + v) * plane + key), o, STREAM);
     }
 }
 
@@ -462,11 +458,6 @@ __global__ __launch_bounds__(NT) void headmix_any(const T *__restrict__ x, const
         *reinterpret_cast<V *>(y + base + o * plane) = out;
     }
 }
-
-// Whether a tensor is larger than the memory-side cache (256 MB).  Non-temporal loads | ordinary loads, us, bf16 dense 16 heads,
-// the lower triangle of a tensor that the kernel ahead has just written: B2 S1008 (65 MB) 21.4 | 13.7, B1 S2048 (134 MB)
-// 38.7 | 24.6 (cold: 36.5 | 30.3), B1 S4096 (537 MB) 127 | 136.
-inline bool streams(int64_t N, int64_t C, int64_t P, int64_t Q, size_t size) { return N * C * P * Q * (int64_t)size > (256 << 20); }
 
 template <typename T, int VEC>
 int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t P, int64_t Q, int G, int causal,

@@ -76,14 +76,10 @@ template <typename V> __device__ __forceinline__ V load_stream(const V *src)
         return *src;
     }
 }
-template <typename V> __device__ __forceinline__ void store_stream(V *dst, const V &v)
+template <typename V> __device__ __forceinline__ void store_any(V *dst, const V &v, bool stream)
 {
-    if constexpr (sizeof(V) == 16) {
-        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(__builtin_bit_cast(u4, v), reinterpret_cast<u4 *>(dst));
-    } else {
-        *dst = v;
-    }
+    if constexpr (sizeof(V) == 16) store_out(dst, v, stream);
+    else *dst = v;
 }
 
 template <int NT> __device__ __forceinline__ float block_max(float v, float *red)
@@ -123,7 +119,7 @@ template <typename T, int G, int NV, int VEC, int NT, bool KB>
 __global__ __launch_bounds__(NT, (!KB && NT == 256 && G * NV == 8) ? RS_OCC : 1) void mix_softmax_mix(const T *__restrict__ x, const void *__restrict__ w1,
                                                       const void *__restrict__ w2, const float *__restrict__ kb,
                                                       T *__restrict__ y, int C, int P, int Q, int causal,
-                                                      int w_dtype, int fill_upper, const int *__restrict__ row_lo)
+                                                      int w_dtype, int fill_upper, const int *__restrict__ row_lo, int stream)
 {
     __shared__ float w1s[G * G];
     __shared__ float w2s[G * G];
@@ -331,7 +327,7 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G * NV == 8) ? RS_OCC : 1)
 #pragma unroll
                 for (int u = 0; u < VEC; ++u) z.v[u] = from_float<T>(0.0f);
 #pragma unroll
-                for (int o = 0; o < G; ++o) store_stream(reinterpret_cast<V *>(y + base + o * plane + q), z);
+                for (int o = 0; o < G; ++o) store_any(reinterpret_cast<V *>(y + base + o * plane + q), z, stream);
             }
             continue;
         }
@@ -341,7 +337,7 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G * NV == 8) ? RS_OCC : 1)
 #pragma unroll
                 for (int u = 0; u < VEC; ++u) z.v[u] = from_float<T>(0.0f);
 #pragma unroll
-                for (int o = 0; o < G; ++o) store_stream(reinterpret_cast<V *>(y + base + o * plane + q), z);
+                for (int o = 0; o < G; ++o) store_any(reinterpret_cast<V *>(y + base + o * plane + q), z, stream);
             }
             continue;
         }
@@ -389,7 +385,7 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G * NV == 8) ? RS_OCC : 1)
             }
             V out;
             pack_vec<T, VEC>(of, out);
-            store_stream(reinterpret_cast<V *>(y + base + o * plane + q), out);
+            store_any(reinterpret_cast<V *>(y + base + o * plane + q), out, stream);
         }
     }
 }
@@ -511,7 +507,7 @@ template <bool IS_MAX, int G, int NW> __device__ __forceinline__ void heads_comb
 template <typename T, int G, int NV, bool HAS1, bool HAS2, int NT, int OCC, bool BAND = false, bool KBIAS = false>
 __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
     const T *__restrict__ x, const T *__restrict__ w1, const T *__restrict__ w2, T *__restrict__ y, int C, int P, int Q,
-    int causal, int fill_upper, const int *__restrict__ row_lo, int tri, const float *__restrict__ key_bias)
+    int causal, int fill_upper, const int *__restrict__ row_lo, int tri, const float *__restrict__ key_bias, int stream)
 {
     constexpr int VEC = 8, NW = NT / 64, H2 = G / 2;
     static_assert(sizeof(T) == 2 && G % 2 == 0, "packed pairs of a 16-bit type");
@@ -550,7 +546,7 @@ __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
             const int q = tid * VEC;
             const rs_u4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int o = 0; o < G; ++o) __builtin_nontemporal_store(z, reinterpret_cast<rs_u4 *>(y + base + o * plane + q));
+            for (int o = 0; o < G; ++o) store_out(reinterpret_cast<rs_u4 *>(y + base + o * plane + q), z, stream);
             return;
         }
     }
@@ -562,7 +558,7 @@ __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
                 if (q >= Q) continue;
                 const rs_u4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int o = 0; o < G; ++o) __builtin_nontemporal_store(z, reinterpret_cast<rs_u4 *>(y + base + o * plane + q));
+                for (int o = 0; o < G; ++o) store_out(reinterpret_cast<rs_u4 *>(y + base + o * plane + q), z, stream);
             }
         }
         return;
@@ -751,7 +747,7 @@ __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
 #pragma unroll
             for (int o = 0; o < G; ++o) {
                 const rs_u4 v = {out[o][0], out[o][1], out[o][2], out[o][3]};
-                __builtin_nontemporal_store(v, reinterpret_cast<rs_u4 *>(y + base + o * plane + q));
+                store_out(reinterpret_cast<rs_u4 *>(y + base + o * plane + q), v, stream);
             }
         }
         if (fill_upper) {  // passes wholly above the diagonal
@@ -761,7 +757,7 @@ __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
                 if (q >= Q) continue;
                 const rs_u4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int o = 0; o < G; ++o) __builtin_nontemporal_store(z, reinterpret_cast<rs_u4 *>(y + base + o * plane + q));
+                for (int o = 0; o < G; ++o) store_out(reinterpret_cast<rs_u4 *>(y + base + o * plane + q), z, stream);
             }
         }
     };
@@ -923,12 +919,13 @@ int launch_fixed(const void *x, const void *w1, const void *w2, const float *kb,
 {
     constexpr int VEC = vec_of<T>::n;
     const int64_t blocks = N * (C / G) * P;
+    const int stream = streams(N, C, P, Q, sizeof(T));
     if (kb || row_lo)
         hipLaunchKernelGGL((mix_softmax_mix<T, G, NV, VEC, NT, true>), dim3((unsigned)blocks), dim3(NT), 0, st, (const T *)x,
-                           w1, w2, kb, (T *)y, (int)C, (int)P, (int)Q, causal, w_dtype, fill_upper, row_lo);
+                           w1, w2, kb, (T *)y, (int)C, (int)P, (int)Q, causal, w_dtype, fill_upper, row_lo, stream);
     else
         hipLaunchKernelGGL((mix_softmax_mix<T, G, NV, VEC, NT, false>), dim3((unsigned)blocks), dim3(NT), 0, st, (const T *)x,
-                           w1, w2, kb, (T *)y, (int)C, (int)P, (int)Q, causal, w_dtype, fill_upper, row_lo);
+                           w1, w2, kb, (T *)y, (int)C, (int)P, (int)Q, causal, w_dtype, fill_upper, row_lo, stream);
     return launch_status();
 }
 
@@ -940,6 +937,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
     // (the kernels without a key bias are the ones without a band mask too: `kb` below stands for "either")
     const float *kb = kb_in;
     const bool plain = !kb_in && !row_lo;
+    const int stream = streams(N, C, P, Q, sizeof(T));
     constexpr int VEC = vec_of<T>::n;
     const bool vec_ok = (Q % VEC == 0) && aligned_to(x, 16) && aligned_to(y, 16);
     const int64_t nv = (Q + 256 * VEC - 1) / (256 * VEC);
@@ -963,7 +961,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
     {                                                                                                                  \
         hipLaunchKernelGGL((mix_softmax_mix_packed<T, g, v, h1, h2, nt, occ, false, true>),                            \
                            dim3((unsigned)(N * (C / g) * P)), dim3(nt), 0, st, (const T *)x, (const T *)w1,            \
-                           (const T *)w2, (T *)y, (int)C, (int)P, (int)Q, causal, fill_upper, nullptr, tri, kb);      \
+                           (const T *)w2, (T *)y, (int)C, (int)P, (int)Q, causal, fill_upper, nullptr, tri, kb, stream); \
         return launch_status();                                                                                        \
     }
 #define MTA_RSK_CASE(g, v, nt, occ)                                                                                    \
@@ -985,7 +983,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
     {                                                                                                                  \
         hipLaunchKernelGGL((mix_softmax_mix_packed<T, g, 1, h1, h2, nt, occ, true>), dim3((unsigned)(N * (C / g) * P)), \
                            dim3(nt), 0, st, (const T *)x, (const T *)w1, (const T *)w2, (T *)y, (int)C, (int)P,        \
-                           (int)Q, causal, fill_upper, row_lo, tri, nullptr);                                          \
+                           (int)Q, causal, fill_upper, row_lo, tri, nullptr, stream);                                  \
         return launch_status();                                                                                        \
     }
 #define MTA_RSB_CASE(g, nt, occ)                                                                                       \
@@ -1002,7 +1000,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
     {                                                                                                                  \
         hipLaunchKernelGGL((mix_softmax_mix_packed<T, g, v, h1, h2, nt, occ>), dim3((unsigned)(N * (C / g) * P)),      \
                            dim3(nt), 0, st, (const T *)x, (const T *)w1, (const T *)w2, (T *)y, (int)C, (int)P,        \
-                           (int)Q, causal, fill_upper, nullptr, tri, nullptr);                                         \
+                           (int)Q, causal, fill_upper, nullptr, tri, nullptr, stream);                                 \
         return launch_status();                                                                                        \
     }
 #define MTA_RSP_CASE(g, v, nt, occ)                                                                                    \

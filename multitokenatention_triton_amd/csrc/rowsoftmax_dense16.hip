@@ -250,7 +250,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
                                                                            int P, int Q, int causal, int fill_upper, int r4,
                                                                            int r8, int wpg, int tri_in, int tri_out,
                                                                            const float *__restrict__ key_bias,
-                                                                           const int *__restrict__ row_lo)
+                                                                           const int *__restrict__ row_lo, int stream)
 {
     constexpr int NW = M16_NW, TPW = M16_TPW, HG = M16_HG;
     __shared__ __align__(16) float kbias[MASKED ? NW * TPW * M16_TK : 4];  // (MASKED) the batch entry's key bias
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
                     const u32x4_t z = {0u, 0u, 0u, 0u};
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        __builtin_nontemporal_store(z, reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)));
+                        store_out(reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)), z, stream);
                 }
                 continue;
             }
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
             if (key < Q && (fill_upper || key <= last)) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    __builtin_nontemporal_store(out[v], reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)));
+                    store_out(reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)), out[v], stream);
             }
         }
         // keys beyond the tiles of this instance lie wholly above the diagonal: +0 on request (plain vector stores; the
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
             for (int key = (TPW * nwr + wr) * M16_TK + ln * 8; key < Q; key += nwr * M16_TK) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    __builtin_nontemporal_store(z, reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)));
+                    store_out(reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)), z, stream);
             }
         }
         p = pn;
@@ -558,6 +558,7 @@ int mix16_softmax_launch(const void *x, const void *w1, const void *w2, void *y,
                          const float *key_bias, const int *row_lo)
 {
     const bool masked = key_bias || row_lo;
+    const int stream = streams(N, C, P, Q, 2);
     if (row_lo && !causal) return MTA_ERR_UNSUPPORTED;
     if (io_dtype == MTA_F32 || w_dtype != io_dtype || (!w1 && !w2) || C % M16_HG != 0 || Q % 8 != 0 ||
         Q > (int64_t)M16_NW * M16_TPW * M16_TK)
@@ -591,12 +592,12 @@ int mix16_softmax_launch(const void *x, const void *w1, const void *w2, void *y,
             hipLaunchKernelGGL((mix16_softmax_rows_kernel<T, h1, h2, true>), dim3((unsigned)(N * (C / M16_HG) * wpg)),  \
                                dim3(64 * M16_NW), 0, st, (const T *)x, (const T *)w1, (const T *)w2, (T *)y, (int)C,    \
                                (int)P, (int)Q, causal, fill_upper, (int)r4, (int)r8, (int)wpg, tri_in, tri_out,         \
-                               key_bias, row_lo);                                                                       \
+                               key_bias, row_lo, stream);                                                                       \
         else                                                                                                            \
             hipLaunchKernelGGL((mix16_softmax_rows_kernel<T, h1, h2>), dim3((unsigned)(N * (C / M16_HG) * wpg)),        \
                                dim3(64 * M16_NW), 0, st, (const T *)x, (const T *)w1, (const T *)w2, (T *)y, (int)C,    \
                                (int)P, (int)Q, causal, fill_upper, (int)r4, (int)r8, (int)wpg, tri_in, tri_out,         \
-                               nullptr, nullptr);                                                                       \
+                               nullptr, nullptr, stream);                                                                       \
     }
 #define MTA_M16_CASES(T)                                          \
     if (w1 && w2) { MTA_M16_ALL(T, true, true) }                  \

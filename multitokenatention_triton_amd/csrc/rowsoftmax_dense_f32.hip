@@ -19,7 +19,7 @@ template <int HB, int NW, int NV>
 __global__ __launch_bounds__(64 * NW) void mix_softmax_dense_f32(const float *__restrict__ x, const void *__restrict__ w1,
                                                                  const void *__restrict__ w2, const float *__restrict__ kb,
                                                                  const int *__restrict__ row_lo, float *__restrict__ y, int C, int HG,
-                                                                 int P, int Q, int causal, int w_dtype, int fill_upper)
+                                                                 int P, int Q, int causal, int w_dtype, int fill_upper, int stream)
 {
     constexpr int NS = 4 * HB;   // heads per lane
     __shared__ float red[2][NW][16 * HB];   // [0] maxima, [1] sums
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(64 * NW) void mix_softmax_dense_f32(const float *__
         if (key >= Q || (key > last && !fill_upper)) continue;
 #pragma unroll
         for (int t = 0; t < NS; ++t)
-            if (head(t) < HG) __builtin_nontemporal_store(out[t], reinterpret_cast<f32x4 *>(y + base + head(t) * plane + key));
+            if (head(t) < HG) store_out(reinterpret_cast<f32x4 *>(y + base + head(t) * plane + key), out[t], stream);
     }
 }
 }  // namespace
@@ -204,10 +204,11 @@ int mix_softmax_dense_f32_launch(const float *x, const void *w1, const void *w2,
     if (HG < 9 || HG > 32 || Q % 4 != 0 || !aligned_to(x, 16) || !aligned_to(y, 16) || Q > mta_headmix_softmax_dense_f32_keys(HG))
         return MTA_ERR_UNSUPPORTED;
     const int64_t blocks = N * (C / HG) * P;
+    const int stream = streams(N, C, P, Q, 4);
 #define MTA_MSD_CASE(hb, nw, nv)                                                                                                   \
     if (HG <= 16 * (hb) && Q <= 64 * (nw) * (nv)) {                                                                                \
         hipLaunchKernelGGL((mix_softmax_dense_f32<hb, nw, nv>), dim3((unsigned)blocks), dim3(64 * (nw)), 0, st, x, w1, w2, kb,     \
-                           row_lo, y, (int)C, HG, (int)P, (int)Q, causal, w_dtype, fill_upper);                                    \
+                           row_lo, y, (int)C, HG, (int)P, (int)Q, causal, w_dtype, fill_upper, stream);                            \
         return launch_status();                                                                                                    \
     }
     MTA_MSD_CASE(1, 4, 1) MTA_MSD_CASE(1, 4, 2) MTA_MSD_CASE(1, 4, 4) MTA_MSD_CASE(1, 8, 4) MTA_MSD_CASE(1, 8, 8)
