@@ -303,7 +303,7 @@ inline int num_blocks(int64_t N, int64_t C, int64_t P, int64_t Q)
 {
     int64_t nb = C <= 32 ? 256 : 1024;
     const int64_t pairs = (N * P + 1) / 2;
-    if (C > 32 && nb > pairs) nb = pairs;
+    if (nb > pairs) nb = pairs;
     const int64_t cap = MAX_WS_BYTES / (C * C * (int64_t)sizeof(float));
     if (nb > cap) nb = cap;
     return (int)(nb < 1 ? 1 : nb);

@@ -37,6 +37,9 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
     return !masked || group <= FUSED_MAX_GROUP || t == at::kFloat || (group == FUSED_MFMA_GROUP && !no_row_lists());
 }
 
+// fp32 groups of more than 8 heads: one kernel, announced to the observer as the stages it stands for
+bool stages_apart(int64_t group, at::ScalarType t) { return t == at::kFloat && group > FUSED_MAX_GROUP; }
+
 // Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
 // heads at about 20 us each, so that two full rounds of tiles are where it meets the two kernels one after the other (us, one
 // kernel | two, 3x3 / 7x7: B1 S512 25 | 12 / 28 | 14, B1 S1024 27 | 21 / 32 | 26, B2 S1008 39 | 41 / 46 | 49, B1 S1536 49 | 39 / 54 | 47,
@@ -185,7 +188,13 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     }
 
     if (one_pass) {
-        mark("mix_softmax_mix");
+        if (stages_apart(g_both, dtype)) {
+            mark("mix_pre");
+            mark("softmax");
+            mark("mix_post");
+        } else {
+            mark("mix_softmax_mix");
+        }
         scores = headmix_softmax(scores, w1, w2, causal, g_both, !own_pv, key_bias, first);
     } else {
         const bool fill = post_conv_identity && !w2 && !own_pv;
@@ -193,7 +202,12 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
             mark("mix_softmax");
             scores = headmix_softmax_tri(scores, w1, OptTensor(), q.size(0), heads, n_keys, g_pre, first, true, key_bias);
         } else if (one_pass_group(g_pre, dtype, n_keys, w1, OptTensor()) && masks_ok(g_pre, dtype, masked)) {
-            mark("mix_softmax");
+            if (stages_apart(g_pre, dtype)) {
+                mark("mix_pre");
+                mark("softmax");
+            } else {
+                mark("mix_softmax");
+            }
             scores = headmix_softmax(scores, w1, OptTensor(), causal, g_pre, fill, key_bias, first);
         } else {
             mark("mix_pre");   // (the softmax kernel that follows never reads above the diagonal)
@@ -206,13 +220,16 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         // kernels (mixing groups of up to 4 heads and the sizes with a vector-staged instance; dense groups of 16).  Under a
         // band mask the conv's result is zeroed at the hidden positions ahead of the mixing: two kernels.
         const int64_t r = post_conv_w.size(1), s = post_conv_w.size(2);
-        const bool mix16 = g_post == 16 && conv_mix16_fills(q.size(0) * (heads / 16), q.size(2), n_keys, causal && own_pv) && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
+        const bool mix16 = g_post == 16 && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
                            post_conv_w.scalar_type() == scores.scalar_type() && w_post.scalar_type() == scores.scalar_type() && n_keys % 8 == 0;
         const bool small_groups = g_post <= 4 && ((r == 3 && s == 3) || (r == 7 && s == 7));
         OptTensor done;
         if (!first && !post_conv_identity && w2 && (small_groups || mix16)) {
             mark("conv_mix_post");
-            done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
+            if (!mix16 || conv_mix16_fills(q.size(0) * (heads / 16), q.size(2), n_keys, causal && own_pv))
+                done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
+            else   // (the same stage as two kernels, the same results)
+                done = headmix(conv2d(scores, post_conv_w, causal, std::nullopt, false), w_post, causal, 0.0, g_post, !own_pv);
         }
         if (done) {
             scores = *done;
@@ -289,8 +306,13 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         }
         const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
         Tensor p;
-        if (one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), o.key_bias || o.first)) {
-            mark("mix_softmax");
+        if ((!stages_apart(g_eff, x.scalar_type()) || o.pre_causal == o.causal) && one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), o.key_bias || o.first)) {
+            if (stages_apart(g_eff, x.scalar_type())) {
+                mark("mix_pre");
+                mark("softmax");
+            } else {
+                mark("mix_softmax");
+            }
             p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
         } else {
             mark("mix_pre");

@@ -370,3 +370,21 @@ def test_fp32_softmax_gradient_sizes(pkg):
         want = pd * (gd - (pd * gd).sum(-1, keepdim=True))
         got = pkg.ops.softmax_bwd(prob.masked_fill(~keep, float("nan")).cuda(), dp.masked_fill(~keep, float("nan")).cuda(), causal)
         torch.testing.assert_close(got.double().cpu(), want, rtol=1e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ks", [3, 5, 7])
+def test_conv_mix16_one_or_two_kernels(pkg, ks, dtype):
+    """Post-softmax conv and dense mixing of 16 heads: the one-kernel form and the two kernels that small grids take hold the same
+    rounding points and the same products; what differs is the order of fp32 sums, i.e. one rounding of the conv result and one
+    of an output of magnitude at most about 8."""
+    g = torch.Generator().manual_seed(31)
+    for n, c, s in ((1, 16, 8), (1, 16, 72), (2, 32, 136)):
+        print(f"conv mix16 {dtype} {ks}x{ks} n={n} c={c} s={s}", flush=True)
+        x = torch.rand(n, c, s, s, generator=g).to(dtype).cuda()
+        wc = O.seeded_conv_weight(c, ks, ks, 0.1, dtype).cuda()
+        wm = torch.block_diag(*[torch.eye(16) + 0.1 * torch.randn(16, 16, generator=g) for _ in range(c // 16)]).to(dtype).cuda()
+        one = pkg.ops.conv2d_headmix(x, wc, wm, True, group_size=16)
+        two = pkg.ops.headmix(pkg.ops.conv2d_causal(x, wc, True), wm, True, 0.0, group_size=16)
+        ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+        torch.testing.assert_close(one.float(), two.float(), rtol=ulp, atol=4 * ulp)
