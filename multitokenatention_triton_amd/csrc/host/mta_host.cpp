@@ -6,6 +6,8 @@
 // ops.hpp; the Python modules keep parameters, masks and the rarely taken routes.
 #include <torch/extension.h>
 
+#include <ATen/ExpandUtils.h>
+
 #include "ops.hpp"
 
 namespace py = pybind11;
@@ -69,11 +71,12 @@ struct Mark {
     }
 };
 
-// the first rows of (B,H,S,D) seen as (B,S,H,D), without a view relation that autograd would track
+// (B,H,S,D) seen as (B,S,H,D), of its first `rows` rows only if that is not negative, without a view relation that autograd
+// would track
 Tensor heads_last(const Tensor &o, int64_t rows)
 {
     at::AutoDispatchBelowADInplaceOrView guard;
-    return (rows == o.size(2) ? o : o.narrow(2, 0, rows)).transpose(1, 2);
+    return (rows < 0 ? o : o.narrow(2, 0, rows)).transpose(1, 2);
 }
 
 // int32 (B,S): p + 1 for the rows p that see no key, 0 for the others (mta_band_zero_fwd then clears those rows)
@@ -83,14 +86,48 @@ Tensor empty_row_ends(const Tensor &empty_rows)
     return at::where(empty_rows, rows.unsqueeze(0), at::zeros({}, rows.options())).contiguous();
 }
 
+// Q, K and V of one batch, head count, length and dtype, which is what the row copies around the kernels take (of fewer than
+// 2^31 elements).  Anything else the library products broadcast.
+bool alike(const Tensor &q, const Tensor &k, const Tensor &v)
+{
+    if (q.dim() != 4 || k.sizes() != q.sizes() || v.dim() != 4 || v.size(0) != q.size(0) || v.size(1) != q.size(1) || v.size(2) != q.size(2))
+        return false;
+    return k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type() && std::max(q.numel(), v.numel()) < (int64_t(1) << 31);
+}
+
+// The sizes of Q K^T, as torch.matmul broadcasts them; raises where the two products of a call do not exist.
+at::DimVector score_sizes(const Tensor &q, const Tensor &k, const Tensor &v)
+{
+    TORCH_CHECK_VALUE(k.dim() == 4 && q.dim() >= 2 && q.dim() <= 4 && v.dim() >= 1, "expected Q, K, V (B,H,S,D), got ", q.sizes(), ", ", k.sizes(), ", ",
+                      v.sizes());
+    TORCH_CHECK(q.size(-1) == k.size(-1), "Q and K must share their head size, got ", q.sizes(), " and ", k.sizes());
+    TORCH_CHECK(v.size(v.dim() > 1 ? -2 : 0) == k.size(2), "K and V must share their length, got ", k.sizes(), " and ", v.sizes());
+    at::DimVector s = at::infer_size_dimvector(q.sizes().slice(0, q.dim() - 2), k.sizes().slice(0, 2));
+    if (v.dim() > 2) at::infer_size_dimvector(s, v.sizes().slice(0, v.dim() - 2));
+    s.push_back(q.size(-2));
+    s.push_back(k.size(2));
+    return s;
+}
+
 // The length the score kernels work on.  They move score rows as 16-byte vectors; under the causal rule a length that is not
 // a multiple of 8 is padded with zero rows: only padding rows see the padding keys, so every result of a real row is what it
-// was (their gradients are zero: the padding rows of the incoming gradient are).  key_bias, first and empty_rows arrive
-// padded.
+// was (their gradients are zero: the padding rows of the incoming gradient are).
 int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool causal)
 {
-    const int64_t s = q.size(2);
-    return causal && s == k.size(2) && s == v.size(2) ? (s + 7) / 8 * 8 : s;
+    const int64_t s = q.size(-2);
+    return causal && alike(q, k, v) ? (s + 7) / 8 * 8 : s;
+}
+
+// key_bias, first and empty_rows arrive with the columns of a padded length: without the columns no row of the call has
+OptTensor cut_columns(const OptTensor &t, int64_t s)
+{
+    return !t || t->size(1) == s ? t : OptTensor(t->narrow(1, 0, s).contiguous());
+}
+
+// (B,H,S,D) with the rows of hidden keys zeroed, where no row copy does it on the way
+Tensor zero_hidden(const Tensor &x, const Tensor &key_bias)
+{
+    return x.masked_fill((key_bias == -INFINITY).unsqueeze(1).unsqueeze(-1), 0);
 }
 
 // round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it.  Nothing where there is no kernel.
@@ -121,15 +158,21 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 // the identity, and their rows of the output, where nothing else would, at the end.
 Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
                          const Tensor &w_post, bool causal, bool pre_identity, int64_t pre_group, bool post_conv_identity, bool post_identity,
-                         int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows, bool planes,
+                         int64_t post_group, const OptTensor &key_bias_, const OptTensor &first_, const OptTensor &empty_rows_, bool planes,
                          double dropout, const py::object &hook)
 {
     at::NoGradGuard no_grad;
     const c10::OptionalDeviceGuard guard(q_.is_cuda() ? std::optional<c10::Device>(q_.device()) : std::nullopt);
     const Mark mark{hook};
-    const int64_t s_real = q_.size(2), s_pad = padded_length(q_, k_, v_, causal);
+    const at::DimVector planes_of = score_sizes(q_, k_, v_);
+    const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, causal);
+    const OptTensor key_bias = cut_columns(key_bias_, s_pad == s_real ? k_.size(2) : s_pad), first = cut_columns(first_, s_pad),
+                    empty_rows = cut_columns(empty_rows_, s_pad);
     Tensor q = q_, k = k_, v = v_;
-    if (s_pad != s_real || key_bias) {
+    if (key_bias && !alike(q_, k_, v_)) {
+        k = zero_hidden(k_, *key_bias);
+        if (!post_conv_identity) v = zero_hidden(v_, *key_bias);
+    } else if (s_pad != s_real || key_bias) {
         RowsCopy rows(s_pad, key_bias);
         if (s_pad != s_real) q = rows.add(q_, false, 1.0);
         k = rows.add(k_, true, 1.0);
@@ -147,7 +190,8 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const auto dtype = q.scalar_type();
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
-    const bool own_pv = q.size(-2) == n_keys && dtype == v.scalar_type() && lower_products_supported(dtype, q.size(-2), v.size(-1), causal);
+    const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && dtype == v.scalar_type() &&
+                        lower_products_supported(dtype, n_keys, v.size(-1), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
     // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
@@ -226,7 +270,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         OptTensor done;
         if (!first && !post_conv_identity && w2 && (small_groups || mix16)) {
             mark("conv_mix_post");
-            if (!mix16 || conv_mix16_fills(q.size(0) * (heads / 16), q.size(2), n_keys, causal && own_pv))
+            if (!mix16 || conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv))
                 done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
             else   // (the same stage as two kernels, the same results)
                 done = headmix(conv2d(scores, post_conv_w, causal, std::nullopt, false), w_post, causal, 0.0, g_post, !own_pv);
@@ -277,10 +321,16 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
     {
         const TrainOptions &o = *opt;
         const Mark &mark = *mark_;
-        const int64_t s_real = q_.size(2), s_pad = padded_length(q_, k_, v_, o.causal);
+        const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, o.causal);
+        const bool rows_alike = alike(q_, k_, v_);
+        const OptTensor key_bias = cut_columns(o.key_bias, s_pad == s_real ? k_.size(2) : s_pad), first = cut_columns(o.first, s_pad),
+                        empty_rows = cut_columns(o.empty_rows, s_pad);
         Tensor q = q_, k = k_, v = v_;
-        if (s_pad != s_real || o.key_bias) {
-            RowsCopy rows(s_pad, o.key_bias);
+        if (key_bias && !rows_alike) {
+            k = zero_hidden(k_, *key_bias);
+            v = zero_hidden(v_, *key_bias);
+        } else if (s_pad != s_real || key_bias) {
+            RowsCopy rows(s_pad, key_bias);
             if (s_pad != s_real) q = rows.add(q_, false, 1.0);
             k = rows.add(k_, true, 1.0);
             v = rows.add(v_, true, 1.0);
@@ -291,52 +341,53 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         Tensor raw, x;   // raw scores (kept where the first stage is two operators), conv result
         if (qk_conv_supported(q, k, conv_w)) {
             mark("qk_conv");
-            x = qk_conv(q, k, conv_w, o.causal, scale, false, o.first);
+            x = qk_conv(q, k, conv_w, o.causal, scale, false, first);
             // The kernel leaves the key blocks that no row of a query block sees unwritten.  The softmax stage does not read
             // a row's hidden stretch, but its weight gradient multiplies what is stored there by a gradient that is 0: the
             // stretch is cleared, so that the product is 0 too.
-            if (o.first) band_zero_(x, *o.first);
+            if (first) band_zero_(x, *first);
         } else {
             mark("qk");
-            const OptTensor lower_raw = o.causal ? lower_scores(q, k, o.first) : OptTensor();
-            TORCH_CHECK(lower_raw || !o.first, "the band mask needs the lower-triangle products");
+            const OptTensor lower_raw = o.causal ? lower_scores(q, k, first) : OptTensor();
+            TORCH_CHECK(lower_raw || !first, "the band mask needs the lower-triangle products");
             raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
             mark("conv_pre");
             x = conv2d(raw, conv_w, o.causal, scale, false);
         }
         const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
         Tensor p;
-        if ((!stages_apart(g_eff, x.scalar_type()) || o.pre_causal == o.causal) && one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), o.key_bias || o.first)) {
+        if ((!stages_apart(g_eff, x.scalar_type()) || o.pre_causal == o.causal) && one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), key_bias || first)) {
             if (stages_apart(g_eff, x.scalar_type())) {
                 mark("mix_pre");
                 mark("softmax");
             } else {
                 mark("mix_softmax");
             }
-            p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
+            p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, key_bias, first);
         } else {
             mark("mix_pre");
             const Tensor m = headmix(x, w_pre, o.pre_causal, fill ? o.pre_fill : 0.0, o.pre_group, fill);
             mark("softmax");
-            p = headmix_softmax(m, OptTensor(), OptTensor(), o.causal, 0, fill, o.key_bias, o.first);
+            p = headmix_softmax(m, OptTensor(), OptTensor(), o.causal, 0, fill, key_bias, first);
         }
-        if (o.empty_rows) band_zero_(p, empty_row_ends(*o.empty_rows));
+        if (empty_rows) band_zero_(p, empty_row_ends(*empty_rows));
         mark("conv_post");
         Tensor c = conv2d(p, post_conv_w, o.causal, std::nullopt, fill);
-        if (o.first) band_zero_(c, *o.first);
+        if (first) band_zero_(c, *first);
         mark("mix_post");
         // the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
-        const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && v.size(-2) == n_keys &&
-                              c.size(-2) == c.size(-1) && lower_products_supported(v.scalar_type(), c.size(-1), v.size(-1), true);
-        TORCH_CHECK(!o.first || lower_pv, "the band mask needs the lower-triangle products");
+        const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && score_planes_of(c.sizes(), v.sizes()) &&
+                              lower_products_supported(v.scalar_type(), n_keys, v.size(-1), true);
+        TORCH_CHECK(!first || lower_pv, "the band mask needs the lower-triangle products");
         Tensor m = headmix(c, w_post, o.post_causal, lower_pv ? 0.0 : o.post_fill, o.post_group, !lower_pv), keep;
         if (o.dropout > 0) std::tie(m, keep) = at::native_dropout(m, o.dropout, true);
         mark("pv");
-        Tensor out = lower_pv ? *causal_pv(m, v, true, o.first, 1.0) : at::matmul(m, v);
+        Tensor out = lower_pv ? *causal_pv(m, v, true, first, 1.0) : at::matmul(m, v);
         mark("end");
-        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, o.first ? *o.first : Tensor(),
-                                o.key_bias ? *o.key_bias : Tensor()});
+        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, first ? *first : Tensor(),
+                                key_bias ? *key_bias : Tensor()});
         ctx->saved_data["s_real"] = s_real;
+        ctx->saved_data["alike"] = rows_alike;
         ctx->saved_data["causal"] = o.causal;
         ctx->saved_data["pre_causal"] = o.pre_causal;
         ctx->saved_data["post_causal"] = o.post_causal;
@@ -344,7 +395,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         ctx->saved_data["post_group"] = o.post_group;
         ctx->saved_data["dropout"] = o.dropout;
         ctx->saved_data["lower_pv"] = lower_pv;
-        return heads_last(out, s_real);
+        return heads_last(out, s_pad == s_real ? -1 : s_real);
     }
 
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
@@ -355,7 +406,8 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         Tensor raw = saved[7];
         const OptTensor first = saved[13].defined() ? OptTensor(saved[13]) : OptTensor(),
                         key_bias = saved[14].defined() ? OptTensor(saved[14]) : OptTensor();
-        const int64_t s_real = ctx->saved_data["s_real"].toInt(), s_pad = q.size(2);
+        const int64_t s_real = ctx->saved_data["s_real"].toInt(), s_pad = q.size(-2);
+        const bool rows_alike = ctx->saved_data["alike"].toBool();
         const bool causal = ctx->saved_data["causal"].toBool(), pre_causal = ctx->saved_data["pre_causal"].toBool(),
                    post_causal = ctx->saved_data["post_causal"].toBool(), lower_pv = ctx->saved_data["lower_pv"].toBool();
         const int64_t pre_group = ctx->saved_data["pre_group"].toInt(), post_group = ctx->saved_data["post_group"].toInt();
@@ -368,7 +420,9 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         torch::autograd::variable_list out(9);
 
         Tensor go;   // (B,H,S,D), padded with zero rows
-        {
+        if (!rows_alike) {
+            go = grads[0].transpose(1, 2).contiguous();
+        } else {
             RowsCopy rows(s_pad, OptTensor());
             go = rows.add(grads[0].transpose(1, 2), false, 1.0);
             rows.run();
@@ -378,6 +432,17 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         Tensor dq, dk, dv;
         double dq_scale = 1.0, dk_scale = 1.0;
         auto results = [&] {
+            if (!rows_alike) {
+                auto leave = [&](const Tensor &g, bool hide, double factor) {
+                    if (!g.defined()) return g;
+                    const Tensor scaled = factor != 1.0 ? g * factor : g;
+                    return hide && key_bias ? zero_hidden(scaled, *key_bias) : scaled;
+                };
+                out[0] = leave(dq, false, dq_scale);
+                out[1] = leave(dk, true, dk_scale);
+                out[2] = leave(dv, true, 1.0);
+                return out;
+            }
             RowsCopy rows(s_real, key_bias);
             auto leave = [&](Tensor &g, bool hide, double factor) {
                 return g.defined() && (cut || (hide && key_bias) || factor != 1.0) ? rows.add(g, hide, factor) : g;
@@ -395,7 +460,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         if (!need_c && !need[6]) return results();
         const OptTensor lower_dm = lower_pv ? lower_scores(go, v, first) : OptTensor();
         TORCH_CHECK(lower_dm || !first);
-        Tensor dm = lower_dm ? *lower_dm : at::matmul(go, v.transpose(2, 3));
+        Tensor dm = lower_dm ? *lower_dm : at::sum_to(at::matmul(go, v.transpose(2, 3)), c.sizes());
         if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
         dm = dm.to(c.scalar_type());
         if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
@@ -442,6 +507,7 @@ Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const
                         double dropout, const py::object &hook)
 {
     const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
+    score_sizes(q, k, v);
     TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout, first, key_bias, empty_rows};
     const Mark mark{hook};
     return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);

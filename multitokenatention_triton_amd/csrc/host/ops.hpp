@@ -211,10 +211,18 @@ inline bool lower_products_supported(at::ScalarType t, int64_t s, int64_t d, boo
     return causal_pv_supported(t, s, d) || (t == at::kFloat && causal && (d == 64 || d == 128) && s % 4 == 0 && s <= (1 << 20));
 }
 
+// whether P (B,H,S,S) and X (B,H,S,D) are what the P V and P^T X kernels take: they index P by X's batch, heads and rows, where
+// the library product broadcasts
+inline bool score_planes_of(c10::IntArrayRef p, c10::IntArrayRef x)
+{
+    return p.size() == 4 && x.size() == 4 && p[0] == x[0] && p[1] == x[1] && p[2] == x[2] && p[3] == x[2];
+}
+
 inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first, double scale)
 {
     const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
-    if (p.scalar_type() != v.scalar_type() || p.size(2) != p.size(3) || !lower_products_supported(p.scalar_type(), v.size(2), v.size(3), causal))
+    if (p.scalar_type() != v.scalar_type() || !score_planes_of(p.sizes(), v.sizes()) ||
+        !lower_products_supported(p.scalar_type(), v.size(2), v.size(3), causal))
         return std::nullopt;
     Tensor o = at::empty(v.sizes(), v.options());
     const int64_t b = v.size(0), h = v.size(1), s = v.size(2), d = v.size(3);
@@ -232,7 +240,8 @@ inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, cons
 inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, double scale)
 {
     const Tensor p = on_gpu(p_, "P"), x = on_gpu(x_, "X");
-    if (p.scalar_type() != x.scalar_type() || p.size(2) != p.size(3) || !lower_products_supported(p.scalar_type(), x.size(2), x.size(3), causal))
+    if (p.scalar_type() != x.scalar_type() || !score_planes_of(p.sizes(), x.sizes()) ||
+        !lower_products_supported(p.scalar_type(), x.size(2), x.size(3), causal))
         return std::nullopt;
     Tensor o = at::empty(x.sizes(), x.options());
     const int64_t b = x.size(0), h = x.size(1), s = x.size(2), d = x.size(3);
@@ -292,6 +301,8 @@ inline Tensor headmix_softmax_tri(const Tensor &x, const OptTensor &w1, const Op
 inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, const OptTensor &first)
 {
     const Tensor v = on_gpu(v_, "V");
+    TORCH_CHECK_VALUE(v.dim() == 4 && p.numel() == v.size(0) * v.size(1) * tri_row_offset(v.size(2)) && p.scalar_type() == v.scalar_type(),
+                      "P in the triangular layout does not belong to a V of shape ", v.sizes());
     Tensor o = at::empty(v.sizes(), v.options());
     check(mta_causal_pv_tri_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), (int)group, code(p, "P"),
                                 stream_of(p)),

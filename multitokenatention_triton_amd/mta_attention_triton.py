@@ -381,7 +381,8 @@ class MTAAttentionTriton(nn.Module):
         self._mark("mix_post")
         # the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
         lower_pv = (self.causal and post.causal and scores.dtype == xv.dtype
-                    and _lower_products_supported(xv, scores.size(-1)) and scores.size(-2) == scores.size(-1))
+                    and _lower_products_supported(xv, scores.size(-1)) and scores.shape[:3] == xv.shape[:3]
+                    and scores.size(-2) == scores.size(-1))
         scores = TritonLinearHeadFunction.apply(scores, post.weight, post.causal, post.output_value, post.group_size,
                                                 not lower_pv, lower)
         scores = F.dropout(scores, p=self.dropout, training=self.training)
@@ -470,6 +471,8 @@ class MTAAttentionTriton(nn.Module):
                 if kind == "keys":
                     return self._forward_native(xq, xk, xv, key_bias=what)
                 if (kind == "band" and self._band_supported(xq, xk)
+                        # (a padded length takes V of the batch and heads of the scores: no library product to broadcast it)
+                        and (xk.size(-2) % 8 == 0 or (xv.shape[:3] == xk.shape[:3] and xv.dtype == xk.dtype))
                         # (rows that see nothing: with 3x5 and 7x9 kernels, which came to the band route last, such masks
                         # stay on the mask passes, whose stages an observer may count on)
                         and (self._band_empty_rows(mask) is None or self.mta_conv_triton.kernel_size not in ((3, 5), (7, 9)))
@@ -516,7 +519,8 @@ class MTAAttentionTriton(nn.Module):
         fu = not cz   # (fill flags of the causal kernels: nothing above the diagonal is anybody's business)
         scale = float(torch.rsqrt(torch.tensor(float(xq.size(-1)))))
         n_keys = xk.size(-2)
-        own_pv = cz and xq.dtype == xv.dtype and ops.causal_pv_supported(xq.dtype, n_keys, xv.size(-1))
+        own_pv = (cz and xq.shape == xk.shape and xv.shape[:3] == xq.shape[:3] and xq.dtype == xv.dtype
+                  and ops.causal_pv_supported(xq.dtype, n_keys, xv.size(-1)))
         self._mark("qk")
         scores = _lower_scores(xq, xk) if cz else None
         if scores is None:
@@ -577,7 +581,7 @@ class MTAAttentionTriton(nn.Module):
     def _band_training_supported(self, xq, xk, xv) -> bool:
         """Whether the differentiable route takes a band mask: data of one dtype and the lower-triangle products (P V and
         its gradients, the recomputed raw scores) as kernels."""
-        return (xq.dtype == xk.dtype == xv.dtype and xq.shape == xk.shape and xv.size(-2) == xk.size(-2)
+        return (xq.dtype == xk.dtype == xv.dtype and xq.shape == xk.shape and xv.shape[:3] == xk.shape[:3]
                 and self.wposm_triton.causal and _lower_kernels(xv) and _lower_kernels(xq))
 
     def _structured_mask(self, mask, bsz: int, s: int):

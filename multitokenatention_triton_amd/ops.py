@@ -601,6 +601,8 @@ def mask_add(x: torch.Tensor, mask: torch.Tensor, causal: bool, out: Optional[to
 def lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """round(a b^T) on and below the diagonal, for a, b (B,H,S,D); see mta_lower_scores_fwd.  Returns ``None`` when
     unsupported."""
+    if a.dim() != 4 or a.shape != b.shape or a.dtype != b.dtype:
+        raise ValueError(f"Q and K must share a (B,H,S,D) shape and dtype, got {tuple(a.shape)}, {tuple(b.shape)}")
     a = _device_tensor(a, "Q")
     b = _device_tensor(b, "K")
     n, h, s, d = a.shape

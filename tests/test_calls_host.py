@@ -1,0 +1,32 @@
+"""CPU-only: calls of the modules that do not fit together are refused ahead of the first stage - with the exception that names
+the misfit, not with the one that says there is no CPU path - so that no kernel reads an operand beyond its end."""
+import pytest
+import torch
+
+import multitokenatention_triton_amd as mta
+
+
+def _module(h=4, dtype=torch.float32, train=False, **kw):
+    mod = mta.MTAAttentionTriton(h, mta.MTAConfig(), 0.0, True, **kw).to(dtype).requires_grad_(train)
+    mod.reset_mta_parameters()
+    seen = []
+    mod._stage_hook = seen.append
+    return mod, seen
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("q,k,v,error,match", [
+    ((2, 4, 16, 64), (2, 4, 16, 64), (2, 8, 16, 64), RuntimeError, "must match"),      # V of more heads
+    ((2, 4, 16, 64), (2, 4, 16, 64), (4, 4, 16, 64), RuntimeError, "must match"),      # ... of more batch entries
+    ((2, 4, 16, 64), (2, 4, 16, 64), (2, 4, 24, 64), RuntimeError, "share their length"),
+    ((2, 4, 13, 64), (2, 4, 13, 64), (2, 4, 16, 64), RuntimeError, "share their length"),
+    ((2, 4, 16, 64), (2, 3, 16, 64), (2, 4, 16, 64), RuntimeError, "must match"),      # K of other heads
+    ((2, 4, 16, 64), (2, 4, 16, 128), (2, 4, 16, 64), RuntimeError, "head size"),
+    ((2, 4, 16, 64), (4, 16, 64), (2, 4, 16, 64), ValueError, "expected Q, K, V"),
+])
+def test_products_that_do_not_exist(q, k, v, error, match, dtype, train):
+    mod, seen = _module(dtype=dtype, train=train)
+    with pytest.raises(error, match=match):
+        mod(*(torch.zeros(s, dtype=dtype) for s in (q, k, v)), None, None)
+    assert seen == []

@@ -1,0 +1,124 @@
+"""Calls beyond the ordinary one (Q, K and V of one shape, whole rows, weights of the data's dtype): what the library products
+take by broadcasting is the same through the kernels.  Against the CPU oracle in fp32, which sees the operands expanded."""
+import pytest
+import torch
+
+from oracle import mta_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+_WEIGHTS = ("mta_conv_triton", "wpsm_triton", "mta_conv_after_sm_triton", "wposm_triton")
+# of the norm: fp32 sums in another order; 16 bits: a chain of about six roundings of 2^-9 / 2^-12 each
+_REL = {torch.float32: 1e-5, torch.bfloat16: 1.5e-2, torch.float16: 2e-3}
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    import multitokenatention_triton_amd as m
+    return m
+
+
+def _module(pkg, h, dtype, wdtype=None, causal=True, use_mask=False, seed=11, **cfg):
+    g = torch.Generator().manual_seed(seed)
+    mod = pkg.MTAAttentionTriton(h, pkg.MTAConfig(**cfg), 0.0, causal, use_mask=use_mask)
+    with torch.no_grad():
+        for name in _WEIGHTS:
+            w = getattr(mod, name).weight
+            if w.dim() == 2:
+                w.copy_(torch.eye(h) + 0.1 * torch.randn(h, h, generator=g))
+            else:
+                w.copy_(O.seeded_conv_weight(h, w.size(1), w.size(2), 0.05, torch.float32, seed=seed))
+    return mod.to(wdtype or dtype).cuda()
+
+
+def _oracle(mod, q, k, v, mask=None):
+    """(output, leaves) of the oracle in fp32; the leaves are q, k, v as given and the four weights."""
+    leaves = [t.float().cpu().clone().requires_grad_(True) for t in (q, k, v)]
+    wl = [getattr(mod, n).weight.detach().float().cpu().clone().requires_grad_(True) for n in _WEIGHTS]
+    b, h = (max(t.size(i) for t in leaves) for i in (0, 1))
+    x = [t.expand(b, mod.n_heads if i < 2 else h, -1, -1) for i, t in enumerate(leaves)]
+    return O.mta_forward(*x, wl[0].unsqueeze(1), wl[1], wl[2].unsqueeze(1), wl[3], mask=mask), leaves + wl
+
+
+def _near(got, want, rel, what=""):
+    got, want = got.detach().float().cpu(), want.detach().float()
+    assert got.shape == want.shape, (what, got.shape, want.shape)
+    assert torch.isfinite(got).all(), what
+    assert float((got - want).norm()) <= rel * float(want.norm()), (what, float((got - want).norm() / want.norm()))
+
+
+@pytest.mark.parametrize("s", [64, 45])
+@pytest.mark.parametrize("dtype,form", [(torch.float32, "v_head"), (torch.float32, "v_batch"), (torch.float32, "k_head"), (torch.float32, "q_batch"),
+                                        (torch.float32, "one_head_many_values"), (torch.float16, "v_head"), (torch.float16, "one_head_many_values")])
+def test_operands_that_broadcast(pkg, dtype, form, s):
+    """V, K or Q of one head or one batch entry, and V of more heads than the scores of a one-head module: the kernels that index
+    the scores by V's sizes are not taken, the result is that of the expanded operands (fp32: with all gradients)."""
+    print(f"broadcast {form} {dtype} s={s}", flush=True)
+    h, d = (1 if form == "one_head_many_values" else 4), 64
+    shapes = [[2, h, s, d] for _ in range(3)]
+    if form == "one_head_many_values":
+        shapes[2][1] = 3
+    else:
+        shapes["qkv".index(form[0])][1 if form.endswith("head") else 0] = 1
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(*sh, generator=g).to(dtype) for sh in shapes)
+    mod = _module(pkg, h, dtype)
+    want, leaves = _oracle(mod, q, k, v)
+    dev = [t.cuda() for t in (q, k, v)]
+    with torch.no_grad():
+        _near(mod(*dev, None, None), want, _REL[dtype], "inference")
+    if dtype != torch.float32:
+        return
+    dev = [t.requires_grad_(True) for t in dev]
+    out = mod(*dev, None, None)
+    _near(out, want, _REL[dtype], "training")
+    go = torch.randn(want.shape, generator=g)
+    want.backward(go)
+    out.backward(go.cuda())
+    for name, a, w in zip("q k v conv pre conv2 post".split(), [t.grad for t in dev] + [getattr(mod, n).weight.grad for n in _WEIGHTS],
+                          [t.grad for t in leaves]):
+        _near(a, w, 1e-4, name)
+
+
+@pytest.mark.parametrize("kind", ["keys", "window"])
+def test_masked_value_heads_that_broadcast(pkg, kind):
+    """Hidden keys and a window with V of one head (fp32, a padded and a whole length): as of the expanded V."""
+    for s in (45, 64):
+        print(f"broadcast under a mask {kind} s={s}", flush=True)
+        mod = _module(pkg, 4, torch.float32, use_mask=True)
+        g = torch.Generator().manual_seed(4)
+        q, k, v = torch.randn(2, 4, s, 64, generator=g), torch.randn(2, 4, s, 64, generator=g), torch.randn(2, 1, s, 64, generator=g)
+        rows = torch.arange(s)
+        visible = (rows[None, :] <= rows[:, None])[None, None].expand(2, 1, s, s).clone()
+        if kind == "keys":
+            visible[1, :, :, s - 9:] = False
+            visible[1, 0, s - 9:, 0] = True
+        else:
+            visible &= (rows[None, :] > rows[:, None] - 17)
+        want, leaves = _oracle(mod, q, k, v, mask=torch.where(visible, 0.0, float("-inf")).expand(2, 4, s, s))
+        dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+        with torch.no_grad():
+            _near(mod(*dev, visible.cuda(), None), want, 1e-5, "inference")
+        out = mod(*dev, visible.cuda(), None)
+        _near(out, want, 1e-5, "training")
+        want.sum().backward()
+        out.sum().backward()
+        for name, a, w in zip("qkv", dev, leaves):
+            _near(a.grad, w.grad, 1e-4, name)
+
+
+def test_more_keys_than_rows(pkg):
+    """causal=False with more keys than query rows (no padding, no row copies): output and the gradients of Q, K and V."""
+    print("more keys than rows", flush=True)
+    mod = _module(pkg, 4, torch.float32, causal=False)
+    g = torch.Generator().manual_seed(5)
+    q, k, v = torch.randn(2, 4, 24, 64, generator=g), torch.randn(2, 4, 40, 64, generator=g), torch.randn(2, 4, 40, 64, generator=g)
+    want, leaves = _oracle(mod, q, k, v, mask=torch.zeros(2, 4, 24, 40))
+    dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    out = mod(*dev, None, None)
+    _near(out, want, 1e-5)
+    go = torch.randn(want.shape, generator=g)
+    want.backward(go)
+    out.backward(go.cuda())
+    for name, a, w in zip("qkv", dev, leaves):
+        _near(a.grad, w.grad, 1e-4, name)
