@@ -109,6 +109,16 @@ at::DimVector score_sizes(const Tensor &q, const Tensor &k, const Tensor &v)
     return s;
 }
 
+// Weights against the heads of the scores: an AssertionError, as the operators raise it, ahead of the first launch.
+void check_weight(const Tensor &w, int64_t dim, int64_t heads, const Tensor &q, const char *what)
+{
+    TORCH_CHECK_VALUE(w.dim() == dim, what, " must have ", dim, " dimensions, got ", w.sizes());
+    TORCH_CHECK(w.device() == q.device(), what, " lives on ", w.device(), ", Q on ", q.device());
+    if (w.size(0) == heads && (dim == 3 || w.size(1) == heads)) return;
+    PyErr_SetString(PyExc_AssertionError, c10::str(what, " ", w.sizes(), " does not match the ", heads, " heads of Q and K").c_str());
+    throw py::error_already_set();
+}
+
 // The length the score kernels work on.  They move score rows as 16-byte vectors; under the causal rule a length that is not
 // a multiple of 8 is padded with zero rows: only padding rows see the padding keys, so every result of a real row is what it
 // was (their gradients are zero: the padding rows of the incoming gradient are).
@@ -165,6 +175,10 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const c10::OptionalDeviceGuard guard(q_.is_cuda() ? std::optional<c10::Device>(q_.device()) : std::nullopt);
     const Mark mark{hook};
     const at::DimVector planes_of = score_sizes(q_, k_, v_);
+    check_weight(conv_w, 3, planes_of[1], q_, "the conv weight");
+    if (!pre_identity) check_weight(w_pre, 2, planes_of[1], q_, "the head weight ahead of the softmax");
+    if (!post_conv_identity) check_weight(post_conv_w, 3, planes_of[1], q_, "the conv weight behind the softmax");
+    if (!post_identity) check_weight(w_post, 2, planes_of[1], q_, "the head weight behind the softmax");
     const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, causal);
     const OptTensor key_bias = cut_columns(key_bias_, s_pad == s_real ? k_.size(2) : s_pad), first = cut_columns(first_, s_pad),
                     empty_rows = cut_columns(empty_rows_, s_pad);
@@ -182,7 +196,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     // (what the padding rows hold is nobody's business)
     auto result = [&](const Tensor &out) { return (s_pad == s_real ? out : out.narrow(2, 0, s_real)).transpose(1, 2); };
     const double scale = score_scale(q);
-    const int64_t heads = w_pre.size(0), n_keys = k.size(-2);
+    const int64_t heads = planes_of[1], n_keys = k.size(-2);
     const OptTensor w1 = pre_identity ? OptTensor() : OptTensor(w_pre), w2 = post_identity ? OptTensor() : OptTensor(w_post);
     const int64_t g_pre = pre_identity ? 1 : pre_group ? pre_group : heads, g_post = post_identity ? 1 : post_group ? post_group : heads;
     const int64_t g_both = lcm(g_pre, g_post);
@@ -507,7 +521,11 @@ Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const
                         double dropout, const py::object &hook)
 {
     const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
-    score_sizes(q, k, v);
+    const int64_t heads = score_sizes(q, k, v)[1];
+    check_weight(conv_w, 3, heads, q, "the conv weight");
+    check_weight(w_pre, 2, heads, q, "the head weight ahead of the softmax");
+    check_weight(post_conv_w, 3, heads, q, "the conv weight behind the softmax");
+    check_weight(w_post, 2, heads, q, "the head weight behind the softmax");
     TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout, first, key_bias, empty_rows};
     const Mark mark{hook};
     return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);

@@ -44,6 +44,16 @@ inline void check(int rc, const char *what)
     TORCH_CHECK(false, what, ": ", mta_strerror(rc), " (code ", rc, ")");
 }
 
+// the kernels index a weight by the data's heads: (C,R,S) conv kernels, (C,C) head weights
+inline void check_conv_weight(const Tensor &w, int64_t heads)
+{
+    TORCH_CHECK(w.dim() == 3 && w.size(0) == heads, "a conv weight of ", heads, " heads must be (", heads, ",R,S), got ", w.sizes());
+}
+inline void check_head_weight(const Tensor &w, int64_t heads)
+{
+    TORCH_CHECK(w.dim() == 2 && w.size(0) == heads && w.size(1) == heads, "Weight must be (", heads, ",", heads, "), got ", w.sizes());
+}
+
 inline const void *ptr(const Tensor &t) { return t.const_data_ptr(); }
 inline const void *ptr(const OptTensor &t) { return t ? t->const_data_ptr() : nullptr; }
 inline void *out_ptr(const Tensor &t) { return t.mutable_data_ptr(); }
@@ -77,6 +87,7 @@ inline Tensor conv2d(const Tensor &x_, const Tensor &w_, bool causal, std::optio
 inline Tensor conv2d_bwd_input(const Tensor &dy_, const Tensor &w_, bool causal, bool fill_upper)
 {
     const Tensor dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    check_conv_weight(w, dy.size(1));
     Tensor dx = at::empty(dy.sizes(), dy.options());
     check(mta_conv2d_bwd_input(ptr(dy), ptr(w), out_ptr(dx), dy.size(0), dy.size(1), dy.size(2), dy.size(3), (int)w.size(1), (int)w.size(2),
                                causal_mode(causal, fill_upper), code(dy, "grad_output"), code(w, "weight"), stream_of(dy)),
@@ -116,6 +127,7 @@ inline Tensor headmix(const Tensor &x_, const Tensor &w_, bool causal, double fi
 inline Tensor headmix_bwd_input(const Tensor &dy_, const Tensor &w_, bool causal, int64_t group, bool fill_upper)
 {
     const Tensor dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    check_head_weight(w, dy.size(1));
     Tensor dx = at::empty(dy.sizes(), dy.options());
     check(mta_headmix_bwd_input(ptr(dy), ptr(w), out_ptr(dx), dy.size(0), dy.size(1), dy.size(2), dy.size(3), (int)group,
                                 causal_mode(causal, fill_upper), code(dy, "grad_output"), code(w, "weight"), stream_of(dy)),
@@ -146,6 +158,8 @@ inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTe
     OptTensor a, b;
     if (w1) a = on_gpu(*w1, "weight");
     if (w2) b = on_gpu(*w2, "weight");
+    for (const OptTensor *w : {&a, &b})
+        if (*w) check_head_weight(**w, x.size(1));
     TORCH_CHECK_TYPE(!a || !b || a->scalar_type() == b->scalar_type(), "w1 and w2 must share a dtype");
     const int wc = a ? code(*a, "weight") : b ? code(*b, "weight") : MTA_F32;
     Tensor y = at::empty(x.sizes(), x.options());
@@ -158,6 +172,8 @@ inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTe
 inline Tensor softmax_bwd(const Tensor &p_, const Tensor &dp_, bool causal, bool fill_upper)
 {
     const Tensor p = on_gpu(p_, "probabilities"), dp = on_gpu(dp_, "grad_output");
+    TORCH_CHECK_VALUE(p.dim() == 4 && p.sizes() == dp.sizes() && p.scalar_type() == dp.scalar_type(),
+                      "probabilities and grad_output must be (N,C,P,Q) tensors of one shape and dtype");
     Tensor dx = at::empty(p.sizes(), p.options());
     check(mta_softmax_bwd(ptr(p), ptr(dp), out_ptr(dx), p.size(0), p.size(1), p.size(2), p.size(3), causal, fill_upper, code(p, "probabilities"),
                           stream_of(p)),
@@ -169,6 +185,8 @@ inline Tensor softmax_bwd(const Tensor &p_, const Tensor &dp_, bool causal, bool
 inline OptTensor conv2d_headmix(const Tensor &x_, const Tensor &wc_, const Tensor &wm_, bool causal, int64_t group, bool fill_upper)
 {
     const Tensor x = on_gpu(x_, "input"), wc = on_gpu(wc_, "conv weight"), wm = on_gpu(wm_, "mix weight");
+    check_conv_weight(wc, x.size(1));
+    check_head_weight(wm, x.size(1));
     Tensor y = at::empty(x.sizes(), x.options());
     const int rc = mta_conv2d_headmix_fwd(ptr(x), ptr(wc), ptr(wm), out_ptr(y), x.size(0), x.size(1), x.size(2), x.size(3), (int)wc.size(1),
                                           (int)wc.size(2), (int)group, causal, fill_upper, code(x, "input"), code(wc, "weight"),
@@ -196,6 +214,7 @@ inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool
 {
     const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
     const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    check_conv_weight(w, h);
     Tensor y = at::empty({b, h, s, s}, q.options());
     const int r = (int)w.size(1), sk = (int)w.size(2), ic = code(q, "Q"), wc = code(w, "W");
     const int rc = first ? mta_qk_conv_band_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, r, sk, (float)scale, fill_upper, ic, wc, stream_of(q))
@@ -277,6 +296,7 @@ inline Tensor qk_conv_tri(const Tensor &q_, const Tensor &k_, const Tensor &w_, 
 {
     const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
     const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    check_conv_weight(w, h);
     Tensor y = at::empty({b * h * tri_row_offset(s)}, q.options());
     check(mta_qk_conv_tri_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, (int)w.size(1), (int)w.size(2), (float)scale, (int)group,
                               code(q, "Q"), code(w, "W"), stream_of(q)),
@@ -290,6 +310,9 @@ inline Tensor headmix_softmax_tri(const Tensor &x, const OptTensor &w1, const Op
     OptTensor a, b;
     if (w1) a = on_gpu(*w1, "weight");
     if (w2) b = on_gpu(*w2, "weight");
+    for (const OptTensor *w : {&a, &b})
+        if (*w) check_head_weight(**w, c);
+    TORCH_CHECK_VALUE(x.dim() == 1 && x.numel() == n * c * tri_row_offset(s), "expected a flat tensor of ", n * c * tri_row_offset(s), " elements");
     Tensor y = out_planes ? at::empty({n, c, s, s}, x.options()) : at::empty(x.sizes(), x.options());
     const int ic = code(x, "input");
     check(mta_headmix_softmax_tri_fwd(ptr(x), ptr(a), ptr(b), ptr(key_bias), ptr(first), out_ptr(y), n, c, s, (int)group, out_planes, ic, ic,

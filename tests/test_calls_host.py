@@ -30,3 +30,32 @@ def test_products_that_do_not_exist(q, k, v, error, match, dtype, train):
     with pytest.raises(error, match=match):
         mod(*(torch.zeros(s, dtype=dtype) for s in (q, k, v)), None, None)
     assert seen == []
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads", [1, 2, 8])
+def test_weights_of_other_head_counts(heads, dtype, train):
+    """A module of 4 heads given tensors of more or fewer: the conv and head kernels index their weights by the data's heads.
+    With the structure declared the stages that would notice later are skipped."""
+    for declare in (False, True):
+        mod, seen = _module(dtype=dtype, train=train)
+        if declare:
+            mod.declare_weight_structure(pre_head_identity=True, post_conv_identity=True, post_head_identity=True)
+        x = torch.zeros(2, heads, 16, 64, dtype=dtype)
+        with pytest.raises(AssertionError, match="heads of Q and K"):
+            mod(x, x, x, None, None)
+        assert seen == []
+
+
+@pytest.mark.parametrize("name", ["mta_conv_triton", "wpsm_triton", "mta_conv_after_sm_triton", "wposm_triton"])
+def test_a_weight_of_another_head_count(name):
+    for train in (False, True):
+        mod, seen = _module(train=train)
+        part = getattr(mod, name)
+        w = part.weight
+        part.weight = torch.nn.Parameter(torch.zeros(8, *((8,) if w.dim() == 2 else w.shape[1:])), requires_grad=train)
+        x = torch.zeros(2, 4, 16, 64)
+        with pytest.raises(AssertionError, match="heads of Q and K"):
+            mod(x, x, x, None, None)
+        assert seen == []
