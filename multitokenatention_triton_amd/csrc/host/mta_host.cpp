@@ -102,6 +102,7 @@ at::DimVector score_sizes(const Tensor &q, const Tensor &k, const Tensor &v)
                       v.sizes());
     TORCH_CHECK(q.size(-1) == k.size(-1), "Q and K must share their head size, got ", q.sizes(), " and ", k.sizes());
     TORCH_CHECK(v.size(v.dim() > 1 ? -2 : 0) == k.size(2), "K and V must share their length, got ", k.sizes(), " and ", v.sizes());
+    TORCH_CHECK(k.device() == q.device() && v.device() == q.device(), "Q, K and V live on ", q.device(), ", ", k.device(), " and ", v.device());
     at::DimVector s = at::infer_size_dimvector(q.sizes().slice(0, q.dim() - 2), k.sizes().slice(0, 2));
     if (v.dim() > 2) at::infer_size_dimvector(s, v.sizes().slice(0, v.dim() - 2));
     s.push_back(q.size(-2));
@@ -128,10 +129,16 @@ int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool ca
     return causal && alike(q, k, v) ? (s + 7) / 8 * 8 : s;
 }
 
-// key_bias, first and empty_rows arrive with the columns of a padded length: without the columns no row of the call has
-OptTensor cut_columns(const OptTensor &t, int64_t s)
+// key_bias (fp32), first (int32) and empty_rows (bool): one value per batch entry of the scores and key (row).  Under the causal
+// rule they arrive with the columns of a padded length; a call that is not padded takes the first `s` of them.
+OptTensor mask_row(const OptTensor &t, at::ScalarType type, const char *what, const at::DimVector &scores, bool causal, int64_t s, const Tensor &q)
 {
-    return !t || t->size(1) == s ? t : OptTensor(t->narrow(1, 0, s).contiguous());
+    if (!t) return t;
+    const int64_t given = causal ? (scores[3] + 7) / 8 * 8 : scores[3];
+    TORCH_CHECK(t->device() == q.device(), what, " lives on ", t->device(), ", Q on ", q.device());
+    TORCH_CHECK_VALUE(t->scalar_type() == type && t->dim() == 2 && t->size(0) == scores[0] && t->size(1) == given, what, " must be ", type, " of shape (",
+                      scores[0], ",", given, "), got ", t->scalar_type(), " ", t->sizes());
+    return (s == given ? *t : t->narrow(1, 0, s)).contiguous();
 }
 
 // (B,H,S,D) with the rows of hidden keys zeroed, where no row copy does it on the way
@@ -180,8 +187,10 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     if (!post_conv_identity) check_weight(post_conv_w, 3, planes_of[1], q_, "the conv weight behind the softmax");
     if (!post_identity) check_weight(w_post, 2, planes_of[1], q_, "the head weight behind the softmax");
     const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, causal);
-    const OptTensor key_bias = cut_columns(key_bias_, s_pad == s_real ? k_.size(2) : s_pad), first = cut_columns(first_, s_pad),
-                    empty_rows = cut_columns(empty_rows_, s_pad);
+    const int64_t columns = s_pad == s_real ? k_.size(2) : s_pad;
+    const OptTensor key_bias = mask_row(key_bias_, at::kFloat, "the key mask", planes_of, causal, columns, q_),
+                    first = mask_row(first_, at::kInt, "the band mask", planes_of, causal, columns, q_),
+                    empty_rows = mask_row(empty_rows_, at::kBool, "the empty rows", planes_of, causal, columns, q_);
     Tensor q = q_, k = k_, v = v_;
     if (key_bias && !alike(q_, k_, v_)) {
         k = zero_hidden(k_, *key_bias);
@@ -337,8 +346,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         const Mark &mark = *mark_;
         const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, o.causal);
         const bool rows_alike = alike(q_, k_, v_);
-        const OptTensor key_bias = cut_columns(o.key_bias, s_pad == s_real ? k_.size(2) : s_pad), first = cut_columns(o.first, s_pad),
-                        empty_rows = cut_columns(o.empty_rows, s_pad);
+        const OptTensor &key_bias = o.key_bias, &first = o.first, &empty_rows = o.empty_rows;
         Tensor q = q_, k = k_, v = v_;
         if (key_bias && !rows_alike) {
             k = zero_hidden(k_, *key_bias);
@@ -521,14 +529,18 @@ Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const
                         double dropout, const py::object &hook)
 {
     const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
-    const int64_t heads = score_sizes(q, k, v)[1];
+    const at::DimVector planes_of = score_sizes(q, k, v);
+    const int64_t heads = planes_of[1], s_pad = padded_length(q, k, v, causal), columns = s_pad == q.size(-2) ? k.size(2) : s_pad;
     check_weight(conv_w, 3, heads, q, "the conv weight");
     check_weight(w_pre, 2, heads, q, "the head weight ahead of the softmax");
     check_weight(post_conv_w, 3, heads, q, "the conv weight behind the softmax");
     check_weight(w_post, 2, heads, q, "the head weight behind the softmax");
-    TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout, first, key_bias, empty_rows};
+    const TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout,
+                         mask_row(first, at::kInt, "the band mask", planes_of, causal, columns, q),
+                         mask_row(key_bias, at::kFloat, "the key mask", planes_of, causal, columns, q),
+                         mask_row(empty_rows, at::kBool, "the empty rows", planes_of, causal, columns, q)};
     const Mark mark{hook};
-    return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, (const TrainOptions *)&o, (const Mark *)&mark);
+    return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, &o, (const Mark *)&mark);
 }
 
 // ---- the two operators ---------------------------------------------------------------------------------------------

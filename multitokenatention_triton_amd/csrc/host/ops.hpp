@@ -160,6 +160,8 @@ inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTe
     if (w2) b = on_gpu(*w2, "weight");
     for (const OptTensor *w : {&a, &b})
         if (*w) check_head_weight(**w, x.size(1));
+    TORCH_CHECK(!key_bias || (key_bias->numel() == x.size(0) * x.size(3) && key_bias->device() == x.device()), "key_bias must be (", x.size(0), ",", x.size(3), ")");
+    TORCH_CHECK(!first || (first->numel() == x.size(0) * x.size(2) && first->device() == x.device()), "first must be (", x.size(0), ",", x.size(2), ")");
     TORCH_CHECK_TYPE(!a || !b || a->scalar_type() == b->scalar_type(), "w1 and w2 must share a dtype");
     const int wc = a ? code(*a, "weight") : b ? code(*b, "weight") : MTA_F32;
     Tensor y = at::empty(x.sizes(), x.options());
@@ -273,6 +275,9 @@ inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, dou
 
 inline void band_zero_(const Tensor &x, const Tensor &first)
 {
+    TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && first.dim() == 2 && first.size(0) == x.size(0) && first.size(1) == x.size(2) &&
+                    first.scalar_type() == at::kInt && first.is_contiguous() && first.device() == x.device(),
+                "a band of ", first.sizes(), " does not belong to scores of ", x.sizes());
     if (is16(x))
         check(mta_band_zero_fwd(out_ptr(x), ptr(first), x.size(0), x.size(1), x.size(2), code(x, "input"), stream_of(x)), "mta_band_zero_fwd");
     else

@@ -457,6 +457,8 @@ class MTAAttentionTriton(nn.Module):
                 return self._forward_native(xq, xk, xv)
             if mask.dim() == 2 and xq.size(0) == 1:
                 assert mask.size(0) == xq.size(0)
+                if mask.size(1) != xk.size(-2):
+                    raise RuntimeError(f"a key mask of {mask.size(1)} keys does not match the {xk.size(-2)} keys of K")
                 if mask.dtype == torch.bool:
                     bias = torch.where(mask, 0.0, float("-inf")).to(torch.float32)
                 else:

@@ -59,3 +59,36 @@ def test_a_weight_of_another_head_count(name):
         with pytest.raises(AssertionError, match="heads of Q and K"):
             mod(x, x, x, None, None)
         assert seen == []
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("s", [13, 16])
+def test_key_masks_that_do_not_fit(s, train):
+    """2-D key masks of another length (also one that pads to the same multiple of 8) and on another device: the kernels read one
+    value per key from the pointer they are given."""
+    mod, seen = _module(train=train, use_mask=True)
+    x = torch.zeros(1, 4, s, 64)
+    for n in (1, s - 1, s + 1, 8):
+        for mask in (torch.ones(1, n, dtype=torch.bool), torch.zeros(1, n)):
+            with pytest.raises(RuntimeError, match="does not match the"):
+                mod(x, x, x, mask, None)
+    with pytest.raises(RuntimeError, match="key mask lives on meta"):
+        mod(x, x, x, torch.ones(1, s, dtype=torch.bool, device="meta"), None)
+    assert seen == []
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_mask_rows_that_do_not_fit(train):
+    """The same for the arrays the module hands to its native routes: batch, length, dtype and device, ahead of the first stage."""
+    mod, seen = _module(train=train)
+    x = torch.zeros(2, 4, 13, 64)     # (causal: 16 columns)
+    good = {"key_bias": torch.zeros(2, 16), "first_visible": torch.zeros(2, 16, dtype=torch.int32), "empty_rows": torch.zeros(2, 16, dtype=torch.bool)}
+    for name, t in good.items():
+        for bad in (t[:1], t[:, :13], t[:, :8], t[0], t.double(), torch.zeros(3, 16, dtype=t.dtype)):
+            with pytest.raises(ValueError, match="must be"):
+                mod._forward_native(x, x, x, **{name: bad})
+        with pytest.raises(RuntimeError, match="lives on meta"):
+            mod._forward_native(x, x, x, **{name: t.to("meta")})
+    with pytest.raises(RuntimeError, match="live on"):
+        mod(x, x, x.to("meta"), None, None)
+    assert seen == []

@@ -122,3 +122,18 @@ def test_more_keys_than_rows(pkg):
     out.backward(go.cuda())
     for name, a, w in zip("qkv", dev, leaves):
         _near(a.grad, w.grad, 1e-4, name)
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_masks_left_on_the_host(pkg, train):
+    """A mask that was not moved to the GPU is refused, for each form that masks take to the kernels."""
+    print(f"masks on the host train={train}", flush=True)
+    mod = _module(pkg, 4, torch.float16, use_mask=True).requires_grad_(train)
+    x = torch.randn(1, 4, 64, 64, dtype=torch.float16, device="cuda")
+    rows = torch.arange(64)
+    causal = (rows[None, :] <= rows[:, None])[None, None]
+    holes = causal & ((rows[None, :] + rows[:, None]) % 5 != 1)
+    for mask in (rows[None] < 50, torch.where(rows[None] < 50, 0.0, -1.0), causal & (rows < 50), causal & (rows[None, :] > rows[:, None] - 9), holes):
+        with pytest.raises(RuntimeError):
+            mod(x, x, x, mask, None)
+    torch.cuda.synchronize()
