@@ -153,9 +153,9 @@ Tensor zero_hidden(const Tensor &x, const Tensor &key_bias)
 OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 {
     if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !a.is_cuda() ||
-        !lower_products_supported(a.scalar_type(), a.size(2), a.size(3), true))
+        !lower_products_supported(a.scalar_type(), a.sizes(), true))
         return std::nullopt;
-    const Tensor x = on_gpu(a, "Q"), y = on_gpu(b, "K");
+    const Tensor x = on_gpu_vectors(a, "Q"), y = on_gpu_vectors(b, "K");
     Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
     check(mta_lower_scores_fwd(ptr(x), ptr(y), is16(x) ? ptr(first) : nullptr, out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
           "mta_lower_scores_fwd");
@@ -214,7 +214,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
     const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && dtype == v.scalar_type() &&
-                        lower_products_supported(dtype, n_keys, v.size(-1), causal);
+                        lower_products_supported(dtype, v.sizes(), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
     // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
@@ -399,7 +399,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         mark("mix_post");
         // the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
         const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && score_planes_of(c.sizes(), v.sizes()) &&
-                              lower_products_supported(v.scalar_type(), n_keys, v.size(-1), true);
+                              lower_products_supported(v.scalar_type(), v.sizes(), true);
         TORCH_CHECK(!first || lower_pv, "the band mask needs the lower-triangle products");
         Tensor m = headmix(c, w_post, o.post_causal, lower_pv ? 0.0 : o.post_fill, o.post_group, !lower_pv), keep;
         if (o.dropout > 0) std::tie(m, keep) = at::native_dropout(m, o.dropout, true);
@@ -497,7 +497,7 @@ struct MtaTraining : torch::autograd::Function<MtaTraining> {
         if (!need_x) return results();
         const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, fill);
         if (need_qk) {
-            const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), k.size(-2), q.size(-1), true);
+            const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), q.sizes(), true);
             const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
             if (first) band_zero_(g, *first);
             if (need[0]) {

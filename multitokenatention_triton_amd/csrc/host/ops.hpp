@@ -34,6 +34,13 @@ inline Tensor on_gpu(const Tensor &t, const char *what)
     return t.is_contiguous() ? t : t.contiguous();
 }
 
+// ... at an address of whole 16-byte vectors: a view into a larger buffer is copied where a library product took it as it was
+inline Tensor on_gpu_vectors(const Tensor &t, const char *what)
+{
+    const Tensor x = on_gpu(t, what);
+    return reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ? x.clone() : x;
+}
+
 inline void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // 0 = ok; negative = argument rejected (ValueError); positive = HIP error (RuntimeError)
@@ -226,10 +233,12 @@ inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool
 }
 
 // whether P V and P^T X run as kernels that read (and P's producer need only write) the lower triangle: 16-bit data, which
-// the kernels also take without the causal rule, or fp32 under it
-inline bool lower_products_supported(at::ScalarType t, int64_t s, int64_t d, bool causal)
+// the kernels also take without the causal rule, or fp32 under it.  x: the (B,H,S,D) operand.
+inline bool lower_products_supported(at::ScalarType t, c10::IntArrayRef x, bool causal)
 {
-    return causal_pv_supported(t, s, d) || (t == at::kFloat && causal && (d == 64 || d == 128) && s % 4 == 0 && s <= (1 << 20));
+    if (x.size() != 4) return false;
+    return causal_pv_supported(t, x[2], x[3]) ||
+           (t == at::kFloat && causal && (x[3] == 64 || x[3] == 128) && x[2] % 4 == 0 && x[2] <= (1 << 20));
 }
 
 // whether P (B,H,S,S) and X (B,H,S,D) are what the P V and P^T X kernels take: they index P by X's batch, heads and rows, where
@@ -241,10 +250,10 @@ inline bool score_planes_of(c10::IntArrayRef p, c10::IntArrayRef x)
 
 inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first, double scale)
 {
-    const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
-    if (p.scalar_type() != v.scalar_type() || !score_planes_of(p.sizes(), v.sizes()) ||
-        !lower_products_supported(p.scalar_type(), v.size(2), v.size(3), causal))
+    if (p_.scalar_type() != v_.scalar_type() || !score_planes_of(p_.sizes(), v_.sizes()) ||
+        !lower_products_supported(p_.scalar_type(), v_.sizes(), causal))
         return std::nullopt;
+    const Tensor p = on_gpu(p_, "P"), v = is16(v_) ? on_gpu(v_, "V") : on_gpu_vectors(v_, "V");
     Tensor o = at::empty(v.sizes(), v.options());
     const int64_t b = v.size(0), h = v.size(1), s = v.size(2), d = v.size(3);
     if (!is16(p)) {   // (the hidden stretch of P holds zeros)
@@ -260,10 +269,10 @@ inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, cons
 
 inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, double scale)
 {
-    const Tensor p = on_gpu(p_, "P"), x = on_gpu(x_, "X");
-    if (p.scalar_type() != x.scalar_type() || !score_planes_of(p.sizes(), x.sizes()) ||
-        !lower_products_supported(p.scalar_type(), x.size(2), x.size(3), causal))
+    if (p_.scalar_type() != x_.scalar_type() || !score_planes_of(p_.sizes(), x_.sizes()) ||
+        !lower_products_supported(p_.scalar_type(), x_.sizes(), causal))
         return std::nullopt;
+    const Tensor p = on_gpu(p_, "P"), x = is16(x_) ? on_gpu(x_, "X") : on_gpu_vectors(x_, "X");
     Tensor o = at::empty(x.sizes(), x.options());
     const int64_t b = x.size(0), h = x.size(1), s = x.size(2), d = x.size(3);
     if (is16(p))

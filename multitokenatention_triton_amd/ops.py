@@ -606,6 +606,8 @@ def lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torch
     a = _device_tensor(a, "Q")
     b = _device_tensor(b, "K")
     n, h, s, d = a.shape
+    if a.dtype == torch.float32 and (a.data_ptr() % 16 or b.data_ptr() % 16):
+        return None   # (the library product takes what is not at the address of a 16-byte vector)
     out = torch.empty((n, h, s, s), dtype=a.dtype, device=a.device)
     first_visible = _band_arg(first_visible, n, s)
     with torch.cuda.device(a.device):

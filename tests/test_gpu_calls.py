@@ -107,6 +107,51 @@ def test_masked_value_heads_that_broadcast(pkg, kind):
             _near(a.grad, w.grad, 1e-4, name)
 
 
+def _misaligned(t):
+    """t at an address that is not that of a 16-byte vector."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+    view = flat[1:].view(t.shape)
+    view.copy_(t)
+    assert view.is_contiguous() and view.data_ptr() % 16
+    return view
+
+
+@pytest.mark.parametrize("mask", [None, "keys", "window", "holes"])
+@pytest.mark.parametrize("dtype,wdtype,which", [(torch.float32, torch.float32, "qkv"), (torch.float32, torch.float32, "v"), (torch.float16, torch.float32, "qk")])
+def test_operands_between_vectors(pkg, dtype, wdtype, which, mask):
+    """Contiguous Q, K and V in the middle of a flat buffer, where the products were the library's before the lower-triangle
+    kernels took them: whole and padded lengths, inference and (fp32) training."""
+    if mask == "holes" and dtype != torch.float32:
+        pytest.skip("the mask passes over 16-bit scores refuse Q and K between vectors")
+    for s in (64, 45):
+        print(f"between vectors {dtype} {which} {mask} s={s}", flush=True)
+        mod = _module(pkg, 4, dtype, wdtype, use_mask=mask is not None)
+        g = torch.Generator().manual_seed(6)
+        q, k, v = (torch.randn(2, 4, s, 64, generator=g).to(dtype) for _ in range(3))
+        rows = torch.arange(s)
+        visible = (rows[None, :] <= rows[:, None])[None, None]
+        if mask == "keys":
+            visible = visible & (rows < s - 7)
+        elif mask == "window":
+            visible = visible & (rows[None, :] > rows[:, None] - 17)
+        elif mask == "holes":
+            visible = visible & ((rows[None, :] + rows[:, None]) % 5 != 1)
+        want, leaves = _oracle(mod, q, k, v, mask=torch.where(visible, 0.0, float("-inf")).expand(2, 4, s, s))
+        dev = [_misaligned(t) if n in which else t.cuda() for n, t in zip("qkv", (q, k, v))]
+        given = None if mask is None else visible.cuda()
+        with torch.no_grad():
+            _near(mod(*dev, given, None), want, _REL[dtype], "inference")
+        if dtype != torch.float32:
+            continue
+        dev = [t.requires_grad_(True) for t in dev]
+        out = mod(*dev, given, None)
+        _near(out, want, _REL[dtype], "training")
+        want.sum().backward()
+        out.sum().backward()
+        for name, a, w in zip("qkv", dev, leaves):
+            _near(a.grad, w.grad, 1e-4, name)
+
+
 def test_more_keys_than_rows(pkg):
     """causal=False with more keys than query rows (no padding, no row copies): output and the gradients of Q, K and V."""
     print("more keys than rows", flush=True)
