@@ -28,6 +28,7 @@ bool no_row_lists()
 bool one_pass_group(int64_t group, at::ScalarType t, int64_t n_keys, const OptTensor &w1, const OptTensor &w2)
 {
     if (group <= FUSED_MAX_GROUP) return true;
+    if (w1 && w2 && w1->scalar_type() != w2->scalar_type()) return false;   // (one kernel takes its two weights in one dtype)
     if (t == at::kFloat) return n_keys % 4 == 0 && n_keys <= mta_headmix_softmax_dense_f32_keys((int)std::min<int64_t>(group, 1 << 20));
     return group == FUSED_MFMA_GROUP && (t == at::kBFloat16 || t == at::kHalf) && n_keys % 8 == 0 && n_keys <= FUSED_MFMA_MAX_KEYS &&
            (!w1 || w1->scalar_type() == t) && (!w2 || w2->scalar_type() == t);

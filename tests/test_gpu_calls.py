@@ -152,6 +152,21 @@ def test_operands_between_vectors(pkg, dtype, wdtype, which, mask):
             _near(a.grad, w.grad, 1e-4, name)
 
 
+@pytest.mark.parametrize("h", [12, 16, 32])
+def test_head_weights_of_two_dtypes(pkg, h):
+    """fp32 data, dense head weights of which one is kept in 16 bits, no conv between them: mix, softmax and mix one by one."""
+    print(f"head weights of two dtypes h={h}", flush=True)
+    for name in ("wpsm_triton", "wposm_triton"):
+        mod = _module(pkg, h, torch.float32).requires_grad_(False)
+        getattr(mod, name).to(torch.bfloat16)
+        mod.mta_conv_after_sm_triton.weight.zero_()[:, -1, 1] = 1.0
+        mod.declare_weight_structure(post_conv_identity=True)
+        g = torch.Generator().manual_seed(8)
+        q, k, v = (torch.randn(2, h, 64, 64, generator=g) for _ in range(3))
+        want, _ = _oracle(mod, q, k, v)
+        _near(mod(q.cuda(), k.cuda(), v.cuda(), None, None), want, 1e-5, name)
+
+
 def test_more_keys_than_rows(pkg):
     """causal=False with more keys than query rows (no padding, no row copies): output and the gradients of Q, K and V."""
     print("more keys than rows", flush=True)
