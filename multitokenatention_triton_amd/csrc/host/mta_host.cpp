@@ -329,222 +329,302 @@ struct TrainOptions {
     bool causal, pre_causal, post_causal;
     double pre_fill, post_fill;
     int64_t pre_group, post_group;   // 0 = dense (the weight gradient is then dense too)
-    double dropout;
     OptTensor first;       // int32 (B,S), a band mask
     OptTensor key_bias;    // fp32 (B,S): added ahead of the softmax; the K and V rows of the keys it hides (-inf) count as zeros
                            // and receive no gradient, as in the reference, whose masked_fill / where cut it
     OptTensor empty_rows;  // bool (B,S), the rows of the band that see no key: their probabilities are cleared
 };
 
-// The reference's operator sequence (mta_attention_triton.py:68-92) as one differentiable function.  Between two stages
-// nothing reads above the diagonal when causal (the kernels never do, in either direction), so nothing is written there,
-// except what goes into a library GEMM.
-struct MtaTraining : torch::autograd::Function<MtaTraining> {
-    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w,
-                          const Tensor &w_pre, const Tensor &post_conv_w, const Tensor &w_post, const TrainOptions *opt, const Mark *mark_)
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+OptTensor option(const Tensor &t) { return t.defined() ? OptTensor(t) : OptTensor(); }
+Tensor tensor(const OptTensor &t) { return t ? *t : Tensor(); }
+
+// The reference's operator sequence (mta_attention_triton.py:68-92) in pieces, forward and backward.  Between two stages nothing
+// reads above the diagonal when causal (the kernels never do, in either direction), so nothing is written there, except what goes
+// into a library GEMM.
+
+// Q K^T -> factor -> conv -> head mixing -> softmax.  raw: the raw scores, kept where the first stage is two operators; x: the
+// conv's result.
+Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, const TrainOptions &o, const Mark &mark, Tensor &raw,
+                     Tensor &x)
+{
+    const double scale = score_scale(q);
+    const bool fill = !o.causal;
+    if (qk_conv_supported(q, k, conv_w)) {
+        mark("qk_conv");
+        x = qk_conv(q, k, conv_w, o.causal, scale, false, o.first);
+        // The kernel leaves the key blocks that no row of a query block sees unwritten.  The softmax stage does not read
+        // a row's hidden stretch, but its weight gradient multiplies what is stored there by a gradient that is 0: the
+        // stretch is cleared, so that the product is 0 too.
+        if (o.first) band_zero_(x, *o.first);
+    } else {
+        mark("qk");
+        const OptTensor lower_raw = o.causal ? lower_scores(q, k, o.first) : OptTensor();
+        TORCH_CHECK(lower_raw || !o.first, "the band mask needs the lower-triangle products");
+        raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
+        mark("conv_pre");
+        x = conv2d(raw, conv_w, o.causal, scale, false);
+    }
+    const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
+    const auto dtype = x.scalar_type();
+    Tensor p;
+    if ((!stages_apart(g_eff, dtype) || o.pre_causal == o.causal) && one_pass_group(g_eff, dtype, n_keys, w_pre, OptTensor()) &&
+        masks_ok(g_eff, dtype, o.key_bias || o.first)) {
+        if (stages_apart(g_eff, dtype)) {
+            mark("mix_pre");
+            mark("softmax");
+        } else {
+            mark("mix_softmax");
+        }
+        p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
+    } else {
+        mark("mix_pre");
+        const Tensor m = headmix(x, w_pre, o.pre_causal, fill ? o.pre_fill : 0.0, o.pre_group, fill);
+        mark("softmax");
+        p = headmix_softmax(m, OptTensor(), OptTensor(), o.causal, 0, fill, o.key_bias, o.first);
+    }
+    if (o.empty_rows) band_zero_(p, empty_row_ends(*o.empty_rows));
+    return p;
+}
+
+// the gradients of q, k, conv_w and w_pre (need[i]: wanted) from the one of the probabilities p
+void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, Tensor raw, const Tensor &x, const Tensor &p,
+                       const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4])
+{
+    const double scale = score_scale(q);
+    // (the head mixing's gradient kernels never read above the diagonal when causal)
+    Tensor ds = softmax_bwd(p, dp, causal, false);
+    dp.reset();
+    if (need[3]) *out[3] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
+    if (!need[0] && !need[1] && !need[2]) return;
+    const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, !causal);
+    ds.reset();
+    if (need[0] || need[1]) {
+        const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), q.sizes(), true);
+        const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
+        if (first) band_zero_(g, *first);
+        Tensor dq, dk;
+        OptTensor own_q, own_k;
+        if (need[0]) own_q = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
+        if (need[0]) dq = own_q ? *own_q : at::matmul(g, k);
+        if (need[1]) own_k = lower ? causal_ptx(g, q, true, scale) : OptTensor();
+        if (need[1]) dk = own_k ? *own_k : at::matmul(g.transpose(2, 3), q);
+        // the factor, where the products were the library's
+        if (need[0] && need[1] && !own_q && !own_k && dq.sizes() == dk.sizes()) {
+            RowsCopy rows(dq.size(2), OptTensor());
+            dq = rows.add(dq, false, scale);
+            dk = rows.add(dk, false, scale);
+            rows.run();
+        } else {
+            if (need[0] && !own_q) dq = dq * scale;
+            if (need[1] && !own_k) dk = dk * scale;
+        }
+        *out[0] = dq;
+        *out[1] = dk;
+    }
+    if (need[2]) {
+        if (!raw.defined()) {   // (the kernel gradient reads its first argument on and below the diagonal only)
+            const OptTensor lower_raw = causal ? lower_scores(q, k, first) : OptTensor();
+            TORCH_CHECK(lower_raw || !first);
+            raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
+        }
+        *out[2] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale);
+    }
+}
+
+// whether M V and its gradients run on the lower triangle of M (the last stage's output): by the library GEMM M is read in full
+bool lower_values(const Tensor &m, const Tensor &v, const TrainOptions &o)
+{
+    const bool lower = o.causal && o.post_causal && m.scalar_type() == v.scalar_type() && score_planes_of(m.sizes(), v.sizes()) &&
+                       lower_products_supported(v.scalar_type(), v.sizes(), true);
+    TORCH_CHECK(!o.first || lower, "the band mask needs the lower-triangle products");
+    return lower;
+}
+
+// M V, seen as (B,S,H,D), its first s_real rows
+Tensor values(const Tensor &m, const Tensor &v, bool lower, int64_t s_real, const OptTensor &first)
+{
+    const Tensor out = lower ? *causal_pv(m, v, true, first, 1.0) : at::matmul(m, v);
+    return heads_last(out, s_real == m.size(2) ? -1 : s_real);
+}
+
+// the incoming gradient as (B,H,S,D), padded with zero rows
+Tensor value_rows(const Tensor &grad, int64_t s_pad)
+{
+    const Tensor go = grad.transpose(1, 2);
+    if (go.dim() != 4 || go.numel() >= (int64_t(1) << 31)) return go.contiguous();   // (beyond what a padded length is used for)
+    RowsCopy rows(s_pad, OptTensor());
+    const Tensor out = rows.add(go, false, 1.0);
+    rows.run();
+    return out;
+}
+
+Tensor values_bwd_v(const Tensor &m, const Tensor &go, bool lower)
+{
+    const OptTensor own = lower ? causal_ptx(m, go, true, 1.0) : OptTensor();
+    return own ? *own : at::matmul(m.transpose(2, 3), go);
+}
+
+// (first: the gradient is formed inside the band)
+Tensor values_bwd_m(const Tensor &go, const Tensor &v, bool lower, const OptTensor &first)
+{
+    const OptTensor own = lower ? lower_scores(go, v, first) : OptTensor();
+    TORCH_CHECK(own || !first);
+    return own ? *own : at::matmul(go, v.transpose(2, 3));
+}
+
+// The pieces as one node: the host's time is what bounds a step of small tensors (a node costs about 8.6 us of it, forward and
+// backward together).  Everything saved stays to the end of backward, so only for score tensors of up to WHOLE_STEP_BYTES, where
+// that is at most five of them more at the peak (80 MB); beyond, the step is the kernels' time and a node per score tensor costs
+// nothing.  us a step, one node | four (timed in turn; from process to process the host's part differs by as much): B1 H8 S256 D64
+// bf16 (1 MB a score tensor) 181 | 205, B1 H16 S512 D128 (8 MB) 174 | 191, B1 H16 S1024 D64 (32 MB) 239 | 239.
+constexpr int64_t WHOLE_STEP_BYTES = int64_t(16) << 20;
+
+struct WholeStep : torch::autograd::Function<WholeStep> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre,
+                          const Tensor &post_conv_w, const Tensor &w_post, int64_t s_pad, double dropout, const TrainOptions *opt, const Mark *mark_)
     {
         const TrainOptions &o = *opt;
         const Mark &mark = *mark_;
-        const int64_t s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, o.causal);
-        const bool rows_alike = alike(q_, k_, v_);
-        const OptTensor &key_bias = o.key_bias, &first = o.first, &empty_rows = o.empty_rows;
+        const int64_t s_real = q_.size(2);
         Tensor q = q_, k = k_, v = v_;
-        if (key_bias && !rows_alike) {
-            k = zero_hidden(k_, *key_bias);
-            v = zero_hidden(v_, *key_bias);
-        } else if (s_pad != s_real || key_bias) {
-            RowsCopy rows(s_pad, key_bias);
+        if (s_pad != s_real || o.key_bias) {
+            RowsCopy rows(s_pad, o.key_bias);
             if (s_pad != s_real) q = rows.add(q_, false, 1.0);
             k = rows.add(k_, true, 1.0);
             v = rows.add(v_, true, 1.0);
             rows.run();
         }
-        const double scale = score_scale(q);
-        const bool fill = !o.causal;
-        Tensor raw, x;   // raw scores (kept where the first stage is two operators), conv result
-        if (qk_conv_supported(q, k, conv_w)) {
-            mark("qk_conv");
-            x = qk_conv(q, k, conv_w, o.causal, scale, false, first);
-            // The kernel leaves the key blocks that no row of a query block sees unwritten.  The softmax stage does not read
-            // a row's hidden stretch, but its weight gradient multiplies what is stored there by a gradient that is 0: the
-            // stretch is cleared, so that the product is 0 too.
-            if (first) band_zero_(x, *first);
-        } else {
-            mark("qk");
-            const OptTensor lower_raw = o.causal ? lower_scores(q, k, first) : OptTensor();
-            TORCH_CHECK(lower_raw || !first, "the band mask needs the lower-triangle products");
-            raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
-            mark("conv_pre");
-            x = conv2d(raw, conv_w, o.causal, scale, false);
-        }
-        const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
-        Tensor p;
-        if ((!stages_apart(g_eff, x.scalar_type()) || o.pre_causal == o.causal) && one_pass_group(g_eff, x.scalar_type(), n_keys, w_pre, OptTensor()) && masks_ok(g_eff, x.scalar_type(), key_bias || first)) {
-            if (stages_apart(g_eff, x.scalar_type())) {
-                mark("mix_pre");
-                mark("softmax");
-            } else {
-                mark("mix_softmax");
-            }
-            p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, key_bias, first);
-        } else {
-            mark("mix_pre");
-            const Tensor m = headmix(x, w_pre, o.pre_causal, fill ? o.pre_fill : 0.0, o.pre_group, fill);
-            mark("softmax");
-            p = headmix_softmax(m, OptTensor(), OptTensor(), o.causal, 0, fill, key_bias, first);
-        }
-        if (empty_rows) band_zero_(p, empty_row_ends(*empty_rows));
+        Tensor raw, x, keep;
+        const Tensor p = probabilities(q, k, conv_w, w_pre, o, mark, raw, x);
         mark("conv_post");
-        Tensor c = conv2d(p, post_conv_w, o.causal, std::nullopt, fill);
-        if (first) band_zero_(c, *first);
+        const Tensor c = conv2d(p, post_conv_w, o.causal, std::nullopt, !o.causal);
+        if (o.first) band_zero_(c, *o.first);
         mark("mix_post");
-        // the last stage's output is read by P V: in full by the library GEMM, on and below the diagonal by our kernels
-        const bool lower_pv = o.causal && o.post_causal && c.scalar_type() == v.scalar_type() && score_planes_of(c.sizes(), v.sizes()) &&
-                              lower_products_supported(v.scalar_type(), v.sizes(), true);
-        TORCH_CHECK(!first || lower_pv, "the band mask needs the lower-triangle products");
-        Tensor m = headmix(c, w_post, o.post_causal, lower_pv ? 0.0 : o.post_fill, o.post_group, !lower_pv), keep;
-        if (o.dropout > 0) std::tie(m, keep) = at::native_dropout(m, o.dropout, true);
+        const bool lower = lower_values(c, v, o);
+        Tensor m = headmix(c, w_post, o.post_causal, lower ? 0.0 : o.post_fill, o.post_group, !lower);
+        if (dropout > 0) std::tie(m, keep) = at::native_dropout(m, dropout, true);
         mark("pv");
-        Tensor out = lower_pv ? *causal_pv(m, v, true, first, 1.0) : at::matmul(m, v);
+        const Tensor out = values(m, v, lower, s_real, o.first);
         mark("end");
-        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, first ? *first : Tensor(),
-                                key_bias ? *key_bias : Tensor()});
+        ctx->save_for_backward({q, k, v, conv_w, w_pre, post_conv_w, w_post, raw, x, p, c, m, keep, tensor(o.first), tensor(o.key_bias)});
         ctx->saved_data["s_real"] = s_real;
-        ctx->saved_data["alike"] = rows_alike;
         ctx->saved_data["causal"] = o.causal;
         ctx->saved_data["pre_causal"] = o.pre_causal;
         ctx->saved_data["post_causal"] = o.post_causal;
         ctx->saved_data["pre_group"] = o.pre_group;
         ctx->saved_data["post_group"] = o.post_group;
-        ctx->saved_data["dropout"] = o.dropout;
-        ctx->saved_data["lower_pv"] = lower_pv;
-        return heads_last(out, s_pad == s_real ? -1 : s_real);
+        ctx->saved_data["dropout"] = dropout;
+        ctx->saved_data["lower"] = lower;
+        return out;
     }
 
-    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads)
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &conv_w = saved[3], &w_pre = saved[4], &post_conv_w = saved[5],
-                     &w_post = saved[6], &x = saved[8], &p = saved[9], &c = saved[10], &m = saved[11], &keep = saved[12];
-        Tensor raw = saved[7];
-        const OptTensor first = saved[13].defined() ? OptTensor(saved[13]) : OptTensor(),
-                        key_bias = saved[14].defined() ? OptTensor(saved[14]) : OptTensor();
-        const int64_t s_real = ctx->saved_data["s_real"].toInt(), s_pad = q.size(-2);
-        const bool rows_alike = ctx->saved_data["alike"].toBool();
+                     &w_post = saved[6], &raw = saved[7], &x = saved[8], &p = saved[9], &c = saved[10], &m = saved[11], &keep = saved[12];
+        const OptTensor first = option(saved[13]), key_bias = option(saved[14]);
+        const int64_t s_real = ctx->saved_data["s_real"].toInt(), s_pad = q.size(2);
         const bool causal = ctx->saved_data["causal"].toBool(), pre_causal = ctx->saved_data["pre_causal"].toBool(),
-                   post_causal = ctx->saved_data["post_causal"].toBool(), lower_pv = ctx->saved_data["lower_pv"].toBool();
+                   post_causal = ctx->saved_data["post_causal"].toBool(), lower = ctx->saved_data["lower"].toBool();
         const int64_t pre_group = ctx->saved_data["pre_group"].toInt(), post_group = ctx->saved_data["post_group"].toInt();
-        const double dropout = ctx->saved_data["dropout"].toDouble(), scale = score_scale(q);
-        const bool fill = !causal;
+        const double dropout = ctx->saved_data["dropout"].toDouble();
         const c10::OptionalDeviceGuard guard(q.device());
         bool need[7];
         for (int i = 0; i < 7; ++i) need[i] = ctx->needs_input_grad(i);
-        const bool need_qk = need[0] || need[1], need_x = need_qk || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
-        torch::autograd::variable_list out(9);
-
-        Tensor go;   // (B,H,S,D), padded with zero rows
-        if (!rows_alike) {
-            go = grads[0].transpose(1, 2).contiguous();
-        } else {
-            RowsCopy rows(s_pad, OptTensor());
-            go = rows.add(grads[0].transpose(1, 2), false, 1.0);
-            rows.run();
-        }
-        // the gradients of Q, K and V leave without the padding, without what the hidden keys' rows hold, and with the factor
-        const bool cut = s_pad != s_real;
-        Tensor dq, dk, dv;
-        double dq_scale = 1.0, dk_scale = 1.0;
-        auto results = [&] {
-            if (!rows_alike) {
-                auto leave = [&](const Tensor &g, bool hide, double factor) {
-                    if (!g.defined()) return g;
-                    const Tensor scaled = factor != 1.0 ? g * factor : g;
-                    return hide && key_bias ? zero_hidden(scaled, *key_bias) : scaled;
-                };
-                out[0] = leave(dq, false, dq_scale);
-                out[1] = leave(dk, true, dk_scale);
-                out[2] = leave(dv, true, 1.0);
-                return out;
-            }
-            RowsCopy rows(s_real, key_bias);
-            auto leave = [&](Tensor &g, bool hide, double factor) {
-                return g.defined() && (cut || (hide && key_bias) || factor != 1.0) ? rows.add(g, hide, factor) : g;
-            };
-            out[0] = leave(dq, false, dq_scale);
-            out[1] = leave(dk, true, dk_scale);
-            out[2] = leave(dv, true, 1.0);
-            rows.run();
-            return out;
-        };
-        if (need[2]) {
-            const OptTensor own = lower_pv ? causal_ptx(m, go, true, 1.0) : OptTensor();
-            dv = own ? *own : at::matmul(m.transpose(2, 3), go);
-        }
-        if (!need_c && !need[6]) return results();
-        const OptTensor lower_dm = lower_pv ? lower_scores(go, v, first) : OptTensor();
-        TORCH_CHECK(lower_dm || !first);
-        Tensor dm = lower_dm ? *lower_dm : at::sum_to(at::matmul(go, v.transpose(2, 3)), c.sizes());
-        if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
-        dm = dm.to(c.scalar_type());
-        if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
-        if (!need_c) return results();
-        const Tensor dc = headmix_bwd_input(dm, w_post, post_causal, post_group, fill);
-        if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
-        if (!need_p) return results();
-        const Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, fill);
-        // (the head mixing's gradient kernels never read above the diagonal when causal)
-        const Tensor ds = softmax_bwd(p, dp, causal, false);
-        if (need[4]) out[4] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
-        if (!need_x) return results();
-        const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, fill);
-        if (need_qk) {
-            const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), q.sizes(), true);
-            const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
-            if (first) band_zero_(g, *first);
-            if (need[0]) {
-                const OptTensor own = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
-                dq = own ? *own : at::matmul(g, k);
-                if (!own) dq_scale = scale;
-            }
-            if (need[1]) {
-                const OptTensor own = lower ? causal_ptx(g, q, true, scale) : OptTensor();
-                dk = own ? *own : at::matmul(g.transpose(2, 3), q);
-                if (!own) dk_scale = scale;
+        const bool need_x = need[0] || need[1] || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
+        variable_list out(11);
+        const Tensor go = value_rows(grads[0], s_pad);
+        if (need[2]) out[2] = values_bwd_v(m, go, lower);
+        if (need_c || need[6]) {
+            Tensor dm = values_bwd_m(go, v, lower, first);
+            if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
+            if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
+            Tensor dc = need_c ? headmix_bwd_input(dm, w_post, post_causal, post_group, !causal) : Tensor();
+            dm.reset();
+            if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
+            if (need_p) {
+                Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, !causal);
+                dc.reset();
+                probabilities_bwd(q, k, conv_w, w_pre, raw, x, p, first, causal, pre_causal, pre_group, std::move(dp), {need[0], need[1], need[3], need[4]},
+                                  {&out[0], &out[1], &out[3], &out[4]});
             }
         }
-        if (need[3]) {
-            if (!raw.defined()) {   // (the kernel gradient reads its first argument on and below the diagonal only)
-                const OptTensor lower_raw = causal ? lower_scores(q, k, first) : OptTensor();
-                TORCH_CHECK(lower_raw || !first);
-                raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
-            }
-            out[3] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale);
-        }
-        return results();
+        // the gradients of Q, K and V leave without the padding and without what the hidden keys' rows hold
+        RowsCopy rows(s_real, key_bias);
+        for (int i = 0; i < 3; ++i)
+            if (out[i].defined() && (s_pad != s_real || (i > 0 && key_bias))) out[i] = rows.add(out[i], i > 0, 1.0);
+        rows.run();
+        return out;
     }
 };
 
-Tensor forward_training(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
-                        const Tensor &w_post, bool causal, bool pre_causal, bool post_causal, double pre_fill, double post_fill,
-                        int64_t pre_group, int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows,
-                        double dropout, const py::object &hook)
-{
-    const c10::OptionalDeviceGuard guard(q.is_cuda() ? std::optional<c10::Device>(q.device()) : std::nullopt);
-    const at::DimVector planes_of = score_sizes(q, k, v);
-    const int64_t heads = planes_of[1], s_pad = padded_length(q, k, v, causal), columns = s_pad == q.size(-2) ? k.size(2) : s_pad;
-    check_weight(conv_w, 3, heads, q, "the conv weight");
-    check_weight(w_pre, 2, heads, q, "the head weight ahead of the softmax");
-    check_weight(post_conv_w, 3, heads, q, "the conv weight behind the softmax");
-    check_weight(w_post, 2, heads, q, "the head weight behind the softmax");
-    const TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group, dropout,
-                         mask_row(first, at::kInt, "the band mask", planes_of, causal, columns, q),
-                         mask_row(key_bias, at::kFloat, "the key mask", planes_of, causal, columns, q),
-                         mask_row(empty_rows, at::kBool, "the empty rows", planes_of, causal, columns, q)};
-    const Mark mark{hook};
-    return MtaTraining::apply(q, k, v, conv_w, w_pre, post_conv_w, w_post, &o, (const Mark *)&mark);
-}
+// ---- ... and as one node per score tensor that is kept: the engine frees what a node has saved and the gradient it was given
+// when the node is done, so that backward holds the four saved tensors (x, p, c, m; raw too where there is one) and one or two
+// gradients at a time.
 
-// ---- the two operators ---------------------------------------------------------------------------------------------
+// The tensors in a padded length, the rows of hidden keys zeroed from the `hide_from`th on; backward: without the padding and
+// without what those rows got.
+struct PadRows : torch::autograd::Function<PadRows> {
+    static variable_list forward(AutogradContext *ctx, at::TensorList xs, int64_t hide_from, int64_t s_pad, const OptTensor *key_bias)
+    {
+        ctx->save_for_backward({tensor(*key_bias)});
+        ctx->saved_data["s_real"] = xs[0].size(2);
+        ctx->saved_data["hide_from"] = hide_from;
+        variable_list out;
+        RowsCopy rows(s_pad, *key_bias);
+        for (const Tensor &x : xs) out.push_back(rows.add(x, (int64_t)out.size() >= hide_from, 1.0));
+        rows.run();
+        return out;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const OptTensor key_bias = option(ctx->get_saved_variables()[0]);
+        const int64_t s_real = ctx->saved_data["s_real"].toInt(), hide_from = ctx->saved_data["hide_from"].toInt();
+        const c10::OptionalDeviceGuard guard(grads[0].device());
+        RowsCopy rows(s_real, key_bias);
+        variable_list out(grads.size() + 3);
+        for (size_t i = 0; i < grads.size(); ++i) {
+            if (!ctx->needs_input_grad(i)) continue;
+            const bool hide = (int64_t)i >= hide_from && key_bias;
+            out[i] = hide || grads[i].size(2) != s_real ? rows.add(grads[i], hide, 1.0) : grads[i];
+        }
+        rows.run();
+        return out;
+    }
+};
+
+struct Probabilities : torch::autograd::Function<Probabilities> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, const TrainOptions *o,
+                          const Mark *mark)
+    {
+        Tensor raw, x;
+        const Tensor p = probabilities(q, k, conv_w, w_pre, *o, *mark, raw, x);
+        ctx->save_for_backward({q, k, conv_w, w_pre, raw, x, p, tensor(o->first)});
+        ctx->saved_data["causal"] = o->causal;
+        ctx->saved_data["pre_causal"] = o->pre_causal;
+        ctx->saved_data["pre_group"] = o->pre_group;
+        return p;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto s = ctx->get_saved_variables();
+        const c10::OptionalDeviceGuard guard(s[0].device());
+        variable_list out(6);
+        probabilities_bwd(s[0], s[1], s[2], s[3], s[4], s[5], s[6], option(s[7]), ctx->saved_data["causal"].toBool(),
+                          ctx->saved_data["pre_causal"].toBool(), ctx->saved_data["pre_group"].toInt(), grads[0].to(s[6].scalar_type()),
+                          {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)},
+                          {&out[0], &out[1], &out[2], &out[3]});
+        return out;
+    }
+};
+
+// the two operators: nodes of their own, and the post-softmax conv and head mixing of a training step
 struct Conv2d : torch::autograd::Function<Conv2d> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &w, bool causal, bool fill_upper, bool grad_fill_upper)
     {
@@ -594,6 +674,75 @@ struct HeadMix : torch::autograd::Function<HeadMix> {
     }
 };
 
+struct Values : torch::autograd::Function<Values> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &m, const Tensor &v, bool lower, int64_t s_real, const OptTensor *first)
+    {
+        ctx->save_for_backward({m, v, tensor(*first)});
+        ctx->saved_data["lower"] = lower;
+        return values(m, v, lower, s_real, *first);
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const auto s = ctx->get_saved_variables();
+        const c10::OptionalDeviceGuard guard(s[0].device());
+        const bool lower = ctx->saved_data["lower"].toBool();
+        const Tensor go = value_rows(grads[0], s[0].size(2));
+        variable_list out(5);
+        if (ctx->needs_input_grad(1)) out[1] = values_bwd_v(s[0], go, lower);
+        if (ctx->needs_input_grad(0)) out[0] = values_bwd_m(go, s[1], lower, option(s[2]));
+        return out;
+    }
+};
+
+Tensor forward_training(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
+                        const Tensor &w_post, bool causal, bool pre_causal, bool post_causal, double pre_fill, double post_fill,
+                        int64_t pre_group, int64_t post_group, const OptTensor &key_bias, const OptTensor &first, const OptTensor &empty_rows,
+                        double dropout, const py::object &hook)
+{
+    const c10::OptionalDeviceGuard guard(q_.is_cuda() ? std::optional<c10::Device>(q_.device()) : std::nullopt);
+    const at::DimVector planes_of = score_sizes(q_, k_, v_);
+    const int64_t heads = planes_of[1], s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, causal), columns = s_pad == s_real ? k_.size(2) : s_pad;
+    check_weight(conv_w, 3, heads, q_, "the conv weight");
+    check_weight(w_pre, 2, heads, q_, "the head weight ahead of the softmax");
+    check_weight(post_conv_w, 3, heads, q_, "the conv weight behind the softmax");
+    check_weight(w_post, 2, heads, q_, "the head weight behind the softmax");
+    const TrainOptions o{causal, pre_causal, post_causal, pre_fill, post_fill, pre_group, post_group,
+                         mask_row(first, at::kInt, "the band mask", planes_of, causal, columns, q_),
+                         mask_row(key_bias, at::kFloat, "the key mask", planes_of, causal, columns, q_),
+                         mask_row(empty_rows, at::kBool, "the empty rows", planes_of, causal, columns, q_)};
+    const Mark mark{hook};
+    const bool rows_alike = alike(q_, k_, v_);
+    if (rows_alike && planes_of[0] * heads * s_pad * s_pad * (int64_t)q_.element_size() <= WHOLE_STEP_BYTES)
+        return WholeStep::apply(q_, k_, v_, conv_w, w_pre, post_conv_w, w_post, s_pad, dropout, &o, &mark);
+    Tensor q = q_, k = k_, v = v_;
+    if (o.key_bias && !rows_alike) {
+        k = zero_hidden(k_, *o.key_bias);
+        v = zero_hidden(v_, *o.key_bias);
+    } else if (s_pad != s_real || o.key_bias) {
+        const bool pad = s_pad != s_real;
+        const Tensor given[3] = {q_, k_, v_};
+        const auto rows = PadRows::apply(at::TensorList(given + !pad, 2 + pad), (int64_t)pad, s_pad, &o.key_bias);
+        if (pad) q = rows[0];
+        k = rows[pad];
+        v = rows[1 + pad];
+    }
+    Tensor t = Probabilities::apply(q, k, conv_w, w_pre, &o, &mark);
+    mark("conv_post");
+    t = Conv2d::apply(t, post_conv_w, causal, !causal, !causal);
+    // (the hidden stretch receives a gradient of 0: the one with respect to the last scores is formed inside the band)
+    if (o.first) band_zero_(t, *o.first);
+    mark("mix_post");
+    const bool lower = lower_values(t, v, o);
+    t = HeadMix::apply(t, w_post, post_causal, post_fill, post_group, !lower, !causal);
+    if (dropout > 0) t = at::dropout(t, dropout, true);
+    mark("pv");
+    t = Values::apply(t, v, lower, s_real, &o.first);
+    mark("end");
+    return t;
+}
+
+// ---- the two operators ---------------------------------------------------------------------------------------------
 bool wants_grad(const Tensor &a, const Tensor &b) { return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad()); }
 
 Tensor conv2d_apply(const Tensor &x, const Tensor &w, bool causal, bool fill_upper, bool grad_fill_upper)

@@ -197,3 +197,140 @@ def test_masks_left_on_the_host(pkg, train):
         with pytest.raises(RuntimeError):
             mod(x, x, x, mask, None)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,scores", [(torch.bfloat16, 5), (torch.float32, 6)])
+def test_training_peak_memory(pkg, dtype, scores):
+    """A training step holds the score tensors that backward needs (conv result, probabilities, post-softmax conv and mixing; the raw
+    scores too where the first stage is two operators) and drops each where it is consumed: at the peak those and one gradient.
+    Everything else is (B,H,S,D) or smaller: half a score tensor covers it (D = 64 against S = 2048, about ten tensors)."""
+    print(f"training peak memory {dtype}", flush=True)
+    b, h, s, d = 1, 4, 2048, 64
+    mod = _module(pkg, h, dtype)
+    q, k, v = (torch.randn(b, h, s, d, device="cuda", dtype=dtype).requires_grad_(True) for _ in range(3))
+    go = torch.randn(b, s, h, d, device="cuda", dtype=dtype)
+
+    def step():
+        for t in (q, k, v, *mod.parameters()):
+            t.grad = None
+        mod(q, k, v, None, None).backward(go)
+
+    step()
+    for t in (q, k, v, *mod.parameters()):
+        t.grad = None
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    step()
+    one = b * h * s * s * q.element_size()
+    peak = (torch.cuda.max_memory_allocated() - before) / one
+    print(f"peak: {peak:.2f} score tensors", flush=True)
+    assert peak <= scores + 0.5, peak
+
+
+def test_backward_twice(pkg):
+    """A graph that is kept gives the same gradients again; one that is not is refused the second time."""
+    print("backward twice", flush=True)
+    for s, use_mask in ((64, False), (45, True)):
+        mod = _module(pkg, 4, torch.bfloat16, use_mask=use_mask)
+        q, k, v = (torch.randn(2, 4, s, 64, device="cuda", dtype=torch.bfloat16).requires_grad_(True) for _ in range(3))
+        mask = None
+        if use_mask:
+            rows = torch.arange(s, device="cuda")
+            mask = ((rows[None, :] <= rows[:, None]) & (rows < s - 7))[None, None]
+        out = mod(q, k, v, mask, None)
+        leaves = (q, k, v, *mod.parameters())
+        first = torch.autograd.grad(out, leaves, torch.ones_like(out), retain_graph=True)
+        again = torch.autograd.grad(out, leaves, torch.ones_like(out))
+        assert all(torch.equal(a, w) for a, w in zip(first, again))
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(out, leaves, torch.ones_like(out))
+
+
+def test_gradients_of_some_inputs(pkg):
+    """Each input alone wanting a gradient, and through saved-tensor hooks: as all together."""
+    print("gradients of some inputs", flush=True)
+    mod = _module(pkg, 4, torch.float16).requires_grad_(False)
+    base = [torch.randn(2, 4, 61, 64, device="cuda", dtype=torch.float16) for _ in range(3)]
+    params = list(mod.parameters())
+
+    def grads(wanted):
+        x = [t.clone().requires_grad_("qkv"[i] in wanted) for i, t in enumerate(base)]
+        for i, p in enumerate(params):
+            p.requires_grad_(str(i) in wanted)
+            p.grad = None
+        mod(*x, None, None).float().square().sum().backward()
+        return {n: t.grad for n, t in zip("qkv0123", [*x, *params])}
+
+    every = grads("qkv0123")
+    for one in "qkv0123":
+        got = grads(one)
+        assert all((t is None) == (n != one) for n, t in got.items())
+        assert torch.equal(got[one], every[one]), one
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.clone())[1], lambda t: t):
+        got = grads("qkv0123")
+    assert all(torch.equal(got[n], t) for n, t in every.items())
+    assert sum(len(sh) == 4 and sh[2] == sh[3] for sh in packed) >= 4     # the score tensors went through the hooks
+
+
+@pytest.mark.parametrize("kind", ["none", "keys", "window", "left"])
+@pytest.mark.parametrize("dtype,s", [(torch.bfloat16, 205), (torch.float32, 208)])
+def test_training_by_one_node_or_several(pkg, dtype, s, kind):
+    """A step whose score tensors are small is one autograd node, a larger one a node per score tensor: a batch on one side of the
+    line against its halves on the other.  The products choose their tiling by the size of the grid: sums in another order."""
+    print(f"one node or several {dtype} s={s} {kind}", flush=True)
+    h, d = 4, 64
+    s8 = (s + 7) // 8 * 8
+    one = h * s8 * s8 * (2 if dtype == torch.bfloat16 else 4)
+    b = ((16 << 20) // one + 2) // 2 * 2
+    assert b * one > (16 << 20) and b // 2 * one <= (16 << 20)
+    mod = _module(pkg, h, dtype, use_mask=kind != "none")
+    x = [torch.randn(b, h, s, d, device="cuda", dtype=dtype) for _ in range(3)]
+    go = torch.randn(b, s, h, d, device="cuda", dtype=dtype)
+    rows = torch.arange(s, device="cuda")
+    mask = (rows[None, :] <= rows[:, None])[None, None].expand(b, 1, s, s).clone()
+    if kind == "keys":
+        mask[1::2, ..., s - 20:] = False
+    elif kind == "window":
+        mask &= rows[None, :] > rows[:, None] - 50
+    elif kind == "left":
+        mask[1::2, ..., :30] = False
+        go[1::2, :30] = 0
+
+    def step(at):
+        leaves = [t[at].clone().requires_grad_(True) for t in x]
+        for p in mod.parameters():
+            p.grad = None
+        out = mod(*leaves, None if kind == "none" else mask[at], None)
+        out.backward(go[at])
+        return [out.detach(), *(t.grad for t in leaves)], [p.grad.float() for p in mod.parameters()]
+
+    whole, whole_w = step(slice(None))
+    first, first_w = step(slice(0, b // 2))
+    second, second_w = step(slice(b // 2, None))
+    rel = {torch.float32: 1e-5, torch.bfloat16: 5e-3}[dtype]
+    for name, a, f, t in zip("out q k v".split(), whole, first, second):
+        _near(a, torch.cat([f, t]).cpu(), rel, name)
+    for name, a, f, t in zip(_WEIGHTS, whole_w, first_w, second_w):
+        _near(a, (f + t).cpu(), rel * 2, name)
+
+
+@pytest.mark.parametrize("b", [2, 52])
+def test_training_dropout(pkg, b):
+    """Dropout on the last score tensor, one node (b = 2) and several: the output is linear in V, so out . go = dV . V for the mask
+    that was drawn, and the same seed draws it again."""
+    print(f"training dropout b={b}", flush=True)
+    mod = _module(pkg, 4, torch.float32)
+    mod.dropout = 0.25
+    x = [torch.randn(b, 4, 205, 64, device="cuda").requires_grad_(True) for _ in range(3)]
+    go = torch.randn(b, 205, 4, 64, device="cuda")
+    grads = []
+    for _ in range(2):
+        torch.manual_seed(5)
+        out = mod(*x, None, None)
+        grads.append(torch.autograd.grad(out, [*x, *mod.parameters()], go))
+        a, w = (out.detach().double() * go.double()).sum(), (grads[-1][2].double() * x[2].detach().double()).sum()
+        assert abs(float(a - w)) <= 1e-5 * float((out.detach().double() * go.double()).norm()) * out.numel() ** 0.5
+    assert all(torch.isfinite(t).all() for t in grads[0])
+    assert all(torch.equal(a, w) for a, w in zip(*grads))
