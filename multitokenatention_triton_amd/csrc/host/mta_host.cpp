@@ -87,10 +87,19 @@ Tensor empty_row_ends(const Tensor &empty_rows)
     return at::where(empty_rows, rows.unsqueeze(0), at::zeros({}, rows.options())).contiguous();
 }
 
+// forward-mode differentiation: the kernels know no tangents
+bool has_tangent(const Tensor &t) { return t.defined() && t._fw_grad(0).defined(); }
+
+void no_tangents(std::initializer_list<const Tensor *> ts, const char *what)
+{
+    for (const Tensor *t : ts) TORCH_CHECK_NOT_IMPLEMENTED(!has_tangent(*t), what, " does not implement forward-mode differentiation");
+}
+
 // Q, K and V of one batch, head count, length and dtype, which is what the row copies around the kernels take (of fewer than
-// 2^31 elements).  Anything else the library products broadcast.
+// 2^31 elements).  Anything else the library products broadcast, and a V with a tangent they differentiate.
 bool alike(const Tensor &q, const Tensor &k, const Tensor &v)
 {
+    if (has_tangent(v)) return false;
     if (q.dim() != 4 || k.sizes() != q.sizes() || v.dim() != 4 || v.size(0) != q.size(0) || v.size(1) != q.size(1) || v.size(2) != q.size(2))
         return false;
     return k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type() && std::max(q.numel(), v.numel()) < (int64_t(1) << 31);
@@ -214,7 +223,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const auto dtype = q.scalar_type();
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
-    const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && dtype == v.scalar_type() &&
+    const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && !has_tangent(v) && dtype == v.scalar_type() &&
                         lower_products_supported(dtype, v.sizes(), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
@@ -701,6 +710,7 @@ Tensor forward_training(const Tensor &q_, const Tensor &k_, const Tensor &v_, co
                         double dropout, const py::object &hook)
 {
     const c10::OptionalDeviceGuard guard(q_.is_cuda() ? std::optional<c10::Device>(q_.device()) : std::nullopt);
+    no_tangents({&q_, &k_, &v_, &conv_w, &w_pre, &post_conv_w, &w_post}, "MTAAttentionTriton");
     const at::DimVector planes_of = score_sizes(q_, k_, v_);
     const int64_t heads = planes_of[1], s_real = q_.size(-2), s_pad = padded_length(q_, k_, v_, causal), columns = s_pad == s_real ? k_.size(2) : s_pad;
     check_weight(conv_w, 3, heads, q_, "the conv weight");
@@ -748,6 +758,7 @@ bool wants_grad(const Tensor &a, const Tensor &b) { return at::GradMode::is_enab
 Tensor conv2d_apply(const Tensor &x, const Tensor &w, bool causal, bool fill_upper, bool grad_fill_upper)
 {
     const c10::OptionalDeviceGuard guard(x.is_cuda() ? std::optional<c10::Device>(x.device()) : std::nullopt);
+    no_tangents({&x, &w}, "Conv2dTriton");
     if (!wants_grad(x, w)) return conv2d(x, w, causal, std::nullopt, fill_upper);
     return Conv2d::apply(x, w, causal, fill_upper, grad_fill_upper);
 }
@@ -755,6 +766,7 @@ Tensor conv2d_apply(const Tensor &x, const Tensor &w, bool causal, bool fill_upp
 Tensor headmix_apply(const Tensor &x, const Tensor &w, bool causal, double fill, int64_t group, bool fill_upper, bool grad_fill_upper)
 {
     const c10::OptionalDeviceGuard guard(x.is_cuda() ? std::optional<c10::Device>(x.device()) : std::nullopt);
+    no_tangents({&x, &w}, "TritonLinearHead");
     if (!wants_grad(x, w)) return headmix(x, w, causal, fill_upper || !causal ? fill : 0.0, group, fill_upper);
     return HeadMix::apply(x, w, causal, fill, group, fill_upper, grad_fill_upper);
 }
@@ -762,6 +774,7 @@ Tensor headmix_apply(const Tensor &x, const Tensor &w, bool causal, double fill,
 // O = softmax(mask(conv(mask0(Q K^T))) * scale) V, without the row statistic a backward pass would keep
 Tensor conv_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &w_, bool causal, std::optional<double> softmax_scale)
 {
+    no_tangents({&q_, &k_, &v_, &w_}, "TritonConvAttention");
     const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), v = on_gpu(v_, "V"), w = on_gpu(w_, "W");
     TORCH_CHECK_VALUE(q.dim() == 4 && q.sizes() == k.sizes() && q.sizes() == v.sizes(), "Q, K, V must share a (B,H,S,D) shape, got ", q.sizes(),
                       ", ", k.sizes(), ", ", v.sizes());

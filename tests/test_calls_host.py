@@ -92,3 +92,29 @@ def test_mask_rows_that_do_not_fit(train):
     with pytest.raises(RuntimeError, match="live on"):
         mod(x, x, x.to("meta"), None, None)
     assert seen == []
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_forward_mode_is_refused(train):
+    """The kernels know no tangents: a dual tensor is refused whether or not something else wants a gradient."""
+    import torch.autograd.forward_ad as fw
+    x, s = torch.zeros(2, 4, 16, 64), torch.zeros(2, 4, 16, 16)
+    conv = mta.Conv2dTriton(4, 3, causal=True).requires_grad_(train)
+    mix = mta.TritonLinearHead(4).requires_grad_(train)
+    attn = mta.TritonConvAttention(4, 3, causal=True).requires_grad_(train)
+    mod, seen = _module(train=True)
+    with fw.dual_level(), torch.set_grad_enabled(train):
+        ds, dx = fw.make_dual(s, torch.ones_like(s)), fw.make_dual(x, torch.ones_like(x))
+        for call in (lambda: conv(ds), lambda: mix(ds)):
+            with pytest.raises(NotImplementedError):
+                call()
+        if not train:
+            for operands in ((dx, x, x), (x, dx, x), (x, x, dx)):
+                with pytest.raises(NotImplementedError):
+                    attn(*operands, True, None)
+    with fw.dual_level():
+        dx = fw.make_dual(x, torch.ones_like(x))
+        for operands in ((dx, x, x), (x, dx, x), (x, x, dx)):
+            with pytest.raises(NotImplementedError):
+                mod(*operands, None, None)
+    assert seen == []

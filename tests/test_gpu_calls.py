@@ -334,3 +334,21 @@ def test_training_dropout(pkg, b):
         assert abs(float(a - w)) <= 1e-5 * float((out.detach().double() * go.double()).norm()) * out.numel() ** 0.5
     assert all(torch.isfinite(t).all() for t in grads[0])
     assert all(torch.equal(a, w) for a, w in zip(*grads))
+
+
+@pytest.mark.parametrize("s", [64, 45])
+def test_tangent_of_the_values(pkg, s):
+    """Inference with a dual V: the output is linear in V, and its tangent is the output for V's tangent (a whole and an odd length,
+    without a mask and under key padding)."""
+    import torch.autograd.forward_ad as fw
+    for use_mask in (False, True):
+        print(f"tangent of the values s={s} mask={use_mask}", flush=True)
+        mod = _module(pkg, 4, torch.float32, use_mask=use_mask).requires_grad_(False)
+        q, k, v, t = (torch.randn(2, 4, s, 64, device="cuda") for _ in range(4))
+        rows = torch.arange(s, device="cuda")
+        mask = ((rows[None, :] <= rows[:, None]) & (rows < s - 7))[None, None] if use_mask else None
+        want, tangent = mod(q, k, v, mask, None), mod(q, k, t, mask, None)
+        with fw.dual_level():
+            got = fw.unpack_dual(mod(q, k, fw.make_dual(v, t), mask, None))
+            _near(got.primal, want.cpu(), 1e-5)
+            _near(got.tangent, tangent.cpu(), 1e-5)
