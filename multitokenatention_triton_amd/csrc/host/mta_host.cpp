@@ -7,6 +7,7 @@
 #include <torch/extension.h>
 
 #include <ATen/ExpandUtils.h>
+#include <ATen/autocast_mode.h>
 
 #include "ops.hpp"
 
@@ -87,6 +88,20 @@ Tensor empty_row_ends(const Tensor &empty_rows)
     return at::where(empty_rows, rows.unsqueeze(0), at::zeros({}, rows.options())).contiguous();
 }
 
+// The dtype that a library product gives data of dtype t: under autocast its own.  The kernels that stand in for library products
+// (fp32 products, padded lengths, raw scores as a stage of their own) are taken where that is the data's dtype; the ones that are
+// a stage by themselves, with weights of the data's dtype, have never been subject to autocast.
+at::ScalarType product_type(at::ScalarType t)
+{
+    return at::autocast::is_autocast_enabled(at::kCUDA) ? at::autocast::get_autocast_dtype(at::kCUDA) : t;
+}
+
+// a b by the library; outside autocast (a backward that runs there) in a's dtype, as it would be inside
+Tensor matmul_as(const Tensor &a, const Tensor &b)
+{
+    return at::matmul(a, b.to(a.scalar_type()));
+}
+
 // forward-mode differentiation: the kernels know no tangents
 bool has_tangent(const Tensor &t) { return t.defined() && t._fw_grad(0).defined(); }
 
@@ -136,7 +151,7 @@ void check_weight(const Tensor &w, int64_t dim, int64_t heads, const Tensor &q, 
 int64_t padded_length(const Tensor &q, const Tensor &k, const Tensor &v, bool causal)
 {
     const int64_t s = q.size(-2);
-    return causal && alike(q, k, v) ? (s + 7) / 8 * 8 : s;
+    return causal && alike(q, k, v) && product_type(q.scalar_type()) == q.scalar_type() ? (s + 7) / 8 * 8 : s;
 }
 
 // key_bias (fp32), first (int32) and empty_rows (bool): one value per batch entry of the scores and key (row).  Under the causal
@@ -220,11 +235,12 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const int64_t g_pre = pre_identity ? 1 : pre_group ? pre_group : heads, g_post = post_identity ? 1 : post_group ? post_group : heads;
     const int64_t g_both = lcm(g_pre, g_post);
     const bool masked = key_bias || first;
-    const auto dtype = q.scalar_type();
+    const bool qk_kernel = qk_conv_supported(q, k, conv_w), as_is = product_type(q.scalar_type()) == q.scalar_type();
+    const auto dtype = qk_kernel ? q.scalar_type() : product_type(q.scalar_type());   // (of the scores)
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
     const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && !has_tangent(v) && dtype == v.scalar_type() &&
-                        lower_products_supported(dtype, v.sizes(), causal);
+                        (as_is || dtype != at::kFloat) && lower_products_supported(dtype, v.sizes(), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
     // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
@@ -252,12 +268,12 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     if (tri_first) {
         mark("qk_conv");
         scores = qk_conv_tri(q, k, conv_w, scale, 16, first);
-    } else if (qk_conv_supported(q, k, conv_w)) {
+    } else if (qk_kernel) {
         mark("qk_conv");
         scores = qk_conv(q, k, conv_w, causal, scale, false, first);
     } else {
         mark("qk");
-        const OptTensor raw = causal ? lower_scores(q, k, first) : OptTensor();
+        const OptTensor raw = causal && as_is ? lower_scores(q, k, first) : OptTensor();
         TORCH_CHECK(raw || !first, "the band mask needs the lower-triangle products");
         scores = raw ? *raw : at::matmul(q, k.transpose(2, 3));
         mark("conv_pre");   // (the stage that follows never reads above the diagonal)
@@ -370,7 +386,8 @@ Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, con
         if (o.first) band_zero_(x, *o.first);
     } else {
         mark("qk");
-        const OptTensor lower_raw = o.causal ? lower_scores(q, k, o.first) : OptTensor();
+        const bool as_is = product_type(q.scalar_type()) == q.scalar_type();
+        const OptTensor lower_raw = o.causal && as_is ? lower_scores(q, k, o.first) : OptTensor();
         TORCH_CHECK(lower_raw || !o.first, "the band mask needs the lower-triangle products");
         raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
         mark("conv_pre");
@@ -411,15 +428,15 @@ void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, c
     const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, !causal);
     ds.reset();
     if (need[0] || need[1]) {
-        const bool lower = causal && q.sizes() == k.sizes() && lower_products_supported(q.scalar_type(), q.sizes(), true);
+        const bool lower = causal && q.sizes() == k.sizes() && dx.scalar_type() == q.scalar_type() && lower_products_supported(q.scalar_type(), q.sizes(), true);
         const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
         if (first) band_zero_(g, *first);
         Tensor dq, dk;
         OptTensor own_q, own_k;
         if (need[0]) own_q = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
-        if (need[0]) dq = own_q ? *own_q : at::matmul(g, k);
+        if (need[0]) dq = own_q ? *own_q : matmul_as(g, k);
         if (need[1]) own_k = lower ? causal_ptx(g, q, true, scale) : OptTensor();
-        if (need[1]) dk = own_k ? *own_k : at::matmul(g.transpose(2, 3), q);
+        if (need[1]) dk = own_k ? *own_k : matmul_as(g.transpose(2, 3), q);
         // the factor, where the products were the library's
         if (need[0] && need[1] && !own_q && !own_k && dq.sizes() == dk.sizes()) {
             RowsCopy rows(dq.size(2), OptTensor());
@@ -473,7 +490,7 @@ Tensor value_rows(const Tensor &grad, int64_t s_pad)
 Tensor values_bwd_v(const Tensor &m, const Tensor &go, bool lower)
 {
     const OptTensor own = lower ? causal_ptx(m, go, true, 1.0) : OptTensor();
-    return own ? *own : at::matmul(m.transpose(2, 3), go);
+    return own ? *own : matmul_as(m.transpose(2, 3), go);
 }
 
 // (first: the gradient is formed inside the band)
@@ -481,7 +498,7 @@ Tensor values_bwd_m(const Tensor &go, const Tensor &v, bool lower, const OptTens
 {
     const OptTensor own = lower ? lower_scores(go, v, first) : OptTensor();
     TORCH_CHECK(own || !first);
-    return own ? *own : at::matmul(go, v.transpose(2, 3));
+    return own ? *own : matmul_as(go, v.transpose(2, 3));
 }
 
 // The pieces as one node: the host's time is what bounds a step of small tensors (a node costs about 8.6 us of it, forward and

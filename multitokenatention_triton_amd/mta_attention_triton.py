@@ -77,11 +77,21 @@ from . import _lib, ops
 from .convolution_2d_trit import Conv2dTriton, Conv2dTritonFunction
 from .triton_linear_head import TritonLinearHead, TritonLinearHeadFunction
 
+def _autocasts(x: torch.Tensor) -> bool:
+    """Whether a library product of ``x`` would come out in another dtype."""
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype
+
+
+def _matmul_as(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """a b by the library in backward: in a's dtype, as it is inside autocast, where backward runs outside of it."""
+    return torch.matmul(a, b.to(a.dtype))
+
+
 def _lower_scores(a: torch.Tensor, b: torch.Tensor, first_visible: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """round(a b^T) on and below the diagonal of a (B,H,S,S) tensor, nothing written above it, for consumers that
     never read there (``mta_lower_scores_fwd``): half the output traffic of the library GEMM.  None where that kernel does
     not apply (ragged lengths, other head sizes): the caller then takes the GEMM."""
-    if a.shape != b.shape or a.dtype != b.dtype:
+    if a.shape != b.shape or a.dtype != b.dtype or (a.dtype == torch.float32 and _autocasts(a)):
         return None
     out = ops.lower_scores(a, b, first_visible)
     if out is not None and first_visible is not None:
@@ -112,11 +122,11 @@ class _ProbsTimesValues(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dp = _lower_scores(grad_output, v) if ctx.lower else None
             if dp is None:
-                dp = torch.matmul(grad_output, v.transpose(2, 3))
+                dp = _matmul_as(grad_output, v.transpose(2, 3))
         if ctx.needs_input_grad[1]:
             dv = ops.causal_ptx(p, grad_output.contiguous(), True) if ctx.lower else None
             if dv is None:
-                dv = torch.matmul(p.transpose(2, 3), grad_output)
+                dv = _matmul_as(p.transpose(2, 3), grad_output)
         return dp, dv, None
 
 
@@ -159,13 +169,13 @@ class _ScaledScoresConv(torch.autograd.Function):
         xq, xk, weight, raw = ctx.saved_tensors
         dq = dk = dw = None
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            lower = ctx.causal and xq.shape == xk.shape and _lower_products_supported(xq, xk.size(-2))
+            lower = ctx.causal and xq.shape == xk.shape and grad_output.dtype == xq.dtype and _lower_products_supported(xq, xk.size(-2))
             g = ops.conv2d_bwd_input(grad_output, weight, ctx.causal, fill_upper=not lower)
             ops.mask_fill(g, ctx.mask_planes, False, lower, out=g)
             if ctx.needs_input_grad[0]:
-                dq = (ops.causal_pv(g, xk, True) if lower else torch.matmul(g, xk)) * ctx.scale
+                dq = (ops.causal_pv(g, xk, True) if lower else _matmul_as(g, xk)) * ctx.scale
             if ctx.needs_input_grad[1]:
-                dk = (ops.causal_ptx(g, xq, True) if lower else torch.matmul(g.transpose(2, 3), xq)) * ctx.scale
+                dk = (ops.causal_ptx(g, xq, True) if lower else _matmul_as(g.transpose(2, 3), xq)) * ctx.scale
         if ctx.needs_input_grad[2]:
             dw = ops.conv2d_bwd_weight(raw, grad_output.to(raw.dtype), tuple(weight.shape[1:]), ctx.causal)
             dw = (dw * ctx.scale).to(weight.dtype)
@@ -474,7 +484,7 @@ class MTAAttentionTriton(nn.Module):
                     return self._forward_native(xq, xk, xv, key_bias=what)
                 if (kind == "band" and self._band_supported(xq, xk)
                         # (a padded length takes V of the batch and heads of the scores: no library product to broadcast it)
-                        and (xk.size(-2) % 8 == 0 or (xv.shape[:3] == xk.shape[:3] and xv.dtype == xk.dtype))
+                        and (xk.size(-2) % 8 == 0 or (xv.shape[:3] == xk.shape[:3] and xv.dtype == xk.dtype and not _autocasts(xq)))
                         # (rows that see nothing: with 3x5 and 7x9 kernels, which came to the band route last, such masks
                         # stay on the mask passes, whose stages an observer may count on)
                         and (self._band_empty_rows(mask) is None or self.mta_conv_triton.kernel_size not in ((3, 5), (7, 9)))
@@ -578,7 +588,7 @@ class MTAAttentionTriton(nn.Module):
         return (xq.shape == xk.shape and xq.dtype == xk.dtype
                 and ((xq.dtype == w.dtype and xq.dtype in (torch.bfloat16, torch.float16)
                       and bool(_lib.load().mta_qk_conv_supported(8, xq.size(-1), w.size(1), w.size(2), _lib.MTA_BF16, _lib.MTA_BF16)))
-                     or _lower_kernels(xq)))
+                     or (_lower_kernels(xq) and not _autocasts(xq))))
 
     def _band_training_supported(self, xq, xk, xv) -> bool:
         """Whether the differentiable route takes a band mask: data of one dtype and the lower-triangle products (P V and

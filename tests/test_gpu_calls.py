@@ -352,3 +352,51 @@ def test_tangent_of_the_values(pkg, s):
             got = fw.unpack_dual(mod(q, k, fw.make_dual(v, t), mask, None))
             _near(got.primal, want.cpu(), 1e-5)
             _near(got.tangent, tangent.cpu(), 1e-5)
+
+
+@pytest.mark.parametrize("mask", [None, "keys", "window", "holes"])
+@pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                          (torch.float16, torch.float16), (torch.float16, torch.float32)])
+def test_autocast(pkg, dtype, wdtype, mask):
+    """Under torch.autocast the products of Q K^T and P V that the library would do come out in autocast's dtype, whichever kernel
+    does them, and so does the output; the scores kernel with weights of its own dtype is no library product.  Backward runs
+    inside and outside, the gradients have the inputs' dtypes."""
+    amp = torch.float16
+    for s in (64, 45):
+        print(f"autocast {dtype} {wdtype} {mask} s={s}", flush=True)
+        if mask == "holes" and s % 8:
+            continue
+        # (16-bit data of another dtype than autocast's: only where the scores kernel takes it, the general kernels take one dtype)
+        own = dtype == wdtype and dtype != torch.float32 and s % 8 == 0 and mask != "holes"
+        if mask is not None and not own and dtype == torch.bfloat16:
+            continue
+        mod = _module(pkg, 4, dtype, wdtype, use_mask=mask is not None)
+        g = torch.Generator().manual_seed(9)
+        q, k, v = (torch.randn(2, 4, s, 64, generator=g).to(dtype) for _ in range(3))
+        rows = torch.arange(s)
+        visible = (rows[None, :] <= rows[:, None])[None, None]
+        if mask == "keys":
+            visible = visible & (rows < s - 7)
+        elif mask == "window":
+            visible = visible & (rows[None, :] > rows[:, None] - 17)
+        elif mask == "holes":
+            visible = visible & ((rows[None, :] + rows[:, None]) % 5 != 1)
+        want, leaves = _oracle(mod, q, k, v, mask=torch.where(visible, 0.0, float("-inf")).expand(2, 4, s, s))
+        want.sum().backward()
+        given = None if mask is None else visible.cuda()
+        dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+        expect = dtype if own else amp
+        rel = _REL[torch.bfloat16 if torch.bfloat16 in (dtype, expect) else torch.float16]
+        with torch.autocast("cuda", dtype=amp), torch.no_grad():
+            plain = mod(*dev, given, None)
+        with torch.autocast("cuda", dtype=amp):     # (a context of its own: autocast keeps the casts it has made without a graph)
+            out = mod(*dev, given, None)
+            inside = torch.autograd.grad(out.float().sum(), dev, retain_graph=True)
+        assert plain.dtype == out.dtype == expect
+        _near(plain, want, rel, "inference")
+        _near(out, want, rel, "training")
+        outside = torch.autograd.grad(out.float().sum(), dev)
+        for grads in (inside, outside):
+            for name, a, w in zip("qkv", grads, leaves):
+                assert a.dtype == dtype
+                _near(a, w.grad, 4 * rel, name)
