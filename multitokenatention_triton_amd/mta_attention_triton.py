@@ -485,9 +485,6 @@ class MTAAttentionTriton(nn.Module):
                 if (kind == "band" and self._band_supported(xq, xk)
                         # (a padded length takes V of the batch and heads of the scores: no library product to broadcast it)
                         and (xk.size(-2) % 8 == 0 or (xv.shape[:3] == xk.shape[:3] and xv.dtype == xk.dtype and not _autocasts(xq)))
-                        # (rows that see nothing: with 3x5 and 7x9 kernels, which came to the band route last, such masks
-                        # stay on the mask passes, whose stages an observer may count on)
-                        and (self._band_empty_rows(mask) is None or self.mta_conv_triton.kernel_size not in ((3, 5), (7, 9)))
                         and (not _wants_grad(xq, xk, xv, self._weights()) or self._band_training_supported(xq, xk, xv))):
                     return self._forward_native(xq, xk, xv, first_visible=what, empty_rows=self._band_empty_rows(mask))
         elif (not self.causal and isinstance(mask, torch.Tensor) and mask.dim() == 4 and xq.size(-2) == xk.size(-2)):

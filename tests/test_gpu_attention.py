@@ -1154,6 +1154,7 @@ def test_mta_use_mask_rows_that_see_nothing(pkg, dtype, post):
     pad = torch.tensor([0, 37])
     keep = torch.arange(s)[None, :] >= pad[:, None]                                   # (B,S): left padding
     visible = (keep[:, None, :, None] & keep[:, None, None, :] & torch.tril(torch.ones(s, s, dtype=torch.bool))[None, None])
+    visible[:, :, 100, 60] = False      # a hole: without it this is a band mask, and no mask pass runs
     want = O.mta_forward(q, k, v, params[0].unsqueeze(1), params[1], params[2].unsqueeze(1), params[3],
                          mask=torch.where(visible, 0.0, float("-inf")).expand(b, h, s, s).contiguous())
     assert torch.isfinite(want.float()).all() and not want[1, :37].any()

@@ -400,3 +400,37 @@ def test_autocast(pkg, dtype, wdtype, mask):
             for name, a, w in zip("qkv", grads, leaves):
                 assert a.dtype == dtype
                 _near(a, w.grad, 4 * rel, name)
+
+
+@pytest.mark.parametrize("dtype,ks", [(torch.bfloat16, (3, 5)), (torch.float16, (7, 9)), (torch.float32, (3, 5)), (torch.bfloat16, (11, 15))])
+def test_left_padded_batches_of_every_kernel_size(pkg, dtype, ks):
+    """A band mask whose padding rows see nothing takes the band route whatever the conv kernel: output against the oracle, gradients
+    against the mask passes on the same mask (the reference's are NaN there)."""
+    print(f"left padding {dtype} {ks}", flush=True)
+    b, h, s, d = 2, 4, 136, 64
+    mod = _module(pkg, h, dtype, use_mask=True, query_kernel_size=ks[0], key_kernel_size=ks[1])
+    g = torch.Generator().manual_seed(10)
+    q, k, v = (torch.randn(b, h, s, d, generator=g).to(dtype) for _ in range(3))
+    keep = torch.arange(s)[None, :] >= torch.tensor([0, 37])[:, None]
+    visible = keep[:, None, None, :] & torch.tril(torch.ones(s, s, dtype=torch.bool))[None, None]
+    want, _ = _oracle(mod, q, k, v, mask=torch.where(visible, 0.0, float("-inf")).expand(b, h, s, s))
+    dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    go = torch.randn(b, s, h, d, generator=g).to(dtype).cuda()
+    go[1, :37] = 0
+    seen, grads = [], []
+    mod._stage_hook = seen.append
+    with torch.no_grad():
+        plain = mod(*dev, visible.cuda(), None)
+    assert "mask" not in seen
+    _near(plain, want, _REL[dtype], "inference")
+    assert not plain[1, :37].any()
+    for passes in (False, True):
+        if passes:
+            mod._band_training_supported = lambda *a: False
+        seen.clear()
+        out = mod(*dev, visible.cuda(), None)
+        assert ("mask" in seen) == passes
+        _near(out, want, _REL[dtype], "training")
+        grads.append(torch.autograd.grad(out, [*dev, *mod.parameters()], go))
+    for a, w in zip(*grads):
+        _near(a, w.cpu(), 10 * _REL[dtype])

@@ -265,8 +265,6 @@ def test_mta_band_mask_two_kernel_first_stage(pkg, dtype, wdtype, h, s, d, kerne
     """Band masks where the scores and their conv are two kernels (fp32 data; weights of another dtype): no mask pass over the
     scores, output and all seven gradients against the oracle given the mask tensor (left: a batch entry whose first rows see
     nothing, forward only - the reference's gradients are NaN there)."""
-    if kind == "left" and kernel == (7, 9):
-        pytest.skip("rows that see nothing stay on the mask passes with 7x9 kernels")
     print(f"band mask two kernels {dtype} {wdtype} h={h} s={s} d={d} {kernel} {kind}", flush=True)
     b = 2
     mod, params = _mta(pkg, h, kernel, (3, 3), wdtype, 61, use_mask=True)
