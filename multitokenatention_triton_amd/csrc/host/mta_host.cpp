@@ -45,13 +45,15 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 bool stages_apart(int64_t group, at::ScalarType t) { return t == at::kFloat && group > FUSED_MAX_GROUP; }
 
 // Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
-// heads at about 20 us each, so that two full rounds of tiles are where it meets the two kernels one after the other (us, one
-// kernel | two, 3x3 / 7x7: B1 S512 25 | 12 / 28 | 14, B1 S1024 27 | 21 / 32 | 26, B2 S1008 39 | 41 / 46 | 49, B1 S1536 49 | 39 / 54 | 47,
-// B1 S2048 54 | 67 / 63 | 80, B4 S1024 51 | 70 / 60 | 83).
+// heads at about 20 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other.
+// us of the forward (H16 D64 fp16, the post-softmax conv 3x3 / 7x7), one kernel | two: 272 tiles (B1 S1024) 68.7 | 60.2 / 72.8 | 64.5,
+// 544 (B2 S1008) 101.0 | 88.3 / 106.4 | 95.6, 600 (B1 S1536) 109.9 | 91.9 / 115.9 | 98.3, 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3,
+// 840 (B2 S1280) 126.1 | 123.9 / 131.8 | 133.3, 1056 (B1 S2048) 155.0 | 164.5 / 161.5 | 175.5, 1088 (B4 S1024) 149.8 | 171.4 /
+// 156.9 | 182.6; the runs of one side differ by up to 2.
 bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only)
 {
     const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64;
-    return planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk) >= 2 * 512;
+    return planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk) >= 800;
 }
 
 int64_t lcm(int64_t a, int64_t b)
