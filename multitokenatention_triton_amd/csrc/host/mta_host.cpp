@@ -41,9 +41,6 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
     return !masked || group <= FUSED_MAX_GROUP || t == at::kFloat || (group == FUSED_MFMA_GROUP && !no_row_lists());
 }
 
-// fp32 groups of more than 8 heads: one kernel, announced to the observer as the stages it stands for
-bool stages_apart(int64_t group, at::ScalarType t) { return t == at::kFloat && group > FUSED_MAX_GROUP; }
-
 // Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
 // heads at about 20 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other.
 // us of the forward (H16 D64 fp16, the post-softmax conv 3x3 / 7x7), one kernel | two: 272 tiles (B1 S1024) 68.7 | 60.2 / 72.8 | 64.5,
@@ -66,7 +63,8 @@ int64_t lcm(int64_t a, int64_t b)
 // 1/sqrt(D) as the reference forms it: in fp32
 double score_scale(const Tensor &q) { return (double)(1.0f / std::sqrt((float)q.size(-1))); }
 
-// the optional observer of the modules: called with a stage's name right before it is enqueued
+// the optional observer of the modules: called with a stage's name right before the kernel (or library call) that does it is
+// enqueued; a kernel that does several operators is one stage with a name of its own
 struct Mark {
     const py::object &hook;
     void operator()(const char *stage) const
@@ -283,13 +281,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     }
 
     if (one_pass) {
-        if (stages_apart(g_both, dtype)) {
-            mark("mix_pre");
-            mark("softmax");
-            mark("mix_post");
-        } else {
-            mark("mix_softmax_mix");
-        }
+        mark("mix_softmax_mix");
         scores = headmix_softmax(scores, w1, w2, causal, g_both, !own_pv, key_bias, first);
     } else {
         const bool fill = post_conv_identity && !w2 && !own_pv;
@@ -297,12 +289,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
             mark("mix_softmax");
             scores = headmix_softmax_tri(scores, w1, OptTensor(), q.size(0), heads, n_keys, g_pre, first, true, key_bias);
         } else if (one_pass_group(g_pre, dtype, n_keys, w1, OptTensor()) && masks_ok(g_pre, dtype, masked)) {
-            if (stages_apart(g_pre, dtype)) {
-                mark("mix_pre");
-                mark("softmax");
-            } else {
-                mark("mix_softmax");
-            }
+            mark("mix_softmax");
             scores = headmix_softmax(scores, w1, OptTensor(), causal, g_pre, fill, key_bias, first);
         } else {
             mark("mix_pre");   // (the softmax kernel that follows never reads above the diagonal)
@@ -317,14 +304,12 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         const int64_t r = post_conv_w.size(1), s = post_conv_w.size(2);
         const bool mix16 = g_post == 16 && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
                            post_conv_w.scalar_type() == scores.scalar_type() && w_post.scalar_type() == scores.scalar_type() && n_keys % 8 == 0;
-        const bool small_groups = g_post <= 4 && ((r == 3 && s == 3) || (r == 7 && s == 7));
+        const bool small_groups = g_post <= 4 && g_post != 3 && ((r == 3 && s == 3) || (r == 7 && s == 7));
         OptTensor done;
-        if (!first && !post_conv_identity && w2 && (small_groups || mix16)) {
+        if (!first && !post_conv_identity && w2 &&
+            (small_groups || (mix16 && conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv)))) {
             mark("conv_mix_post");
-            if (!mix16 || conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv))
-                done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
-            else   // (the same stage as two kernels, the same results)
-                done = headmix(conv2d(scores, post_conv_w, causal, std::nullopt, false), w_post, causal, 0.0, g_post, !own_pv);
+            done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
         }
         if (done) {
             scores = *done;
@@ -398,14 +383,10 @@ Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, con
     const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
     const auto dtype = x.scalar_type();
     Tensor p;
-    if ((!stages_apart(g_eff, dtype) || o.pre_causal == o.causal) && one_pass_group(g_eff, dtype, n_keys, w_pre, OptTensor()) &&
+    // (fp32 groups of more than 8 heads: with the head weight's own causal rule apart from the module's the mixing stays alone)
+    if ((dtype != at::kFloat || g_eff <= FUSED_MAX_GROUP || o.pre_causal == o.causal) && one_pass_group(g_eff, dtype, n_keys, w_pre, OptTensor()) &&
         masks_ok(g_eff, dtype, o.key_bias || o.first)) {
-        if (stages_apart(g_eff, dtype)) {
-            mark("mix_pre");
-            mark("softmax");
-        } else {
-            mark("mix_softmax");
-        }
+        mark("mix_softmax");
         p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);
     } else {
         mark("mix_pre");

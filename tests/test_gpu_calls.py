@@ -434,3 +434,29 @@ def test_left_padded_batches_of_every_kernel_size(pkg, dtype, ks):
         grads.append(torch.autograd.grad(out, [*dev, *mod.parameters()], go))
     for a, w in zip(*grads):
         _near(a, w.cpu(), 10 * _REL[dtype])
+
+
+def test_observer_hears_the_kernels_that_run(pkg):
+    """One mark per kernel: the fp32 one-pass mixing and softmax of more than 8 heads is one stage, in inference and in training, and
+    conv + mixing of 16 heads is two where the grid makes it two kernels.  The figures of a stage are those of what it names."""
+    print("observer", flush=True)
+    for dtype, s, want in ((torch.float32, 64, ["qk", "conv_pre", "mix_softmax", "conv_post", "mix_post", "pv", "end"]),
+                           (torch.float16, 64, ["qk_conv", "mix_softmax", "conv_post", "mix_post", "pv", "end"]),
+                           (torch.float16, 2048, ["qk_conv", "mix_softmax", "conv_mix_post", "pv", "end"])):
+        mod = _module(pkg, 16, dtype)
+        x = [torch.randn(1, 16, s, 64, device="cuda", dtype=dtype) for _ in range(3)]
+        seen = []
+        mod._stage_hook = seen.append
+        with torch.no_grad():
+            mod(*x, None, None)
+        assert seen == want
+        if dtype == torch.float32:
+            seen.clear()
+            mod(*x, None, None)
+            assert seen == want
+            with torch.no_grad():
+                mod.mta_conv_after_sm_triton.weight.zero_()[:, -1, 1] = 1.0
+                mod.declare_weight_structure(post_conv_identity=True)
+                seen.clear()
+                mod(*x, None, None)
+            assert seen == ["qk", "conv_pre", "mix_softmax_mix", "pv", "end"]
