@@ -56,10 +56,16 @@ struct qk_chunks { int big, small; };
 // How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 16000 on the grid
 // runs in several rounds whatever the length and 48/24 keeps the rebuilt columns few; below, items as short as it takes to
 // have two or three per CU, down to one key block, win although each rebuilds one key block's worth of columns: the grid is
-// otherwise a fraction of the chip, each workgroup walking its keys alone.  Measured (us, with 48/24 -> with this rule):
-// B1 H8 S256 D64 3x3 (80 blocks) 13.3 -> 7.6; B1 H16 S512 D128 5x5 (448) 23.3 -> 11.5; B2 H16 S512 D64 6x11 (896) 22.6 -> 13.4;
-// B4 H16 S512 (1792) 26.3 -> 22.0; B1 H8 S2048 D64 (2450) 48.9 -> 23.9; B1 H16 S2048 D128 7x7 (4900) 60.4 -> 40.8.
-// (B1 H16 S4096 D128 7x7, 18900 blocks: 133 instead of 140 launched alone, but the forward it is part of 508.5 instead of 504.1.)
+// otherwise a fraction of the chip, each workgroup walking its keys alone.  us, 48/24 | as short as the rule makes them:
+// B1 H8 S256 D64 3x3 (80 blocks) 13.3 | 7.6; B1 H16 S512 D128 5x5 (448) 23.3 | 11.5; B2 H16 S512 D64 6x11 (896) 22.6 | 13.4;
+// B4 H16 S512 (1792) 26.3 | 22.0; B1 H8 S2048 D64 (2450) 48.9 | 23.9.
+// Where the line lies, the kernel alone (in brackets the forward with groups of 4 heads / with all weights dense; three processes
+// a side, which differ by up to 3 on the kernel and 2 on a forward), 48/24 | 16/8: B1 H16 S2048 D128 7x7 (5216) 62 | 51 (117 | 108 /
+// 184 | 171); B1 H32 S2048 D64 5x5 (10432) 58 | 56 (158 | 156 / 394 | 392); B2 H16 S2048 D128 6x11 (10432) 68 | 69 (165 | 166 /
+// 298 | 293); B1 H16 S3072 D128 3x3 (10688) 65 | 63 (199 | 190 / 309 | 297); B1 H16 S3712 D64 7x9 (15088) 82 | 81 (236 | 235 /
+// 386 | 383); B3 H16 S2048 D128 7x7 (15648) 99 | 103 (241 | 245 / 395 | 396); B1 H16 S4096 D128 7x7 (19104) 121 | 126 (300 | 299 /
+// 485 | 490); B4 H16 S2048 D64 3x3 (20864) 87 | 90 (242 | 246 / 462 | 471); B2 H16 S3072 D128 6x11 (21376) 133 | 136 (332 | 331 /
+// 536 | 545); B2 H16 S4096 D128 6x11 (38208) 225 | 236 (538 | 546 / 887 | 898).
 inline qk_chunks qk_chunk_rule(int64_t blocks, int64_t head_blocks, int nqb)
 {
     if (blocks >= 16000) return {48, 24};
