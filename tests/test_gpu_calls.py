@@ -460,3 +460,42 @@ def test_observer_hears_the_kernels_that_run(pkg):
                 seen.clear()
                 mod(*x, None, None)
             assert seen == ["qk", "conv_pre", "mix_softmax_mix", "pv", "end"]
+
+
+@pytest.mark.parametrize("dtype,d,dv", [(torch.float32, 64, 128), (torch.float32, 128, 32), (torch.float16, 64, 128), (torch.float16, 128, 32),
+                                        (torch.float32, 32, 64)])
+def test_values_of_another_head_size(pkg, dtype, d, dv):
+    """V of another head size than Q and K, one the P V kernels know or not: a whole and a padded length."""
+    for s in (64, 45):
+        print(f"values of another head size {dtype} {d} {dv} s={s}", flush=True)
+        mod = _module(pkg, 4, dtype)
+        g = torch.Generator().manual_seed(12)
+        q, k, v = (torch.randn(2, 4, s, n, generator=g).to(dtype) for n in (d, d, dv))
+        want, leaves = _oracle(mod, q, k, v)
+        dev = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+        with torch.inference_mode():
+            _near(mod(*dev, None, None), want, _REL[dtype], "inference")
+        out = mod(*dev, None, None)
+        _near(out, want, _REL[dtype], "training")
+        go = torch.randn(want.shape, generator=g)
+        want.backward(go.to(dtype).float())
+        out.backward(go.to(dtype).cuda())
+        for name, a, w in zip("qkv", dev, leaves):
+            _near(a.grad, w.grad, {torch.float32: 1e-4, torch.float16: 1e-2}[dtype], name)
+
+
+def test_calls_that_stay_refused(pkg):
+    """Empty tensors and functorch transforms: an exception, nothing launched."""
+    print("refused calls", flush=True)
+    for train in (False, True):
+        for dtype in (torch.float32, torch.float16):
+            mod = _module(pkg, 4, dtype).requires_grad_(train)
+            for shape in ((0, 4, 64, 64), (2, 4, 0, 64), (0, 4, 45, 64)):
+                x = torch.zeros(shape, device="cuda", dtype=dtype)
+                with pytest.raises(ValueError):
+                    mod(x, x, x, None, None)
+            x = torch.zeros(3, 2, 4, 64, 64, device="cuda", dtype=dtype)
+            for call in (lambda t: mod(t, t, t, None, None), lambda t: mod.mta_conv_triton(t), lambda t: mod.wpsm_triton(t)):
+                with pytest.raises(RuntimeError):
+                    torch.func.vmap(call)(x)
+    torch.cuda.synchronize()
