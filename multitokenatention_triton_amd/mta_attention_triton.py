@@ -28,19 +28,18 @@ Inference (no input or parameter requires grad, or grad mode is off):
     padding of an encoder batch); any other boolean or additive mask (holes, a plane per
     head, finite values) runs on the single-stage kernels with the reference's three
     elementwise mask steps as passes over a byte per position (``mta_mask_fill_fwd``;
-    ``mta_mask_add_fwd`` for finite values); only lengths that are not a multiple of 8 take
-    the reference's elementwise steps around the kernels.
+    ``mta_mask_add_fwd`` for finite values); only such masks over lengths that are not a
+    multiple of 8 take the reference's elementwise steps around the kernels.
 
-Training (something requires grad): the stages run one by one through autograd
-Functions, as in the reference, so that ``backward()`` works: the two conv and the two
-head-mixing stages with their HIP gradient kernels (convolution_2d_trit /
-triton_linear_head); the 1/sqrt(D) factor folded into the pre-softmax conv and, in
+Training (something requires grad): the stages run one by one, as in the reference, in one
+autograd node while the score tensors are small and in one per score tensor beyond, so that
+``backward()`` works and frees what it has used: the two conv and the two head-mixing stages
+with their HIP gradient kernels; the 1/sqrt(D) factor folded into the pre-softmax conv and, in
 backward, into the (B,H,S,D) gradients of Q and K; pre-softmax head mixing and softmax as
 one forward kernel where the inference route has one, with the softmax gradient taken from
-the stored 16-bit probabilities (``mta_softmax_bwd``; no fp32 copy of the score tensor in
+the stored probabilities (``mta_softmax_bwd``; no fp32 copy of the score tensor in
 either direction).  Under the causal rule the products around the score tensors (P V, the
-gradients it leaves, the recomputed raw scores) touch the lower triangle only; torch
-differentiates the dropout.  ``use_mask=True`` in training: the same two families of masks
+gradients it leaves, the recomputed raw scores) touch the lower triangle only.  ``use_mask=True`` in training: the same two families of masks
 go through these operators -- hidden keys as a key bias inside the softmax kernel and
 zeroed K and V rows, band masks inside the scores and softmax kernels, with the gradients
 around them formed inside the band; masks of arbitrary content as mask passes between the
