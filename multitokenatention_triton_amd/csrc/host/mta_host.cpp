@@ -8,6 +8,7 @@
 
 #include <ATen/ExpandUtils.h>
 #include <ATen/autocast_mode.h>
+#include <torch/csrc/autograd/anomaly_mode.h>
 
 #include "ops.hpp"
 
@@ -723,7 +724,8 @@ Tensor forward_training(const Tensor &q_, const Tensor &k_, const Tensor &v_, co
                          mask_row(empty_rows, at::kBool, "the empty rows", planes_of, causal, columns, q_)};
     const Mark mark{hook};
     const bool rows_alike = alike(q_, k_, v_);
-    if (rows_alike && planes_of[0] * heads * s_pad * s_pad * (int64_t)q_.element_size() <= WHOLE_STEP_BYTES)
+    // (anomaly mode looks for NaN in what goes from node to node, also above the diagonal, where nobody writes)
+    if (rows_alike && (planes_of[0] * heads * s_pad * s_pad * (int64_t)q_.element_size() <= WHOLE_STEP_BYTES || torch::autograd::AnomalyMode::is_enabled()))
         return WholeStep::apply(q_, k_, v_, conv_w, w_pre, post_conv_w, w_post, s_pad, dropout, &o, &mark);
     Tensor q = q_, k = k_, v = v_;
     if (o.key_bias && !rows_alike) {

@@ -499,3 +499,17 @@ def test_calls_that_stay_refused(pkg):
                 with pytest.raises(RuntimeError):
                     torch.func.vmap(call)(x)
     torch.cuda.synchronize()
+
+
+def test_anomaly_mode(pkg):
+    """torch.autograd.detect_anomaly over a step whose score tensors are large: what lies above the diagonal between the stages, memory
+    that nobody wrote (here: NaN), is not taken for a gradient."""
+    print("anomaly mode", flush=True)
+    mod = _module(pkg, 4, torch.bfloat16)
+    q, k, v = (torch.randn(1, 4, 2048, 64, device="cuda", dtype=torch.bfloat16).requires_grad_(True) for _ in range(3))
+    poison = [torch.full((1, 4, 2048, 2048), float("nan"), device="cuda", dtype=torch.bfloat16) for _ in range(12)]
+    del poison
+    with torch.autograd.detect_anomaly():
+        out = mod(q, k, v, None, None)
+        out.sum().backward()
+    assert all(torch.isfinite(t.grad).all() for t in (q, k, v, *mod.parameters()))
