@@ -370,6 +370,21 @@ int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *worksp
  * block diagonal by construction). */
 int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
                               int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream);
+
+/* mta_headmix_bwd_input and mta_headmix_bwd_weight_as in one pass over x and dy: dx and dw as those two define them (dw 0 outside
+ * the groups).  Mixing groups of 2, 4, 8, 12, 16 and 32 heads, Q of whole 16-byte vectors, x, dy and dx aligned to them, 16-bit
+ * data of groups of 12 and more with weights of the same dtype; MTA_ERR_UNSUPPORTED otherwise, and where
+ * mta_headmix_grads_workspace (device memory, as for the weight gradients) returns 0. */
+int64_t mta_headmix_grads_workspace(int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int with_softmax,
+                                    int io_dtype, int w_dtype);
+int mta_headmix_grads(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes,
+                      int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream);
+/* mta_softmax_bwd ahead of them in the same pass: dy = s * (ds - sum_k s ds), rounded to the I/O dtype, from the probabilities s
+ * and their gradient ds.  When causal nothing is written above the diagonal.  Workspace with with_softmax = 1; rows of up to
+ * 4096 keys (32 heads: 2048), fp32 half as many. */
+int mta_softmax_headmix_grads(const void *s, const void *ds, const void *x, const void *w, void *dx, void *dw, void *workspace,
+                              int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal,
+                              int io_dtype, int w_dtype, void *stream);
 /* y[i][b,h,p,:] = p < S_in and not hidden ? x[i][b,h,p,:] * scale[i] : 0 for i < count <= 3: rows of (B,H,S_in,D[i]) tensors
  * into dense (B,H,S_out,D[i]) ones - padded with zero rows or cut -, x with the strides x_strides[3i .. 3i+2] (batch entry,
  * head, row; elements; the last dimension dense).  hide[i] != 0: the rows with key_bias[b * bias_stride + p] = -inf (fp32)

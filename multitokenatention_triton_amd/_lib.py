@@ -58,6 +58,9 @@ SIGNATURES = {
     "mta_headmix_bwd_input": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_headmix_bwd_weight_workspace": (_i64, [_i64, _i64, _i64, _i64]),
     "mta_headmix_bwd_weight": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp]),
+    "mta_headmix_grads_workspace": (_i64, [_i64, _i64, _i64, _i64, _int, _int, _int, _int, _int]),
+    "mta_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
+    "mta_softmax_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_headmix_bwd_weight_as": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_rows_copy": (_int, [_int] + [_vp] * 7 + [_i64] * 5 + [_int, _vp]),
     "mta_causal_pv_scaled_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),

@@ -399,18 +399,41 @@ Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, con
     return p;
 }
 
+// The gradients of a head mixing with respect to its input and its weight (those that are wanted).  One kernel where it is both;
+// small: also for one of them, which costs nothing there and gives the bits that it has beside the other.
+std::pair<Tensor, Tensor> headmix_bwd(const Tensor &dy, const Tensor &x, const Tensor &w, bool causal, int64_t group, bool fill_upper, bool need_x,
+                                      bool need_w, bool small)
+{
+    if ((need_x && need_w) || (small && (need_x || need_w))) {
+        if (auto both = headmix_grads(std::nullopt, dy, x, w, causal, group, fill_upper))
+            return {need_x ? both->first : Tensor(), need_w ? both->second : Tensor()};
+    }
+    return {need_x ? headmix_bwd_input(dy, w, causal, group, fill_upper) : Tensor(),
+            need_w ? headmix_bwd_weight(x, dy.to(x.scalar_type()), w, causal, group) : Tensor()};
+}
+
 // the gradients of q, k, conv_w and w_pre (need[i]: wanted) from the one of the probabilities p
 void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, Tensor raw, const Tensor &x, const Tensor &p,
                        const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4])
 {
     const double scale = score_scale(q);
     // (the head mixing's gradient kernels never read above the diagonal when causal)
-    Tensor ds = softmax_bwd(p, dp, causal, false);
-    dp.reset();
-    if (need[3]) *out[3] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
-    if (!need[0] && !need[1] && !need[2]) return;
-    const Tensor dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, !causal);
-    ds.reset();
+    Tensor dx;
+    const bool need_x = need[0] || need[1] || need[2];
+    // (one kernel for the three gradients, also where one of them is for nobody: it reads less than the two that it takes otherwise)
+    const auto all = causal == pre_causal ? headmix_grads(p, dp, x, w_pre, causal, pre_group, !causal) : std::nullopt;
+    if (all) {
+        dp.reset();
+        if (need[3]) *out[3] = all->second;
+        if (!need_x) return;
+        dx = all->first;
+    } else {
+        Tensor ds = softmax_bwd(p, dp, causal, false);
+        dp.reset();
+        if (need[3]) *out[3] = headmix_bwd_weight(x, ds, w_pre, pre_causal, pre_group);
+        if (!need_x) return;
+        dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, !causal);
+    }
     if (need[0] || need[1]) {
         const bool lower = causal && q.sizes() == k.sizes() && dx.scalar_type() == q.scalar_type() && lower_products_supported(q.scalar_type(), q.sizes(), true);
         const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
@@ -552,8 +575,8 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
         if (need_c || need[6]) {
             Tensor dm = values_bwd_m(go, v, lower, first);
             if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
-            if (need[6]) out[6] = headmix_bwd_weight(c, dm, w_post, post_causal, post_group);
-            Tensor dc = need_c ? headmix_bwd_input(dm, w_post, post_causal, post_group, !causal) : Tensor();
+            Tensor dc;
+            std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], true);
             dm.reset();
             if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
             if (need_p) {
@@ -678,8 +701,8 @@ struct HeadMix : torch::autograd::Function<HeadMix> {
         const int64_t group = ctx->saved_data["group"].toInt();
         torch::autograd::variable_list out(7);
         const Tensor dy = on_gpu(grads[0], "grad_output");
-        if (ctx->needs_input_grad(0)) out[0] = headmix_bwd_input(dy, saved[1], causal, group, ctx->saved_data["grad_fill_upper"].toBool());
-        if (ctx->needs_input_grad(1)) out[1] = headmix_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, group);
+        std::tie(out[0], out[1]) = headmix_bwd(dy, saved[0], saved[1], causal, group, ctx->saved_data["grad_fill_upper"].toBool(),
+                                               ctx->needs_input_grad(0), ctx->needs_input_grad(1), false);
         return out;
     }
 };

@@ -157,6 +157,30 @@ inline Tensor headmix_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tens
     return dw;
 }
 
+// The gradients of the head mixing with respect to its input and its weight in one pass; with `probs`, dy is the gradient of the
+// softmax behind it (of the probabilities `probs`).  Nothing where there is no kernel.
+inline std::optional<std::pair<Tensor, Tensor>> headmix_grads(const OptTensor &probs_, const Tensor &dy_, const Tensor &x_, const Tensor &w_, bool causal,
+                                                              int64_t group, bool fill_upper)
+{
+    if (dy_.dim() != 4 || dy_.scalar_type() != x_.scalar_type() || dy_.sizes() != x_.sizes()) return std::nullopt;
+    const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    const OptTensor probs = probs_ ? OptTensor(on_gpu(*probs_, "probabilities")) : probs_;
+    TORCH_CHECK(!probs || (probs->sizes() == x.sizes() && probs->scalar_type() == x.scalar_type()), "probabilities and input must share shape and dtype");
+    check_head_weight(w, x.size(1));
+    const int64_t n = x.size(0), c = x.size(1), p = x.size(2), q = x.size(3);
+    const int ic = code(x, "input"), wc = code(w, "weight"), mode = causal_mode(causal, fill_upper);
+    const int64_t bytes = mta_headmix_grads_workspace(n, c, p, q, (int)group, mode, probs.has_value(), ic, wc);
+    if (bytes <= 0) return std::nullopt;
+    Tensor dx = at::empty(x.sizes(), x.options()), dw = at::empty(w.sizes(), w.options()), ws = at::empty({bytes}, x.options().dtype(at::kByte));
+    const int rc = probs ? mta_softmax_headmix_grads(ptr(probs), ptr(dy), ptr(x), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q,
+                                                     (int)group, causal, ic, wc, stream_of(x))
+                         : mta_headmix_grads(ptr(x), ptr(dy), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, (int)group, mode, ic, wc,
+                                             stream_of(x));
+    if (rc == MTA_ERR_UNSUPPORTED) return std::nullopt;
+    check(rc, "mta_headmix_grads");
+    return std::make_pair(dx, dw);
+}
+
 inline Tensor headmix_softmax(const Tensor &x_, const OptTensor &w1, const OptTensor &w2, bool causal, int64_t group, bool fill_upper,
                               const OptTensor &key_bias, const OptTensor &first)
 {

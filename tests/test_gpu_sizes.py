@@ -386,3 +386,74 @@ def test_conv_mix16_one_or_two_kernels(pkg, ks, dtype):
         two = pkg.ops.headmix(pkg.ops.conv2d_causal(x, wc, True), wm, True, 0.0, group_size=16)
         ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
         torch.testing.assert_close(one.float(), two.float(), rtol=ulp, atol=4 * ulp)
+
+
+def _unit(dtype):
+    return {torch.float32: 2.0 ** -22, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,group", [(2, 0), (4, 0), (8, 0), (12, 0), (16, 0), (32, 0), (16, 2), (8, 4), (24, 12), (32, 16), (16, 8)])
+def test_headmix_both_gradients(pkg, c, group, dtype):
+    """The head mixing's two gradients in one pass, at edges of its tiles (vectors, 64 or 128 keys, 256 or 512) and with NaN above the
+    diagonal.  Against float64: dx is one rounding of an fp32 sum of at most 32 products; dw fp32 sums of n products in an order
+    whose error sqrt(n)*2^-22 of the sum of magnitudes covers."""
+    g = torch.Generator().manual_seed(41)
+    half_step = 2.0 ** -25 if dtype == torch.float16 else 0.0   # (rounding of a subnormal result)
+    for p, q, mode in ((1, 8, "fill"), (8, 8, "lower"), (72, 72, "fill"), (65, 136, "all"), (136, 136, "lower"), (200, 520, "fill"), (33, 1032, "all"),
+                       (264, 264, "lower")):
+        print(f"headmix gradients c={c} group={group} {p}x{q} {mode} {dtype}", flush=True)
+        causal, n = mode != "all", 3 if p == 65 else 2
+        x, dy = (torch.randn(n, c, p, q, generator=g).to(dtype) for _ in range(2))
+        w = (torch.eye(c) + 0.3 * torch.randn(c, c, generator=g)).to(dtype)
+        block = torch.arange(c) // (group or c)
+        same = block[:, None] == block[None, :]
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        xd, dyd, wd = x.double().masked_fill(~keep, 0.0), dy.double().masked_fill(~keep, 0.0), w.double() * same
+        want = torch.einsum("oi,nopq->nipq", wd, dyd)
+        want_w = torch.einsum("nopq,nipq->oi", dyd, xd) * same
+        size_w = torch.einsum("nopq,nipq->oi", dyd.abs(), xd.abs())
+        sent = torch.full(x.shape, 7.0, dtype=dtype, device="cuda")
+        # (the entries of w outside its blocks are nobody's)
+        dx, dw = pkg.ops.headmix_grads(dy.masked_fill(~keep, float("nan")).cuda(), x.masked_fill(~keep, float("nan")).cuda(),
+                                       w.masked_fill(~same, float("inf")).cuda(), causal, group_size=group, fill_upper=mode == "fill", out=sent)
+        dx, dw = dx.cpu().double(), dw.cpu().double()
+        assert ((dx - want).abs() <= _unit(dtype) * 1.01 * want.abs() + 2.0 ** -19 * torch.einsum("oi,nopq->nipq", wd.abs(), dyd.abs()) + half_step)[..., keep].all()
+        if mode == "fill":
+            assert (dx[..., ~keep] == 0.0).all()
+        assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,group,longest", [(2, 0, 4096), (4, 0, 4096), (8, 0, 4096), (12, 0, 4096), (16, 0, 4096), (32, 0, 2048), (8, 4, 4096), (32, 16, 4096)])
+def test_softmax_and_headmix_gradients(pkg, c, group, longest, dtype):
+    """Softmax gradient, mixing and weight gradient in one pass: rows of one wavefront and of several, of one tile per wavefront and
+    of several, the longest row, NaN above the diagonal.  Against float64: the score gradient is rounded to the dtype (one unit u
+    of its magnitude), dx once more, dw's sums as above; fp32: the order of a row's sum of p * dp, below 4."""
+    g = torch.Generator().manual_seed(43)
+    longest = longest // 2 if dtype == torch.float32 else longest
+    u = _unit(dtype) if dtype != torch.float32 else 2.0 ** -20
+    for n, p, q, causal in ((2, 1, 8, True), (1, 8, 8, True), (3, 72, 72, True), (1, 136, 136, True), (1, 520, 520, True), (2, 3, 264, False), (1, 2, 1032, False),
+                            (1, 3, longest - 8, False), (1, 2, longest, False)):
+        if q > longest:
+            continue
+        print(f"softmax + headmix gradients c={c} group={group} {n}x{p}x{q} causal={causal} {dtype}", flush=True)
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        s = torch.softmax(torch.randn(n, c, p, q, generator=g).masked_fill(~keep, float("-inf")), -1).to(dtype)
+        ds, x = (torch.randn(n, c, p, q, generator=g).to(dtype) for _ in range(2))
+        w = (torch.eye(c) + 0.3 * torch.randn(c, c, generator=g)).to(dtype)
+        block = torch.arange(c) // (group or c)
+        same = block[:, None] == block[None, :]
+        sd, dsd, xd, wd = s.double().masked_fill(~keep, 0.0), ds.double().masked_fill(~keep, 0.0), x.double().masked_fill(~keep, 0.0), w.double() * same
+        dy = sd * (dsd - (sd * dsd).sum(-1, keepdim=True))
+        most = sd * (dsd.abs() + (sd * dsd.abs()).sum(-1, keepdim=True))   # (what a rounding of one of its terms is relative to)
+        want, size = torch.einsum("oi,nopq->nipq", wd, dy), torch.einsum("oi,nopq->nipq", wd.abs(), dy.abs() + 2.0 ** -19 / u * most)
+        want_w = torch.einsum("nopq,nipq->oi", dy, xd) * same
+        size_w = torch.einsum("nopq,nipq->oi", dy.abs() + 2.0 ** -19 / u * most, xd.abs())
+        tiny = 2.0 ** -24 * 32 if dtype == torch.float16 else 0.0   # (fp16: subnormal score gradients)
+        nan = float("nan")
+        dx, dw = pkg.ops.headmix_grads(ds.masked_fill(~keep, nan).cuda(), x.masked_fill(~keep, nan).cuda(), w.cuda(), causal, group_size=group,
+                                       probs=s.masked_fill(~keep, nan).cuda())
+        dx, dw = dx.cpu().double(), dw.cpu().double()
+        assert ((dx - want).abs() <= 2.02 * u * size + tiny)[..., keep].all()
+        assert ((dw - want_w).abs() <= u * want_w.abs() + 1.01 * u * size_w + tiny * xd.abs().sum()).all()
