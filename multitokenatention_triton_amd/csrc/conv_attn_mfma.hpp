@@ -579,8 +579,11 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         // One product needs one fresh 1 KB score fragment from LDS, and a wavefront that waits for each fragment
         // where it is used spends four times the products' own time here.  The reads are therefore issued NLD
         // products ahead, from assembly (see lds_read16_at), into a ring of registers; every product is preceded by
-        // a wait that leaves exactly the younger operations outstanding.  The result of an output block is taken up
-        // LAG products into the next block, when it is long complete.
+        // a wait that leaves exactly the younger operations outstanding.  Two neighbouring output blocks are worked on in
+        // turns: the R products of one block add into the same registers, each waiting for the one before (one block at a
+        // time | two: attention B1 H16 S2048 D64 6x11 83.8 | 79.9 us, B4 H8 S1024 D128 11x15 65.9 | 64.4, B1 H32 S8192 D128 6x11
+        // 1096 | 1080; the scores kernel, with three wavefronts per SIMD to fill the gaps, the same within 1 %).  Their results
+        // are taken up LAG products into the next two, when they are long complete.
         constexpr int NB = 2 * NCB, NREAD = NB * R;
         // score fragments in flight (scores only: 8 and 12 measure the same, 15 spills; the attention kernel, at the
         // 256-register limit, spills from 6 on)
@@ -590,10 +593,10 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         static_assert(NREAD > NLD && R >= LAG && NLD <= 15, "pipeline deeper than the work or than the counter");
         const unsigned xa = lds_addr(Sc) + (unsigned)(((trow[0] + cshift - (R - 1)) * F_SLD + kg * 8) * (int)sizeof(T));
         u32x4_t ring[NSLOT];
-        f32x4 cacc[2];
+        f32x4 cacc[4];
         auto issue = [&](auto ic) __attribute__((always_inline)) {
             constexpr int n = decltype(ic)::value;
-            constexpr int blk = n / R, i = n % R;
+            constexpr int blk = n / (2 * R) * 2 + (n & 1), i = n % (2 * R) / 2;   // output block, kernel row
             ring[n % NSLOT] = lds_read16_at(xa, (((blk / NCB) * 16 + i) * F_SLD + (blk % NCB) * 16) * (int)sizeof(T));
         };
         // what happens to output block b = rb*NCB + cb (rows crow[rb], keys j*64 + 16cb ..) once it is complete
@@ -603,7 +606,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         auto finish = [&](auto bc) __attribute__((always_inline)) {
             constexpr int b = decltype(bc)::value;
             constexpr int rb = b / NCB, cb = b % NCB;
-            const f32x4 a = cacc[b & 1];
+            const f32x4 a = cacc[b & 3];
             const int p_ = cprow[rb];
             if constexpr (SCORES_ONLY) {
                 // Blocks leave in pairs, like the scores above: after the exchange a lane holds 8 consecutive keys of
@@ -647,11 +650,11 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 if constexpr (cb == 0) mloc = -INFINITY;
                 if (!c_plain) {
                     MTA_KEEP_BRANCH();
+                    // (the column from a laundered lane index: formed here, not by every key block)
+                    const int left = (causal ? (p_ < S - 1 ? p_ : S - 1) : S - 1) - (j * F_BK + cb * 16) - opaque_lane(kg) * 4;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int col = j * F_BK + cb * 16 + kg * 4 + v;
-                        if (!(col < S && !(causal && col > p_))) v4[v] = -INFINITY;
-                    }
+                    for (int v = 0; v < 4; ++v)
+                        if (v > left) v4[v] = -INFINITY;
                 }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
@@ -696,19 +699,20 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         static_for<NLD>(issue);
         static_for<NREAD>([&](auto ic) __attribute__((always_inline)) {
             constexpr int n = decltype(ic)::value;
-            constexpr int blk = n / R, i = n % R;
+            constexpr int blk = n / (2 * R) * 2 + (n & 1), i = n % (2 * R) / 2;
             if constexpr (n + NLD < NREAD) issue(std::integral_constant<int, n + NLD>{});
             // LDS operations younger than read n: exactly the reads issued after it
             constexpr int younger = (n + NLD < NREAD ? n + NLD : NREAD - 1) - n;
             lds_wait_upto<younger>(ring[n % NSLOT]);
-            if constexpr (i == 0) cacc[blk & 1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            mma16(cacc[blk & 1], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
+            if constexpr (i == 0) cacc[blk & 3] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            mma16(cacc[blk & 3], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (blk >= 1 && i == LAG - 1) {
-                finish(std::integral_constant<int, blk - 1>{});
+            if constexpr (blk >= 2 && i == LAG - 1) {
+                finish(std::integral_constant<int, blk - 2>{});
                 __builtin_amdgcn_sched_barrier(0);
             }
         });
+        finish(std::integral_constant<int, NB - 2>{});
         finish(std::integral_constant<int, NB - 1>{});
         if constexpr (SCORES_ONLY) return;
 
