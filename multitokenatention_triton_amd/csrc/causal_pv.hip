@@ -33,11 +33,9 @@ constexpr int P_BK = 64;  // keys per iteration (128 measured no faster): each l
                                  // iteration, back to back, so that DRAM pages are used in long runs
 constexpr int P_KS = P_BK / 32;  // 32-key contraction steps per iteration
 
-// SPLIT = 2: two such groups of wavefronts in a workgroup share the query rows and take the even and the odd key
-// blocks; the second group's sums reach the first through LDS at the end.  For grids that put one workgroup on a CU
-// (few heads): twice the loads in flight for the same bytes.
-template <typename T, int D, int SPLIT>
-__global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_pv_kernel(
+// This kernel stays for (B,H,S,S) planes of 4096 keys and more in grids of 2048 row blocks and more (product_form()).
+template <typename T, int D>
+__global__ __launch_bounds__(P_NT, P_OCC) void causal_pv_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int nqb, int64_t total_wg,
     int64_t per_xcd, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
 {
@@ -45,17 +43,13 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
     constexpr int TILE = P_BK * D;           // elements per V block
     constexpr int ROUNDS = (TILE / 8 + P_NT - 1) / P_NT;
     constexpr int DB = D / 16;
-    static_assert(SPLIT == 1 || (size_t)SPLIT * TILE * sizeof(T) == (size_t)DB * P_NT * 16, "the sums of one row block fit one V buffer pair");
     // Double buffer as two separate arrays, and a loop body instantiated once per array: the compiler then sees that
     // the LDS reads of one block never touch the asynchronous copy in flight into the other.  With one array it
     // cannot, and waits for the copy (and for every load issued before it) ahead of the first LDS read.
-    __shared__ __align__(16) T v_a_all[SPLIT * TILE];
-    __shared__ __align__(16) T v_b_all[SPLIT * TILE];
+    __shared__ __align__(16) T v_a[TILE];
+    __shared__ __align__(16) T v_b[TILE];
 
-    const int grp = SPLIT == 2 ? (int)(threadIdx.x >> 8) : 0;  // which key blocks: j % SPLIT == grp
-    T *const v_a = v_a_all + grp * TILE;
-    T *const v_b = v_b_all + grp * TILE;
-    const int tid = threadIdx.x & (P_NT - 1);
+    const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     // XCD-aware order: XCD x (workgroup id % 8) takes the x-th eighth of the (batch*head, query block) list, so
     // the workgroups that share one head's V run on one L2; within a head the longest query blocks come first
@@ -138,14 +132,10 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
         j0 = (fmin > 0 ? fmin : 0) / P_BK;
         if (j0 > j_end) j0 = j_end;
     }
-    // this group's key blocks: jg, jg + SPLIT, ... (by the block's own parity, whatever the first block is: a band mask
-    // that skips blocks of zeros leaves every sum as it is, bit for bit)
-    const int jg = SPLIT == 2 ? j0 + ((j0 & 1) != grp) : j0;
-    const int nsteps = (j_end - j0) / SPLIT + 1;  // of the group that starts at j0: the other one idles in its last step
-    if (jg <= j_end) issue_v(jg, v_a);
+    issue_v(j0, v_a);
     // P fragments are fetched one key block ahead, alternately into two register sets
     frag8<T> p_a[2][P_KS], p_b[2][P_KS];
-    load_p(jg, p_a);
+    load_p(j0, p_a);
 
     f32x4 oacc[2][DB];
 #pragma unroll
@@ -156,10 +146,9 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
     auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pcur)[2][P_KS], frag8<T> (&pnext)[2][P_KS]) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0);  // V block j and the P fragments have arrived
         __syncthreads();                // for every wavefront; reads of the other buffer are finished
-        if (SPLIT == 2 && j > j_end) return;  // (the other group's last block: this one only meets it at the barrier)
-        if (j + SPLIT <= j_end) {
-            issue_v(j + SPLIT, Vn);
-            load_p(j + SPLIT, pnext);
+        if (j + 1 <= j_end) {
+            issue_v(j + 1, Vn);
+            load_p(j + 1, pnext);
         }
         // mask the fragments of this block: keys beyond the row (causal) or the sequence count as 0
         frag8<T> pf[2][P_KS];
@@ -202,32 +191,11 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    for (int i = 0, j = jg;; j += SPLIT) {
+    for (int j = j0;;) {
         step(j, v_a, v_b, p_a, p_b);
-        if (++i >= nsteps) break;
-        j += SPLIT;
+        if (++j > j_end) break;
         step(j, v_b, v_a, p_b, p_a);
-        if (++i >= nsteps) break;
-    }
-
-    if constexpr (SPLIT == 2) {
-        // the second group's sums travel through the V buffers (rows' first block in one, second in the other)
-        typedef __attribute__((address_space(3))) f32x4 lds_f4;
-        __syncthreads();  // nobody reads V any more
-        if (grp == 1) {
-#pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                reinterpret_cast<f32x4 *>(v_a_all)[db * P_NT + tid] = oacc[0][db];
-                reinterpret_cast<f32x4 *>(v_b_all)[db * P_NT + tid] = oacc[1][db];
-            }
-        }
-        __syncthreads();
-        if (grp == 1) continue;  // (the barrier ahead of the second row block is met at the top of the loop)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            oacc[0][db] += reinterpret_cast<const f32x4 *>(v_a_all)[db * P_NT + tid];
-            oacc[1][db] += reinterpret_cast<const f32x4 *>(v_b_all)[db * P_NT + tid];
-        }
+        if (++j > j_end) break;
     }
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -247,8 +215,8 @@ __global__ __launch_bounds__(P_NT * SPLIT, SPLIT == 2 ? 1 : P_OCC) void causal_p
 // The two products with 32 output rows per workgroup, whose four wavefronts take every fourth 32-row step of the contraction
 // each, on operands of their own in LDS (no barrier in the loop), and add their sums up at the end.  With 128 rows per
 // wavefront group a short sequence is a few dozen workgroups that each walk their keys alone; this is 8 times as many with a
-// quarter of the steps.  The price is that a V (X) block serves 32 rows instead of 128, so long sequences of many heads,
-// whose grids fill the chip anyway, keep the kernels above and below (narrow_grid()).
+// quarter of the steps.  The price is that a V (X) block serves 32 rows, so only grids that fill the chip in no other way
+// take it (product_form()).
 constexpr int RB = 2, N_ROWS = 16 * RB;   // 16-row blocks, output rows per workgroup (64 rows: the sums leave too few registers)
 constexpr int N_STEP = 32;                // contraction rows per step
 // the sums of the four wavefronts, added in their order: wavefront w takes 16-wide blocks w, w+4, ... of the head dim
@@ -400,6 +368,189 @@ __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__res
     });
 }
 
+// The workgroup's (batch, head) and its rank among that head's row blocks, longest first.  XCD x (workgroup id % 8) takes its own
+// heads (operands that row blocks share stay in one L2), hpx of them each where they divide evenly: all heads' longest blocks
+// first.  snake: the grid is resident at once, two workgroups per CU - the second half comes in reverse, so that a CU gets a
+// long block and a short one.
+__device__ __forceinline__ bool mid_item(int64_t &bh, int &rank, int nrb, int64_t total_wg, int64_t per_xcd, int hpx, int snake)
+{
+    if (hpx > 0) {
+        const int n = hpx * nrb;
+        int pos = (int)(blockIdx.x >> 3);
+        if (snake && pos >= n / 2) pos = n - 1 - (pos - n / 2);
+        bh = (int64_t)(blockIdx.x & 7) * hpx + pos % hpx;
+        rank = pos / hpx;
+        return true;
+    }
+    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    bh = lid / nrb;
+    rank = (int)(lid % nrb);
+    return lid < total_wg;
+}
+
+// The sums of GR groups of GT threads added up in the first group (true there): the upper half of the groups hand theirs to the
+// lower half through the two operand buffers, which together hold just that, until one is left.
+template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mid_sums(T *a, T *b, f32x4 (&oacc)[DB], int grp, int tid)
+{
+    __syncthreads();   // nobody reads operands any more
+#pragma unroll
+    for (int h = GR / 2; h > 0; h /= 2) {
+        auto place = [&](int g, int db) -> f32x4 & {
+            const int at = g * DB + db;
+            return at < h * DB / 2 ? reinterpret_cast<f32x4 *>(a)[at * GT + tid] : reinterpret_cast<f32x4 *>(b)[(at - h * DB / 2) * GT + tid];
+        };
+        if (grp >= h && grp < 2 * h) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) place(grp - h, db) = oacc[db];
+        }
+        __syncthreads();
+        if (grp < h) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) oacc[db] += place(grp, db);
+        }
+        if (h > 1) __syncthreads();
+    }
+    return grp == 0;
+}
+
+// ---- grids between the two --------------------------------------------------------------------------------------------
+// RW wavefronts of 16 rows share a block of V (64 keys) in LDS, GR groups of them take every GR-th block; 16 wavefronts per CU in
+// every form (two workgroups of 8 or one of 16).  A wavefront of 16 rows instead of 32 reads its V fragments from LDS for one
+// product each instead of two, which the LDS has room for, and leaves the registers (95 instead of 180) for twice the
+// wavefronts: the reads of P and V that one waits for fly beside the others' products.
+template <typename T, int D, int RW, int GR>
+__global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1)) void causal_pv_mid_kernel(
+    const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int nrb, int64_t total_wg, int64_t per_xcd, int hpx,
+    int snake, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+{
+    constexpr int CPR = D / 8, TILE = P_BK * D, GT = 64 * RW, ROUNDS = TILE / 8 / GT, DB = D / 16, ROWS = 16 * RW;
+    static_assert(TILE / 8 % GT == 0 && (GT / CPR) % 16 == 0, "whole copy rounds that keep the swizzle phase");
+    __shared__ __align__(16) T v_a_all[GR * TILE];
+    __shared__ __align__(16) T v_b_all[GR * TILE];
+    const int tid = threadIdx.x % GT, grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    T *const v_a = v_a_all + grp * TILE;
+    T *const v_b = v_b_all + grp * TILE;
+    int64_t bh;
+    int rank;
+    if (!mid_item(bh, rank, nrb, total_wg, per_xcd, hpx, snake)) return;
+    const int q0 = (nrb - 1 - rank) * ROWS;
+    const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
+    const T *Vp = V + bh * (int64_t)S * D;
+    T *Op = O + bh * (int64_t)S * D;
+
+    const int row0 = tid / CPR, voff0 = row0 * D + ((tid % CPR) ^ v_swizzle<D>(row0)) * 8;
+    auto issue_v = [&](int j, T *dst) {   // keys past the sequence re-read the last one: their probabilities are masked
+        const bool inside = (j + 1) * P_BK <= S;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            int off = j * TILE + voff0 + r * (GT / CPR) * D;
+            if (!inside) {
+                const int key = j * P_BK + row0 + r * (GT / CPR);
+                off -= (key >= S ? key - (S - 1) : 0) * D;
+            }
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Vp + off), (lds_void_t *)(dst + (r * GT + wave * 64) * 8), 16, 0, 0);
+        }
+    };
+    const int w0 = q0 + wave * 16, prow = w0 + ln;
+    const int pc = prow < S ? prow : S - 1;
+    const T *prow_ptr = tri_gl > 0 ? Pp + tri_gl * tri_rowoff(pc) + (int)(bh % tri_gl) * tri_rowlen(pc) : Pp + (int64_t)pc * S;
+    const int lim = causal ? pc : S - 1;   // last key of this lane's row
+    auto load_p = [&](int j, frag8<T> (&pf)[P_KS]) {
+#pragma unroll
+        for (int ks = 0; ks < P_KS; ++ks) {
+            const int key = j * P_BK + ks * 32 + kg * 8;
+            pf[ks] = *reinterpret_cast<const frag8<T> *>(prow_ptr + (key <= lim ? key : 0));
+        }
+    };
+    const int q_last = (q0 + ROWS - 1 < S - 1) ? q0 + ROWS - 1 : S - 1;
+    const int j_end = causal ? q_last / P_BK : (S - 1) / P_BK;
+    int j0 = 0;
+    if (band_lo) {   // the blocks ahead of the first key any of these rows sees hold zeros
+        int f = S;
+        for (int r = lane; r < ROWS; r += 64)
+            if (q0 + r < S) {
+                const int b = band_lo[(bh / H) * (int64_t)S + q0 + r];
+                f = b < f ? b : f;
+            }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const int o = __shfl_xor(f, off);
+            f = o < f ? o : f;
+        }
+        f = __builtin_amdgcn_readfirstlane(f);
+        j0 = (f > 0 ? f : 0) / P_BK;
+        if (j0 > j_end) j0 = j_end;
+    }
+    // this group's blocks, by the block's own number (what a band mask skips leaves every sum as it is)
+    const int jg = j0 + ((grp - j0) & (GR - 1)), nsteps = (j_end - j0) / GR + 1;
+    f32x4 oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    frag8<T> p_a[P_KS], p_b[P_KS];
+    if (jg <= j_end) issue_v(jg, v_a);
+    load_p(jg, p_a);
+    // lane's place in a block of V for the transpose reads: rows kg*8 + ln/4 (+4), whose swizzle no other part of the row
+    // number touches; head-dim block db is an exclusive or away
+    const int vrow = kg * 8 + (ln >> 2), vat = vrow * D + ((((ln & 3) >> 1) ^ v_swizzle<D>(vrow)) * 8) + (ln & 1) * 4;
+    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pf)[P_KS], frag8<T> (&pn)[P_KS]) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);   // V block j and the P fragments have arrived
+        __syncthreads();                 // for every wavefront; reads of the other buffer are finished
+        if (j > j_end) return;
+        if (j + GR <= j_end) {
+            issue_v(j + GR, Vn);
+            load_p(j + GR, pn);
+        }
+        if (causal && j * P_BK > w0 + 15) return;   // wholly above the diagonal for these rows
+        if (j * P_BK + P_BK - 1 > (causal ? w0 : S - 1)) {
+#pragma unroll
+            for (int ks = 0; ks < P_KS; ++ks) {
+                const int left = lim - (j * P_BK + ks * 32 + kg * 8);
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    if (t > left) pf[ks].v[t] = from_float<T>(0.0f);
+            }
+        }
+        auto load_vf = [&](int blk, frag8<T> &dst) {
+            const int ks = blk / DB, db = blk % DB;
+            const T *pa = Vb + (vat ^ (db * 16)) + ks * 32 * D;
+            struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pa),
+                                           __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(pa + 4 * D))};
+            dst = __builtin_bit_cast(frag8<T>, both);
+        };
+        constexpr int AHEAD = 2;
+        frag8<T> vf[AHEAD + 1];
+#pragma unroll
+        for (int b = 0; b < AHEAD; ++b) load_vf(b, vf[b]);
+#pragma unroll
+        for (int blk = 0; blk < P_KS * DB; ++blk) {
+            if (blk + AHEAD < P_KS * DB) load_vf(blk + AHEAD, vf[(blk + AHEAD) % (AHEAD + 1)]);
+            __builtin_amdgcn_sched_barrier(0);
+            mma16(oacc[blk % DB], vf[blk % (AHEAD + 1)], pf[blk / DB]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int i = 0, j = jg;;) {
+        step(j, v_a, v_b, p_a, p_b);
+        if (++i >= nsteps) break;
+        j += GR;
+        step(j, v_b, v_a, p_b, p_a);
+        if (++i >= nsteps) break;
+        j += GR;
+    }
+    if constexpr (GR > 1) {
+        if (!mid_sums<T, DB, GT, GR>(v_a_all, v_b_all, oacc, grp, tid)) return;
+    }
+    if (prow >= S) return;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[db][v] * scale);
+        *reinterpret_cast<quad *>(Op + (int64_t)prow * D + db * 16 + kg * 4) = out;
+    }
+}
+
 // swizzle of a P tile of 32 keys (4 chunks per row): the transpose read serves rows 0..3 and 8..11 (+4, +16) together, and
 // rows 8 apart share banks
 __device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1); }
@@ -514,229 +665,226 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
 // ---- the transposed product --------------------------------------------------------------------------------------
 // O[k, :] = sum over p of P[p, k] X[p, :], p >= k only when causal: the gradients that the two matrix products of the
 // attention leave on their right-hand operands (dV = P^T dO, dK = G^T Q), whose left factor is only defined - and only
-// read - on and below the diagonal.
-//
-// A workgroup owns 128 keys (output rows; 32 per wavefront, two blocks of 16) and walks the query rows from its first
-// key downwards in blocks of 64.  O^T += X^T P on 16x16x32 MFMAs with the query rows as contraction index: both
-// operands are copied global -> LDS asynchronously as row-major blocks (64 rows of X, 64 rows x 128 keys of P; double
-// buffered, 16-byte chunks XOR-swizzled by row) and both fragments come out of them through the LDS transpose read,
-// which hands a lane four consecutive rows of one column: X^T with the head dim as operand row, P with the key as
-// operand column.  P is streamed from memory once; the X blocks are re-read from L2 by every key block above them.
-constexpr int T_KB = 32 * P_WAVES;  // keys per workgroup
-constexpr int T_PB = 64;            // query rows per step
-constexpr int T_KS = T_PB / 32;
-
-template <typename T, int D>
-__global__ __launch_bounds__(P_NT, P_OCC) void causal_ptx_kernel(const T *__restrict__ P, const T *__restrict__ X,
-                                                                 T *__restrict__ O, int S, int causal, int nkb, int64_t total_wg,
-                                                                 int64_t per_xcd, float scale)
+// read - on and below the diagonal.  O^T += X^T P on 16x16x32 MFMAs with the query rows as contraction index: both operands are
+// copied global -> LDS asynchronously as row-major blocks (double buffered, 16-byte chunks XOR-swizzled by row) and both
+// fragments come out of them through the LDS transpose read, which hands a lane four consecutive rows of one column.
+// Grids between the two: RW wavefronts of 16 keys share a block of PB query rows (X and P), GR groups of them take every GR-th
+// block; grid order and sums as in causal_pv_mid_kernel.
+template <typename T, int D, int RW, int GR, int PB>
+__global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
+                                                                         int causal, int nkb, int64_t total_wg, int64_t per_xcd, int hpx, int snake,
+                                                                         float scale)
 {
-    constexpr int XT = T_PB * D, PT = T_PB * T_KB;  // elements per X block / P tile
-    constexpr int XC = D / 8, PC = T_KB / 8;        // 16-byte chunks per row
-    constexpr int XR = XT / 8 / P_NT, PR = PT / 8 / P_NT;
-    static_assert(XT / 8 % P_NT == 0 && PT / 8 % P_NT == 0, "whole copy rounds");
-    constexpr int DB = D / 16;
-    __shared__ __align__(16) T x_a[XT];
-    __shared__ __align__(16) T x_b[XT];
-    __shared__ __align__(16) T p_a[PT];
-    __shared__ __align__(16) T p_b[PT];
-
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, ln = lane & 15, kg = lane >> 4;
-    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (lid >= total_wg) return;
-    // two key blocks per workgroup, pi and nkb-1-pi: under the causal rule the first has the most query rows and the
-    // second the fewest, so that every workgroup gets the same amount of work
-    const int npairs = (nkb + 1) / 2;
-    const int pi = (int)(lid % npairs);
-    const int64_t bh = lid / npairs;
+    constexpr int XC = D / 8, KB = 16 * RW, PC = KB / 8, XT = PB * D, PT = PB * KB, GT = 64 * RW, XR = XT / 8 / GT, PR = PT / 8 / GT, DB = D / 16,
+                  KS = PB / 32;
+    static_assert(XT / 8 % GT == 0 && PT / 8 % GT == 0 && GT / XC % 16 == 0 && GT / PC % 16 == 0, "whole copy rounds that keep the swizzle phase");
+    __shared__ __align__(16) T x_a_all[GR * XT];
+    __shared__ __align__(16) T x_b_all[GR * XT];
+    __shared__ __align__(16) T p_a_all[GR * PT];
+    __shared__ __align__(16) T p_b_all[GR * PT];
+    const int tid = threadIdx.x % GT, grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    T *const x_a = x_a_all + grp * XT;
+    T *const x_b = x_b_all + grp * XT;
+    T *const p_a = p_a_all + grp * PT;
+    T *const p_b = p_b_all + grp * PT;
+    int64_t bh;
+    int kb;
+    if (!mid_item(bh, kb, nkb, total_wg, per_xcd, hpx, snake)) return;
+    const int k0 = kb * KB;   // (the first keys have the most query rows)
     const T *Pp = P + bh * (int64_t)S * S;
     const T *Xp = X + bh * (int64_t)S * D;
     T *Op = O + bh * (int64_t)S * D;
-  for (int half = 0; half < 2; ++half) {
-    const int kb = half == 0 ? pi : nkb - 1 - pi;
-    if (half == 1 && kb == pi) break;  // odd number of blocks: the middle one is alone
-    const int k0 = kb * T_KB;
-    if (half == 1) __syncthreads();    // the buffers are reused: everybody has finished reading them
 
-    // block j = query rows 64j ..; rows past the sequence re-read the last row, keys past it the block's first chunk:
-    // what they bring in is masked (rows) or belongs to output rows that are not stored (keys)
-    auto issue = [&](int j, T *xdst, T *pdst) {
+    const int xrow0 = tid / XC, xoff0 = xrow0 * D + ((tid % XC) ^ v_swizzle<D>(xrow0)) * 8;
+    const int prow0 = tid / PC;
+    int pchunk = (tid % PC) ^ v_swizzle<KB>(prow0);
+    if (k0 + pchunk * 8 >= S) pchunk = 0;   // (keys past the sequence: rows of the result that nobody stores)
+    auto issue = [&](int j, T *xdst, T *pdst) {   // rows past the sequence re-read the last one: they are masked
+        const bool inside = (j + 1) * PB <= S;
 #pragma unroll
         for (int r = 0; r < XR; ++r) {
-            const int slot = r * P_NT + tid;
-            const int row = slot / XC, c = (slot % XC) ^ v_swizzle<D>(row);
-            int pr = j * T_PB + row;
-            pr = pr >= S ? S - 1 : pr;
-            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + (int64_t)pr * D + c * 8),
-                                             (lds_void_t *)(xdst + (r * P_NT + wave * 64) * 8), 16, 0, 0);
+            const int row = j * PB + xrow0 + r * (GT / XC), back = inside || row < S ? 0 : row - (S - 1);
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + ((int64_t)j * XT + xoff0 + (r * (GT / XC) - back) * D)),
+                                             (lds_void_t *)(xdst + (r * GT + wave * 64) * 8), 16, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < PR; ++r) {
-            const int slot = r * P_NT + tid;
-            const int row = slot / PC;
-            int c = (slot % PC) ^ v_swizzle<T_KB>(row);
-            if (k0 + c * 8 >= S) c = 0;
-            int pr = j * T_PB + row;
-            pr = pr >= S ? S - 1 : pr;
-            __builtin_amdgcn_global_load_lds((glb_void_t *)(Pp + (int64_t)pr * S + k0 + c * 8),
-                                             (lds_void_t *)(pdst + (r * P_NT + wave * 64) * 8), 16, 0, 0);
+            const int row = j * PB + prow0 + r * (GT / PC), from = inside || row < S ? row : S - 1;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Pp + (int64_t)from * S + k0 + pchunk * 8), (lds_void_t *)(pdst + (r * GT + wave * 64) * 8), 16,
+                                             0, 0);
         }
     };
-    // operand fragment out of a row-major block of LD columns: contraction slots t = 0..7 of step ks are the block's rows
-    // 32ks + 8kg + t, the operand's row / column is column 16*blk + ln of the block
-    auto frag_of = [&](const T *tile, auto ldc, int ks, int blk) {
-        constexpr int LD = decltype(ldc)::value;
-        const int row_a = ks * 32 + kg * 8 + (ln >> 2), row_b = row_a + 4;
-        const int ch = blk * 2 + ((ln & 3) >> 1);
-        const int sub = (ln & 1) * 4;
-        const T *pa = tile + row_a * LD + ((ch ^ v_swizzle<LD>(row_a)) * 8) + sub;
-        const T *pb = tile + row_b * LD + ((ch ^ v_swizzle<LD>(row_b)) * 8) + sub;
-        struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pa),
-                                       __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pb)};
+    // a lane's place in a block for the transpose reads: rows kg*8 + ln/4 (+4; 32 further per step), whose swizzle no other part
+    // of the row number touches; 16-wide column block c is an exclusive or away
+    const int trow = kg * 8 + (ln >> 2), half = (ln & 3) >> 1, sub = (ln & 1) * 4;
+    const int xat = trow * D + ((half ^ v_swizzle<D>(trow)) * 8) + sub, pat = trow * KB + (((wave * 2 + half) ^ v_swizzle<KB>(trow)) * 8) + sub;
+    auto read_tr = [&](const T *at, int ld) {
+        struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)at),
+                                       __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(at + 4 * ld))};
         return __builtin_bit_cast(frag8<T>, both);
     };
-
-    // this lane's two output rows (keys)
-    int krow[2];
+    const int w0 = k0 + wave * 16, krow = w0 + ln;
+    const int j_start = causal ? k0 / PB : 0, j_end = (S - 1) / PB;
+    const int jg = j_start + ((grp - j_start) & (GR - 1)), nsteps = (j_end - j_start) / GR + 1;
+    f32x4 oacc[DB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) krow[rb] = k0 + (wave * 2 + rb) * 16 + ln;
-    const int j_start = causal ? k0 / T_PB : 0, j_end = (S - 1) / T_PB;
-    f32x4 oacc[2][DB];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) oacc[rb][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    issue(j_start, x_a, p_a);
-
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (jg <= j_end) issue(jg, x_a, p_a);
     auto step = [&](int j, const T *Xb, const T *Pb, T *Xn, T *Pn) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0);  // block j has arrived
-        __syncthreads();                // for every wavefront; reads of the other buffers are finished
-        if (j < j_end) issue(j + 1, Xn, Pn);
-        // P fragments of this wavefront's two key blocks; query rows above the key (causal: P is undefined there) or
-        // past the sequence count as 0
-        frag8<T> pf[2][T_KS];
-        const int pbase = j * T_PB;
-        const bool edge = pbase + T_PB > S || (causal && pbase < k0 + T_KB - 1);  // (wavefront-uniform)
+        __builtin_amdgcn_s_waitcnt(0);   // block j has arrived
+        __syncthreads();                 // for every wavefront; reads of the other buffers are finished
+        if (j > j_end) return;
+        if (j + GR <= j_end) issue(j + GR, Xn, Pn);
+        const int pbase = j * PB;
+        if (causal && pbase + PB - 1 < w0) return;   // every row of the block lies above these keys
+        const bool edge = pbase + PB > S || (causal && pbase < w0 + 15);
+        frag8<T> pf[KS];
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+        for (int ks = 0; ks < KS; ++ks) {
+            pf[ks] = read_tr(Pb + pat + ks * 32 * KB, KB);
+            if (edge) {   // query rows above the key (causal: P is undefined there) or past the sequence count as 0
+                const int first = (causal ? krow : 0) - (pbase + ks * 32 + kg * 8), end = S - (pbase + ks * 32 + kg * 8);
 #pragma unroll
-            for (int ks = 0; ks < T_KS; ++ks) {
-                pf[rb][ks] = frag_of(Pb, std::integral_constant<int, T_KB>{}, ks, wave * 2 + rb);
-                if (edge) {
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const int p = pbase + ks * 32 + kg * 8 + t;
-                        if (p >= S || (causal && p < krow[rb])) pf[rb][ks].v[t] = from_float<T>(0.0f);
-                    }
-                }
+                for (int t = 0; t < 8; ++t)
+                    if (t < first || t >= end) pf[ks].v[t] = from_float<T>(0.0f);
             }
-        frag8<T> xf[2];
-        xf[0] = frag_of(Xb, std::integral_constant<int, D>{}, 0, 0);
+        }
+        constexpr int AHEAD = 2;
+        frag8<T> xf[AHEAD + 1];
 #pragma unroll
-        for (int blk = 0; blk < T_KS * DB; ++blk) {
-            const int ks = blk / DB, db = blk % DB;
-            if (blk + 1 < T_KS * DB) xf[(blk + 1) & 1] = frag_of(Xb, std::integral_constant<int, D>{}, (blk + 1) / DB, (blk + 1) % DB);
-            __builtin_amdgcn_sched_barrier(0);  // (the instruction scheduler would move the reads back behind the products)
-            mma16(oacc[0][db], xf[blk & 1], pf[0][ks]);
-            mma16(oacc[1][db], xf[blk & 1], pf[1][ks]);
+        for (int b = 0; b < AHEAD; ++b) xf[b] = read_tr(Xb + (xat ^ (b % DB * 16)) + b / DB * 32 * D, D);
+#pragma unroll
+        for (int blk = 0; blk < KS * DB; ++blk) {
+            constexpr int N = KS * DB;
+            const int nb = blk + AHEAD;
+            if (nb < N) xf[nb % (AHEAD + 1)] = read_tr(Xb + (xat ^ (nb % DB * 16)) + nb / DB * 32 * D, D);
+            __builtin_amdgcn_sched_barrier(0);
+            mma16(oacc[blk % DB], xf[blk % (AHEAD + 1)], pf[blk / DB]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    for (int j = j_start;;) {
+    for (int i = 0, j = jg;;) {
         step(j, x_a, p_a, x_b, p_b);
-        if (++j > j_end) break;
+        if (++i >= nsteps) break;
+        j += GR;
         step(j, x_b, p_b, x_a, p_a);
-        if (++j > j_end) break;
+        if (++i >= nsteps) break;
+        j += GR;
     }
-
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-        if (krow[rb] >= S) continue;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) {
-            struct alignas(8) quad { T v[4]; } out;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[rb][db][v] * scale);
-            *reinterpret_cast<quad *>(Op + (int64_t)krow[rb] * D + db * 16 + kg * 4) = out;
-        }
+    if constexpr (GR > 1) {
+        if (!mid_sums<T, DB, GT, GR>(x_a_all, x_b_all, oacc, grp, tid)) return;
     }
-  }
+    if (krow >= S) return;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[db][v] * scale);
+        *reinterpret_cast<quad *>(Op + (int64_t)krow * D + db * 16 + kg * 4) = out;
+    }
 }
 
-// MTA_PV_SPLIT in the environment: 1 / 2 / 3 = always one group / two groups / the narrow kernels (comparison switch)
-int pv_force()
+// ---- which kernel ------------------------------------------------------------------------------------------------------
+// What bounds both products is the bytes a CU can pull through the L2 (about 9 TB/s over the chip): the scores once, and the other
+// operand (V, X) once for every block of output rows.  Larger blocks need less of it, smaller ones fill the chip: the line
+// runs by the number of 64-row blocks.  us, narrow | 64 rows, four groups | 64 rows, two groups | 128 rows, two groups | 128 rows, one
+// group | the wide kernel (P V; P^T X had pairs of 128 keys per workgroup there), rotating P tensors:
+//   P V    B2 H4 S2048 D128 (256 blocks)  18.3 | 19.3 | 21.5 | 28.8 | 32.7 | 48.0      B1 H16 S1024 D128 (256)   13.9 | 12.5 | 12.9 | 17.4 | 18.6 | 29.6
+//          B1 H8 S3072 D128 (384)         36.2 | 33.2 | 39.2 | 50.2 | 59.4 | 72.4      B2 H16 S1008 D64 (512)    16.3 | 11.9 | 11.6 | 13.7 | 15.3 | 28.8
+//          B1 H16 S2048 D128 (512)        34.2 | 29.8 | 28.6 | 36.3 | 41.9 | 51.7      B2 H12 S2048 D128 (768)   58.4 | 53.3 | 40.7 | 45.3 | 51.4 | 55.2
+//          B1 H16 S4096 D128 (1024)       118  | 113  | 91.7 | 84.6 | 101  | 95.7      B4 H16 S1024 D128 (1024)  45.1 | 36.2 | 28.0 | 28.1 | 26.2 | 31.8
+//          B2 H16 S3072 D64 (1536)        105  | 88.6 | 76.9 | 85.3 | 86.3 | 97.3      B2 H16 S3072 D128 (1536)  137  | 114  | 98.6 | 98.0 | 89.9 | 111
+//          B4 H32 S2048 D64 (2048)        181  | 164  | 131  | 146  | 126  | 140       B2 H16 S4096 D64 (2048)   177  | 156  | 135  | 150  | 135  | 126
+//          in the triangular layout B2 H16 S4096 D128 (2048) 236 | 194 | 167 | 160 | 145 | 152, B4 H16 S4096 D128 465 | 388 | 331 | 318 | 282 | 305
+//   P^T X  B1 H12 S1000 D64 (192)         10.3 | 11.2 | 11.4 | 11.5 | 12.7 | 19.5      B1 H16 S1536 D128 (384)   17.3 | 16.2 | 18.5 | 21.7 | 24.7 | 34.1
+//          B1 H32 S1024 D128 (512)        19.6 | 16.2 | 14.1 | 17.2 | 18.6 | 26.7      B1 H16 S2048 D64 (512)    25.8 | 21.7 | 26.1 | 24.9 | 29.7 | 34.9
+//          B1 H16 S3072 D128 (768)        66.7 | 61.2 | 53.2 | 48.8 | 56.2 | 59.0      B1 H16 S4096 D64 (1024)   85.2 | 67.7 | 82.0 | 69.6 | 73.3 | 72.0
+//          B4 H16 S1024 D64 (1024)        27.2 | 20.1 | 18.6 | 21.2 | 19.5 | 23.3      B2 H16 S2048 D128 (1024)  64.8 | 69.0 | 49.9 | 51.1 | 50.4 | 53.6
+//          B3 H16 S2048 D128 (1536)       94.1 | 91.2 | 68.3 | 68.1 | 60.8 | 70.0      B4 H32 S2048 D64 (2048)   171  | 129  | 118  | 137  | 122  | 141
+// All but the narrow kernel add a row up in the same order (the even and the odd key blocks apart, with four groups by fours).
+enum product_kernel { WIDE = 1, R64_2, NARROW, R64_4, R128_2, R128_1 };
+
+product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bool tri)
 {
+    // MTA_PV_SPLIT in the environment: 1 .. 6 = always that kernel of the list above (comparison switch; P^T X has no wide one)
     static const int force = [] { const char *e = getenv("MTA_PV_SPLIT"); return e ? atoi(e) : 0; }();
-    return force;
+    if (force >= WIDE && force <= R128_1) return force == WIDE && transposed ? R128_1 : (product_kernel)force;
+    const int64_t n = heads * ((S + 63) / 64);
+    if (n < 256) return NARROW;
+    if (n < 450) return R64_4;
+    if (transposed) {
+        if (D == 64) return n < 2048 && S > 1024 ? R64_4 : R64_2;
+        if (n < 1024) return S <= 1024 ? R64_2 : n <= 512 ? R64_4 : R128_2;
+        return n < 1536 && S > 2048 ? R128_2 : R128_1;
+    }
+    if (n >= 2048) return S >= 4096 && !tri ? WIDE : R128_1;
+    if (D == 64 || n < 1024) return R64_2;
+    return n < 1536 && S >= 2048 ? R128_2 : R128_1;
 }
-// Whether a product whose wide grid has that many workgroups (pairs of 128-row blocks) runs on the narrow kernels.  The line
-// lies where the two meet (us, wide -> narrow; P V in the triangular layout / P^T X): B1 H16 D128 S512 16.6 -> 6.7 / 17.8 -> 6.6;
-// S1024 24.3 -> 12.8 / 25.3 -> 10.8; S2048 (128 workgroups) 48.8 -> 27.3 / 40.8 -> 24.5; S4096 (256) 95 -> 118 / 77 -> 102;
-// B4 S1024 (256) 33.4 -> 37.5 / 27.7 -> 34.0; D64, half the bytes per V row: B1 H32 S2048 (256) 45.3 -> 36.1 / 30.1 -> 30.9,
-// B1 H16 S4096 (256) 93 -> 88 / 61 -> 70.
-bool narrow_grid(int64_t wide_wg, int most)
+
+// A kernel's grid: workgroups of `threads` threads, a block of `rows` output rows (WIDE: a pair of them) each; f(grid, blocks per
+// head, workgroups, workgroups per XCD, heads per XCD, snake).  False where it is too large.
+template <typename F> bool product_grid(int64_t heads, int64_t S, int rows, int threads, int causal, bool pairs, F &&f)
 {
-    if (pv_force()) return pv_force() == 3;
-    return wide_wg <= most;
+    const int64_t blocks = (S + rows - 1) / rows, wg = heads * (pairs ? (blocks + 1) / 2 : blocks), per_xcd = (wg + 7) / 8;
+    if (per_xcd * 8 > 0x7fffffffLL) return false;
+    const int hpx = heads % 8 == 0 ? (int)(heads / 8) : 0;
+    f(dim3((unsigned)(per_xcd * 8)), (int)blocks, wg, per_xcd, hpx, (int)(causal && wg <= device_cu_count() * (threads == 512 ? 2 : 1)));
+    return true;
 }
 
 template <typename T, int D>
 int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, float scale, hipStream_t st)
 {
-    int nkb = (int)((S + T_KB - 1) / T_KB);
-    int64_t total_wg = B * H * ((nkb + 1) / 2);
-    const bool narrow = narrow_grid(total_wg, 192);
-    if (narrow) {
-        nkb = (int)((S + N_ROWS - 1) / N_ROWS);
-        total_wg = B * H * nkb;
+    auto mid = [&](auto kern, int rows, int threads) {
+        return product_grid(B * H, S, rows, threads, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int hpx, int snake) {
+            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, blocks, wg, per_xcd, hpx, snake, scale);
+        });
+    };
+    bool fits = false;
+    switch (product_form(B * H, S, D, true, false)) {
+    case NARROW:
+        fits = product_grid(B * H, S, N_ROWS, 256, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int, int) {
+            hipLaunchKernelGGL((causal_ptx_narrow_kernel<T, D>), grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, blocks, wg,
+                               per_xcd, scale);
+        });
+        break;
+    case R64_4: fits = mid(causal_ptx_mid_kernel<T, D, 4, 4, 32>, 64, 1024); break;
+    case R64_2: fits = mid(causal_ptx_mid_kernel<T, D, 4, 2, 32>, 64, 512); break;
+    case R128_2: fits = mid(causal_ptx_mid_kernel<T, D, 8, 2, 64>, 128, 1024); break;
+    default: fits = mid(causal_ptx_mid_kernel<T, D, 8, 1, 64>, 128, 512); break;
     }
-    const int64_t per_xcd = (total_wg + 7) / 8;
-    if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
-    dim3 grid((unsigned)(per_xcd * 8));
-    if (narrow) {
-        auto kern = causal_ptx_narrow_kernel<T, D>;
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg, per_xcd, scale);
-        return launch_status();
-    }
-    auto kern = causal_ptx_kernel<T, D>;
-    hipLaunchKernelGGL(kern, grid, dim3(P_NT), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, nkb, total_wg,
-                       per_xcd, scale);
-    return launch_status();
+    return fits ? launch_status() : MTA_ERR_SHAPE;
 }
 
 template <typename T, int D>
 int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st,
            const int *band_lo = nullptr, int tri_gl = 0, float scale = 1.0f)
 {
-    int nqb = (int)((S + P_BQ - 1) / P_BQ);
-    int64_t total_wg = B * H * ((nqb + 1) / 2);
-    const bool narrow = narrow_grid(total_wg, D == 64 ? 256 : 192);
-    if (narrow) {
-        nqb = (int)((S + N_ROWS - 1) / N_ROWS);
-        total_wg = B * H * nqb;
+    auto mid = [&](auto kern, int rows, int threads) {
+        return product_grid(B * H, S, rows, threads, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int hpx, int snake) {
+            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, blocks, wg, per_xcd, hpx, snake, band_lo,
+                               (int)H, tri_gl, scale);
+        });
+    };
+    auto plain = [&](auto kern, int rows, bool pairs) {
+        return product_grid(B * H, S, rows, 256, causal, pairs, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int, int) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, blocks, wg, per_xcd, band_lo, (int)H, tri_gl,
+                               scale);
+        });
+    };
+    static_assert(P_NT == 256, "the wide kernel's workgroup");
+    bool fits = false;
+    switch (product_form(B * H, S, D, false, tri_gl > 0)) {
+    case NARROW: fits = plain(causal_pv_narrow_kernel<T, D>, N_ROWS, false); break;
+    case R64_4: fits = mid(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024); break;
+    case R64_2: fits = mid(causal_pv_mid_kernel<T, D, 4, 2>, 64, 512); break;
+    case R128_2: fits = mid(causal_pv_mid_kernel<T, D, 8, 2>, 128, 1024); break;
+    case R128_1: fits = mid(causal_pv_mid_kernel<T, D, 8, 1>, 128, 512); break;
+    default: fits = plain(causal_pv_kernel<T, D>, P_BQ, true); break;
     }
-    const int64_t per_xcd = (total_wg + 7) / 8;
-    if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
-    dim3 grid((unsigned)(per_xcd * 8));
-    if (narrow) {
-        auto kern = causal_pv_narrow_kernel<T, D>;
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb, total_wg, per_xcd,
-                           band_lo, (int)H, tri_gl, scale);
-        return launch_status();
-    }
-    // a grid of at most one workgroup per CU runs the two-group instance (key blocks split between them)
-    const bool split = pv_force() ? pv_force() == 2 : total_wg <= device_cu_count();
-    if (split) {
-        auto kern = causal_pv_kernel<T, D, 2>;
-        hipLaunchKernelGGL(kern, grid, dim3(P_NT * 2), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
-                           total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
-    } else {
-        auto kern = causal_pv_kernel<T, D, 1>;
-        hipLaunchKernelGGL(kern, grid, dim3(P_NT), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
-                           total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
-    }
-    return launch_status();
+    return fits ? launch_status() : MTA_ERR_SHAPE;
 }
 }  // namespace
 

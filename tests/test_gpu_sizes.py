@@ -457,3 +457,36 @@ def test_softmax_and_headmix_gradients(pkg, c, group, longest, dtype):
         dx, dw = dx.cpu().double(), dw.cpu().double()
         assert ((dx - want).abs() <= 2.02 * u * size + tiny)[..., keep].all()
         assert ((dw - want_w).abs() <= u * want_w.abs() + 1.01 * u * size_w + tiny * xd.abs().sum()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,s,d", [(256, 40, 64), (130, 136, 128), (520, 8, 64), (512, 40, 64), (250, 136, 128), (1030, 40, 128), (600, 136, 128), (2100, 40, 64),
+                                       (32, 1160, 128), (32, 2056, 128), (12, 2056, 64)])
+def test_products_by_grid_size(pkg, heads, s, d, dtype):
+    """P V and P^T X on the kernels that the number of row blocks chooses (64 or 128 rows, key blocks shared by one, two or four groups
+    of wavefronts): one block, edges of the 64- and 128-row blocks and of the groups' shares, NaN above the diagonal, a band
+    mask, the triangular layout.  Against the fp32 product of the same 16-bit values: one rounding of a result, and fp32 sums
+    of s products below 1 * 4 in another order."""
+    g = torch.Generator(device="cuda").manual_seed(47)
+    print(f"products heads={heads} s={s} d={d} {dtype}", flush=True)
+    p = torch.rand((1, heads, s, s), generator=g, device="cuda").to(dtype)
+    x = torch.randn((1, heads, s, d), generator=g, device="cuda").to(dtype)
+    low = torch.tril(torch.ones(s, s, dtype=torch.bool, device="cuda"))
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    some = [0, 1, heads // 2, heads - 1]
+    close = dict(rtol=ulp * 1.01, atol=s * 2.0 ** -20)
+    poisoned = p.masked_fill(~low, float("nan"))
+    o, y = pkg.ops.causal_pv(poisoned, x, True), pkg.ops.causal_ptx(poisoned, x, True)
+    full_o, full_y = pkg.ops.causal_pv(p, x, False), pkg.ops.causal_ptx(p, x, False)
+    for h in some:
+        a, b = p[0, h].float().masked_fill(~low, 0.0), x[0, h].float()
+        torch.testing.assert_close(o[0, h].float(), a @ b, **close)
+        torch.testing.assert_close(y[0, h].float(), a.t().contiguous() @ b, **close)
+        torch.testing.assert_close(full_o[0, h].float(), p[0, h].float() @ b, **close)
+        torch.testing.assert_close(full_y[0, h].float(), p[0, h].float().t().contiguous() @ b, **close)
+    if heads % 2 == 0:
+        assert torch.equal(pkg.ops.causal_pv_tri(pkg.ops.tri_pack(poisoned, 2), x, 2), o)
+    first = (torch.arange(s, device="cuda") - s // 3).clamp(min=0).int()[None]
+    keys = torch.arange(s, device="cuda")
+    banded = poisoned.masked_fill(keys[None, :] < first[0][:, None], 0.0)
+    assert torch.equal(pkg.ops.causal_pv(banded, x, True, first_visible=first), pkg.ops.causal_pv(banded, x, True))

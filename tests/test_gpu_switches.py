@@ -29,6 +29,8 @@ GROUPS = [
     # P V of small grids on the one-group kernel that large grids run (by default they split the key blocks between two
     # groups of wavefronts)
     ({"MTA_PV_SPLIT": "1"}, ["tests/test_gpu_attention.py"], "test_causal_pv"),
+    # ... and on 128-row blocks whose key blocks two groups share
+    ({"MTA_PV_SPLIT": "5"}, ["tests/test_gpu_attention.py"], "test_causal_pv"),
     # mix -> softmax -> mix for groups of 16 heads with a workgroup per row (by default workgroups take lists of rows)
     # the inference route with its score tensors as (B,H,S,S) planes (by default: the triangular layout)
     ({"MTA_SCORE_LAYOUT": "planes"}, ["tests/test_gpu_attention.py"],
