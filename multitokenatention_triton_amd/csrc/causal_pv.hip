@@ -244,8 +244,8 @@ __device__ __forceinline__ void narrow_reduce(T *a, T *b, const f32x4 (&oacc)[RB
 
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
-                                                                  int causal, int nrb, int64_t total_wg, int64_t per_xcd,
-                                                                  const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+                                                                  int causal, int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl,
+                                                                  float scale)
 {
     constexpr int CPR = D / 8, TILE = N_STEP * D, ROUNDS = TILE / 8 / 64, DB = D / 16;
     __shared__ __align__(16) T v_a_all[4 * TILE];
@@ -254,10 +254,9 @@ __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__res
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     T *const v_a = v_a_all + wave * TILE;
     T *const v_b = v_b_all + wave * TILE;
-    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (lid >= total_wg) return;
-    const int64_t bh = lid / nrb;
-    const int q0 = (nrb - 1 - (int)(lid % nrb)) * N_ROWS;   // longest rows first
+    int bh, rank;
+    if (!longest_first(heads, nrb, cus, bh, rank)) return;
+    const int q0 = (nrb - 1 - rank) * N_ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
     const T *Vp = V + bh * (int64_t)S * D;
     T *Op = O + bh * (int64_t)S * D;
@@ -368,26 +367,6 @@ __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__res
     });
 }
 
-// The workgroup's (batch, head) and its rank among that head's row blocks, longest first.  XCD x (workgroup id % 8) takes its own
-// heads (operands that row blocks share stay in one L2), hpx of them each where they divide evenly: all heads' longest blocks
-// first.  snake: the grid is resident at once, two workgroups per CU - the second half comes in reverse, so that a CU gets a
-// long block and a short one.
-__device__ __forceinline__ bool mid_item(int64_t &bh, int &rank, int nrb, int64_t total_wg, int64_t per_xcd, int hpx, int snake)
-{
-    if (hpx > 0) {
-        const int n = hpx * nrb;
-        int pos = (int)(blockIdx.x >> 3);
-        if (snake && pos >= n / 2) pos = n - 1 - (pos - n / 2);
-        bh = (int64_t)(blockIdx.x & 7) * hpx + pos % hpx;
-        rank = pos / hpx;
-        return true;
-    }
-    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    bh = lid / nrb;
-    rank = (int)(lid % nrb);
-    return lid < total_wg;
-}
-
 // The sums of GR groups of GT threads added up in the first group (true there): the upper half of the groups hand theirs to the
 // lower half through the two operand buffers, which together hold just that, until one is left.
 template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mid_sums(T *a, T *b, f32x4 (&oacc)[DB], int grp, int tid)
@@ -420,8 +399,8 @@ template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mi
 // wavefronts: the reads of P and V that one waits for fly beside the others' products.
 template <typename T, int D, int RW, int GR>
 __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1)) void causal_pv_mid_kernel(
-    const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int nrb, int64_t total_wg, int64_t per_xcd, int hpx,
-    int snake, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+    const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
+    const int *__restrict__ band_lo, int H, int tri_gl, float scale)
 {
     constexpr int CPR = D / 8, TILE = P_BK * D, GT = 64 * RW, ROUNDS = TILE / 8 / GT, DB = D / 16, ROWS = 16 * RW;
     static_assert(TILE / 8 % GT == 0 && (GT / CPR) % 16 == 0, "whole copy rounds that keep the swizzle phase");
@@ -431,9 +410,8 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     T *const v_a = v_a_all + grp * TILE;
     T *const v_b = v_b_all + grp * TILE;
-    int64_t bh;
-    int rank;
-    if (!mid_item(bh, rank, nrb, total_wg, per_xcd, hpx, snake)) return;
+    int bh, rank;
+    if (!longest_first(heads, nrb, cus, bh, rank)) return;
     const int q0 = (nrb - 1 - rank) * ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
     const T *Vp = V + bh * (int64_t)S * D;
@@ -557,7 +535,7 @@ __device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1);
 
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
-                                                                   int causal, int nkb, int64_t total_wg, int64_t per_xcd, float scale)
+                                                                   int causal, int heads, int nkb, int cus, float scale)
 {
     constexpr int XC = D / 8, XT = N_STEP * D, PCH = N_ROWS / 8, XR = XT / 8 / 64, PT = N_STEP * N_ROWS, PR = PT / 8 / 64, DB = D / 16;
     __shared__ __align__(16) T x_a_all[4 * XT];
@@ -570,10 +548,9 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
     T *const x_b = x_b_all + wave * XT;
     T *const p_a = p_a_all + wave * PT;
     T *const p_b = p_b_all + wave * PT;
-    const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (lid >= total_wg) return;
-    const int64_t bh = lid / nkb;
-    const int k0 = (int)(lid % nkb) * N_ROWS;   // under the causal rule the first keys have the most query rows
+    int bh, rank;
+    if (!longest_first(heads, nkb, cus, bh, rank)) return;
+    const int k0 = rank * N_ROWS;   // under the causal rule the first keys have the most query rows
     const T *Pp = P + bh * (int64_t)S * S;
     const T *Xp = X + bh * (int64_t)S * D;
     T *Op = O + bh * (int64_t)S * D;
@@ -672,7 +649,7 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
 // block; grid order and sums as in causal_pv_mid_kernel.
 template <typename T, int D, int RW, int GR, int PB>
 __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
-                                                                         int causal, int nkb, int64_t total_wg, int64_t per_xcd, int hpx, int snake,
+                                                                         int causal, int heads, int nkb, int cus,
                                                                          float scale)
 {
     constexpr int XC = D / 8, KB = 16 * RW, PC = KB / 8, XT = PB * D, PT = PB * KB, GT = 64 * RW, XR = XT / 8 / GT, PR = PT / 8 / GT, DB = D / 16,
@@ -688,9 +665,8 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
     T *const x_b = x_b_all + grp * XT;
     T *const p_a = p_a_all + grp * PT;
     T *const p_b = p_b_all + grp * PT;
-    int64_t bh;
-    int kb;
-    if (!mid_item(bh, kb, nkb, total_wg, per_xcd, hpx, snake)) return;
+    int bh, kb;
+    if (!longest_first(heads, nkb, cus, bh, kb)) return;
     const int k0 = kb * KB;   // (the first keys have the most query rows)
     const T *Pp = P + bh * (int64_t)S * S;
     const T *Xp = X + bh * (int64_t)S * D;
@@ -790,7 +766,8 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
 // operand (V, X) once for every block of output rows.  Larger blocks need less of it, smaller ones fill the chip: the line
 // runs by the number of 64-row blocks.  us, narrow | 64 rows, four groups | 64 rows, two groups | 128 rows, two groups | 128 rows, one
 // group | the wide kernel (P V; P^T X had pairs of 128 keys per workgroup there), rotating P tensors:
-//   P V    B2 H4 S2048 D128 (256 blocks)  18.3 | 19.3 | 21.5 | 28.8 | 32.7 | 48.0      B1 H16 S1024 D128 (256)   13.9 | 12.5 | 12.9 | 17.4 | 18.6 | 29.6
+//   P V    B2 H4 S2048 D128 (256 blocks)  15.6 | 18.8 | 21.5 | 28.8 | 32.7 | 48.0      B1 H16 S1024 D128 (256)   11.4 | 12.2 | 12.9 | 17.4 | 18.6 | 29.6
+//          B1 H12 S1536 D64 (288)         11.6 | 13.1 | 16.2 | 20.4 | 23.5 | 37.9      B1 H12 S1536 D128 (288)   16.1 | 16.1
 //          B1 H8 S3072 D128 (384)         36.2 | 33.2 | 39.2 | 50.2 | 59.4 | 72.4      B2 H16 S1008 D64 (512)    16.3 | 11.9 | 11.6 | 13.7 | 15.3 | 28.8
 //          B1 H16 S2048 D128 (512)        34.2 | 29.8 | 28.6 | 36.3 | 41.9 | 51.7      B2 H12 S2048 D128 (768)   58.4 | 53.3 | 40.7 | 45.3 | 51.4 | 55.2
 //          B1 H16 S4096 D128 (1024)       118  | 113  | 91.7 | 84.6 | 101  | 95.7      B4 H16 S1024 D128 (1024)  45.1 | 36.2 | 28.0 | 28.1 | 26.2 | 31.8
@@ -811,7 +788,7 @@ product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bo
     static const int force = [] { const char *e = getenv("MTA_PV_SPLIT"); return e ? atoi(e) : 0; }();
     if (force >= WIDE && force <= R128_1) return force == WIDE && transposed ? R128_1 : (product_kernel)force;
     const int64_t n = heads * ((S + 63) / 64);
-    if (n < 256) return NARROW;
+    if (n <= 256) return NARROW;   // (resident at once: a CU gets a long and a short block)
     if (n < 450) return R64_4;
     if (transposed) {
         if (D == 64) return n < 2048 && S > 1024 ? R64_4 : R64_2;
@@ -823,68 +800,59 @@ product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bo
     return n < 1536 && S >= 2048 ? R128_2 : R128_1;
 }
 
-// A kernel's grid: workgroups of `threads` threads, a block of `rows` output rows (WIDE: a pair of them) each; f(grid, blocks per
-// head, workgroups, workgroups per XCD, heads per XCD, snake).  False where it is too large.
-template <typename F> bool product_grid(int64_t heads, int64_t S, int rows, int threads, int causal, bool pairs, F &&f)
+// A kernel's grid: a workgroup per block of `rows` output rows, `resident` of them on a CU at once; f(grid, blocks per head, cus as
+// longest_first() takes it).  False where the grid is too large.
+template <typename F> bool product_grid(int64_t heads, int64_t S, int rows, int resident, int causal, F &&f)
 {
-    const int64_t blocks = (S + rows - 1) / rows, wg = heads * (pairs ? (blocks + 1) / 2 : blocks), per_xcd = (wg + 7) / 8;
-    if (per_xcd * 8 > 0x7fffffffLL) return false;
-    const int hpx = heads % 8 == 0 ? (int)(heads / 8) : 0;
-    f(dim3((unsigned)(per_xcd * 8)), (int)blocks, wg, per_xcd, hpx, (int)(causal && wg <= device_cu_count() * (threads == 512 ? 2 : 1)));
+    const int64_t blocks = (S + rows - 1) / rows, wg = (heads * blocks + 7) / 8 * 8;
+    if (wg > 0x7fffffffLL) return false;
+    f(dim3((unsigned)wg), (int)blocks, causal && wg <= (int64_t)resident * device_cu_count() ? device_cu_count() / 8 : 0);
     return true;
 }
 
 template <typename T, int D>
 int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, float scale, hipStream_t st)
 {
-    auto mid = [&](auto kern, int rows, int threads) {
-        return product_grid(B * H, S, rows, threads, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int hpx, int snake) {
-            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, blocks, wg, per_xcd, hpx, snake, scale);
+    auto go = [&](auto kern, int rows, int threads, int resident) {
+        const bool fits = product_grid(B * H, S, rows, resident, causal, [&](dim3 grid, int blocks, int cus) {
+            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, (int)(B * H), blocks, cus, scale);
         });
+        return fits ? launch_status() : MTA_ERR_SHAPE;
     };
-    bool fits = false;
     switch (product_form(B * H, S, D, true, false)) {
-    case NARROW:
-        fits = product_grid(B * H, S, N_ROWS, 256, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int, int) {
-            hipLaunchKernelGGL((causal_ptx_narrow_kernel<T, D>), grid, dim3(256), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, blocks, wg,
-                               per_xcd, scale);
-        });
-        break;
-    case R64_4: fits = mid(causal_ptx_mid_kernel<T, D, 4, 4, 32>, 64, 1024); break;
-    case R64_2: fits = mid(causal_ptx_mid_kernel<T, D, 4, 2, 32>, 64, 512); break;
-    case R128_2: fits = mid(causal_ptx_mid_kernel<T, D, 8, 2, 64>, 128, 1024); break;
-    default: fits = mid(causal_ptx_mid_kernel<T, D, 8, 1, 64>, 128, 512); break;
+    case NARROW: return go(causal_ptx_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 3 : 2);
+    case R64_4: return go(causal_ptx_mid_kernel<T, D, 4, 4, 32>, 64, 1024, 1);
+    case R64_2: return go(causal_ptx_mid_kernel<T, D, 4, 2, 32>, 64, 512, 2);
+    case R128_2: return go(causal_ptx_mid_kernel<T, D, 8, 2, 64>, 128, 1024, 1);
+    default: return go(causal_ptx_mid_kernel<T, D, 8, 1, 64>, 128, 512, 2);
     }
-    return fits ? launch_status() : MTA_ERR_SHAPE;
 }
 
 template <typename T, int D>
 int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st,
            const int *band_lo = nullptr, int tri_gl = 0, float scale = 1.0f)
 {
-    auto mid = [&](auto kern, int rows, int threads) {
-        return product_grid(B * H, S, rows, threads, causal, false, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int hpx, int snake) {
-            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, blocks, wg, per_xcd, hpx, snake, band_lo,
-                               (int)H, tri_gl, scale);
+    auto go = [&](auto kern, int rows, int threads, int resident) {
+        const bool fits = product_grid(B * H, S, rows, resident, causal, [&](dim3 grid, int blocks, int cus) {
+            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, (int)(B * H), blocks, cus, band_lo, (int)H,
+                               tri_gl, scale);
         });
+        return fits ? launch_status() : MTA_ERR_SHAPE;
     };
-    auto plain = [&](auto kern, int rows, bool pairs) {
-        return product_grid(B * H, S, rows, 256, causal, pairs, [&](dim3 grid, int blocks, int64_t wg, int64_t per_xcd, int, int) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, blocks, wg, per_xcd, band_lo, (int)H, tri_gl,
-                               scale);
-        });
-    };
-    static_assert(P_NT == 256, "the wide kernel's workgroup");
-    bool fits = false;
     switch (product_form(B * H, S, D, false, tri_gl > 0)) {
-    case NARROW: fits = plain(causal_pv_narrow_kernel<T, D>, N_ROWS, false); break;
-    case R64_4: fits = mid(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024); break;
-    case R64_2: fits = mid(causal_pv_mid_kernel<T, D, 4, 2>, 64, 512); break;
-    case R128_2: fits = mid(causal_pv_mid_kernel<T, D, 8, 2>, 128, 1024); break;
-    case R128_1: fits = mid(causal_pv_mid_kernel<T, D, 8, 1>, 128, 512); break;
-    default: fits = plain(causal_pv_kernel<T, D>, P_BQ, true); break;
+    case NARROW: return go(causal_pv_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 4 : 2);
+    case R64_4: return go(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024, 1);
+    case R64_2: return go(causal_pv_mid_kernel<T, D, 4, 2>, 64, 512, 2);
+    case R128_2: return go(causal_pv_mid_kernel<T, D, 8, 2>, 128, 1024, 1);
+    case R128_1: return go(causal_pv_mid_kernel<T, D, 8, 1>, 128, 512, 2);
+    default: break;
     }
-    return fits ? launch_status() : MTA_ERR_SHAPE;
+    const int nqb = (int)((S + P_BQ - 1) / P_BQ);
+    const int64_t total_wg = B * H * ((nqb + 1) / 2), per_xcd = (total_wg + 7) / 8;
+    if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
+    hipLaunchKernelGGL((causal_pv_kernel<T, D>), dim3((unsigned)(per_xcd * 8)), dim3(P_NT), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
+                       total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
+    return launch_status();
 }
 }  // namespace
 

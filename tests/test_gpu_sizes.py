@@ -490,3 +490,20 @@ def test_products_by_grid_size(pkg, heads, s, d, dtype):
     keys = torch.arange(s, device="cuda")
     banded = poisoned.masked_fill(keys[None, :] < first[0][:, None], 0.0)
     assert torch.equal(pkg.ops.causal_pv(banded, x, True, first_visible=first), pkg.ops.causal_pv(banded, x, True))
+
+
+@pytest.mark.parametrize("heads,s,d", [(288, 4, 64), (160, 68, 128), (256, 36, 64), (512, 36, 64), (260, 128, 128), (768, 36, 64), (400, 100, 128)])
+def test_fp32_products_by_grid_size(pkg, heads, s, d):
+    """P V and P^T X in fp32 on the kernels that share V (X) in LDS, which the number of row blocks chooses: one block, edges of the
+    32- and 64-row blocks and of the groups' shares, NaN above the diagonal.  Bound as in test_fp32_lower_products."""
+    lib, st = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(53)
+    print(f"fp32 products heads={heads} s={s} d={d}", flush=True)
+    p = torch.randn((1, heads, s, s), generator=g, device="cuda")
+    x = torch.randn((1, heads, s, d), generator=g, device="cuda")
+    low = torch.tril(torch.ones(s, s, dtype=torch.bool, device="cuda"))
+    pd, out = p.masked_fill(~low, float("nan")), torch.full_like(x, float("nan"))
+    lower, xd = p.double().masked_fill(~low, 0.0).cpu(), x.double().cpu()
+    for entry, left in ((lib.mta_causal_pv_f32, lower), (lib.mta_causal_ptx_f32, lower.transpose(2, 3))):
+        assert entry(pd.data_ptr(), x.data_ptr(), out.data_ptr(), 1, heads, s, d, 0.5, st) == 0
+        assert ((out.cpu().double() - 0.5 * (left @ xd)).abs() <= s ** 0.5 * 2.0 ** -22 * 0.5 * (left.abs() @ xd.abs()) + 1e-30).all()
