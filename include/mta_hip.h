@@ -371,6 +371,30 @@ int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *worksp
 int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
                               int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream);
 
+/* The partial results of a weight gradient, as the entry points named *_partials leave them in their workspace (which has to stay
+ * until they are added up): `rows` blocks of `entries` fp32 values, `parts` of each, to be added, multiplied by `scale` and stored
+ * to dw in `dtype`, block after block; side > 0: a (rows, rows) matrix with side x side blocks on its diagonal, 0 elsewhere
+ * (and, mask > 0, outside the diagonal blocks of that size). */
+typedef struct mta_partials {
+    const void *partial;
+    void *dw;
+    int32_t rows, entries, parts, side, mask, dtype;
+    float scale;
+} mta_partials;
+/* Adds up the partial results of up to MTA_MAX_SUMS gradients in one launch.  The *_partials entry points are the ones they are
+ * named after without that launch; their other arguments mean the same. */
+#define MTA_MAX_SUMS 8
+int mta_sum_partials(int count, const mta_partials *jobs, void *stream);
+int mta_conv2d_bwd_weight_partials(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
+                                   int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale,
+                                   int io_dtype, int w_dtype, mta_partials *job, void *stream);
+int mta_headmix_grads_partials(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace,
+                               int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal,
+                               int io_dtype, int w_dtype, mta_partials *job, void *stream);
+int mta_softmax_headmix_grads_partials(const void *s, const void *ds, const void *x, const void *w, void *dx, void *dw,
+                                       void *workspace, int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q,
+                                       int group_size, int causal, int io_dtype, int w_dtype, mta_partials *job, void *stream);
+
 /* mta_headmix_bwd_input and mta_headmix_bwd_weight_as in one pass over x and dy: dx and dw as those two define them (dw 0 outside
  * the groups).  Mixing groups of 2, 4, 8, 12, 16 and 32 heads, Q of whole 16-byte vectors, x, dy and dx aligned to them, 16-bit
  * data of groups of 12 and more with weights of the same dtype; MTA_ERR_UNSUPPORTED otherwise, and where

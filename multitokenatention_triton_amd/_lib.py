@@ -20,6 +20,13 @@ MTA_CAUSAL_LOWER_ONLY = 2  # `causal` of the conv / head-mixing entry points: no
 _c = ctypes
 _vp, _i64, _int, _f32 = _c.c_void_p, _c.c_int64, _c.c_int, _c.c_float
 
+
+class Partials(_c.Structure):
+    """mta_partials of include/mta_hip.h"""
+    _fields_ = [("partial", _vp), ("dw", _vp), ("rows", _c.c_int32), ("entries", _c.c_int32), ("parts", _c.c_int32), ("side", _c.c_int32),
+                ("mask", _c.c_int32), ("dtype", _c.c_int32), ("scale", _f32)]
+
+
 # name -> (restype, argtypes); one entry per declaration in include/mta_hip.h
 SIGNATURES = {
     "mta_abi_version": (_int, []),
@@ -61,6 +68,10 @@ SIGNATURES = {
     "mta_headmix_grads_workspace": (_i64, [_i64, _i64, _i64, _i64, _int, _int, _int, _int, _int]),
     "mta_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_softmax_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
+    "mta_sum_partials": (_int, [_int, _vp, _vp]),
+    "mta_conv2d_bwd_weight_partials": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _f32, _int, _int, _vp, _vp]),
+    "mta_headmix_grads_partials": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp, _vp]),
+    "mta_softmax_headmix_grads_partials": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp, _vp]),
     "mta_headmix_bwd_weight_as": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_rows_copy": (_int, [_int] + [_vp] * 7 + [_i64] * 5 + [_int, _vp]),
     "mta_causal_pv_scaled_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),

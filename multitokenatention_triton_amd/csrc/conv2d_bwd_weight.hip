@@ -374,35 +374,6 @@ __global__ __launch_bounds__(NT) void conv2d_bwd_weight_any(const T *__restrict_
     for (int tap = tid; tap < RS; tap += NT) partial[((int64_t)c * bpc + sp.sub) * RS + tap] = sums[tap];
 }
 
-// dw[c][t] = scale * sum over the channel's partial kernels, in the weight's dtype: 64 entries per workgroup, the partial
-// kernels dealt to 16 wavefronts (each adds its share in index order), the 16 sums added in wavefront order.  (A thread per
-// entry walking its 64 partial kernels alone took 11 us at 16 channels, 6x11; this takes 4.)
-constexpr int RED_SLICES = 16;
-__global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *__restrict__ partial, void *__restrict__ dw, int total,
-                                                                   int RS, int bpc, float scale, int out_dtype)
-{
-    __shared__ float red[RED_SLICES][64];
-    const int le = threadIdx.x & 63, sl = threadIdx.x >> 6;
-    const int e = blockIdx.x * 64 + le;  // (c, tap)
-    float s = 0.0f;
-    if (e < total) {
-        const float *src = partial + (int64_t)(e / RS) * bpc * RS + e % RS;
-#pragma unroll 4
-        for (int b = sl; b < bpc; b += RED_SLICES) s += src[(int64_t)b * RS];
-    }
-    red[sl][le] = s;
-    __syncthreads();
-    if (sl == 0 && e < total) {
-        float t = 0.0f;
-#pragma unroll
-        for (int k = 0; k < RED_SLICES; ++k) t += red[k][le];
-        t *= scale;
-        if (out_dtype == MTA_F32) ((float *)dw)[e] = t;
-        else if (out_dtype == MTA_BF16) ((bf16_t *)dw)[e] = from_float<bf16_t>(t);
-        else ((f16_t *)dw)[e] = from_float<f16_t>(t);
-    }
-}
-
 // workgroups per channel: enough persistent workgroups to fill the device, at most `cap` partial kernels in total
 inline int blocks_per_channel(int64_t N, int64_t C, int64_t H, int64_t W, int64_t cap)
 {
@@ -432,7 +403,7 @@ int check_args(const void *x, const void *dy, const void *dw, int64_t N, int64_t
 
 template <typename T>
 int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int64_t N, int64_t C, int64_t H, int64_t W,
-           int R, int S, int causal, float scale, int w_dtype, hipStream_t st)
+           int R, int S, int causal, float scale, int w_dtype, mta_partials *job, hipStream_t st)
 {
     const int tiles_m = (int)((H + TM - 1) / TM), tiles_n = (int)((W + TN - 1) / TN);
     const int vec_ok = (W % 8 == 0 && aligned_to(dy, 16)) ? 1 : 0;
@@ -458,7 +429,7 @@ int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int
                            (const T *)x, (const T *)dy, partial, (int)N, (int)C, (int)H, (int)W, causal, rows_m,      \
                            (int)nseg, bm);                                                                           \
         bpc = bm;                                                                                                    \
-        goto reduce;                                                                                                 \
+        goto done;                                                                                                   \
     }
             MTA_CONV_CASE(3, 3)
             MTA_CONV_CASE(3, 5)
@@ -471,7 +442,7 @@ int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int
 #undef MTA_CONV_CASE
         }
     }
-    if (launch_weight_rows<T>(x, dy, partial, bpc, N, C, H, W, R, S, causal, st)) goto reduce;
+    if (launch_weight_rows<T>(x, dy, partial, bpc, N, C, H, W, R, S, causal, st)) goto done;
     {
         const size_t lds = sizeof(float) * ((size_t)(TM + R - 1) * (TN + S) + (size_t)TM * TN + (size_t)R * S);
         auto kern = conv2d_bwd_weight_any<T>;
@@ -482,15 +453,9 @@ int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int
         hipLaunchKernelGGL(kern, grid, dim3(NT), lds, st, (const T *)x, (const T *)dy, partial, (int)N, (int)C, (int)H,
                            (int)W, R, S, causal, tiles_m, tiles_n, bpc);
     }
-reduce:
-    {
-        const int rc = launch_status();
-        if (rc != MTA_OK) return rc;
-        const int total = (int)(C * R * S);
-        hipLaunchKernelGGL(reduce_partials, dim3((unsigned)((total + 63) / 64)), dim3(64 * RED_SLICES), 0, st, partial, dw, total,
-                           R * S, bpc, scale, w_dtype);
-        return launch_status();
-    }
+done:
+    *job = {partial, dw, (int32_t)C, R * S, bpc, 0, 0, w_dtype, scale};
+    return launch_status();
 }
 
 // ---- scratch buffer of the entry point that allocates nothing -----------------------------------------------------
@@ -527,19 +492,29 @@ extern "C" int64_t mta_conv2d_bwd_weight_workspace(int64_t N, int64_t C, int64_t
     return (int64_t)blocks_per_channel(N, C, H, W, MAX_PARTIALS) * C * R * S * (int64_t)sizeof(float);
 }
 
-extern "C" int mta_conv2d_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
-                                        int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype,
-                                        int w_dtype, void *stream)
+extern "C" int mta_conv2d_bwd_weight_partials(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                                              int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype,
+                                              int w_dtype, mta_partials *job, void *stream)
 {
+    if (!job) return MTA_ERR_NULL;
     const int rc = check_args(x, dy, dw, N, C, H, W, R, S, io_dtype, w_dtype);
     if (rc != MTA_OK) return rc;
     if (!workspace) return MTA_ERR_NULL;
     if (!aligned_to(workspace, 16)) return MTA_ERR_ALIGN;
     const int bpc = blocks_per_channel(N, C, H, W, MAX_PARTIALS);
     if (workspace_bytes < (int64_t)bpc * C * R * S * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
-    MTA_DISPATCH_IO(io_dtype, return launch<io_t>(x, dy, dw, (float *)workspace, bpc, N, C, H, W, R, S, causal, scale, w_dtype,
+    MTA_DISPATCH_IO(io_dtype, return launch<io_t>(x, dy, dw, (float *)workspace, bpc, N, C, H, W, R, S, causal, scale, w_dtype, job,
                                                   (hipStream_t)stream));
     return MTA_ERR_DTYPE;
+}
+
+extern "C" int mta_conv2d_bwd_weight_as(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                                        int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype,
+                                        int w_dtype, void *stream)
+{
+    mta_partials job;
+    const int rc = mta_conv2d_bwd_weight_partials(x, dy, dw, workspace, workspace_bytes, N, C, H, W, R, S, causal, scale, io_dtype, w_dtype, &job, stream);
+    return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
 }
 
 extern "C" int mta_conv2d_bwd_weight(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,
@@ -560,7 +535,7 @@ extern "C" int mta_conv2d_bwd_weight_noalloc(const void *x, const void *dy, void
     const int bpc = blocks_per_channel(N, C, H, W, cap < MAX_PARTIALS ? cap : MAX_PARTIALS);
     float *ws = static_scratch(&rc);
     if (!ws) return rc;
-    MTA_DISPATCH_IO(io_dtype, return launch<io_t>(x, dy, dw, ws, bpc, N, C, H, W, R, S, causal, 1.0f, MTA_F32,
-                                                  (hipStream_t)stream));
-    return MTA_ERR_DTYPE;
+    mta_partials job;
+    MTA_DISPATCH_IO(io_dtype, rc = launch<io_t>(x, dy, dw, ws, bpc, N, C, H, W, R, S, causal, 1.0f, MTA_F32, &job, (hipStream_t)stream));
+    return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
 }

@@ -758,33 +758,6 @@ __global__ __launch_bounds__(512, TPW == 1 ? 4 : 2) void dense_softmax_grads(con
     }
 }
 
-// dw[o,i] = sum of the partial matrices' entries, in the weight's dtype, 0 outside the groups; `parts` matrices of G x G per
-// group.  16 entries per workgroup, the matrices dealt to 64 threads each, in a fixed order.
-constexpr int RED = 64;
-__global__ __launch_bounds__(16 * RED) void sum_partials(const float *__restrict__ partial, void *__restrict__ dw, int C, int G, int parts, int out_dtype)
-{
-    __shared__ float red[RED][17];
-    const int le = threadIdx.x & 15, sl = threadIdx.x >> 4, e = blockIdx.x * 16 + le, o = e / C, i = e % C;
-    const bool in = e < C * C && o / G == i / G;
-    float s = 0.0f;
-    if (in) {
-        const float *from = partial + (int64_t)(o / G) * parts * (G * G) + (o % G) * G + i % G;
-#pragma unroll 16
-        for (int b = sl; b < parts; b += RED) s += from[(int64_t)b * (G * G)];
-    }
-    red[sl][le] = s;
-    __syncthreads();
-    if (sl == 0 && e < C * C) {
-        float t = 0.0f;
-#pragma unroll
-        for (int k = 0; k < RED; ++k) t += red[k][le];
-        if (!in) t = 0.0f;
-        if (out_dtype == MTA_F32) ((float *)dw)[e] = t;
-        else if (out_dtype == MTA_BF16) ((bf16_t *)dw)[e] = from_float<bf16_t>(t);
-        else ((f16_t *)dw)[e] = from_float<f16_t>(t);
-    }
-}
-
 // ---- host ------------------------------------------------------------------------------------------------------------------
 // What a call is cut into: workgroups per group of heads (= partial matrices per group).  0: no kernel.
 struct cut {
@@ -839,10 +812,10 @@ int check_args(const void *a, const void *b, const void *c, const void *w, const
     return MTA_OK;
 }
 
-int add_up(const void *ws, void *dw, int64_t C, int64_t G, int64_t parts, int w_dtype, hipStream_t st)
+// `parts` matrices of G x G per group
+mta_partials job_of(const void *ws, void *dw, int64_t C, int64_t G, int64_t parts, int w_dtype)
 {
-    hipLaunchKernelGGL(sum_partials, dim3((unsigned)((C * C + 15) / 16)), dim3(16 * RED), 0, st, (const float *)ws, dw, (int)C, (int)G, (int)parts, w_dtype);
-    return launch_status();
+    return {ws, dw, (int32_t)C, (int32_t)(G * G), (int32_t)parts, (int32_t)G, 0, w_dtype, 1.0f};
 }
 
 template <typename T>
@@ -905,9 +878,11 @@ extern "C" int64_t mta_headmix_grads_workspace(int64_t N, int64_t C, int64_t P, 
     return (with_softmax ? N : 1) * (C / G) * c.parts * G * G * (int64_t)sizeof(float);
 }
 
-extern "C" int mta_headmix_grads(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
-                                 int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream)
+extern "C" int mta_headmix_grads_partials(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes,
+                                          int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype,
+                                          mta_partials *job, void *stream)
 {
+    if (!job) return MTA_ERR_NULL;
     const int rc = check_args(x, dy, x, w, dx, dw, workspace, N, C, P, Q, group_size, io_dtype, w_dtype);
     if (rc != MTA_OK) return rc;
     causal = causal == MTA_CAUSAL_LOWER_ONLY ? 2 : causal ? 1 : 0;
@@ -917,14 +892,23 @@ extern "C" int mta_headmix_grads(const void *x, const void *dy, const void *w, v
     if (workspace_bytes < C / G * c.parts * G * G * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
     MTA_DISPATCH_IO(io_dtype, launch_grads<io_t>(x, dy, w, dx, workspace, c, N, C, P, Q, G, causal, w_dtype, w_dtype == io_dtype, st));
-    const int rl = launch_status();
-    return rl != MTA_OK ? rl : add_up(workspace, dw, C, G, c.parts, w_dtype, st);
+    *job = job_of(workspace, dw, C, G, c.parts, w_dtype);
+    return launch_status();
 }
 
-extern "C" int mta_softmax_headmix_grads(const void *s, const void *ds, const void *x, const void *w, void *dx, void *dw, void *workspace,
-                                         int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype,
-                                         int w_dtype, void *stream)
+extern "C" int mta_headmix_grads(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                                 int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype, int w_dtype, void *stream)
 {
+    mta_partials job;
+    const int rc = mta_headmix_grads_partials(x, dy, w, dx, dw, workspace, workspace_bytes, N, C, P, Q, group_size, causal, io_dtype, w_dtype, &job, stream);
+    return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
+}
+
+extern "C" int mta_softmax_headmix_grads_partials(const void *s, const void *ds, const void *x, const void *w, void *dx, void *dw, void *workspace,
+                                                  int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal,
+                                                  int io_dtype, int w_dtype, mta_partials *job, void *stream)
+{
+    if (!job) return MTA_ERR_NULL;
     const int rc = check_args(s, ds, x, w, dx, dw, workspace, N, C, P, Q, group_size, io_dtype, w_dtype);
     if (rc != MTA_OK) return rc;
     causal = causal ? 1 : 0;
@@ -937,6 +921,16 @@ extern "C" int mta_softmax_headmix_grads(const void *s, const void *ds, const vo
     hipError_t attr = hipSuccess;
     MTA_DISPATCH_IO(io_dtype, attr = launch_softmax_grads<io_t>(s, ds, x, w, dx, workspace, c, N, C, P, Q, G, causal, w_dtype, w_dtype == io_dtype, st));
     if (attr != hipSuccess) return (int)attr;
-    const int rl = launch_status();
-    return rl != MTA_OK ? rl : add_up(workspace, dw, C, G, N * c.parts, w_dtype, st);
+    *job = job_of(workspace, dw, C, G, N * c.parts, w_dtype);
+    return launch_status();
+}
+
+extern "C" int mta_softmax_headmix_grads(const void *s, const void *ds, const void *x, const void *w, void *dx, void *dw, void *workspace,
+                                         int64_t workspace_bytes, int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int io_dtype,
+                                         int w_dtype, void *stream)
+{
+    mta_partials job;
+    const int rc = mta_softmax_headmix_grads_partials(s, ds, x, w, dx, dw, workspace, workspace_bytes, N, C, P, Q, group_size, causal, io_dtype, w_dtype, &job,
+                                                      stream);
+    return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
 }

@@ -266,34 +266,6 @@ __global__ __launch_bounds__(NT) void headmix_bwd_weight_any(const T *__restrict
     for (int pair = tid; pair < CC; pair += NT) partial[(int64_t)blockIdx.x * CC + pair] = sums[pair];
 }
 
-// dw[e] = sum of the partial matrices' entries e, in the weight's dtype (group > 0: 0 outside the diagonal blocks), in a fixed order: 64 entries per workgroup, the partial matrices dealt
-// to 16 wavefronts (each adds its share in index order), the 16 sums added in wavefront order
-constexpr int RED_SLICES = 16;
-__global__ __launch_bounds__(64 * RED_SLICES) void reduce_partials(const float *__restrict__ partial,
-                                                                   void *__restrict__ dw, int CC, int nparts, int C, int group,
-                                                                   int out_dtype)
-{
-    __shared__ float red[RED_SLICES][64];
-    const int le = threadIdx.x & 63, sl = threadIdx.x >> 6;
-    const int e = blockIdx.x * 64 + le;
-    float s = 0.0f;
-    if (e < CC) {
-#pragma unroll 8
-        for (int b = sl; b < nparts; b += RED_SLICES) s += partial[(int64_t)b * CC + e];
-    }
-    red[sl][le] = s;
-    __syncthreads();
-    if (sl == 0 && e < CC) {
-        float t = 0.0f;
-#pragma unroll
-        for (int k = 0; k < RED_SLICES; ++k) t += red[k][le];
-        if (group > 0 && e / C / group != e % C / group) t = 0.0f;
-        if (out_dtype == MTA_F32) ((float *)dw)[e] = t;
-        else if (out_dtype == MTA_BF16) ((bf16_t *)dw)[e] = from_float<bf16_t>(t);
-        else ((f16_t *)dw)[e] = from_float<f16_t>(t);
-    }
-}
-
 constexpr int64_t MAX_WS_BYTES = 8 << 20;  // partial matrices never take more than this
 
 // Persistent workgroups (= partial matrices) for a problem, at most.  Matrix-core kernels: one per CU, which has 64 to 128 KB
@@ -370,10 +342,8 @@ extern "C" int mta_headmix_bwd_weight_as(const void *x, const void *dy, void *dw
         rc = launch_partials<io_t>((const io_t *)x, (const io_t *)dy, partial, nb, (int)N, (int)C, (int)P, (int)Q, causal, st);
     });
     if (rc != MTA_OK) return rc;
-    const int CC = (int)(C * C);
-    hipLaunchKernelGGL(reduce_partials, dim3((unsigned)((CC + 63) / 64)), dim3(64 * RED_SLICES), 0, st, partial, dw, CC, nb, (int)C,
-                       group_size, w_dtype);
-    return launch_status();
+    const mta_partials job{partial, dw, (int32_t)C, (int32_t)(C * C), nb, (int32_t)C, group_size, w_dtype, 1.0f};
+    return mta_sum_partials(1, &job, stream);
 }
 
 extern "C" int mta_headmix_bwd_weight(const void *x, const void *dy, void *dw, void *workspace, int64_t workspace_bytes,

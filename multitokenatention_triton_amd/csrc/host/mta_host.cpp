@@ -402,10 +402,10 @@ Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, con
 // The gradients of a head mixing with respect to its input and its weight (those that are wanted).  One kernel where it is both;
 // small: also for one of them, which costs nothing there and gives the bits that it has beside the other.
 std::pair<Tensor, Tensor> headmix_bwd(const Tensor &dy, const Tensor &x, const Tensor &w, bool causal, int64_t group, bool fill_upper, bool need_x,
-                                      bool need_w, bool small)
+                                      bool need_w, bool small, Sums &sums)
 {
     if ((need_x && need_w) || (small && (need_x || need_w))) {
-        if (auto both = headmix_grads(std::nullopt, dy, x, w, causal, group, fill_upper))
+        if (auto both = headmix_grads(std::nullopt, dy, x, w, causal, group, fill_upper, sums))
             return {need_x ? both->first : Tensor(), need_w ? both->second : Tensor()};
     }
     return {need_x ? headmix_bwd_input(dy, w, causal, group, fill_upper) : Tensor(),
@@ -414,14 +414,14 @@ std::pair<Tensor, Tensor> headmix_bwd(const Tensor &dy, const Tensor &x, const T
 
 // the gradients of q, k, conv_w and w_pre (need[i]: wanted) from the one of the probabilities p
 void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, Tensor raw, const Tensor &x, const Tensor &p,
-                       const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4])
+                       const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4], Sums &sums)
 {
     const double scale = score_scale(q);
     // (the head mixing's gradient kernels never read above the diagonal when causal)
     Tensor dx;
     const bool need_x = need[0] || need[1] || need[2];
     // (one kernel for the three gradients, also where one of them is for nobody: it reads less than the two that it takes otherwise)
-    const auto all = causal == pre_causal ? headmix_grads(p, dp, x, w_pre, causal, pre_group, !causal) : std::nullopt;
+    const auto all = causal == pre_causal ? headmix_grads(p, dp, x, w_pre, causal, pre_group, !causal, sums) : std::nullopt;
     if (all) {
         dp.reset();
         if (need[3]) *out[3] = all->second;
@@ -463,7 +463,7 @@ void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, c
             TORCH_CHECK(lower_raw || !first);
             raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
         }
-        *out[2] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale);
+        *out[2] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale, sums);
     }
 }
 
@@ -570,22 +570,24 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
         for (int i = 0; i < 7; ++i) need[i] = ctx->needs_input_grad(i);
         const bool need_x = need[0] || need[1] || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
         variable_list out(11);
+        Sums sums;
         const Tensor go = value_rows(grads[0], s_pad);
         if (need[2]) out[2] = values_bwd_v(m, go, lower);
         if (need_c || need[6]) {
             Tensor dm = values_bwd_m(go, v, lower, first);
             if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
             Tensor dc;
-            std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], true);
+            std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], true, sums);
             dm.reset();
-            if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0);
+            if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0, sums);
             if (need_p) {
                 Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, !causal);
                 dc.reset();
                 probabilities_bwd(q, k, conv_w, w_pre, raw, x, p, first, causal, pre_causal, pre_group, std::move(dp), {need[0], need[1], need[3], need[4]},
-                                  {&out[0], &out[1], &out[3], &out[4]});
+                                  {&out[0], &out[1], &out[3], &out[4]}, sums);
             }
         }
+        sums.run();
         // the gradients of Q, K and V leave without the padding and without what the hidden keys' rows hold
         RowsCopy rows(s_real, key_bias);
         for (int i = 0; i < 3; ++i)
@@ -649,10 +651,12 @@ struct Probabilities : torch::autograd::Function<Probabilities> {
         const auto s = ctx->get_saved_variables();
         const c10::OptionalDeviceGuard guard(s[0].device());
         variable_list out(6);
+        Sums sums;
         probabilities_bwd(s[0], s[1], s[2], s[3], s[4], s[5], s[6], option(s[7]), ctx->saved_data["causal"].toBool(),
                           ctx->saved_data["pre_causal"].toBool(), ctx->saved_data["pre_group"].toInt(), grads[0].to(s[6].scalar_type()),
                           {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)},
-                          {&out[0], &out[1], &out[2], &out[3]});
+                          {&out[0], &out[1], &out[2], &out[3]}, sums);
+        sums.run();
         return out;
     }
 };
@@ -676,7 +680,9 @@ struct Conv2d : torch::autograd::Function<Conv2d> {
         torch::autograd::variable_list out(5);
         const Tensor dy = on_gpu(grads[0], "grad_output");
         if (ctx->needs_input_grad(0)) out[0] = conv2d_bwd_input(dy, saved[1], causal, ctx->saved_data["grad_fill_upper"].toBool());
-        if (ctx->needs_input_grad(1)) out[1] = conv2d_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, 1.0);
+        Sums sums;
+        if (ctx->needs_input_grad(1)) out[1] = conv2d_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, 1.0, sums);
+        sums.run();
         return out;
     }
 };
@@ -701,8 +707,10 @@ struct HeadMix : torch::autograd::Function<HeadMix> {
         const int64_t group = ctx->saved_data["group"].toInt();
         torch::autograd::variable_list out(7);
         const Tensor dy = on_gpu(grads[0], "grad_output");
+        Sums sums;
         std::tie(out[0], out[1]) = headmix_bwd(dy, saved[0], saved[1], causal, group, ctx->saved_data["grad_fill_upper"].toBool(),
-                                               ctx->needs_input_grad(0), ctx->needs_input_grad(1), false);
+                                               ctx->needs_input_grad(0), ctx->needs_input_grad(1), false, sums);
+        sums.run();
         return out;
     }
 };

@@ -102,8 +102,33 @@ inline Tensor conv2d_bwd_input(const Tensor &dy_, const Tensor &w_, bool causal,
     return dx;
 }
 
-// the gradient of a (C,R,S) kernel, times `scale`, in the dtype of `like`
-inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tensor &like, bool causal, double scale)
+// Weight gradients whose partial results one launch adds up (run(); until then the gradients hold nothing).  Keeps the workspaces
+// that far; all on the stream of the first one.
+struct Sums {
+    // the entry of a gradient about to be computed into dw by way of ws
+    mta_partials *add(const Tensor &dw, const Tensor &ws)
+    {
+        if (count == MTA_MAX_SUMS) run();
+        kept[count] = {dw, ws};
+        if (count == 0) stream = stream_of(ws);
+        return &jobs[count++];
+    }
+    void drop() { kept[--count] = {}; }   // ... and was not, after all
+    void run()
+    {
+        check(mta_sum_partials(count, jobs, stream), "mta_sum_partials");
+        while (count) drop();
+    }
+
+  private:
+    mta_partials jobs[MTA_MAX_SUMS];
+    std::pair<Tensor, Tensor> kept[MTA_MAX_SUMS];
+    int count = 0;
+    void *stream = nullptr;
+};
+
+// the gradient of a (C,R,S) kernel, times `scale`, in the dtype of `like` (in `sums`)
+inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tensor &like, bool causal, double scale, Sums &sums)
 {
     const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output");
     TORCH_CHECK_VALUE(x.sizes() == dy.sizes() && x.scalar_type() == dy.scalar_type(), "input and grad_output must share shape and dtype");
@@ -112,8 +137,8 @@ inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tenso
     Tensor dw = at::empty({c, r, s}, like.options());
     const int64_t bytes = std::max<int64_t>(mta_conv2d_bwd_weight_workspace(n, c, h, w, r, s), 16);
     Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
-    check(mta_conv2d_bwd_weight_as(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, h, w, r, s, causal, (float)scale, code(x, "input"),
-                                   code(like, "weight"), stream_of(x)),
+    check(mta_conv2d_bwd_weight_partials(ptr(x), ptr(dy), out_ptr(dw), out_ptr(ws), bytes, n, c, h, w, r, s, causal, (float)scale, code(x, "input"),
+                                         code(like, "weight"), sums.add(dw, ws), stream_of(x)),
           "mta_conv2d_bwd_weight");
     return dw;
 }
@@ -158,9 +183,9 @@ inline Tensor headmix_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tens
 }
 
 // The gradients of the head mixing with respect to its input and its weight in one pass; with `probs`, dy is the gradient of the
-// softmax behind it (of the probabilities `probs`).  Nothing where there is no kernel.
+// softmax behind it (of the probabilities `probs`).  Nothing where there is no kernel.  (dw: in `sums`)
 inline std::optional<std::pair<Tensor, Tensor>> headmix_grads(const OptTensor &probs_, const Tensor &dy_, const Tensor &x_, const Tensor &w_, bool causal,
-                                                              int64_t group, bool fill_upper)
+                                                              int64_t group, bool fill_upper, Sums &sums)
 {
     if (dy_.dim() != 4 || dy_.scalar_type() != x_.scalar_type() || dy_.sizes() != x_.sizes()) return std::nullopt;
     const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
@@ -172,11 +197,15 @@ inline std::optional<std::pair<Tensor, Tensor>> headmix_grads(const OptTensor &p
     const int64_t bytes = mta_headmix_grads_workspace(n, c, p, q, (int)group, mode, probs.has_value(), ic, wc);
     if (bytes <= 0) return std::nullopt;
     Tensor dx = at::empty(x.sizes(), x.options()), dw = at::empty(w.sizes(), w.options()), ws = at::empty({bytes}, x.options().dtype(at::kByte));
-    const int rc = probs ? mta_softmax_headmix_grads(ptr(probs), ptr(dy), ptr(x), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q,
-                                                     (int)group, causal, ic, wc, stream_of(x))
-                         : mta_headmix_grads(ptr(x), ptr(dy), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, (int)group, mode, ic, wc,
-                                             stream_of(x));
-    if (rc == MTA_ERR_UNSUPPORTED) return std::nullopt;
+    mta_partials *job = sums.add(dw, ws);
+    const int rc = probs ? mta_softmax_headmix_grads_partials(ptr(probs), ptr(dy), ptr(x), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q,
+                                                              (int)group, causal, ic, wc, job, stream_of(x))
+                         : mta_headmix_grads_partials(ptr(x), ptr(dy), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, p, q, (int)group, mode,
+                                                      ic, wc, job, stream_of(x));
+    if (rc == MTA_ERR_UNSUPPORTED) {
+        sums.drop();
+        return std::nullopt;
+    }
     check(rc, "mta_headmix_grads");
     return std::make_pair(dx, dw);
 }

@@ -55,6 +55,15 @@ def test_argument_validation_needs_no_gpu():
     assert lib.mta_conv_attn_fwd(p, p, p, p, None, 1, 1, 8, 64, 3, 3, 1, 0.1, 0, 0, None) == -1
     # dtype
     assert lib.mta_conv2d_fwd(p, p, p, 1, 1, 8, 8, 3, 3, 1, 7, 0, None) == -2
+    # sums: how many, of what
+    one = _lib.Partials(p, p, 2, 4, 1, 2, 0, 0, 1.0)
+    assert lib.mta_sum_partials(0, None, None) == 0
+    assert lib.mta_sum_partials(9, ctypes.byref(one), None) == -3
+    assert lib.mta_sum_partials(1, None, None) == -1
+    for field, value, code in (("dw", None, -1), ("dtype", 7, -2), ("rows", 3, -3), ("entries", 5, -3), ("parts", 0, -3)):
+        bad = _lib.Partials(p, p, 2, 4, 1, 2, 0, 0, 1.0)
+        setattr(bad, field, value)
+        assert lib.mta_sum_partials(1, ctypes.byref(bad), None) == code
     # shape
     assert lib.mta_conv2d_fwd(p, p, p, 0, 1, 8, 8, 3, 3, 1, 0, 0, None) == -3
     # softmax gradient: null pointer, dtype, shape

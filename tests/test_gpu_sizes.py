@@ -425,6 +425,37 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("count", [1, 3, 8])
+def test_sums_of_partial_results(pkg, count, dtype):
+    """Several gradients' partial results in one launch: one block per channel (conv kernels), one per group on the diagonal, a whole
+    matrix cut to its groups; numbers of entries and of partial results about 16 and 64.  Against float64: an fp32 sum of n values in
+    any order is within n * 2^-24 of the sum of magnitudes, one rounding to the dtype."""
+    lib, code = pkg._lib.load(), {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    g = torch.Generator().manual_seed(47)
+    kinds = [(3, 15, 1, 0, 0), (2, 66, 63, 0, 0), (8, 4, 130, 2, 0), (16, 256, 65, 16, 4), (1, 1, 64, 0, 0), (5, 17, 2, 0, 0), (6, 36, 1, 6, 0), (12, 9, 1000, 3, 0)]
+    jobs, want = (pkg._lib.Partials * count)(), []
+    for i, (rows, entries, parts, side, mask) in enumerate(kinds[:count]):
+        blocks = rows // side if side else rows
+        data = torch.randn(blocks, parts, entries, generator=g)
+        scale = 0.5 if side == 0 else 1.0
+        sums, sizes = data.double().sum(1) * scale, data.double().abs().sum(1) * scale
+        if side:
+            sums, sizes = (torch.block_diag(*t.view(blocks, side, side)) for t in (sums, sizes))
+            if mask:
+                sums, sizes = (t * torch.block_diag(*[torch.ones(mask, mask)] * (rows // mask)) for t in (sums, sizes))
+        dw = torch.full((sums.numel() + 8,), 7.0, dtype=dtype, device="cuda")
+        kept = data.cuda()
+        jobs[i] = pkg._lib.Partials(kept.data_ptr(), dw.data_ptr(), rows, entries, parts, side, mask, code, scale)
+        want.append((kept, dw, sums.flatten(), sizes.flatten(), parts))
+    assert lib.mta_sum_partials(count, jobs, torch.cuda.current_stream().cuda_stream) == 0
+    half_step = 2.0 ** -25 if dtype == torch.float16 else 0.0   # (rounding of a subnormal result)
+    for _, dw, sums, sizes, parts in want:
+        got = dw.cpu().double()
+        assert (got[sums.numel():] == 7.0).all()
+        assert ((got[:sums.numel()] - sums).abs() <= _unit(dtype) * 1.01 * sums.abs() + parts * 2.0 ** -24 * sizes + half_step).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("c,group,longest", [(2, 0, 4096), (4, 0, 4096), (8, 0, 4096), (12, 0, 4096), (16, 0, 4096), (32, 0, 2048), (8, 4, 4096), (32, 16, 4096)])
 def test_softmax_and_headmix_gradients(pkg, c, group, longest, dtype):
     """Softmax gradient, mixing and weight gradient in one pass: rows of one wavefront and of several, of one tile per wavefront and
