@@ -149,51 +149,58 @@ int launch_valu(const void *x, const void *w, void *y, int64_t N, int64_t C, int
 // the input rows that neighbouring strips re-read (halos) in the L2.
 #define MTA_CONV_STORE(ptr, val) store_out((ptr), (val), STREAM)
 
-constexpr int M_NW = 4;            // wavefronts per workgroup: (16-row block, 128-key half) of the workgroup's strip each
+constexpr int M_NW = 4;            // wavefronts per workgroup, each with 16 rows x 128 keys of the workgroup's strip
 constexpr int M_WT = 64 * M_NW;    // threads per workgroup
-constexpr int M_TM = 32;           // strip rows
-constexpr int M_TN = 256;          // strip cols: two halves of 8 column blocks of 16
-constexpr int M_HALF = M_TN / 2;   // keys per wavefront
-constexpr int M_RPB = M_TN / M_TM;  // row strips per M_TN x M_TN block of the lower triangle
-// persistent workgroups per CU: four where two strip buffers take a quarter of the LDS (kernels of up to 6 rows: 37 staged
-// rows of 544 bytes are 1258 slots, five copy rounds, 20 KB), else three; kernels of more than 7 rows keep that many more
-// Toeplitz fragments in registers and are compiled for two
-template <int R> constexpr int wg_per_cu() { return R > 7 ? 2 : (R > 6 ? 3 : 4); }
-static_assert(M_NW == 4 && M_TM == 32 && M_TN % M_TM == 0 && M_RPB % 2 == 0, "strip geometry");
+constexpr int M_HALF = 128;        // keys per wavefront: 8 column blocks of 16
+// A strip: 64 rows x 128 keys (NARROW) or 32 x 256; which one, see narrow_strips()
+template <bool NARROW> struct strip_geom {
+    static constexpr int TM = NARROW ? 64 : 32, TN = NARROW ? 128 : 256;
+    static constexpr int RB = TM / 16;     // row blocks of 16
+    static constexpr int RPB = TN / TM;    // row strips per TN x TN block of the lower triangle
+    static_assert(RB * (TN / M_HALF) == M_NW, "a wavefront for each 16 x 128 outputs");
+};
+// Persistent workgroups per CU: four, as long as two strip buffers take a quarter of the LDS (five copy rounds, 20 KB) and a
+// wavefront 128 registers; three for wide strips of more than 6 kernel rows, and for more than 7.  They are what hides the latency:
+// the kernel of 6 x 11 over the lower triangle of B1 H16 S2048 fp16 took 41.6, 39.9, 33.7 us with two, three, four (from cache).
+template <int R, bool NARROW> constexpr int wg_per_cu() { return R > (NARROW ? 7 : 6) ? 3 : 4; }
 
 // 16 outputs + S-1 taps (+ alignment shift) must fit the 32-key contraction of one 16x16x32 MFMA
-template <int R, int S> struct mfma_geom {
+template <int R, int S, bool NARROW> struct mfma_geom : strip_geom<NARROW> {
+    using strip_geom<NARROW>::TM;
+    using strip_geom<NARROW>::TN;
     static constexpr int PADW = (S - 1) / 2;
     static constexpr int HL = (PADW + 7) & ~7;             // left halo, rounded so 16-byte loads stay aligned
     static constexpr int SHIFT = HL - PADW;                // first tap's offset inside a block's 32-key window
     static constexpr bool fits = SHIFT + 16 + S - 1 <= 32;
-    static constexpr int TW = M_TN - 16 + 32;              // staged columns
+    static constexpr int TW = TN - 16 + 32;                // staged columns
     // Row stride in LDS.  A fragment read takes 16 bytes per lane from 16 consecutive rows (lane group kg at byte offset
     // 16 kg); the LDS serves lanes 0-7 together with lanes 24-31 (8-15 with 16-23, ...), i.e. rows 0-7 at one offset with
     // rows 8-15 at the next: with a stride of 2 (mod 8) 16-byte slots those sixteen accesses fall on sixteen different
-    // slots of the 256-byte bank line (3 (mod 8), one padding slot after the 34 of data, put rows 3 and 8 on the same one).
+    // slots of the 256-byte bank line (3 (mod 8), one padding slot after the data, put rows 3 and 8 on the same one).
     static constexpr int LD = TW;
     static_assert((LD / 8) % 8 == 2, "row stride of the staged strip");
-    static constexpr int ROWS = M_TM + R - 1;
-    // results of the wavefronts that own key half `h` go back to LDS columns h * RES_OFF .. + M_HALF - 1, which no
-    // wavefront of the other half reads as input (half 0 reads columns 0 .. M_HALF+15, half 1 columns M_HALF ..)
+    static constexpr int ROWS = TM + R - 1;
+    // Where a wavefront's results wait in LDS.  NARROW: in its own row block, once every wavefront has read its input.  Else the
+    // results of key half `h` go back to LDS columns h * RES_OFF .. + M_HALF - 1 of rows that the other row block does not read,
+    // which no wavefront of the other half reads as input (half 0 reads columns 0 .. M_HALF+15, half 1 columns M_HALF ..).
     static constexpr int RES_OFF = M_HALF + 16;
-    static_assert(RES_OFF + M_HALF <= LD, "result columns of the second half");
+    static_assert(NARROW || RES_OFF + M_HALF <= LD, "result columns of the second half");
 };
 
-// Position t of a work item inside its plane -> (strip row tm (M_TM rows), strip col tn (M_TN keys)).
+// Position t of a work item inside its plane -> (strip row tm (TM rows), strip col tn (TN keys)).
 // `tri` (causal, square, lower triangle only): the strips that touch the lower triangle, row strip by row strip from
-// the top, each from the left up to the diagonal: row strip tm has tm / M_RPB + 1 of them, so M_RPB/2 * b * (b+1) items
+// the top, each from the left up to the diagonal: row strip tm has tm / RPB + 1 of them, so RPB/2 * b * (b+1) items
 // precede block row b.  Otherwise: all strips, row-major.
-__device__ __forceinline__ void decode_item(int t, int tiles_n, int tri, int &tm, int &tn)
+template <bool NARROW> __device__ __forceinline__ void decode_item(int t, int tiles_n, int tri, int &tm, int &tn)
 {
     if (tri) {
-        constexpr int HB = M_RPB / 2;
+        constexpr int RPB = strip_geom<NARROW>::RPB, HB = RPB / 2;
+        static_assert(RPB % 2 == 0, "row strips per block row");
         int b = (int)((sqrtf((float)t / (float)HB + 0.25f) - 0.5f));
         while (HB * (b + 1) * (b + 2) <= t) ++b;
         while (HB * b * (b + 1) > t) --b;
         const int rem = t - HB * b * (b + 1);
-        tm = b * M_RPB + rem / (b + 1);
+        tm = b * RPB + rem / (b + 1);
         tn = rem % (b + 1);
     } else {
         tm = t / tiles_n;
@@ -201,11 +208,12 @@ __device__ __forceinline__ void decode_item(int t, int tiles_n, int tri, int &tm
     }
 }
 
-// +0 over an M_TM x M_TN region, all threads of the workgroup.  FULL: the region lies inside the tensor; the stores are
-// then unconditional (exactly M_TM*M_TN/8/M_WT vector-memory instructions per lane)
-template <typename T, bool STREAM, bool FULL = false>
+// +0 over a TM x TN region (of strips that write whole rows), all threads of the workgroup.  FULL: the region lies inside the tensor; the stores are
+// then unconditional (exactly TM*TN/8/M_WT vector-memory instructions per lane)
+template <typename T, bool NARROW, bool STREAM, bool FULL = false>
 __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int q0, int tid)
 {
+    constexpr int M_TM = strip_geom<NARROW>::TM, M_TN = strip_geom<NARROW>::TN;
     constexpr int VEC = 8, VPRW = M_TN / VEC, RPP = M_WT / VPRW;  // vectors per row, rows per pass
     pack16<T> z;
 #pragma unroll
@@ -225,18 +233,17 @@ __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int
 }
 
 // Persistent four-wavefront workgroups: each walks a run of M_TM x M_TN strips dealt round-robin within its XCD's share
-// of the item list.  Wavefront w owns row block w & 1 (16 rows) and key half w >> 1 (128 keys) of the strip: it issues a
-// quarter of the staging copies and computes its 16 x 128 outputs.  The wavefronts meet at two barriers per strip (the
-// strip has landed and the previous strip's buffer may be overwritten; the results are in LDS); latency is hidden by the
-// other workgroups resident on the CU, each in its own phase (loading / matrix cores / storing) with its own two LDS
-// strip buffers of (M_TM + R - 1) rows x 272 keys.
+// of the item list.  A wavefront owns a row block of 16 rows and 128 keys of the strip: it issues a quarter of the staging
+// copies and computes its 16 x 128 outputs.  The wavefronts meet at two barriers per strip (the strip has landed and the
+// previous strip's buffer may be overwritten; the strip is no longer needed as input, or the results are in LDS); latency is
+// hidden by the other workgroups resident on the CU, each in its own phase (loading / matrix cores / storing) with its own
+// two LDS strip buffers of (M_TM + R - 1) rows x (M_TN + 16) keys.
 //
 // Item order.  Strips are taken row strip by row strip, each from the left, so that an XCD's workgroups sweep whole
 // rows of the output together, zero strips included: under the causal rule a strip wholly above the diagonal is an
 // item like the others, whose workgroup stores +0 over it (no copy, no products).  Written this way - every row of the
-// output completed within a short time, 512 contiguous bytes per row and strip - the tensor moves through memory a tenth
-// faster than with 32 x 128 strips taken block by block and the part above the diagonal filled by workgroups of their
-// own.  Odd planes are walked backwards, so that a workgroup's share alternates between the cheap strips above the
+// output completed within a short time - the tensor moves through memory a tenth faster than with strips taken block by
+// block and the part above the diagonal filled by workgroups of their own.  Odd planes are walked backwards, so that a workgroup's share alternates between the cheap strips above the
 // diagonal and the others.  MTA_CAUSAL_LOWER_ONLY on a square tensor enumerates the strips that touch the lower
 // triangle only.
 //
@@ -245,13 +252,14 @@ __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int
 // Toeplitz fragment (4 VGPRs per kernel row, kept while the channel is unchanged), B operand = 16 contiguous
 // bytes of one staged row per lane.  A wavefront sustains about one such 1 KB LDS operand per 35 cycles whatever the
 // addresses, against 16 cycles for the product: the products of a strip are therefore split over four wavefronts (on
-// four SIMDs).  Results go back through LDS rows that are no longer needed as input (row block 0: the strip's first 16
-// staged rows; row block 1: the last 16 staged rows of its window; see mfma_geom::RES_OFF for the columns); after a
+// four SIMDs).  Results go back through LDS rows that are no longer needed as input.  NARROW: after a barrier a wavefront
+// writes its row block's own 16 rows and stores them, four 256-byte rows per instruction.  Else row block 0 takes the
+// strip's first 16 staged rows, row block 1 the last 16 of its window (see mfma_geom::RES_OFF for the columns); after a
 // barrier wavefront w stores strip rows 8w .. 8w+7 whole, two 512-byte rows per instruction.
 //
 // Staging.  A strip whose halo lies wholly inside the tensor and on or below the diagonal (the common case, decided per
 // workgroup) is copied global -> LDS by global_load_lds_dwordx4: no registers, no masks, no LDS store instructions.
-// The LDS row stride is 34 16-byte slots (see mfma_geom::LD), and thread t of copy round `it` owns slot it*256+t.  Any
+// The LDS row stride is 34 or 18 16-byte slots (see mfma_geom::LD), and thread t of copy round `it` owns slot it*256+t.  Any
 // other strip is copied slot by slot under a predicate - a slot inside the plane and on or below the diagonal is
 // copied, any other is written as zeros while the buffer waits for its data - and after landing only the one vector
 // per row that straddles the diagonal is masked in LDS.  Nothing is read from outside the tensor.
@@ -266,18 +274,19 @@ __device__ __forceinline__ void zero_fill_strip(T *yp, int H, int W, int p0, int
 //
 // BWD: the gradient with respect to the input (see conv2d_valu): kernel rows reversed in both axes, the R-1 halo rows
 // below the strip instead of above it.  Key sizes are odd here, so the key halos are the same on both sides.
-template <typename T, int R, int S, bool SCALED, bool BWD, bool STREAM>
-__global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
+template <typename T, int R, int S, bool SCALED, bool BWD, bool STREAM, bool NARROW>
+__global__ __launch_bounds__(M_WT, (wg_per_cu<R, NARROW>())) void conv2d_mfma(
     const T *__restrict__ x, const T *__restrict__ w, T *__restrict__ y, int C, int H, int W, int causal, float in_scale,
     int tiles_n, int ipp, int64_t total, int64_t per_xcd, int nw, int tri)
 {
-    using G = mfma_geom<R, S>;
+    using G = mfma_geom<R, S, NARROW>;
+    constexpr int M_TM = G::TM, M_TN = G::TN;
     static_assert(!BWD || (S % 2 == 1 && !SCALED), "the backward instance assumes symmetric key halos and no scale");
     static_assert(sizeof(T) == 2, "16-bit data");
     constexpr int TOP = BWD ? 0 : R - 1;                    // halo rows above the strip (the others lie below it)
     constexpr int LD = G::LD, VEC = 8;
-    constexpr int VPR = G::TW / VEC;                        // data vectors per staged row (34)
-    constexpr int SPR = LD / VEC;                           // 16-byte slots per LDS row (35)
+    constexpr int VPR = G::TW / VEC;                        // data vectors per staged row (34 or 18)
+    constexpr int SPR = LD / VEC;                           // 16-byte slots per LDS row
     constexpr int SLOTS = G::ROWS * SPR;
     constexpr int STAGE_IT = (SLOTS + M_WT - 1) / M_WT;     // copies per strip and lane (the last round may be partial)
     static_assert(SPR == VPR, "no padding slots");
@@ -307,8 +316,8 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
     const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     // (the wavefront index through readfirstlane: everything derived from it is then scalar)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rb0 = (wave & 1) * 16;         // first strip row of this wavefront's row block
-    const int ch = wave >> 1;                // its key half
+    const int rb0 = (wave % G::RB) * 16;     // first strip row of this wavefront's row block
+    const int ch = wave / G::RB;             // its key half
     frag8<T> tz[R];
     int cur_channel = -1;
     const bool reflect = causal != 0 && !tri;  // odd planes backwards
@@ -395,14 +404,14 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
         podd_nx = (int)(plane0 & 1);
     }
     int tm, tn;
-    decode_item((reflect && podd_nx) ? ipp - 1 - t_nx : t_nx, tiles_n, tri, tm, tn);
+    decode_item<NARROW>((reflect && podd_nx) ? ipp - 1 - t_nx : t_nx, tiles_n, tri, tm, tn);
     if (kind_of(tm * M_TM, tn * M_TN) == 0) {
         fetch_weights(chan_nx, 0);
         if (!SCALED) prefetch(pbase_nx, tm * M_TM, tn * M_TN, tiles, is_interior(tm * M_TM, tn * M_TN));
     }
 
     constexpr int ST = 16 * (M_HALF / VEC) / 64;  // stores per strip and lane (a wavefront's 16 x 128 outputs) ...
-    static_assert(ST == M_TM * (M_TN / VEC) / M_WT, "... and per zero strip");
+    static_assert(ST == M_TM * (M_TN / VEC) / M_WT && ST == 4, "... and per zero strip");
     int younger = -1;                      // stores certainly issued after the copy in flight (-1: unknown)
     int parity = 0;
     for (int item = 0; item < n_items; ++item, parity ^= 1) {
@@ -532,7 +541,7 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
                 chan_nx = chan_nx + 1 == C ? 0 : chan_nx + 1;
                 podd_nx ^= 1;
             }
-            decode_item((reflect && podd_nx) ? ipp - 1 - t_nx : t_nx, tiles_n, tri, tm, tn);
+            decode_item<NARROW>((reflect && podd_nx) ? ipp - 1 - t_nx : t_nx, tiles_n, tri, tm, tn);
             if (kind_of(tm * M_TM, tn * M_TN) == 0) {
                 fetch_weights(chan_nx, parity ^ 1);  // (before the copy: the loop-top wait counts what is younger than the copy)
                 if (!SCALED) prefetch(pbase_nx, tm * M_TM, tn * M_TN, other, is_interior(tm * M_TM, tn * M_TN));
@@ -541,10 +550,10 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
         if (kind != 0) {
             if (kind == 1) {
                 if (full_out) {
-                    zero_fill_strip<T, STREAM, true>(yp, H, W, p0, q0, tid);
+                    zero_fill_strip<T, NARROW, STREAM, true>(yp, H, W, p0, q0, tid);
                     younger = ST;
                 } else {
-                    zero_fill_strip<T, STREAM>(yp, H, W, p0, q0, tid);
+                    zero_fill_strip<T, NARROW, STREAM>(yp, H, W, p0, q0, tid);
                     younger = -1;
                 }
             }
@@ -553,7 +562,7 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
 
         // ---- this wavefront's 16 x 128 outputs: 8 column blocks of 16x16 on 16x16x32 MFMAs (one per kernel row: the
         // 32-key window holds the 16 outputs' taps).  Lane (row ln, group kg) holds keys 4*kg..4*kg+3 of each block.
-        const int res0 = rb0 == 0 ? 0 : rb0 + R - 1;                 // staged rows that receive the results
+        const int res0 = NARROW || rb0 == 0 ? rb0 : rb0 + R - 1;        // staged rows that receive the results
         const int qw = q0 + ch * M_HALF;                             // first key of this wavefront's outputs
         {
             constexpr int NCB = M_HALF / 16;
@@ -565,8 +574,9 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
             // into a ring of registers, and a product waits only for its own operand (LDS operations complete in order:
             // exactly the reads issued after it may be outstanding).  Source order is pinned (the scheduler would regroup
             // reads and products).  Blocks above the diagonal are computed like the others and masked below.
-            // (operands in flight: 12, or 6 where four workgroups per CU leave a wavefront 128 registers)
-            constexpr int NLD_MAX = wg_per_cu<R>() >= 4 ? 6 : 12;
+            // (operands in flight: 6, or 4 beside the fragments of 7 rows, where four workgroups per CU leave a wavefront 128
+            // registers; 12 where three do, 9 beside the fragments of 11 rows)
+            constexpr int NLD_MAX = wg_per_cu<R, NARROW>() < 4 ? (R > 7 ? 9 : 12) : (R > 6 ? 4 : 6);
             constexpr int NPROD = NCB * R, NLD = 2 * R < NLD_MAX ? 2 * R : NLD_MAX, NSLOT = NLD + 1;
             static_assert(NLD <= 15 && NPROD > NLD, "lgkmcnt field; pipeline deeper than the work");
             u32x4 ring[NSLOT];
@@ -587,7 +597,9 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
                 mma16(acc[cb], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
                 __builtin_amdgcn_sched_barrier(0);
             });
-            // results into the staged rows res0.. (read by this wavefront only, and no longer needed by it)
+            // results into the staged rows res0.. (NARROW: once every wavefront has read what it needs of them; else read by this
+            // wavefront only, and no longer needed by it)
+            if (NARROW) wg_barrier();
             const int prow = p0 + rb0 + ln;
             const unsigned ra = tile_lds + (unsigned)((res0 + ln) * LD + ch * G::RES_OFF + kg * 4) * sizeof(T);
 #pragma unroll
@@ -603,25 +615,26 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
                 lds_store8_at(ra, (int)(cb * 16 * sizeof(T)), lo, hi);
             }
         }
-        // ---- coalesced stores.  The four wavefronts' results lie in LDS; after a barrier wavefront w stores rows 8w .. 8w+7
-        // of the strip in full, two 512-byte rows per instruction (the halves of a row come from two wavefronts' results):
-        // whole rows in one instruction move a few percent faster through memory than 256-byte pieces of four rows ----
+        // ---- coalesced stores.  NARROW: a wavefront stores the 16 rows that it computed, four 256-byte pieces of rows per
+        // instruction.  Else, after a barrier, wavefront w stores rows 8w .. 8w+7 of the strip in full, two 512-byte rows per
+        // instruction (the halves of a row come from two wavefronts' results): whole rows in one instruction move a few percent
+        // faster through memory ----
         lds_wait();
-        wg_barrier();
+        if (!NARROW) wg_barrier();
         {
             // (uniform row base + one 32-bit per-lane byte offset: no 64-bit address arithmetic per store)
-            const int sr0 = wave * 8;                                   // first strip row this wavefront stores
-            const int sres = sr0 < 16 ? sr0 : sr0 + R - 1;              // ... and where its results lie (see res0)
+            const int sr0 = NARROW ? rb0 : wave * 8;                       // first strip row this wavefront stores
+            const int sres = NARROW || sr0 < 16 ? sr0 : sr0 + R - 1;       // ... and where its results lie (see res0)
+            constexpr int RPS = NARROW ? 4 : 2;                            // rows per instruction
             char *ybase = reinterpret_cast<char *>(yp + (int64_t)(p0 + sr0) * W + q0);
             const int lane_o = opaque(lane);  // (row offsets formed here, not kept in registers across the loop)
-            const int r_l = lane_o >> 5, hf = (lane_o >> 4) & 1, cv = (lane_o & 15) * VEC;
+            const int r_l = NARROW ? lane_o >> 4 : lane_o >> 5, hf = NARROW ? 0 : (lane_o >> 4) & 1, cv = (lane_o & 15) * VEC;
             const unsigned yoff = (unsigned)(r_l * W + hf * M_HALF + cv) * (unsigned)sizeof(T);
-            const int64_t ystep = (int64_t)2 * W * (int64_t)sizeof(T);
-            static_assert(ST == 4, "four row pairs per wavefront");
+            const int64_t ystep = (int64_t)RPS * W * (int64_t)sizeof(T);
             u32x4 v[4];
             const unsigned va = tile_lds + (unsigned)((sres + r_l) * LD + hf * G::RES_OFF + cv) * sizeof(T);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = lds_load16_at(va, (int)(k * 2 * LD * sizeof(T)));
+            for (int k = 0; k < 4; ++k) v[k] = lds_load16_at(va, (int)(k * RPS * LD * sizeof(T)));
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : : "memory");
             if (full_out) {  // unconditional: exactly ST vector-memory instructions
 #pragma unroll
@@ -629,7 +642,7 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const int r = k * 2 + r_l;
+                    const int r = k * RPS + r_l;
                     if (p0 + sr0 + r < H && q0 + hf * M_HALF + cv < W) MTA_CONV_STORE(reinterpret_cast<u32x4 *>(ybase + k * ystep + yoff), v[k]);
                 }
             }
@@ -638,23 +651,23 @@ __global__ __launch_bounds__(M_WT, wg_per_cu<R>()) void conv2d_mfma(
     }
 }
 
-template <typename T, int R, int S, bool BWD>
+template <typename T, int R, int S, bool BWD, bool NARROW>
 int launch_mfma(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int causal,
                 float in_scale, int use_scale, hipStream_t st)
 {
-    const int64_t tiles_m = (H + M_TM - 1) / M_TM, tiles_n = (W + M_TN - 1) / M_TN;
+    using G = strip_geom<NARROW>;
+    const int64_t tiles_m = (H + G::TM - 1) / G::TM, tiles_n = (W + G::TN - 1) / G::TN;
     // causal, square, and the caller wants nothing written above the diagonal: only the strips that touch the lower triangle
     const int tri = (causal == 2 && H == W) ? 1 : 0;
-    const int64_t nbf = tiles_m / M_RPB, kl = tiles_m % M_RPB;
-    const int64_t ipp64 = tri ? (M_RPB / 2) * nbf * (nbf + 1) + kl * (nbf + 1) : tiles_m * tiles_n;
+    const int64_t nbf = tiles_m / G::RPB, kl = tiles_m % G::RPB;
+    const int64_t ipp64 = tri ? G::RPB * nbf * (nbf + 1) / 2 + kl * (nbf + 1) : tiles_m * tiles_n;
     if (ipp64 > (1 << 24)) return MTA_ERR_SHAPE;  // decode_item's float sqrt is exact well beyond this
     const int ipp = (int)ipp64;
     const int64_t total = N * C * ipp64;
     const int64_t per_xcd = (total + 7) / 8;
     // persistent workgroups per XCD: as many as fit when only the strips of the lower triangle are walked; with the zero
     // strips in the list three per CU move the tensor fastest (measured at (2,16,2048,2048): 84 us against 85.5 with four)
-    const int wgs = tri ? wg_per_cu<R>() : (wg_per_cu<R>() < 3 ? wg_per_cu<R>() : 3);
-    int nw = device_cu_count() * wgs / 8;
+    int nw = device_cu_count() * (tri ? wg_per_cu<R, NARROW>() : 3) / 8;
     if (nw < 1) nw = 1;
     if (per_xcd < nw) nw = (int)per_xcd;
     dim3 grid((unsigned)(nw * 8));
@@ -664,13 +677,30 @@ int launch_mfma(const void *x, const void *w, void *y, int64_t N, int64_t C, int
     };
     const bool stream = streams(N, C, H, W, sizeof(T));
     if constexpr (BWD) {
-        go(stream ? conv2d_mfma<T, R, S, false, true, true> : conv2d_mfma<T, R, S, false, true, false>);
+        go(stream ? conv2d_mfma<T, R, S, false, true, true, NARROW> : conv2d_mfma<T, R, S, false, true, false, NARROW>);
     } else if (use_scale) {
-        go(stream ? conv2d_mfma<T, R, S, true, false, true> : conv2d_mfma<T, R, S, true, false, false>);
+        go(stream ? conv2d_mfma<T, R, S, true, false, true, NARROW> : conv2d_mfma<T, R, S, true, false, false, NARROW>);
     } else {
-        go(stream ? conv2d_mfma<T, R, S, false, false, true> : conv2d_mfma<T, R, S, false, false, false>);
+        go(stream ? conv2d_mfma<T, R, S, false, false, true, NARROW> : conv2d_mfma<T, R, S, false, false, false, NARROW>);
     }
     return launch_status();
+}
+
+// 64 x 128 strips of 7 kernel rows need a quarter of the LDS (32 x 256 ones a little more: three workgroups per CU, not four), and
+// they cover the triangle with less beside it; but their rows are written in pieces of 256 bytes, not 512, which costs where whole
+// rows are written and where the stores are non-temporal.  32 x 256 | 64 x 128, us, bf16, nothing in the caches:
+//   only the lower triangle   B1 H16 S1024  B1 H16 S2048  B2 H16 S2048  B4 H16 S2048  B1 H8 S4096  B1 H16 S4096
+//     3x3                       14.8 | 14.1   40.4 | 37.9     62 | 65      120 | 128    58.3 | 60.3   110 | 111
+//     6x11                      15.6 | 15.2   41.2 | 39.4     67 | 67      130 | 132    60.3 | 62.0   113 | 116
+//     7x7                       18.6 | 15.8   46.3 | 39.9     83 | 68      160 | 134    65.5 | 62.7   119 | 118
+//     11x15 (two per CU)        22.5 | 20.4   54   | 45.7    104 | 82      195 | 156    81.8 | 74.5   155 | 139
+//   whole rows
+//     6x11                      18.6 | 17.5   50.9 | 52.3     84 | 95      159 | 175     102 | 106    154 | 173
+//     7x7                       19.8 | 17.8   51.5 | 52.3     84 | 95      161 | 176     105 | 106    155 | 173
+//     11x15 (two per CU)        24   | 21     56   | 54      102 | 96      193 | 179     129 | 117    181 | 175
+inline bool narrow_strips(int64_t N, int64_t C, int64_t H, int64_t W, int causal, int R)
+{
+    return R > 7 || (causal == 2 && H == W && (R > 6 || !streams(N, C, H, W, 2)));
 }
 
 // returns 1 when no MFMA instantiation covers (R,S) -- the caller then takes the VALU path
@@ -681,8 +711,14 @@ int dispatch_mfma(const void *x, const void *w, void *y, int64_t N, int64_t C, i
     if constexpr (sizeof(T) != 2) return 1;
     else {
 #define MTA_CONV_CASE(r, s)                                       \
-    static_assert(mfma_geom<r, s>::fits, "window exceeds 32 keys"); \
-    if (R == r && S == s) return launch_mfma<T, r, s, BWD>(x, w, y, N, C, H, W, causal, in_scale, use_scale, st);
+    static_assert(mfma_geom<r, s, true>::fits, "window exceeds 32 keys");                                                  \
+    if (R == r && S == s) {                                                                                                \
+        if constexpr (r <= 7) {                                                                                            \
+            if (!narrow_strips(N, C, H, W, causal, r))                                                                       \
+                return launch_mfma<T, r, s, BWD, false>(x, w, y, N, C, H, W, causal, in_scale, use_scale, st);             \
+        }                                                                                                                  \
+        return launch_mfma<T, r, s, BWD, true>(x, w, y, N, C, H, W, causal, in_scale, use_scale, st);                      \
+    }
     MTA_CONV_CASE(3, 3)
     MTA_CONV_CASE(3, 5)
     MTA_CONV_CASE(5, 5)

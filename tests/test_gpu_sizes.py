@@ -424,6 +424,45 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
         assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,k", [(3, 3), (6, 11), (7, 7), (7, 9), (11, 15)])
+def test_conv_of_the_lower_triangle_by_strips(pkg, r, k, dtype):
+    """The conv and its input gradient on the lower triangle only, at edges of the 64 x 128 strips and of the planes, NaN above the
+    diagonal; and with every output written, where 11 rows take the same strips.  Against float64: an fp32 sum of at most r*k exact
+    products, one rounding to the dtype."""
+    import torch.nn.functional as F
+    g, pad = torch.Generator().manual_seed(53), (k - 1) // 2
+    half_step = 2.0 ** -25 if dtype == torch.float16 else 0.0   # (rounding of a subnormal result)
+    for n, c, s in ((1, 1, 8), (2, 3, 56), (1, 2, 64), (3, 2, 72), (1, 3, 128), (2, 2, 136), (1, 2, 192), (1, 1, 264), (2, 3, 328)):
+        print(f"conv of the lower triangle {r}x{k} {n}x{c}x{s} {dtype}", flush=True)
+        keep = torch.tril(torch.ones(s, s, dtype=torch.bool))
+        x, w = torch.randn(n, c, s, s, generator=g).to(dtype), torch.randn(c, r, k, generator=g).to(dtype)
+        xd, wd = x.double().masked_fill(~keep, 0.0), w.double()[:, None]
+        fwd = lambda t, u: F.conv2d(F.pad(t, (pad, pad, r - 1, 0)), u, groups=c)  # noqa: E731
+        bwd = lambda t, u: F.conv2d(F.pad(t, (pad, pad, 0, r - 1)), u.flip(2, 3), groups=c)  # noqa: E731
+        dirty = x.masked_fill(~keep, float("nan")).cuda()
+        for op, ref in ((pkg.ops.conv2d_causal, fwd), (pkg.ops.conv2d_bwd_input, bwd)):
+            want, size = ref(xd, wd), ref(xd.abs(), wd.abs())
+            for fill in (False, True):
+                got = op(dirty, w.cuda(), True, fill_upper=fill).cpu().double()
+                bad = (got - want).abs() > _unit(dtype) * 1.01 * want.abs() + r * k * 2.0 ** -24 * size + half_step
+                assert not bad[..., keep].any()
+                if fill:
+                    assert (got[..., ~keep] == 0.0).all()
+
+
+@pytest.mark.parametrize("r,k", [(3, 3), (6, 11)])
+def test_conv_strips_of_large_and_of_small_tensors_agree(pkg, r, k):
+    """A tensor beyond 128 MB takes 32 x 256 strips on its lower triangle, its parts 64 x 128: the same sums in the same order."""
+    x = torch.randn(2, 4, 2944, 2944, device="cuda").to(torch.bfloat16)
+    w = torch.randn(4, r, k, device="cuda").to(torch.bfloat16)
+    assert x.numel() * 2 > 128 << 20 >= x[:1].numel() * 2
+    for op in (pkg.ops.conv2d_causal, pkg.ops.conv2d_bwd_input):
+        whole = op(x, w, True, fill_upper=False).tril()
+        for i in range(2):
+            assert torch.equal(whole[i:i + 1], op(x[i:i + 1], w, True, fill_upper=False).tril())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("count", [1, 3, 8])
 def test_sums_of_partial_results(pkg, count, dtype):
