@@ -154,6 +154,8 @@ int mta_headmix_softmax_band_fwd(const void *x, const void *w1, const void *w2, 
 /* Longest row that the entry points above take in one pass over memory for fp32 scores in dense groups of `group_size`
  * heads (rows of whole 16-byte vectors, 16-byte aligned tensors); 0: no such kernel for this group size. */
 int64_t mta_headmix_softmax_dense_f32_keys(int group_size);
+/* ... and 16-bit scores with weights of the same dtype (and Q % 8 == 0). */
+int64_t mta_headmix_softmax_dense16_keys(int group_size);
 
 /* Depthwise causal conv followed by head mixing, the conv result never written:
  *   t[h] = round(conv2d(x[h], w_conv[h]))                     as mta_conv2d_fwd

@@ -51,6 +51,7 @@ SIGNATURES = {
     "mta_qk_conv_band_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _f32, _int, _int, _int, _vp]),
     "mta_headmix_softmax_band_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _int, _vp]),
     "mta_headmix_softmax_dense_f32_keys": (_i64, [_int]),
+    "mta_headmix_softmax_dense16_keys": (_i64, [_int]),
     "mta_conv2d_tril_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_headmix_tril_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp]),
     "mta_softmax_bwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp]),

@@ -18,7 +18,7 @@ namespace mta_host {
 namespace {
 
 // largest mixing group the one-pass mix/softmax/mix kernel keeps in registers, and what its matrix-core variant takes
-constexpr int64_t FUSED_MAX_GROUP = 8, FUSED_MFMA_GROUP = 16, FUSED_MFMA_MAX_KEYS = 4096;
+constexpr int64_t FUSED_MAX_GROUP = 8, FUSED_MFMA_GROUP = 16;
 
 bool no_row_lists()
 {
@@ -32,14 +32,14 @@ bool one_pass_group(int64_t group, at::ScalarType t, int64_t n_keys, const OptTe
     if (group <= FUSED_MAX_GROUP) return true;
     if (w1 && w2 && w1->scalar_type() != w2->scalar_type()) return false;   // (one kernel takes its two weights in one dtype)
     if (t == at::kFloat) return n_keys % 4 == 0 && n_keys <= mta_headmix_softmax_dense_f32_keys((int)std::min<int64_t>(group, 1 << 20));
-    return group == FUSED_MFMA_GROUP && (t == at::kBFloat16 || t == at::kHalf) && n_keys % 8 == 0 && n_keys <= FUSED_MFMA_MAX_KEYS &&
+    return (t == at::kBFloat16 || t == at::kHalf) && n_keys % 8 == 0 && n_keys <= mta_headmix_softmax_dense16_keys((int)std::min<int64_t>(group, 1 << 20)) &&
            (!w1 || w1->scalar_type() == t) && (!w2 || w2->scalar_type() == t);
 }
 
 // the 16-bit matrix-core variant for groups of 16 takes a key bias or a band mask in its row-list form only
 bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 {
-    return !masked || group <= FUSED_MAX_GROUP || t == at::kFloat || (group == FUSED_MFMA_GROUP && !no_row_lists());
+    return !masked || group != FUSED_MFMA_GROUP || t == at::kFloat || !no_row_lists();
 }
 
 // Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
@@ -384,8 +384,9 @@ Tensor probabilities(const Tensor &q, const Tensor &k, const Tensor &conv_w, con
     const int64_t heads = w_pre.size(0), n_keys = k.size(-2), g_eff = o.pre_group ? o.pre_group : heads;
     const auto dtype = x.scalar_type();
     Tensor p;
-    // (fp32 groups of more than 8 heads: with the head weight's own causal rule apart from the module's the mixing stays alone)
-    if ((dtype != at::kFloat || g_eff <= FUSED_MAX_GROUP || o.pre_causal == o.causal) && one_pass_group(g_eff, dtype, n_keys, w_pre, OptTensor()) &&
+    // (groups of more than 8 heads, but for 16 in 16 bits: with the head weight's own causal rule apart from the module's the mixing
+    // stays alone)
+    if ((g_eff <= FUSED_MAX_GROUP || (dtype != at::kFloat && g_eff == FUSED_MFMA_GROUP) || o.pre_causal == o.causal) && one_pass_group(g_eff, dtype, n_keys, w_pre, OptTensor()) &&
         masks_ok(g_eff, dtype, o.key_bias || o.first)) {
         mark("mix_softmax");
         p = headmix_softmax(x, w_pre, OptTensor(), o.causal, o.pre_group, fill, o.key_bias, o.first);

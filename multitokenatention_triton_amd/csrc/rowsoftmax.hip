@@ -23,6 +23,9 @@ namespace mta {
 int mix16_softmax_launch(const void *x, const void *w1, const void *w2, void *y, int64_t N, int64_t C, int64_t P, int64_t Q,
                          int causal, int fill_upper, int io_dtype, int w_dtype, hipStream_t st, int tri_in = 0, int tri_out = 0,
                          const float *key_bias = nullptr, const int *row_lo = nullptr);
+// rowsoftmax_dense32.hip: the same pass for 16-bit data and groups of 9 to 32 heads
+int mix_softmax_dense_launch(const void *x, const void *w1, const void *w2, const float *kb, const int *row_lo, void *y, int64_t N,
+                             int64_t C, int64_t P, int64_t Q, int HG, int causal, int io_dtype, int w_dtype, int fill_upper, hipStream_t st);
 // rowsoftmax_dense_f32.hip: the same pass for fp32 and groups of 9 to 32 heads
 int mix_softmax_dense_f32_launch(const float *x, const void *w1, const void *w2, const float *kb, const int *row_lo, float *y, int64_t N,
                                  int64_t C, int64_t P, int64_t Q, int HG, int causal, int w_dtype, int fill_upper, hipStream_t st);
@@ -952,6 +955,10 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
             if (rc != MTA_ERR_UNSUPPORTED) return rc;
         }
         if (tri_in != tri_out) return MTA_ERR_UNSUPPORTED;
+        if (!tri_in && !no_packed) {
+            const int rc = mix_softmax_dense_launch(x, w1, w2, kb_in, row_lo, y, N, C, P, Q, G, causal, io_code, w_dtype, fill_upper, st);
+            if (rc != MTA_ERR_UNSUPPORTED) return rc;
+        }
         const bool packed_ok = vec_ok && !no_packed && w_dtype == io_code && (w1 || w2) && (!w1 || aligned_to(w1, 4)) &&
                                (!w2 || aligned_to(w2, 4)) && C % 2 == 0 && Q <= 256 * VEC * 4;
         // key bias without a band mask: the packed kernel's KBIAS instances, one per group size (the one for the longest

@@ -425,6 +425,55 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,group", [(9, 0), (12, 0), (24, 12), (17, 0), (24, 0), (32, 0), (64, 32)])
+def test_mix_softmax_of_dense_groups(pkg, c, group, dtype):
+    """16-bit groups of 9 to 32 heads in one pass: rows about a tile of 128 keys, of one and several wavefronts and passes, the longest
+    row; one and two weights; a key bias; a band mask (rows that start inside a tile, behind one, behind all attended keys); NaN above
+    the diagonal.  Against float64 with the stages' roundings: a mixed score that rounds to its neighbour, 2u|s| away, moves every
+    probability of the row by as much, twice (numerator and sum)."""
+    g = torch.Generator().manual_seed(59)
+    u, hg = _unit(dtype), group or c
+    half_step = 2.0 ** -25 if dtype == torch.float16 else 0.0   # (rounding of a subnormal result)
+    block = torch.arange(c) // hg
+    same = block[:, None] == block[None, :]
+    longest = 4096 if hg <= 16 else 2048
+    for n, p, q, causal, two, bias, band in ((2, 8, 8, True, False, False, False), (1, 136, 136, True, True, False, False), (2, 130, 136, True, False, True, False),
+                                             (1, 264, 264, True, True, False, True), (1, 520, 520, True, False, True, True), (2, 3, 264, False, True, True, False),
+                                             (1, 3, 1032, False, False, False, False), (1, 2, longest - 8, False, True, False, False), (1, 2, longest, False, False, True, False)):
+        print(f"mix + softmax of dense groups c={c} group={group} {n}x{p}x{q} causal={causal} two={two} bias={bias} band={band} {dtype}", flush=True)
+        keep = torch.tril(torch.ones(p, q, dtype=torch.bool)) if causal else torch.ones(p, q, dtype=torch.bool)
+        x = torch.randn(n, c, p, q, generator=g).to(dtype)
+        w1, w2 = ((torch.eye(c) + 0.2 * torch.randn(c, c, generator=g)).to(dtype) for _ in range(2))
+        kb = torch.where(torch.rand(n, q, generator=g) < 0.2, float("-inf"), 0.25) if bias else None
+        if bias:
+            kb[:, 0] = 0.0
+        first = None
+        if band:   # (the last row sees nothing)
+            first = torch.clamp(torch.arange(p) - q // 3, min=0).int().repeat(n, 1)
+            first[:, -1] = p
+        s = torch.einsum("oi,nipq->nopq", w1.double() * same, x.double()).to(dtype)
+        if bias:
+            s = (s.float() + kb[:, None, None, :]).to(dtype)
+        seen = keep[None, None].expand(n, 1, p, q)
+        if band:
+            seen = seen & (torch.arange(q)[None, None, None, :] >= first[:, None, :, None])
+        s = s.double().masked_fill(~seen, float("-inf"))
+        off = 4 * u * s.masked_fill(s.isinf(), 0.0).abs().amax(-1, keepdim=True)
+        want = torch.softmax(s, -1)
+        size = want
+        if two:
+            want = torch.einsum("oi,nipq->nopq", w2.double() * same, want.to(dtype).double())
+            size = torch.einsum("oi,nipq->nopq", w2.double().abs() * same, size)
+        got = pkg.ops.headmix_softmax(x.masked_fill(~keep, float("nan")).cuda(), w1.masked_fill(~same, float("inf")).cuda(),
+                                      w2.masked_fill(~same, float("inf")).cuda() if two else None, causal, group_size=group or None, fill_upper=causal,
+                                      key_bias=kb.cuda() if bias else None, first_visible=first.cuda() if band else None).cpu().double()
+        rows = p - 1 if band else p
+        assert ((got - want).abs() <= (off + 3 * u) * size + half_step * (hg + 1))[..., :rows, :].all()
+        if causal:
+            assert (got[..., ~keep] == 0.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("r,k", [(3, 3), (6, 11), (7, 7), (7, 9), (11, 15)])
 def test_conv_of_the_lower_triangle_by_strips(pkg, r, k, dtype):
     """The conv and its input gradient on the lower triangle only, at edges of the 64 x 128 strips and of the planes, NaN above the
