@@ -1,4 +1,5 @@
-// Depthwise causal conv, then dense mixing of a group of 16 heads, in one pass, both on the matrix cores (16-bit data):
+// Depthwise causal conv, then mixing of 16 heads - one dense group, or groups of 2 or 4 of them - in one pass, the conv and the dense
+// mixing on the matrix cores (16-bit data):
 //
 //   c[n,h,p,q] = round( sum_{i<R,j<S} wc[h,i,j] * xm[n,h,p+i-(R-1), q+j-(S-1)/2] )      (xm: x, 0 where q > p)
 //   y[n,o,p,q] = sum_h wm[o,h] * c[n,h,p,q]                                            (0 where q > p)
@@ -22,6 +23,7 @@
 // contraction of v_mfma_f32_16x16x16 wants the heads spread over the lane groups instead.  Two exchanges between rows
 // of lanes (v_permlane32_swap, v_permlane16_swap) transpose (head quad) x (key quad): afterwards lane group g holds heads
 // 4g .. 4g+3 for all 16 keys of the block, and per key one product with the 16 x 16 weight gives the lane 4 output heads.
+// Groups of 2 or 4 heads lie within a lane then: packed dot products over the group's heads only, so that a NaN stays in its group.
 // The outputs go through LDS (swizzled, 16 KB, one output head of every lane group per round) so that the global
 // stores are whole 128-byte rows.
 #include "common.hpp"
@@ -31,6 +33,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -71,6 +74,14 @@ __device__ __forceinline__ f32x4 xm_mma16(bf16_t, xm_u2 a, xm_u2 b)
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(xm_s4, a), __builtin_bit_cast(xm_s4, b),
                                                      f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
+__device__ __forceinline__ float xm_dot2(bf16_t, unsigned a, unsigned b, float c)
+{
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(mta_bf16x2, a), __builtin_bit_cast(mta_bf16x2, b), c, false);
+}
+__device__ __forceinline__ float xm_dot2(f16_t, unsigned a, unsigned b, float c)
+{
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(mta_f16x2, a), __builtin_bit_cast(mta_f16x2, b), c, false);
+}
 __device__ __forceinline__ f32x4 xm_mma16(f16_t, xm_u2 a, xm_u2 b)
 {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(xm_h4, a), __builtin_bit_cast(xm_h4, b),
@@ -105,7 +116,7 @@ constexpr int X_ROT = 19;  // by how many workgroups the dealing of an XCD's ite
 
 template <int R> constexpr int x_occ() { return 2; }  // persistent workgroups per CU
 
-template <typename T, int R, int S>
+template <typename T, int R, int S, int GROUP>
 __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__restrict__ x, const T *__restrict__ wc,
                                                                    const T *__restrict__ wm, T *__restrict__ y, int C, int H,
                                                                    int W, int causal, int fill_upper, int tiles_n, int ipp,
@@ -277,7 +288,8 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
     bool pre_issued = false;  // the first NBUF-1 windows of `cur` were put in flight during the previous item
     int prev_st = 0;          // stores this wavefront issued at the end of the previous item (-1: unknown)
     int cur_g = -1;
-    xm_u2 wf = {0u, 0u};
+    constexpr int NWF = GROUP == X_HG ? 1 : 4;
+    xm_u2 wf[NWF] = {};
 
     for (int item = 0; item < n_items; ++item) {
         const bool has_next = item + 1 < n_items;
@@ -310,9 +322,15 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
         if (c_g != cur_g) {
             cur_g = c_g;
             build_table(cur_g);
-            // weight fragment of the mixing: lane (output head ln, group kg) holds wm[o][4kg .. 4kg+3]
-            wf = *reinterpret_cast<const xm_u2 *>(wm + (int64_t)(cur_g * X_HG + ln) * C + cur_g * X_HG + kg * 4);
-            asm volatile("s_waitcnt vmcnt(0)" : "+v"(wf) : : "memory");  // (rare: everything in flight is waited for here)
+            // weight fragment of the mixing: lane (output head ln, group kg) holds wm[o][4kg .. 4kg+3]; of groups within a lane: wm[4kg+v]
+            // [4kg .. 4kg+3], what lies outside the groups unused
+#pragma unroll
+            for (int v = 0; v < NWF; ++v) {
+                const int o = GROUP == X_HG ? ln : kg * 4 + v;
+                wf[v] = *reinterpret_cast<const xm_u2 *>(wm + (int64_t)(cur_g * X_HG + o) * C + cur_g * X_HG + kg * 4);
+            }
+#pragma unroll
+            for (int v = 0; v < NWF; ++v) asm volatile("s_waitcnt vmcnt(0)" : "+v"(wf[v]) : : "memory");  // (rare: everything in flight is waited for here)
             prev_st = -1;
         }
         const int h0 = p0 - TOP, k0 = q0 - G::HL;
@@ -456,7 +474,15 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
                 const unsigned sel = (t & 1) ? 0x07060302u : 0x05040100u;
                 const xm_u2 col = {__builtin_amdgcn_perm(cres[4 * kq + 1][cb][part], cres[4 * kq + 0][cb][part], sel),
                                    __builtin_amdgcn_perm(cres[4 * kq + 3][cb][part], cres[4 * kq + 2][cb][part], sel)};
-                macc[j] = xm_mma16(T{}, wf, col);
+                if constexpr (GROUP == X_HG) {
+                    macc[j] = xm_mma16(T{}, wf[0], col);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        if constexpr (GROUP == 4) macc[j][v] = xm_dot2(T{}, wf[v][1], col[1], xm_dot2(T{}, wf[v][0], col[0], 0.0f));
+                        else macc[j][v] = xm_dot2(T{}, wf[v][v / 2], col[v / 2], 0.0f);
+                    }
+                }
             }
             const int qb = q0 + kh * X_HALF + cb * 16;
 #pragma unroll
@@ -578,7 +604,7 @@ xm_split make_split(int64_t npg, int64_t tiles_m, int64_t tiles_n, int causal, i
     return sp;
 }
 
-template <typename T, int R, int S>
+template <typename T, int R, int S, int GROUP>
 int launch_x(const void *x, const void *wc, const void *wm, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int causal,
              int fill_upper, hipStream_t st)
 {
@@ -588,13 +614,17 @@ int launch_x(const void *x, const void *wc, const void *wm, void *y, int64_t N, 
     const int64_t ipp64 = tri ? nbf * (nbf + 1) + kl * (nbf + 1) : tiles_m * tiles_n;
     if (ipp64 > (1 << 24)) return MTA_ERR_SHAPE;
     const int64_t npg = N * (C / X_HG);
+    // Groups within a lane: below 400 tiles of 16 heads, less than a round of the persistent workgroups, the kernel that computes on the
+    // vector units is as fast (this | that, us, bf16, 3x3, groups of 4: 272 tiles (B1 H16 S1024) 27.6 | 25, 440 (B4 S640) 28.8 | 34, 1056
+    // (B1 S2048) 57 | 108, 4160 (B1 S4096) 148 | 329).
+    if (GROUP < X_HG && npg * ipp64 < 400) return MTA_ERR_UNSUPPORTED;
     const xm_split sp = make_split<R, S>(npg, tiles_m, tiles_n, causal, fill_upper, tri, ipp64);
     int64_t longest = 0;
     for (int k = 0; k < 8; ++k) longest = std::max(longest, sp.start[k + 1] - sp.start[k]);
     int nw = device_cu_count() * x_occ<R>() / 8;
     if (nw < 1) nw = 1;
     if (longest < nw) nw = (int)std::max<int64_t>(longest, 1);
-    hipLaunchKernelGGL((conv_mix16_mfma<T, R, S>), dim3((unsigned)(nw * 8)), dim3(X_WT), 0, st, (const T *)x, (const T *)wc,
+    hipLaunchKernelGGL((conv_mix16_mfma<T, R, S, GROUP>), dim3((unsigned)(nw * 8)), dim3(X_WT), 0, st, (const T *)x, (const T *)wc,
                        (const T *)wm, (T *)y, (int)C, (int)H, (int)W, causal, fill_upper, (int)tiles_n, (int)ipp64, sp, nw, tri);
     return launch_status();
 }
@@ -603,18 +633,26 @@ int launch_x(const void *x, const void *wc, const void *wm, void *y, int64_t N, 
 namespace mta {
 // Returns MTA_ERR_UNSUPPORTED when no instance covers the arguments (the caller then takes another kernel).
 int conv_mix16_dispatch(const void *x, const void *wc, const void *wm, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,
-                        int S, int causal, int fill_upper, int io_dtype, hipStream_t st)
+                        int S, int group, int causal, int fill_upper, int io_dtype, hipStream_t st)
 {
     // MTA_CONV_MIX16_OFF=1 in the environment keeps groups of 16 heads on the other kernels (for comparisons)
     static const bool off = [] { const char *e = getenv("MTA_CONV_MIX16_OFF"); return e && e[0] == '1'; }();
     if (off || io_dtype == MTA_F32 || C % X_HG != 0 || W % 8 != 0 || !aligned_to(x, 16) || !aligned_to(y, 16) ||
         !aligned_to(wm, 8) || !aligned_to(wc, 16))
         return MTA_ERR_UNSUPPORTED;
+    auto go = [&](auto type, auto r, auto s) -> int {
+        using T = decltype(type);
+        if (group == 16) return launch_x<T, r(), s(), 16>(x, wc, wm, y, N, C, H, W, causal, fill_upper, st);
+        if (group == 4) return launch_x<T, r(), s(), 4>(x, wc, wm, y, N, C, H, W, causal, fill_upper, st);
+        if (group == 2) return launch_x<T, r(), s(), 2>(x, wc, wm, y, N, C, H, W, causal, fill_upper, st);
+        return MTA_ERR_UNSUPPORTED;
+    };
 #define MTA_XM_CASE(r, s)                                                                                            \
     static_assert(xgeom<r, s>::fits, "window exceeds 32 keys");                                                        \
     if (R == r && S == s) {                                                                                          \
-        if (io_dtype == MTA_BF16) return launch_x<bf16_t, r, s>(x, wc, wm, y, N, C, H, W, causal, fill_upper, st);    \
-        return launch_x<f16_t, r, s>(x, wc, wm, y, N, C, H, W, causal, fill_upper, st);                               \
+        const std::integral_constant<int, r> r_{};                                                                   \
+        const std::integral_constant<int, s> s_{};                                                                   \
+        return io_dtype == MTA_BF16 ? go(bf16_t{}, r_, s_) : go(f16_t{}, r_, s_);                                     \
     }
     MTA_XM_CASE(3, 3)
     MTA_XM_CASE(5, 5)

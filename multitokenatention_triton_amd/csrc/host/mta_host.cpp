@@ -42,16 +42,18 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
     return !masked || group != FUSED_MFMA_GROUP || t == at::kFloat || !no_row_lists();
 }
 
-// Whether conv + dense mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
+// Whether conv + mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
 // heads at about 20 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other.
 // us of the forward (H16 D64 fp16, the post-softmax conv 3x3 / 7x7), one kernel | two: 272 tiles (B1 S1024) 68.7 | 60.2 / 72.8 | 64.5,
 // 544 (B2 S1008) 101.0 | 88.3 / 106.4 | 95.6, 600 (B1 S1536) 109.9 | 91.9 / 115.9 | 98.3, 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3,
 // 840 (B2 S1280) 126.1 | 123.9 / 131.8 | 133.3, 1056 (B1 S2048) 155.0 | 164.5 / 161.5 | 175.5, 1088 (B4 S1024) 149.8 | 171.4 /
 // 156.9 | 182.6; the runs of one side differ by up to 2.
+// A whole round is as good: 440 tiles (B4 S640, groups of 4, the two stages alone) 28.8 | 34.8 / 32.3 | 37.6.  Groups of 2 or 4 heads:
+// 1056 tiles 57 | 60 / 64 | 62, 2112 (B2 S2048) 92 | 120 / 98 | 125, 4160 (B1 S4096) 148 | 232 / 163 | 238.
 bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only)
 {
-    const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64;
-    return planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk) >= 800;
+    const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64, tiles = planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk);
+    return tiles >= 800 || (tiles >= 400 && tiles <= 512);
 }
 
 int64_t lcm(int64_t a, int64_t b)
@@ -300,12 +302,17 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
         }
         if (empty_rows && !post_conv_identity) band_zero_(scores, empty_row_ends(*empty_rows));
         // conv and mix in one pass, the conv result never written: taken where it measures at least as fast as the two
-        // kernels (mixing groups of up to 4 heads and the sizes with a vector-staged instance; dense groups of 16).  Under a
-        // band mask the conv's result is zeroed at the hidden positions ahead of the mixing: two kernels.
+        // kernels.  Under a band mask the conv's result is zeroed at the hidden positions ahead of the mixing: two kernels.
+        // - 16 heads at a time (dense groups of 16, or groups of 2 or 4) on the matrix cores, where there are tiles enough.
+        // - groups of up to 4 heads and the sizes with a vector-staged instance, on the vector units: 3x3 in fp32, and while the
+        //   tensor is so small that a launch counts.  One kernel | two, us, the lower triangle, 3x3 / 7x7: bf16 groups of 4, 12 x 768^2
+        //   13 | 21 / 21 | 21, 12 x 1024^2 24 | 24 / 37 | 25, 32 x 1448^2 75 | 60 / 104 | 64, 12 x 2912^2 103 | 95 / 146 | 101; fp32 groups
+        //   of 2, 16 x 512^2 13 | 20 / 22 | 22, 12 x 1024^2 27 | 30 / 54 | 36, 16 x 1536^2 52 | 70 / 106 | 81, 16 x 2048^2 115 | 117 / 268 | 141.
         const int64_t r = post_conv_w.size(1), s = post_conv_w.size(2);
-        const bool mix16 = g_post == 16 && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
+        const bool mix16 = (g_post == 16 || ((g_post == 2 || g_post == 4) && heads % 16 == 0)) && ((r == 3 && s == 3) || (r == 5 && s == 5) || (r == 7 && s == 7)) && is16(scores) &&
                            post_conv_w.scalar_type() == scores.scalar_type() && w_post.scalar_type() == scores.scalar_type() && n_keys % 8 == 0;
-        const bool small_groups = g_post <= 4 && g_post != 3 && ((r == 3 && s == 3) || (r == 7 && s == 7));
+        const bool small_groups = g_post <= 4 && g_post != 3 &&
+                                  ((r == 3 && s == 3 && (dtype == at::kFloat || scores.numel() <= 12 << 20)) || (r == 7 && s == 7 && scores.numel() <= 6 << 20));
         OptTensor done;
         if (!first && !post_conv_identity && w2 &&
             (small_groups || (mix16 && conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv)))) {

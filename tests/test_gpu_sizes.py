@@ -425,6 +425,30 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,k", [(3, 3), (5, 5), (7, 7)])
+@pytest.mark.parametrize("n,c,s,group", [(4, 16, 640, 4), (2, 32, 648, 2), (1, 16, 1288, 4)])
+def test_conv_and_small_groups_on_the_matrix_cores(pkg, n, c, s, group, r, k, dtype):
+    """Conv and mixing of groups of 2 or 4 in one pass against the two kernels (the same roundings; sums of at most 4 products in
+    another order: a neighbour of the result), NaN above the diagonal, and NaN in one head that must stay in its group."""
+    g = torch.Generator().manual_seed(61)
+    block = torch.arange(c) // group
+    same = block[:, None] == block[None, :]
+    x = torch.randn(n, c, s, s, generator=g).to(dtype).cuda()
+    x = x.masked_fill(~torch.tril(torch.ones(s, s, dtype=torch.bool, device="cuda")), float("nan"))
+    w = torch.randn(c, r, k, generator=g).to(dtype).cuda()
+    wm = (torch.eye(c) + 0.3 * torch.randn(c, c, generator=g)).to(dtype).masked_fill(~same, float("inf")).cuda()
+    ulp = 2 * _unit(dtype)
+    for fill in (False, True):
+        one = pkg.ops.conv2d_headmix(x, w, wm, True, group_size=group, fill_upper=fill)
+        two = pkg.ops.headmix(pkg.ops.conv2d_causal(x, w, True, fill_upper=False), wm, True, 0.0, group_size=group, fill_upper=fill)
+        one, two = (t if fill else t.tril() for t in (one, two))
+        torch.testing.assert_close(one.float(), two.float(), rtol=ulp, atol=4 * ulp)
+    x[0, 5] = float("nan")
+    one = pkg.ops.conv2d_headmix(x, w, wm, True, group_size=group, fill_upper=True)
+    assert one.isnan().any(-1).any(-1).nonzero().tolist() == [[0, h] for h in range(c) if h // group == 5 // group]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("c,group", [(9, 0), (12, 0), (24, 12), (17, 0), (24, 0), (32, 0), (64, 32)])
 def test_mix_softmax_of_dense_groups(pkg, c, group, dtype):
     """16-bit groups of 9 to 32 heads in one pass: rows about a tile of 128 keys, of one and several wavefronts and passes, the longest
