@@ -69,10 +69,10 @@ __device__ __forceinline__ split_t split_of(int block, int C, int bpc)
 // ---- matrix-core kernel -------------------------------------------------------------------------------------------
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 constexpr int MB = 2;            // 16-row blocks of dy per work item (against MB + 1 blocks of x)
-constexpr int HV = 2;            // 32-key halves per step: a step takes whole 128-byte lines of its rows, the two
-                                 // halves of a line in load instructions issued back to back
 constexpr int MROWS = 16 * MB;   // rows of dy per work item
-constexpr int KSTEP = 32 * HV;   // keys per step
+// 32-key halves per step (HV): with two a step takes whole 128-byte lines of its rows, the two halves of a line in load instructions
+// issued back to back; with one the three sets of pieces take 60 registers instead of 120, and a wavefront's share of a small tensor
+// is a chain of shorter steps that can be dealt more evenly.  See launch().
 
 // Eight consecutive keys k0..k0+7 (k0 a multiple of 8, possibly -8) of row h.  The forward pass's masks -- 0 outside the
 // plane and, under the causal rule, for keys beyond the row index -- are applied in two parts: piece_ok() picks the
@@ -99,13 +99,13 @@ __device__ __forceinline__ u4 mask_piece(u4 v, int h, int k0, int H, int W, int 
     return v;
 }
 
-// One step of a wavefront covers 32 keys: lane (r, g) loads the eight keys kb + 8g .. +7 of its rows -- MB 16-row blocks
+// One step of a wavefront covers 32 HV keys: lane (r, g) loads the eight keys kb + 8g .. +7 of its rows -- MB 16-row blocks
 // of dy and the MB + 1 blocks of x around them -- and nothing else.  The products pair the dy keys of the lane group to
 // the LEFT (k-8 .. k-1, k = kb + 8g) with the 24-key window k-16 .. k+7 of x, whose first two thirds are the pieces of
 // the two lane groups to the left as well: those come over ds_bpermute (for the first groups of a step, from the step
 // before, which stays in registers), not from memory.  With every lane loading its whole window itself (three pieces
 // per block of x: 11 loads per step instead of 5) the kernel's time followed the number of load instructions.
-struct step_pieces {
+template <int HV> struct step_pieces {
     u4 dy[MB][HV];
     u4 x[MB + 1][HV];
 };
@@ -124,9 +124,9 @@ template <typename T> __device__ __forceinline__ u4 load16(const T *plane, unsig
 }
 
 // `inner` (wavefront-uniform): every piece of the step lies inside the plane and on or below the diagonal.  kb may be
-// -32 (the step ahead of a row's first, whose pieces all read as 0).
-template <typename T>
-__device__ __forceinline__ void load_step(step_pieces &o, const T *xp, const T *dyp, const lane_rows &rows, int p0, int kb,
+// -32 HV (the step ahead of a row's first, whose pieces all read as 0).
+template <int HV, typename T>
+__device__ __forceinline__ void load_step(step_pieces<HV> &o, const T *xp, const T *dyp, const lane_rows &rows, int p0, int kb,
                                           int r, int g, int H, int W, int causal, bool inner)
 {
     if (inner) {
@@ -156,10 +156,11 @@ __device__ __forceinline__ void load_step(step_pieces &o, const T *xp, const T *
     }
 }
 
-__device__ __forceinline__ void mask_step(step_pieces &o, int p0, int kb, int r, int g, int H, int W, int causal)
+template <int HV>
+__device__ __forceinline__ void mask_step(step_pieces<HV> &o, int p0, int kb, int r, int g, int H, int W, int causal)
 {
-    // rows of this item start at p0 - 16, the step's last key is kb + KSTEP - 1
-    const bool edge = causal && kb + KSTEP - 1 > p0 - 16;
+    // rows of this item start at p0 - 16, the step's last key is kb + 32 HV - 1
+    const bool edge = causal && kb + 32 * HV - 1 > p0 - 16;
 #pragma unroll
     for (int hv = 0; hv < HV; ++hv) {
         const int k = kb + 32 * hv + 8 * g;
@@ -185,8 +186,8 @@ __device__ __forceinline__ u4 piece_from_left(const u4 &prev, const u4 &cur, int
 
 // The 2*MB*S products of a step: block mb of dy against blocks mb and mb+1 of x, every key offset j.  The operand of
 // offset j is the 24-key window of x from key 8 + j - pad on (a byte shift of two registers for odd starts).
-template <typename T, int S>
-__device__ __forceinline__ void accumulate_step(f32x4 (&acc)[2][S], const step_pieces &prev, const step_pieces &cur, int lane)
+template <typename T, int S, int HV>
+__device__ __forceinline__ void accumulate_step(f32x4 (&acc)[2][S], const step_pieces<HV> &prev, const step_pieces<HV> &cur, int lane)
 {
     constexpr int PW = (S - 1) / 2;
 #pragma unroll
@@ -225,13 +226,14 @@ __device__ __forceinline__ void accumulate_step(f32x4 (&acc)[2][S], const step_p
     }
 }
 
-template <typename T, int R, int S>
-__global__ __launch_bounds__(NT) void conv2d_bwd_weight_mfma(const T *__restrict__ x, const T *__restrict__ dy,
+template <typename T, int R, int S, int HV>
+__global__ __launch_bounds__(NT, HV == 1 ? 2 : 1) void conv2d_bwd_weight_mfma(const T *__restrict__ x, const T *__restrict__ dy,
                                                              float *__restrict__ partial, int N, int C, int H, int W,
                                                              int causal, int tiles_m, int nseg, int bpc)
 {
     static_assert(R <= 17 && S <= 16 && (S - 1) / 2 <= 8, "window of 24 keys, two 16-row blocks of halo");
     __shared__ float tile[2 * S][16][17];
+    constexpr int KSTEP = 32 * HV;   // keys per step
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int c = blockIdx.x / bpc, sub = blockIdx.x % bpc;
 
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(NT) void conv2d_bwd_weight_mfma(const T *__restrict
         // through this step's products, and the step before supplies the left neighbours of this step's first lane
         // groups.  The last step fetches itself again, so that the loads in flight never depend on a branch; the step
         // ahead of the segment's first is fetched for its pieces only.
-        step_pieces sa, sb, sc;
+        step_pieces<HV> sa, sb, sc;
         load_step(sa, xp, dyp, rows, p0, KSTEP * (t0 - 1), r, g, H, W, causal, inner(t0 - 1));
         load_step(sb, xp, dyp, rows, p0, KSTEP * t0, r, g, H, W, causal, inner(t0));
         if (!inner(t0 - 1)) mask_step(sa, p0, KSTEP * (t0 - 1), r, g, H, W, causal);
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(NT) void conv2d_bwd_weight_mfma(const T *__restrict
             const int tn = t + 1 < t1 ? t + 1 : t;                                                      \
             load_step(NX, xp, dyp, rows, p0, KSTEP * tn, r, g, H, W, causal, inner(tn));                \
             if (!inner(t)) mask_step(CU, p0, KSTEP * t, r, g, H, W, causal);                            \
-            accumulate_step<T, S>(acc, PV, CU, lane);                                                   \
+            accumulate_step<T, S, HV>(acc, PV, CU, lane);                                                   \
         }
         for (;;) {
             MTA_CBW_STEP(sa, sb, sc)
@@ -417,17 +419,31 @@ int launch(const void *x, const void *dy, void *dw, float *partial, int bpc, int
             const int rows_m = (int)((H + MROWS - 1) / MROWS);
             int bm = (int)((512 + C - 1) / C);
             if (bm > bpc) bm = bpc;
-            int64_t nseg = ((int64_t)8 * bm + N * rows_m - 1) / (N * rows_m);
-            const int64_t seg_cap = W / 256 > 1 ? W / 256 : 1;
+            // Steps of 32 keys in segments of 128 or more (of 64 while there are fewer of them than wavefronts) up to 32 M elements and
+            // for the 15-key kernel, which then fits twice per CU; steps of 64 keys in segments of 256 or more for the others.  us, fp16,
+            // the lower triangle, nothing in the caches, 64 | 32:  16 x 512^2 3x3 20.4 | 16.8, 7x7 21.6 | 15.7, 11x15 35.9 | 20.0;
+            // 16 x 1024^2 22.3 | 19.9, 23.6 | 20.7, 38.5 | 25.8;  128 x 320^2 23.1 | 18.8, 25.6 | 19.5, 43.5 | 25.5;  16 x 1376^2 26.9 | 26.0,
+            // 29.0 | 27.4, 47.8 | 33.8;  128 x 680^2 46.4 | 48.5, 49.7 | 50.4, 75 | 58;  32 x 2048^2 62 | 69, 69 | 73, 104 | 86.
+            const bool fine = S > 11 || N * C * H * W <= 32 << 20;
+            int64_t nseg = ((int64_t)8 * bm + N * rows_m - 1) / (N * rows_m), seg_cap = W / (fine ? 128 : 256);
+            if (fine && N * rows_m * seg_cap < 4 * bm) seg_cap = W / 64;
             if (nseg > seg_cap) nseg = seg_cap;
-            if (nseg > 8) nseg = 8;
+            if (nseg > (fine ? 32 : 8)) nseg = fine ? 32 : 8;
+            if (nseg < 1) nseg = 1;
             if (bm > N * rows_m * nseg) bm = (int)(N * rows_m * nseg);
             if (N * rows_m * nseg > 0x3fffffffLL) return MTA_ERR_SHAPE;  // the kernel counts items in 32 bits
 #define MTA_CONV_CASE(r, s)                                                                                          \
     if (R == r && S == s) {                                                                                          \
-        hipLaunchKernelGGL((conv2d_bwd_weight_mfma<T, r, s>), dim3((unsigned)(C * bm)), dim3(NT), 0, st,              \
-                           (const T *)x, (const T *)dy, partial, (int)N, (int)C, (int)H, (int)W, causal, rows_m,      \
-                           (int)nseg, bm);                                                                           \
+        auto go = [&](auto kern) {                                                                                   \
+            hipLaunchKernelGGL(kern, dim3((unsigned)(C * bm)), dim3(NT), 0, st, (const T *)x, (const T *)dy, partial, \
+                               (int)N, (int)C, (int)H, (int)W, causal, rows_m, (int)nseg, bm);                       \
+        };                                                                                                           \
+        if constexpr (s <= 11) {                                                                                     \
+            if (fine) go(conv2d_bwd_weight_mfma<T, r, s, 1>);                                                        \
+            else go(conv2d_bwd_weight_mfma<T, r, s, 2>);                                                             \
+        } else {                                                                                                     \
+            go(conv2d_bwd_weight_mfma<T, r, s, 1>);                                                                  \
+        }                                                                                                            \
         bpc = bm;                                                                                                    \
         goto done;                                                                                                   \
     }

@@ -424,6 +424,19 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
         assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("r,k", [(3, 3), (6, 11), (7, 9)])
+def test_conv_kernel_gradient_of_large_and_of_small_tensors(pkg, r, k, causal):
+    """Beyond 32 M elements the kernel gradient takes steps of 64 keys, its batch entries one by one steps of 32: fp32 sums of the same
+    exact products in another order, whose error sqrt(n)*2^-22 of the sum of magnitudes covers."""
+    x, dy = (torch.randn(2, 5, 2048, 2040, device="cuda").to(torch.bfloat16) for _ in range(2))
+    assert x.numel() > 32 << 20 >= x[:1].numel()
+    whole = pkg.ops.conv2d_bwd_weight(x, dy, (r, k), causal)
+    parts = sum(pkg.ops.conv2d_bwd_weight(x[i:i + 1], dy[i:i + 1], (r, k), causal).double() for i in range(2))
+    size = pkg.ops.conv2d_bwd_weight(x.abs(), dy.abs(), (r, k), causal).double()
+    assert ((whole.double() - parts).abs() <= (2 * 2048 * 2040) ** 0.5 * 2.0 ** -22 * size).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("r,k", [(3, 3), (5, 5), (7, 7)])
 @pytest.mark.parametrize("n,c,s,group", [(4, 16, 640, 4), (2, 32, 648, 2), (1, 16, 1288, 4)])
