@@ -117,9 +117,10 @@ template <int NT> __device__ __forceinline__ float block_sum(float v, float *red
 
 // Register-resident row: Q <= NT*VEC*NV.
 // (KB: with a key bias and / or a first visible key per query row.  An instantiation of its own, compiled without the
-// occupancy target: the bias vector costs the registers that target leaves none of.)
+// occupancy target: the bias vector costs the registers that target leaves none of; nor have 8 heads any left, which spilled: 8 x 2048^2
+// fp16 with fp32 weights 101 -> 44 us without it.)
 template <typename T, int G, int NV, int VEC, int NT, bool KB>
-__global__ __launch_bounds__(NT, (!KB && NT == 256 && G * NV == 8) ? RS_OCC : 1) void mix_softmax_mix(const T *__restrict__ x, const void *__restrict__ w1,
+__global__ __launch_bounds__(NT, (!KB && NT == 256 && G < 8 && G * NV == 8) ? RS_OCC : 1) void mix_softmax_mix(const T *__restrict__ x, const void *__restrict__ w1,
                                                       const void *__restrict__ w2, const float *__restrict__ kb,
                                                       T *__restrict__ y, int C, int P, int Q, int causal,
                                                       int w_dtype, int fill_upper, const int *__restrict__ row_lo, int stream)
