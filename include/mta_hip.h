@@ -304,6 +304,11 @@ int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t B, int64_t
 int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
                               float scale, int io_dtype, void *stream);
 
+/* Both products of one P (the gradients of Q and K): o = scale * P V, ot = scale * P^T X, as mta_causal_pv_scaled_fwd and
+ * mta_causal_ptx_scaled_fwd give them, bit by bit; in one launch where both grids are small. */
+int mta_causal_products(const void *p, const void *v, const void *x, void *o, void *ot, int64_t B, int64_t H, int64_t S, int64_t D,
+                        int causal, float scale, int io_dtype, void *stream);
+
 /* The three products on the lower triangle for fp32 tensors, D in {64,128}, S % 4 == 0 (MTA_ERR_UNSUPPORTED otherwise), causal:
  *   mta_lower_scores_f32:  out[p,q] = sum_d a[p,d] b[q,d] for q <= p (QK^T of mta_attention_triton.py:69, and dP = dO V^T);
  *                          nothing is written above the diagonal beyond the 16-byte vectors that straddle it (zeros)

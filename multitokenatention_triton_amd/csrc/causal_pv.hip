@@ -243,19 +243,17 @@ __device__ __forceinline__ void narrow_reduce(T *a, T *b, const f32x4 (&oacc)[RB
 }
 
 template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
-                                                                  int causal, int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl,
-                                                                  float scale)
+__device__ __forceinline__ void pv_narrow(T *lds, unsigned wg, const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal,
+                                          int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
 {
     constexpr int CPR = D / 8, TILE = N_STEP * D, ROUNDS = TILE / 8 / 64, DB = D / 16;
-    __shared__ __align__(16) T v_a_all[4 * TILE];
-    __shared__ __align__(16) T v_b_all[4 * TILE];
+    T *const v_a_all = lds, *const v_b_all = lds + 4 * TILE;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     T *const v_a = v_a_all + wave * TILE;
     T *const v_b = v_b_all + wave * TILE;
     int bh, rank;
-    if (!longest_first(heads, nrb, cus, bh, rank)) return;
+    if (!longest_first(wg, heads, nrb, cus, bh, rank)) return;
     const int q0 = (nrb - 1 - rank) * N_ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
     const T *Vp = V + bh * (int64_t)S * D;
@@ -365,6 +363,15 @@ __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__res
         for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v] * scale);
         *reinterpret_cast<quad *>(Op + (int64_t)prow[rb] * D + db * 16 + kg * 4) = out;
     });
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
+                                                                  int causal, int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl,
+                                                                  float scale)
+{
+    __shared__ __align__(16) T lds[8 * N_STEP * D];
+    pv_narrow<T, D>(lds, blockIdx.x, P, V, O, S, causal, heads, nrb, cus, band_lo, H, tri_gl, scale);
 }
 
 // The sums of GR groups of GT threads added up in the first group (true there): the upper half of the groups hand theirs to the
@@ -534,14 +541,11 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
 __device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1); }
 
 template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
-                                                                   int causal, int heads, int nkb, int cus, float scale)
+__device__ __forceinline__ void ptx_narrow(T *lds, unsigned wg, const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S, int causal,
+                                           int heads, int nkb, int cus, float scale)
 {
     constexpr int XC = D / 8, XT = N_STEP * D, PCH = N_ROWS / 8, XR = XT / 8 / 64, PT = N_STEP * N_ROWS, PR = PT / 8 / 64, DB = D / 16;
-    __shared__ __align__(16) T x_a_all[4 * XT];
-    __shared__ __align__(16) T x_b_all[4 * XT];
-    __shared__ __align__(16) T p_a_all[4 * PT];
-    __shared__ __align__(16) T p_b_all[4 * PT];
+    T *const x_a_all = lds, *const x_b_all = lds + 4 * XT, *const p_a_all = lds + 8 * XT, *const p_b_all = p_a_all + 4 * PT;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     T *const x_a = x_a_all + wave * XT;
@@ -549,7 +553,7 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
     T *const p_a = p_a_all + wave * PT;
     T *const p_b = p_b_all + wave * PT;
     int bh, rank;
-    if (!longest_first(heads, nkb, cus, bh, rank)) return;
+    if (!longest_first(wg, heads, nkb, cus, bh, rank)) return;
     const int k0 = rank * N_ROWS;   // under the causal rule the first keys have the most query rows
     const T *Pp = P + bh * (int64_t)S * S;
     const T *Xp = X + bh * (int64_t)S * D;
@@ -637,6 +641,29 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__re
         for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(sum[v] * scale);
         *reinterpret_cast<quad *>(Op + (int64_t)krow[rb] * D + db * 16 + kg * 4) = out;
     });
+}
+
+template <typename T, int D> constexpr int ptx_narrow_lds() { return 8 * N_STEP * D + 8 * N_STEP * N_ROWS; }   // elements
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
+                                                                   int causal, int heads, int nkb, int cus, float scale)
+{
+    __shared__ __align__(16) T lds[ptx_narrow_lds<T, D>()];
+    ptx_narrow<T, D>(lds, blockIdx.x, P, X, O, S, causal, heads, nkb, cus, scale);
+}
+
+// Both products of one P, a workgroup of each in turns within an XCD: what a training step has left behind the gradient of the
+// scores.  Two small grids, each bound by its own latency, and two launches of a step that the host bounds; one | two, us, bf16:
+// B1 H8 S256 D64 4.5 | 8.5, B1 H16 S512 D128 8.1 | 13.8, B1 H16 S1024 D64 13.2 | 15.6, B1 H8 S2048 D64 19.7 | 26.2, D128 29.6 | 33.3.
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void causal_products_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, const T *__restrict__ X,
+                                                                        T *__restrict__ O, T *__restrict__ Ot, int S, int causal, int heads, int blocks,
+                                                                        int cus, float scale)
+{
+    __shared__ __align__(16) T lds[ptx_narrow_lds<T, D>()];
+    const unsigned wg = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+    if (blockIdx.x & 8) ptx_narrow<T, D>(lds, wg, P, X, Ot, S, causal, heads, blocks, cus, scale);
+    else pv_narrow<T, D>(lds, wg, P, V, O, S, causal, heads, blocks, cus, nullptr, 1, 0, scale);
 }
 
 // ---- the transposed product --------------------------------------------------------------------------------------
@@ -933,4 +960,30 @@ extern "C" int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, 
     if (io_dtype == MTA_BF16)
         return D == 64 ? launch_t<bf16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<bf16_t, 128>(p, x, o, B, H, S, causal, scale, st);
     return D == 64 ? launch_t<f16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<f16_t, 128>(p, x, o, B, H, S, causal, scale, st);
+}
+
+// o = scale * P V and ot = scale * P^T X with the lower triangle of P (causal; else all of it)
+extern "C" int mta_causal_products(const void *p, const void *v, const void *x, void *o, void *ot, int64_t B, int64_t H, int64_t S, int64_t D,
+                                   int causal, float scale, int io_dtype, void *stream)
+{
+    if (!p || !v || !x || !o || !ot) return MTA_ERR_NULL;
+    const bool one = io_dtype != MTA_F32 && dtype_size(io_dtype) && B > 0 && H > 0 && S > 0 && S <= (1 << 24) && B * H <= 65535 && (D == 64 || D == 128) &&
+                     S % 8 == 0 && aligned_to(p, 16) && aligned_to(v, 16) && aligned_to(x, 16) && aligned_to(o, 16) && aligned_to(ot, 16) &&
+                     product_form(B * H, S, (int)D, false, false) == NARROW && product_form(B * H, S, (int)D, true, false) == NARROW;
+    if (!one) {
+        const int rc = mta_causal_pv_scaled_fwd(p, v, o, B, H, S, D, causal, scale, io_dtype, stream);
+        return rc != MTA_OK ? rc : mta_causal_ptx_scaled_fwd(p, x, ot, B, H, S, D, causal, scale, io_dtype, stream);
+    }
+    const int64_t blocks = (S + N_ROWS - 1) / N_ROWS, wg = (B * H * blocks + 7) / 8 * 8;
+    const int cus = causal && 2 * wg <= (int64_t)(D == 64 ? 3 : 2) * device_cu_count() ? device_cu_count() / 16 : 0;
+    auto go = [&](auto type, auto d) {
+        using T = decltype(type);
+        hipLaunchKernelGGL((causal_products_narrow_kernel<T, d()>), dim3((unsigned)(2 * wg)), dim3(256), 0, (hipStream_t)stream, (const T *)p, (const T *)v,
+                           (const T *)x, (T *)o, (T *)ot, (int)S, causal, (int)(B * H), (int)blocks, cus, scale);
+    };
+    const std::integral_constant<int, 64> d64{};
+    const std::integral_constant<int, 128> d128{};
+    if (io_dtype == MTA_BF16) D == 64 ? go(bf16_t{}, d64) : go(bf16_t{}, d128);
+    else D == 64 ? go(f16_t{}, d64) : go(f16_t{}, d128);
+    return launch_status();
 }

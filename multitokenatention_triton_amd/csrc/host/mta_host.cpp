@@ -448,9 +448,12 @@ void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, c
         if (first) band_zero_(g, *first);
         Tensor dq, dk;
         OptTensor own_q, own_k;
-        if (need[0]) own_q = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
+        if (lower && need[0] && need[1]) {
+            if (const auto both = causal_products(g, k, q, scale)) std::tie(own_q, own_k) = *both;
+        }
+        if (need[0] && !own_q) own_q = lower ? causal_pv(g, k, true, OptTensor(), scale) : OptTensor();
         if (need[0]) dq = own_q ? *own_q : matmul_as(g, k);
-        if (need[1]) own_k = lower ? causal_ptx(g, q, true, scale) : OptTensor();
+        if (need[1] && !own_k) own_k = lower ? causal_ptx(g, q, true, scale) : OptTensor();
         if (need[1]) dk = own_k ? *own_k : matmul_as(g.transpose(2, 3), q);
         // the factor, where the products were the library's
         if (need[0] && need[1] && !own_q && !own_k && dq.sizes() == dk.sizes()) {

@@ -335,6 +335,20 @@ inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, dou
     return o;
 }
 
+// P v and P^T x, both times `scale`, of 16-bit tensors and a causal P
+inline std::optional<std::pair<Tensor, Tensor>> causal_products(const Tensor &p_, const Tensor &v_, const Tensor &x_, double scale)
+{
+    if (!is16(p_) || p_.scalar_type() != v_.scalar_type() || p_.scalar_type() != x_.scalar_type() || v_.sizes() != x_.sizes() ||
+        !score_planes_of(p_.sizes(), v_.sizes()) || !lower_products_supported(p_.scalar_type(), v_.sizes(), true))
+        return std::nullopt;
+    const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V"), x = on_gpu(x_, "X");
+    Tensor o = at::empty(v.sizes(), v.options()), ot = at::empty(x.sizes(), x.options());
+    check(mta_causal_products(ptr(p), ptr(v), ptr(x), out_ptr(o), out_ptr(ot), v.size(0), v.size(1), v.size(2), v.size(3), true, (float)scale,
+                              code(p, "P"), stream_of(p)),
+          "mta_causal_products");
+    return std::make_pair(o, ot);
+}
+
 inline void band_zero_(const Tensor &x, const Tensor &first)
 {
     TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && first.dim() == 2 && first.size(0) == x.size(0) && first.size(1) == x.size(2) &&

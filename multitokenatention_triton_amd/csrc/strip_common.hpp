@@ -93,16 +93,16 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f)
     static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-// The (batch, head) and the rank of a workgroup's block in a grid of heads x blocks whose blocks get shorter with their rank (rows
+// The (batch, head) and the rank of workgroup wg's block in a grid of heads x blocks whose blocks get shorter with their rank (rows
 // under the causal rule): all heads' longest blocks first, so that the short ones fill the end of the grid.  Workgroup ids are
 // dealt to the 8 XCDs round-robin; where the heads divide evenly an XCD keeps its own, whose operands then stay in its L2.
 // cus > 0: the grid is resident at once, a round of `cus` workgroups per XCD after the other - every second round comes in
 // reverse, so that a CU gets a long block and a short one.  False beyond the grid.
-__device__ __forceinline__ bool longest_first(int heads, int blocks, int cus, int &bh, int &rank)
+__device__ __forceinline__ bool longest_first(unsigned wg, int heads, int blocks, int cus, int &bh, int &rank)
 {
     const bool own = heads % 8 == 0;
     const int n = (own ? heads / 8 : heads) * blocks, round = own ? cus : 8 * cus;
-    int pos = own ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    int pos = own ? (int)(wg >> 3) : (int)wg;
     if (pos >= n) return false;
     if (round > 0 && (pos / round & 1)) {
         const int first = pos / round * round, end = first + round < n ? first + round : n;
@@ -110,8 +110,12 @@ __device__ __forceinline__ bool longest_first(int heads, int blocks, int cus, in
     }
     const int h = own ? heads / 8 : heads;
     rank = pos / h;
-    bh = own ? (int)(blockIdx.x & 7) * h + pos % h : pos % h;
+    bh = own ? (int)(wg & 7) * h + pos % h : pos % h;
     return true;
+}
+__device__ __forceinline__ bool longest_first(int heads, int blocks, int cus, int &bh, int &rank)
+{
+    return longest_first(blockIdx.x, heads, blocks, cus, bh, rank);
 }
 
 inline int device_cu_count()

@@ -424,6 +424,27 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
         assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_both_products_of_a_matrix(pkg, d, dtype):
+    """The two products in one call: the bits of the single ones, in one launch (grids of up to 256 blocks, heads that divide over the
+    XCDs and that do not, one block, a last block in part) and in two; NaN above the diagonal."""
+    lib, code = pkg._lib.load(), {torch.bfloat16: 1, torch.float16: 2}[dtype]
+    for b, h, s, causal in ((1, 1, 8, True), (1, 8, 256, True), (2, 3, 72, True), (1, 16, 1000, True), (3, 5, 264, False), (1, 8, 2048, True), (1, 16, 1096, True)):
+        print(f"both products {b}x{h}x{s}x{d} causal={causal} {dtype}", flush=True)
+        p = torch.randn(b, h, s, s, device="cuda").to(dtype)
+        if causal:
+            p = p.masked_fill(~torch.tril(torch.ones(s, s, dtype=torch.bool, device="cuda")), float("nan"))
+        v, x = (torch.randn(b, h, s, d, device="cuda").to(dtype) for _ in range(2))
+        got, want = ([torch.full_like(v, 7.0) for _ in range(2)] for _ in range(2))
+        st = torch.cuda.current_stream().cuda_stream
+        at = lambda t: t.data_ptr()  # noqa: E731
+        assert lib.mta_causal_products(at(p), at(v), at(x), at(got[0]), at(got[1]), b, h, s, d, causal, 0.37, code, st) == 0
+        assert lib.mta_causal_pv_scaled_fwd(at(p), at(v), at(want[0]), b, h, s, d, causal, 0.37, code, st) == 0
+        assert lib.mta_causal_ptx_scaled_fwd(at(p), at(x), at(want[1]), b, h, s, d, causal, 0.37, code, st) == 0
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and not got[0].isnan().any()
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("r,k", [(3, 3), (6, 11), (7, 9)])
 def test_conv_kernel_gradient_of_large_and_of_small_tensors(pkg, r, k, causal):
