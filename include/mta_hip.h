@@ -304,6 +304,11 @@ int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t B, int64_t
 int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
                               float scale, int io_dtype, void *stream);
 
+/* mta_causal_ptx_scaled_fwd with X where its rows lie: row p of head h of batch entry b from element b*x_batch + h*x_head + p*x_row
+ * on, all multiples of 8 (the gradient of an output that was laid out (B,S,H,D)).  16-bit data. */
+int mta_causal_ptx_rows_fwd(const void *p, const void *x, int64_t x_batch, int64_t x_head, int64_t x_row, void *o, int64_t B,
+                            int64_t H, int64_t S, int64_t D, int causal, float scale, int io_dtype, void *stream);
+
 /* Both products of one P (the gradients of Q and K): o = scale * P V, ot = scale * P^T X, as mta_causal_pv_scaled_fwd and
  * mta_causal_ptx_scaled_fwd give them, bit by bit; in one launch where both grids are small. */
 int mta_causal_products(const void *p, const void *v, const void *x, void *o, void *ot, int64_t B, int64_t H, int64_t S, int64_t D,
@@ -320,6 +325,9 @@ int mta_causal_products(const void *p, const void *v, const void *x, void *o, vo
  * first visible key are 0; key blocks that no row of a block of 128 sees are left unwritten. */
 int mta_lower_scores_fwd(const void *a, const void *b, const void *first_visible, void *out, int64_t B, int64_t H, int64_t S, int64_t D,
                          int io_dtype, void *stream);
+/* mta_lower_scores_fwd with a where its rows lie, as mta_causal_ptx_rows_fwd's X.  16-bit data. */
+int mta_lower_scores_rows_fwd(const void *a, int64_t a_batch, int64_t a_head, int64_t a_row, const void *b, const void *first_visible,
+                              void *out, int64_t B, int64_t H, int64_t S, int64_t D, int io_dtype, void *stream);
 int mta_lower_scores_f32(const void *a, const void *b, void *out, int64_t B, int64_t H, int64_t S, int64_t D, void *stream);
 int mta_causal_pv_f32(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);
 int mta_causal_ptx_f32(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream);

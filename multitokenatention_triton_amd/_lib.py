@@ -78,6 +78,8 @@ SIGNATURES = {
     "mta_causal_pv_scaled_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),
     "mta_causal_ptx_scaled_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),
     "mta_causal_products": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),
+    "mta_lower_scores_rows_fwd": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
+    "mta_causal_ptx_rows_fwd": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int, _vp]),
     "mta_lower_scores_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "mta_lower_scores_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "mta_causal_pv_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp]),

@@ -542,7 +542,7 @@ __device__ __forceinline__ int p_swizzle(int row) { return 2 * ((row >> 3) & 1);
 
 template <typename T, int D>
 __device__ __forceinline__ void ptx_narrow(T *lds, unsigned wg, const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S, int causal,
-                                           int heads, int nkb, int cus, float scale)
+                                           int heads, int nkb, int cus, float scale, int H, row_strides xs)
 {
     constexpr int XC = D / 8, XT = N_STEP * D, PCH = N_ROWS / 8, XR = XT / 8 / 64, PT = N_STEP * N_ROWS, PR = PT / 8 / 64, DB = D / 16;
     T *const x_a_all = lds, *const x_b_all = lds + 4 * XT, *const p_a_all = lds + 8 * XT, *const p_b_all = p_a_all + 4 * PT;
@@ -556,7 +556,8 @@ __device__ __forceinline__ void ptx_narrow(T *lds, unsigned wg, const T *__restr
     if (!longest_first(wg, heads, nkb, cus, bh, rank)) return;
     const int k0 = rank * N_ROWS;   // under the causal rule the first keys have the most query rows
     const T *Pp = P + bh * (int64_t)S * S;
-    const T *Xp = X + bh * (int64_t)S * D;
+    const T *Xp = X + bh / H * xs.batch + bh % H * xs.head;
+    const int xrow = (int)xs.row;
     T *Op = O + bh * (int64_t)S * D;
     auto issue = [&](int j, T *xdst, T *pdst) {   // rows past the sequence re-read the last row, keys past it the first chunk
 #pragma unroll
@@ -564,7 +565,7 @@ __device__ __forceinline__ void ptx_narrow(T *lds, unsigned wg, const T *__restr
             const int slot = r * 64 + lane, row = slot / XC, c = (slot % XC) ^ v_swizzle<D>(row);
             int pr = j * N_STEP + row;
             pr = pr >= S ? S - 1 : pr;
-            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + (int64_t)pr * D + c * 8), (lds_void_t *)(xdst + r * 64 * 8), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + (int64_t)pr * xrow + c * 8), (lds_void_t *)(xdst + r * 64 * 8), 16, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < PR; ++r) {
@@ -646,10 +647,10 @@ __device__ __forceinline__ void ptx_narrow(T *lds, unsigned wg, const T *__restr
 template <typename T, int D> constexpr int ptx_narrow_lds() { return 8 * N_STEP * D + 8 * N_STEP * N_ROWS; }   // elements
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_ptx_narrow_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
-                                                                   int causal, int heads, int nkb, int cus, float scale)
+                                                                   int causal, int heads, int nkb, int cus, float scale, int H, row_strides xs)
 {
     __shared__ __align__(16) T lds[ptx_narrow_lds<T, D>()];
-    ptx_narrow<T, D>(lds, blockIdx.x, P, X, O, S, causal, heads, nkb, cus, scale);
+    ptx_narrow<T, D>(lds, blockIdx.x, P, X, O, S, causal, heads, nkb, cus, scale, H, xs);
 }
 
 // Both products of one P, a workgroup of each in turns within an XCD: what a training step has left behind the gradient of the
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(256, 2) void causal_products_narrow_kernel(const T 
 {
     __shared__ __align__(16) T lds[ptx_narrow_lds<T, D>()];
     const unsigned wg = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
-    if (blockIdx.x & 8) ptx_narrow<T, D>(lds, wg, P, X, Ot, S, causal, heads, blocks, cus, scale);
+    if (blockIdx.x & 8) ptx_narrow<T, D>(lds, wg, P, X, Ot, S, causal, heads, blocks, cus, scale, heads, row_strides{0, (int64_t)S * D, D});
     else pv_narrow<T, D>(lds, wg, P, V, O, S, causal, heads, blocks, cus, nullptr, 1, 0, scale);
 }
 
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(256, 2) void causal_products_narrow_kernel(const T 
 template <typename T, int D, int RW, int GR, int PB>
 __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
                                                                          int causal, int heads, int nkb, int cus,
-                                                                         float scale)
+                                                                         float scale, int H, row_strides xs)
 {
     constexpr int XC = D / 8, KB = 16 * RW, PC = KB / 8, XT = PB * D, PT = PB * KB, GT = 64 * RW, XR = XT / 8 / GT, PR = PT / 8 / GT, DB = D / 16,
                   KS = PB / 32;
@@ -696,10 +697,11 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
     if (!longest_first(heads, nkb, cus, bh, kb)) return;
     const int k0 = kb * KB;   // (the first keys have the most query rows)
     const T *Pp = P + bh * (int64_t)S * S;
-    const T *Xp = X + bh * (int64_t)S * D;
+    const T *Xp = X + bh / H * xs.batch + bh % H * xs.head;
+    const int xrow = (int)xs.row;
     T *Op = O + bh * (int64_t)S * D;
 
-    const int xrow0 = tid / XC, xoff0 = xrow0 * D + ((tid % XC) ^ v_swizzle<D>(xrow0)) * 8;
+    const int xrow0 = tid / XC, xoff0 = xrow0 * xrow + ((tid % XC) ^ v_swizzle<D>(xrow0)) * 8;
     const int prow0 = tid / PC;
     int pchunk = (tid % PC) ^ v_swizzle<KB>(prow0);
     if (k0 + pchunk * 8 >= S) pchunk = 0;   // (keys past the sequence: rows of the result that nobody stores)
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
 #pragma unroll
         for (int r = 0; r < XR; ++r) {
             const int row = j * PB + xrow0 + r * (GT / XC), back = inside || row < S ? 0 : row - (S - 1);
-            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + ((int64_t)j * XT + xoff0 + (r * (GT / XC) - back) * D)),
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Xp + ((int64_t)j * PB * xrow + xoff0 + (r * (GT / XC) - back) * xrow)),
                                              (lds_void_t *)(xdst + (r * GT + wave * 64) * 8), 16, 0, 0);
         }
 #pragma unroll
@@ -838,11 +840,12 @@ template <typename F> bool product_grid(int64_t heads, int64_t S, int rows, int 
 }
 
 template <typename T, int D>
-int launch_t(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int causal, float scale, hipStream_t st)
+int launch_t(const void *p, const void *x, row_strides xs, void *o, int64_t B, int64_t H, int64_t S, int causal, float scale, hipStream_t st)
 {
     auto go = [&](auto kern, int rows, int threads, int resident) {
         const bool fits = product_grid(B * H, S, rows, resident, causal, [&](dim3 grid, int blocks, int cus) {
-            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, (int)(B * H), blocks, cus, scale);
+            hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)x, (T *)o, (int)S, causal, (int)(B * H), blocks, cus, scale, (int)H,
+                               xs);
         });
         return fits ? launch_status() : MTA_ERR_SHAPE;
     };
@@ -950,16 +953,24 @@ extern "C" int mta_causal_ptx_fwd(const void *p, const void *x, void *o, int64_t
 extern "C" int mta_causal_ptx_scaled_fwd(const void *p, const void *x, void *o, int64_t B, int64_t H, int64_t S, int64_t D, int causal,
                                          float scale, int io_dtype, void *stream)
 {
+    return mta_causal_ptx_rows_fwd(p, x, H * S * D, S * D, D, o, B, H, S, D, causal, scale, io_dtype, stream);
+}
+
+extern "C" int mta_causal_ptx_rows_fwd(const void *p, const void *x, int64_t x_batch, int64_t x_head, int64_t x_row, void *o, int64_t B, int64_t H,
+                                       int64_t S, int64_t D, int causal, float scale, int io_dtype, void *stream)
+{
     if (!p || !x || !o) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
     if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535) return MTA_ERR_SHAPE;
     if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
-    if (!aligned_to(p, 16) || !aligned_to(x, 16) || !aligned_to(o, 16)) return MTA_ERR_ALIGN;
-    if (io_dtype == MTA_F32 || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
+    if (!aligned_to(p, 16) || !aligned_to(x, 16) || !aligned_to(o, 16) || x_batch % 8 != 0 || x_head % 8 != 0 || x_row % 8 != 0) return MTA_ERR_ALIGN;
+    if (x_batch < 0 || x_head < 0 || x_row <= 0) return MTA_ERR_SHAPE;
+    if (io_dtype == MTA_F32 || S % 8 != 0 || x_row > (1 << 20)) return MTA_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
+    const row_strides xs{x_batch, x_head, x_row};
     if (io_dtype == MTA_BF16)
-        return D == 64 ? launch_t<bf16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<bf16_t, 128>(p, x, o, B, H, S, causal, scale, st);
-    return D == 64 ? launch_t<f16_t, 64>(p, x, o, B, H, S, causal, scale, st) : launch_t<f16_t, 128>(p, x, o, B, H, S, causal, scale, st);
+        return D == 64 ? launch_t<bf16_t, 64>(p, x, xs, o, B, H, S, causal, scale, st) : launch_t<bf16_t, 128>(p, x, xs, o, B, H, S, causal, scale, st);
+    return D == 64 ? launch_t<f16_t, 64>(p, x, xs, o, B, H, S, causal, scale, st) : launch_t<f16_t, 128>(p, x, xs, o, B, H, S, causal, scale, st);
 }
 
 // o = scale * P V and ot = scale * P^T X with the lower triangle of P (causal; else all of it)

@@ -138,6 +138,9 @@ inline int launch_status()
         else { using io_t = mta::f16_t; __VA_ARGS__; }                \
     } while (0)
 
+// where the rows of a (B,H,S,D) operand lie, in elements; row 0: contiguous
+struct row_strides { int64_t batch, head, row; };
+
 // conv_mix16.hip: depthwise conv + dense mixing of groups of 16 heads on the matrix cores; MTA_ERR_UNSUPPORTED when no
 // instance covers the arguments
 int conv_mix16_dispatch(const void *x, const void *wc, const void *wm, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,

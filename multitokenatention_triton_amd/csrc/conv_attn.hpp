@@ -18,6 +18,7 @@ struct conv_attn_args {
     int tri_gl;           // scores only: > 0 = triangular layout, groups of that many heads
     bool scores_only;
     hipStream_t st;
+    row_strides qs = {0, 0, 0};   // a 1x1 kernel's q where its rows do not follow one another
 };
 int conv_attn_mfma_bf16(const conv_attn_args &a);
 int conv_attn_mfma_f16(const conv_attn_args &a);

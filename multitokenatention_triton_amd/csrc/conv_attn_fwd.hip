@@ -458,6 +458,21 @@ extern "C" int mta_lower_scores_fwd(const void *a, const void *b, const void *fi
                                               (hipStream_t)stream});
 }
 
+extern "C" int mta_lower_scores_rows_fwd(const void *a, int64_t a_batch, int64_t a_head, int64_t a_row, const void *b, const void *first_visible,
+                                         void *out, int64_t B, int64_t H, int64_t S, int64_t D, int io_dtype, void *stream)
+{
+    if (!a || !b || !out) return MTA_ERR_NULL;
+    if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535 || a_batch < 0 || a_head < 0 || a_row <= 0) return MTA_ERR_SHAPE;
+    if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
+    if (!aligned_to(a, 16) || !aligned_to(b, 16) || !aligned_to(out, 16) || (first_visible && !aligned_to(first_visible, 4)) || a_batch % 8 != 0 ||
+        a_head % 8 != 0 || a_row % 8 != 0)
+        return MTA_ERR_ALIGN;
+    if (io_dtype == MTA_F32 || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
+    return conv_attn_mfma_dispatch(io_dtype, {a, b, nullptr, nullptr, out, nullptr, B, H, S, D, 1, 1, 1, 1.0f, 0, (const int *)first_visible, 0, true,
+                                              (hipStream_t)stream, {a_batch, a_head, a_row}});
+}
+
 // mta_qk_conv_fwd (causal) / mta_qk_conv_band_fwd (first_visible not NULL) with the scores stored in the triangular
 // layout (see tri_rowoff in common.hpp), groups of `group` heads interleaved by rows: B*H*tri_rowoff(S) elements, nothing
 // above the diagonal.

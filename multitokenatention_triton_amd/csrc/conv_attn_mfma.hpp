@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
                                                              float scale, int H, int nqb, int fill_upper, int64_t total_wg,
                                                              int64_t per_xcd, int jc_len, int items_per_bh, int hpx,
-                                                             item_table tbl, const int *__restrict__ band_lo, int tri_gl)
+                                                             item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
     using G = fused_geom<R, SK, NW>;
@@ -284,7 +284,9 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     }
     const int head = (int)(bh % H);
     const int q0 = qb * G::BQ;
-    const T *Qp = Q + bh * (int64_t)S * D;
+    const bool q_strided = RAW && qs.row != 0;
+    const T *Qp = Q + (q_strided ? bh / H * qs.batch + head * qs.head : bh * (int64_t)S * D);
+    const int64_t q_row = q_strided ? qs.row : D;
     const T *Kp = K + bh * (int64_t)S * D;
     const T *Vp = SCORES_ONLY ? Kp : V + bh * (int64_t)S * D;
     // (scores only, tri_gl > 0: the scores go out in the triangular layout, groups of tri_gl heads interleaved by rows;
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= S ? S - 1 : prow[rb]);
-            qf[rb][ks] = *reinterpret_cast<const frag8<T> *>(Qp + (int64_t)pc * D + ks * 32 + kg * 8);
+            qf[rb][ks] = *reinterpret_cast<const frag8<T> *>(Qp + pc * q_row + ks * 32 + kg * 8);
             if (prow[rb] < 0 || prow[rb] >= S) qf[rb][ks] = zero_frag<T>();  // rows outside the sequence are conv padding
         }
     }
@@ -809,7 +811,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
 
 template <typename T, int D, int R, int SK, bool SCORES_ONLY, bool BAND = false>
 int launch_mfma(const void *q, const void *k, const void *v, const void *w, void *o, float *lse, int64_t B, int64_t H,
-                int64_t S, int causal, float scale, int fill_upper, hipStream_t st, const int *band_lo = nullptr, int tri_gl = 0)
+                int64_t S, int causal, float scale, int fill_upper, hipStream_t st, const int *band_lo = nullptr, int tri_gl = 0,
+                row_strides qs = {0, 0, 0})
 {
     constexpr int NW = 4;
     constexpr int F_NT = 64 * NW;
@@ -879,7 +882,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     dim3 grid((unsigned)(per_xcd * 8));
     hipLaunchKernelGGL(kern, grid, dim3(F_NT), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
                        lse, (int)S, causal, scale, (int)H, nqb, fill_upper, total_wg, per_xcd, jc_len, (int)items_per_bh,
-                       (B * H) % 8 == 0 ? (int)(B * H / 8) : 0, tbl, band_lo, tri_gl);
+                       (B * H) % 8 == 0 ? (int)(B * H / 8) : 0, tbl, band_lo, tri_gl, qs);
     return launch_status();
 }
 
@@ -887,12 +890,12 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
 template <typename T, int D, bool SCORES_ONLY, bool BAND = false>
 int dispatch_mfma(const void *q, const void *k, const void *v, const void *w, void *o, float *lse, int64_t B, int64_t H,
                   int64_t S, int R, int Sk, int causal, float scale, int fill_upper, hipStream_t st, const int *band_lo = nullptr,
-                  int tri_gl = 0)
+                  int tri_gl = 0, row_strides qs = {0, 0, 0})
 {
     if constexpr (sizeof(T) == 2) {
         if constexpr (SCORES_ONLY) {   // no conv (weights are not read)
             if (R == 1 && Sk == 1)
-                return launch_mfma<T, D, 1, 1, true, BAND>(q, k, v, w, o, lse, B, H, S, causal, scale, fill_upper, st, band_lo, 0);
+                return launch_mfma<T, D, 1, 1, true, BAND>(q, k, v, w, o, lse, B, H, S, causal, scale, fill_upper, st, band_lo, 0, qs);
         }
 #define MTA_FUSED_CASE(r, s) \
     if (R == r && Sk == s) return launch_mfma<T, D, r, s, SCORES_ONLY, BAND>(q, k, v, w, o, lse, B, H, S, causal, scale, fill_upper, st, band_lo, tri_gl);
@@ -915,8 +918,8 @@ template <typename T, int D> int dispatch_mfma_d(const conv_attn_args &a)
 {
     if (!a.scores_only) return dispatch_mfma<T, D, false>(a.q, a.k, a.v, a.w, a.o, a.lse, a.B, a.H, a.S, a.R, a.Sk, a.causal, a.scale, 0, a.st);
     if (a.band_lo)
-        return dispatch_mfma<T, D, true, true>(a.q, a.k, nullptr, a.w, a.o, nullptr, a.B, a.H, a.S, a.R, a.Sk, 1, a.scale, a.fill_upper, a.st, a.band_lo, a.tri_gl);
-    return dispatch_mfma<T, D, true>(a.q, a.k, nullptr, a.w, a.o, nullptr, a.B, a.H, a.S, a.R, a.Sk, a.causal, a.scale, a.fill_upper, a.st, nullptr, a.tri_gl);
+        return dispatch_mfma<T, D, true, true>(a.q, a.k, nullptr, a.w, a.o, nullptr, a.B, a.H, a.S, a.R, a.Sk, 1, a.scale, a.fill_upper, a.st, a.band_lo, a.tri_gl, a.qs);
+    return dispatch_mfma<T, D, true>(a.q, a.k, nullptr, a.w, a.o, nullptr, a.B, a.H, a.S, a.R, a.Sk, a.causal, a.scale, a.fill_upper, a.st, nullptr, a.tri_gl, a.qs);
 }
 template <typename T> int dispatch_mfma_type(const conv_attn_args &a) { return a.D == 64 ? dispatch_mfma_d<T, 64>(a) : dispatch_mfma_d<T, 128>(a); }
 }  // namespace

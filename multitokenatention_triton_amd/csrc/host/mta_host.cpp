@@ -183,9 +183,14 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
     if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || !a.is_cuda() ||
         !lower_products_supported(a.scalar_type(), a.sizes(), true))
         return std::nullopt;
-    const Tensor x = on_gpu_vectors(a, "Q"), y = on_gpu_vectors(b, "K");
+    const bool in_place = rows_in_place(a);
+    const Tensor x = in_place ? a : on_gpu_vectors(a, "Q"), y = on_gpu_vectors(b, "K");
     Tensor out = at::empty({x.size(0), x.size(1), x.size(2), x.size(2)}, x.options());
-    check(mta_lower_scores_fwd(ptr(x), ptr(y), is16(x) ? ptr(first) : nullptr, out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
+    if (in_place)
+        check(mta_lower_scores_rows_fwd(ptr(x), x.stride(0), x.stride(1), x.stride(2), ptr(y), ptr(first), out_ptr(out), x.size(0), x.size(1), x.size(2),
+                                        x.size(3), code(x, "Q"), stream_of(x)),
+              "mta_lower_scores_fwd");
+    else check(mta_lower_scores_fwd(ptr(x), ptr(y), is16(x) ? ptr(first) : nullptr, out_ptr(out), x.size(0), x.size(1), x.size(2), x.size(3), code(x, "Q"), stream_of(x)),
           "mta_lower_scores_fwd");
     if (first) band_zero_(out, *first);
     return out;
@@ -494,10 +499,13 @@ Tensor values(const Tensor &m, const Tensor &v, bool lower, int64_t s_real, cons
     return heads_last(out, s_real == m.size(2) ? -1 : s_real);
 }
 
-// the incoming gradient as (B,H,S,D), padded with zero rows
-Tensor value_rows(const Tensor &grad, int64_t s_pad)
+// the incoming gradient as (B,H,S,D), padded with zero rows; a copy (6 us at B1 H16 S2048 D128 in 16 bits, and a launch of a small step)
+// only where rows are added or the products do not take rows where they lie
+Tensor value_rows(const Tensor &grad, int64_t s_pad, const Tensor &m, bool lower)
 {
     const Tensor go = grad.transpose(1, 2);
+    // (the lower-triangle kernels read 16-bit rows where they lie)
+    if (lower && go.dim() == 4 && go.size(2) == s_pad && go.scalar_type() == m.scalar_type() && rows_in_place(go)) return go;
     if (go.dim() != 4 || go.numel() >= (int64_t(1) << 31)) return go.contiguous();   // (beyond what a padded length is used for)
     RowsCopy rows(s_pad, OptTensor());
     const Tensor out = rows.add(go, false, 1.0);
@@ -582,7 +590,7 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
         const bool need_x = need[0] || need[1] || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
         variable_list out(11);
         Sums sums;
-        const Tensor go = value_rows(grads[0], s_pad);
+        const Tensor go = value_rows(grads[0], s_pad, m, lower);
         if (need[2]) out[2] = values_bwd_v(m, go, lower);
         if (need_c || need[6]) {
             Tensor dm = values_bwd_m(go, v, lower, first);
@@ -739,7 +747,7 @@ struct Values : torch::autograd::Function<Values> {
         const auto s = ctx->get_saved_variables();
         const c10::OptionalDeviceGuard guard(s[0].device());
         const bool lower = ctx->saved_data["lower"].toBool();
-        const Tensor go = value_rows(grads[0], s[0].size(2));
+        const Tensor go = value_rows(grads[0], s[0].size(2), s[0], lower);
         variable_list out(5);
         if (ctx->needs_input_grad(1)) out[1] = values_bwd_v(s[0], go, lower);
         if (ctx->needs_input_grad(0)) out[0] = values_bwd_m(go, s[1], lower, option(s[2]));

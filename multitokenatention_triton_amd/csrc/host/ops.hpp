@@ -320,15 +320,28 @@ inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, cons
     return o;
 }
 
+// whether the rows of a (B,H,S,D) tensor that is not contiguous can be read where they lie (16-bit data, whole 16-byte vectors)
+inline bool rows_in_place(const Tensor &x)
+{
+    return x.dim() == 4 && x.is_cuda() && is16(x) && !x.is_contiguous() && x.stride(3) == 1 && x.stride(2) > 0 && x.stride(2) <= (1 << 20) &&
+           x.stride(2) % 8 == 0 && x.stride(1) >= 0 && x.stride(1) % 8 == 0 && x.stride(0) >= 0 && x.stride(0) % 8 == 0 &&
+           reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 == 0;
+}
+
 inline OptTensor causal_ptx(const Tensor &p_, const Tensor &x_, bool causal, double scale)
 {
     if (p_.scalar_type() != x_.scalar_type() || !score_planes_of(p_.sizes(), x_.sizes()) ||
         !lower_products_supported(p_.scalar_type(), x_.sizes(), causal))
         return std::nullopt;
-    const Tensor p = on_gpu(p_, "P"), x = is16(x_) ? on_gpu(x_, "X") : on_gpu_vectors(x_, "X");
+    const bool in_place = rows_in_place(x_);
+    const Tensor p = on_gpu(p_, "P"), x = in_place ? x_ : is16(x_) ? on_gpu(x_, "X") : on_gpu_vectors(x_, "X");
     Tensor o = at::empty(x.sizes(), x.options());
     const int64_t b = x.size(0), h = x.size(1), s = x.size(2), d = x.size(3);
-    if (is16(p))
+    if (in_place)
+        check(mta_causal_ptx_rows_fwd(ptr(p), ptr(x), x.stride(0), x.stride(1), x.stride(2), out_ptr(o), b, h, s, d, causal, (float)scale, code(p, "P"),
+                                      stream_of(p)),
+              "mta_causal_ptx_fwd");
+    else if (is16(p))
         check(mta_causal_ptx_scaled_fwd(ptr(p), ptr(x), out_ptr(o), b, h, s, d, causal, (float)scale, code(p, "P"), stream_of(p)), "mta_causal_ptx_fwd");
     else
         check(mta_causal_ptx_f32(ptr(p), ptr(x), out_ptr(o), b, h, s, d, (float)scale, stream_of(p)), "mta_causal_ptx_f32");

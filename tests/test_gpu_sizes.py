@@ -426,6 +426,27 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128])
+def test_operands_read_where_their_rows_lie(pkg, d, dtype):
+    """P^T X and the lower scores with an operand laid out (B,S,H,D), a batch slice of one, and rows further apart: the bits that a
+    contiguous copy gives, for every form of the product."""
+    lib, code = pkg._lib.load(), {torch.bfloat16: 1, torch.float16: 2}[dtype]
+    st = torch.cuda.current_stream().cuda_stream
+    for b, h, s, apart in ((1, 1, 8, 0), (2, 8, 256, 0), (2, 3, 72, 8), (1, 16, 1096, 0), (2, 16, 1000, 0), (3, 16, 1024, 16), (4, 32, 784, 0)):
+        print(f"rows in place {b}x{h}x{s}x{d} {apart} {dtype}", flush=True)
+        x = torch.randn(b, s, h, d + apart, device="cuda").to(dtype)[..., :d].transpose(1, 2)
+        other = torch.randn(b, h, s, d, device="cuda").to(dtype)
+        p = torch.randn(b, h, s, s, device="cuda").to(dtype)
+        got, want = ([torch.zeros(b, h, s, n, dtype=dtype, device="cuda") for n in (d, s)] for _ in range(2))
+        y = x.contiguous()
+        assert lib.mta_causal_ptx_rows_fwd(p.data_ptr(), x.data_ptr(), *x.stride()[:3], got[0].data_ptr(), b, h, s, d, 1, 0.5, code, st) == 0
+        assert lib.mta_causal_ptx_scaled_fwd(p.data_ptr(), y.data_ptr(), want[0].data_ptr(), b, h, s, d, 1, 0.5, code, st) == 0
+        assert lib.mta_lower_scores_rows_fwd(x.data_ptr(), *x.stride()[:3], other.data_ptr(), None, got[1].data_ptr(), b, h, s, d, code, st) == 0
+        assert lib.mta_lower_scores_fwd(y.data_ptr(), other.data_ptr(), None, want[1].data_ptr(), b, h, s, d, code, st) == 0
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1].tril(), want[1].tril())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
 def test_both_products_of_a_matrix(pkg, d, dtype):
     """The two products in one call: the bits of the single ones, in one launch (grids of up to 256 blocks, heads that divide over the
     XCDs and that do not, one block, a last block in part) and in two; NaN above the diagonal."""
