@@ -15,8 +15,8 @@
 //           vector of key q is four products' operand);
 //   ptx:    contraction p = 4j + g, output row q = 2r + w of product w (P's pair), column d as above (X's vector)
 // (lane = 16g + r).  A line fetched by one lane's load is used up by its neighbours in the same instruction.
-// us against the library GEMM (scores / pv / ptx): B1 H4 S256 D64 5.8 / 5.5 / 5.5 against 24 / 21 / 22, where launching is all
-// there is; B1 H16 S512 11 / 8 / 9 against 21 / 20 / 21; B1 H32 S1024 38 / 38 / 31 against 55 / 36 / 35 (the library's operand
+// us against the library GEMM (scores / pv / ptx): B1 H4 S256 D64 3.9 / 4.4 / 5.5 against 24 / 21 / 22, where launching is all
+// there is; B1 H16 S512 10 / 8 / 9 against 21 / 20 / 21; B1 H32 S1024 38 / 38 / 31 against 55 / 36 / 35 (the library's operand
 // has to be filled above the diagonal first, which is another 15 us).
 #include "common.hpp"
 #include "mfma.hpp"
@@ -27,17 +27,16 @@ using namespace mta;
 
 __device__ __forceinline__ void mma4(f32x4 &c, float a, float b) { c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// ---- scores: a wavefront owns 32 query rows x 64 keys, a workgroup 64 x 128 -----------------------------------------------
-constexpr int SC_ROWS = 64, SC_KEYS = 128;
+// ---- scores: a wavefront owns 16 W query rows x 32 W keys, a workgroup 32 W x 64 W ----------------------------------------
+template <int W> constexpr int sc_rows() { return 32 * W; }
 
 // tiles on or below the diagonal of the first n rows of tiles, two tile rows per tile column
 __host__ __device__ __forceinline__ int sc_tiles(int n) { return (n / 2) * (n / 2 + 1) + (n & 1) * (n / 2 + 1); }
 
-template <int D>
+template <int D, int W>
 __global__ __launch_bounds__(256) void lower_scores_f32(const float *__restrict__ A, const float *__restrict__ Bm, float *__restrict__ C,
                                                         int S, int heads, int tiles, int cus)
 {
-    static_assert(SC_KEYS == 2 * SC_ROWS, "two tile rows per tile column");
     int bh, tile;
     if (!longest_first(heads, tiles, cus, bh, tile)) return;
     // tile row: the largest n with sc_tiles(n) <= tile
@@ -46,25 +45,25 @@ __global__ __launch_bounds__(256) void lower_scores_f32(const float *__restrict_
     while (sc_tiles(tr + 1) <= tile) ++tr;
     const int tc = tile - sc_tiles(tr);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int p0 = tr * SC_ROWS + (wave & 1) * 32, q0 = tc * SC_KEYS + (wave >> 1) * 64;
-    if (p0 >= S || q0 >= S || q0 > p0 + 31) return;   // (outside, or wholly above the diagonal)
+    const int p0 = tr * sc_rows<W>() + (wave & 1) * 16 * W, q0 = tc * 2 * sc_rows<W>() + (wave >> 1) * 32 * W;
+    if (p0 >= S || q0 >= S || q0 > p0 + 16 * W - 1) return;   // (outside, or wholly above the diagonal)
     const float *Ap = A + (int64_t)bh * S * D + g * 4, *Bp = Bm + (int64_t)bh * S * D + g * 4;
-    int arow[2], brow[4];
+    int arow[W], brow[2 * W];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) arow[i] = (p0 + 16 * i + r < S ? p0 + 16 * i + r : S - 1) * D;
+    for (int i = 0; i < W; ++i) arow[i] = (p0 + 16 * i + r < S ? p0 + 16 * i + r : S - 1) * D;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) brow[i] = (q0 + 16 * i + r < S ? q0 + 16 * i + r : S - 1) * D;
-    f32x4 acc[4][2];
+    for (int i = 0; i < 2 * W; ++i) brow[i] = (q0 + 16 * i + r < S ? q0 + 16 * i + r : S - 1) * D;
+    f32x4 acc[2 * W][W];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2 * W; ++i)
 #pragma unroll
-        for (int k = 0; k < 2; ++k) acc[i][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4 a[2][2], b[2][4];
+        for (int k = 0; k < W; ++k) acc[i][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 a[2][W], b[2][2 * W];
     auto fetch = [&](int s, int set) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[set][i] = *reinterpret_cast<const f32x4 *>(Ap + arow[i] + 16 * s);
+        for (int i = 0; i < W; ++i) a[set][i] = *reinterpret_cast<const f32x4 *>(Ap + arow[i] + 16 * s);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) b[set][i] = *reinterpret_cast<const f32x4 *>(Bp + brow[i] + 16 * s);
+        for (int i = 0; i < 2 * W; ++i) b[set][i] = *reinterpret_cast<const f32x4 *>(Bp + brow[i] + 16 * s);
     };
     fetch(0, 0);
 #pragma unroll
@@ -73,18 +72,18 @@ __global__ __launch_bounds__(256) void lower_scores_f32(const float *__restrict_
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 2 * W; ++i)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) mma4(acc[i][k], b[s & 1][i][t], a[s & 1][k][t]);
+                for (int k = 0; k < W; ++k) mma4(acc[i][k], b[s & 1][i][t], a[s & 1][k][t]);
     }
     // acc[i][k][v]: key q0 + 16i + 4g + v of query row p0 + 16k + r
     float *Cp = C + (int64_t)bh * S * S;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < W; ++k) {
         const int p = p0 + 16 * k + r;
         if (p >= S) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 2 * W; ++i) {
             const int q = q0 + 16 * i + 4 * g;
             if (q > p) continue;
             f32x4 o = acc[i][k];
@@ -196,14 +195,16 @@ __device__ __forceinline__ void reduce_waves(f32x4 *part, int wave, int lane, GE
     }
 }
 
-// ---- pv: a workgroup owns 32 query rows, its wavefronts every fourth step of 16 keys ---------------------------------------
-constexpr int RB = 2, PV_ROWS = 16 * RB;
+// ---- pv: a workgroup owns 16 query rows, its wavefronts every fourth step of 16 keys ---------------------------------------
+// (Short grids: a wavefront's chain of steps is what they wait for, and with 32 rows a step takes twice as long.  us, 32 rows | 16: B1
+// H4 S256 D64 5.5 | 4.4, S1024 12.2 | 8.2, B1 H8 S512 D128 11.6 | 7.5, B1 H16 S512 D64 8.4 | 7.7, B1 H4 S768 D128 15.7 | 9.7.)
+constexpr int RB = 1, PV_ROWS = 16 * RB;
 template <int D>
 __global__ __launch_bounds__(256, 2) void causal_pv_f32(const float *__restrict__ P, const float *__restrict__ V, float *__restrict__ O, int S,
                                                      int heads, int tiles, int cus, float scale)
 {
-    constexpr int NB = D / 64;
-    __shared__ f32x4 part[4 * 8 * 64];
+    constexpr int NB = D / 64, CH = 4 * RB * NB < 8 ? 4 * RB * NB : 8;
+    __shared__ f32x4 part[4 * CH * 64];
     int bh, tile;
     if (!longest_first(heads, tiles, cus, bh, tile)) return;
     const int p0 = (tiles - 1 - tile) * PV_ROWS;   // longest rows first
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(256, 2) void causal_pv_f32(const float *__restrict_
     }
     // vectors over u (four consecutive columns): acc[k][b][.][v] of row prow[k] is columns 64b + 16g + 4v .. + 3
     float *Op = O + (int64_t)bh * S * D;
-    reduce_waves<4 * RB * NB, 8>(part, wave, lane,
+    reduce_waves<4 * RB * NB, CH>(part, wave, lane,
         [&](int e) {
             const int k = e / (4 * NB), b = e / 4 % NB, v = e % 4;
             return f32x4{acc[k][b][0][v], acc[k][b][1][v], acc[k][b][2][v], acc[k][b][3][v]};
@@ -612,9 +613,11 @@ extern "C" int mta_lower_scores_f32(const void *a, const void *b, void *out, int
     if (scores_slabs(B * H * n * (n + 1) / 2))
         return D == 64 ? launch(lower_scores_f32_slabs<64>, B * H, n * (n + 1) / 2, 256, 0, (hipStream_t)stream, a, b, out, S)
                        : launch(lower_scores_f32_slabs<128>, B * H, n * (n + 1) / 2, 256, 0, (hipStream_t)stream, a, b, out, S);
-    const int64_t tiles = sc_tiles((int)((S + SC_ROWS - 1) / SC_ROWS));
-    return D == 64 ? launch(lower_scores_f32<64>, B * H, tiles, 256, 0, (hipStream_t)stream, a, b, out, S)
-                   : launch(lower_scores_f32<128>, B * H, tiles, 256, 0, (hipStream_t)stream, a, b, out, S);
+    // Grids that leave most of the chip idle: tiles of a quarter, whose wavefronts are done in a quarter of the time (us, 64 x 128 | 32 x 64:
+    // B1 H4 S256 D64 (24 workgroups of 64 x 128) 5.7 | 3.9, H8 (48) 5.7 | 3.9, H4 S512 (80) 6.2 | 5.2, H8 S512 (160) 6.4 | 6.8).
+    const int64_t large = sc_tiles((int)((S + sc_rows<2>() - 1) / sc_rows<2>())), small = sc_tiles((int)((S + sc_rows<1>() - 1) / sc_rows<1>()));
+    auto go = [&](auto d64, auto d128, int64_t tiles) { return launch(D == 64 ? d64 : d128, B * H, tiles, 256, 0, (hipStream_t)stream, a, b, out, S); };
+    return B * H * large <= 100 ? go(lower_scores_f32<64, 1>, lower_scores_f32<128, 1>, small) : go(lower_scores_f32<64, 2>, lower_scores_f32<128, 2>, large);
 }
 
 extern "C" int mta_causal_pv_f32(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D, float scale, void *stream)
@@ -625,7 +628,7 @@ extern "C" int mta_causal_pv_f32(const void *p, const void *v, void *o, int64_t 
     auto go = [&](auto d64, auto d128, int64_t blocks, int threads, int resident) {
         return launch(D == 64 ? d64 : d128, B * H, blocks, threads, resident, (hipStream_t)stream, p, v, o, S, scale);
     };
-    if (B * H * b32 <= 256) return go(causal_pv_f32<64>, causal_pv_f32<128>, b32, 256, 3);
+    if (B * H * b32 <= 256) return go(causal_pv_f32<64>, causal_pv_f32<128>, (S + PV_ROWS - 1) / PV_ROWS, 256, 3);
     if (B * H * b64 < 512) return go(causal_pv_f32_shared<64, 2, 4, 32>, causal_pv_f32_shared<128, 2, 4, 16>, b32, 512, 2);
     if (B * H * b64 < 768) return go(causal_pv_f32_shared<64, 4, 2, 64>, causal_pv_f32_shared<128, 4, 2, 32>, b64, 512, 2);
     return go(causal_pv_f32_shared<64, 4, 1, 64>, causal_pv_f32_shared<128, 4, 1, 32>, b64, 256, 4);

@@ -424,6 +424,23 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
         assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("s", [8, 100, 396, 512])
+def test_fp32_scores_by_tile(pkg, s, d):
+    """fp32 scores of 8 heads on tiles of 64 x 128 (of few: 32 x 64), of 2 heads at a time on tiles of 32 x 64: the same sums in the same
+    order, bit by bit, and nothing written above the diagonal beyond its vectors."""
+    lib, st = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    a, b = (torch.randn(1, 8, s, d, device="cuda") for _ in range(2))
+    whole, part = (torch.full((1, 8, s, s), 7.0, device="cuda") for _ in range(2))
+    assert lib.mta_lower_scores_f32(a.data_ptr(), b.data_ptr(), whole.data_ptr(), 1, 8, s, d, st) == 0
+    for h in range(0, 8, 2):
+        assert lib.mta_lower_scores_f32(a[0, h].data_ptr(), b[0, h].data_ptr(), part[0, h].data_ptr(), 1, 2, s, d, st) == 0
+    assert torch.equal(whole, part)
+    want = (a.double() @ b.double().transpose(2, 3)).tril()
+    size = (a.double().abs() @ b.double().abs().transpose(2, 3))
+    assert ((whole.double().tril() - want).abs() <= d * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128])
 def test_operands_read_where_their_rows_lie(pkg, d, dtype):
