@@ -2,9 +2,10 @@
 //
 // When causal, only keys q <= p of P are read: nothing above the diagonal is touched (it may be
 // uninitialised memory), which halves the traffic of the plain batched GEMM this replaces.
-// HBM-bound: the P triangle is streamed once, V blocks are re-read from L2.
+// What bounds it is the bytes through a CU's path to the L2: the P triangle once, V once per block of rows; product_form() says
+// which kernel a grid takes.
 //
-// P_WAVES wavefronts own a block of 32 query rows each; a wavefront owns two blocks of 16 rows.  O^T += V^T P^T on
+// The wide one: P_WAVES wavefronts own a block of 32 query rows each; a wavefront owns two blocks of 16 rows.  O^T += V^T P^T on
 // 16x16x32 MFMAs: lane (r = lane%16, g = lane/16) owns query row r of a block and supplies P^T
 // fragments straight from global memory (16 contiguous bytes = 8 keys of its row, loaded one key
 // block ahead), V blocks of 64 keys are copied global -> LDS asynchronously (double buffered,
