@@ -77,6 +77,17 @@ template <> struct vec_of<f16_t> { static constexpr int n = 8; };
 
 template <typename T> struct alignas(16) pack16 { T v[vec_of<T>::n]; };
 
+// zeros in the elements of a 16-byte vector at `key` that lie beyond `last`
+typedef unsigned int mta_u32x4 __attribute__((ext_vector_type(4)));
+template <typename T> __device__ __forceinline__ void zero_beyond(mta_u32x4 &v, int key, int last)
+{
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if constexpr (vec_of<T>::n == 8) v[u] &= (key + 2 * u <= last ? 0x0000ffffu : 0u) | (key + 2 * u + 1 <= last ? 0xffff0000u : 0u);
+        else v[u] &= key + u <= last ? 0xffffffffu : 0u;
+    }
+}
+
 // A 16-byte vector of a kernel's output.  `stream` (wavefront-uniform): non-temporal, past the caches - for tensors that the
 // kernel behind would not find there anyway; see streams().
 template <typename V> __device__ __forceinline__ void store_out(V *dst, const V &v, bool stream)

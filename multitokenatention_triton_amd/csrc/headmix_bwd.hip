@@ -48,16 +48,6 @@ template <bool STREAM> __device__ __forceinline__ u4 load_vec(const void *base, 
 }
 __device__ __forceinline__ u4 *vec_at(void *base, unsigned off) { return reinterpret_cast<u4 *>(static_cast<char *>(base) + off); }
 
-// zeros in the elements of a vector at `key` that lie beyond `last`
-template <typename T> __device__ __forceinline__ void zero_beyond(u4 &v, int key, int last)
-{
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        if constexpr (vec_of<T>::n == 8) v[u] &= (key + 2 * u <= last ? 0x0000ffffu : 0u) | (key + 2 * u + 1 <= last ? 0xffff0000u : 0u);
-        else v[u] &= key + u <= last ? 0xffffffffu : 0u;
-    }
-}
-
 // dword u of a vector as fp32 values (two of a 16-bit type), and back
 template <typename T> __device__ __forceinline__ void widen(unsigned v, float (&f)[vec_of<T>::n / 4])
 {

@@ -846,9 +846,9 @@ __global__ __launch_bounds__(256) void softmax_rows_wave(const T *__restrict__ x
                 if (fill_upper) __builtin_nontemporal_store(rs_u4{0u, 0u, 0u, 0u}, reinterpret_cast<rs_u4 *>(yr + q));
                 continue;
             }
-            // (keys beyond the last attended one carry probability 0 and come out as +0)
-            const rs_u4 out = {pack2<T>(sv[k][0] * inv, sv[k][1] * inv), pack2<T>(sv[k][2] * inv, sv[k][3] * inv),
-                               pack2<T>(sv[k][4] * inv, sv[k][5] * inv), pack2<T>(sv[k][6] * inv, sv[k][7] * inv)};
+            rs_u4 out = {pack2<T>(sv[k][0] * inv, sv[k][1] * inv), pack2<T>(sv[k][2] * inv, sv[k][3] * inv),
+                         pack2<T>(sv[k][4] * inv, sv[k][5] * inv), pack2<T>(sv[k][6] * inv, sv[k][7] * inv)};
+            if (q + VEC - 1 > last) zero_beyond<T>(out, q, last);  // +0 beyond the last attended key (0 * NaN where the row's sum is NaN)
             __builtin_nontemporal_store(out, reinterpret_cast<rs_u4 *>(yr + q));
         }
     }

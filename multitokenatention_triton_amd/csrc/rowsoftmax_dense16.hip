@@ -221,11 +221,10 @@ __global__ __launch_bounds__(64 * NW, 4) void mix16_softmax_kernel(const T *__re
                 for (int v = 0; v < 4; ++v) o[j][v] = s[i][j][v] * inv[v];
             }
         }
-        // (keys beyond the last attended one carry probability 0 and come out as +0)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const u32x4_t out = {pack2<T>(o[0][v], o[1][v]), pack2<T>(o[2][v], o[3][v]), pack2<T>(o[4][v], o[5][v]),
-                                 pack2<T>(o[6][v], o[7][v])};
+            u32x4_t out = {pack2<T>(o[0][v], o[1][v]), pack2<T>(o[2][v], o[3][v]), pack2<T>(o[4][v], o[5][v]), pack2<T>(o[6][v], o[7][v])};
+            if (key + 7 > last) zero_beyond<T>(out, key, last);  // (0 * NaN where the row's sum is NaN, 0 * inf in the second mix)
             __builtin_nontemporal_store(out, reinterpret_cast<u32x4_t *>(y + base + (int64_t)(kg * 4 + v) * plane + key));
         }
     }
@@ -502,8 +501,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
                 }
                 continue;
             }
-            // (keys beyond the last attended one carry probability 0 and come out as +0; above the diagonal they are
-            // stored on request only)  Two keys at a time, packed at once: few registers between product and store.
+            // Two keys at a time, packed at once: few registers between product and store.
             u32x4_t out[4];
 #pragma unroll
             for (int jp = 0; jp < 4; ++jp) {
@@ -524,6 +522,10 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
                 }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) out[v][jp] = pack2<T>(o[0][v], o[1][v]);
+            }
+            if (q0 + M16_TK - 1 > last) {  // +0 beyond the last attended key: 0 * NaN where the row's sum is NaN, 0 * inf in the second mix
+#pragma unroll
+                for (int v = 0; v < 4; ++v) zero_beyond<T>(out[v], key, last);
             }
             if (key < Q && (fill_upper || key <= last)) {
 #pragma unroll

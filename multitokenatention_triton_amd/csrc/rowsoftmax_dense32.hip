@@ -294,7 +294,10 @@ __global__ __launch_bounds__(64 * NW, (dense_waves<HB, NV, HAS2, MASKED>())) voi
             for (int t = 0; t < NS; ++t) out[t][j / 2] = pack2<T>(e[0][t], e[1][t]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        // (keys beyond the last attended one carry probability 0 and come out as +0)
+        if (tile(k) * TK + TK - 1 > last) {   // +0 beyond the last attended key: 0 * NaN where the row's sum is NaN, 0 * inf in the second mix
+#pragma unroll
+            for (int t = 0; t < NS; ++t) zero_beyond<T>(out[t], key, last);
+        }
         if (key >= Q || (key > last && !fill_upper)) continue;
 #pragma unroll
         for (int t = 0; t < NS; ++t)

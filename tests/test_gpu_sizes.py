@@ -722,3 +722,54 @@ def test_fp32_products_by_grid_size(pkg, heads, s, d):
     for entry, left in ((lib.mta_causal_pv_f32, lower), (lib.mta_causal_ptx_f32, lower.transpose(2, 3))):
         assert entry(pd.data_ptr(), x.data_ptr(), out.data_ptr(), 1, heads, s, d, 0.5, st) == 0
         assert ((out.cpu().double() - 0.5 * (left @ xd)).abs() <= s ** 0.5 * 2.0 ** -22 * 0.5 * (left.abs() @ xd.abs()) + 1e-30).all()
+
+
+def _bits(t):
+    return t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+
+
+# groups of heads (0: a softmax without weights) and rows for the kernels of the softmax stage: one tile, several, several wavefronts
+_SOFTMAX_GROUPS = (0, 2, 3, 4, 8, 9, 12, 16, 32)
+_SOFTMAX_ROWS = (20, 24, 136, 264, 1040)
+
+
+def _softmax_weights(group, dtype, g):
+    c = group or 2
+    w = [(torch.eye(c) + 0.2 * torch.randn(c, c, generator=g)).to(dtype).cuda() for _ in range(2)]
+    return c, ((None, None),) if group == 0 else ((w[0], None), (None, w[1]), (w[0], w[1]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", _SOFTMAX_GROUPS)
+def test_softmax_rows_that_are_not_finite_keep_the_fill(pkg, group, dtype):
+    """A row with a NaN, or with every attended key hidden by the bias, is NaN on and below the diagonal and +0 above it (left alone
+    or +0 without the fill); an infinity in the second weight stays below the diagonal; the other rows keep their bits."""
+    g = torch.Generator().manual_seed(67)
+    for s in _SOFTMAX_ROWS:
+        c, weights = _softmax_weights(group, dtype, g)
+        x = torch.randn(1, c, s, s, generator=g).to(dtype).cuda()
+        upper = torch.triu(torch.ones(s, s, dtype=torch.bool, device="cuda"), 1)
+        rows = torch.tensor([1, s // 3, s // 2, s - 2], device="cuda")
+        others = torch.ones(s, dtype=torch.bool, device="cuda")
+        others[rows] = False
+        bad = x.clone()
+        bad[0, 0, rows, rows // 2] = float("nan")
+        bias = torch.zeros(1, s, device="cuda")
+        bias[0, :s // 2] = float("-inf")
+        for w1, w2 in weights:
+            print(f"softmax of NaN group={group} s={s} {w1 is not None} {w2 is not None} {dtype}", flush=True)
+            run = lambda t, v2=w2, **k: pkg.ops.headmix_softmax(t, w1, v2, True, group_size=group, **k)  # noqa: E731
+            got, clean = run(bad), run(x)
+            assert (_bits(got)[..., upper] == 0).all()
+            mixed = slice(None) if w1 is not None or w2 is not None else slice(0, 1)   # (one weight mixes the NaN into every head)
+            assert got[0, mixed][:, rows][..., ~upper[rows]].isnan().all()
+            assert torch.equal(_bits(got)[:, :, others], _bits(clean)[:, :, others])
+            above = run(bad, fill_upper=False, out=torch.full_like(x, 7.0))[..., upper]
+            assert ((above == 7.0) | (_bits(above) == 0)).all()
+            hidden = run(x, key_bias=bias)
+            assert (_bits(hidden)[..., upper] == 0).all() and hidden[:, :, :s // 2][..., ~upper[:s // 2]].isnan().all()
+            assert torch.isfinite(hidden[:, :, s // 2:]).all()
+            if w2 is not None:
+                w_inf = w2.clone()
+                w_inf[0, c - 1] = float("inf")
+                assert (_bits(run(x, w_inf))[..., upper] == 0).all()

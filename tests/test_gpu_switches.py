@@ -14,8 +14,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 GROUPS = [
     # vector-ALU head mixing for 16 and 32 heads; the general softmax and fused kernels for 16-bit data
     ({"MTA_HEADMIX_NO_MFMA": "1", "MTA_SOFTMAX_NO_PACKED": "1", "MTA_FUSED_FORCE_GENERAL": "1"},
-     ["tests/test_gpu_ops.py", "tests/test_gpu_attention.py"],
-     "test_headmix_parity or (test_mix_softmax_mix_parity and not f32 and not (case12 or case13 or case14 or case15 or case16 or case17 or case18)) or test_conv_attention_parity "
+     ["tests/test_gpu_ops.py", "tests/test_gpu_attention.py", "tests/test_gpu_sizes.py"],
+     "(test_softmax_rows and ([4-dtype1] or [8-dtype2])) or test_headmix_parity or (test_mix_softmax_mix_parity and not f32 and not (case12 or case13 or case14 or case15 or case16 or case17 or case18)) or test_conv_attention_parity "
      "or test_mta_general"),   # (the cases of groups of 16 heads run the same kernel under these switches: left out)
     # another cut of the scores kernel's work items (long / short items of 20 / 7 key blocks, 30 % of a key range short)
     ({"MTA_QK_CHUNK_LONG": "20", "MTA_QK_CHUNK_SHORT": "7", "MTA_QK_SHORT_PERCENT": "30"},
@@ -38,7 +38,7 @@ GROUPS = [
      "or test_mta_use_mask_key or test_mta_general"),
     # the softmax without weights with a workgroup per row (by default short rows take a wavefront per row)
     ({"MTA_SOFTMAX_NO_WAVE_ROWS": "1"}, ["tests/test_gpu_ops.py"], "test_mix_softmax_mix_parity and not f32 and (case21 or case22 or case23)"),
-    ({"MTA_MIX16_NO_ROW_LISTS": "1"}, ["tests/test_gpu_ops.py"], "(test_mix_softmax_mix_parity and not f32 and (case12 or case13 or case14 or case15 or case18)) or test_mix_softmax_mix_dense16"),
+    ({"MTA_MIX16_NO_ROW_LISTS": "1"}, ["tests/test_gpu_ops.py", "tests/test_gpu_sizes.py"], "(test_softmax_rows_that and ([16-dtype1] or [16-dtype2])) or (test_mix_softmax_mix_parity and not f32 and (case12 or case13 or case14 or case15 or case18)) or test_mix_softmax_mix_dense16"),
     # (the cases with groups of 16 heads, rows of up to 3000 keys: all three kinds of rows)
 ]
 
