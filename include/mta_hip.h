@@ -146,7 +146,8 @@ int mta_headmix_softmax_bias_fwd(const void *x, const void *w1, const void *w2, 
  * mixed score becomes -inf ahead of the softmax) when q < first_visible[n, p]; NULL = no band (identical to the entry
  * point above).  With the causal rule this is the `scores + mask` of mta_attention_triton.py:77-78 for every mask of
  * the form "row p sees the keys first_visible[p] .. p" - sliding windows, packed documents - without the (B,H,S,S)
- * mask tensor.  key_bias may be given as well.  A row without a visible key comes out as NaN. */
+ * mask tensor.  key_bias may be given as well.  A row without a visible key (first_visible[n, p] beyond its last attended
+ * key) is NaN at every attended key. */
 int mta_headmix_softmax_band_fwd(const void *x, const void *w1, const void *w2, const void *key_bias,
                                  const void *first_visible, void *y, int64_t N, int64_t C, int64_t P, int64_t Q,
                                  int group_size, int causal, int fill_upper, int io_dtype, int w_dtype, void *stream);

@@ -77,6 +77,16 @@ template <> struct vec_of<f16_t> { static constexpr int n = 8; };
 
 template <typename T> struct alignas(16) pack16 { T v[vec_of<T>::n]; };
 
+// The first visible key of a query row under a band mask, `last`: its last attended key; last + 1: the row sees none.
+__device__ __forceinline__ int first_key(const int *row_lo, int64_t row, int last)
+{
+    const int lo = row_lo[row];
+    return lo < 0 ? 0 : lo > last ? last + 1 : lo;
+}
+// What a 16-byte vector of keys that a band mask hides holds behind the softmax: +0, or, in a row that sees none, NaN (in
+// every type), as the softmax of -inf gives.
+__device__ __forceinline__ unsigned hidden_bits(int lo, int last) { return lo > last ? 0x7fc07fc0u : 0u; }
+
 // zeros in the elements of a 16-byte vector at `key` that lie beyond `last`
 typedef unsigned int mta_u32x4 __attribute__((ext_vector_type(4)));
 template <typename T> __device__ __forceinline__ void zero_beyond(mta_u32x4 &v, int key, int last)

@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G < 8 && G * NV == 8) ? RS
     // computed (its outputs are +0)
     int lo = 0;
     if constexpr (KB) {
-        if (row_lo) lo = row_lo[n * P + p];
+        if (row_lo) lo = first_key(row_lo, n * P + p, last);
     }
     auto hid = [&](int k) { return KB && (k * NT + wave * 64 + 64) * VEC <= lo; };
     auto gone = [&](int k) { return dead(k) || hid(k); };
@@ -325,11 +325,11 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G < 8 && G * NV == 8) ? RS
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int q = (k * NT + tid) * VEC;
-        if (hid(k) && !dead(k)) {  // pass wholly ahead of the row's first visible key: +0
+        if (hid(k) && !dead(k)) {  // pass wholly ahead of the row's first visible key: +0, NaN if there is none
             if (q < Q) {
-                V z;
-#pragma unroll
-                for (int u = 0; u < VEC; ++u) z.v[u] = from_float<T>(0.0f);
+                static_assert(sizeof(V) == 16, "whole vectors");
+                const unsigned h = hidden_bits(lo, last);
+                const V z = __builtin_bit_cast(V, mta_u32x4{h, h, h, h});
 #pragma unroll
                 for (int o = 0; o < G; ++o) store_any(reinterpret_cast<V *>(y + base + o * plane + q), z, stream);
             }
@@ -543,12 +543,12 @@ __global__ __launch_bounds__(NT, OCC) void mix_softmax_mix_packed(
     const int nlw = last / (64 * VEC) + 1 < NW ? last / (64 * VEC) + 1 : NW;
     int lo = 0, flw = 0;  // band mask: first visible key, and the wavefront whose slice holds it
     if constexpr (BAND) {
-        lo = row_lo[n * P + p];
-        lo = lo < 0 ? 0 : lo;
+        lo = first_key(row_lo, n * P + p, last);
         flw = lo / (64 * VEC) < nlw - 1 ? lo / (64 * VEC) : nlw - 1;  // (a row that sees no key: NaN from the last slice)
-        if (wave < flw) {  // slice wholly ahead of the first visible key (and below the diagonal): +0
+        if (wave < flw) {  // slice wholly ahead of the first visible key (and below the diagonal): +0, NaN if there is none
             const int q = tid * VEC;
-            const rs_u4 z = {0u, 0u, 0u, 0u};
+            const unsigned h = hidden_bits(lo, last);
+            const rs_u4 z = {h, h, h, h};
 #pragma unroll
             for (int o = 0; o < G; ++o) store_out(reinterpret_cast<rs_u4 *>(y + base + o * plane + q), z, stream);
             return;

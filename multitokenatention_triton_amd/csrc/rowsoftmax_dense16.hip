@@ -242,7 +242,7 @@ __global__ __launch_bounds__(64 * NW, 4) void mix16_softmax_kernel(const T *__re
 // MASKED instances: key_bias (fp32 (N,Q), or NULL) is added to the mixed, rounded scores and the sum rounded again (the
 // reference's `scores + mask` for one value per key; the batch entry's bias row waits in LDS); row_lo (int32 (N,P), or
 // NULL) is the first key a row sees (band mask): the keys ahead of it count as -inf, and a tile that lies wholly ahead of
-// it is neither copied nor computed - it is stored as +0.
+// it is neither copied nor computed - it is stored as +0 (as NaN where the row sees no key).
 template <typename T, bool HAS1, bool HAS2, bool MASKED = false>
 __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(const T *__restrict__ x, const T *__restrict__ w1,
                                                                            const T *__restrict__ w2, T *__restrict__ y, int C,
@@ -297,11 +297,10 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
     __syncthreads();  // (also: nothing is in flight when the loop starts counting)
     // first visible key of row p (0 without a band mask)
     auto lo_of = [&](int p) {
-        int lo = 0;
         if constexpr (MASKED) {
-            if (row_lo && p >= 0) lo = row_lo[n * P + p];
+            if (row_lo && p >= 0) return first_key(row_lo, n * P + p, causal && p < Q - 1 ? p : Q - 1);
         }
-        return lo < 0 ? 0 : lo;
+        return 0;
     };
 
     // (ln, kg: the lane's key octet and head quad, handed in by the loop: see there)
@@ -440,7 +439,7 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
                 const f32x4 q4 = src[c];
                 r = fmaxf(fmaxf(r, fmaxf(q4[0], q4[1])), fmaxf(q4[2], q4[3]));
             }
-            m[v] = r;  // finite: the row's first key is always attended
+            m[v] = r;  // (finite, but for the rows of which a mask hides every key)
         }
 
         // ---- exponentials and their sums ----
@@ -492,9 +491,10 @@ __global__ __launch_bounds__(64 * M16_NW, 1) void mix16_softmax_rows_kernel(cons
             const int key = q0 + ln * 8;
             if (!active || q0 >= Q || (q0 > last && !fill_upper)) continue;  // (wavefront-uniform; lane 0 of the others stores)
             nst += 4;
-            if (q0 > last || q0 + M16_TK <= lo) {  // (wavefront-uniform) wholly above the diagonal, stored on request, or wholly hidden: +0
+            if (q0 > last || q0 + M16_TK <= lo) {  // (wavefront-uniform) wholly above the diagonal, stored on request, or wholly hidden: +0 (NaN)
                 if (key < Q) {
-                    const u32x4_t z = {0u, 0u, 0u, 0u};
+                    const unsigned h = MASKED && q0 <= last ? hidden_bits(lo, last) : 0u;
+                    const u32x4_t z = {h, h, h, h};
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
                         store_out(reinterpret_cast<u32x4_t *>(yrow + ((unsigned)(kg * 4 + v) * yplane + (unsigned)key) * (unsigned)sizeof(T)), z, stream);

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64 * NW, (dense_waves<HB, NV, HAS2, MASKED>())) voi
     const int64_t n = b / groups;
     const int64_t plane = (int64_t)P * Q, base = (n * C + (int64_t)g * HG) * plane + (int64_t)p * Q;
     const int last = causal ? (p < Q - 1 ? p : Q - 1) : Q - 1;   // last attended key
-    const int lo = MASKED && row_lo ? row_lo[n * P + p] : 0;     // band mask: first visible key
+    const int lo = MASKED && row_lo ? first_key(row_lo, n * P + p, last) : 0;   // band mask: first visible key
     // tiles with a visible key: [first, end)
     const int first = lo / TK, end = last / TK + 1;
     auto tile = [&](int k) { return k * NW + wave; };
@@ -95,11 +95,12 @@ __global__ __launch_bounds__(64 * NW, (dense_waves<HB, NV, HAS2, MASKED>())) voi
     for (int k = 0; k < NV; ++k) {
         any |= live(k);
         if (live(k)) continue;
-        const int key = tile(k) * TK + 8 * ln;   // +0 ahead of the visible keys, and beyond the attended ones on request
+        const int key = tile(k) * TK + 8 * ln;   // +0 (NaN) ahead of the visible keys, and +0 beyond the attended ones on request
         if (key >= Q || (key > last && !fill_upper)) continue;
+        const unsigned z = tile(k) < end ? hidden_bits(lo, last) : 0u;
 #pragma unroll
         for (int t = 0; t < NS; ++t)
-            if (head(t) < HG) store_out(at(y, t, key), u32x4{0u, 0u, 0u, 0u}, stream);
+            if (head(t) < HG) store_out(at(y, t, key), u32x4{z, z, z, z}, stream);
     }
     if (!any) return;
 

@@ -32,7 +32,7 @@ __global__ __launch_bounds__(64 * NW) void mix_softmax_dense_f32(const float *__
     const int64_t n = b / groups;
     const int64_t plane = (int64_t)P * Q, base = (n * C + (int64_t)g * HG) * plane + (int64_t)p * Q;
     const int last = causal ? (p < Q - 1 ? p : Q - 1) : Q - 1;   // last attended key
-    const int lo = row_lo ? row_lo[n * P + p] : 0;               // band mask: first visible key
+    const int lo = row_lo ? first_key(row_lo, n * P + p, last) : 0;   // band mask: first visible key
     auto head = [&](int t) { return 16 * (t >> 2) + 4 * kg + (t & 3); };
     auto key0 = [&](int k) { return (k * NW + wave) * 64; };
     // a pass wholly beyond the attended keys, or wholly ahead of the first visible one, is neither read nor computed
@@ -166,8 +166,9 @@ __global__ __launch_bounds__(64 * NW) void mix_softmax_dense_f32(const float *__
         const int key = key0(k) + 4 * ln;
         f32x4 out[NS];
         if (gone(k)) {
+            const float z = dead(k) ? 0.0f : __uint_as_float(hidden_bits(lo, last));
 #pragma unroll
-            for (int t = 0; t < NS; ++t) out[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int t = 0; t < NS; ++t) out[t] = f32x4{z, z, z, z};
         } else {
 #pragma unroll
             for (int t = 0; t < NS; ++t)   // (what is no head has weight 0 and must be finite: its row sums are over zeros)

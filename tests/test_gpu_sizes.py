@@ -773,3 +773,31 @@ def test_softmax_rows_that_are_not_finite_keep_the_fill(pkg, group, dtype):
                 w_inf = w2.clone()
                 w_inf[0, c - 1] = float("inf")
                 assert (_bits(run(x, w_inf))[..., upper] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", _SOFTMAX_GROUPS)
+def test_softmax_rows_without_a_visible_key(pkg, group, dtype):
+    """Rows whose first visible key lies behind their last one, at every place in a tile: NaN at all keys up to the diagonal, as the
+    softmax of -inf is, and the fill above it; the other rows keep their bits.  In (N,C,S,S) planes and in the triangular layout."""
+    g = torch.Generator().manual_seed(71)
+    for s in _SOFTMAX_ROWS:
+        c, weights = _softmax_weights(group, dtype, g)
+        x = torch.randn(1, c, s, s, generator=g).to(dtype).cuda()
+        p = torch.arange(s, device="cuda")
+        upper, empty = p[None, :] > p[:, None], p % 4 != 0      # (p + 1 = 64, 128, 256, ... among the empty rows)
+        first = torch.where(empty, p + 1 + 3 * (p % 4 == 2), p // 2).int()[None]
+        seen = torch.where(empty, 0, p // 2).int()[None]
+        for bias in (None, torch.full((1, s), 0.25, device="cuda")):
+            for w1, w2 in weights:
+                print(f"softmax of nothing group={group} s={s} {w1 is not None} {w2 is not None} bias={bias is not None} {dtype}", flush=True)
+                run = lambda lo: pkg.ops.headmix_softmax(x, w1, w2, True, group_size=group, key_bias=bias, first_visible=lo)  # noqa: E731
+                got, want = run(first), run(seen)
+                assert (_bits(got)[..., upper] == 0).all()
+                assert got[:, :, empty][..., ~upper[empty]].isnan().all()
+                assert torch.equal(_bits(got)[:, :, ~empty], _bits(want)[:, :, ~empty])
+                code = pkg.ops._code(x, "input")
+                if group and pkg._lib.load().mta_headmix_softmax_tri_supported(c, s, group, 0, code, code, w1 is not None, w2 is not None, 1, bias is not None):
+                    tri = pkg.ops.headmix_softmax_tri(pkg.ops.tri_pack(x, group), w1, w2, 1, c, s, group, key_bias=bias, first_visible=first)
+                    tri = pkg.ops.tri_unpack(tri, 1, c, s, group)[..., ~upper]
+                    assert torch.equal(tri.nan_to_num(7.0), got[..., ~upper].nan_to_num(7.0))
