@@ -413,7 +413,7 @@ int mta_softmax_headmix_grads_partials(const void *s, const void *ds, const void
 
 /* mta_headmix_bwd_input and mta_headmix_bwd_weight_as in one pass over x and dy: dx and dw as those two define them (dw 0 outside
  * the groups).  Mixing groups of 2, 4, 8, 12, 16 and 32 heads, Q of whole 16-byte vectors, x, dy and dx aligned to them, 16-bit
- * data of groups of 12 and more with weights of the same dtype; MTA_ERR_UNSUPPORTED otherwise, and where
+ * data of groups of 8 and more with weights of the same dtype; MTA_ERR_UNSUPPORTED otherwise, and where
  * mta_headmix_grads_workspace (device memory, as for the weight gradients) returns 0. */
 int64_t mta_headmix_grads_workspace(int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causal, int with_softmax,
                                     int io_dtype, int w_dtype);

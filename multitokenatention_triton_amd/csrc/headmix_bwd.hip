@@ -26,7 +26,10 @@
 //
 // In the kernels behind the softmax gradient a row's workgroup walks "load, sum, barrier, load x, products, store".  Measured
 // and not kept (bf16 B1 H16 S2048, 66 us): x loaded ahead of the barrier 69, the next row's vectors loaded ahead 120 (they spill),
-// 16 wavefronts of one tile instead of 8 of two 66.
+// 16 wavefronts of one tile instead of 8 of two 66.  Four tiles per wavefront (rows of more than 2048 keys, fp32 1024) hold 256
+// registers and spill: 104 to 120 bytes a lane with 12 and 16 heads in 16 bits, 52 with 16 in fp32; so do 32 heads in 16 bits, 8 bytes
+// with one tile and 44 with two.  With the tile-at-a-time order below that is what is left; B1 H16 S4096 runs at 3.7 TB/s all the same
+// (4.1 at S2048, which does not spill).
 #include "common.hpp"
 #include "mfma.hpp"
 
@@ -157,7 +160,7 @@ template <int KEYS> struct chunk_walk {
     }
 };
 
-// ---- groups of 2, 4 or 8 heads: a lane holds them all ----------------------------------------------------------------------
+// ---- groups of 2 or 4 heads: a lane holds them all -------------------------------------------------------------------------
 // The group's weights in scalar registers: fp32 values w[o][i], or (PAIRS: 16-bit data, weights of the same dtype) the pairs
 // (w[2j][i], w[2j+1][i]) that the packed dot products take.
 template <typename T, int G, bool PAIRS> struct lane_weights {
@@ -404,7 +407,7 @@ __global__ __launch_bounds__(512) void lane_softmax_grads(const T *__restrict__ 
     }
 }
 
-// ---- groups of 12, 16 or 32 heads: matrix cores ------------------------------------------------------------------------------
+// ---- groups of 8, 12, 16 or 32 heads: matrix cores ---------------------------------------------------------------------------
 template <typename T, int HG> struct dense {
     static constexpr int V = vec_of<T>::n;
     static constexpr bool F32 = V == 4;

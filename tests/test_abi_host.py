@@ -133,6 +133,25 @@ def test_triangular_layout_entry_points_validate_and_answer_on_the_host():
     assert ops.tri_row_offset(65) == 4096 + 128 and ops.tri_row_offset(4096) == sum(64 * (r // 64 + 1) for r in range(4096))
 
 
+def test_one_pass_head_mixing_gradients_exist_for_what_the_header_names():
+    """Groups of 2, 4, 8, 12, 16 and 32 heads, rows of whole vectors; 16-bit data of groups of 8 and more with weights of the same
+    dtype; behind the softmax gradient rows of up to 4096 keys (32 heads: 2048), fp32 half as many."""
+    ask = _lib.load().mta_headmix_grads_workspace   # (N, C, P, Q, group, causal, with_softmax, io, w); dtypes 0 fp32, 1 bf16, 2 fp16
+    for softmax in (0, 1):
+        for group in range(1, 40):
+            known = group in (2, 4, 8, 12, 16, 32)
+            for io, w in ((0, 0), (0, 1), (1, 1), (2, 2), (1, 0), (2, 0), (1, 2)):
+                takes = known and (group < 8 or io == 0 or w == io)
+                assert (ask(1, 2 * group, 64, 64, group, 1, softmax, io, w) > 0) == takes, (softmax, group, io, w)
+                assert ask(1, 2 * group, 64, 64 - 2, group, 1, softmax, io, w) == 0
+            if known:
+                longest = 2048 if group == 32 else 4096
+                for io in (0, 1):
+                    most = longest // 2 if io == 0 else longest
+                    assert ask(1, group, 8, most, 0, 0, softmax, io, io) > 0
+                    assert (ask(1, group, 8, most + 8, 0, 0, softmax, io, io) > 0) == (not softmax)
+
+
 def test_check_maps_codes_to_exceptions():
     with pytest.raises(ValueError, match="kernel size"):
         _lib.check(-4, "x")
