@@ -192,26 +192,31 @@ def headmix_grads(dy: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, causa
                   probs: Optional[torch.Tensor] = None, fill_upper: bool = True, out: Optional[torch.Tensor] = None):
     """Both gradients of ``headmix`` (input, weight in its dtype) in one pass; with ``probs``, dy is the gradient of the softmax
     that follows and the result above the diagonal is unwritten.  None where there is no kernel; see mta_headmix_grads."""
-    dy, x, weight = _device_tensor(dy, "grad_output"), _device_tensor(x, "input"), _device_tensor(weight, "weight")
+    dy, x, weight = _device_tensor(dy, "grad_output"), _device_tensor(x, "input"), _device_tensor(weight.detach(), "weight")
     if x.dim() != 4 or x.shape != dy.shape or x.dtype != dy.dtype:
         raise ValueError("input and grad_output must be (N,C,P,Q) tensors of one shape and dtype")
     n, c, p, q = x.shape
+    assert tuple(weight.shape) == (c, c), f"Weight must be ({c},{c}), got {tuple(weight.shape)}"
+    if probs is not None:
+        probs = _device_tensor(probs, "probabilities")
+        if probs.shape != x.shape or probs.dtype != x.dtype:
+            raise ValueError("probabilities and input must share shape and dtype")
+    if len({t.device for t in (dy, x, weight, x if probs is None else probs)}) > 1:
+        raise ValueError("input, grad_output, weight and probabilities must lie on one device")
+    dx = _out_like(x, out)
     lib, group = _lib.load(), int(group_size or 0)
     mode = _causal_mode(causal, fill_upper)
     codes = _code(x, "input"), _code(weight, "weight")
     nbytes = lib.mta_headmix_grads_workspace(n, c, p, q, group, mode, int(probs is not None), *codes)
     if nbytes <= 0:
         return None
-    dx, dw = torch.empty_like(x) if out is None else out, torch.empty_like(weight)
+    dw = torch.empty_like(weight)
     ws = _workspace(nbytes, x.device)
     with torch.cuda.device(x.device):
         if probs is None:
             rc = lib.mta_headmix_grads(x.data_ptr(), dy.data_ptr(), weight.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(),
                                        n, c, p, q, group, mode, *codes, _stream(x))
         else:
-            probs = _device_tensor(probs, "probabilities")
-            if probs.shape != x.shape or probs.dtype != x.dtype:
-                raise ValueError("probabilities and input must share shape and dtype")
             rc = lib.mta_softmax_headmix_grads(probs.data_ptr(), dy.data_ptr(), x.data_ptr(), weight.data_ptr(), dx.data_ptr(), dw.data_ptr(),
                                                ws.data_ptr(), ws.numel(), n, c, p, q, group, int(bool(causal)), *codes, _stream(x))
     if rc == _lib.MTA_ERR_UNSUPPORTED:

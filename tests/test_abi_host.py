@@ -152,6 +152,22 @@ def test_one_pass_head_mixing_gradients_exist_for_what_the_header_names():
                     assert (ask(1, group, 8, most + 8, 0, 0, softmax, io, io) > 0) == (not softmax)
 
 
+def test_head_mixing_gradients_check_what_the_kernel_indexes(monkeypatch):
+    """A head weight that is not (C,C), probabilities or a result of another shape, dtype or layout: refused ahead of the library."""
+    monkeypatch.setattr(ops, "_device_tensor", lambda t, what: t)   # (no GPU here: the tensors stay on the CPU)
+    x = torch.zeros(1, 8, 16, 16)
+    w = torch.eye(8)
+    for weight in (torch.eye(4), torch.eye(16), torch.zeros(8, 4), torch.zeros(8)):
+        with pytest.raises(AssertionError, match=r"Weight must be \(8,8\)"):
+            ops.headmix_grads(x, x, weight)
+    for out in (torch.zeros(1, 8, 16, 8), torch.zeros(1, 8, 16, 16, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 32)[..., ::2], torch.zeros(1, 16, 8, 16).transpose(1, 2)):
+        with pytest.raises(ValueError, match="out must be"):
+            ops.headmix_grads(x, x, w, out=out)
+    for probs in (torch.zeros(1, 8, 16, 8), torch.zeros(1, 8, 16, 16, dtype=torch.float16)):
+        with pytest.raises(ValueError, match="probabilities and input"):
+            ops.headmix_grads(x, x, w, probs=probs)
+
+
 def test_check_maps_codes_to_exceptions():
     with pytest.raises(ValueError, match="kernel size"):
         _lib.check(-4, "x")
