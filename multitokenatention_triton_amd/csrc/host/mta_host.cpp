@@ -48,12 +48,16 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 // 544 (B2 S1008) 101.0 | 88.3 / 106.4 | 95.6, 600 (B1 S1536) 109.9 | 91.9 / 115.9 | 98.3, 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3,
 // 840 (B2 S1280) 126.1 | 123.9 / 131.8 | 133.3, 1056 (B1 S2048) 155.0 | 164.5 / 161.5 | 175.5, 1088 (B4 S1024) 149.8 | 171.4 /
 // 156.9 | 182.6; the runs of one side differ by up to 2.
-// A whole round is as good: 440 tiles (B4 S640, groups of 4, the two stages alone) 28.8 | 34.8 / 32.3 | 37.6.  Groups of 2 or 4 heads:
-// 1056 tiles 57 | 60 / 64 | 62, 2112 (B2 S2048) 92 | 120 / 98 | 125, 4160 (B1 S4096) 148 | 232 / 163 | 238.
-bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only)
+// Groups of 2 or 4 heads: 1056 tiles 57 | 60 / 64 | 62, 2112 (B2 S2048) 92 | 120 / 98 | 125, 4160 (B1 S4096) 148 | 232 / 163 | 238.
+// Tiles for one round that is nearly full and surely fits are as good for them (what is left to spare takes up an uneven deal over the
+// XCDs; the whole forward, B H16 D64, bf16 groups of 4 / fp16 groups of 2, 3x3): 420 tiles (B1 S1280) 79.2 | 77.3 / 78.1 | 77.4, (B2 S896)
+// 81.9 | 81.6 / 81.1 | 82.5, 440 (B4 S640) 84.5 | 84.9 / 84.5 | 89.1, 448 (B8 S448) 87.9 | 92.4 / 89.3 | 99.8, 480 (B2 S960) 83.6 | 84.7 /
+// 83.2 | 86.1, but 506 (B1 S1408) 93.9 | 83.5 / 92.1 | 83.4.  The dense 16 heads gain nothing there: 420 (B1 S1280) 80.0 | 77.5, 440 85.1 | 81.1,
+// 448 85.9 | 85.2, 480 81.9 | 80.5, 506 95.2 | 86.1, 7x7 at 506 100.9 | 90.4.
+bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only, bool dense)
 {
     const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64, tiles = planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk);
-    return tiles >= 800 || (tiles >= 400 && tiles <= 512);
+    return tiles >= 800 || (!dense && tiles >= 430 && tiles <= 490);
 }
 
 int64_t lcm(int64_t a, int64_t b)
@@ -320,7 +324,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
                                   ((r == 3 && s == 3 && (dtype == at::kFloat || scores.numel() <= 12 << 20)) || (r == 7 && s == 7 && scores.numel() <= 6 << 20));
         OptTensor done;
         if (!first && !post_conv_identity && w2 &&
-            (small_groups || (mix16 && conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv)))) {
+            (small_groups || (mix16 && conv_mix16_fills(scores.size(0) * (heads / 16), scores.size(2), n_keys, causal && own_pv, g_post == 16)))) {
             mark("conv_mix_post");
             done = conv2d_headmix(scores, post_conv_w, w_post, causal, g_post, !own_pv);
         }

@@ -1140,6 +1140,22 @@ def test_mta_use_mask_left_padded_batch(pkg, case):
     assert not got[last, :int(pad[last])].any()
 
 
+@pytest.mark.parametrize("b,s,group,one", [(1, 1408, 16, False), (2, 960, 16, False), (4, 640, 16, False), (1, 1920, 16, True),
+                                           (1, 1408, 4, False), (2, 960, 4, True), (4, 640, 2, True), (1, 1280, 2, False), (1, 1920, 4, True)])
+def test_post_conv_and_mixing_in_one_kernel_or_two(pkg, b, s, group, one):
+    """Which grids take the one-kernel form: whole rounds of its persistent workgroups, for groups of 2 or 4 heads also one that is
+    nearly full (tiles of 32 x 64 on the lower triangle: 506, 480, 440, 930; 506, 480, 440, 420, 930)."""
+    print(f"conv + mixing b={b} s={s} group={group}", flush=True)
+    params = _config_like(16, group, 3, 3, 0.05, torch.bfloat16, post="random")
+    mod = _mta_module(pkg, 16, 3, 3, 3, 3, *params, torch.bfloat16, structure="infer")
+    stages = []
+    mod._stage_hook = stages.append
+    q, k, v = (torch.randn(b, 16, s, 64, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    with torch.no_grad():
+        assert torch.isfinite(mod(q, k, v, None, None).float()).all()
+    assert ("conv_mix_post" in stages) == one and ("mix_post" in stages) != one, stages
+
+
 @pytest.mark.parametrize("post", ["identity", "random"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_mta_use_mask_rows_that_see_nothing(pkg, dtype, post):
