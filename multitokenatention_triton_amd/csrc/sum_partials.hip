@@ -4,23 +4,30 @@
 // What bounds it is its own launch: a few KB to a few MB, and 4 us alone on the stream.  So a launch takes several gradients: the
 // backward of a whole module adds up its four at the end (a training step of B1 H8 S256 D64 bf16, bound by the host: 21 launches
 // -> 18, 174 -> 168 us; B1 H16 S2048 D128 fp16, where the pre-softmax pair shares one: 607 -> 605).  16 entries per workgroup, an
-// entry's partial results dealt to 64 threads (each adds its share in index order, 16 in flight), the 64 sums added in thread order.
+// entry's partial results dealt to 16 threads, or 64 where there are more than one round of loads of 16 threads takes (256): each adds
+// its share in index order, 16 loads in flight whatever is left of it (a loop that unrolls by 16 walked a share of four as a chain of
+// four latencies), then four threads of a wavefront, then the wavefronts in order.  With the gradient's first kernel, that loop and 64
+// threads always | 16 threads | 64, us: B2 H16 S1001 head weight (256 partial results) 36.8 | 35.4 | 36.2, B1 H32 S1024 (512) 24.9 | 23.1 | 23.2,
+// B1 H16 S1024 (1024) 18.0 | 17.7 | 17.8, B2 H32 S2048 groups of 4 (2048) 176 | 180 | 176; B2 H16 S1000 conv 3x3 (32) 26.4 | 26.6 | 27.5.
+// One gradient has an argument block of its own (370 bytes less to fetch: 0.2 us).
 #include "common.hpp"
 
 namespace {
 using namespace mta;
 
-constexpr int ENTRIES = 16, SHARES = 64;
-struct jobs_arg {
-    int first[MTA_MAX_SUMS + 1];   // workgroups of the jobs ahead
-    mta_partials job[MTA_MAX_SUMS];
+constexpr int ENTRIES = 16, BATCH = 16;
+template <int N> struct jobs_arg {
+    int first[N + 1];   // workgroups of the jobs ahead
+    mta_partials job[N];
 };
 
-__global__ __launch_bounds__(ENTRIES * SHARES) void sum_partials(const jobs_arg jobs, int count)
+template <int N, int SHARES> __global__ __launch_bounds__(ENTRIES * SHARES) void sum_partials(const jobs_arg<N> jobs, int count)
 {
-    __shared__ float red[SHARES][ENTRIES + 1];
+    __shared__ float red[ENTRIES * SHARES / 64][ENTRIES];
     int n = 0;
-    while (n + 1 < count && (int)blockIdx.x >= jobs.first[n + 1]) ++n;
+    if constexpr (N > 1) {
+        while (n + 1 < count && (int)blockIdx.x >= jobs.first[n + 1]) ++n;
+    }
     const mta_partials &j = jobs.job[n];
     const int le = threadIdx.x % ENTRIES, sl = threadIdx.x / ENTRIES, e = ((int)blockIdx.x - jobs.first[n]) * ENTRIES + le;
     // entry e of the result: which block, which entry of it
@@ -39,15 +46,23 @@ __global__ __launch_bounds__(ENTRIES * SHARES) void sum_partials(const jobs_arg 
     float s = 0.0f;
     if (in) {
         const float *from = (const float *)j.partial + (int64_t)block * j.parts * entries + at;
-#pragma unroll 16
-        for (int b = sl; b < j.parts; b += SHARES) s += from[(int64_t)b * entries];
+        for (int b = sl; b < j.parts; b += BATCH * SHARES) {
+            float v[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) v[u] = from[(int64_t)(b + u * SHARES < j.parts ? b + u * SHARES : b) * entries];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) s += b + u * SHARES < j.parts ? v[u] : 0.0f;
+        }
     }
-    red[sl][le] = s;
+    static_assert(ENTRIES == 16 && SHARES % 4 == 0, "four shares of an entry in a wavefront");
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    red[threadIdx.x >> 6][le] = s;
     __syncthreads();
     if (sl != 0 || e >= (j.side > 0 ? j.rows * j.rows : j.rows * entries)) return;
     float t = 0.0f;
 #pragma unroll
-    for (int k = 0; k < SHARES; ++k) t += red[k][le];
+    for (int k = 0; k < ENTRIES * SHARES / 64; ++k) t += red[k][le];
     t = in ? t * j.scale : 0.0f;
     if (j.dtype == MTA_F32) ((float *)j.dw)[e] = t;
     else if (j.dtype == MTA_BF16) ((bf16_t *)j.dw)[e] = from_float<bf16_t>(t);
@@ -60,7 +75,8 @@ extern "C" int mta_sum_partials(int count, const mta_partials *jobs, void *strea
     if (count < 0 || count > MTA_MAX_SUMS) return MTA_ERR_SHAPE;
     if (count == 0) return MTA_OK;
     if (!jobs) return MTA_ERR_NULL;
-    jobs_arg a{};
+    jobs_arg<MTA_MAX_SUMS> a{};
+    int most = 0;
     for (int i = 0; i < count; ++i) {
         const mta_partials &j = jobs[i];
         if (!j.partial || !j.dw) return MTA_ERR_NULL;
@@ -69,7 +85,13 @@ extern "C" int mta_sum_partials(int count, const mta_partials *jobs, void *strea
         if (j.rows <= 0 || j.entries <= 0 || j.parts <= 0 || total > (1 << 26) || (j.side > 0 && (j.rows % j.side || j.entries != j.side * j.side))) return MTA_ERR_SHAPE;
         a.job[i] = j;
         a.first[i + 1] = a.first[i] + (int)((total + ENTRIES - 1) / ENTRIES);
+        most = j.parts > most ? j.parts : most;
     }
-    hipLaunchKernelGGL(sum_partials, dim3((unsigned)a.first[count]), dim3(ENTRIES * SHARES), 0, (hipStream_t)stream, a, count);
-    return launch_status();
+    auto go = [&](auto kern, int shares, const auto &arg) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)a.first[count]), dim3(ENTRIES * shares), 0, (hipStream_t)stream, arg, count);
+        return launch_status();
+    };
+    const jobs_arg<1> one{{0, a.first[1]}, {a.job[0]}};
+    if (most <= 16 * BATCH) return count == 1 ? go(sum_partials<1, 16>, 16, one) : go(sum_partials<MTA_MAX_SUMS, 16>, 16, a);
+    return count == 1 ? go(sum_partials<1, 64>, 64, one) : go(sum_partials<MTA_MAX_SUMS, 64>, 64, a);
 }

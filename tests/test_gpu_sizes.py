@@ -424,6 +424,45 @@ def test_headmix_both_gradients(pkg, c, group, dtype):
         assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * size_w + half_step).all()
 
 
+@pytest.mark.parametrize("parts", [1, 15, 16, 17, 255, 256, 257, 1023, 1025, 2048])
+def test_sums_by_number_of_partial_results(pkg, parts):
+    """One gradient and three of them at once, edges of a thread's share and of a round of loads; conv kernels (entries no multiple of
+    16), a dense head weight, one of groups, one masked to them.  Against float64: fp32 sums of at most 2048 values of magnitude up to
+    about 5 in shares of at most 33, then 18: 51 roundings of at most 2^-24 of the sum of magnitudes, and one of the result."""
+    import ctypes
+    lib, st, Partials = pkg._lib.load(), torch.cuda.current_stream().cuda_stream, pkg._lib.Partials
+    g = torch.Generator(device="cuda").manual_seed(parts)
+    blocks = lambda t: torch.block_diag(*t)   # noqa: E731
+    jobs, want, size, dws = [], [], [], []
+    same = torch.block_diag(*[torch.ones(4, 4, device="cuda")] * 3).double()
+    for rows, entries, side, mask, n, dtype in ((3, 66, 0, 0, parts, torch.float32), (12, 16, 4, 0, parts, torch.bfloat16), (12, 144, 12, 4, max(1, parts // 3), torch.float16)):
+        count = rows if side == 0 else rows // side
+        p = torch.randn(count, n, entries, generator=g, device="cuda")
+        exact, most = ((t.double().sum(1) * 0.5) for t in (p, p.abs()))
+        if side:
+            exact, most = (blocks(list(t.view(count, side, side))) for t in (exact, most))
+        if mask:
+            exact, most = exact * same, most * same
+        dw = torch.full(exact.shape, 7.0, dtype=dtype, device="cuda")
+        jobs.append((p, Partials(p.data_ptr(), dw.data_ptr(), rows, entries, n, side, mask, {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype], 0.5)))
+        want.append(exact), size.append(most), dws.append(dw)
+
+    def check():
+        for exact, most, dw in zip(want, size, dws):
+            assert ((dw.double() - exact).abs() <= 51 * 2.0 ** -24 * most + _unit(dw.dtype) * 1.01 * exact.abs()).all()
+
+    for i in range(3):
+        assert lib.mta_sum_partials(1, ctypes.byref(jobs[i][1]), st) == 0
+    check()
+    alone = [dw.clone() for dw in dws]
+    for dw in dws:
+        dw.fill_(7.0)
+    assert lib.mta_sum_partials(3, (Partials * 3)(*(j for _, j in jobs)), st) == 0
+    check()
+    if parts <= 256 or parts // 3 > 256:   # (else the three take 64 threads an entry and the last one alone 16)
+        assert all(torch.equal(a, b) for a, b in zip(alone, dws))
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("s", [8, 100, 396, 512])
 def test_fp32_scores_by_tile(pkg, s, d):
