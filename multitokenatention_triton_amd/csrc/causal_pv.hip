@@ -405,7 +405,8 @@ template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mi
 // every form (two workgroups of 8 or one of 16).  A wavefront of 16 rows instead of 32 reads its V fragments from LDS for one
 // product each instead of two, which the LDS has room for, and leaves the registers (95 instead of 180) for twice the
 // wavefronts: the reads of P and V that one waits for fly beside the others' products.
-template <typename T, int D, int RW, int GR>
+// SUMS = 2: a group adds its even and its odd steps up apart, so that two groups leave a row's sum in the order in which four do.
+template <typename T, int D, int RW, int GR, int SUMS = 1>
 __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1)) void causal_pv_mid_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
     const int *__restrict__ band_lo, int H, int tri_gl, float scale)
@@ -470,16 +471,18 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
     }
     // this group's blocks, by the block's own number (what a band mask skips leaves every sum as it is)
     const int jg = j0 + ((grp - j0) & (GR - 1)), nsteps = (j_end - j0) / GR + 1;
-    f32x4 oacc[DB];
+    f32x4 sums[SUMS][DB];
 #pragma unroll
-    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) sums[i][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     frag8<T> p_a[P_KS], p_b[P_KS];
     if (jg <= j_end) issue_v(jg, v_a);
     load_p(jg, p_a);
     // lane's place in a block of V for the transpose reads: rows kg*8 + ln/4 (+4), whose swizzle no other part of the row
     // number touches; head-dim block db is an exclusive or away
     const int vrow = kg * 8 + (ln >> 2), vat = vrow * D + ((((ln & 3) >> 1) ^ v_swizzle<D>(vrow)) * 8) + (ln & 1) * 4;
-    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pf)[P_KS], frag8<T> (&pn)[P_KS]) __attribute__((always_inline)) {
+    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pf)[P_KS], frag8<T> (&pn)[P_KS], f32x4 (&oacc)[DB]) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0);   // V block j and the P fragments have arrived
         __syncthreads();                 // for every wavefront; reads of the other buffer are finished
         if (j > j_end) return;
@@ -517,12 +520,17 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
         }
     };
     for (int i = 0, j = jg;;) {
-        step(j, v_a, v_b, p_a, p_b);
+        step(j, v_a, v_b, p_a, p_b, sums[0]);
         if (++i >= nsteps) break;
         j += GR;
-        step(j, v_b, v_a, p_b, p_a);
+        step(j, v_b, v_a, p_b, p_a, sums[SUMS - 1]);
         if (++i >= nsteps) break;
         j += GR;
+    }
+    f32x4 (&oacc)[DB] = sums[0];
+    if constexpr (SUMS == 2) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[db] += sums[1][db];
     }
     if constexpr (GR > 1) {
         if (!mid_sums<T, DB, GT, GR>(v_a_all, v_b_all, oacc, grp, tid)) return;
@@ -809,7 +817,9 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
 //          B1 H16 S3072 D128 (768)        66.7 | 61.2 | 53.2 | 48.8 | 56.2 | 59.0      B1 H16 S4096 D64 (1024)   85.2 | 67.7 | 82.0 | 69.6 | 73.3 | 72.0
 //          B4 H16 S1024 D64 (1024)        27.2 | 20.1 | 18.6 | 21.2 | 19.5 | 23.3      B2 H16 S2048 D128 (1024)  64.8 | 69.0 | 49.9 | 51.1 | 50.4 | 53.6
 //          B3 H16 S2048 D128 (1536)       94.1 | 91.2 | 68.3 | 68.1 | 60.8 | 70.0      B4 H32 S2048 D64 (2048)   171  | 129  | 118  | 137  | 122  | 141
-// All but the narrow kernel add a row up in the same order (the even and the odd key blocks apart, with four groups by fours).
+// The fp32 sums of a row have three orders: block by block (the wide kernel, 128 rows with one group), the even and the odd blocks apart
+// (two groups), every fourth block apart (four groups, also as two with two sums each; the narrow kernel's four wavefronts).  So a head's last bit may differ
+// between batch sizes that take different kernels.
 enum product_kernel { WIDE = 1, R64_2, NARROW, R64_4, R128_2, R128_1 };
 
 product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bool tri)
@@ -872,7 +882,12 @@ int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t 
     };
     switch (product_form(B * H, S, D, false, tri_gl > 0)) {
     case NARROW: return go(causal_pv_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 4 : 2);
-    case R64_4: return go(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024, 1);
+    // (Under a band mask a block of rows has few key blocks: two workgroups per CU, two groups in each, that add in the same order.  P V,
+    // narrow | four groups | two, us: window of S/4, B1 H16 S1440 (368 blocks) D64 11.4 | 12.5 | 11.0, D128 16.1 | 16.3 | 12.8; B1 H8 S3584 (448)
+    // 16.0 | 19.2 | 14.6, 24.8 | 23.6 | 18.9, with S/2 22.7 | 27.5 | 21.2, 37.0 | 33.8 | 28.0.  Few blocks beyond one for every CU are left to four
+    // groups, which are ahead there where the window is long: B1 H4 S4992 (312) S/4 15.0 | 20.8 | 15.8, 24.8 | 25.6 | 19.9, S/2 19.7 | 21.8 | 24.1,
+    // 28.1 | 26.2 | 28.8; S4352 (272) S/4 12.1 | 13.5 | 13.3, 17.4 | 17.8 | 16.5, S/2 19.7 | 19.6 | 23.0, 28.2 | 24.4 | 27.5.)
+    case R64_4: return band_lo && B * H * ((S + 63) / 64) >= 300 ? go(causal_pv_mid_kernel<T, D, 4, 2, 2>, 64, 512, 2) : go(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024, 1);
     case R64_2: return go(causal_pv_mid_kernel<T, D, 4, 2>, 64, 512, 2);
     case R128_2: return go(causal_pv_mid_kernel<T, D, 8, 2>, 128, 1024, 1);
     case R128_1: return go(causal_pv_mid_kernel<T, D, 8, 1>, 128, 512, 2);
