@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/mta_hip.h"
 
 namespace mta {
@@ -150,6 +152,20 @@ inline int launch_status()
 {
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? MTA_OK : (int)e;
+}
+
+inline int device_cu_count()
+{
+    // (atomic slots: concurrent first calls on a device both query and both store the same value, without a data race)
+    static std::atomic<int> cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cached[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 #define MTA_DISPATCH_IO(dt, ...)                                      \

@@ -207,7 +207,7 @@ struct item_table {
 // BAND (scores-only kernel): a mask of the form "key k of query row p is visible iff band_lo[b, p] <= k <= p" - the
 // scores of the hidden keys enter the conv as 0, as the reference's masked_fill ahead of its conv leaves them
 // (mta_attention_triton.py:70-73).
-template <typename T, int D, int R, int SK, bool SCORES_ONLY, int NW, bool BAND = false>
+template <typename T, int D, int R, int SK, bool SCORES_ONLY, int NW, bool BAND, int TURNS>
 __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7)) ? 2 : QK_OCC) : (R > 7 ? 1 : 2)) void conv_attn_fwd_mfma(const T *__restrict__ Q, const T *__restrict__ K,
                                                              const T *__restrict__ V, const T *__restrict__ Wt,
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
@@ -581,11 +581,9 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         // One product needs one fresh 1 KB score fragment from LDS, and a wavefront that waits for each fragment
         // where it is used spends four times the products' own time here.  The reads are therefore issued NLD
         // products ahead, from assembly (see lds_read16_at), into a ring of registers; every product is preceded by
-        // a wait that leaves exactly the younger operations outstanding.  Two neighbouring output blocks are worked on in
-        // turns: the R products of one block add into the same registers, each waiting for the one before (one block at a
-        // time | two: attention B1 H16 S2048 D64 6x11 83.8 | 79.9 us, B4 H8 S1024 D128 11x15 65.9 | 64.4, B1 H32 S8192 D128 6x11
-        // 1096 | 1080; the scores kernel, with three wavefronts per SIMD to fill the gaps, the same within 1 %).  Their results
-        // are taken up LAG products into the next two, when they are long complete.
+        // a wait that leaves exactly the younger operations outstanding.  The R products of one output block add into the same
+        // registers, each waiting for the one before; with TURNS = 2 two neighbouring blocks are worked on in turns (which is
+        // chosen where: launch_mfma()).  A block's results are taken up LAG products into the next turn, when they are long complete.
         constexpr int NB = 2 * NCB, NREAD = NB * R;
         // score fragments in flight (scores only: 8 and 12 measure the same, 15 spills; the attention kernel, at the
         // 256-register limit, spills from 6 on)
@@ -595,10 +593,10 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         static_assert(NREAD > NLD && R >= LAG && NLD <= 15, "pipeline deeper than the work or than the counter");
         const unsigned xa = lds_addr(Sc) + (unsigned)(((trow[0] + cshift - (R - 1)) * F_SLD + kg * 8) * (int)sizeof(T));
         u32x4_t ring[NSLOT];
-        f32x4 cacc[4];
+        f32x4 cacc[2 * TURNS];
         auto issue = [&](auto ic) __attribute__((always_inline)) {
             constexpr int n = decltype(ic)::value;
-            constexpr int blk = n / (2 * R) * 2 + (n & 1), i = n % (2 * R) / 2;   // output block, kernel row
+            constexpr int blk = n / (TURNS * R) * TURNS + n % TURNS, i = n % (TURNS * R) / TURNS;   // output block, kernel row
             ring[n % NSLOT] = lds_read16_at(xa, (((blk / NCB) * 16 + i) * F_SLD + (blk % NCB) * 16) * (int)sizeof(T));
         };
         // what happens to output block b = rb*NCB + cb (rows crow[rb], keys j*64 + 16cb ..) once it is complete
@@ -608,7 +606,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         auto finish = [&](auto bc) __attribute__((always_inline)) {
             constexpr int b = decltype(bc)::value;
             constexpr int rb = b / NCB, cb = b % NCB;
-            const f32x4 a = cacc[b & 3];
+            const f32x4 a = cacc[b % (2 * TURNS)];
             const int p_ = cprow[rb];
             if constexpr (SCORES_ONLY) {
                 // Blocks leave in pairs, like the scores above: after the exchange a lane holds 8 consecutive keys of
@@ -701,21 +699,20 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         static_for<NLD>(issue);
         static_for<NREAD>([&](auto ic) __attribute__((always_inline)) {
             constexpr int n = decltype(ic)::value;
-            constexpr int blk = n / (2 * R) * 2 + (n & 1), i = n % (2 * R) / 2;
+            constexpr int blk = n / (TURNS * R) * TURNS + n % TURNS, i = n % (TURNS * R) / TURNS;
             if constexpr (n + NLD < NREAD) issue(std::integral_constant<int, n + NLD>{});
             // LDS operations younger than read n: exactly the reads issued after it
             constexpr int younger = (n + NLD < NREAD ? n + NLD : NREAD - 1) - n;
             lds_wait_upto<younger>(ring[n % NSLOT]);
-            if constexpr (i == 0) cacc[blk & 3] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            mma16(cacc[blk & 3], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
+            if constexpr (i == 0) cacc[blk % (2 * TURNS)] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            mma16(cacc[blk % (2 * TURNS)], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (blk >= 2 && i == LAG - 1) {
-                finish(std::integral_constant<int, blk - 2>{});
+            if constexpr (blk >= TURNS && i == LAG - 1) {
+                finish(std::integral_constant<int, blk - TURNS>{});
                 __builtin_amdgcn_sched_barrier(0);
             }
         });
-        finish(std::integral_constant<int, NB - 2>{});
-        finish(std::integral_constant<int, NB - 1>{});
+        static_for<TURNS>([&](auto b) __attribute__((always_inline)) { finish(std::integral_constant<int, NB - TURNS + decltype(b)::value>{}); });
         if constexpr (SCORES_ONLY) return;
 
         // ---- O^T += V^T P^T ; V^T fragments via the LDS transpose read of the row-major V block ----
@@ -820,7 +817,18 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
     static_assert(G::fits, "conv window exceeds the 32-key MFMA contraction");
     const int nqb = (int)((S + G::BQ - 1) / G::BQ);
-    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND>;
+    // Output blocks of the conv in turns (1 | 2, us): the scores kernels gain up to 1.5 % (bf16 6x11 B1 H16 S2048 D64 34.3 | 33.9, B4 H16
+    // S1024 D128 39.8 | 39.3, fp16 7x7 B1 H16 S2048 D128 41.6 | 41.2), the attention kernel of 11 rows -1 to 2 % (fp16 B1 H16 S2048 D64 103.8 |
+    // 102.2, bf16 D128 119.9 | 118.7, B4 H12 D64 151.3 | 152.3).  Of up to 7 rows it is slower in bf16 (3x3 B1 H32 S4096 D128 275.9 | 278.8, 6x11
+    // B1 H8 S2048 D64 78.9 | 79.9, 7x7 B1 H16 S2048 D128 98.8 | 99.6, larger grids within 0.5 %) and in fp16 with 3 rows (B1 H8 S2048 D64 75.2 | 76.4);
+    // fp16 with 5 to 7 rows loses while its workgroups fit the chip at once (6x11 D64 B1 H8 S2048 82.0 | 84.4, H16 83.2 | 85.4, D128 98.3 |
+    // 99.4), and gains beyond (7x7 D64 B4 H12 S2048 120.3 | 119.6, 6x11 D128 B1 H32 S4096 313 | 310).
+    constexpr bool BY_GRID = !SCORES_ONLY && __is_same(T, f16_t) && R > 3 && R <= 7;
+    constexpr int TURNS = SCORES_ONLY || R > 7 || BY_GRID ? 2 : 1;
+    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND, TURNS>;
+    if constexpr (BY_GRID) {
+        if (B * H * nqb <= 2 * (int64_t)device_cu_count()) kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND, 1>;
+    }
     // key blocks per work item: all of them for the attention kernel; QK_CHUNK for the scores-only kernel
     const int jc_len = SCORES_ONLY ? QK_CHUNK : (int)((S + F_BK - 1) / F_BK) + 1;
     int64_t items_per_bh = 0;

@@ -4,7 +4,6 @@
 
 #include "common.hpp"
 
-#include <atomic>
 #include <type_traits>
 #include <utility>
 
@@ -126,20 +125,6 @@ __device__ __forceinline__ bool longest_first(unsigned wg, int heads, int blocks
 __device__ __forceinline__ bool longest_first(int heads, int blocks, int cus, int &bh, int &rank)
 {
     return longest_first(blockIdx.x, heads, blocks, cus, bh, rank);
-}
-
-inline int device_cu_count()
-{
-    // (atomic slots: concurrent first calls on a device both query and both store the same value, without a data race)
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    int n = cached[dev].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
 }
 
 }  // namespace

@@ -463,6 +463,21 @@ def test_sums_by_number_of_partial_results(pkg, parts):
         assert all(torch.equal(a, b) for a, b in zip(alone, dws))
 
 
+@pytest.mark.parametrize("r,k", [(3, 3), (5, 5), (6, 11), (7, 7), (11, 15)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_fp16_attention_by_grid(pkg, d, r, k):
+    """fp16 attention of 600 workgroups and, of the same heads, 2 x 300, which the chip holds at once: other instances for 5 to 7 kernel
+    rows, the same sums in the same order."""
+    g = torch.Generator(device="cuda").manual_seed(59)
+    q, kk, v = (torch.randn(1, 300, 136, d, generator=g, device="cuda").half() for _ in range(3))
+    w = (0.1 * torch.randn(300, r, k, generator=g, device="cuda")).half()
+    run = lambda lo, hi: pkg.ops.conv_attn_fwd(q[:, lo:hi].contiguous(), kk[:, lo:hi].contiguous(), v[:, lo:hi].contiguous(), w[lo:hi], True, d ** -0.5)   # noqa: E731
+    first = lambda out: out[0] if isinstance(out, tuple) else out   # noqa: E731
+    whole = first(run(0, 300))
+    assert torch.isfinite(whole.float()).all()
+    assert torch.equal(whole, torch.cat([first(run(0, 150)), first(run(150, 300))], 1))
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("s", [8, 100, 396, 512])
 def test_fp32_scores_by_tile(pkg, s, d):
