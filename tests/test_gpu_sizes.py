@@ -728,6 +728,53 @@ def test_softmax_and_headmix_gradients(pkg, c, group, longest, dtype):
         assert ((dw - want_w).abs() <= u * want_w.abs() + 1.01 * u * size_w + tiny * xd.abs().sum()).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,group", [(2, 0), (4, 0), (8, 0), (12, 0), (16, 0), (32, 0), (16, 4), (16, 8)])
+def test_headmix_gradients_of_many_rows(pkg, c, group, dtype):
+    """The same kernels with more rows than wavefronts: a wavefront of the first takes several chunks, of rows of two batch entries
+    too (an odd number of rows each), a workgroup of the one behind the softmax gradient several rows, whose wavefronts end one after
+    the other.  Against float64 on the GPU, bounds as in the tests of the small sizes above."""
+    g = torch.Generator(device="cuda").manual_seed(53)
+    lanes = (group or c) <= 4
+    half_step = 2.0 ** -25 if dtype == torch.float16 else 0.0
+    block = torch.arange(c, device="cuda") // (group or c)
+    same = block[:, None] == block[None, :]
+    w = (torch.eye(c, device="cuda") + 0.3 * torch.randn(c, c, generator=g, device="cuda")).to(dtype)
+    wd = w.double() * same
+    mix = lambda t: torch.matmul(wd.t(), t.flatten(2)).view_as(t)   # noqa: E731
+    size_of = lambda t: torch.matmul(wd.abs().t(), t.flatten(2)).view_as(t)   # noqa: E731
+    contract = lambda a, b: torch.matmul(a.transpose(0, 1).flatten(1), b.transpose(0, 1).flatten(1).t()) * same   # noqa: E731
+    nan = float("nan")
+    for n, p, q, mode in ((3, 3001, 520, "lower") if lanes else (3, 1501, 264, "lower"), (2, 8193, 8, "fill"), (2, 8193, 16, "all")):
+        print(f"headmix gradients c={c} group={group} {n}x{p}x{q} {mode} {dtype}", flush=True)
+        causal = mode != "all"
+        keep = torch.ones(p, q, dtype=torch.bool, device="cuda")
+        keep = keep.tril() if causal else keep
+        x, dy = (torch.randn(n, c, p, q, generator=g, device="cuda").to(dtype) for _ in range(2))
+        xd, dyd = x.double().masked_fill(~keep, 0.0), dy.double().masked_fill(~keep, 0.0)
+        dx, dw = pkg.ops.headmix_grads(dy.masked_fill(~keep, nan), x.masked_fill(~keep, nan), w, causal, group_size=group, fill_upper=mode == "fill")
+        dx, dw, want, want_w = dx.double(), dw.double(), mix(dyd), contract(dyd, xd)
+        assert ((dx - want).abs() <= _unit(dtype) * 1.01 * want.abs() + 2.0 ** -19 * size_of(dyd.abs()) + half_step)[..., keep].all()
+        if mode == "fill":
+            assert (dx[..., ~keep] == 0.0).all()
+        assert ((dw - want_w).abs() <= _unit(dtype) * want_w.abs() + (n * p * q) ** 0.5 * 2.0 ** -22 * contract(dyd.abs(), xd.abs()) + half_step).all()
+    u = _unit(dtype) if dtype != torch.float32 else 2.0 ** -20
+    tiny = 2.0 ** -24 * 32 if dtype == torch.float16 else 0.0
+    for n, p, q, causal in ((3, 1301, 264, True), (2, 2600, 40, True), (1, 4200, 136, False)):
+        print(f"softmax + headmix gradients c={c} group={group} {n}x{p}x{q} causal={causal} {dtype}", flush=True)
+        keep = torch.ones(p, q, dtype=torch.bool, device="cuda")
+        keep = keep.tril() if causal else keep
+        s = torch.softmax(torch.randn(n, c, p, q, generator=g, device="cuda").masked_fill(~keep, float("-inf")), -1).to(dtype)
+        ds, x = (torch.randn(n, c, p, q, generator=g, device="cuda").to(dtype) for _ in range(2))
+        sd, dsd, xd = (t.double().masked_fill(~keep, 0.0) for t in (s, ds, x))
+        dy = sd * (dsd - (sd * dsd).sum(-1, keepdim=True))
+        most = dy.abs() + 2.0 ** -19 / u * sd * (dsd.abs() + (sd * dsd.abs()).sum(-1, keepdim=True))
+        dx, dw = pkg.ops.headmix_grads(ds.masked_fill(~keep, nan), x.masked_fill(~keep, nan), w, causal, group_size=group, probs=s.masked_fill(~keep, nan))
+        dx, dw, want_w = dx.double(), dw.double(), contract(dy, xd)
+        assert ((dx - mix(dy)).abs() <= 2.02 * u * size_of(most) + tiny)[..., keep].all()
+        assert ((dw - want_w).abs() <= u * want_w.abs() + 1.01 * u * contract(most, xd.abs()) + tiny * xd.abs().sum()).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,s,d", [(256, 40, 64), (130, 136, 128), (520, 8, 64), (512, 40, 64), (250, 136, 128), (1030, 40, 128), (600, 136, 128), (2100, 40, 64),
                                        (32, 1160, 128), (32, 2056, 128), (12, 2056, 64)])
