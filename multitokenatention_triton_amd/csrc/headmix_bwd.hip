@@ -788,8 +788,7 @@ cut cut_of(int64_t N, int64_t C, int64_t P, int64_t Q, int group_size, int causa
         const int64_t full = 2 * ((Q + keys - 1) / keys), slots = causal == 2 && P / keys + 2 < full ? P / keys + 2 : full;
         const int64_t enough = ((N * P + 1) / 2 * slots + NT / 64 - 1) / (NT / 64), most = lanes ? 2048 : G == 32 ? 512 : 1024;   // (see above; 32 heads, fp32 B1 S1024: 512 | 1024 43 | 54 us)
         c.slots = (unsigned)slots;
-        c.parts = most < 1 ? 1 : most;
-        if (c.parts > enough) c.parts = enough;
+        c.parts = most < enough ? most : enough;
     }
     return c;
 }

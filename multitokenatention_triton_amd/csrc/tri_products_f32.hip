@@ -360,6 +360,10 @@ __global__ __launch_bounds__(256, 2) void causal_ptx_f32(const float *__restrict
 //        45.0 | 33.9 | 32.3 | 29.0, B4 H16 S1024 D64 (1024) 71.4 | 56.3 | 50.8 | 46.3, B2 H32 S1024 D128 148 | 91.5 | 86.9 | 82.7
 //   ptx  (no RW = 2) B4 H8 S768 D64 (n64 = 384) 18.0 | - | 19.4 | 21.3, B1 H32 S1024 D64 (512) 29.2 | - | 26.3 | 28.5, D128 50.5 | - | 44.6 |
 //        46.8, B1 H16 S2048 D128 (512) 91.1 | - | 81.2 | 86.1, B4 H16 S1024 D64 (1024) 56.0 | - | 52.5 | 49.9
+// The line of ptx at 512 is two blocks for every CU, where RW GR = 4 2 is ahead at both head sizes.  Between 384 and 512, the kernel above |
+// 4 2, us: D64 416 (S1024) 28.8 | 26.6, (S2048) 51.0 | 45.2, 480 (S3072) 73.8 | 68.1, 488 (S3904) 86.8 | 83.5, 496 (S512) 20.9 | 16.4; D128 416
+// (S1024) 47.0 | 46.0, (S2048) 82.5 | 85.3, 448 (S1024) 46.0 | 46.3, (S2048) 86.6 | 85.6, 480 (S1024) 51.4 | 46.9, (S3072) 127 | 126, 488 (S3904)
+// 154 | 158, 496 (S512) 32.1 | 27.7: head size 64 would gain from 416 on.
 // The sums of GR groups of GT threads, N vectors each, added up in the first group (true there): the upper half of the groups hand
 // theirs to the lower half through LDS until one is left.
 template <int N, int GT, int GR> __device__ __forceinline__ bool group_sums(float *lds, f32x4 (&acc)[N], int grp, int tid)
