@@ -902,3 +902,20 @@ def test_softmax_rows_without_a_visible_key(pkg, group, dtype):
                     tri = pkg.ops.headmix_softmax_tri(pkg.ops.tri_pack(x, group), w1, w2, 1, c, s, group, key_bias=bias, first_visible=first)
                     tri = pkg.ops.tri_unpack(tri, 1, c, s, group)[..., ~upper]
                     assert torch.equal(tri.nan_to_num(7.0), got[..., ~upper].nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", _SOFTMAX_GROUPS)
+def test_softmax_of_a_window_wider_than_its_rows(pkg, group, dtype):
+    """First visible keys below 0, by less than a tile and by several: the bits that 0 gives, row by row, beside rows that hide keys."""
+    g = torch.Generator().manual_seed(73)
+    for s in _SOFTMAX_ROWS:
+        c, weights = _softmax_weights(group, dtype, g)
+        x = torch.randn(1, c, s, s, generator=g).to(dtype).cuda()
+        p = torch.arange(s, device="cuda")
+        first = torch.where(p % 3 == 0, p - s - 1, torch.where(p % 3 == 1, p // 2, p - 5 * s - 700)).int()[None]
+        for w1, w2 in weights:
+            print(f"softmax of a wide window group={group} s={s} {w1 is not None} {w2 is not None} {dtype}", flush=True)
+            run = lambda lo: _bits(pkg.ops.headmix_softmax(x, w1, w2, True, group_size=group, first_visible=lo))  # noqa: E731
+            got = run(first)
+            assert torch.equal(got, run(first.clamp(min=0))) and not got.view(dtype).isnan().any()
