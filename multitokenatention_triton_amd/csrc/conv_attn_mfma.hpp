@@ -17,7 +17,7 @@ using namespace mta;
 // =======================================================================================
 // 16-bit fast path: everything on 16x16x32 MFMAs, conv included.
 //
-//  * 8 wavefronts own 256 score rows (HR halo rows + 256-HR output rows); a wavefront owns two
+//  * 4 wavefronts own 128 score rows (HR halo rows + 128-HR output rows); a wavefront owns two
 //    blocks of 16 rows.  Lane (r = lane%16, g = lane/16) owns query row r of a block; the
 //    16x16 accumulator layout gives it keys 4g..4g+3 of every 16-key block, so a query row is
 //    spread over 4 lanes and row reductions cost two lane exchanges.
@@ -37,13 +37,21 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 
-// The workgroup has NW wavefronts and owns 32*NW score rows: 8 for the attention kernel (one workgroup per CU,
-// K and V blocks shared by 256 rows), 4 for the scores-only kernel (three workgroups per CU, which overlap each
-// other's barriers and memory latency).
-// The attention kernel reads the LDS operands of the next group of matrix products before it issues the current group;
-// the instruction scheduler largely undoes that (it moves reads down towards their use, which saves registers).  Pinning
-// the source order there was measured and is slower (1.60 -> 1.72 ms at the benchmark shape, 12-14 spilled registers).
-// The scores-only kernel pins its conv phase by hand instead (reads issued from assembly, see below).
+// The workgroup has NW = 4 wavefronts and owns 128 score rows; two workgroups per CU for the attention kernel (three at D = 64 up
+// to 7 kernel rows), three for the scores-only one, which overlap each other's barriers and memory latency.
+// What bounds the attention kernel: matrix products (896 flops executed per score at 6x11, D = 128: Q K^T and P V 256 each, the
+// conv as Toeplitz products 384) beside the vector ALU (the exponentials) and the LDS, which would each take 40 to 60 % of its
+// time alone.  So the vector work is kept small (one maximum, one multiply-add, one exponential and half a conversion and a sum
+// per score: no rounding between the conv and the probabilities) and is written between the products of the same wavefront:
+// the first row block's probabilities among the second one's conv products, half of the second one's among those of P V.
+// The loop has one body: K, V and the buffer the next block goes to are offsets into one LDS array (all reads of it are issued
+// from assembly, so that the compiler cannot wait for the copy in flight), a key block that the diagonal or the end of the
+// sequence does not touch branches around its masks, and every LDS operand is read several products ahead into a ring of
+// registers.  211 registers (248 before, with three bodies): 11 kernel rows run two workgroups per CU as well.
+// us, with the logits rounded twice in the I/O dtype and the softmax of a row block in one piece -> now: bf16 6x11 B1 H32 S8192
+// D128 1067 -> 990 (executed 1.0 PFLOP/s; an 8192^3 library product reaches 1.08), 3x3 B1 H32 S4096 D128 276 -> 246, 7x7 B1 H16
+// S2048 D128 98.9 -> 87.0, 6x11 B1 H8 S2048 D64 78.8 -> 66.7, 5x5 B2 H32 S4096 D64 378 -> 341; fp16 7x9 B4 H12 S2048 D64 120 -> 93,
+// 11x15 B1 H32 S4096 D128 595 -> 360.
 constexpr int F_BK = 64;   // keys per iteration
 constexpr int QK_OCC = 3;     // wavefronts per SIMD the scores-only kernel is compiled for (three workgroups per CU)
 constexpr int QK_CHUNK = 32;  // key blocks per work item of the scores-only kernel when no item table is built
@@ -100,6 +108,13 @@ __device__ __forceinline__ void lds_write16_at(unsigned addr, int off, u32x4_t v
 {
     asm volatile("ds_write_b128 %0, %1 offset:%2" : : "v"(addr), "v"(v), "n"(off) : "memory");
 }
+// the transpose read of 8 bytes
+__device__ __forceinline__ u32x2_t lds_read_tr8_at(unsigned addr, int off)
+{
+    u32x2_t v;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(off) : "memory");
+    return v;
+}
 template <int N> __device__ __forceinline__ void lds_wait_upto(u32x4_t &v)
 {
     asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N) : "memory");
@@ -152,6 +167,16 @@ __device__ __forceinline__ float sum_across_groups(float v)
     v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// A tap of the attention kernel, whose softmax takes maxima ahead of the factor and therefore a factor > 0: the tap carries its
+// sign (an exact change of the sign bit), and for 0 its value.
+template <typename T> __device__ __forceinline__ T signed_tap(T w, float scale)
+{
+    uint16_t b = __builtin_bit_cast(uint16_t, w);
+    if (scale < 0.0f) b ^= 0x8000u;
+    if (scale == 0.0f) return from_float<T>(to_float(w) * 0.0f);
+    return __builtin_bit_cast(T, b);
 }
 
 // Inside a rarely taken, wavefront-uniform `if`: keeps it a branch.  Without it the compiler turns the masks of the
@@ -207,8 +232,8 @@ struct item_table {
 // BAND (scores-only kernel): a mask of the form "key k of query row p is visible iff band_lo[b, p] <= k <= p" - the
 // scores of the hidden keys enter the conv as 0, as the reference's masked_fill ahead of its conv leaves them
 // (mta_attention_triton.py:70-73).
-template <typename T, int D, int R, int SK, bool SCORES_ONLY, int NW, bool BAND, int TURNS>
-__global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7)) ? 2 : QK_OCC) : (R > 7 ? 1 : 2)) void conv_attn_fwd_mfma(const T *__restrict__ Q, const T *__restrict__ K,
+template <typename T, int D, int R, int SK, bool SCORES_ONLY, int NW, bool BAND>
+__global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7)) ? 2 : QK_OCC) : 2) void conv_attn_fwd_mfma(const T *__restrict__ Q, const T *__restrict__ K,
                                                              const T *__restrict__ V, const T *__restrict__ Wt,
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
                                                              float scale, int H, int nqb, int fill_upper, int64_t total_wg,
@@ -227,24 +252,20 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     constexpr int NCB = F_BK / 16;                 // 16-key blocks per iteration
     static_assert(ROUNDS >= 1, "block smaller than one copy round");
 
-    // Every buffer is an array of its own, and the key-block loop body is instantiated once per K/V buffer: the
-    // compiler then sees that LDS reads never touch the asynchronous copy in flight into the other buffer.  With one
-    // block of dynamic LDS it cannot, and waits for the copy ahead of the first LDS read that follows its issue.
-    // The scores-only kernel double-buffers K in B0 / B1.  The attention kernel rotates K and V through three
-    // buffers: in an iteration K(j) sits in one, V(j) in another; K(j+1) is copied into the third from the top of the
-    // iteration on, and V(j+1) into K(j)'s buffer once the score phase is over (the barrier in the middle of the
-    // iteration).  Three 16 KB buffers and the score tile are 68 KB: two workgroups per CU, which overlap each
-    // other's vector-ALU and matrix-core phases (a single workgroup's wavefronts meet at two barriers per key block
-    // and are all in the same phase at the same time).
-    __shared__ __align__(16) T B0[TILE];
-    __shared__ __align__(16) T B1[TILE];
-    __shared__ __align__(16) T B2[SCORES_ONLY ? 8 : TILE];
+    // The scores-only kernel double-buffers K in B0 / B1, arrays of their own with a loop body each: the compiler then sees that LDS
+    // reads never touch the asynchronous copy in flight into the other one.  The attention kernel rotates K and V through the
+    // three buffers of KV: in an iteration K(j) sits in one, V(j) in another; K(j+1) is copied into the third from the top of the
+    // iteration on, and V(j+1) into K(j)'s buffer once the score phase is over (the barrier in the middle of the iteration).
+    // Three 16 KB buffers and the score tile are 68 KB: two workgroups per CU.
+    __shared__ __align__(16) T B0[SCORES_ONLY ? TILE : 8];
+    __shared__ __align__(16) T B1[SCORES_ONLY ? TILE : 8];
+    __shared__ __align__(256) T KV[SCORES_ONLY ? 8 : 3 * TILE];
     __shared__ __align__(16) T Sc[RAW ? 8 : F_SR * F_SLD];                // score tile
     // zero-padded kernel rows, only needed until the Toeplitz fragments are built: they borrow a buffer that
     // receives its first copy after that (LDS is granted in 1280-byte units; the array's own 648 bytes were the
     // difference between two and three workgroups per CU for the scores-only kernel)
     static_assert(R * G::WZ_LD <= TILE, "kernel rows do not fit the borrowed buffer");
-    T *const wz = SCORES_ONLY ? B1 : B2;
+    T *const wz = SCORES_ONLY ? B1 : KV + 2 * TILE;
 
     const int tid = threadIdx.x;
     // (the wavefront index through readfirstlane: everything derived from it is then scalar, branches included)
@@ -368,8 +389,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     }
     // one key block earlier only fills the retained score columns (before the first one: the right pad, if any)
     const int j_start = RAW ? j_lo : j_lo > 0 ? j_lo - 1 : (G::PWR > 0 ? -1 : 0);
-    issue_k(j_start, B0);
-    if (!SCORES_ONLY) issue_v(j_start, B1);
+    issue_k(j_start, SCORES_ONLY ? B0 : KV);
+    if (!SCORES_ONLY) issue_v(j_start, KV + TILE);
 
     if constexpr (!RAW) {
     // zero the score tile once (columns past HC+BK are read by the last window but never written)
@@ -383,7 +404,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         const int i = e / G::WZ_LD, jj = e % G::WZ_LD - G::WZ_OFF;
         const bool ok = jj >= 0 && jj < SK;
         const T wv = Wt[head * R * SK + (ok ? i * SK + jj : 0)];
-        wz[e] = ok ? wv : from_float<T>(0.0f);
+        wz[e] = ok ? signed_tap<T>(wv, SCORES_ONLY ? 1.0f : scale) : from_float<T>(0.0f);
     }
     }
 
@@ -432,7 +453,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
         for (int db = 0; db < DB; ++db) oacc[rb][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_i[2] = {-INFINITY, -INFINITY}, l_i[2] = {0.0f, 0.0f};
+    float m_i[2] = {-INFINITY, -INFINITY}, l_i[2] = {0.0f, 0.0f};   // (maxima of the conv's results, ahead of the factor)
+    const float scale_abs = scale == 0.0f ? 1.0f : fabsf(scale), scale2 = scale_abs * 1.4426950408889634f;
 
     // retained columns: each thread moves one 16-byte vector per round (HC/8 vectors per row)
     constexpr int TAIL_VECS = F_SR * (G::HC / 8);
@@ -462,11 +484,16 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         row_stored[rb] = tr_ >= G::HR && tr_ < wave * 32 + 32 && cprow[rb] < S;
     }
 
+    auto plain = [&](int j) {
+        const int cbase = j * F_BK + G::PWR;
+        return j >= 0 && cbase + F_BK <= S && (!causal || cbase + F_BK - 1 <= pmin) && (!BAND || cbase >= fmax_w);
+    };
     // PLAIN: the key block (its scores and its conv outputs) lies inside the sequence and on or below the diagonal
     // for all 32 rows of this wavefront: no masks and no per-sub-block tests (most blocks of a long sequence)
     auto block = [&](auto plain_tag, int j, const T *Kb, const T *Vb, T *Kn, T *Vn) __attribute__((always_inline)) {
         constexpr bool PLAIN = decltype(plain_tag)::value;
         const int cbase = j * F_BK + G::PWR;  // first key of the new score block
+        const bool whole = PLAIN || (!SCORES_ONLY && plain(j));   // (the attention kernel has one body, with a branch around its masks)
         // (a vector type, read by every lane: a struct read under a lane condition travels through scratch memory)
         u32x4_t tailreg[TAIL_IT > 0 ? TAIL_IT : 1];
 #pragma unroll
@@ -503,7 +530,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
             auto epilogue = [&](auto cbc) __attribute__((always_inline)) {
                 constexpr int cb = decltype(cbc)::value;
                 // key block wholly inside the sequence and on or below the diagonal for all 32 rows: no masks
-                const bool s_plain = PLAIN || (cbase + cb * 16 >= 0 && cbase + cb * 16 + 16 <= S && (!causal || cbase + cb * 16 + 15 <= pmin) &&
+                const bool s_plain = PLAIN || !SCORES_ONLY ? PLAIN || whole : (cbase + cb * 16 >= 0 && cbase + cb * 16 + 16 <= S && (!causal || cbase + cb * 16 + 15 <= pmin) &&
                                                (!BAND || cbase + cb * 16 >= fmax_w));
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb) {
@@ -582,11 +609,15 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         // where it is used spends four times the products' own time here.  The reads are therefore issued NLD
         // products ahead, from assembly (see lds_read16_at), into a ring of registers; every product is preceded by
         // a wait that leaves exactly the younger operations outstanding.  The R products of one output block add into the same
-        // registers, each waiting for the one before; with TURNS = 2 two neighbouring blocks are worked on in turns (which is
-        // chosen where: launch_mfma()).  A block's results are taken up LAG products into the next turn, when they are long complete.
+        // registers, each waiting for the one before; with TURNS = 2 two neighbouring blocks are worked on in turns, which gives the
+        // scores kernels up to 1.5 % (1 | 2, us: bf16 6x11 B1 H16 S2048 D64 34.3 | 33.9, B4 H16 S1024 D128 39.8 | 39.3, fp16 7x7 B1 H16
+        // S2048 D128 41.6 | 41.2) and the attention kernel nothing (bf16 6x11 B1 H32 S8192 D128 986 | 994, D64 B1 H8 S2048 66.7 | 67.2, fp16
+        // 7x9 D64 B4 H12 93.6 | 93.5, 11x15 D128 B1 H32 S4096 362 | 359).  A block's results are taken up LAG products into the next turn,
+        // when they are long complete.
+        constexpr int TURNS = SCORES_ONLY ? 2 : 1;
         constexpr int NB = 2 * NCB, NREAD = NB * R;
-        // score fragments in flight (scores only: 8 and 12 measure the same, 15 spills; the attention kernel, at the
-        // 256-register limit, spills from 6 on)
+        // score fragments in flight (scores only: 8 and 12 measure the same, 15 spills; attention: 4 and 8 the same, and 8 with 7 kernel
+        // rows at D = 64 takes the third workgroup of a CU: fp16 7x9 B4 H12 S2048 92.7 | 105.4 us)
         constexpr int NLD = SCORES_ONLY ? 8 : 4;
         constexpr int NSLOT = NLD + 1;
         constexpr int LAG = 2;
@@ -601,7 +632,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         };
         // what happens to output block b = rb*NCB + cb (rows crow[rb], keys j*64 + 16cb ..) once it is complete
         uint32_t held[2];           // scores only: the even block of a pair, packed
-        float sv[NCB][4], mloc;     // attention: the row block's scaled logits and their running maximum
+        float sv[2][NCB][4], mloc, mneg[2];   // attention: a row block's logits, their maximum; minus the running maximum as the exponent takes it
         frag8<T> pf[2][2];          // attention: probabilities, in the operand layout of the P V products
         auto finish = [&](auto bc) __attribute__((always_inline)) {
             constexpr int b = decltype(bc)::value;
@@ -640,15 +671,9 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                     }
                 }
             } else {
-                // conv output and scaled logits are rounded to the I/O dtype, as the unfused pipeline stores them
-                float v4[4];
-                unpack2<T>(pack2<T>(a[0], a[1]), v4[0], v4[1]);
-                unpack2<T>(pack2<T>(a[2], a[3]), v4[2], v4[3]);
-                unpack2<T>(pack2<T>(v4[0] * scale, v4[1] * scale), v4[0], v4[1]);
-                unpack2<T>(pack2<T>(v4[2] * scale, v4[3] * scale), v4[2], v4[3]);
-                const bool c_plain = PLAIN || (j * F_BK + cb * 16 + 16 <= S && (!causal || j * F_BK + cb * 16 + 15 <= pmin));
-                if constexpr (cb == 0) mloc = -INFINITY;
-                if (!c_plain) {
+                // (fp32 from here to the probabilities: the factor goes into the exponential's multiply-add)
+                float v4[4] = {a[0], a[1], a[2], a[3]};
+                if (!whole) {
                     MTA_KEEP_BRANCH();
                     // (the column from a laundered lane index: formed here, not by every key block)
                     const int left = (causal ? (p_ < S - 1 ? p_ : S - 1) : S - 1) - (j * F_BK + cb * 16) - opaque_lane(kg) * 4;
@@ -657,36 +682,17 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                         if (v > left) v4[v] = -INFINITY;
                 }
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    sv[cb][v] = v4[v];
-                    mloc = fmaxf(mloc, v4[v]);
-                }
-                if constexpr (cb == NCB - 1) {  // the row block is complete: online softmax (a row lives in 4 lanes)
-                    mloc = max_across_groups(mloc);
-                    const float m_new = fmaxf(m_i[rb], mloc);
+                for (int v = 0; v < 4; ++v) sv[rb][cb][v] = v4[v];
+                const float m4 = fmaxf(fmaxf(v4[0], v4[1]), v4[2]);
+                mloc = cb == 0 ? fmaxf(m4, v4[3]) : fmaxf(fmaxf(mloc, m4), v4[3]);
+                if constexpr (cb == NCB - 1) {  // the row block is complete: its running maximum (a row lives in 4 lanes)
+                    const float m_new = fmaxf(m_i[rb], max_across_groups(mloc));
                     const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-                    // exp(x - m) = exp2(x*log2(e) - m*log2(e)): one multiply-add and one v_exp per element
-                    constexpr float LOG2E = 1.4426950408889634f;
-                    const float mneg = -m_use * LOG2E;
-                    const float alpha = __builtin_amdgcn_exp2f(fmaf(m_i[rb], LOG2E, mneg));
+                    // exp(scale*(x - m)) = exp2(x*scale*log2(e) - m*scale*log2(e)): one multiply-add and one v_exp per element
+                    mneg[rb] = -m_use * scale2;
+                    const float alpha = __builtin_amdgcn_exp2f(fmaf(m_i[rb], scale2, mneg[rb]));
                     m_i[rb] = m_new;
-                    float lsum = 0.0f;
-                    const uint32_t ones = pack2<T>(1.0f, 1.0f);
-#pragma unroll
-                    for (int c = 0; c < NCB; ++c) {
-                        float e[4];
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) e[v] = __builtin_amdgcn_exp2f(fmaf(sv[c][v], LOG2E, mneg));
-                        const uint32_t lo = pack2<T>(e[0], e[1]), hi = pack2<T>(e[2], e[3]);
-                        // the row sum runs over the rounded probabilities (what the P V products see): a packed dot
-                        // product with (1, 1) adds a pair in one instruction
-                        lsum = dot2_io<T>(lo, ones, lsum);
-                        lsum = dot2_io<T>(hi, ones, lsum);
-                        uint32_t *dst = reinterpret_cast<uint32_t *>(&pf[rb][c >> 1]) + (c & 1) * 2;
-                        dst[0] = lo;
-                        dst[1] = hi;
-                    }
-                    l_i[rb] = l_i[rb] * alpha + lsum;
+                    l_i[rb] *= alpha;
                     // (once the running maxima have settled, alpha is 1 in every lane for most key blocks: the 4*DB
                     // multiplications are skipped for the wavefront then)
                     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
@@ -695,6 +701,18 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                     }
                 }
             }
+        };
+        // two of a row block's probabilities: keys 16*(h/2) + 4*kg + 2*(h%2), + 1.  The row sum runs over the rounded ones (what
+        // the P V products see): a packed dot product with (1, 1).  The empty statements keep the work where it is written,
+        // among the matrix products; the compiler moves it down to where the probabilities are used.
+        auto probs = [&](auto rbc, auto hc) __attribute__((always_inline)) {
+            constexpr int rb = decltype(rbc)::value, h = decltype(hc)::value, c = h / 2, v = h % 2 * 2;
+            const float e0 = __builtin_amdgcn_exp2f(fmaf(sv[rb][c][v], scale2, mneg[rb]));
+            const float e1 = __builtin_amdgcn_exp2f(fmaf(sv[rb][c][v + 1], scale2, mneg[rb]));
+            uint32_t pk = pack2<T>(e0, e1);
+            l_i[rb] = dot2_io<T>(pk, pack2<T>(1.0f, 1.0f), l_i[rb]);
+            asm volatile("" : "+v"(pk), "+v"(l_i[rb]));
+            reinterpret_cast<uint32_t *>(&pf[rb][c >> 1])[(c & 1) * 2 + h % 2] = pk;
         };
         static_for<NLD>(issue);
         static_for<NREAD>([&](auto ic) __attribute__((always_inline)) {
@@ -711,39 +729,55 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 finish(std::integral_constant<int, blk - TURNS>{});
                 __builtin_amdgcn_sched_barrier(0);
             }
-        });
-        static_for<TURNS>([&](auto b) __attribute__((always_inline)) { finish(std::integral_constant<int, NB - TURNS + decltype(b)::value>{}); });
-        if constexpr (SCORES_ONLY) return;
-
-        // ---- O^T += V^T P^T ; V^T fragments via the LDS transpose read of the row-major V block ----
-        {
-            // slots 0..3: keys 32ks+4kg+(0..3); slots 4..7: keys 32ks+16+4kg+(0..3) -- the order of pf
-            frag8<T> vf[2];
-            auto load_vf = [&](int blk, frag8<T> &dst) {  // blk = ks * DB + db
-                const int ks = blk / DB, db = blk % DB;
-                const int key_a = ks * 32 + kg * 4 + (ln >> 2), key_b = key_a + 16;
-                const int ch = db * 2 + ((ln & 3) >> 1);  // 16-byte chunk holding head dims 16db+4(ln%4)..
-                const int sub = (ln & 1) * 4;             // element offset inside the chunk
-                const T *pa = Vb + key_a * D + ((ch ^ v_swizzle4<D>(key_a)) * 8) + sub;
-                const T *pb = Vb + key_b * D + ((ch ^ v_swizzle4<D>(key_b)) * 8) + sub;
-                struct { v4s_t a, b; } both = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pa),
-                                               __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)pb)};
-                dst = __builtin_bit_cast(frag8<T>, both);
-            };
-            load_vf(0, vf[0]);
-#pragma unroll
-            for (int blk = 0; blk < 2 * DB; ++blk) {
-                const int ks = blk / DB, db = blk % DB;
-                if (blk + 1 < 2 * DB) load_vf(blk + 1, vf[(blk + 1) & 1]);
-                mma16(oacc[0][db], vf[blk & 1], pf[0][ks]);
-                mma16(oacc[1][db], vf[blk & 1], pf[1][ks]);
+            // the first row block's probabilities, a pair at a time among the second one's products
+            if constexpr (!SCORES_ONLY) {
+                constexpr int n0 = NREAD / 2 + TURNS * LAG - 1, every = (NREAD - 1 - n0) / 8;
+                static_assert(every >= 1, "fewer products than pairs");
+                if constexpr (n > n0 && (n - n0) % every == 0 && (n - n0) / every <= 8) {
+                    probs(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - n0) / every - 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
+        });
+        if constexpr (SCORES_ONLY) {
+            static_for<TURNS>([&](auto b) __attribute__((always_inline)) { finish(std::integral_constant<int, NB - TURNS + decltype(b)::value>{}); });
+            return;
+        } else {
+            // ---- O^T += V^T P^T ; V^T fragments via the LDS transpose read of the row-major V block, VLD of them ahead ----
+            // slots 0..3 of a fragment: keys 32ks+4kg+(0..3); slots 4..7: keys 32ks+16+4kg+(0..3) -- the order of pf.
+            // A lane reads at key 4kg + ln/4 (its swizzle is the same 16 keys on) and the 16-byte chunk 2db + (ln%4)/2 of the
+            // row; the swizzle and the block number db meet in address bits 5..7, which nothing else touches.
+            constexpr int NV = 2 * DB, VLD = 4, VSLOT = VLD + 1;
+            static_assert(NV > VLD && 2 * VLD <= 15, "pipeline deeper than the work or than the counter");
+            const int key_a = kg * 4 + (ln >> 2);
+            const unsigned va = lds_addr(Vb) + (unsigned)((key_a * D + v_swizzle4<D>(key_a) * 8 + ((ln & 3) >> 1) * 8 + (ln & 1) * 4) * (int)sizeof(T));
+            struct { u32x2_t a, b; } vring[VSLOT];
+            auto vissue = [&](auto ic) __attribute__((always_inline)) {
+                constexpr int n = decltype(ic)::value, ks = n / DB, db = n % DB;
+                const unsigned at = va ^ (unsigned)(db * 32);
+                vring[n % VSLOT].a = lds_read_tr8_at(at, ks * 32 * D * (int)sizeof(T));
+                vring[n % VSLOT].b = lds_read_tr8_at(at, (ks * 32 + 16) * D * (int)sizeof(T));
+            };
+            static_for<VLD>(vissue);
+            static_for<TURNS>([&](auto b) __attribute__((always_inline)) { finish(std::integral_constant<int, NB - TURNS + decltype(b)::value>{}); });
+            // the second row block's probabilities: those of the first 32 keys, then the rest among the products with these
+            static_for<4>([&](auto h) __attribute__((always_inline)) { probs(std::integral_constant<int, 1>{}, h); });
+            static_for<NV>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int n = decltype(ic)::value, ks = n / DB, db = n % DB;
+                if constexpr (n + VLD < NV) vissue(std::integral_constant<int, n + VLD>{});
+                constexpr int younger = 2 * ((n + VLD < NV ? n + VLD : NV - 1) - n);
+                asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(vring[n % VSLOT].a), "+v"(vring[n % VSLOT].b) : "n"(younger) : "memory");
+                const frag8<T> vf = __builtin_bit_cast(frag8<T>, vring[n % VSLOT]);
+                mma16(oacc[0][db], vf, pf[0][ks]);
+                mma16(oacc[1][db], vf, pf[1][ks]);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (ks == 0 && db % (DB / 4) == 0) {
+                    probs(std::integral_constant<int, 1>{}, std::integral_constant<int, 4 + db / (DB / 4)>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            });
         }
         }
-    };
-    auto plain = [&](int j) {  // (scores-only kernel: a second body per buffer rotation makes the attention kernel spill)
-        const int cbase = j * F_BK + G::PWR;
-        return SCORES_ONLY && j >= 0 && cbase + F_BK <= S && (!causal || cbase + F_BK - 1 <= pmin) && (!BAND || cbase >= fmax_w);
     };
     if constexpr (SCORES_ONLY) {
         for (int j = j_start;;) {  // block(tag, j, K(j), V(j), where K(j+1) goes, where V(j+1) goes)
@@ -755,13 +789,13 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
             if (++j > j_end) break;
         }
     } else {
-        for (int j = j_start;;) {
-            block(std::false_type{}, j, B0, B1, B2, B0);
-            if (++j > j_end) break;
-            block(std::false_type{}, j, B2, B0, B1, B2);
-            if (++j > j_end) break;
-            block(std::false_type{}, j, B1, B2, B0, B1);
-            if (++j > j_end) break;
+        int kb = 0, vb = TILE, nb = 2 * TILE;   // where K(j) and V(j) are, and the third buffer
+        for (int j = j_start; j <= j_end; ++j) {
+            block(std::false_type{}, j, KV + kb, KV + vb, KV + nb, KV + kb);
+            const int k_next = nb;
+            nb = vb;
+            vb = kb;
+            kb = k_next;
         }
     }
 
@@ -795,7 +829,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         const int tr_ = wave * 32 + rb * 16 + ln_o + cshift, p_ = q0 - G::HR + tr_;
         if (tr_ >= G::HR && tr_ < wave * 32 + 32 && p_ < S) {
             const float inv = 1.0f / l_row;
-            if (Lse != nullptr && kg_o == 0) Lse[bh * (int64_t)S + p_] = m_i[rb] + __logf(l_row);
+            if (Lse != nullptr && kg_o == 0) Lse[bh * (int64_t)S + p_] = m_i[rb] * scale_abs + __logf(l_row);
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const uint32_t lo = pack2<T>(oacc[rb][db][0] * inv, oacc[rb][db][1] * inv);
@@ -817,18 +851,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
     static_assert(G::fits, "conv window exceeds the 32-key MFMA contraction");
     const int nqb = (int)((S + G::BQ - 1) / G::BQ);
-    // Output blocks of the conv in turns (1 | 2, us): the scores kernels gain up to 1.5 % (bf16 6x11 B1 H16 S2048 D64 34.3 | 33.9, B4 H16
-    // S1024 D128 39.8 | 39.3, fp16 7x7 B1 H16 S2048 D128 41.6 | 41.2), the attention kernel of 11 rows -1 to 2 % (fp16 B1 H16 S2048 D64 103.8 |
-    // 102.2, bf16 D128 119.9 | 118.7, B4 H12 D64 151.3 | 152.3).  Of up to 7 rows it is slower in bf16 (3x3 B1 H32 S4096 D128 275.9 | 278.8, 6x11
-    // B1 H8 S2048 D64 78.9 | 79.9, 7x7 B1 H16 S2048 D128 98.8 | 99.6, larger grids within 0.5 %) and in fp16 with 3 rows (B1 H8 S2048 D64 75.2 | 76.4);
-    // fp16 with 5 to 7 rows loses while its workgroups fit the chip at once (6x11 D64 B1 H8 S2048 82.0 | 84.4, H16 83.2 | 85.4, D128 98.3 |
-    // 99.4), and gains beyond (7x7 D64 B4 H12 S2048 120.3 | 119.6, 6x11 D128 B1 H32 S4096 313 | 310).
-    constexpr bool BY_GRID = !SCORES_ONLY && __is_same(T, f16_t) && R > 3 && R <= 7;
-    constexpr int TURNS = SCORES_ONLY || R > 7 || BY_GRID ? 2 : 1;
-    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND, TURNS>;
-    if constexpr (BY_GRID) {
-        if (B * H * nqb <= 2 * (int64_t)device_cu_count()) kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND, 1>;
-    }
+    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND>;
     // key blocks per work item: all of them for the attention kernel; QK_CHUNK for the scores-only kernel
     const int jc_len = SCORES_ONLY ? QK_CHUNK : (int)((S + F_BK - 1) / F_BK) + 1;
     int64_t items_per_bh = 0;

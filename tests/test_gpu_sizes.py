@@ -35,6 +35,25 @@ def test_conv_attention_kernel_sizes(pkg, dtype, r, sk, d, causal):
         torch.testing.assert_close(got.float(), want.float(), **tol(dtype))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("factor", [-0.08, 0.0, 0.08])
+@pytest.mark.parametrize("dtype,d,r,sk", [(torch.bfloat16, 128, 6, 11), (torch.float16, 64, 3, 3), (torch.float16, 128, 11, 15)])
+def test_conv_attention_factor(pkg, dtype, d, r, sk, factor, causal):
+    """Factors of either sign and 0 (the kernel's maxima are taken ahead of the factor): one row, one 64-key block and its edges, the
+    edge of a query block and rows that take more than one of them.  Output and row statistic against the oracle in fp32; bounds as for
+    the default factor (test_conv_attention_lse), which is no smaller: the scores are rounded to 16 bits ahead of it."""
+    for s in (1, 64, 65, 130, 200):
+        print(f"conv_attention {dtype} {r}x{sk} d={d} s={s} factor={factor} causal={causal}", flush=True)
+        q, k, v = O.seeded_qkv(1, 2, s, d, dtype, seed=44)
+        w = O.seeded_conv_weight(2, r, sk, 0.05, dtype)
+        scores = O.conv_attention_scores(q.float(), k.float(), w.float(), causal, 1.0)
+        scores = torch.where(torch.isinf(scores), scores, scores * factor)   # (a key above the diagonal has no weight, whatever the factor)
+        o, lse = pkg.ops.conv_attn_fwd(q.cuda(), k.cuda(), v.cuda(), w.cuda(), causal, factor, return_lse=True)
+        want = torch.matmul(torch.softmax(scores, -1), v.float())
+        torch.testing.assert_close(o.cpu().float(), want, **tol(dtype))
+        torch.testing.assert_close(lse.cpu(), torch.logsumexp(scores, -1), rtol=2.0 ** -7, atol=2e-2)
+
+
 @pytest.mark.parametrize("dtype,r,sk", [(torch.bfloat16, 3, 5), (torch.float16, 7, 9)])
 def test_qk_conv_kernel_sizes(pkg, dtype, r, sk):
     """The scores stage at the same sizes; bound as in test_qk_conv_parity: two 16-bit roundings of scores of magnitude
