@@ -736,7 +736,7 @@ template <bool BWD>
 int conv2d_entry(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,
                  int S, int causal, float in_scale, int use_scale, int io_dtype, int w_dtype, void *stream)
 {
-    // MTA_CONV_FORCE_VALU=1 in the environment keeps 16-bit inputs on the fp32-FMA kernel (for comparisons)
+    // MTA_CONV_FORCE_VALU=1 in the environment keeps everything on the fp32-FMA kernels (for comparisons)
     static const bool force_valu = [] { const char *e = getenv("MTA_CONV_FORCE_VALU"); return e && e[0] == '1'; }();
     if (!x || !w || !y) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
@@ -754,6 +754,10 @@ int conv2d_entry(const void *x, const void *w, void *y, int64_t N, int64_t C, in
     MTA_DISPATCH_IO(io_dtype, {
         if (mfma_ok) {
             const int rc = dispatch_mfma<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, st);
+            if (rc != 1) return rc;
+        }
+        if (!force_valu) {
+            const int rc = conv2d_split_dispatch(x, w, y, N, C, H, W, R, S, BWD, causal, in_scale, use_scale, io_dtype, w_dtype, st);
             if (rc != 1) return rc;
         }
         const int rc = dispatch_rows<io_t, BWD>(x, w, y, N, C, H, W, R, S, causal, in_scale, use_scale, w_dtype, st);

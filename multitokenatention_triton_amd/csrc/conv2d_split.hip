@@ -1,0 +1,410 @@
+// Depthwise conv of 11x15 kernels, forward and input gradient, for what the kernels of conv2d_causal.hip on the matrix cores do not
+// take (fp32 data; 16-bit data with weights of another dtype or rows that are not whole 16-byte vectors): on the bf16 matrix
+// cores, with the 32 bits kept.
+//
+// Every fp32 value is the sum of three bf16 values (8 + 8 + 8 bits of its significand; each one the rounded remainder of those
+// before it), exactly: x = x0 + x1 + x2, w = w0 + w1 + w2 (fp16: two parts, bf16: one).  Of the products of parts the six with
+// i + j <= 2 are formed; each is exact in fp32, what is left out is below 2^-26 |x w|, a quarter of the last place that one fp32
+// multiply-add rounds away.  A kernel row is applied as in conv2d_causal.hip, as a banded Toeplitz product (one 32-key window
+// holds the taps of 16 outputs), once per pair of parts: w0 x0 adds into one accumulator, the small ones into two others, and a
+// result is their sum.  So an output takes R roundings of its own size where multiply-adds took R*S: the error against 64 bits
+// (2-norm) is 0.55e-7 forward and 1.0e-7 for the input gradient, where they left 1.3e-7 and 2.9e-7 (scores, 333^2 and 512^2).
+//
+// Why: R*S multiply-adds on the vector units (0.079 PFLOP/s without packed fp32 forms) bound the row-sliding kernels from about 50
+// taps on.  The Toeplitz form executes 6 * 64 * R flops for the 2*R*S of an output, at 2.5 PFLOP/s: 2.5 times the vector rate.
+// us, conv2d_rows -> this, fp32: lower triangle 16 planes of 512^2 23 -> 18.5, 12 of 801^2 32 -> 28.5, 16 of 1024^2 58 -> 38, 32 of
+// 1024^2 105 -> 68, 16 of 2048^2 177 -> 128; whole rows 31 -> 20, 34 -> 31, 86 -> 43, 152 -> 80, 260 -> 151.  Smaller kernels stay
+// there, lower triangle | whole rows: 7x9 16 of 1024^2 29.7 | 39.4 against 29.4 | 34.5 here, 16 of 512^2 13.9 | 16.4 against 15.3 |
+// 16.5, 16 of 2048^2 92 | 128 against 98 | 140; 6x11 and 5x7 alike or slower.
+// What bounds it: half of the time the matrix cores are busy (16 of 2048^2: 62 of 128 us); without the loads, stores and
+// the splitting the products take 95 us - their operands' LDS reads, the barrier of a strip and the blocks beside the
+// triangle - and the CU's path to the L2 (1.5 times the strip in, the strip out) the rest.
+// What is not finite, or so large that a part overflows, takes multiply-adds after all; a strip whose largest value is so small
+// that parts underflow is staged once more, 2^100 times as large (its results are taken back).
+//
+// Shape.  A workgroup of four wavefronts takes strips of 32 rows x 128 keys of one plane, one after the other, two workgroups per
+// CU.  A strip and its halo are loaded four keys per lane, two strips ahead, into registers; split and written to one of two LDS
+// buffers (a plane of bf16 per part with rows of 288 bytes, for which a fragment read - 16 rows x 64 bytes - is free of bank
+// conflicts) a vector at a time between the products of the strip before.  The Toeplitz fragments of the plane's kernel stay in
+// registers (3 * R * 4 of them); they come out of a table of all windows of every kernel row.
+#include "conv2d_rows.hpp"
+#include "mfma.hpp"
+
+#include <type_traits>
+
+namespace {
+using namespace mta;
+
+constexpr int P_TM = 32, P_TN = 128;       // strip
+constexpr int P_HL = 8;                    // keys staged left (and right) of it
+constexpr int P_LD = P_TN + 2 * P_HL;      // keys of a staged row
+constexpr int P_QUADS = P_LD / 4;
+
+typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+
+// two values' parts, packed: a part is the rounded remainder.  (The packed dot product with (-1, 0) or (0, -1) takes one of the two
+// values off a remainder without unpacking it: one instruction in place of two.)
+template <int N> __device__ __forceinline__ void split2(float a, float b, uint32_t (&part)[N])
+{
+    // (constants the compiler cannot see: it would fold (-1, 0) into the inline constant -1.0, which the instruction takes for (0, -1))
+    uint32_t minus_lo = 0x0000bf80u, minus_hi = 0xbf800000u;
+    asm("" : "+s"(minus_lo), "+s"(minus_hi));
+    const mta_bf16x2 lo = __builtin_bit_cast(mta_bf16x2, minus_lo), hi = __builtin_bit_cast(mta_bf16x2, minus_hi);
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        part[s] = pack2<bf16_t>(a, b);
+        if (s == N - 1) break;
+        const mta_bf16x2 h = __builtin_bit_cast(mta_bf16x2, part[s]);
+        a = __builtin_amdgcn_fdot2_f32_bf16(h, lo, a, false);
+        b = __builtin_amdgcn_fdot2_f32_bf16(h, hi, b, false);
+    }
+}
+
+// strips that touch the lower triangle (all of them unless `tri`), column of strips by column of strips
+__host__ __device__ __forceinline__ int p_first(int tn, int tri) { return tri ? tn * P_TN / P_TM : 0; }
+inline int64_t p_count(int64_t H, int64_t W, int tri)
+{
+    const int tiles_m = (int)((H + P_TM - 1) / P_TM), tiles_n = (int)((W + P_TN - 1) / P_TN);
+    int64_t n = 0;
+    for (int tn = 0; tn < tiles_n; ++tn) n += tiles_m > p_first(tn, tri) ? tiles_m - p_first(tn, tri) : 0;
+    return n;
+}
+
+// What a set of values holds, from the largest magnitude of their first parts: bits of a strip's state word
+enum : unsigned { P_HUGE = 1, P_USUAL = 2, P_NONZERO = 4 };
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void raise(uint32_t &top, uint32_t part)
+{
+    top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top), __builtin_bit_cast(u16x2, part & 0x7fff7fffu)));
+}
+__device__ __forceinline__ unsigned state_of(uint32_t tops)   // of a wavefront's values
+{
+    const unsigned top = max(tops & 0xffffu, tops >> 16);
+    return (__builtin_amdgcn_ballot_w64(top >= 0x7f80u) ? P_HUGE : 0u) | (__builtin_amdgcn_ballot_w64(top >= (27u << 7)) ? P_USUAL : 0u) |
+           (__builtin_amdgcn_ballot_w64(top != 0u) ? P_NONZERO : 0u);
+}
+__device__ __forceinline__ bool tiny(unsigned state) { return (state & (P_USUAL | P_NONZERO)) == P_NONZERO; }
+
+template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
+
+template <typename T, int R, int S, bool BWD>
+__global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
+                                                       int W, int causal, float in_scale, int use_scale, int w_dtype, int planes, int total, int per_plane)
+{
+    constexpr int PAD = BWD ? S - 1 - (S - 1) / 2 : (S - 1) / 2, SHIFT = P_HL - PAD;   // first tap's slot in a 32-key window
+    static_assert(SHIFT >= 0 && SHIFT + 16 + S - 1 <= 32 && S - 1 - PAD <= P_HL, "the taps of 16 outputs in a window of 32 keys");
+    constexpr int ROWS = P_TM + R - 1, RPI = 256 / P_QUADS, IT = (ROWS + RPI - 1) / RPI;   // a round of loads: RPI rows, four threads idle
+    constexpr int PLANE = ROWS * P_LD;                 // bf16 values of one part
+    constexpr int NE = S + 7;                          // windows of a kernel row that hold a tap: first slot - SHIFT - ln = -7 .. S-1
+    constexpr int XP = parts_of<T>(), WP = 3;          // parts of a value, of a tap
+    __shared__ __align__(16) uint16_t xs[2][XP * PLANE];
+    static_assert(WP * R * (NE + 1) * 8 + WP * R * (S + 16) <= 2 * XP * PLANE, "the table of windows borrows the strips' LDS");
+    __shared__ unsigned state[4];                      // of the strips staged, one in three in turns; [3]: of the kernel
+    constexpr float UP = 1.2676506002282294e30f, DOWN = 1.0f / UP;   // 2^100
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    // (planes dealt to the XCDs where they divide evenly: a plane's strips share their halo rows in one L2)
+    int plane, first;
+    if (planes % 8 == 0) {
+        const int pos = (int)(blockIdx.x >> 3);
+        plane = (int)(blockIdx.x & 7) * (planes / 8) + pos / per_plane;
+        first = pos % per_plane;
+    } else {
+        plane = (int)blockIdx.x / per_plane;
+        first = (int)blockIdx.x % per_plane;
+    }
+    const int c = plane % C;
+    const T *xp = x + plane * (int64_t)H * W;
+    T *yp = y + plane * (int64_t)H * W;
+    const bool tri = causal != 0;
+
+    struct strip { int p0, q0; };
+    // strips in the order that this workgroup takes them: `per_plane` further on each time (a column holds many of those steps: found
+    // afresh from its number, a strip cost a loop over the columns)
+    const int tiles_m = (H + P_TM - 1) / P_TM;
+    int col = 0, at = first;
+    auto next_strip = [&]() {
+        for (int n; at >= (n = tiles_m > p_first(col, tri) ? tiles_m - p_first(col, tri) : 0); ++col) at -= n;
+        const strip t{(p_first(col, tri) + at) * P_TM, col * P_TN};
+        at += per_plane;
+        return t;
+    };
+    auto top_row = [](strip t) { return BWD ? t.p0 : t.p0 - (R - 1); };
+    // no value of the strip or its halo lies outside the plane or above the diagonal
+    auto inside = [&](strip t) {
+        const int h0 = top_row(t);
+        return h0 >= 0 && h0 + ROWS <= H && t.q0 >= P_HL && t.q0 + P_TN + P_HL <= W && (!causal || t.q0 + P_TN + P_HL - 1 <= h0);
+    };
+    quad4<T> raw[IT];
+    const int lr = tid / P_QUADS, lk = tid % P_QUADS * 4;      // this lane's row in a round of loads, and its keys
+    // (rows and keys outside the plane re-read the nearest inside)
+    auto fetch = [&](strip t, int it) __attribute__((always_inline)) {
+        const int h0 = top_row(t), base = h0 < 0 ? 0 : h0, k = t.q0 - P_HL + lk, h = h0 + lr + it * RPI;
+        const char *from = reinterpret_cast<const char *>(xp + (int64_t)base * W);
+        const int hc = h < base ? base : (h >= H ? H - 1 : h), kc = k < 0 ? 0 : (k > W - 4 ? W - 4 : k);
+        __builtin_memcpy(&raw[it], from + (unsigned)((hc - base) * W + kc) * (unsigned)sizeof(T), sizeof(raw[it]));
+    };
+    // vector `it` of a strip: masked, scaled, split, to LDS
+    auto stage = [&](strip t, bool plain, int it, uint16_t *to, float by, uint32_t &top) __attribute__((always_inline)) {
+        const int r = lr + it * RPI;
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = to_float(raw[it].v[u]);
+        if (!plain) {
+            asm volatile("" : : : "memory");   // (kept a branch)
+            const int k = t.q0 - P_HL + lk, h = top_row(t) + r;
+            masked_quad<T>(raw[it], k, W, (h < 0 || h >= H) ? -1 : (causal && h < W - 1 ? h : W - 1), v);
+        }
+        if (use_scale || by != 1.0f) {
+            asm volatile("" : : : "memory");
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = (use_scale ? round_to<T>(v[u] * in_scale) : v[u]) * by;
+        }
+        uint32_t a[XP], b[XP];
+        split2<XP>(v[0], v[1], a);
+        split2<XP>(v[2], v[3], b);
+        if (lr < RPI && ((it + 1) * RPI <= ROWS || r < ROWS)) {
+            raise(top, a[0]);
+            raise(top, b[0]);
+#pragma unroll
+            for (int s = 0; s < XP; ++s) *reinterpret_cast<uint2 *>(to + s * PLANE + r * P_LD + lk) = make_uint2(a[s], b[s]);
+        }
+    };
+    strip t{0, 0}, next{0, 0};
+    if (first < total) {
+        t = next_strip();
+#pragma unroll
+        for (int it = 0; it < IT; ++it) fetch(t, it);     // in flight while the kernel is prepared
+    }
+
+    // ---- the kernel's fragments: lane (ln, kg), slot t holds tap 8*kg + t - SHIFT - ln ----
+    frag8<bf16_t> tz[WP][R];
+    float unscale = 1.0f;
+    unsigned w_state;
+    {
+        constexpr int NT = (R * (S + 16) + 255) / 256;
+        uint16_t *const table = xs[0], *const taps = table + WP * R * (NE + 1) * 8;   // [part][row][8 zeros, S taps, 8 zeros]
+        if (tid < 4) state[tid] = 0;
+        float v[NT];
+        uint32_t top = 0;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int e = n * 256 + tid, i = e / (S + 16), j = e % (S + 16) - 8;
+            v[n] = i < R && j >= 0 && j < S ? load_any(w, w_dtype, (int64_t)c * R * S + (BWD ? R * S - 1 - (i * S + j) : i * S + j)) : 0.0f;
+            raise(top, pack2<bf16_t>(v[n], 0.0f));
+        }
+        __syncthreads();
+        const unsigned mine = state_of(top);
+        if (lane == 0) atomicOr(&state[3], mine);
+        __syncthreads();
+        w_state = state[3];
+        if (tiny(w_state)) unscale = DOWN;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int e = n * 256 + tid;
+            uint32_t part[WP];
+            split2<WP>(tiny(w_state) ? v[n] * UP : v[n], 0.0f, part);
+            if (e < R * (S + 16)) {
+#pragma unroll
+                for (int s = 0; s < WP; ++s) taps[s * R * (S + 16) + e] = (uint16_t)part[s];
+            }
+        }
+        __syncthreads();
+        for (int e = tid; e < WP * R * (NE + 1); e += 256) {
+            const int row = e / (NE + 1), k = e % (NE + 1);   // window k: taps k-7 .. k; the last one: none
+            u16x8 win;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) win[u] = k < NE ? taps[row * (S + 16) + 1 + k + u] : (uint16_t)0;
+            *reinterpret_cast<u16x8 *>(table + e * 8) = win;
+        }
+        __syncthreads();
+        const int from = 8 * kg - SHIFT - ln + 7;
+#pragma unroll
+        for (int s = 0; s < WP; ++s)
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+                tz[s][i] = *reinterpret_cast<const frag8<bf16_t> *>(table + ((s * R + i) * (NE + 1) + (from >= 0 && from < NE ? from : NE)) * 8);
+        __syncthreads();
+    }
+    if (first < total) {
+        const bool plain = inside(t);
+        uint32_t top = 0;
+#pragma unroll
+        for (int it = 0; it < IT; ++it) stage(t, plain, it, xs[0], 1.0f, top);
+        const unsigned mine = state_of(top);
+        if (lane == 0) atomicOr(&state[0], mine);
+        if (first + per_plane < total) {
+            next = next_strip();
+#pragma unroll
+            for (int it = 0; it < IT; ++it) fetch(next, it);
+        }
+    }
+    __syncthreads();
+
+    for (int id = first, n = 0, n3 = 0; id < total; id += per_plane, n ^= 1) {
+        const unsigned now = state[n3];
+        const int n3_next = n3 == 2 ? 0 : n3 + 1;
+        if (tid == 0) state[n3_next == 2 ? 0 : n3_next + 1] = 0;   // (the next but one: nobody reads or writes it before the barrier below)
+        float down = unscale;
+        if (tiny(now) || (now & P_HUGE)) {
+            asm volatile("" : : : "memory");
+            if (!(now & P_HUGE)) {     // all of it so small that parts underflow: staged once more, 2^100 times as large
+                quad4<T> keep[IT];
+#pragma unroll
+                for (int it = 0; it < IT; ++it) keep[it] = raw[it];
+                uint32_t top = 0;
+#pragma unroll
+                for (int it = 0; it < IT; ++it) {
+                    fetch(t, it);
+                    stage(t, false, it, xs[n], UP, top);
+                    raw[it] = keep[it];
+                }
+                __syncthreads();
+                down *= DOWN;
+            }
+        }
+        const bool more = id + per_plane < total, more2 = id + 2 * per_plane < total;
+        const strip after = more2 ? next_strip() : t;   // (asked for either way: behind a branch around the loads their waits would be waits for all)
+        const bool plain = inside(next);
+        // ---- four blocks of 16 x 16 per wavefront (16 rows x 64 keys), in halves of the kernel rows.  The operands of a kernel row are read
+        // while the row before is multiplied (the order is pinned).  Between the halves the next strip's vectors go to the other
+        // buffer, one by one, and those of the strip behind it are asked for ----
+        const uint16_t *xw = xs[n] + ((wave & 1) * 16 + ln) * P_LD + (wave >> 1) * 64 + kg * 8;
+        frag8<bf16_t> f[2][XP];
+        auto read = [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < XP; ++s) f[m & 1][s] = *reinterpret_cast<const frag8<bf16_t> *>(xw + s * PLANE + m % R * P_LD + m / R * 16);
+        };
+        const int lower = causal ? (t.p0 + (wave & 1) * 16 + 15 - t.q0 - (wave >> 1) * 64) >> 4 : 3;   // last block that touches the triangle
+        // (address of a lane's results: a uniform base and a byte offset within the strip)
+        const int pl = (wave & 1) * 16 + ln, ql = (wave >> 1) * 64 + kg * 4;
+        char *const ybase = reinterpret_cast<char *>(yp + (int64_t)t.p0 * W + t.q0);
+        const unsigned yoff = (unsigned)(pl * W + ql) * (unsigned)sizeof(T);
+        const bool whole = t.p0 + P_TM <= H && t.q0 + P_TN <= W && (!causal || t.q0 + P_TN - 1 <= t.p0) && !((now | w_state) & P_HUGE);
+        uint32_t top = 0;
+        read(0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            f32x4 big{0.0f, 0.0f, 0.0f, 0.0f}, small0 = big, small1 = big;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                if (b <= lower) {
+#pragma unroll
+                    for (int i = half ? R / 2 : 0; i < (half ? R : R / 2); ++i) {
+                        const int m = b * R + i;
+                        if (m + 1 < 4 * R) read(m + 1);
+                        if constexpr (XP > 2) mma16(small0, tz[0][i], f[m & 1][2]);
+                        mma16(small1, tz[1][i], f[m & 1][0]);
+                        if constexpr (XP > 1) mma16(small0, tz[1][i], f[m & 1][1]);
+                        if constexpr (XP > 1) mma16(small1, tz[0][i], f[m & 1][1]);
+                        mma16(small0, tz[2][i], f[m & 1][0]);
+                        mma16(big, tz[0][i], f[m & 1][0]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                constexpr int LEAD = 8 - IT;     // (not ahead of the last strip's stores: loads and stores complete on one counter)
+                const int it = b * 2 + half - LEAD;
+                if (it >= 0) {
+                    if (more) stage(next, plain, it, xs[n ^ 1], 1.0f, top);
+                    fetch(after, it);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // (stores of 16 rows x 64 bytes; the second half of a 128-byte line follows with the next block)
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = big[u] + (small0[u] + small1[u]);
+            if (down != 1.0f) {
+                asm volatile("" : : : "memory");
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] *= down;
+            }
+            if (whole) {
+                asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));   // (one store, not one shared in part with the other branch)
+                quad4<T> o;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[u]);
+                __builtin_memcpy(ybase + yoff + b * 16 * (int)sizeof(T), &o, sizeof(o));
+            } else {
+                const int p = t.p0 + pl, q = t.q0 + ql + b * 16;
+                if (!((now | w_state) & P_HUGE) && p < H && q < W && !(causal == 2 && q > p)) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[u] = causal && q + u > p ? 0.0f : v[u];
+                    store_quad<T>(yp + (int64_t)p * W, q, W, v);
+                }
+            }
+        }
+        if ((now | w_state) & P_HUGE) {   // values that do not split: multiply-adds, tap by tap
+            for (int e = opaque(tid); e < P_TM * P_TN; e += 256) {
+                const int pe = t.p0 + e / P_TN, q = t.q0 + e % P_TN;
+                if (pe >= H || q >= W || (causal == 2 && q > pe)) continue;
+                float sum = 0.0f;
+                for (int i = 0; i < R && !(causal && q > pe); ++i) {
+                    const int h = BWD ? pe + i : pe - (R - 1) + i;
+                    if (h < 0 || h >= H) continue;
+                    for (int j = 0; j < S; ++j) {
+                        const int k = q - PAD + j;
+                        if (k < 0 || k >= W || (causal && k > h)) continue;
+                        float v = to_float(xp[(int64_t)h * W + k]);
+                        if (use_scale) v = round_to<T>(v * in_scale);
+                        sum = fmaf(load_any(w, w_dtype, (int64_t)c * R * S + (BWD ? R * S - 1 - (i * S + j) : i * S + j)), v, sum);
+                    }
+                }
+                yp[(int64_t)pe * W + q] = from_float<T>(sum);
+            }
+        }
+        if (more) {
+            const unsigned mine = state_of(top);
+            if (lane == 0) atomicOr(&state[n3_next], mine);
+        }
+        t = next;
+        next = after;
+        n3 = n3_next;
+        __syncthreads();
+    }
+    if (causal == 1) {     // the strips wholly above the diagonal
+        const int tiles = tiles_m * ((W + P_TN - 1) / P_TN);
+        for (int id = first; id < tiles; id += per_plane) {
+            const int p0 = id % tiles_m * P_TM, q0 = id / tiles_m * P_TN;
+            if (q0 <= p0 + P_TM - 1) continue;
+            for (int e = tid; e < P_TM * (P_TN / 4); e += 256) {
+                const int p = p0 + e / (P_TN / 4), q = q0 + e % (P_TN / 4) * 4;
+                T *dst = yp + (int64_t)p * W + q;
+                const T zero = from_float<T>(0.0f);
+                const quad4<T> z = {{zero, zero, zero, zero}};
+                if (p >= H || q >= W) continue;
+                if (q + 4 <= W) {
+                    __builtin_memcpy(dst, &z, sizeof(z));
+                } else {
+                    asm volatile("" : : : "memory");
+                    for (int u = 0; u < W - q; ++u) dst[u] = zero;
+                }
+            }
+        }
+    }
+}
+
+template <typename T, int R, int S, bool BWD>
+int launch_split(const void *x, const void *w, void *y, int64_t planes, int64_t C, int64_t H, int64_t W, int causal, float in_scale, int use_scale,
+                 int w_dtype, hipStream_t st)
+{
+    const int64_t total = p_count(H, W, causal != 0);
+    if (total > 0x3fffffffLL) return MTA_ERR_SHAPE;
+    int64_t per_plane = (2 * device_cu_count() + planes - 1) / planes;   // one round of resident workgroups
+    if (per_plane > total) per_plane = total;
+    hipLaunchKernelGGL((conv2d_split<T, R, S, BWD>), dim3((unsigned)(planes * per_plane)), dim3(256), 0, st, (const T *)x, w, (T *)y, (int)C, (int)H,
+                       (int)W, causal, in_scale, use_scale, w_dtype, (int)planes, (int)total, (int)per_plane);
+    return launch_status();
+}
+}  // namespace
+
+int mta::conv2d_split_dispatch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,
+                               float in_scale, int use_scale, int io_dtype, int w_dtype, hipStream_t st)
+{
+    if (R != 11 || S != 15 || W < 4) return 1;
+    MTA_DISPATCH_IO(io_dtype, {
+        return bwd ? launch_split<io_t, 11, 15, true>(x, w, y, N * C, C, H, W, causal, in_scale, use_scale, w_dtype, st)
+                   : launch_split<io_t, 11, 15, false>(x, w, y, N * C, C, H, W, causal, in_scale, use_scale, w_dtype, st);
+    });
+    return 1;
+}

@@ -938,3 +938,69 @@ def test_softmax_of_a_window_wider_than_its_rows(pkg, group, dtype):
             run = lambda lo: _bits(pkg.ops.headmix_softmax(x, w1, w2, True, group_size=group, first_visible=lo))  # noqa: E731
             got = run(first)
             assert torch.equal(got, run(first.clamp(min=0))) and not got.view(dtype).isnan().any()
+
+
+def _conv64(x, w, causal, bwd):
+    """The depthwise conv (or its input gradient) in 64 bits, and the sum of the magnitudes it adds up."""
+    r, k = w.shape[-2:]
+    x, w = x.double(), w.double()
+    low = torch.ones(x.shape[-2:], dtype=torch.bool, device=x.device).tril()
+    if causal:
+        x = torch.where(low, x, 0.0)
+    pad, padr = (k - 1) // 2, k - 1 - (k - 1) // 2
+    x = torch.nn.functional.pad(x, (padr, pad, 0, r - 1) if bwd else (pad, padr, r - 1, 0))
+    w = w.flip(-1, -2) if bwd else w
+    both = [torch.nn.functional.conv2d(a.cpu(), b.cpu()[:, None], groups=x.shape[1]).cuda() for a, b in ((x, w), (x.abs(), w.abs()))]
+    return [torch.where(low, y, 0.0) for y in both] if causal else both
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                          (torch.float16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("h,w", [(1, 4), (31, 127), (33, 129), (64, 128), (40, 300), (300, 70), (389, 389)])
+def test_conv_11x15_split(pkg, h, w, dtype, wdtype):
+    """11x15 kernels on the parts of the values (fp32; 16-bit data with other weights or of odd widths): edges of the 32 x 128 strips,
+    planes that take one strip and several in turns, wide and tall ones; forward, scaled, lower triangle only, input gradient; causal
+    or not.  Bound: 165 products and sums of 32 bits in any order, (165 + 2) 2^-24 of the sum of their magnitudes, and one rounding
+    of the result to its type."""
+    g = torch.Generator(device="cuda").manual_seed(61)
+    x = torch.randn(2, 3, h, w, generator=g, device="cuda").to(dtype)
+    k = (0.1 * torch.randn(3, 11, 15, generator=g, device="cuda")).to(wdtype)
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+
+    def close(got, x, causal, bwd):
+        want, size = _conv64(x, k, causal, bwd)
+        assert ((got.double() - want).abs() <= 167 * 2.0 ** -24 * size + ulp * want.abs() + 2.0 ** -25 * (dtype == torch.float16)).all()
+
+    for causal in (True, False):
+        close(pkg.ops.conv2d_causal(x, k, causal), x, causal, False)
+        close(pkg.ops.conv2d_bwd_input(x, k, causal), x, causal, True)
+    close(pkg.ops.conv2d_causal(x, k, True, in_scale=0.3), (x.float() * 0.3).to(dtype), True, False)
+    out = torch.full_like(x, 7.0)
+    pkg.ops.conv2d_causal(x, k, True, out=out, fill_upper=False)
+    close(torch.tril(out), x, True, False)
+
+
+@pytest.mark.parametrize("bwd", [False, True])
+def test_conv_11x15_split_values(pkg, bwd):
+    """Values that do not split into bf16 parts: infinities and NaN stay where a tap takes them, the largest numbers are not taken for
+    infinite, and data or weights so small that their parts underflow keep their 32 bits."""
+    g = torch.Generator(device="cuda").manual_seed(62)
+    k = 0.1 * torch.randn(2, 11, 15, generator=g, device="cuda")
+    run = (lambda x, k: pkg.ops.conv2d_bwd_input(x, k, True)) if bwd else (lambda x, k: pkg.ops.conv2d_causal(x, k, True))
+    x = torch.randn(1, 2, 200, 200, generator=g, device="cuda")
+    plain = run(x, k)
+    for value in (float("inf"), float("-inf"), float("nan")):
+        y = x.clone()
+        y[0, 0, 120, 60] = value
+        got = run(y, k)
+        touched = torch.zeros(200, 200, dtype=torch.bool, device="cuda")
+        touched[(slice(110, 121) if bwd else slice(120, 131)), 53:68] = True
+        assert not torch.isfinite(got[0, 0][touched.tril()]).any()
+        torch.testing.assert_close(got[0, 0][~touched], plain[0, 0][~touched], rtol=1e-4, atol=1e-5)
+        assert torch.equal(got[0, 1], plain[0, 1])
+    y = torch.zeros_like(x)
+    y[0, 0, 150, 70] = 3.4e38
+    want = _conv64(y, 0.01 * k, True, bwd)[0]
+    torch.testing.assert_close(run(y, 0.01 * k).double(), want, rtol=2.0 ** -22, atol=0.0)
+    for sx, sk in ((2.0 ** -115, 1.0), (1.0, 2.0 ** -115), (2.0 ** -60, 2.0 ** -60)):
+        torch.testing.assert_close(run(x * sx, k * sk) * (1 / (sx * sk)), plain, rtol=2.0 ** -20, atol=2.0 ** -20)
