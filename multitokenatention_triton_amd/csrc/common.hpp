@@ -186,4 +186,6 @@ int conv_mix16_dispatch(const void *x, const void *wc, const void *wm, void *y, 
 // causal as in conv2d_causal.hip); 1 where it has no instance
 int conv2d_split_dispatch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,
                           float in_scale, int use_scale, int io_dtype, int w_dtype, hipStream_t st);
+// tri_products_split.hip: lower-triangle scores of fp32 operands on the bf16 matrix cores with the 32 bits kept
+int lower_scores_split_launch(const void *a, const void *b, void *c, int64_t heads, int64_t S, int64_t D, hipStream_t st);
 }  // namespace mta

@@ -28,9 +28,7 @@
 // conflicts) a vector at a time between the products of the strip before.  The Toeplitz fragments of the plane's kernel stay in
 // registers (3 * R * 4 of them); they come out of a table of all windows of every kernel row.
 #include "conv2d_rows.hpp"
-#include "mfma.hpp"
-
-#include <type_traits>
+#include "split.hpp"
 
 namespace {
 using namespace mta;
@@ -41,24 +39,6 @@ constexpr int P_LD = P_TN + 2 * P_HL;      // keys of a staged row
 constexpr int P_QUADS = P_LD / 4;
 
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
-
-// two values' parts, packed: a part is the rounded remainder.  (The packed dot product with (-1, 0) or (0, -1) takes one of the two
-// values off a remainder without unpacking it: one instruction in place of two.)
-template <int N> __device__ __forceinline__ void split2(float a, float b, uint32_t (&part)[N])
-{
-    // (constants the compiler cannot see: it would fold (-1, 0) into the inline constant -1.0, which the instruction takes for (0, -1))
-    uint32_t minus_lo = 0x0000bf80u, minus_hi = 0xbf800000u;
-    asm("" : "+s"(minus_lo), "+s"(minus_hi));
-    const mta_bf16x2 lo = __builtin_bit_cast(mta_bf16x2, minus_lo), hi = __builtin_bit_cast(mta_bf16x2, minus_hi);
-#pragma unroll
-    for (int s = 0; s < N; ++s) {
-        part[s] = pack2<bf16_t>(a, b);
-        if (s == N - 1) break;
-        const mta_bf16x2 h = __builtin_bit_cast(mta_bf16x2, part[s]);
-        a = __builtin_amdgcn_fdot2_f32_bf16(h, lo, a, false);
-        b = __builtin_amdgcn_fdot2_f32_bf16(h, hi, b, false);
-    }
-}
 
 // strips that touch the lower triangle (all of them unless `tri`), column of strips by column of strips
 __host__ __device__ __forceinline__ int p_first(int tn, int tri) { return tri ? tn * P_TN / P_TM : 0; }

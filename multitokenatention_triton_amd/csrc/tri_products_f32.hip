@@ -591,10 +591,9 @@ int check(const void *a, const void *b, const void *c, int64_t B, int64_t H, int
     return MTA_OK;
 }
 
-// Whether the scores run on tiles of 128 x 128 in LDS slabs: from half a workgroup per CU on (us, direct | slabs, D64 / D128:
-// B1 H8 S512, 80 tiles, 6.7 | 9.4 / 9.5 | 13.2; B1 H16 S512, 160, 14.8 | 9.9 / 17.5 | 14.2; B1 H16 S1024, 576, 24.7 | 23.5 / 39.5 | 35.5;
-// B1 H32 S1024, 1152, 40.7 | 38.8 / 69.3 | 63.8; B1 H16 S2048, 2176, 73.2 | 62.5 / 127 | 105).
-bool scores_slabs(int64_t tiles) { return tiles >= 128; }
+// Scores on tiles of 128 x 128 in LDS slabs from half a workgroup per CU on, on the bf16 matrix cores (tri_products_split.hip) from 300 tiles on, and
+// at D = 128 instead of the slabs: us, direct | slabs | split: D64 B1 H8 S512 (80 tiles) 6.2 | 9.4 | 8.5, B1 H16 S512 (160) 14.8 | 9.4 | 9.1, B2 H16
+// S512 (320) - | 15.1 | 12.7, B1 H16 S1024 (576) 24.7 | 22.2 | 17.6; D128 (80) 8.4 | 13.2 | 11.1, (160) 17.5 | 14.7 | 11.7, (576) 39.5 | 34.4 | 26.2.
 
 // resident: workgroups that a CU holds at once
 template <typename K, typename... ARGS>
@@ -614,9 +613,9 @@ extern "C" int mta_lower_scores_f32(const void *a, const void *b, void *out, int
     const int rc = check(a, b, out, B, H, S, D);
     if (rc != MTA_OK) return rc;
     const int64_t n = (S + SL_TILE - 1) / SL_TILE;
-    if (scores_slabs(B * H * n * (n + 1) / 2))
-        return D == 64 ? launch(lower_scores_f32_slabs<64>, B * H, n * (n + 1) / 2, 256, 0, (hipStream_t)stream, a, b, out, S)
-                       : launch(lower_scores_f32_slabs<128>, B * H, n * (n + 1) / 2, 256, 0, (hipStream_t)stream, a, b, out, S);
+    const int64_t tiles = B * H * (n * (n + 1) / 2);
+    if (tiles >= (D == 64 ? 300 : 128)) return lower_scores_split_launch(a, b, out, B * H, S, D, (hipStream_t)stream);
+    if (tiles >= 128) return launch(lower_scores_f32_slabs<64>, B * H, n * (n + 1) / 2, 256, 0, (hipStream_t)stream, a, b, out, S);
     // Grids that leave most of the chip idle: tiles of a quarter, whose wavefronts are done in a quarter of the time (us, 64 x 128 | 32 x 64:
     // B1 H4 S256 D64 (24 workgroups of 64 x 128) 5.7 | 3.9, H8 (48) 5.7 | 3.9, H4 S512 (80) 6.2 | 5.2, H8 S512 (160) 6.4 | 6.8).
     const int64_t large = sc_tiles((int)((S + sc_rows<2>() - 1) / sc_rows<2>())), small = sc_tiles((int)((S + sc_rows<1>() - 1) / sc_rows<1>()));

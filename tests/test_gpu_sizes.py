@@ -1004,3 +1004,39 @@ def test_conv_11x15_split_values(pkg, bwd):
     torch.testing.assert_close(run(y, 0.01 * k).double(), want, rtol=2.0 ** -22, atol=0.0)
     for sx, sk in ((2.0 ** -115, 1.0), (1.0, 2.0 ** -115), (2.0 ** -60, 2.0 ** -60)):
         torch.testing.assert_close(run(x * sx, k * sk) * (1 / (sx * sk)), plain, rtol=2.0 ** -20, atol=2.0 ** -20)
+
+
+@pytest.mark.parametrize("heads,s,d", [(300, 4, 64), (300, 132, 64), (37, 388, 64), (9, 1000, 64), (16, 1024, 64), (130, 60, 128), (130, 64, 128), (23, 388, 128),
+                                       (5, 1036, 128)])
+def test_fp32_scores_split(pkg, heads, s, d):
+    """fp32 scores of the larger grids, on the parts of the operands: edges of the 128-row blocks and of the steps of 64 (32) keys, runs of two
+    and more.  Bound: d products and sums of 32 bits in any order.  Nothing written above the diagonal beyond its vectors; an infinite
+    operand gives what fp32 products give, and operands so small that their parts underflow keep their bits."""
+    lib, st = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(63)
+    a, b = (torch.randn(1, heads, s, d, generator=g, device="cuda") for _ in range(2))
+    row = torch.arange(s, device="cuda")
+    beyond = row[None, :] > (row[:, None] | 3)
+
+    def run(a, b):
+        out = torch.full((1, heads, s, s), 7.0, device="cuda")
+        assert lib.mta_lower_scores_f32(a.data_ptr(), b.data_ptr(), out.data_ptr(), 1, heads, s, d, st) == 0
+        assert (out[..., beyond] == 7.0).all() and (out[..., (row[None, :] > row[:, None]) & ~beyond] == 0.0).all()
+        return out.tril()
+
+    want = (a.double() @ b.double().transpose(2, 3)).tril()
+    size = (a.double().abs() @ b.double().abs().transpose(2, 3)).tril()
+    plain = run(a, b)
+    assert ((plain.double() - want).abs() <= d * 2.0 ** -24 * size).all()
+    for value in (float("inf"), float("nan"), 3.4e38):
+        x, y = a.clone(), 0.01 * b
+        x[0, 1, s - 2, 5] = value
+        got, clean = run(x, y), run(a, y)
+        hit = x[0, 1, s - 2] @ y[0, 1].T
+        assert torch.equal(torch.isnan(got[0, 1, s - 2, :s - 1]), torch.isnan(hit[:s - 1]))
+        torch.testing.assert_close(got[0, 1, s - 2, :s - 1], hit[:s - 1], rtol=2.0 ** -20, atol=0.0, equal_nan=True)
+        got[0, 1, s - 2] = clean[0, 1, s - 2]
+        assert torch.equal(got[0, 2:], clean[0, 2:])
+        torch.testing.assert_close(got, clean, rtol=1e-4, atol=1e-5)
+    for sx, sy in ((2.0 ** -115, 1.0), (1.0, 2.0 ** -115)):
+        assert ((run(a * sx, b * sy).double() / (sx * sy) - want).abs() <= d * 2.0 ** -24 * size).all()
