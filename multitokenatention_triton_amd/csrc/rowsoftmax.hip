@@ -486,17 +486,17 @@ template <bool IS_MAX, int G, int NW> __device__ __forceinline__ void heads_redu
 // entry l, NW neighbouring lanes fold with DPP steps, and one lane per head is read out as a wavefront-uniform value.
 template <bool IS_MAX, int G, int NW> __device__ __forceinline__ void heads_combine(const float *src, int nlw, int lane, float (&out)[G], int flw = 0)
 {
-    static_assert(NW * G <= 64 && (NW == 4 || NW == 8), "one entry per lane");
+    static_assert(NW * G <= 64 && (NW == 1 || NW == 2 || NW == 4 || NW == 8), "one entry per lane");
     const float neutral = IS_MAX ? -INFINITY : 0.0f;
     const float got = src[lane & (NW * G - 1)];
     float v = ((lane & (NW - 1)) < nlw && (lane & (NW - 1)) >= flw) ? got : neutral, r;
     if constexpr (IS_MAX) {
-        MTA_RS_DPP_STEP("v_max_f32", "quad_perm:[1,0,3,2]")
-        MTA_RS_DPP_STEP("v_max_f32", "quad_perm:[2,3,0,1]")
+        if constexpr (NW >= 2) { MTA_RS_DPP_STEP("v_max_f32", "quad_perm:[1,0,3,2]") }
+        if constexpr (NW >= 4) { MTA_RS_DPP_STEP("v_max_f32", "quad_perm:[2,3,0,1]") }
         if constexpr (NW == 8) { MTA_RS_DPP_STEP("v_max_f32", "row_half_mirror") }
     } else {
-        MTA_RS_DPP_STEP("v_add_f32", "quad_perm:[1,0,3,2]")
-        MTA_RS_DPP_STEP("v_add_f32", "quad_perm:[2,3,0,1]")
+        if constexpr (NW >= 2) { MTA_RS_DPP_STEP("v_add_f32", "quad_perm:[1,0,3,2]") }
+        if constexpr (NW >= 4) { MTA_RS_DPP_STEP("v_add_f32", "quad_perm:[2,3,0,1]") }
         if constexpr (NW == 8) { MTA_RS_DPP_STEP("v_add_f32", "row_half_mirror") }
     }
 #pragma unroll
@@ -962,8 +962,13 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         }
         const bool packed_ok = vec_ok && !no_packed && w_dtype == io_code && (w1 || w2) && (!w1 || aligned_to(w1, 4)) &&
                                (!w2 || aligned_to(w2, 4)) && C % 2 == 0 && Q <= 256 * VEC * 4;
-        // key bias without a band mask: the packed kernel's KBIAS instances, one per group size (the one for the longest
-        // rows; with 4 heads and one weight the 512-thread shape)
+        // No more wavefronts per row than its 512 keys each ask for: what bounds short rows is the start of workgroups and
+        // wavefronts, and those beyond the row are started too.  us, always 256 threads (key bias: 256 or 512) -> 64 up to 512
+        // keys, 128 up to 1024, 256 up to 2048, groups of 4 / 2 / 8 heads, second weight only: B4 H16 S512 16.5 / 21.7 / 16.9 -> 11.9 /
+        // 12.6 / 12.9, with a key bias 23.4 / 25.0 / 17.4 -> 12.3 / 12.8 / 13.2, a band 17.8 / 24.0 / 16.8 -> 12.1 / 12.9 / 13.1; B4 H16 S1024 36.4 / 44.4 /
+        // 39.3 -> 30.0 / 32.8 / 32.0, key bias 50.1 / 53.8 / 41.0 -> 31.6 / 34.7 / 33.5; key bias B2 H16 S1536 41.8 / 45.1 / 36.6 -> 33.2 / 38.6 / 36.6.
+        // The partial results of the wavefronts that are left out were neutral: the bits stay.
+        // key bias without a band mask: the packed kernel's KBIAS instances
         if (packed_ok && kb && !row_lo && aligned_to(kb, 16)) {
 #define MTA_RSK_LAUNCH(g, v, h1, h2, nt, occ)                                                                          \
     {                                                                                                                  \
@@ -978,9 +983,11 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         if (w1) MTA_RSK_LAUNCH(g, v, true, false, nt, occ)                                                             \
         MTA_RSK_LAUNCH(g, v, false, true, nt, occ)                                                                     \
     }
-            MTA_RSK_CASE(2, 4, 256, RS_OCC)
+            MTA_RSK_CASE(2, 1, 64, 1) MTA_RSK_CASE(2, 1, 128, 1) MTA_RSK_CASE(2, 1, 256, 1) MTA_RSK_CASE(2, 4, 256, RS_OCC)
+            MTA_RSK_CASE(4, 1, 64, 1) MTA_RSK_CASE(4, 1, 128, 1) MTA_RSK_CASE(4, 1, 256, 1)
             if (!(w1 && w2)) MTA_RSK_CASE(4, 1, 512, 8)
-            MTA_RSK_CASE(4, 2, 256, RS_OCC) MTA_RSK_CASE(8, 1, 256, 4)  // (8 heads: a register budget without spills)
+            MTA_RSK_CASE(4, 2, 256, RS_OCC)
+            MTA_RSK_CASE(8, 1, 64, 1) MTA_RSK_CASE(8, 1, 128, 1) MTA_RSK_CASE(8, 1, 256, 4)  // (8 heads: a register budget without spills)
 #undef MTA_RSK_CASE
 #undef MTA_RSK_LAUNCH
         }
@@ -999,6 +1006,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         if (w1) MTA_RSB_LAUNCH(g, true, false, nt, occ)                                                                \
         MTA_RSB_LAUNCH(g, false, true, nt, occ)                                                                        \
     }
+            MTA_RSB_CASE(2, 64, 1) MTA_RSB_CASE(2, 128, 1) MTA_RSB_CASE(4, 64, 1) MTA_RSB_CASE(4, 128, 1) MTA_RSB_CASE(8, 64, 1) MTA_RSB_CASE(8, 128, 1)
             MTA_RSB_CASE(2, 256, 1) MTA_RSB_CASE(4, 256, 1) MTA_RSB_CASE(4, 512, 8) MTA_RSB_CASE(8, 256, RS_OCC)
 #undef MTA_RSB_CASE
 #undef MTA_RSB_LAUNCH
@@ -1017,6 +1025,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         if (w1) MTA_RSP_LAUNCH(g, v, true, false, nt, occ)                                                             \
         MTA_RSP_LAUNCH(g, v, false, true, nt, occ)                                                                     \
     }
+            MTA_RSP_CASE(2, 1, 64, 1) MTA_RSP_CASE(2, 1, 128, 1) MTA_RSP_CASE(4, 1, 64, 1) MTA_RSP_CASE(4, 1, 128, 1) MTA_RSP_CASE(8, 1, 64, 1) MTA_RSP_CASE(8, 1, 128, 1)
             MTA_RSP_CASE(2, 1, 256, 1) MTA_RSP_CASE(2, 2, 256, 1) MTA_RSP_CASE(2, 4, 256, RS_OCC) MTA_RSP_CASE(4, 1, 256, 1)
             // 4 heads x up to 4096 keys: with one weight, 8 wavefronts of one pass each (63 registers: 8 wavefronts per
             // SIMD; measured 2 % faster than 4 wavefronts of two passes); with both weights the latter is 4 % faster
@@ -1046,7 +1055,13 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
     }
     if (vec_ok) {
 #define MTA_RS_CASE(g, v)                                                                   \
-    if (G == g && nv <= v) return launch_fixed<T, g, v>(x, w1, w2, kb, row_lo, y, N, C, P, Q, causal, w_dtype, fill_upper, st);
+    if (G == g && nv <= v) {                                                                \
+        if constexpr (v == 1 && sizeof(T) == 4) {                                           \
+            if (Q <= 64 * VEC) return launch_fixed<T, g, 1, 64>(x, w1, w2, kb, row_lo, y, N, C, P, Q, causal, w_dtype, fill_upper, st);   \
+            if (Q <= 128 * VEC) return launch_fixed<T, g, 1, 128>(x, w1, w2, kb, row_lo, y, N, C, P, Q, causal, w_dtype, fill_upper, st); \
+        }                                                                                   \
+        return launch_fixed<T, g, v>(x, w1, w2, kb, row_lo, y, N, C, P, Q, causal, w_dtype, fill_upper, st); \
+    }
         MTA_RS_CASE(1, 1) MTA_RS_CASE(1, 2) MTA_RS_CASE(1, 4) MTA_RS_CASE(1, 8)
         MTA_RS_CASE(2, 1) MTA_RS_CASE(2, 2) MTA_RS_CASE(2, 4)
         MTA_RS_CASE(4, 1) MTA_RS_CASE(4, 2) MTA_RS_CASE(4, 4)

@@ -1040,3 +1040,33 @@ def test_fp32_scores_split(pkg, heads, s, d):
         torch.testing.assert_close(got, clean, rtol=1e-4, atol=1e-5)
     for sx, sy in ((2.0 ** -115, 1.0), (1.0, 2.0 ** -115)):
         assert ((run(a * sx, b * sy).double() / (sx * sy) - want).abs() <= d * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+def test_softmax_wavefronts_per_row(pkg, group, dtype):
+    """Mix + softmax + mix of short rows on one, two and four wavefronts per row: row p of a causal plane knows only its first p + 1 keys, so
+    the planes cut out of a wider one, which takes more wavefronts, get the same bits - without a mask, under a key bias and
+    under a band, with one weight and with both.  The wide plane against torch (two roundings of the data type)."""
+    g = torch.Generator(device="cuda").manual_seed(64)
+    n, h, wide = 2, 16, 1600
+    x = torch.randn(n, h, wide, wide, generator=g, device="cuda").to(dtype)
+    block = torch.arange(h, device="cuda") // group
+    w1, w2 = ((torch.eye(h, device="cuda") + 0.1 * torch.randn(h, h, generator=g, device="cuda")) * (block[:, None] == block[None]) for _ in range(2))
+    w1, w2 = w1.to(dtype), w2.to(dtype)
+    bias = torch.zeros(n, wide, device="cuda")
+    bias[0, 100:180] = bias[1, 7:300] = float("-inf")
+    lo = (torch.arange(wide, device="cuda") - 150).clamp(min=0).to(torch.int32).expand(n, wide).contiguous()
+    for a, b in ((None, None),) if group == 1 else ((None, w2), (w1, None), (w1, w2)):
+        for kb, band in ((None, None), (bias, None), (None, lo)):
+            run = lambda s: pkg.ops.headmix_softmax(x[..., :s, :s].contiguous(), a, b, True, group_size=group, fill_upper=False,   # noqa: E731
+                                                    key_bias=None if kb is None else kb[:, :s].contiguous(),
+                                                    first_visible=None if band is None else band[:, :s].contiguous()).tril()
+            whole = run(wide)
+            for s in (8, 248, 256, 264, 504, 512, 520, 1016, 1024, 1032):
+                assert torch.equal(whole[..., :s, :s], run(s)), (s, a is None, b is None, kb is None, band is None)
+    s = x.float() if group == 1 else torch.matmul(w1.float(), x.float().flatten(2)).view_as(x).to(dtype).float()
+    want = torch.softmax(s.masked_fill(torch.ones(wide, wide, dtype=torch.bool, device="cuda").triu(1), float("-inf")), -1)
+    got = pkg.ops.headmix_softmax(x, None if group == 1 else w1, None, True, group_size=group, fill_upper=False).tril()
+    ulp = {torch.float32: 2.0 ** -18, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    torch.testing.assert_close(got.float(), want, rtol=ulp * (1.0 if group == 1 else 8.0), atol=1e-6)
