@@ -236,8 +236,8 @@ template <typename T, int D, int R, int SK, bool SCORES_ONLY, int NW, bool BAND>
 __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7)) ? 2 : QK_OCC) : 2) void conv_attn_fwd_mfma(const T *__restrict__ Q, const T *__restrict__ K,
                                                              const T *__restrict__ V, const T *__restrict__ Wt,
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
-                                                             float scale, int H, int nqb, int fill_upper, int64_t total_wg,
-                                                             int64_t per_xcd, int jc_len, int items_per_bh, int hpx,
+                                                             float scale, int H, int nqb, int fill_upper, unsigned total_wg,
+                                                             unsigned per_xcd, int jc_len, unsigned items_per_bh, int hpx,
                                                              item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
@@ -276,18 +276,23 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     // When the (batch, head) pairs divide evenly over the XCDs (hpx > 0 of them each), the items of an XCD's heads are
     // taken rank by rank - the longest item of each head, then the second longest of each, ... - so that the long items
     // all start early and the short ones fill the end of the grid (workgroups start in index order as slots free up).
-    int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (lid >= total_wg) return;
-    if (hpx > 0) {
-        const int64_t pos = blockIdx.x >> 3;
-        lid = ((int64_t)(blockIdx.x & 7) * hpx + pos % hpx) * items_per_bh + pos / hpx;
-    }
     // Work item = (batch*head, query block, chunk of jc_len key blocks).  The scores-only kernel splits the key
     // range of a query block (its output columns are independent; a chunk starts one key block early to rebuild
     // the retained halo columns), so that items are short and equal and the grid runs in several even rounds;
     // the attention kernel accumulates over all keys and gets jc_len = all of them.
-    const int64_t bh = lid / items_per_bh;
-    int item = (int)(lid % items_per_bh), qb = nqb - 1, jc = 0;
+    // (32-bit divisions, one or two: 64-bit ones were half a microsecond of a workgroup's start)
+    const unsigned xcd = blockIdx.x & 7u, pos = blockIdx.x >> 3;
+    if (xcd * per_xcd + pos >= total_wg) return;
+    int bh, item;
+    if (hpx > 0) {
+        item = (int)(pos / (unsigned)hpx);
+        bh = (int)(xcd * (unsigned)hpx + (pos - (unsigned)item * (unsigned)hpx));
+    } else {
+        const unsigned lid = xcd * per_xcd + pos;
+        bh = (int)(lid / items_per_bh);
+        item = (int)(lid - (unsigned)bh * items_per_bh);
+    }
+    int qb = nqb - 1, jc = 0;
     int tbl_lo = -1, tbl_len = 0;
     if (tbl.n > 0) {
         const unsigned e = tbl.e[item];
@@ -303,18 +308,18 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         }
         jc = item;
     }
-    const int head = (int)(bh % H);
+    const int head = (int)((unsigned)bh % (unsigned)H);
     const int q0 = qb * G::BQ;
     const bool q_strided = RAW && qs.row != 0;
-    const T *Qp = Q + (q_strided ? bh / H * qs.batch + head * qs.head : bh * (int64_t)S * D);
+    const T *Qp = Q + (q_strided ? (int64_t)(bh / H) * qs.batch + head * qs.head : (int64_t)bh * S * D);
     const int64_t q_row = q_strided ? qs.row : D;
-    const T *Kp = K + bh * (int64_t)S * D;
-    const T *Vp = SCORES_ONLY ? Kp : V + bh * (int64_t)S * D;
+    const T *Kp = K + (int64_t)bh * S * D;
+    const T *Vp = SCORES_ONLY ? Kp : V + (int64_t)bh * S * D;
     // (scores only, tri_gl > 0: the scores go out in the triangular layout, groups of tri_gl heads interleaved by rows;
     // nothing above the diagonal is stored then)
     const bool tri = SCORES_ONLY && tri_gl > 0;
-    T *Op = tri ? O + (bh / (tri ? tri_gl : 1)) * ((tri ? tri_gl : 1) * tri_rowoff(S)) : O + bh * (int64_t)S * (SCORES_ONLY ? S : D);
-    const int tri_i = tri ? (int)(bh % tri_gl) : 0;
+    T *Op = tri ? O + ((unsigned)bh / (unsigned)(tri ? tri_gl : 1)) * ((tri ? tri_gl : 1) * tri_rowoff(S)) : O + (int64_t)bh * S * (SCORES_ONLY ? S : D);
+    const int tri_i = tri ? (int)((unsigned)bh % (unsigned)tri_gl) : 0;
 
     // asynchronous copy of key block j into buffer `buf`: K rows cb.., V rows j*BK..; out-of-range keys
     // re-read a valid row (their scores are zeroed / their probabilities are 0 later)
@@ -389,6 +394,30 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     }
     // one key block earlier only fills the retained score columns (before the first one: the right pad, if any)
     const int j_start = RAW ? j_lo : j_lo > 0 ? j_lo - 1 : (G::PWR > 0 ? -1 : 0);
+    // What the start waits for is asked for at once, this wavefront's rows of Q and the kernel's taps ahead of the first blocks of K and V:
+    // behind them, the taps waited for the blocks and Q was asked for when those had come.  With the 32-bit divisions above, scores
+    // kernel, us: bf16 6x11 B2 H16 S1008 D64 22.3 -> 21.1, B4 H16 S1024 D128 40.6 -> 40.1, 7x7 B1 H16 S1024 D64 18.6 -> 17.7, B1 H16 S2048 D128 42.1 ->
+    // 40.9, 6x11 B2 H16 S2048 D128 69.7 -> 67.5, S4096 240 -> 236, 11x15 B2 H16 S640 D128 21.1 -> 19.8.
+    int trow[2], prow[2];   // this lane's two query rows
+    frag8<T> qf[2][KS];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+        trow[rb] = wave * 32 + rb * 16 + ln;
+        prow[rb] = q0 - G::HR + trow[rb];
+        const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= S ? S - 1 : prow[rb]);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qf[rb][ks] = *reinterpret_cast<const frag8<T> *>(Qp + pc * q_row + ks * 32 + kg * 8);
+    }
+    constexpr int WZ_IT = (R * G::WZ_LD + F_NT - 1) / F_NT;
+    T taps[RAW ? 1 : WZ_IT];
+    if constexpr (!RAW) {
+#pragma unroll
+        for (int n = 0; n < WZ_IT; ++n) {
+            const int e = n * F_NT + tid, i = e / G::WZ_LD, jj = e % G::WZ_LD - G::WZ_OFF;
+            taps[n] = Wt[head * R * SK + (i < R && jj >= 0 && jj < SK ? i * SK + jj : 0)];
+        }
+    }
+    asm volatile("" : : : "memory");
     issue_k(j_start, SCORES_ONLY ? B0 : KV);
     if (!SCORES_ONLY) issue_v(j_start, KV + TILE);
 
@@ -400,28 +429,17 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         for (int u = 0; u < 8; ++u) z.v[u] = from_float<T>(0.0f);
         *reinterpret_cast<pack16<T> *>(Sc + e * 8) = z;
     }
-    for (int e = tid; e < R * G::WZ_LD; e += F_NT) {
-        const int i = e / G::WZ_LD, jj = e % G::WZ_LD - G::WZ_OFF;
-        const bool ok = jj >= 0 && jj < SK;
-        const T wv = Wt[head * R * SK + (ok ? i * SK + jj : 0)];
-        wz[e] = ok ? signed_tap<T>(wv, SCORES_ONLY ? 1.0f : scale) : from_float<T>(0.0f);
+#pragma unroll
+    for (int n = 0; n < WZ_IT; ++n) {
+        const int e = n * F_NT + tid, jj = e % G::WZ_LD - G::WZ_OFF;
+        if (e < R * G::WZ_LD) wz[e] = jj >= 0 && jj < SK ? signed_tap<T>(taps[n], SCORES_ONLY ? 1.0f : scale) : from_float<T>(0.0f);
     }
     }
-
-    // this lane's two query rows
-    int trow[2], prow[2];
-    frag8<T> qf[2][KS];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-        trow[rb] = wave * 32 + rb * 16 + ln;
-        prow[rb] = q0 - G::HR + trow[rb];
+    for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= S ? S - 1 : prow[rb]);
-            qf[rb][ks] = *reinterpret_cast<const frag8<T> *>(Qp + pc * q_row + ks * 32 + kg * 8);
+        for (int ks = 0; ks < KS; ++ks)
             if (prow[rb] < 0 || prow[rb] >= S) qf[rb][ks] = zero_frag<T>();  // rows outside the sequence are conv padding
-        }
-    }
     // band mask: first visible key of this lane's two rows, and the largest of them over the wavefront's 32 rows (a key
     // block that starts at or beyond it is visible to all of them)
     int flo[2] = {0, 0}, fmax_w = 0;
@@ -912,7 +930,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     if (per_xcd * 8 > 0x7fffffffLL || items_per_bh > 0x7fffffffLL) return MTA_ERR_SHAPE;
     dim3 grid((unsigned)(per_xcd * 8));
     hipLaunchKernelGGL(kern, grid, dim3(F_NT), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
-                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, total_wg, per_xcd, jc_len, (int)items_per_bh,
+                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)per_xcd, jc_len, (unsigned)items_per_bh,
                        (B * H) % 8 == 0 ? (int)(B * H / 8) : 0, tbl, band_lo, tri_gl, qs);
     return launch_status();
 }
