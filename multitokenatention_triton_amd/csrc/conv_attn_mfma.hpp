@@ -237,7 +237,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                                                              const T *__restrict__ V, const T *__restrict__ Wt,
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
                                                              float scale, int H, int nqb, int fill_upper, unsigned total_wg,
-                                                             unsigned per_xcd, int jc_len, unsigned items_per_bh, int hpx,
+                                                             unsigned heads, int jc_len,
                                                              item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
@@ -270,28 +270,21 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     const int tid = threadIdx.x;
     // (the wavefront index through readfirstlane: everything derived from it is then scalar, branches included)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
-    // XCD-aware order: workgroup ids are dealt round-robin to the 8 XCDs, so XCD x takes the x-th eighth of the
-    // (batch*head, query block) list: the workgroups sharing one head's K and V run on one L2.  Within a head
-    // the longest (last) query blocks come first.
-    // When the (batch, head) pairs divide evenly over the XCDs (hpx > 0 of them each), the items of an XCD's heads are
-    // taken rank by rank - the longest item of each head, then the second longest of each, ... - so that the long items
+    // The items are taken rank by rank - the longest item of every head, then the second longest of each, ... - so that the long items
     // all start early and the short ones fill the end of the grid (workgroups start in index order as slots free up).
+    // Workgroup ids are dealt round-robin to the 8 XCDs: with heads in multiples of 8 an XCD keeps its own, whose K and V stay in its L2
+    // (of 12 heads an XCD sees 3, of 4 one).  With other numbers of heads an XCD used to take an eighth of the list head by head - of 4
+    // heads one XCD a head's long items and another its short ones.  us, that -> this, bf16 6x11, scores | attention: B1 H4 S3008 D128
+    // 26.5 -> 24.1 | 117 -> 117, B1 H12 S2048 D64 33.7 -> 27.7 | 66.7 -> 67.2, S3712 D64 76.3 -> 67.5 | 152 -> 122, S4096 D128 101 -> 93 | 210 -> 170,
+    // B1 H20 S2048 D128 53.2 -> 45.8 | 106 -> 88.6; without a conv B1 H12 S2048 D64 16.9 -> 14.4, S2560 23.8 -> 20.1, but S3344 33.9 -> 36.2.
     // Work item = (batch*head, query block, chunk of jc_len key blocks).  The scores-only kernel splits the key
     // range of a query block (its output columns are independent; a chunk starts one key block early to rebuild
     // the retained halo columns), so that items are short and equal and the grid runs in several even rounds;
     // the attention kernel accumulates over all keys and gets jc_len = all of them.
-    // (32-bit divisions, one or two: 64-bit ones were half a microsecond of a workgroup's start)
-    const unsigned xcd = blockIdx.x & 7u, pos = blockIdx.x >> 3;
-    if (xcd * per_xcd + pos >= total_wg) return;
-    int bh, item;
-    if (hpx > 0) {
-        item = (int)(pos / (unsigned)hpx);
-        bh = (int)(xcd * (unsigned)hpx + (pos - (unsigned)item * (unsigned)hpx));
-    } else {
-        const unsigned lid = xcd * per_xcd + pos;
-        bh = (int)(lid / items_per_bh);
-        item = (int)(lid - (unsigned)bh * items_per_bh);
-    }
+    // (a 32-bit division: the 64-bit ones that this took were half a microsecond of a workgroup's start)
+    if (blockIdx.x >= total_wg) return;
+    int item = (int)(blockIdx.x / heads);
+    const int bh = (int)(blockIdx.x - (unsigned)item * heads);
     int qb = nqb - 1, jc = 0;
     int tbl_lo = -1, tbl_len = 0;
     if (tbl.n > 0) {
@@ -926,12 +919,11 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
             items_per_bh = n;
         }
     }
-    const int64_t total_wg = B * H * items_per_bh, per_xcd = (total_wg + 7) / 8;
-    if (per_xcd * 8 > 0x7fffffffLL || items_per_bh > 0x7fffffffLL) return MTA_ERR_SHAPE;
-    dim3 grid((unsigned)(per_xcd * 8));
+    const int64_t total_wg = B * H * items_per_bh;
+    if (total_wg > 0x7fffffffLL) return MTA_ERR_SHAPE;
+    dim3 grid((unsigned)total_wg);
     hipLaunchKernelGGL(kern, grid, dim3(F_NT), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
-                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)per_xcd, jc_len, (unsigned)items_per_bh,
-                       (B * H) % 8 == 0 ? (int)(B * H / 8) : 0, tbl, band_lo, tri_gl, qs);
+                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)(B * H), jc_len, tbl, band_lo, tri_gl, qs);
     return launch_status();
 }
 
