@@ -132,12 +132,12 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f)
 // The scores-only kernel writes the scores of 16-key blocks cb-1 and cb (cb odd, both row blocks: two writes) right
 // after step (cb+1)*KS + LAG - 1 of its score phase; the last pair after the loop.  Number of those writes issued at the
 // end of a step in [lo, hi).
-constexpr int score_writes_between(int lo, int hi, int KS, int NCB, int LAG)
+constexpr int score_writes_between(int lo, int hi, int KS, int NCB, int LAG, int RB)
 {
     int c = 0;
     for (int cb = 1; cb + 1 < NCB; cb += 2) {
         const int s = (cb + 1) * KS + LAG - 1;
-        if (s >= lo && s < hi) c += 2;
+        if (s >= lo && s < hi) c += RB;
     }
     return c;
 }
@@ -201,8 +201,8 @@ template <int D> __device__ __forceinline__ int v_swizzle4(int key)
     else return 2 * ((key >> 1) & 3);
 }
 
-template <int R, int SK, int NW> struct fused_geom {
-    static constexpr int F_SR = 32 * NW;
+template <int R, int SK> struct fused_geom {
+    static constexpr int F_SR = 128;
     static constexpr int HR = (R - 1 + 7) & ~7;    // halo rows above the block (recomputed)
     static constexpr int HC = (SK - 1 + 7) & ~7;   // score columns kept from the previous key block
     static constexpr int BQ = F_SR - HR;           // output rows per workgroup
@@ -241,9 +241,10 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                                                              item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
-    using G = fused_geom<R, SK, NW>;
+    using G = fused_geom<R, SK>;
     constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
-    constexpr int F_NT = 64 * NW, F_SR = 32 * NW;
+    constexpr int F_NT = 64 * NW, F_SR = 128, RB = F_SR / (16 * NW);   // (RB: blocks of 16 rows per wavefront)
+    static_assert(RB == 2 || (RB == 1 && !SCORES_ONLY), "the scores-only kernel is written for two");
     constexpr int CPR = D / 8;                     // 16-byte chunks per K/V row
     constexpr int TILE = F_BK * D;                 // elements per K or V block
     constexpr int ROUNDS = TILE / 8 / F_NT;        // copy instructions per block per lane
@@ -391,11 +392,11 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     // behind them, the taps waited for the blocks and Q was asked for when those had come.  With the 32-bit divisions above, scores
     // kernel, us: bf16 6x11 B2 H16 S1008 D64 22.3 -> 21.1, B4 H16 S1024 D128 40.6 -> 40.1, 7x7 B1 H16 S1024 D64 18.6 -> 17.7, B1 H16 S2048 D128 42.1 ->
     // 40.9, 6x11 B2 H16 S2048 D128 69.7 -> 67.5, S4096 240 -> 236, 11x15 B2 H16 S640 D128 21.1 -> 19.8.
-    int trow[2], prow[2];   // this lane's two query rows
-    frag8<T> qf[2][KS];
+    int trow[RB], prow[RB];   // this lane's query rows
+    frag8<T> qf[RB][KS];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-        trow[rb] = wave * 32 + rb * 16 + ln;
+    for (int rb = 0; rb < RB; ++rb) {
+        trow[rb] = wave * (16 * RB) + rb * 16 + ln;
         prow[rb] = q0 - G::HR + trow[rb];
         const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= S ? S - 1 : prow[rb]);
 #pragma unroll
@@ -429,17 +430,17 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     }
     }
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             if (prow[rb] < 0 || prow[rb] >= S) qf[rb][ks] = zero_frag<T>();  // rows outside the sequence are conv padding
     // band mask: first visible key of this lane's two rows, and the largest of them over the wavefront's 32 rows (a key
     // block that starts at or beyond it is visible to all of them)
-    int flo[2] = {0, 0}, fmax_w = 0;
+    int flo[2] = {0, 0}, fmax_w = 0;   // (scores only: two row blocks)
     if constexpr (BAND) {
         const int64_t brow = (bh / H) * (int64_t)S;
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) flo[rb] = (prow[rb] >= 0 && prow[rb] < S) ? band_lo[brow + prow[rb]] : 0;
+        for (int rb = 0; rb < RB; ++rb) flo[rb] = (prow[rb] >= 0 && prow[rb] < S) ? band_lo[brow + prow[rb]] : 0;
         int m = flo[0] > flo[1] ? flo[0] : flo[1];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
@@ -459,12 +460,17 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         for (int t = 0; t < 8; ++t) tz[i].v[t] = src[t];
     }
 
-    f32x4 oacc[2][DB];
+    f32x4 oacc[RB][DB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int db = 0; db < DB; ++db) oacc[rb][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_i[2] = {-INFINITY, -INFINITY}, l_i[2] = {0.0f, 0.0f};   // (maxima of the conv's results, ahead of the factor)
+    float m_i[RB], l_i[RB];   // (maxima of the conv's results, ahead of the factor)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        m_i[rb] = -INFINITY;
+        l_i[rb] = 0.0f;
+    }
     const float scale_abs = scale == 0.0f ? 1.0f : fabsf(scale), scale2 = scale_abs * 1.4426950408889634f;
 
     // retained columns: each thread moves one 16-byte vector per round (HC/8 vectors per row)
@@ -478,21 +484,21 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         const int idx = it * F_NT + tid;
         tail_off[it] = idx < TAIL_VECS ? (idx / VPRW) * F_SLD + (idx % VPRW) * 8 : -1;
     }
-    // the two 16-row blocks of this wavefront span rows pmin..pmin+31 of the sequence
-    const int pmin = q0 - G::HR + wave * 32;
+    // the 16-row blocks of this wavefront span rows pmin .. pmin + 16 RB - 1 of the sequence
+    const int pmin = q0 - G::HR + wave * (16 * RB);
     // Rows of the conv (and of everything after it: softmax, P V, the stores).  The first wavefront's rows are taken
     // R-1 further down than the rows it computes scores for: its conv windows then start at tile row 0 instead of
     // above the tile, every fragment address is the same affine function of (row block, kernel row), and what it
     // leaves out are halo rows nobody stores.  Its last R-1 rows belong to the second wavefront too and are not
     // stored from here.
     const int cshift = wave == 0 ? R - 1 : 0;
-    int cprow[2];
-    bool row_stored[2];
+    int cprow[RB];
+    bool row_stored[RB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RB; ++rb) {
         const int tr_ = trow[rb] + cshift;
         cprow[rb] = prow[rb] + cshift;
-        row_stored[rb] = tr_ >= G::HR && tr_ < wave * 32 + 32 && cprow[rb] < S;
+        row_stored[rb] = tr_ >= G::HR && tr_ < (wave + 1) * (16 * RB) && cprow[rb] < S;
     }
 
     auto plain = [&](int j) {
@@ -532,8 +538,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 ka[ks] = lds_addr(Kb) + (unsigned)((ln * D + (((ks * 4 + kg) ^ (ln & (CPR - 1))) * 8)) * (int)sizeof(T));
             const unsigned wa = lds_addr(Sc) + (unsigned)((trow[0] * F_SLD + G::HC + (kg & 1) * 16 + (kg >> 1) * 8) * (int)sizeof(T));
             u32x4_t kring[KSLOT];
-            f32x4 sacc[2][2];
-            uint32_t held[2][2];
+            f32x4 sacc[2][RB];
+            uint32_t held[RB][2];
             auto kissue = [&](auto ic) __attribute__((always_inline)) {
                 constexpr int n = decltype(ic)::value;
                 kring[n % KSLOT] = lds_read16_at(ka[n % KS], (n / KS) * 16 * D * (int)sizeof(T));
@@ -544,7 +550,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 const bool s_plain = PLAIN || !SCORES_ONLY ? PLAIN || whole : (cbase + cb * 16 >= 0 && cbase + cb * 16 + 16 <= S && (!causal || cbase + cb * 16 + 15 <= pmin) &&
                                                (!BAND || cbase + cb * 16 >= fmax_w));
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb) {
+                for (int rb = 0; rb < RB; ++rb) {
                     const f32x4 a = sacc[cb & 1][rb];
                     uint32_t lo = pack2<T>(a[0], a[1]), hi = pack2<T>(a[2], a[3]);
                     if (SCORES_ONLY) {  // MTA scales the scores before the conv, in the I/O dtype: round, scale, round again
@@ -590,14 +596,14 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 constexpr int cb = n / KS, ks = n % KS;
                 if constexpr (n + KLD < NSTEP) kissue(std::integral_constant<int, n + KLD>{});
                 // LDS operations younger than read n: the reads issued after it and the score writes issued since
-                constexpr int younger = (n + KLD < NSTEP ? n + KLD : NSTEP - 1) - n + (RAW ? 0 : score_writes_between(n > KLD ? n - KLD : 0, n, KS, NCB, LAG));
+                constexpr int younger = (n + KLD < NSTEP ? n + KLD : NSTEP - 1) - n + (RAW ? 0 : score_writes_between(n > KLD ? n - KLD : 0, n, KS, NCB, LAG, RB));
                 lds_wait_upto<(younger < 15 ? younger : 15)>(kring[n % KSLOT]);
                 if constexpr (ks == 0) {
-                    sacc[cb & 1][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    sacc[cb & 1][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) sacc[cb & 1][rb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
-                mma16(sacc[cb & 1][0], __builtin_bit_cast(frag8<T>, kring[n % KSLOT]), qf[0][ks]);
-                mma16(sacc[cb & 1][1], __builtin_bit_cast(frag8<T>, kring[n % KSLOT]), qf[1][ks]);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) mma16(sacc[cb & 1][rb], __builtin_bit_cast(frag8<T>, kring[n % KSLOT]), qf[rb][ks]);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (cb >= 1 && ks == LAG - 1) {
                     epilogue(std::integral_constant<int, cb - 1>{});
@@ -626,7 +632,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         // 7x9 D64 B4 H12 93.6 | 93.5, 11x15 D128 B1 H32 S4096 362 | 359).  A block's results are taken up LAG products into the next turn,
         // when they are long complete.
         constexpr int TURNS = SCORES_ONLY ? 2 : 1;
-        constexpr int NB = 2 * NCB, NREAD = NB * R;
+        constexpr int NB = RB * NCB, NREAD = NB * R;
         // score fragments in flight (scores only: 8 and 12 measure the same, 15 spills; attention: 4 and 8 the same, and 8 with 7 kernel
         // rows at D = 64 takes the third workgroup of a CU: fp16 7x9 B4 H12 S2048 92.7 | 105.4 us)
         constexpr int NLD = SCORES_ONLY ? 8 : 4;
@@ -643,8 +649,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
         };
         // what happens to output block b = rb*NCB + cb (rows crow[rb], keys j*64 + 16cb ..) once it is complete
         uint32_t held[2];           // scores only: the even block of a pair, packed
-        float sv[2][NCB][4], mloc, mneg[2];   // attention: a row block's logits, their maximum; minus the running maximum as the exponent takes it
-        frag8<T> pf[2][2];          // attention: probabilities, in the operand layout of the P V products
+        float sv[RB][NCB][4], mloc, mneg[RB];   // attention: a row block's logits, their maximum; minus the running maximum as the exponent takes it
+        frag8<T> pf[RB][2];         // attention: probabilities, in the operand layout of the P V products
         auto finish = [&](auto bc) __attribute__((always_inline)) {
             constexpr int b = decltype(bc)::value;
             constexpr int rb = b / NCB, cb = b % NCB;
@@ -741,7 +747,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                 __builtin_amdgcn_sched_barrier(0);
             }
             // the first row block's probabilities, a pair at a time among the second one's products
-            if constexpr (!SCORES_ONLY) {
+            if constexpr (!SCORES_ONLY && RB == 2) {
                 constexpr int n0 = NREAD / 2 + TURNS * LAG - 1, every = (NREAD - 1 - n0) / 8;
                 static_assert(every >= 1, "fewer products than pairs");
                 if constexpr (n > n0 && (n - n0) % every == 0 && (n - n0) / every <= 8) {
@@ -771,19 +777,19 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
             };
             static_for<VLD>(vissue);
             static_for<TURNS>([&](auto b) __attribute__((always_inline)) { finish(std::integral_constant<int, NB - TURNS + decltype(b)::value>{}); });
-            // the second row block's probabilities: those of the first 32 keys, then the rest among the products with these
-            static_for<4>([&](auto h) __attribute__((always_inline)) { probs(std::integral_constant<int, 1>{}, h); });
+            // the last row block's probabilities: those of the first 32 keys, then the rest among the products with these
+            static_for<4>([&](auto h) __attribute__((always_inline)) { probs(std::integral_constant<int, RB - 1>{}, h); });
             static_for<NV>([&](auto ic) __attribute__((always_inline)) {
                 constexpr int n = decltype(ic)::value, ks = n / DB, db = n % DB;
                 if constexpr (n + VLD < NV) vissue(std::integral_constant<int, n + VLD>{});
                 constexpr int younger = 2 * ((n + VLD < NV ? n + VLD : NV - 1) - n);
                 asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(vring[n % VSLOT].a), "+v"(vring[n % VSLOT].b) : "n"(younger) : "memory");
                 const frag8<T> vf = __builtin_bit_cast(frag8<T>, vring[n % VSLOT]);
-                mma16(oacc[0][db], vf, pf[0][ks]);
-                mma16(oacc[1][db], vf, pf[1][ks]);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) mma16(oacc[rb][db], vf, pf[rb][ks]);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (ks == 0 && db % (DB / 4) == 0) {
-                    probs(std::integral_constant<int, 1>{}, std::integral_constant<int, 4 + db / (DB / 4)>{});
+                    probs(std::integral_constant<int, RB - 1>{}, std::integral_constant<int, 4 + db / (DB / 4)>{});
                     __builtin_amdgcn_sched_barrier(0);
                 }
             });
@@ -835,10 +841,10 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     const int lane_e = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     const int ln_o = lane_e & 15, kg_o = lane_e >> 4;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RB; ++rb) {
         const float l_row = sum_across_groups(l_i[rb]);
-        const int tr_ = wave * 32 + rb * 16 + ln_o + cshift, p_ = q0 - G::HR + tr_;
-        if (tr_ >= G::HR && tr_ < wave * 32 + 32 && p_ < S) {
+        const int tr_ = wave * (16 * RB) + rb * 16 + ln_o + cshift, p_ = q0 - G::HR + tr_;
+        if (tr_ >= G::HR && tr_ < (wave + 1) * (16 * RB) && p_ < S) {
             const float inv = 1.0f / l_row;
             if (Lse != nullptr && kg_o == 0) Lse[bh * (int64_t)S + p_] = m_i[rb] * scale_abs + __logf(l_row);
 #pragma unroll
@@ -856,13 +862,20 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
                 int64_t S, int causal, float scale, int fill_upper, hipStream_t st, const int *band_lo = nullptr, int tri_gl = 0,
                 row_strides qs = {0, 0, 0})
 {
-    constexpr int NW = 4;
-    constexpr int F_NT = 64 * NW;
-    using G = fused_geom<R, SK, NW>;
+    using G = fused_geom<R, SK>;
     constexpr bool RAW = SCORES_ONLY && R == 1 && SK == 1;
     static_assert(G::fits, "conv window exceeds the 32-key MFMA contraction");
     const int nqb = (int)((S + G::BQ - 1) / G::BQ);
-    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, NW, BAND>;
+    // Attention kernel: eight wavefronts of 16 rows instead of four of 32 - the chain of steps that a workgroup is gets a fifth shorter, a CU
+    // holds two of these at D = 64 and one at 128 - up to 2 1/4 and 1 3/4 workgroups per CU.  us, four | eight: 6x11 B1 H8 S296 D128 (24
+    // workgroups) 19.0 | 15.8, B1 H16 S640 D64 (96) 26.3 | 21.6, D128 32.4 | 27.1, B1 H32 S1300 D64 (352) 49.7 | 41.0, D128 61.9 | 49.6, B1 H24 S2048
+    // D128 (432) 91.5 | 78.8, H26 (468) 91.8 | 88.1, H28 (504) 92.0 | 91.9, H32 (576) 94.4 | 103.5, D64 (504) 73.7 | 63.4, (576) 76.0 | 68.2, B2 H60 S600
+    // D64 (600) 31.9 | 31.6, B4 H32 S512 (640) 27.7 | 30.6; 3x3, 7x9 and 11x15 alike.
+    const bool few = !SCORES_ONLY && 4 * B * H * nqb <= (D == 64 ? 9 : 7) * (int64_t)device_cu_count();
+    auto kern = conv_attn_fwd_mfma<T, D, R, SK, SCORES_ONLY, 4, BAND>;
+    if constexpr (!SCORES_ONLY) {
+        if (few) kern = conv_attn_fwd_mfma<T, D, R, SK, false, 8, BAND>;
+    }
     // key blocks per work item: all of them for the attention kernel; QK_CHUNK for the scores-only kernel
     const int jc_len = SCORES_ONLY ? QK_CHUNK : (int)((S + F_BK - 1) / F_BK) + 1;
     int64_t items_per_bh = 0;
@@ -922,7 +935,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
     const int64_t total_wg = B * H * items_per_bh;
     if (total_wg > 0x7fffffffLL) return MTA_ERR_SHAPE;
     dim3 grid((unsigned)total_wg);
-    hipLaunchKernelGGL(kern, grid, dim3(F_NT), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
+    hipLaunchKernelGGL(kern, grid, dim3(few ? 512 : 256), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
                        lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)(B * H), jc_len, tbl, band_lo, tri_gl, qs);
     return launch_status();
 }

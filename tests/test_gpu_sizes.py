@@ -1070,3 +1070,20 @@ def test_softmax_wavefronts_per_row(pkg, group, dtype):
     got = pkg.ops.headmix_softmax(x, None if group == 1 else w1, None, True, group_size=group, fill_upper=False).tril()
     ulp = {torch.float32: 2.0 ** -18, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
     torch.testing.assert_close(got.float(), want, rtol=ulp * (1.0 if group == 1 else 8.0), atol=1e-6)
+
+
+@pytest.mark.parametrize("dtype,r,k", [(torch.bfloat16, 3, 3), (torch.float16, 7, 9), (torch.bfloat16, 11, 15)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_attention_of_few_workgroups(pkg, d, dtype, r, k):
+    """Attention on eight wavefronts of 16 rows (small grids) and on four of 32: the same bits for the same heads, whether they are alone or
+    among so many that the larger grid takes the other form; edges of the 112- to 120-row query blocks and of the 64-key blocks."""
+    g = torch.Generator(device="cuda").manual_seed(65)
+    for s in (1, 17, 64, 113, 121, 250):
+        q, kk, v = (torch.randn(1, 600, s, d, generator=g, device="cuda").to(dtype) for _ in range(3))
+        w = (0.1 * torch.randn(600, r, k, generator=g, device="cuda")).to(dtype)
+        for causal in (True, False):
+            run = lambda lo, hi: pkg.ops.conv_attn_fwd(q[:, lo:hi].contiguous(), kk[:, lo:hi].contiguous(), v[:, lo:hi].contiguous(), w[lo:hi], causal,   # noqa: E731
+                                                       None, return_lse=True)
+            (many, many_lse), (few, few_lse) = run(0, 600), run(590, 600)
+            assert torch.equal(many[:, 590:], few) and torch.equal(many_lse[:, 590:], few_lse), (s, causal)
+            assert torch.isfinite(many.float()).all()
