@@ -70,6 +70,8 @@ SIGNATURES = {
     "mta_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_softmax_headmix_grads": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_sum_partials": (_int, [_int, _vp, _vp]),
+    "mta_conv2d_grads": (_int, [_vp] * 6 + [_i64] * 5 + [_int, _int, _int, _f32, _int, _int, _vp]),
+    "mta_conv2d_grads_partials": (_int, [_vp] * 6 + [_i64] * 5 + [_int, _int, _int, _f32, _int, _int, _vp, _vp]),
     "mta_conv2d_bwd_weight_partials": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _f32, _int, _int, _vp, _vp]),
     "mta_headmix_grads_partials": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp, _vp]),
     "mta_softmax_headmix_grads_partials": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp, _vp]),

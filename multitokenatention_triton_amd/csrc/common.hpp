@@ -182,6 +182,10 @@ struct row_strides { int64_t batch, head, row; };
 // instance covers the arguments
 int conv_mix16_dispatch(const void *x, const void *wc, const void *wm, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R,
                         int S, int group, int causal, int fill_upper, int io_dtype, hipStream_t st);
+// conv2d_grads.hip: both gradients of the conv in one pass over dy; bpc partial kernels per channel fit into `partial`, then: were left
+// there.  MTA_ERR_UNSUPPORTED where it has no instance
+int conv2d_grads_launch(const void *x, const void *dy, const void *w, void *dx, float *partial, int *bpc, int64_t N, int64_t C, int64_t H, int64_t W,
+                        int R, int S, int causal, int io_dtype, hipStream_t st);
 // conv2d_split.hip: depthwise conv (11x15) on the bf16 matrix cores with the 32 bits of data and weights kept (forward or input gradient;
 // causal as in conv2d_causal.hip); 1 where it has no instance
 int conv2d_split_dispatch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,

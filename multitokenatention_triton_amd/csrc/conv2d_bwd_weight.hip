@@ -18,7 +18,8 @@
 // key offset j the sums over q of dy[p,q] * x[p',q+j-pad] for 16 rows p and 16 rows p' are one 16x16 product with the
 // keys as contraction index, and the taps (i,j) are the entries p'-p = i-(R-1) of it.  Every 16-row block of dy meets
 // the two 16-row blocks of x that hold its R-1 rows of halo, and all blocks add into the same 2*S accumulators, since
-// only p'-p matters.  The operand of offset j is the lane's 24-key window of x shifted by j keys in registers.
+// only p'-p matters.  The operand of offset j is the lane's 24-key window of x shifted by j keys in registers.  Calls that want the
+// input gradient as well take conv2d_grads.hip.
 #include <atomic>
 
 #include "common.hpp"
@@ -553,5 +554,34 @@ extern "C" int mta_conv2d_bwd_weight_noalloc(const void *x, const void *dy, void
     if (!ws) return rc;
     mta_partials job;
     MTA_DISPATCH_IO(io_dtype, rc = launch<io_t>(x, dy, dw, ws, bpc, N, C, H, W, R, S, causal, 1.0f, MTA_F32, &job, (hipStream_t)stream));
+    return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
+}
+
+extern "C" int mta_conv2d_grads_partials(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes,
+                                         int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype,
+                                         int w_dtype, mta_partials *job, void *stream)
+{
+    if (!job || !w || !dx) return MTA_ERR_NULL;
+    const int rc = check_args(x, dy, dw, N, C, H, W, R, S, io_dtype, w_dtype);
+    if (rc != MTA_OK) return rc;
+    if (!aligned_to(w, dtype_size(w_dtype)) || !aligned_to(dx, dtype_size(io_dtype))) return MTA_ERR_ALIGN;
+    if (!workspace) return MTA_ERR_NULL;
+    if (!aligned_to(workspace, 16)) return MTA_ERR_ALIGN;
+    int bpc = blocks_per_channel(N, C, H, W, MAX_PARTIALS);
+    if (workspace_bytes < (int64_t)bpc * C * R * S * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
+    static const bool force_valu = [] { const char *e = getenv("MTA_CONV_FORCE_VALU"); return e && e[0] == '1'; }();
+    if (force_valu || io_dtype == MTA_F32 || w_dtype != io_dtype || W % 8 != 0 || !aligned_to(x, 16) || !aligned_to(dy, 16) || !aligned_to(dx, 16))
+        return MTA_ERR_UNSUPPORTED;
+    const int mode = causal == MTA_CAUSAL_LOWER_ONLY ? 2 : (causal ? 1 : 0);
+    const int done = conv2d_grads_launch(x, dy, w, dx, (float *)workspace, &bpc, N, C, H, W, R, S, mode, io_dtype, (hipStream_t)stream);
+    if (done == MTA_OK) *job = {workspace, dw, (int32_t)C, R * S, bpc, 0, 0, w_dtype, scale};
+    return done;
+}
+
+extern "C" int mta_conv2d_grads(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
+                                int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype, int w_dtype, void *stream)
+{
+    mta_partials job;
+    const int rc = mta_conv2d_grads_partials(x, dy, w, dx, dw, workspace, workspace_bytes, N, C, H, W, R, S, causal, scale, io_dtype, w_dtype, &job, stream);
     return rc != MTA_OK ? rc : mta_sum_partials(1, &job, stream);
 }

@@ -429,9 +429,9 @@ std::pair<Tensor, Tensor> headmix_bwd(const Tensor &dy, const Tensor &x, const T
             need_w ? headmix_bwd_weight(x, dy.to(x.scalar_type()), w, causal, group) : Tensor()};
 }
 
-// the gradients of q, k, conv_w and w_pre (need[i]: wanted) from the one of the probabilities p
+// the gradients of q, k, conv_w and w_pre (need[i]: wanted) from the one of the probabilities p.  small: as in headmix_bwd
 void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, const Tensor &w_pre, Tensor raw, const Tensor &x, const Tensor &p,
-                       const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4], Sums &sums)
+                       const OptTensor &first, bool causal, bool pre_causal, int64_t pre_group, Tensor dp, const bool (&need)[4], Tensor *(&&out)[4], bool small, Sums &sums)
 {
     const double scale = score_scale(q);
     // (the head mixing's gradient kernels never read above the diagonal when causal)
@@ -451,9 +451,24 @@ void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, c
         if (!need_x) return;
         dx = headmix_bwd_input(ds, w_pre, pre_causal, pre_group, !causal);
     }
+    auto stage_input = [&] {   // (the kernel gradient reads its first argument on and below the diagonal only)
+        if (raw.defined()) return;
+        const OptTensor lower_raw = causal ? lower_scores(q, k, first) : OptTensor();
+        TORCH_CHECK(lower_raw || !first);
+        raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
+    };
+    const bool lower = causal && q.sizes() == k.sizes() && dx.scalar_type() == q.scalar_type() && lower_products_supported(q.scalar_type(), q.sizes(), true);
+    Tensor g;
+    if (need[2] && (need[0] || need[1] || small)) {
+        const bool formed = !raw.defined();   // (formed here: no further tensor for the gradient)
+        stage_input();
+        if (auto both = conv2d_grads(raw, dx, conv_w, causal, !lower, scale, sums, formed)) {
+            std::tie(g, *out[2]) = *both;
+            raw.reset();
+        }
+    }
     if (need[0] || need[1]) {
-        const bool lower = causal && q.sizes() == k.sizes() && dx.scalar_type() == q.scalar_type() && lower_products_supported(q.scalar_type(), q.sizes(), true);
-        const Tensor g = conv2d_bwd_input(dx, conv_w, causal, !lower);
+        if (!g.defined()) g = conv2d_bwd_input(dx, conv_w, causal, !lower);
         if (first) band_zero_(g, *first);
         Tensor dq, dk;
         OptTensor own_q, own_k;
@@ -477,12 +492,8 @@ void probabilities_bwd(const Tensor &q, const Tensor &k, const Tensor &conv_w, c
         *out[0] = dq;
         *out[1] = dk;
     }
-    if (need[2]) {
-        if (!raw.defined()) {   // (the kernel gradient reads its first argument on and below the diagonal only)
-            const OptTensor lower_raw = causal ? lower_scores(q, k, first) : OptTensor();
-            TORCH_CHECK(lower_raw || !first);
-            raw = lower_raw ? *lower_raw : at::matmul(q, k.transpose(2, 3));
-        }
+    if (need[2] && !out[2]->defined()) {
+        stage_input();
         *out[2] = conv2d_bwd_weight(raw, dx, conv_w, causal, scale, sums);
     }
 }
@@ -602,12 +613,16 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
             Tensor dc;
             std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], true, sums);
             dm.reset();
-            if (need[5]) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0, sums);
+            Tensor dp;
+            if (need[5]) {   // (alone, too: see headmix_bwd)
+                if (auto both = conv2d_grads(p, dc, post_conv_w, causal, !causal, 1.0, sums)) std::tie(dp, out[5]) = *both;
+            }
+            if (need[5] && !out[5].defined()) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0, sums);
             if (need_p) {
-                Tensor dp = conv2d_bwd_input(dc, post_conv_w, causal, !causal);
+                if (!dp.defined()) dp = conv2d_bwd_input(dc, post_conv_w, causal, !causal);
                 dc.reset();
                 probabilities_bwd(q, k, conv_w, w_pre, raw, x, p, first, causal, pre_causal, pre_group, std::move(dp), {need[0], need[1], need[3], need[4]},
-                                  {&out[0], &out[1], &out[3], &out[4]}, sums);
+                                  {&out[0], &out[1], &out[3], &out[4]}, true, sums);
             }
         }
         sums.run();
@@ -678,7 +693,7 @@ struct Probabilities : torch::autograd::Function<Probabilities> {
         probabilities_bwd(s[0], s[1], s[2], s[3], s[4], s[5], s[6], option(s[7]), ctx->saved_data["causal"].toBool(),
                           ctx->saved_data["pre_causal"].toBool(), ctx->saved_data["pre_group"].toInt(), grads[0].to(s[6].scalar_type()),
                           {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)},
-                          {&out[0], &out[1], &out[2], &out[3]}, sums);
+                          {&out[0], &out[1], &out[2], &out[3]}, false, sums);
         sums.run();
         return out;
     }
@@ -702,9 +717,13 @@ struct Conv2d : torch::autograd::Function<Conv2d> {
         const bool causal = ctx->saved_data["causal"].toBool();
         torch::autograd::variable_list out(5);
         const Tensor dy = on_gpu(grads[0], "grad_output");
-        if (ctx->needs_input_grad(0)) out[0] = conv2d_bwd_input(dy, saved[1], causal, ctx->saved_data["grad_fill_upper"].toBool());
+        const bool fill_upper = ctx->saved_data["grad_fill_upper"].toBool();
         Sums sums;
-        if (ctx->needs_input_grad(1)) out[1] = conv2d_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, 1.0, sums);
+        if (ctx->needs_input_grad(0) && ctx->needs_input_grad(1)) {
+            if (auto both = conv2d_grads(saved[0], dy, saved[1], causal, fill_upper, 1.0, sums)) std::tie(out[0], out[1]) = *both;
+        }
+        if (ctx->needs_input_grad(0) && !out[0].defined()) out[0] = conv2d_bwd_input(dy, saved[1], causal, fill_upper);
+        if (ctx->needs_input_grad(1) && !out[1].defined()) out[1] = conv2d_bwd_weight(saved[0], dy.to(saved[0].scalar_type()), saved[1], causal, 1.0, sums);
         sums.run();
         return out;
     }

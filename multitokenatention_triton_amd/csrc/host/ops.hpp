@@ -143,6 +143,30 @@ inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tenso
     return dw;
 }
 
+// Both gradients of the conv in one pass over dy, the kernel's times `scale` (in `sums`); over_x: the input's gradient takes the place of x.
+// Nothing where there is no kernel.
+inline std::optional<std::pair<Tensor, Tensor>> conv2d_grads(const Tensor &x_, const Tensor &dy_, const Tensor &w_, bool causal, bool fill_upper,
+                                                             double scale, Sums &sums, bool over_x = false)
+{
+    if (dy_.scalar_type() == at::kFloat || dy_.scalar_type() != x_.scalar_type() || dy_.scalar_type() != w_.scalar_type() || dy_.sizes() != x_.sizes())
+        return std::nullopt;
+    const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
+    check_conv_weight(w, dy.size(1));
+    const int64_t n = x.size(0), c = x.size(1), h = x.size(2), wd = x.size(3);
+    const int r = (int)w.size(1), s = (int)w.size(2);
+    const int64_t bytes = std::max<int64_t>(mta_conv2d_bwd_weight_workspace(n, c, h, wd, r, s), 16);
+    Tensor dx = over_x ? x : at::empty(dy.sizes(), dy.options());
+    Tensor dw = at::empty(w.sizes(), w.options()), ws = at::empty({bytes}, x.options().dtype(at::kByte));
+    const int rc = mta_conv2d_grads_partials(ptr(x), ptr(dy), ptr(w), out_ptr(dx), out_ptr(dw), out_ptr(ws), bytes, n, c, h, wd, r, s,
+                                             causal_mode(causal, fill_upper), (float)scale, code(x, "input"), code(w, "weight"), sums.add(dw, ws), stream_of(x));
+    if (rc == MTA_ERR_UNSUPPORTED) {
+        sums.drop();
+        return std::nullopt;
+    }
+    check(rc, "mta_conv2d_grads");
+    return std::make_pair(dx, dw);
+}
+
 inline Tensor headmix(const Tensor &x_, const Tensor &w_, bool causal, double fill, int64_t group, bool fill_upper)
 {
     const Tensor x = on_gpu(x_, "input"), w = on_gpu(w_, "weight");

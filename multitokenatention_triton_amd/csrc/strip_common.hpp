@@ -10,6 +10,7 @@
 namespace {
 using namespace mta;
 
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // Returns its argument, opaquely: what is derived from the result cannot be hoisted out of the (rarely taken) block
@@ -69,13 +70,19 @@ __device__ __forceinline__ unsigned lds_load_u16(unsigned addr)
 }
 __device__ __forceinline__ void lds_store8_at(unsigned addr, int off, unsigned lo, unsigned hi)
 {
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
     const u32x2 v = {lo, hi};
     asm volatile("ds_write_b64 %0, %1 offset:%2" : : "v"(addr), "v"(v), "n"(off) : "memory");
 }
 __device__ __forceinline__ void lds_store16(unsigned addr, u32x4 v)
 {
     asm volatile("ds_write_b128 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
+// the transpose read: of 16 lanes, lane l at 8 bytes (16-bit elements 4 (l % 4) ..) of row l / 4; it gets element l of the four rows
+__device__ __forceinline__ u32x2 lds_load_tr8_at(unsigned addr, int off)
+{
+    u32x2 v;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(off) : "memory");
+    return v;
 }
 __device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
 __device__ __forceinline__ void lds_wait(u32x4 &a) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a) : : "memory"); }

@@ -150,6 +150,29 @@ def conv2d_bwd_weight(x: torch.Tensor, dy: torch.Tensor, kernel_size, causal: bo
     return dw
 
 
+def conv2d_grads(x: torch.Tensor, dy: torch.Tensor, weight: torch.Tensor, causal: bool, fill_upper: bool = True, over_x: bool = False):
+    """Both gradients of ``conv2d_causal`` (input, kernel in the weight's dtype) in one pass over dy; ``over_x``: the input's takes
+    the place of x.  None where there is no kernel; see mta_conv2d_grads."""
+    x, dy, weight = _device_tensor(x, "input"), _device_tensor(dy, "grad_output"), _device_tensor(weight.detach(), "weight")
+    if x.dim() != 4 or x.shape != dy.shape or x.dtype != dy.dtype:
+        raise ValueError("input and grad_output must share shape and dtype")
+    n, c, h, w = x.shape
+    c_out, r, s = weight.shape
+    assert c == c_out, "This implementation assumes depthwise convolution (C_in == C_out)"
+    if len({t.device for t in (x, dy, weight)}) > 1:
+        raise ValueError("input, grad_output and weight must lie on one device")
+    lib = _lib.load()
+    dx, dw = x if over_x else torch.empty_like(x), torch.empty_like(weight)
+    ws = _workspace(lib.mta_conv2d_bwd_weight_workspace(n, c, h, w, r, s), x.device)
+    with torch.cuda.device(x.device):
+        rc = lib.mta_conv2d_grads(x.data_ptr(), dy.data_ptr(), weight.data_ptr(), dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(),
+                                  n, c, h, w, r, s, _causal_mode(causal, fill_upper), 1.0, _code(x, "input"), _code(weight, "weight"), _stream(x))
+    if rc == _lib.MTA_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "mta_conv2d_grads")
+    return dx, dw
+
+
 def headmix_bwd_input(dy: torch.Tensor, weight: torch.Tensor, causal: bool = True,
                       group_size: Optional[int] = None, fill_upper: bool = True,
                       out: Optional[torch.Tensor] = None) -> torch.Tensor:

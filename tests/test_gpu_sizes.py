@@ -1087,3 +1087,41 @@ def test_attention_of_few_workgroups(pkg, d, dtype, r, k):
             (many, many_lse), (few, few_lse) = run(0, 600), run(590, 600)
             assert torch.equal(many[:, 590:], few) and torch.equal(many_lse[:, 590:], few_lse), (s, causal)
             assert torch.isfinite(many.float()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,k", [(3, 3), (3, 5), (5, 5), (5, 7), (6, 11), (7, 7), (7, 9), (11, 15)])
+def test_conv_both_gradients(pkg, r, k, dtype):
+    """Both gradients of the conv in one pass over dy against the two kernels: dx bit for bit; dw, the same exact products summed in fp32 in
+    another order and rounded to the weight's dtype, within sqrt(n)*2^-22 of the sum of magnitudes and half a unit.  Edges of the 64 x 128
+    strips, fewer strips than workgroups and several rounds of them, more channels than workgroups; whole rows, the lower triangle, no
+    mask on planes that are not square; NaN above the diagonal of both operands."""
+    g = torch.Generator(device="cuda").manual_seed(67)
+    for b, c, h, w, causal, fill in ((1, 2, 8, 8, True, True), (2, 3, 64, 64, True, False), (1, 2, 136, 136, True, True), (2, 2, 200, 200, True, False),
+                                     (1, 520, 72, 72, True, True), (3, 1, 1288, 1288, True, True), (1, 2, 1096, 1096, True, False),
+                                     (2, 3, 65, 136, False, True), (1, 2, 200, 128, False, True), (1, 1, 3, 520, False, True)):
+        x, dy = (torch.randn(b, c, h, w, generator=g, device="cuda").to(dtype) for _ in range(2))
+        weight = torch.randn(c, r, k, generator=g, device="cuda").to(dtype)
+        size = pkg.ops.conv2d_bwd_weight(x.abs(), dy.abs(), (r, k), causal).double()
+        if causal:
+            above = ~torch.tril(torch.ones(h, w, dtype=torch.bool, device="cuda"))
+            x, dy = x.masked_fill(above, float("nan")), dy.masked_fill(above, float("nan"))
+        dx, dw = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill)
+        want = pkg.ops.conv2d_bwd_input(dy, weight, causal, fill_upper=fill)
+        assert torch.equal(dx, want) if fill else torch.equal(dx.tril(), want.tril()), (b, c, h, w)
+        exact = pkg.ops.conv2d_bwd_weight(x, dy, (r, k), causal).double()
+        bound = (b * h * w) ** 0.5 * 2.0 ** -22 * size + exact.abs() * _unit(dtype) + (2.0 ** -25 if dtype == torch.float16 else 0.0)
+        assert dw.dtype == dtype and ((dw.double() - exact).abs() <= bound).all(), (b, c, h, w)
+        _, again = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill, over_x=True)   # the gradient in x's place
+        assert torch.equal(again, dw) and (torch.equal(x, dx) if fill else torch.equal(x.tril(), dx.tril())), (b, c, h, w)
+
+
+def test_conv_both_gradients_refuses(pkg):
+    """No kernel: other dtypes, sizes and alignments than those of the two matrix-core kernels, and causal planes that are not square."""
+    def ask(h, w, r=3, k=3, causal=True, io=torch.bfloat16, wd=torch.bfloat16, shift=0):
+        x, dy = (torch.randn(2 * h * w + shift, device="cuda").to(io)[shift:].view(1, 2, h, w) for _ in range(2))
+        return pkg.ops.conv2d_grads(x, dy, torch.randn(2, r, k, device="cuda").to(wd), causal)
+    assert ask(64, 64) is not None and ask(64, 72, causal=False) is not None
+    for call in (dict(h=64, w=72), dict(h=68, w=68), dict(h=64, w=64, r=4, k=5), dict(h=64, w=64, io=torch.float32, wd=torch.float32),
+                 dict(h=64, w=64, wd=torch.float32), dict(h=64, w=64, shift=1)):
+        assert ask(**call) is None, call
