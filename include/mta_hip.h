@@ -402,8 +402,8 @@ typedef struct mta_partials {
 #define MTA_MAX_SUMS 8
 int mta_sum_partials(int count, const mta_partials *jobs, void *stream);
 /* mta_conv2d_bwd_input and mta_conv2d_bwd_weight_as in one pass over dy: dx and dw as those two define them.  16-bit data with weights
- * of the same dtype, W of whole 16-byte vectors, x, dy and dx aligned to them, kernels with a matrix-core instantiation;
- * MTA_ERR_UNSUPPORTED otherwise.  dx may be x itself (not a part of it).  Workspace as for the weight gradient alone
+ * of the same dtype, W of whole 16-byte vectors, x, dy and dx aligned to them: kernels with a matrix-core instantiation, causal planes
+ * square.  Else: kernels of 3x3, 3x5, 5x5 and 5x7, W >= 4.  MTA_ERR_UNSUPPORTED otherwise.  dx may be x itself (not a part of it).  Workspace as for the weight gradient alone
  * (mta_conv2d_bwd_weight_workspace). */
 int mta_conv2d_grads(const void *x, const void *dy, const void *w, void *dx, void *dw, void *workspace, int64_t workspace_bytes, int64_t N,
                      int64_t C, int64_t H, int64_t W, int R, int S, int causal, float scale, int io_dtype, int w_dtype, void *stream);

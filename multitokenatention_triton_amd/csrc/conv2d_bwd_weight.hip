@@ -570,10 +570,11 @@ extern "C" int mta_conv2d_grads_partials(const void *x, const void *dy, const vo
     int bpc = blocks_per_channel(N, C, H, W, MAX_PARTIALS);
     if (workspace_bytes < (int64_t)bpc * C * R * S * (int64_t)sizeof(float)) return MTA_ERR_WORKSPACE;
     static const bool force_valu = [] { const char *e = getenv("MTA_CONV_FORCE_VALU"); return e && e[0] == '1'; }();
-    if (force_valu || io_dtype == MTA_F32 || w_dtype != io_dtype || W % 8 != 0 || !aligned_to(x, 16) || !aligned_to(dy, 16) || !aligned_to(dx, 16))
-        return MTA_ERR_UNSUPPORTED;
+    if (force_valu) return MTA_ERR_UNSUPPORTED;
+    const bool mfma = io_dtype != MTA_F32 && w_dtype == io_dtype && W % 8 == 0 && aligned_to(x, 16) && aligned_to(dy, 16) && aligned_to(dx, 16);
     const int mode = causal == MTA_CAUSAL_LOWER_ONLY ? 2 : (causal ? 1 : 0);
-    const int done = conv2d_grads_launch(x, dy, w, dx, (float *)workspace, &bpc, N, C, H, W, R, S, mode, io_dtype, (hipStream_t)stream);
+    const int done = mfma ? conv2d_grads_launch(x, dy, w, dx, (float *)workspace, &bpc, N, C, H, W, R, S, mode, io_dtype, (hipStream_t)stream)
+                          : conv2d_grads_rows_launch(x, dy, w, dx, (float *)workspace, &bpc, N, C, H, W, R, S, mode, io_dtype, w_dtype, (hipStream_t)stream);
     if (done == MTA_OK) *job = {workspace, dw, (int32_t)C, R * S, bpc, 0, 0, w_dtype, scale};
     return done;
 }

@@ -148,8 +148,7 @@ inline Tensor conv2d_bwd_weight(const Tensor &x_, const Tensor &dy_, const Tenso
 inline std::optional<std::pair<Tensor, Tensor>> conv2d_grads(const Tensor &x_, const Tensor &dy_, const Tensor &w_, bool causal, bool fill_upper,
                                                              double scale, Sums &sums, bool over_x = false)
 {
-    if (dy_.scalar_type() == at::kFloat || dy_.scalar_type() != x_.scalar_type() || dy_.scalar_type() != w_.scalar_type() || dy_.sizes() != x_.sizes())
-        return std::nullopt;
+    if (dy_.scalar_type() != x_.scalar_type() || dy_.sizes() != x_.sizes()) return std::nullopt;
     const Tensor x = on_gpu(x_, "input"), dy = on_gpu(dy_, "grad_output"), w = on_gpu(w_, "weight");
     check_conv_weight(w, dy.size(1));
     const int64_t n = x.size(0), c = x.size(1), h = x.size(2), wd = x.size(3);

@@ -1117,11 +1117,41 @@ def test_conv_both_gradients(pkg, r, k, dtype):
 
 
 def test_conv_both_gradients_refuses(pkg):
-    """No kernel: other dtypes, sizes and alignments than those of the two matrix-core kernels, and causal planes that are not square."""
-    def ask(h, w, r=3, k=3, causal=True, io=torch.bfloat16, wd=torch.bfloat16, shift=0):
+    """No kernel: causal planes that are not square on the matrix cores, and for what those do not take - other dtypes, widths and
+    alignments - kernels of more than 35 taps."""
+    def ask(h, w, r=7, k=7, causal=True, io=torch.bfloat16, wd=torch.bfloat16, shift=0):
         x, dy = (torch.randn(2 * h * w + shift, device="cuda").to(io)[shift:].view(1, 2, h, w) for _ in range(2))
         return pkg.ops.conv2d_grads(x, dy, torch.randn(2, r, k, device="cuda").to(wd), causal)
     assert ask(64, 64) is not None and ask(64, 72, causal=False) is not None
     for call in (dict(h=64, w=72), dict(h=68, w=68), dict(h=64, w=64, r=4, k=5), dict(h=64, w=64, io=torch.float32, wd=torch.float32),
-                 dict(h=64, w=64, wd=torch.float32), dict(h=64, w=64, shift=1)):
+                 dict(h=64, w=64, wd=torch.float32), dict(h=64, w=64, shift=1), dict(h=3, w=3, r=3, k=3)):
         assert ask(**call) is None, call
+
+
+@pytest.mark.parametrize("dtype,wd", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("r,k", [(3, 3), (3, 5), (5, 5), (5, 7)])
+def test_conv_both_gradients_by_rows(pkg, r, k, dtype, wd):
+    """Both gradients of the conv in one pass on the vector units against the two kernels: dx bit for bit (fp16: or the neighbour, since
+    a last multiply-add may be rounded to 16 bits with or without a stop at 32); dw, fp32 sums in another order, within sqrt(n)*2^-22 of
+    the sum of magnitudes (and half a unit of a 16-bit weight).  Strips of 4 and 8 rows, one wavefront's and
+    several rounds of them, the edges of their 240 to 248 keys, the narrowest rows; whole rows, the lower triangle, no mask, planes
+    that are not square; NaN above the diagonal of both operands; the gradient in x's place."""
+    g = torch.Generator(device="cuda").manual_seed(68)
+    for b, c, h, w, causal, fill in ((1, 2, 5, 5, True, True), (2, 3, 65, 65, True, False), (1, 2, 249, 249, True, True), (2, 2, 121, 121, True, False),
+                                     (2, 3, 65, 4, False, True), (1, 2, 30, 301, True, True), (1, 2, 301, 30, True, True), (1, 1100, 41, 41, True, True),
+                                     (8, 16, 489, 489, True, True), (8, 16, 489, 489, True, False)):
+        x, dy = (torch.randn(b, c, h, w, generator=g, device="cuda").to(dtype) for _ in range(2))
+        weight = torch.randn(c, r, k, generator=g, device="cuda").to(wd)
+        size = pkg.ops.conv2d_bwd_weight(x.abs(), dy.abs(), (r, k), causal).double()
+        if causal:
+            above = ~torch.tril(torch.ones(h, w, dtype=torch.bool, device="cuda"))
+            x, dy = x.masked_fill(above, float("nan")), dy.masked_fill(above, float("nan"))
+        dx, dw = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill)
+        want = pkg.ops.conv2d_bwd_input(dy, weight, causal, fill_upper=fill)
+        at, of = (dx, want) if fill else (dx.tril(), want.tril())
+        torch.testing.assert_close(at, of, rtol=2.0 ** -10 if dtype == torch.float16 else 0.0, atol=2.0 ** -24 if dtype == torch.float16 else 0.0)
+        exact = pkg.ops.conv2d_bwd_weight(x, dy, (r, k), causal).double()
+        half = 0.0 if wd == torch.float32 else exact.abs() * _unit(wd) + 2.0 ** -25
+        assert dw.dtype == wd and ((dw.double() - exact).abs() <= (b * h * w) ** 0.5 * 2.0 ** -22 * size + half).all(), (b, c, h, w)
+        _, again = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill, over_x=True)
+        assert torch.equal(again, dw) and (torch.equal(x, dx) if fill else torch.equal(x.tril(), dx.tril())), (b, c, h, w)
