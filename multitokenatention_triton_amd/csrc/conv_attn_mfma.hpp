@@ -38,7 +38,9 @@ typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 
 // The workgroup has NW = 4 wavefronts and owns 128 score rows; two workgroups per CU for the attention kernel (three at D = 64 up
-// to 7 kernel rows), three for the scores-only one, which overlap each other's barriers and memory latency.
+// to 7 kernel rows), three for the scores-only one, which overlap each other's barriers and memory latency.  Attention over small
+// grids: NW = 8 with one block of 16 rows each, see launch_mfma.  (The scores-only kernel on eight, with the fragments of K read twice as
+// often: 6x11 B2 H16 S512 D64 12.5 -> 17.4 us, B4 H16 S1024 D128 38.4 -> 43.2.)
 // What bounds the attention kernel: matrix products (896 flops executed per score at 6x11, D = 128: Q K^T and P V 256 each, the
 // conv as Toeplitz products 384) beside the vector ALU (the exponentials) and the LDS, which would each take 40 to 60 % of its
 // time alone.  So the vector work is kept small (one maximum, one multiply-add, one exponential and half a conversion and a sum
