@@ -189,7 +189,7 @@ int conv2d_grads_launch(const void *x, const void *dy, const void *w, void *dx, 
 // conv2d_grads_rows.hip: the same on the vector units, for other types and widths
 int conv2d_grads_rows_launch(const void *x, const void *dy, const void *w, void *dx, float *partial, int *bpc, int64_t N, int64_t C, int64_t H,
                              int64_t W, int R, int S, int causal, int io_dtype, int w_dtype, hipStream_t st);
-// conv2d_split.hip: depthwise conv (11x15) on the bf16 matrix cores with the 32 bits of data and weights kept (forward or input gradient;
+// conv2d_split.hip: depthwise conv of large kernels on the bf16 matrix cores with the 32 bits of data and weights kept (forward or input gradient;
 // causal as in conv2d_causal.hip); 1 where it has no instance
 int conv2d_split_dispatch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,
                           float in_scale, int use_scale, int io_dtype, int w_dtype, hipStream_t st);

@@ -1,10 +1,10 @@
-// Depthwise conv of 11x15 kernels, forward and input gradient, for what the kernels of conv2d_causal.hip on the matrix cores do not
-// take (fp32 data; 16-bit data with weights of another dtype or rows that are not whole 16-byte vectors): on the bf16 matrix
-// cores, with the 32 bits kept.
+// Depthwise conv of large kernels, forward and input gradient, for what the kernels of conv2d_causal.hip on the matrix cores do not
+// take (11x15: fp32 data; that and smaller ones: 16-bit data with weights of another dtype or rows that are not whole 16-byte
+// vectors): on the bf16 matrix cores, with the 32 bits kept.
 //
 // Every fp32 value is the sum of three bf16 values (8 + 8 + 8 bits of its significand; each one the rounded remainder of those
-// before it), exactly: x = x0 + x1 + x2, w = w0 + w1 + w2 (fp16: two parts, bf16: one).  Of the products of parts the six with
-// i + j <= 2 are formed; each is exact in fp32, what is left out is below 2^-26 |x w|, a quarter of the last place that one fp32
+// before it), exactly: x = x0 + x1 + x2, w = w0 + w1 + w2 (fp16: two parts, bf16: one).  Of the products of parts the six (bf16 data with
+// fp32 weights: three) with i + j <= 2 are formed; each is exact in fp32, what is left out is below 2^-26 |x w|, a quarter of the last place that one fp32
 // multiply-add rounds away.  A kernel row is applied as in conv2d_causal.hip, as a banded Toeplitz product (one 32-key window
 // holds the taps of 16 outputs), once per pair of parts: w0 x0 adds into one accumulator, the small ones into two others, and a
 // result is their sum.  So an output takes R roundings of its own size where multiply-adds took R*S: the error against 64 bits
@@ -16,6 +16,9 @@
 // 1024^2 105 -> 68, 16 of 2048^2 177 -> 128; whole rows 31 -> 20, 34 -> 31, 86 -> 43, 152 -> 80, 260 -> 151.  Smaller kernels stay
 // there, lower triangle | whole rows: 7x9 16 of 1024^2 29.7 | 39.4 against 29.4 | 34.5 here, 16 of 512^2 13.9 | 16.4 against 15.3 |
 // 16.5, 16 of 2048^2 92 | 128 against 98 | 140; 6x11 and 5x7 alike or slower.
+// 16-bit data with fp32 weights, lower triangle of 16 planes of 1024^2, bf16 | fp16: 5x7 22.2 -> 18.6 | 22.2 -> 22.7, 7x7 26.0 -> 20.6 | (kept) 26.4,
+// 6x11 29.4 -> 19.5 | 29.6 -> 24.6, 7x9 28.9 -> 20.8 | 29.4 -> 25.8; bf16 16 of 512^2 6x11 13.0 -> 10.8, 32 of 2048^2 6x11 152 -> 115, 7x7 121 -> 117 (5x7
+// 109 -> 114: kept); weights of the data's type, whole rows of 16 planes of 1001^2: bf16 7x7 34.6 -> 23.3, 6x11 40.4 -> 22.9, fp16 6x11 40.8 -> 28.1.
 // What bounds it: half of the time the matrix cores are busy (16 of 2048^2: 62 of 128 us); without the loads, stores and
 // the splitting the products take 95 us - their operands' LDS reads, the barrier of a strip and the blocks beside the
 // triangle - and the CU's path to the L2 (1.5 times the strip in, the strip out) the rest.
@@ -67,7 +70,7 @@ __device__ __forceinline__ bool tiny(unsigned state) { return (state & (P_USUAL 
 
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
-template <typename T, int R, int S, bool BWD>
+template <typename T, int WP, int R, int S, bool BWD>
 __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
                                                        int W, int causal, float in_scale, int use_scale, int w_dtype, int planes, int total, int per_plane)
 {
@@ -76,7 +79,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
     constexpr int ROWS = P_TM + R - 1, RPI = 256 / P_QUADS, IT = (ROWS + RPI - 1) / RPI;   // a round of loads: RPI rows, four threads idle
     constexpr int PLANE = ROWS * P_LD;                 // bf16 values of one part
     constexpr int NE = S + 7;                          // windows of a kernel row that hold a tap: first slot - SHIFT - ln = -7 .. S-1
-    constexpr int XP = parts_of<T>(), WP = 3;          // parts of a value, of a tap
+    constexpr int XP = parts_of<T>();                  // parts of a value (WP: of a tap)
     __shared__ __align__(16) uint16_t xs[2][XP * PLANE];
     static_assert(WP * R * (NE + 1) * 8 + WP * R * (S + 16) <= 2 * XP * PLANE, "the table of windows borrows the strips' LDS");
     __shared__ unsigned state[4];                      // of the strips staged, one in three in turns; [3]: of the kernel
@@ -274,10 +277,10 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
                         const int m = b * R + i;
                         if (m + 1 < 4 * R) read(m + 1);
                         if constexpr (XP > 2) mma16(small0, tz[0][i], f[m & 1][2]);
-                        mma16(small1, tz[1][i], f[m & 1][0]);
-                        if constexpr (XP > 1) mma16(small0, tz[1][i], f[m & 1][1]);
+                        if constexpr (WP > 1) mma16(small1, tz[WP > 1 ? 1 : 0][i], f[m & 1][0]);
+                        if constexpr (XP > 1 && WP > 1) mma16(small0, tz[WP > 1 ? 1 : 0][i], f[m & 1][1]);
                         if constexpr (XP > 1) mma16(small1, tz[0][i], f[m & 1][1]);
-                        mma16(small0, tz[2][i], f[m & 1][0]);
+                        if constexpr (WP > 2) mma16(small0, tz[WP > 2 ? 2 : 0][i], f[m & 1][0]);
                         mma16(big, tz[0][i], f[m & 1][0]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
@@ -364,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
     }
 }
 
-template <typename T, int R, int S, bool BWD>
+template <typename T, int WP, int R, int S, bool BWD>
 int launch_split(const void *x, const void *w, void *y, int64_t planes, int64_t C, int64_t H, int64_t W, int causal, float in_scale, int use_scale,
                  int w_dtype, hipStream_t st)
 {
@@ -372,19 +375,49 @@ int launch_split(const void *x, const void *w, void *y, int64_t planes, int64_t 
     if (total > 0x3fffffffLL) return MTA_ERR_SHAPE;
     int64_t per_plane = (2 * device_cu_count() + planes - 1) / planes;   // one round of resident workgroups
     if (per_plane > total) per_plane = total;
-    hipLaunchKernelGGL((conv2d_split<T, R, S, BWD>), dim3((unsigned)(planes * per_plane)), dim3(256), 0, st, (const T *)x, w, (T *)y, (int)C, (int)H,
+    hipLaunchKernelGGL((conv2d_split<T, WP, R, S, BWD>), dim3((unsigned)(planes * per_plane)), dim3(256), 0, st, (const T *)x, w, (T *)y, (int)C, (int)H,
                        (int)W, causal, in_scale, use_scale, w_dtype, (int)planes, (int)total, (int)per_plane);
     return launch_status();
+}
+
+// weights of the data's own type have its parts, others three
+template <typename T>
+int dispatch_split(const void *x, const void *w, void *y, int64_t planes, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,
+                   float in_scale, int use_scale, bool same, int w_dtype, hipStream_t st)
+{
+#define MTA_SPLIT(wp, r, s)                                                                                                     \
+    (bwd ? launch_split<T, wp, r, s, true>(x, w, y, planes, C, H, W, causal, in_scale, use_scale, w_dtype, st)                  \
+         : launch_split<T, wp, r, s, false>(x, w, y, planes, C, H, W, causal, in_scale, use_scale, w_dtype, st))
+#define MTA_CONV_CASE(r, s)                                                                                                     \
+    if (R == r && S == s) {                                                                                                     \
+        if constexpr (sizeof(T) == 2) {                                                                                         \
+            if (same) return MTA_SPLIT(parts_of<T>(), r, s);                                                                    \
+        }                                                                                                                       \
+        return MTA_SPLIT(3, r, s);                                                                                              \
+    }
+    MTA_CONV_CASE(11, 15)
+    // 16-bit data: fewer parts, so that smaller kernels gain as well.  bf16: from 49 taps on, 5x7 up to 32 M elements; fp16, with twice the parts:
+    // from 60 taps on (7x7: S1024 26.4 | 25.4, but B2 H12 S640 19.1 | 21.7, B2 H16 S2048 123 | 143)
+    if constexpr (sizeof(T) == 2) {
+        MTA_CONV_CASE(6, 11)
+        MTA_CONV_CASE(7, 9)
+        if constexpr (parts_of<T>() == 1) {
+            MTA_CONV_CASE(7, 7)
+            if (planes * H * W <= 32 << 20) {
+                MTA_CONV_CASE(5, 7)
+            }
+        }
+    }
+#undef MTA_CONV_CASE
+#undef MTA_SPLIT
+    return 1;
 }
 }  // namespace
 
 int mta::conv2d_split_dispatch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t H, int64_t W, int R, int S, bool bwd, int causal,
                                float in_scale, int use_scale, int io_dtype, int w_dtype, hipStream_t st)
 {
-    if (R != 11 || S != 15 || W < 4) return 1;
-    MTA_DISPATCH_IO(io_dtype, {
-        return bwd ? launch_split<io_t, 11, 15, true>(x, w, y, N * C, C, H, W, causal, in_scale, use_scale, w_dtype, st)
-                   : launch_split<io_t, 11, 15, false>(x, w, y, N * C, C, H, W, causal, in_scale, use_scale, w_dtype, st);
-    });
+    if (W < 4) return 1;
+    MTA_DISPATCH_IO(io_dtype, return dispatch_split<io_t>(x, w, y, N * C, C, H, W, R, S, bwd, causal, in_scale, use_scale, w_dtype == io_dtype, w_dtype, st));
     return 1;
 }

@@ -1131,8 +1131,9 @@ def test_conv_both_gradients_refuses(pkg):
 @pytest.mark.parametrize("dtype,wd", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("r,k", [(3, 3), (3, 5), (5, 5), (5, 7)])
 def test_conv_both_gradients_by_rows(pkg, r, k, dtype, wd):
-    """Both gradients of the conv in one pass on the vector units against the two kernels: dx bit for bit (fp16: or the neighbour, since
-    a last multiply-add may be rounded to 16 bits with or without a stop at 32); dw, fp32 sums in another order, within sqrt(n)*2^-22 of
+    """Both gradients of the conv in one pass on the vector units against the two kernels: dx bit for bit in fp32; in 16 bits the same
+    sums in another order (5x7), or a last multiply-add rounded to 16 bits with or without a stop at 32: 2^-24 of the magnitudes for each
+    of its r k steps on either side, and the neighbour; dw, fp32 sums in another order, within sqrt(n)*2^-22 of
     the sum of magnitudes (and half a unit of a 16-bit weight).  Strips of 4 and 8 rows, one wavefront's and
     several rounds of them, the edges of their 240 to 248 keys, the narrowest rows; whole rows, the lower triangle, no mask, planes
     that are not square; NaN above the diagonal of both operands; the gradient in x's place."""
@@ -1149,9 +1150,40 @@ def test_conv_both_gradients_by_rows(pkg, r, k, dtype, wd):
         dx, dw = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill)
         want = pkg.ops.conv2d_bwd_input(dy, weight, causal, fill_upper=fill)
         at, of = (dx, want) if fill else (dx.tril(), want.tril())
-        torch.testing.assert_close(at, of, rtol=2.0 ** -10 if dtype == torch.float16 else 0.0, atol=2.0 ** -24 if dtype == torch.float16 else 0.0)
+        if dtype == torch.float32:
+            assert torch.equal(at, of), (b, c, h, w)
+        else:
+            near = pkg.ops.conv2d_bwd_input(torch.where(dy.isnan(), torch.zeros_like(dy), dy).abs(), weight.abs(), causal).double()
+            near = 2 * (r * k + 2) * 2.0 ** -24 * near + 2 * _unit(dtype) * of.double().abs() + 2.0 ** -24
+            assert ((at.double() - of.double()).abs() <= near).all(), (b, c, h, w)
         exact = pkg.ops.conv2d_bwd_weight(x, dy, (r, k), causal).double()
         half = 0.0 if wd == torch.float32 else exact.abs() * _unit(wd) + 2.0 ** -25
         assert dw.dtype == wd and ((dw.double() - exact).abs() <= (b * h * w) ** 0.5 * 2.0 ** -22 * size + half).all(), (b, c, h, w)
         _, again = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill, over_x=True)
         assert torch.equal(again, dw) and (torch.equal(x, dx) if fill else torch.equal(x.tril(), dx.tril())), (b, c, h, w)
+
+
+@pytest.mark.parametrize("dtype,wd,r,k", [(d, w, *rk) for d, w, sizes in (
+    (torch.bfloat16, torch.float32, ((5, 7), (7, 7), (6, 11), (7, 9))), (torch.bfloat16, torch.bfloat16, ((5, 7), (7, 7), (6, 11), (7, 9))),
+    (torch.float16, torch.float32, ((6, 11), (7, 9))), (torch.float16, torch.float16, ((6, 11), (7, 9))), (torch.bfloat16, torch.float16, ((6, 11),))) for rk in sizes])
+def test_conv_split_of_16_bit_data(pkg, dtype, wd, r, k):
+    """16-bit data with other weights, or of odd widths, on the parts of the values: edges of the 32 x 128 strips, several strips in turns; an
+    infinite value stays where a tap takes it.  Bound: r k products and sums of 32 bits in any order, and one rounding to 16 bits."""
+    g = torch.Generator(device="cuda").manual_seed(69)
+    w = (0.1 * torch.randn(3, r, k, generator=g, device="cuda")).to(wd)
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for h, wid in ((1, 5), (31, 33), (33, 129), (128, 120) if wd != dtype else (128, 121), (333, 333)):
+        x = torch.randn(2, 3, h, wid, generator=g, device="cuda").to(dtype)
+        for causal in (True, False):
+            for bwd in (False, True):
+                got = pkg.ops.conv2d_bwd_input(x, w, causal) if bwd else pkg.ops.conv2d_causal(x, w, causal)
+                want, size = _conv64(x, w, causal, bwd)
+                bound = (r * k + 2) * 2.0 ** -24 * size + ulp * want.abs() + 2.0 ** -25
+                assert ((got.double() - want).abs() <= bound).all(), (h, wid, causal, bwd)
+    x[0, 0, 200, 100] = float("inf")
+    got, plain = pkg.ops.conv2d_causal(x, w, True), pkg.ops.conv2d_causal(x.masked_fill(x == float("inf"), 0.0), w, True)
+    touched = torch.zeros(333, 333, dtype=torch.bool, device="cuda")
+    touched[200:200 + r, 100 - (k - 1 - (k - 1) // 2):101 + (k - 1) // 2] = True
+    assert not torch.isfinite(got[0, 0][touched.tril()]).any()
+    torch.testing.assert_close(got[0, 0][~touched].float(), plain[0, 0][~touched].float(), rtol=2 * ulp, atol=2.0 ** -20)
+    assert torch.equal(got[0, 1], plain[0, 1])
