@@ -846,6 +846,43 @@ Tensor headmix_apply(const Tensor &x, const Tensor &w, bool causal, double fill,
     return HeadMix::apply(x, w, causal, fill, group, fill_upper, grad_fill_upper);
 }
 
+// Conv-attention in fp32 as scores, conv, softmax and P V, one kernel each, over as many planes at a time as a scratch of 256 MB holds
+// (two or three of them; a plane of S = 8192 fills one).  Nothing where the fused kernel is taken.
+OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &w, bool causal, double scale)
+{
+    constexpr int64_t SCRATCH = 256 << 20;
+    if (q_.scalar_type() != at::kFloat || !causal || q_.numel() == 0) return std::nullopt;
+    const int64_t b = q_.size(0), h = q_.size(1), s_real = q_.size(2), d = q_.size(3), s = (s_real + 7) / 8 * 8, plane = s * s * 4;
+    const int64_t r = w.size(1), sk = w.size(2);
+    if (plane > SCRATCH || !lower_products_supported(at::kFloat, {b, h, s, d}, true) || !conv_attn_in_stages(b * h, s_real, d, r, sk)) return std::nullopt;
+    Tensor q = q_, k = k_, v = v_;
+    if (s != s_real) {   // (the products take rows that are whole vectors)
+        RowsCopy rows(s, OptTensor());
+        q = rows.add(q_, false, 1.0);
+        k = rows.add(k_, false, 1.0);
+        v = rows.add(v_, false, 1.0);
+        rows.run();
+    } else {
+        v = on_gpu_vectors(v, "V");
+    }
+    Tensor o = at::empty(q.sizes(), q.options());
+    // equal parts: of the batch, or of one batch entry's heads
+    auto part = [](int64_t count, int64_t most) { const int64_t parts = (count + most - 1) / most; return (count + parts - 1) / parts; };
+    const int64_t nb = h * plane <= SCRATCH ? part(b, SCRATCH / (h * plane)) : 1, nh = h * plane <= SCRATCH ? h : part(h, SCRATCH / plane);
+    for (int64_t b0 = 0; b0 < b; b0 += nb)
+        for (int64_t h0 = 0; h0 < h; h0 += nh) {
+            const int64_t bs = std::min(nb, b - b0), hs = std::min(nh, h - h0);
+            auto of = [&](const Tensor &x) { return x.narrow(0, b0, bs).narrow(1, h0, hs); };   // (contiguous: all heads, or one batch entry)
+            const OptTensor raw = lower_scores(of(q), of(k), OptTensor());
+            TORCH_CHECK(raw, "no kernel for the lower-triangle products");
+            Tensor p = conv2d(*raw, w.narrow(0, h0, hs), true, scale, false);
+            p = headmix_softmax(p, OptTensor(), OptTensor(), true, 0, false, OptTensor(), OptTensor());
+            const Tensor vs = of(v), os = of(o);
+            check(mta_causal_pv_f32(ptr(p), ptr(vs), out_ptr(os), bs, hs, s, d, 1.0f, stream_of(p)), "mta_causal_pv_f32");
+        }
+    return s == s_real ? o : o.narrow(2, 0, s_real).contiguous();
+}
+
 // O = softmax(mask(conv(mask0(Q K^T))) * scale) V, without the row statistic a backward pass would keep
 Tensor conv_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &w_, bool causal, std::optional<double> softmax_scale)
 {
@@ -856,8 +893,9 @@ Tensor conv_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Ten
     TORCH_CHECK_TYPE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(), "Q, K, V must share a dtype");
     TORCH_CHECK(w.dim() == 3 && w.size(0) == q.size(1), "CHANNEL_DIM == NUM_HEADS");
     const c10::OptionalDeviceGuard guard(q.device());
-    Tensor o = at::empty(q.sizes(), q.options());
     const double scale = softmax_scale ? *softmax_scale : 1.0 / std::sqrt((double)q.size(3));
+    if (OptTensor staged = conv_attn_stages(q, k, v, w, causal, scale)) return *staged;
+    Tensor o = at::empty(q.sizes(), q.options());
     check(mta_conv_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(w), out_ptr(o), q.size(0), q.size(1), q.size(2), q.size(3), (int)w.size(1), (int)w.size(2),
                             causal, (float)scale, code(q, "Q"), code(w, "W"), stream_of(q)),
           "mta_conv_attn_fwd");

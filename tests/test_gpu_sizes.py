@@ -35,6 +35,28 @@ def test_conv_attention_kernel_sizes(pkg, dtype, r, sk, d, causal):
         torch.testing.assert_close(got.float(), want.float(), **tol(dtype))
 
 
+@pytest.mark.parametrize("b,h,s,d,r,sk", [
+    (1, 3, 64, 128, 6, 11), (1, 2, 65, 128, 3, 3), (2, 3, 129, 64, 11, 15), (1, 2, 200, 64, 3, 5), (2, 2, 257, 64, 5, 7),   # whole and ragged lengths
+    (3, 4, 2300, 64, 7, 9),      # the batch entries in turns
+    (2, 5, 4104, 128, 5, 5),     # the heads of a batch entry in turns, a last part that is smaller
+])
+@pytest.mark.parametrize("factor", [None, -0.3])
+def test_conv_attention_fp32_stages(pkg, b, h, s, d, r, sk, factor):
+    """fp32 conv-attention of sizes that take scores, conv, softmax and P V one after the other, against the fused kernel (which writes the
+    row statistic), which the tests above hold against the oracle: the two orders of sums differ by a few 2^-24 of the scores, whose
+    exponentials turn that into relative errors; both 2-norms are below 5e-7."""
+    print(f"conv_attention stages b={b} h={h} s={s} d={d} {r}x{sk}", flush=True)
+    q, k, v = (x.cuda() for x in O.seeded_qkv(b, h, s, d, torch.float32, seed=47))
+    module = pkg.TritonConvAttention(h, (r, sk), causal=True).cuda()
+    with torch.no_grad():
+        module.weight.copy_(O.seeded_conv_weight(h, r, sk, 0.05, torch.float32))
+        got = module(q, k, v, True, factor)[0]
+    want, _ = pkg.ops.conv_attn_fwd(q, k, v, module.weight.detach(), True, factor, return_lse=True)
+    assert got.shape == want.shape and got.is_contiguous()
+    assert ((got - want).double().norm() / want.double().norm()).item() < 2e-6
+    torch.testing.assert_close(got, want, **tol(torch.float32))
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("factor", [-0.08, 0.0, 0.08])
 @pytest.mark.parametrize("dtype,d,r,sk", [(torch.bfloat16, 128, 6, 11), (torch.float16, 64, 3, 3), (torch.float16, 128, 11, 15)])
