@@ -500,6 +500,13 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
             return launch_status();
         }
     }
+    if constexpr (VEC == 4 && sizeof(T) == 4) {
+        // 32 heads, rows that a workgroup covers with half vectors as well: twice the wavefronts, of half the registers, each half as long a chain
+        // of loads and FMAs.  us, 4 | 2 keys per lane, fp32: lower triangle B1 S64 15.5 | 11.9, S256 13.1 | 11.5, S512 16.5 | 14.3, B4 S256 18.1 | 15.4,
+        // S512 44 | 35; whole causal rows B4 S512 49 | 44.  Two workgroups a row lose: S1024 38.7 | 42.6, with 128 threads of 4 keys 44.3; rows
+        // without a triangle from 512 keys on, whose lanes are all busy: B4 S512 53 | 58.
+        if (G == 32 && Q <= (causal ? 512 : 256)) return launch<T, 2>(x, w, y, N, C, P, Q, G, causal, fill, w_dtype, wt, w_same_dtype, st);
+    }
     const int qchunks = (int)((Q + (int64_t)NT * VEC - 1) / ((int64_t)NT * VEC));
 #define MTA_HM_CASE(g)                                                                                         \
     if (G == g) {                                                                                              \

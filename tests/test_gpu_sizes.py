@@ -35,6 +35,25 @@ def test_conv_attention_kernel_sizes(pkg, dtype, r, sk, d, causal):
         torch.testing.assert_close(got.float(), want.float(), **tol(dtype))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("c,group", [(32, None), (64, 32)])
+@pytest.mark.parametrize("q", [4, 60, 256, 260, 508, 512, 516])
+def test_headmix_fp32_32_heads_short_rows(pkg, q, c, group, causal):
+    """fp32 mixing of 32 heads around the row lengths where the lanes' share changes, forward and input gradient, against 64 bits: 32 products
+    and sums of values around 1, each within 2^-24 of the running sum: 32 * 2^-24 * sqrt(32) < 2e-5."""
+    print(f"headmix fp32 q={q} c={c} group={group} causal={causal}", flush=True)
+    torch.manual_seed(3)
+    x, w = torch.randn(2, c, q, q), torch.randn(c, c)
+    if group:
+        block = torch.arange(c) // group
+        w = w * (block[:, None] == block[None, :])
+    keep = torch.ones(q, q).tril() if causal else torch.ones(q, q)
+    for fn, m in ((pkg.ops.headmix, w), (pkg.ops.headmix_bwd_input, w.t())):
+        want = torch.einsum("oi,nipq->nopq", m.double(), x.double()) * keep
+        got = fn(x.cuda(), w.cuda(), causal, group_size=group).cpu()
+        torch.testing.assert_close(got.double(), want, rtol=0, atol=2e-5)
+
+
 @pytest.mark.parametrize("b,h,s,d,r,sk", [
     (1, 3, 64, 128, 6, 11), (1, 2, 65, 128, 3, 3), (2, 3, 129, 64, 11, 15), (1, 2, 200, 64, 3, 5), (2, 2, 257, 64, 5, 7),   # whole and ragged lengths
     (3, 4, 2300, 64, 7, 9),      # the batch entries in turns
