@@ -22,8 +22,14 @@
 // What bounds it: half of the time the matrix cores are busy (16 of 2048^2: 62 of 128 us); without the loads, stores and
 // the splitting the products take 95 us - their operands' LDS reads, the barrier of a strip and the blocks beside the
 // triangle - and the CU's path to the L2 (1.5 times the strip in, the strip out) the rest.
-// What is not finite, or so large that a part overflows, takes multiply-adds after all; a strip whose largest value is so small
-// that parts underflow is staged once more, 2^100 times as large (its results are taken back).
+// Values that have three parts are split 2^24 times as large, results taken back: every fp32 value below 2^104 then has parts that are normal
+// numbers (the smallest denormal's only bit is 2^-125), however small it is and whatever lies beside it, and the products of parts of
+// small values stay above the denormals as well.  Results that are not finite then - an operand was not, or is larger, or a sum of
+// scaled products is beyond 2^128, one of 2^80 and more - take multiply-adds after all, one by one.  (An infinite part makes every result
+// non-finite whose window of slots holds it, also under a zero of the Toeplitz fragment: what is finite is exact.)
+// (A look at every strip's largest value, with strips of tiny values staged once more, cost 2 to 4 % in fp32 and 4 to 8 % in 16 bits and could
+// not see small values beside ordinary ones: lower triangle of 16 planes, fp32 512^2 19.2 -> 18.5 us, 2048^2 130.9 -> 127.9, bf16 with fp32
+// weights 1024^2 6x11 20.6 -> 19.5, fp16 7x9 26.4 -> 25.1.)
 //
 // Shape.  A workgroup of four wavefronts takes strips of 32 rows x 128 keys of one plane, one after the other, two workgroups per
 // CU.  A strip and its halo are loaded four keys per lane, two strips ahead, into registers; split and written to one of two LDS
@@ -53,21 +59,6 @@ inline int64_t p_count(int64_t H, int64_t W, int tri)
     return n;
 }
 
-// What a set of values holds, from the largest magnitude of their first parts: bits of a strip's state word
-enum : unsigned { P_HUGE = 1, P_USUAL = 2, P_NONZERO = 4 };
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void raise(uint32_t &top, uint32_t part)
-{
-    top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top), __builtin_bit_cast(u16x2, part & 0x7fff7fffu)));
-}
-__device__ __forceinline__ unsigned state_of(uint32_t tops)   // of a wavefront's values
-{
-    const unsigned top = max(tops & 0xffffu, tops >> 16);
-    return (__builtin_amdgcn_ballot_w64(top >= 0x7f80u) ? P_HUGE : 0u) | (__builtin_amdgcn_ballot_w64(top >= (27u << 7)) ? P_USUAL : 0u) |
-           (__builtin_amdgcn_ballot_w64(top != 0u) ? P_NONZERO : 0u);
-}
-__device__ __forceinline__ bool tiny(unsigned state) { return (state & (P_USUAL | P_NONZERO)) == P_NONZERO; }
-
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
 template <typename T, int WP, int R, int S, bool BWD>
@@ -82,8 +73,8 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
     constexpr int XP = parts_of<T>();                  // parts of a value (WP: of a tap)
     __shared__ __align__(16) uint16_t xs[2][XP * PLANE];
     static_assert(WP * R * (NE + 1) * 8 + WP * R * (S + 16) <= 2 * XP * PLANE, "the table of windows borrows the strips' LDS");
-    __shared__ unsigned state[4];                      // of the strips staged, one in three in turns; [3]: of the kernel
-    constexpr float UP = 1.2676506002282294e30f, DOWN = 1.0f / UP;   // 2^100
+    constexpr float UP_X = XP == 3 ? SPLIT_UP : 1.0f, UP_W = WP == 3 ? SPLIT_UP : 1.0f, DOWN = 1.0f / (UP_X * UP_W);   // (see above)
+    const float by = use_scale ? in_scale * UP_X : UP_X;   // fp32 data: factor and scale in one
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
     // (planes dealt to the XCDs where they divide evenly: a plane's strips share their halo rows in one L2)
@@ -128,7 +119,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
         __builtin_memcpy(&raw[it], from + (unsigned)((hc - base) * W + kc) * (unsigned)sizeof(T), sizeof(raw[it]));
     };
     // vector `it` of a strip: masked, scaled, split, to LDS
-    auto stage = [&](strip t, bool plain, int it, uint16_t *to, float by, uint32_t &top) __attribute__((always_inline)) {
+    auto stage = [&](strip t, bool plain, int it, uint16_t *to) __attribute__((always_inline)) {
         const int r = lr + it * RPI;
         float v[4];
 #pragma unroll
@@ -138,17 +129,18 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
             const int k = t.q0 - P_HL + lk, h = top_row(t) + r;
             masked_quad<T>(raw[it], k, W, (h < 0 || h >= H) ? -1 : (causal && h < W - 1 ? h : W - 1), v);
         }
-        if (use_scale || by != 1.0f) {
+        if constexpr (XP == 3) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] *= by;
+        } else if (use_scale) {
             asm volatile("" : : : "memory");
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = (use_scale ? round_to<T>(v[u] * in_scale) : v[u]) * by;
+            for (int u = 0; u < 4; ++u) v[u] = round_to<T>(v[u] * in_scale);
         }
         uint32_t a[XP], b[XP];
         split2<XP>(v[0], v[1], a);
         split2<XP>(v[2], v[3], b);
         if (lr < RPI && ((it + 1) * RPI <= ROWS || r < ROWS)) {
-            raise(top, a[0]);
-            raise(top, b[0]);
 #pragma unroll
             for (int s = 0; s < XP; ++s) *reinterpret_cast<uint2 *>(to + s * PLANE + r * P_LD + lk) = make_uint2(a[s], b[s]);
         }
@@ -162,31 +154,20 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
 
     // ---- the kernel's fragments: lane (ln, kg), slot t holds tap 8*kg + t - SHIFT - ln ----
     frag8<bf16_t> tz[WP][R];
-    float unscale = 1.0f;
-    unsigned w_state;
     {
         constexpr int NT = (R * (S + 16) + 255) / 256;
         uint16_t *const table = xs[0], *const taps = table + WP * R * (NE + 1) * 8;   // [part][row][8 zeros, S taps, 8 zeros]
-        if (tid < 4) state[tid] = 0;
         float v[NT];
-        uint32_t top = 0;
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const int e = n * 256 + tid, i = e / (S + 16), j = e % (S + 16) - 8;
             v[n] = i < R && j >= 0 && j < S ? load_any(w, w_dtype, (int64_t)c * R * S + (BWD ? R * S - 1 - (i * S + j) : i * S + j)) : 0.0f;
-            raise(top, pack2<bf16_t>(v[n], 0.0f));
         }
-        __syncthreads();
-        const unsigned mine = state_of(top);
-        if (lane == 0) atomicOr(&state[3], mine);
-        __syncthreads();
-        w_state = state[3];
-        if (tiny(w_state)) unscale = DOWN;
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const int e = n * 256 + tid;
             uint32_t part[WP];
-            split2<WP>(tiny(w_state) ? v[n] * UP : v[n], 0.0f, part);
+            split2<WP>(v[n] * UP_W, 0.0f, part);
             if (e < R * (S + 16)) {
 #pragma unroll
                 for (int s = 0; s < WP; ++s) taps[s * R * (S + 16) + e] = (uint16_t)part[s];
@@ -211,11 +192,8 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
     }
     if (first < total) {
         const bool plain = inside(t);
-        uint32_t top = 0;
 #pragma unroll
-        for (int it = 0; it < IT; ++it) stage(t, plain, it, xs[0], 1.0f, top);
-        const unsigned mine = state_of(top);
-        if (lane == 0) atomicOr(&state[0], mine);
+        for (int it = 0; it < IT; ++it) stage(t, plain, it, xs[0]);
         if (first + per_plane < total) {
             next = next_strip();
 #pragma unroll
@@ -224,28 +202,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
     }
     __syncthreads();
 
-    for (int id = first, n = 0, n3 = 0; id < total; id += per_plane, n ^= 1) {
-        const unsigned now = state[n3];
-        const int n3_next = n3 == 2 ? 0 : n3 + 1;
-        if (tid == 0) state[n3_next == 2 ? 0 : n3_next + 1] = 0;   // (the next but one: nobody reads or writes it before the barrier below)
-        float down = unscale;
-        if (tiny(now) || (now & P_HUGE)) {
-            asm volatile("" : : : "memory");
-            if (!(now & P_HUGE)) {     // all of it so small that parts underflow: staged once more, 2^100 times as large
-                quad4<T> keep[IT];
-#pragma unroll
-                for (int it = 0; it < IT; ++it) keep[it] = raw[it];
-                uint32_t top = 0;
-#pragma unroll
-                for (int it = 0; it < IT; ++it) {
-                    fetch(t, it);
-                    stage(t, false, it, xs[n], UP, top);
-                    raw[it] = keep[it];
-                }
-                __syncthreads();
-                down *= DOWN;
-            }
-        }
+    for (int id = first, n = 0; id < total; id += per_plane, n ^= 1) {
         const bool more = id + per_plane < total, more2 = id + 2 * per_plane < total;
         const strip after = more2 ? next_strip() : t;   // (asked for either way: behind a branch around the loads their waits would be waits for all)
         const bool plain = inside(next);
@@ -263,8 +220,8 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
         const int pl = (wave & 1) * 16 + ln, ql = (wave >> 1) * 64 + kg * 4;
         char *const ybase = reinterpret_cast<char *>(yp + (int64_t)t.p0 * W + t.q0);
         const unsigned yoff = (unsigned)(pl * W + ql) * (unsigned)sizeof(T);
-        const bool whole = t.p0 + P_TM <= H && t.q0 + P_TN <= W && (!causal || t.q0 + P_TN - 1 <= t.p0) && !((now | w_state) & P_HUGE);
-        uint32_t top = 0;
+        const bool whole = t.p0 + P_TM <= H && t.q0 + P_TN <= W && (!causal || t.q0 + P_TN - 1 <= t.p0);
+        float bad = 0.0f;   // not 0: a result that is not finite
         read(0);
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
@@ -288,7 +245,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
                 constexpr int LEAD = 8 - IT;     // (not ahead of the last strip's stores: loads and stores complete on one counter)
                 const int it = b * 2 + half - LEAD;
                 if (it >= 0) {
-                    if (more) stage(next, plain, it, xs[n ^ 1], 1.0f, top);
+                    if (more) stage(next, plain, it, xs[n ^ 1]);
                     fetch(after, it);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -296,11 +253,9 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
             // (stores of 16 rows x 64 bytes; the second half of a 128-byte line follows with the next block)
             float v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = big[u] + (small0[u] + small1[u]);
-            if (down != 1.0f) {
-                asm volatile("" : : : "memory");
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] *= down;
+            for (int u = 0; u < 4; ++u) {
+                v[u] = (big[u] + (small0[u] + small1[u])) * DOWN;
+                bad = fmaf(v[u], 0.0f, bad);
             }
             if (whole) {
                 asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));   // (one store, not one shared in part with the other branch)
@@ -310,19 +265,22 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
                 __builtin_memcpy(ybase + yoff + b * 16 * (int)sizeof(T), &o, sizeof(o));
             } else {
                 const int p = t.p0 + pl, q = t.q0 + ql + b * 16;
-                if (!((now | w_state) & P_HUGE) && p < H && q < W && !(causal == 2 && q > p)) {
+                if (p < H && q < W && !(causal == 2 && q > p)) {
 #pragma unroll
                     for (int u = 0; u < 4; ++u) v[u] = causal && q + u > p ? 0.0f : v[u];
                     store_quad<T>(yp + (int64_t)p * W, q, W, v);
                 }
             }
         }
-        if ((now | w_state) & P_HUGE) {   // values that do not split: multiply-adds, tap by tap
-            for (int e = opaque(tid); e < P_TM * P_TN; e += 256) {
-                const int pe = t.p0 + e / P_TN, q = t.q0 + e % P_TN;
-                if (pe >= H || q >= W || (causal == 2 && q > pe)) continue;
+        if (__builtin_amdgcn_ballot_w64(bad != 0.0f) != 0) {   // this lane's results that are not finite: multiply-adds, tap by tap
+#pragma unroll 1
+            for (int e = opaque(0); e < 16; ++e) {
+                const int pe = t.p0 + pl, q = t.q0 + ql + (e >> 2) * 16 + (e & 3);
+                if (pe >= H || q >= W || (causal && q > pe)) continue;
+                T *const at = yp + (int64_t)pe * W + q;
+                if (__builtin_isfinite(to_float(*at))) continue;
                 float sum = 0.0f;
-                for (int i = 0; i < R && !(causal && q > pe); ++i) {
+                for (int i = 0; i < R; ++i) {
                     const int h = BWD ? pe + i : pe - (R - 1) + i;
                     if (h < 0 || h >= H) continue;
                     for (int j = 0; j < S; ++j) {
@@ -333,16 +291,11 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
                         sum = fmaf(load_any(w, w_dtype, (int64_t)c * R * S + (BWD ? R * S - 1 - (i * S + j) : i * S + j)), v, sum);
                     }
                 }
-                yp[(int64_t)pe * W + q] = from_float<T>(sum);
+                *at = from_float<T>(sum);
             }
-        }
-        if (more) {
-            const unsigned mine = state_of(top);
-            if (lane == 0) atomicOr(&state[n3_next], mine);
         }
         t = next;
         next = after;
-        n3 = n3_next;
         __syncthreads();
     }
     if (causal == 1) {     // the strips wholly above the diagonal

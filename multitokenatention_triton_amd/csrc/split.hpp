@@ -1,7 +1,8 @@
 // fp32 values as sums of bf16 parts, for products on the bf16 matrix cores that keep the 32 bits.
 //
 // x = x0 + x1 + x2, each part the bf16 value nearest to the remainder of those before it: 8 + 8 + 8 bits, exactly x while the parts
-// neither overflow (|x| of 3.39e38 and more rounds to infinity) nor underflow (below about 2^-109).  Of the nine products of
+// neither overflow (|x| of 3.39e38 and more rounds to infinity) nor underflow (below about 2^-109; 2^24 x has normal parts
+// whatever x is, SPLIT_UP).  Of the nine products of
 // parts of a product x w the six x_i w_j with i + j <= 2 are formed; each is exact in fp32, and what is left out is below
 // 2^-26 |x w|, a quarter of the last place that one fp32 multiply-add rounds away.
 #pragma once
@@ -10,6 +11,8 @@
 #include "mfma.hpp"
 
 namespace mta {
+
+constexpr float SPLIT_UP = 16777216.0f;   // 2^24: fp32's last bit, 2^-149, becomes a normal number
 
 // two values' parts, packed.  (The packed dot product with (-1, 0) or (0, -1) takes one of the two values off a remainder without
 // unpacking it: one instruction in place of two.  Constants the compiler cannot see: it would fold (-1, 0) into the inline constant

@@ -1047,6 +1047,26 @@ def test_conv_11x15_split_values(pkg, bwd):
         torch.testing.assert_close(run(x * sx, k * sk) * (1 / (sx * sk)), plain, rtol=2.0 ** -20, atol=2.0 ** -20)
 
 
+@pytest.mark.parametrize("bwd", [False, True])
+def test_conv_11x15_split_range(pkg, bwd):
+    """The 32 bits are kept at the ends of fp32's range, whatever lies beside a value: tiny taps under huge data and the reverse (every sum finite,
+    of values that a common factor of 2^100 overflows), values and taps down to the denormals beside ordinary ones, products at the
+    smallest normal number, sums of 2^80 and more.  Bound: 165 products and sums of 32 bits, and the last place of a denormal for each."""
+    g = torch.Generator(device="cuda").manual_seed(75)
+    x, k = torch.randn(1, 2, 200, 200, generator=g, device="cuda"), 0.1 * torch.randn(2, 11, 15, generator=g, device="cuda")
+    far, top, one = x.clone(), k.clone(), torch.zeros_like(x)
+    far[..., 60:] *= 2.0 ** -126
+    far[..., 110:] *= 2.0 ** -9
+    top[:, :5] *= 2.0 ** -115
+    one[..., 100, 80] = 1.7
+    for a, w in ((torch.full_like(x, 2.0 ** 122), torch.full_like(k, 1.9 * 2.0 ** -101)), (torch.full_like(x, 1.9 * 2.0 ** -101), torch.full_like(k, 2.0 ** 122)),
+                 (far, k), (one, top), (x * 2.0 ** -60, k * 2.0 ** -60), (x * 2.0 ** -64, k * 2.0 ** -64), (x * 2.0 ** 85, k), (x, k * 2.0 ** 100),
+                 (x * 2.0 ** 110, k * 2.0 ** -110)):
+        got = pkg.ops.conv2d_bwd_input(a, w, True) if bwd else pkg.ops.conv2d_causal(a, w, True)
+        want, size = _conv64(a, w, True, bwd)
+        assert ((got.double() - want).abs() <= 167 * (2.0 ** -24 * size + 2.0 ** -149)).all()
+
+
 @pytest.mark.parametrize("heads,s,d", [(300, 4, 64), (300, 132, 64), (37, 388, 64), (9, 1000, 64), (16, 1024, 64), (130, 60, 128), (130, 64, 128), (23, 388, 128),
                                        (5, 1036, 128)])
 def test_fp32_scores_split(pkg, heads, s, d):
