@@ -1,10 +1,10 @@
 // fp32 values as sums of bf16 parts, for products on the bf16 matrix cores that keep the 32 bits.
 //
 // x = x0 + x1 + x2, each part the bf16 value nearest to the remainder of those before it: 8 + 8 + 8 bits, exactly x while the parts
-// neither overflow (|x| of 3.39e38 and more rounds to infinity) nor underflow (below about 2^-109; 2^24 x has normal parts
-// whatever x is, SPLIT_UP).  Of the nine products of
-// parts of a product x w the six x_i w_j with i + j <= 2 are formed; each is exact in fp32, and what is left out is below
-// 2^-26 |x w|, a quarter of the last place that one fp32 multiply-add rounds away.
+// neither overflow (|x| of 3.39e38 and more rounds to infinity) nor underflow (below about 2^-109).  So the values are split 2^24
+// times as large (SPLIT_UP) and the results taken back: every |x| below 2^104 has parts that are normal numbers then, and only sums
+// of 2^80 and more overflow.  Of the nine products of parts of a product x w the six x_i w_j with i + j <= 2 are formed; each is exact
+// in fp32, and what is left out is below 2^-26 |x w|, a quarter of the last place that one fp32 multiply-add rounds away.
 #pragma once
 
 #include "common.hpp"
@@ -49,20 +49,15 @@ __device__ __forceinline__ void split8(f32x4 lo, f32x4 hi, frag8<bf16_t> (&part)
 
 __device__ __forceinline__ void mma4(f32x4 &c, float a, float b) { c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// Whether a wavefront's sums may not be what fp32 products give: one of them is not finite (an operand was not, or a part of one
-// overflowed: every product with it is infinite or NaN; or the sum itself), or all are so small that parts may have underflowed.
-template <int N> __device__ __forceinline__ bool unsafe(const f32x4 *acc)
+// Whether one of a wavefront's sums is not finite: an operand was not, or a part of one overflowed (every product with it is infinite or
+// NaN), or the sum itself did.
+template <int N> __device__ __forceinline__ bool not_finite(const f32x4 *acc)
 {
-    float bad = 0.0f, top = 0.0f;
+    float bad = 0.0f;
 #pragma unroll
     for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; v += 2) {
-            bad = fmaf(acc[i][v], 0.0f, bad);
-            bad = fmaf(acc[i][v + 1], 0.0f, bad);
-            top = fmaxf(fmaxf(top, fabsf(acc[i][v])), fabsf(acc[i][v + 1]));
-        }
-    return __builtin_amdgcn_ballot_w64(bad != 0.0f) != 0 ||
-           (__builtin_amdgcn_ballot_w64(top >= 0x1p-80f) == 0 && __builtin_amdgcn_ballot_w64(top != 0.0f) != 0);
+        for (int v = 0; v < 4; ++v) bad = fmaf(acc[i][v], 0.0f, bad);
+    return __builtin_amdgcn_ballot_w64(bad != 0.0f) != 0;
 }
 }  // namespace mta

@@ -12,7 +12,10 @@
 // against 64 bits (2-norm): D64 1.4e-7 -> 0.5e-7, D128 2.0e-7 -> 0.65e-7.
 // Runs of 1 | 2 | 4 steps: D64 B1 H16 S1024 (1152 steps) 18.7 | 17.6 | 20.4, B1 H32 S1024 (2304) 34.4 | 31.9 | 28.8, B1 H16 S2048 (4352) 56.3 | 46.3
 // | 42.1; D128, twice as many, B2 H16 S512 17.5 | 17.3 | 18.2, B1 H16 S2048 88.0 | 70.8 | 63.8.
-// A wavefront whose sums are not finite, or all so small that parts may have underflowed, forms them again with fp32 products.
+// Operands are split 2^24 times as large (split.hpp); a wavefront with a sum that is not finite then forms its step again with fp32
+// products.  (Unscaled, with a look at the sums, which cannot tell small operands against large ones: 1 to 4 % faster, and up to 12000
+// times the error of 32-bit sums.  us with nothing in the caches, that -> this: D64 B1 H16 S512 9.8 -> 9.8, S1024 19.3 -> 20.2, S2048 54.0 -> 53.8;
+// D128 11.6 -> 12.1, 27.1 -> 27.4, 68.3 -> 69.1.)
 // (P V and P^T X in this form, with a V block per 64 rows: as fast as on the fp32 instructions - B1 H32 S1024 D64 26.1 | 28.3, B1 H32 S2048 D128 155 |
 // 138 us - since V passes that path as often as P does.)
 #include "split.hpp"
@@ -59,8 +62,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void lower_scores_split(const
     auto stage = [&](int i, uint16_t *to) __attribute__((always_inline)) {
         const int slot = i * 256 + tid, key = slot / (D / 4), q = slot % (D / 4);
         uint32_t a[3], b[3];
-        split2<3>(raw[i][0], raw[i][1], a);
-        split2<3>(raw[i][2], raw[i][3], b);
+        split2<3>(raw[i][0] * SPLIT_UP, raw[i][1] * SPLIT_UP, a);
+        split2<3>(raw[i][2] * SPLIT_UP, raw[i][3] * SPLIT_UP, b);
         uint16_t *at = to + key * D + ((q >> 1) ^ (key & (CPR - 1))) * 8 + (q & 1) * 4;
 #pragma unroll
         for (int s = 0; s < 3; ++s) *reinterpret_cast<uint2 *>(at + s * PLANE) = make_uint2(a[s], b[s]);
@@ -75,7 +78,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void lower_scores_split(const
         for (int ks = 0; ks < KS; ++ks) {
             const f32x4 lo = *reinterpret_cast<const f32x4 *>(Ap + (int64_t)p * D + ks * 32 + kg * 8);
             const f32x4 hi = *reinterpret_cast<const f32x4 *>(Ap + (int64_t)p * D + ks * 32 + kg * 8 + 4);
-            split8(lo, hi, a[rb][ks]);
+            split8(lo * SPLIT_UP, hi * SPLIT_UP, a[rb][ks]);
         }
     }
 #pragma unroll
@@ -142,7 +145,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void lower_scores_split(const
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int rb = 0; rb < 2; ++rb) acc[cb][rb] = big[rb] + small[rb];
+            for (int rb = 0; rb < 2; ++rb) acc[cb][rb] = (big[rb] + small[rb]) * (1.0f / SPLIT_UP / SPLIT_UP);
             // the next step's keys to the other buffer, those of the one behind it asked for
 #pragma unroll
             for (int i = cb * QUADS / NCB; i < (cb + 1) * QUADS / NCB; ++i) {
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void lower_scores_split(const
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        again = live && unsafe<NCB * 2>(&acc[0][0]);
+        again = live && not_finite<NCB * 2>(&acc[0][0]);
         if (again) {   // fp32 products, from memory: contraction d = 16s + 4kg + t, four steps' operand in a lane's vector of its row
 #pragma unroll 1
             for (int e = 0; e < NCB * 2; ++e) {

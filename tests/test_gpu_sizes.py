@@ -1103,6 +1103,26 @@ def test_fp32_scores_split(pkg, heads, s, d):
         assert ((run(a * sx, b * sy).double() / (sx * sy) - want).abs() <= d * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("heads,s,d", [(64, 512, 64), (64, 260, 128)])
+def test_fp32_scores_split_range(pkg, heads, s, d):
+    """The 32 bits are kept at the ends of fp32's range: tiny operands against huge ones, tiny rows and keys down to the denormals beside ordinary
+    ones, products at the smallest normal number, sums of 2^80 and more.  Bound: d products and sums of 32 bits, and the last place of a
+    denormal for each."""
+    lib, st = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(76)
+    a, b = (torch.randn(1, heads, s, d, generator=g, device="cuda") for _ in range(2))
+    rows, keys = a.clone(), b.clone()
+    rows[:, :, ::2] *= 2.0 ** -118
+    rows[:, :, ::6] *= 2.0 ** -16
+    keys[:, :, 1::3] *= 2.0 ** -125
+    for x, y in ((a * 2.0 ** -120, b * 2.0 ** 110), (a * 2.0 ** 120, b * 2.0 ** -126), (rows, b), (a, keys), (rows, keys), (a * 2.0 ** -60, b * 2.0 ** -60),
+                 (a * 2.0 ** -64, b * 2.0 ** -64), (a * 2.0 ** 45, b * 2.0 ** 45), (a * 2.0 ** 110, b)):
+        out = torch.empty(1, heads, s, s, device="cuda")
+        assert lib.mta_lower_scores_f32(x.data_ptr(), y.data_ptr(), out.data_ptr(), 1, heads, s, d, st) == 0
+        want, size = ((u.double() @ v.double().transpose(2, 3)).tril() for u, v in ((x, y), (x.abs(), y.abs())))
+        assert ((out.tril().double() - want).abs() <= d * (2.0 ** -24 * size + 2.0 ** -149)).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("group", [1, 2, 4, 8])
 def test_softmax_wavefronts_per_row(pkg, group, dtype):
