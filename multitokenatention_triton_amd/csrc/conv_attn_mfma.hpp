@@ -709,15 +709,17 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                     const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
                     // exp(scale*(x - m)) = exp2(x*scale*log2(e) - m*scale*log2(e)): one multiply-add and one v_exp per element
                     mneg[rb] = -m_use * scale2;
-                    const float alpha = __builtin_amdgcn_exp2f(fmaf(m_i[rb], scale2, mneg[rb]));
-                    m_i[rb] = m_new;
-                    l_i[rb] *= alpha;
-                    // (once the running maxima have settled, alpha is 1 in every lane for most key blocks: the 4*DB
-                    // multiplications are skipped for the wavefront then)
-                    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+                    // Where no row's maximum has moved (most key blocks, once the maxima have settled) the 4*DB multiplications are skipped.
+                    // The factor of a row whose maximum stays is 1 by that, not by its exponent: mneg is rounded, and the sums would drift
+                    // by that rounding at every key block (0.5 % of a row of 8192 keys at logits of 772) and be multiplied at nearly every one.
+                    // us: 6x11 B1 H32 S8192 D128 1007 -> 989, 5x5 B2 H32 S4096 D64 354 -> 345, 3x3 B1 H32 S4096 D128 244 -> 240.
+                    if (__builtin_amdgcn_ballot_w64(m_new != m_i[rb]) != 0) {
+                        const float alpha = m_new != m_i[rb] ? __builtin_amdgcn_exp2f(fmaf(m_i[rb], scale2, mneg[rb])) : 1.0f;
+                        l_i[rb] *= alpha;
 #pragma unroll
                         for (int db = 0; db < DB; ++db) oacc[rb][db] *= alpha;
                     }
+                    m_i[rb] = m_new;
                 }
             }
         };

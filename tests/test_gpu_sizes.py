@@ -95,6 +95,24 @@ def test_conv_attention_factor(pkg, dtype, d, r, sk, factor, causal):
         torch.testing.assert_close(lse.cpu(), torch.logsumexp(scores, -1), rtol=2.0 ** -7, atol=2e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,d", [(1, 64), (20, 64), (1, 128), (20, 128)])
+def test_conv_attention_sums_do_not_drift(pkg, h, d, dtype):
+    """128 key blocks of equal logits, 772, whose product with log2(e) is rounded by a unit of 6e-5: a row's sum stays the number of its
+    keys, and its first and its last block weigh the same.  Bound: the statistic's own rounding, 2^-14 at 772, and one of the logarithm.
+    Eight wavefronts of 16 rows (one head) and four of 32."""
+    s = 8192
+    q, k, v = (torch.zeros(1, h, s, d, dtype=dtype, device="cuda") for _ in range(3))
+    q[..., 0], k[..., 0], k[..., 1], q[..., 1] = 27.75, 27.75, 1.0, 1.9375   # (27.75^2 + 1.9375 = 772)
+    v[:, :, :64, 0] = v[:, :, -64:, 1] = 64.0
+    w = torch.zeros(h, 3, 3, dtype=dtype, device="cuda")
+    w[:, -1, 1] = 1.0
+    o, lse = pkg.ops.conv_attn_fwd(q, k, v, w, True, 1.0, return_lse=True)
+    want = 772.0 + torch.log(torch.arange(1, s + 1, dtype=torch.float64, device="cuda"))
+    assert (lse.double() - want).abs().max().item() <= 2.0 ** -13
+    assert torch.equal(o[:, :, -1, 0], o[:, :, -1, 1])
+
+
 @pytest.mark.parametrize("dtype,r,sk", [(torch.bfloat16, 3, 5), (torch.float16, 7, 9)])
 def test_qk_conv_kernel_sizes(pkg, dtype, r, sk):
     """The scores stage at the same sizes; bound as in test_qk_conv_parity: two 16-bit roundings of scores of magnitude
