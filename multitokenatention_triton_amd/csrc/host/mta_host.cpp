@@ -854,6 +854,9 @@ OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_,
     if (q_.scalar_type() != at::kFloat || !causal || q_.numel() == 0) return std::nullopt;
     const int64_t b = q_.size(0), h = q_.size(1), s_real = q_.size(2), d = q_.size(3), s = (s_real + 7) / 8 * 8, plane = s * s * 4;
     const int64_t r = w.size(1), sk = w.size(2);
+    for (const Tensor *x : {&q_, &k_, &v_})   // (what the fused kernel refuses stays refused)
+        if (reinterpret_cast<uintptr_t>(ptr(*x)) % 16) return std::nullopt;
+    if (b * h > 65535) return std::nullopt;
     if (plane > SCRATCH || !lower_products_supported(at::kFloat, {b, h, s, d}, true) || !conv_attn_in_stages(b * h, s_real, d, r, sk)) return std::nullopt;
     Tensor q = q_, k = k_, v = v_;
     if (s != s_real) {   // (the products take rows that are whole vectors)
@@ -862,8 +865,6 @@ OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_,
         k = rows.add(k_, false, 1.0);
         v = rows.add(v_, false, 1.0);
         rows.run();
-    } else {
-        v = on_gpu_vectors(v, "V");
     }
     Tensor o = at::empty(q.sizes(), q.options());
     // equal parts: of the batch, or of one batch entry's heads

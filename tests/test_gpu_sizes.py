@@ -76,6 +76,23 @@ def test_conv_attention_fp32_stages(pkg, b, h, s, d, r, sk, factor):
     torch.testing.assert_close(got, want, **tol(torch.float32))
 
 
+@pytest.mark.parametrize("s", [512, 513])
+def test_conv_attention_fp32_refuses(pkg, s):
+    """fp32 conv-attention refuses the same calls where it runs in stages: operands that do not lie at whole 16-byte vectors, more than 65535
+    planes."""
+    module = pkg.TritonConvAttention(4, (6, 11), causal=True).cuda()
+    ok = torch.zeros(1, 4, s, 64, device="cuda")
+    off = torch.zeros(ok.numel() + 1, device="cuda")[1:].view_as(ok)
+    many = torch.zeros(1, 65536, s, 64, device="cuda")
+    with torch.no_grad():
+        module(ok, ok, ok, True, None)
+        for q, k, v in ((off, ok, ok), (ok, off, ok), (ok, ok, off)):
+            with pytest.raises(ValueError):
+                module(q, k, v, True, None)
+        with pytest.raises(ValueError):
+            pkg.TritonConvAttention(65536, (6, 11), causal=True).cuda()(many, many, many, True, None)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("factor", [-0.08, 0.0, 0.08])
 @pytest.mark.parametrize("dtype,d,r,sk", [(torch.bfloat16, 128, 6, 11), (torch.float16, 64, 3, 3), (torch.float16, 128, 11, 15)])
