@@ -3,8 +3,8 @@
 Mirrors TritonConvAttention (conv_attention_triton.py:476-502) and TritonAttention
 (:359-452) of the reference.  O = softmax(mask(conv(mask0(Q K^T))) * scale) V is computed
 by ``mta_conv_attn_fwd`` with score tiles kept in LDS; causal fp32 forwards without
-gradients run as scores, conv, softmax and P V where that is faster, over at most 256 MB of
-scores at a time.  The reference also returns the (B,H,S,S) QK scratch it fills in global
+gradients run as scores, conv, softmax and P V where that is faster, by way of at most
+512 MB of scores in scratch tensors.  The reference also returns the (B,H,S,S) QK scratch it fills in global
 memory; this build keeps none and returns ``None`` in its place (the reference's own harness accepts that,
 compare_conv_attention2.py:171-187).
 """

@@ -846,8 +846,10 @@ Tensor headmix_apply(const Tensor &x, const Tensor &w, bool causal, double fill,
     return HeadMix::apply(x, w, causal, fill, group, fill_upper, grad_fill_upper);
 }
 
-// Conv-attention in fp32 as scores, conv, softmax and P V, one kernel each, over as many planes at a time as a scratch of 256 MB holds
-// (two or three of them; a plane of S = 8192 fills one).  Nothing where the fused kernel is taken.
+// Conv-attention in fp32 as scores, conv, softmax and P V, one kernel each, over as many planes at a time as 256 MB hold (one of S = 8192).
+// us, parts of 128 MB | 256: 6x11 B1 H32 S4096 D128 2755 | 2234, B8 H32 S1024 D128 1391 | 1237, 7x9 B3 H4 S2300 D64 310 | 246.  Scratch: 512 MB
+// at most, for scores, conv and softmax, or, where three do not fit, the softmax where the scores were (two | three: 3x3 B1 H4 S1024 D64
+// 39.4 | 37.1, B1 H8 51.9 | 49.3, 7x7 B1 H8 S768 D128 54.9 | 53.0; from 100 MB a tensor on alike).  Nothing where the fused kernel is taken.
 OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &w, bool causal, double scale)
 {
     constexpr int64_t SCRATCH = 256 << 20;
@@ -870,16 +872,21 @@ OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_,
     // equal parts: of the batch, or of one batch entry's heads
     auto part = [](int64_t count, int64_t most) { const int64_t parts = (count + most - 1) / most; return (count + parts - 1) / parts; };
     const int64_t nb = h * plane <= SCRATCH ? part(b, SCRATCH / (h * plane)) : 1, nh = h * plane <= SCRATCH ? h : part(h, SCRATCH / plane);
+    const Tensor raw = at::empty({nb, nh, s, s}, q.options()), conv = at::empty({nb, nh, s, s}, q.options()),
+                 probs = 3 * nb * nh * plane <= 2 * SCRATCH ? at::empty({nb, nh, s, s}, q.options()) : raw;
+    void *const st = stream_of(q), *const x = out_ptr(raw), *const y = out_ptr(conv), *const p = out_ptr(probs);
+    const auto *qp = q.const_data_ptr<float>(), *kp = k.const_data_ptr<float>(), *vp = v.const_data_ptr<float>();
+    const auto *wp = static_cast<const char *>(ptr(w));
     for (int64_t b0 = 0; b0 < b; b0 += nb)
-        for (int64_t h0 = 0; h0 < h; h0 += nh) {
-            const int64_t bs = std::min(nb, b - b0), hs = std::min(nh, h - h0);
-            auto of = [&](const Tensor &x) { return x.narrow(0, b0, bs).narrow(1, h0, hs); };   // (contiguous: all heads, or one batch entry)
-            const OptTensor raw = lower_scores(of(q), of(k), OptTensor());
-            TORCH_CHECK(raw, "no kernel for the lower-triangle products");
-            Tensor p = conv2d(*raw, w.narrow(0, h0, hs), true, scale, false);
-            p = headmix_softmax(p, OptTensor(), OptTensor(), true, 0, false, OptTensor(), OptTensor());
-            const Tensor vs = of(v), os = of(o);
-            check(mta_causal_pv_f32(ptr(p), ptr(vs), out_ptr(os), bs, hs, s, d, 1.0f, stream_of(p)), "mta_causal_pv_f32");
+        for (int64_t h0 = 0; h0 < h; h0 += nh) {   // (a part lies in one piece: all heads, or one batch entry)
+            const int64_t bs = std::min(nb, b - b0), hs = std::min(nh, h - h0), at = (b0 * h + h0) * s * d;
+            check(mta_lower_scores_f32(qp + at, kp + at, x, bs, hs, s, d, st), "mta_lower_scores_f32");
+            check(mta_conv2d_scaled_fwd(x, wp + h0 * r * sk * w.element_size(), y, bs, hs, s, s, (int)r, (int)sk, causal_mode(true, false), (float)scale,
+                                        MTA_F32, code(w, "W"), st),
+                  "mta_conv2d_fwd");
+            check(mta_headmix_softmax_band_fwd(y, nullptr, nullptr, nullptr, nullptr, p, bs, hs, s, s, 0, true, false, MTA_F32, MTA_F32, st),
+                  "mta_headmix_softmax_band_fwd");
+            check(mta_causal_pv_f32(p, vp + at, o.mutable_data_ptr<float>() + at, bs, hs, s, d, 1.0f, st), "mta_causal_pv_f32");
         }
     return s == s_real ? o : o.narrow(2, 0, s_real).contiguous();
 }
@@ -895,7 +902,10 @@ Tensor conv_attn(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Ten
     TORCH_CHECK(w.dim() == 3 && w.size(0) == q.size(1), "CHANNEL_DIM == NUM_HEADS");
     const c10::OptionalDeviceGuard guard(q.device());
     const double scale = softmax_scale ? *softmax_scale : 1.0 / std::sqrt((double)q.size(3));
-    if (OptTensor staged = conv_attn_stages(q, k, v, w, causal, scale)) return *staged;
+    try {
+        if (OptTensor staged = conv_attn_stages(q, k, v, w, causal, scale)) return *staged;
+    } catch (const c10::OutOfMemoryError &) {   // (the fused kernel needs none of it)
+    }
     Tensor o = at::empty(q.sizes(), q.options());
     check(mta_conv_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(w), out_ptr(o), q.size(0), q.size(1), q.size(2), q.size(3), (int)w.size(1), (int)w.size(2),
                             causal, (float)scale, code(q, "Q"), code(w, "W"), stream_of(q)),

@@ -76,6 +76,31 @@ def test_conv_attention_fp32_stages(pkg, b, h, s, d, r, sk, factor):
     torch.testing.assert_close(got, want, **tol(torch.float32))
 
 
+@pytest.mark.parametrize("b,h,s", [(4, 16, 1024), (5, 4, 1500), (1, 4, 5792), (1, 2, 8192)])
+def test_conv_attention_fp32_scratch(pkg, b, h, s):
+    """What fp32 conv-attention in stages allocates beside its result: up to 512 MB in two or three tensors of scores (and padded operands where
+    the length is ragged); and where that cannot be had, the fused kernel's result."""
+    module = pkg.TritonConvAttention(h, (6, 11), causal=True).cuda()
+    q, k, v = (x.cuda() for x in O.seeded_qkv(b, h, s, 64, torch.float32, seed=48))
+    with torch.no_grad():
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        got = module(q, k, v, True, None)[0]
+        beside = torch.cuda.max_memory_allocated() - before - (1 if s % 8 == 0 else 5) * q.numel() * 4
+        assert s * s * 4 < beside <= 516 << 20
+        del got
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        try:
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 6 * q.numel() * 4 + (24 << 20)) / total)
+            got = module(q, k, v, True, None)[0]
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+    want, _ = pkg.ops.conv_attn_fwd(q, k, v, module.weight.detach(), True, None, return_lse=True)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("s", [512, 513])
 def test_conv_attention_fp32_refuses(pkg, s):
     """fp32 conv-attention refuses the same calls where it runs in stages: operands that do not lie at whole 16-byte vectors, more than 65535
