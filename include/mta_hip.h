@@ -210,6 +210,10 @@ int mta_qk_conv_fwd(const void *q, const void *k, const void *w, void *s_out, in
  * anything.  Host-side only; needs no GPU. */
 int mta_qk_conv_supported(int64_t S, int64_t D, int R, int Sk, int io_dtype, int w_dtype);
 
+/* 1 when a causal fp32 mta_conv_attn_fwd of these sizes is faster as mta_lower_scores_fwd, mta_conv2d_scaled_fwd, a softmax without
+ * weights and mta_causal_pv_f32 by way of score tensors (lengths that are no multiple of 8 padded by the caller).  Host-side only. */
+int mta_conv_attn_in_stages(int64_t B, int64_t H, int64_t S, int64_t D, int R, int Sk, int causal, int io_dtype);
+
 /* mta_qk_conv_fwd under a band mask (causal by construction): first_visible is int32, (B,S); the score of key k of
  * query row p enters the conv as 0 unless first_visible[b, p] <= k <= p - the `scores.masked_fill(mask == -inf, 0)`
  * ahead of the conv of mta_attention_triton.py:70-73 for masks of that form.  What is defined are the outputs at visible

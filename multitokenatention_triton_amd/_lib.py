@@ -39,6 +39,7 @@ SIGNATURES = {
     "mta_conv2d_headmix_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _int, _int, _int, _int, _vp]),
     "mta_qk_conv_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _f32, _int, _int, _int, _vp]),
     "mta_qk_conv_supported": (_int, [_i64, _i64, _int, _int, _int, _int]),
+    "mta_conv_attn_in_stages": (_int, [_i64] * 4 + [_int] * 4),
     "mta_causal_pv_band_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
     "mta_band_zero_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "mta_band_zero_fwd": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp]),

@@ -22,6 +22,9 @@
 // softmax / PV of a block lag the scores by the right-hand pad so that every tap is
 // already there.  One extra leading key block (mostly out-of-range keys) primes that halo.
 #include <algorithm>
+#include <cmath>
+
+#include <algorithm>
 
 #include <type_traits>
 #include <utility>
@@ -414,6 +417,25 @@ static bool scores_instance(int R, int Sk)
 {
     return (R == 3 && (Sk == 3 || Sk == 5)) || (R == 5 && (Sk == 5 || Sk == 7)) || (R == 6 && Sk == 11) ||
            (R == 7 && (Sk == 7 || Sk == 9)) || (R == 11 && Sk == 15);
+}
+
+// Whether fp32 conv-attention runs as four kernels with the scores in memory.  In the fused kernel a workgroup of 128 rows walks the keys
+// alone, conv and softmax on the vector units between two products: a chain of key blocks of 8 to 20 us, and no faster in all with two
+// workgroups per CU.  The four kernels spread over the chip at any size, but move 16 bytes of scores per position and cost four launches
+// (22 us), lengths that are no multiple of 8 two more copies.  The estimates below follow what was measured on 200 sizes; us, fused | four:
+// 3x3 D64 B1 H4 S64 14.6 | 21.7, S192 30 | 22, S1024 129 | 39, H16 S2048 360 | 220; 6x11 D128 B1 H4 S65 43 | 31, S512 143 | 30, S2048 545 | 109;
+// 7x9 D64 B4 H8 S65 28 | 31, S2048 713 | 474; 11x15 D64 B2 H12 S2048 1036 | 502; fused is left with small D = 64 grids and with many planes of
+// small kernels: 5x5 D64 B4 H32 S192 34 | 46, S777 288 | 369, S1024 401 | 472.  The error against 64 bits is smaller in four kernels throughout.
+extern "C" int mta_conv_attn_in_stages(int64_t B, int64_t H, int64_t S, int64_t D, int R, int Sk, int causal, int io_dtype)
+{
+    // (the kernel sizes that have instances of both)
+    if (io_dtype != MTA_F32 || !causal || B <= 0 || H <= 0 || B * H > 65535 || S < 64 || S > (1 << 20) || (D != 64 && D != 128) || !scores_instance(R, Sk)) return 0;
+    const double planes = (double)(B * H), s = (double)S, taps = (double)(R * Sk), positions = planes * s * s * 1e-6, blocks = (double)((S + 63) / 64);
+    const double rows = (double)(128 - (R - 1 + 7) / 8 * 8), items = planes * std::ceil(s / rows);
+    const double chain = std::max(blocks, items * (blocks + 1) / 2 * 1.25 / device_cu_count());   // key blocks one after the other on a CU
+    const double fused = D == 64 ? 6 + (7 + 0.073 * taps) * chain : 10 + (13.5 + 0.047 * taps) * chain;
+    const double four = std::max(22.0, 16 + 0.09 * planes + (D == 64 ? 3.3 : 3.9) * positions) + (S % 8 ? 9 + 6.4e-6 * planes * s * (double)D : 0);
+    return four < 0.95 * fused ? 1 : 0;
 }
 
 extern "C" int mta_qk_conv_supported(int64_t S, int64_t D, int R, int Sk, int io_dtype, int w_dtype)

@@ -858,8 +858,7 @@ OptTensor conv_attn_stages(const Tensor &q_, const Tensor &k_, const Tensor &v_,
     const int64_t r = w.size(1), sk = w.size(2);
     for (const Tensor *x : {&q_, &k_, &v_})   // (what the fused kernel refuses stays refused)
         if (reinterpret_cast<uintptr_t>(ptr(*x)) % 16) return std::nullopt;
-    if (b * h > 65535) return std::nullopt;
-    if (plane > SCRATCH || !lower_products_supported(at::kFloat, {b, h, s, d}, true) || !conv_attn_in_stages(b * h, s_real, d, r, sk)) return std::nullopt;
+    if (plane > SCRATCH || !lower_products_supported(at::kFloat, {b, h, s, d}, true) || !mta_conv_attn_in_stages(b, h, s_real, d, (int)r, (int)sk, causal, MTA_F32)) return std::nullopt;
     Tensor q = q_, k = k_, v = v_;
     if (s != s_real) {   // (the products take rows that are whole vectors)
         RowsCopy rows(s, OptTensor());

@@ -318,27 +318,6 @@ inline bool lower_products_supported(at::ScalarType t, c10::IntArrayRef x, bool 
            (t == at::kFloat && causal && (x[3] == 64 || x[3] == 128) && x[2] % 4 == 0 && x[2] <= (1 << 20));
 }
 
-// Whether fp32 conv-attention runs as four kernels with the scores in memory.  In the fused kernel a workgroup of 128 rows walks the keys
-// alone, conv and softmax on the vector units between two products: a chain of key blocks of 8 to 20 us, and no faster in all with two
-// workgroups per CU.  The four kernels spread over the chip at any size, but move 16 bytes of scores per position and cost four launches
-// (22 us), lengths that are no multiple of 8 two more copies.  The estimates below follow what was measured on 200 sizes; us, fused | four:
-// 3x3 D64 B1 H4 S64 14.6 | 21.7, S192 30 | 22, S1024 129 | 39, H16 S2048 360 | 220; 6x11 D128 B1 H4 S65 43 | 31, S512 143 | 30, S2048 545 | 109;
-// 7x9 D64 B4 H8 S65 28 | 31, S2048 713 | 474; 11x15 D64 B2 H12 S2048 1036 | 502; fused is left with small D = 64 grids and with many planes of
-// small kernels: 5x5 D64 B4 H32 S192 34 | 46, S777 288 | 369, S1024 401 | 472.  The error against 64 bits is smaller in four kernels throughout.
-inline bool conv_attn_in_stages(int64_t planes, int64_t s, int64_t d, int64_t r, int64_t sk)
-{
-    constexpr int64_t sizes[][2] = {{3, 3}, {3, 5}, {5, 5}, {5, 7}, {6, 11}, {7, 7}, {7, 9}, {11, 15}};   // (where both have kernels of that size)
-    bool known = false;
-    for (const auto &size : sizes) known = known || (r == size[0] && sk == size[1]);
-    if (!known || s < 64) return false;
-    const double taps = (double)(r * sk), positions = (double)planes * s * s * 1e-6, blocks = (double)((s + 63) / 64);
-    const double rows = (double)(128 - (r - 1 + 7) / 8 * 8), items = planes * std::ceil(s / rows);
-    const double chain = std::max(blocks, items * (blocks + 1) / 2 * 1.25 / 256);   // key blocks one after the other on a CU
-    const double fused = d == 64 ? 6 + (7 + 0.073 * taps) * chain : 10 + (13.5 + 0.047 * taps) * chain;
-    const double four = std::max(22.0, 16 + 0.09 * planes + (d == 64 ? 3.3 : 3.9) * positions) + (s % 8 ? 9 + 6.4e-6 * planes * s * d : 0);
-    return four < 0.95 * fused;
-}
-
 // whether P (B,H,S,S) and X (B,H,S,D) are what the P V and P^T X kernels take: they index P by X's batch, heads and rows, where
 // the library product broadcasts
 inline bool score_planes_of(c10::IntArrayRef p, c10::IntArrayRef x)

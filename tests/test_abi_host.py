@@ -280,6 +280,11 @@ def test_forward_route_follows_grad_mode():
     announced to the stage hook only if the library has it: the one-kernel scores stage for 16-bit data, the matrix
     product and the scaled conv for fp32 (mta_qk_conv_supported is a host-side question)."""
     lib = _lib.load()
+    stages = lib.mta_conv_attn_in_stages
+    assert stages(1, 4, 512, 128, 6, 11, 1, 0) == 1 and stages(1, 4, 64, 64, 3, 3, 1, 0) == 0 and stages(4, 32, 1024, 64, 5, 5, 1, 0) == 0
+    for call in ((1, 4, 512, 128, 6, 11, 0, 0), (1, 4, 512, 128, 6, 11, 1, 1), (1, 4, 512, 96, 6, 11, 1, 0), (1, 4, 512, 128, 4, 4, 1, 0),
+                 (1, 65536, 512, 64, 6, 11, 1, 0), (1, 4, 63, 128, 6, 11, 1, 0)):   # no causal rule, 16 bits, sizes without the kernels
+        assert stages(*call) == 0, call
     assert lib.mta_qk_conv_supported(4096, 128, 6, 11, 1, 1) == 1 and lib.mta_qk_conv_supported(4096, 128, 11, 15, 2, 2) == 1
     assert lib.mta_qk_conv_supported(4096, 128, 6, 11, 0, 0) == 0      # fp32
     assert lib.mta_qk_conv_supported(4096, 128, 6, 11, 1, 0) == 0      # weights of another dtype

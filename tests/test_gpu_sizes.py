@@ -56,7 +56,8 @@ def test_headmix_fp32_32_heads_short_rows(pkg, q, c, group, causal):
 
 @pytest.mark.parametrize("b,h,s,d,r,sk", [
     (1, 3, 64, 128, 6, 11), (1, 2, 65, 128, 3, 3), (2, 3, 129, 64, 11, 15), (1, 2, 200, 64, 3, 5), (2, 2, 257, 64, 5, 7),   # whole and ragged lengths
-    (3, 4, 2300, 64, 7, 9),      # the batch entries in turns
+    (3, 4, 2300, 64, 7, 9),      # all at once (256 MB)
+    (5, 4, 2300, 64, 7, 9),      # the batch entries in turns, three and two
     (2, 5, 4104, 128, 5, 5),     # the heads of a batch entry in turns, a last part that is smaller
 ])
 @pytest.mark.parametrize("factor", [None, -0.3])
@@ -65,6 +66,7 @@ def test_conv_attention_fp32_stages(pkg, b, h, s, d, r, sk, factor):
     row statistic), which the tests above hold against the oracle: the two orders of sums differ by a few 2^-24 of the scores, whose
     exponentials turn that into relative errors; both 2-norms are below 5e-7."""
     print(f"conv_attention stages b={b} h={h} s={s} d={d} {r}x{sk}", flush=True)
+    assert pkg._lib.load().mta_conv_attn_in_stages(b, h, s, d, r, sk, 1, 0) == 1
     q, k, v = (x.cuda() for x in O.seeded_qkv(b, h, s, d, torch.float32, seed=47))
     module = pkg.TritonConvAttention(h, (r, sk), causal=True).cuda()
     with torch.no_grad():
