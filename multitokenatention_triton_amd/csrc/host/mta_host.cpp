@@ -603,6 +603,7 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
         bool need[7];
         for (int i = 0; i < 7; ++i) need[i] = ctx->needs_input_grad(i);
         const bool need_x = need[0] || need[1] || need[3], need_p = need_x || need[4], need_c = need_p || need[5];
+        const bool small = (int64_t)p.nbytes() <= WHOLE_STEP_BYTES;   // (anomaly mode takes this node at any size)
         variable_list out(11);
         Sums sums;
         const Tensor go = value_rows(grads[0], s_pad, m, lower);
@@ -611,10 +612,10 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
             Tensor dm = values_bwd_m(go, v, lower, first);
             if (dropout > 0) dm = at::native_dropout_backward(dm, keep, dropout < 1 ? 1.0 / (1.0 - dropout) : 0.0);
             Tensor dc;
-            std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], true, sums);
+            std::tie(dc, out[6]) = headmix_bwd(dm, c, w_post, post_causal, post_group, !causal, need_c, need[6], small, sums);
             dm.reset();
             Tensor dp;
-            if (need[5]) {   // (alone, too: see headmix_bwd)
+            if (need[5] && (need_p || small)) {   // (alone, too: see headmix_bwd)
                 if (auto both = conv2d_grads(p, dc, post_conv_w, causal, !causal, 1.0, sums)) std::tie(dp, out[5]) = *both;
             }
             if (need[5] && !out[5].defined()) out[5] = conv2d_bwd_weight(p, dc, post_conv_w, causal, 1.0, sums);
@@ -622,7 +623,7 @@ struct WholeStep : torch::autograd::Function<WholeStep> {
                 if (!dp.defined()) dp = conv2d_bwd_input(dc, post_conv_w, causal, !causal);
                 dc.reset();
                 probabilities_bwd(q, k, conv_w, w_pre, raw, x, p, first, causal, pre_causal, pre_group, std::move(dp), {need[0], need[1], need[3], need[4]},
-                                  {&out[0], &out[1], &out[3], &out[4]}, true, sums);
+                                  {&out[0], &out[1], &out[3], &out[4]}, small, sums);
             }
         }
         sums.run();

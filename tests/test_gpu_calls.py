@@ -513,3 +513,20 @@ def test_anomaly_mode(pkg):
         out = mod(q, k, v, None, None)
         out.sum().backward()
     assert all(torch.isfinite(t.grad).all() for t in (q, k, v, *mod.parameters()))
+
+
+@pytest.mark.parametrize("name", ["mta_conv_triton", "mta_conv_after_sm_triton", "wposm_triton"])
+def test_anomaly_mode_of_one_weight(pkg, name):
+    """A step over large score tensors in which one weight wants a gradient: anomaly mode, whose step is one node, forms that gradient alone as
+    the other nodes do - the same bits, where the kernel for both gradients of a conv adds up in another order."""
+    print(f"anomaly mode of {name}", flush=True)
+    mod = _module(pkg, 4, torch.float32).requires_grad_(False)
+    weight = getattr(mod, name).weight.requires_grad_(True)
+    q, k, v = (torch.randn(1, 4, 1280, 64, device="cuda") for _ in range(3))   # (26 MB a score tensor)
+    grads = []
+    for anomaly in (False, True):
+        weight.grad = None
+        with torch.autograd.set_detect_anomaly(anomaly):
+            mod(q, k, v, None, None).square().sum().backward()
+        grads.append(weight.grad)
+    assert torch.equal(*grads)
