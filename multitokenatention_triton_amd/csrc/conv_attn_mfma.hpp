@@ -239,7 +239,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
                                                              const T *__restrict__ V, const T *__restrict__ Wt,
                                                              T *__restrict__ O, float *__restrict__ Lse, int S, int causal,
                                                              float scale, int H, int nqb, int fill_upper, unsigned total_wg,
-                                                             unsigned heads, int jc_len,
+                                                             unsigned heads, unsigned per_xcd, int jc_len,
                                                              item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
 {
     static_assert(!BAND || SCORES_ONLY, "the band mask belongs to the scores-only kernel");
@@ -279,15 +279,22 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY ? ((R > 7 || (BAND && R >= 7))
     // (of 12 heads an XCD sees 3, of 4 one).  With other numbers of heads an XCD used to take an eighth of the list head by head - of 4
     // heads one XCD a head's long items and another its short ones.  us, that -> this, bf16 6x11, scores | attention: B1 H4 S3008 D128
     // 26.5 -> 24.1 | 117 -> 117, B1 H12 S2048 D64 33.7 -> 27.7 | 66.7 -> 67.2, S3712 D64 76.3 -> 67.5 | 152 -> 122, S4096 D128 101 -> 93 | 210 -> 170,
-    // B1 H20 S2048 D128 53.2 -> 45.8 | 106 -> 88.6; without a conv B1 H12 S2048 D64 16.9 -> 14.4, S2560 23.8 -> 20.1, but S3344 33.9 -> 36.2.
+    // B1 H20 S2048 D128 53.2 -> 45.8 | 106 -> 88.6; without a conv B1 H12 S2048 D64 16.9 -> 14.4, S2560 23.8 -> 20.1.  per_xcd: the old deal, see
+    // launch_mfma.
     // Work item = (batch*head, query block, chunk of jc_len key blocks).  The scores-only kernel splits the key
     // range of a query block (its output columns are independent; a chunk starts one key block early to rebuild
     // the retained halo columns), so that items are short and equal and the grid runs in several even rounds;
     // the attention kernel accumulates over all keys and gets jc_len = all of them.
     // (a 32-bit division: the 64-bit ones that this took were half a microsecond of a workgroup's start)
-    if (blockIdx.x >= total_wg) return;
-    int item = (int)(blockIdx.x / heads);
-    const int bh = (int)(blockIdx.x - (unsigned)item * heads);
+    unsigned id = blockIdx.x;
+    if (RAW && per_xcd) id = (id & 7) * per_xcd + (id >> 3);
+    if (id >= total_wg) return;
+    int item = (int)(id / heads), bh = (int)(id - (unsigned)item * heads);
+    if (RAW && per_xcd) {
+        const unsigned items = total_wg / heads;
+        bh = (int)(id / items);
+        item = (int)(id - (unsigned)bh * items);
+    }
     int qb = nqb - 1, jc = 0;
     int tbl_lo = -1, tbl_len = 0;
     if (tbl.n > 0) {
@@ -937,10 +944,18 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
         }
     }
     const int64_t total_wg = B * H * items_per_bh;
-    if (total_wg > 0x7fffffffLL) return MTA_ERR_SHAPE;
-    dim3 grid((unsigned)total_wg);
+    if (total_wg > 0x7ffffff0LL) return MTA_ERR_SHAPE;
+    // Raw scores of long rows that are not whole 128-byte lines, of heads in other numbers than multiples of 8: an XCD takes an eighth of the
+    // list, head by head.  Rank by rank, neighbouring items of a row end the same lines on two XCDs.  us, rank by rank | head by head, nothing in the
+    // caches, D64: B1 H12 S3344 63.7 | 60.4, S3400 73.7 | 68.9, S4008 100 | 94.6, H20 105 | 102, 122 | 117, 164 | 160, H28 S4008 234 | 221, B3 H12 302 | 287;
+    // either way at up to 3072 keys (H28 S3000 133 | 126, H12 55.8 | 58.0, H20 S1704 30.9 | 34.0); slower from 5000 on (H12 151 | 157, H20 263 | 267),
+    // with 4 heads (S4008 31.7 | 32.8), of whole lines (H12 S3008 37.4 | 44.7, H28 S4096 160 | 175), and mostly with a conv (6x11 H12 S4008 102 |
+    // 109).
+    const bool by_head = RAW && S % 64 != 0 && S > 3072 && S <= 4096 && (B * H) % 8 != 0 && B * H > 8;
+    const int64_t per_xcd = by_head ? (total_wg + 7) / 8 : 0;
+    dim3 grid((unsigned)(by_head ? per_xcd * 8 : total_wg));
     hipLaunchKernelGGL(kern, grid, dim3(few ? 512 : 256), 0, st, (const T *)q, (const T *)k, (const T *)v, (const T *)w, (T *)o,
-                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)(B * H), jc_len, tbl, band_lo, tri_gl, qs);
+                       lse, (int)S, causal, scale, (int)H, nqb, fill_upper, (unsigned)total_wg, (unsigned)(B * H), (unsigned)per_xcd, jc_len, tbl, band_lo, tri_gl, qs);
     return launch_status();
 }
 

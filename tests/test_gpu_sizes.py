@@ -344,6 +344,24 @@ def test_lower_scores_without_conv(pkg, d, dtype):
         assert torch.equal(got[..., low].float(), (a @ c.transpose(2, 3))[..., low])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,h,s", [(1, 9, 3080), (3, 5, 3080), (1, 12, 4088), (1, 9, 3072), (1, 16, 3080)])
+def test_lower_scores_of_ragged_rows(pkg, b, h, s, dtype):
+    """Raw scores of 3072 to 4096 keys and heads that do not divide among the XCDs, whose items go out head by head where the rows are no
+    whole lines: the bits of each head alone, with a band mask too; nothing missing and nothing else on and below the diagonal."""
+    g = torch.Generator(device="cuda").manual_seed(77)
+    a, c = (torch.randn(b, h, s, 64, generator=g, device="cuda").to(dtype) for _ in range(2))
+    low = torch.ones(s, s, dtype=torch.bool, device="cuda").tril()
+    first = (torch.arange(s, device="cuda") - 700).clamp(min=0).to(torch.int32).expand(b, s).contiguous()
+    for band in (None, first):
+        got = pkg.ops.lower_scores(a, c, band)
+        for i in range(b):
+            for j in range(h):
+                alone = pkg.ops.lower_scores(a[i:i + 1, j:j + 1], c[i:i + 1, j:j + 1], None if band is None else band[i:i + 1])
+                inside = low if band is None else low & (torch.arange(s, device="cuda")[None] >= first[0][:, None])
+                assert torch.equal(got[i, j][inside], alone[0, 0][inside]), (i, j)
+
+
 @pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("r,sk", [(3, 3), (3, 5), (5, 5), (5, 7), (6, 11), (7, 7), (7, 9), (11, 15)])
 def test_row_sliding_conv(pkg, r, sk, dtype, wdtype):
