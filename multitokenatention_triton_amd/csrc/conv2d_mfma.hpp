@@ -177,12 +177,13 @@ __global__ __launch_bounds__(M_WT, (wg_per_cu<R, NARROW, DW>())) void conv2d_mfm
     constexpr int WRAW_IT = (WRAW_DW + 63) / 64;
     constexpr int WRAW_SLOT = (SLOTS + 3) & ~3;              // (64-byte aligned)
     constexpr int NEED_SLOTS = WRAW_SLOT + WRAW_IT * 16;     // (a copy instruction of the kernel rows covers 16 slots)
-    constexpr int BUF_SLOTS = NEED_SLOTS > STAGE_IT * M_WT ? (NEED_SLOTS + 3) / 4 * 4 : STAGE_IT * M_WT;
+    constexpr int BUF_SLOTS = NEED_SLOTS > STAGE_IT * M_WT ? (NEED_SLOTS + 15) / 16 * 16 : STAGE_IT * M_WT;
     constexpr int BUF = BUF_SLOTS * VEC;                     // elements per LDS strip buffer
     // DW: behind it x over the strip's own positions, a wavefront's 16 rows after the other; 16-byte piece c of row r at c ^ 2 (r % 8):
     // a transpose read takes 32 bytes of 8 consecutive rows at a time, which lie in different banks then
     constexpr int XBUF = DW ? 16 * M_HALF : 0;               // elements per wavefront
     constexpr int BUFX = BUF + M_NW * XBUF;
+    static_assert(!DW || (BUF * sizeof(T) % 256 == 0 && BUFX * sizeof(T) % 256 == 0), "the exclusive or on an address of x is one on its place in 256 bytes");
     __shared__ __align__(256) T tiles[2 * BUFX];              // double buffer: strip n is computed while strip n+1 lands
     using V16 = pack16<T>;
 
