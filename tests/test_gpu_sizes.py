@@ -1080,7 +1080,7 @@ def _conv64(x, w, causal, bwd):
 @pytest.mark.parametrize("h,w", [(1, 4), (31, 127), (33, 129), (64, 128), (40, 300), (300, 70), (389, 389)])
 def test_conv_11x15_split(pkg, h, w, dtype, wdtype):
     """11x15 kernels on the parts of the values (fp32; 16-bit data with other weights or of odd widths): edges of the 32 x 128 strips,
-    planes that take one strip and several in turns, wide and tall ones; forward, scaled, lower triangle only, input gradient; causal
+    planes of one strip and of several (a workgroup each; several in turns: test_conv_split_strips_in_turns), wide and tall ones; forward, scaled, lower triangle only, input gradient; causal
     or not.  Bound: 165 products and sums of 32 bits in any order, (165 + 2) 2^-24 of the sum of their magnitudes, and one rounding
     of the result to its type."""
     g = torch.Generator(device="cuda").manual_seed(61)
@@ -1145,6 +1145,52 @@ def test_conv_11x15_split_range(pkg, bwd):
         got = pkg.ops.conv2d_bwd_input(a, w, True) if bwd else pkg.ops.conv2d_causal(a, w, True)
         want, size = _conv64(a, w, True, bwd)
         assert ((got.double() - want).abs() <= 167 * (2.0 ** -24 * size + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("n,c,h,w", [(2, 8, 1000, 1001), (1, 16, 777, 777), (3, 7, 700, 801)])
+@pytest.mark.parametrize("dtype,wdtype,r,k", [(torch.float32, torch.float32, 11, 15), (torch.bfloat16, torch.float32, 6, 11), (torch.float16, torch.float16, 7, 9)])
+def test_conv_split_strips_in_turns(pkg, dtype, wdtype, r, k, n, c, h, w):
+    """Convs on the parts of the values where a workgroup walks several strips (two workgroups per CU: 32 or 25 per plane here), planes dealt to the XCDs
+    and not: forward, lower triangle only, input gradient, causal or not; in the middle of a walk an infinite value, whose
+    results come from multiply-adds, and in fp32 a stretch of tiny ones.  Bounds as for planes of few strips."""
+    g = torch.Generator(device="cuda").manual_seed(79)
+    x, weight = torch.randn(n, c, h, w, generator=g, device="cuda").to(dtype), (0.1 * torch.randn(c, r, k, generator=g, device="cuda")).to(wdtype)
+    hit = (n - 1, c // 2, h // 2, w // 4)
+    if dtype == torch.float32:
+        x[:, :, h // 2 + 40:h // 2 + 100, :w // 3] *= 2.0 ** -125
+    low = torch.ones(h, w, dtype=torch.bool, device="cuda").tril()
+    ulp = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    left = (k - 1) // 2
+    for causal in (True, False):
+        for bwd in (False, True):
+            taps = weight.flip(-1, -2) if bwd else weight
+            pads = (k - 1 - left, left, 0, r - 1) if bwd else (left, k - 1 - left, r - 1, 0)
+            data = torch.nn.functional.pad(torch.where(low, x, torch.zeros_like(x)) if causal else x, pads).double()
+            want, size = torch.zeros(n, c, h, w, dtype=torch.float64, device="cuda"), torch.zeros(n, c, h, w, dtype=torch.float64, device="cuda")
+            for i in range(r):
+                for j in range(k):
+                    piece, tap = data[..., i:i + h, j:j + w], taps[:, i, j].double().view(1, c, 1, 1)
+                    want.addcmul_(piece, tap)
+                    size.addcmul_(piece.abs(), tap.abs())
+            bound = (r * k + 2) * 2.0 ** -24 * size + ulp * want.abs() + (2.0 ** -25 if dtype == torch.float16 else r * k * 2.0 ** -149)
+            keep = low if causal else torch.ones_like(low)
+            rows = slice(hit[2] - r + 1, hit[2] + 1) if bwd else slice(hit[2], hit[2] + r)
+            reach = slice(hit[3] - (left if bwd else k - 1 - left), hit[3] + (k - 1 - left if bwd else left) + 1)
+            for fill in (True, False):
+                for infinite in (False, True):
+                    y = x.clone()
+                    if infinite:
+                        y[hit] = float("inf")
+                    got = pkg.ops.conv2d_bwd_input(y, weight, causal, fill_upper=fill) if bwd else pkg.ops.conv2d_causal(y, weight, causal, fill_upper=fill)
+                    off = ~((got.double() - want).abs() <= bound) & keep
+                    if fill and causal:
+                        assert not got[..., ~low].any()
+                    if infinite:
+                        seen = torch.zeros_like(off)
+                        seen[hit[0], hit[1], rows, reach] = True
+                        assert not torch.isfinite(got[seen & keep]).any()
+                        off &= ~seen
+                    assert not off.any(), (causal, bwd, fill, infinite)
 
 
 @pytest.mark.parametrize("heads,s,d", [(300, 4, 64), (300, 132, 64), (37, 388, 64), (9, 1000, 64), (16, 1024, 64), (130, 60, 128), (130, 64, 128), (23, 388, 128),
@@ -1255,7 +1301,7 @@ def test_attention_of_few_workgroups(pkg, d, dtype, r, k):
 def test_conv_both_gradients(pkg, r, k, dtype):
     """Both gradients of the conv in one pass over dy against the two kernels: dx bit for bit; dw, the same exact products summed in fp32 in
     another order and rounded to the weight's dtype, within sqrt(n)*2^-22 of the sum of magnitudes and half a unit.  Edges of the 64 x 128
-    strips, fewer strips than workgroups and several rounds of them, more channels than workgroups; whole rows, the lower triangle, no
+    strips, fewer strips than workgroups, more channels than workgroups (several rounds of strips: the test below); whole rows, the lower triangle, no
     mask on planes that are not square; NaN above the diagonal of both operands."""
     g = torch.Generator(device="cuda").manual_seed(67)
     for b, c, h, w, causal, fill in ((1, 2, 8, 8, True, True), (2, 3, 64, 64, True, False), (1, 2, 136, 136, True, True), (2, 2, 200, 200, True, False),
@@ -1275,6 +1321,27 @@ def test_conv_both_gradients(pkg, r, k, dtype):
         assert dw.dtype == dtype and ((dw.double() - exact).abs() <= bound).all(), (b, c, h, w)
         _, again = pkg.ops.conv2d_grads(x, dy, weight, causal, fill_upper=fill, over_x=True)   # the gradient in x's place
         assert torch.equal(again, dw) and (torch.equal(x, dx) if fill else torch.equal(x.tril(), dx.tril())), (b, c, h, w)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,k", [(3, 3), (6, 11), (7, 7), (11, 15)])
+def test_conv_both_gradients_in_rounds(pkg, r, k, dtype):
+    """... where a workgroup walks several strips of its channel, in uneven rounds (two workgroups per CU: 32 per channel of 16, 64 of 8, 12 of 43)
+    over one plane and several: dx bit for bit, dw within the bound above, in x's place the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(78)
+    for b, c, s, fill in ((1, 16, 1096, True), (2, 16, 520, False), (3, 16, 776, True), (1, 8, 1800, False), (2, 43, 456, True)):
+        x, dy = (torch.randn(b, c, s, s, generator=g, device="cuda").to(dtype) for _ in range(2))
+        weight = torch.randn(c, r, k, generator=g, device="cuda").to(dtype)
+        size = pkg.ops.conv2d_bwd_weight(x.abs(), dy.abs(), (r, k), True).double()
+        above = ~torch.tril(torch.ones(s, s, dtype=torch.bool, device="cuda"))
+        x, dy = x.masked_fill(above, float("nan")), dy.masked_fill(above, float("nan"))
+        dx, dw = pkg.ops.conv2d_grads(x, dy, weight, True, fill_upper=fill)
+        want, exact = pkg.ops.conv2d_bwd_input(dy, weight, True, fill_upper=fill), pkg.ops.conv2d_bwd_weight(x, dy, (r, k), True).double()
+        assert torch.equal(dx, want) if fill else torch.equal(dx.tril(), want.tril()), (b, c, s)
+        bound = (b * s * s) ** 0.5 * 2.0 ** -22 * size + exact.abs() * _unit(dtype) + (2.0 ** -25 if dtype == torch.float16 else 0.0)
+        assert ((dw.double() - exact).abs() <= bound).all(), (b, c, s)
+        _, again = pkg.ops.conv2d_grads(x, dy, weight, True, fill_upper=fill, over_x=True)
+        assert torch.equal(again, dw) and (torch.equal(x, dx) if fill else torch.equal(x.tril(), dx.tril())), (b, c, s)
 
 
 def test_conv_both_gradients_refuses(pkg):
@@ -1328,7 +1395,7 @@ def test_conv_both_gradients_by_rows(pkg, r, k, dtype, wd):
     (torch.bfloat16, torch.float32, ((5, 7), (7, 7), (6, 11), (7, 9))), (torch.bfloat16, torch.bfloat16, ((5, 7), (7, 7), (6, 11), (7, 9))),
     (torch.float16, torch.float32, ((6, 11), (7, 9))), (torch.float16, torch.float16, ((6, 11), (7, 9))), (torch.bfloat16, torch.float16, ((6, 11),))) for rk in sizes])
 def test_conv_split_of_16_bit_data(pkg, dtype, wd, r, k):
-    """16-bit data with other weights, or of odd widths, on the parts of the values: edges of the 32 x 128 strips, several strips in turns; an
+    """16-bit data with other weights, or of odd widths, on the parts of the values: edges of the 32 x 128 strips; an
     infinite value stays where a tap takes it.  Bound: r k products and sums of 32 bits in any order, and one rounding to 16 bits."""
     g = torch.Generator(device="cuda").manual_seed(69)
     w = (0.1 * torch.randn(3, r, k, generator=g, device="cuda")).to(wd)
