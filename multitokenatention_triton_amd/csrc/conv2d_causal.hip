@@ -8,10 +8,11 @@
 // tiles that lie entirely above the diagonal (they only receive their +0 fill), and
 // applies the causal output rule on store.
 //
-// Three compute paths:
+// Four compute paths:
 //   conv2d_valu  fp32 FMAs from an fp32 LDS tile (8 outputs per lane); any I/O and weight dtype, any kernel size.
 //   conv2d_rows  fp32 FMAs, sliding down the rows in registers (conv2d_rows.hpp); any I/O and weight dtype, the kernel
 //                sizes known at compile time.
+//   conv2d_split 11x15, and the larger of the others in 16 bits, of what conv2d_mfma does not take (conv2d_split.hip).
 //   conv2d_mfma  16-bit I/O with weights of the same dtype.  The 6x11 conv costs 66 FMAs
 //                per output, which on the vector ALU takes longer than moving the tensor
 //                through HBM.  Each kernel row is therefore applied as a banded (Toeplitz)

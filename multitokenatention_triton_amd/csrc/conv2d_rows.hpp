@@ -1,6 +1,7 @@
 // Row-sliding fp32-FMA kernels of the depthwise conv: forward, input gradient and kernel gradient for the I/O types, weight
 // types and widths the matrix-core kernels do not take (fp32; 16-bit data with weights of another dtype or with rows that are
-// not whole 16-byte vectors), kernel sizes known at compile time.
+// not whole 16-byte vectors), kernel sizes known at compile time.  conv2d_split.hip comes first in the forward and the input gradient of
+// 11x15, and of 6x11, 7x9, 7x7 (bf16) and small 5x7 (bf16) in 16 bits: those instances here are what MTA_CONV_FORCE_VALU=1 takes.
 //
 // A wavefront owns a strip of M rows and walks down the input rows.  A lane loads four consecutive keys of a row (one load
 // instruction per row: 256 keys), several rows ahead, and takes the halo from its neighbours' registers (DPP shifts by one
@@ -117,7 +118,8 @@ template <typename G, int M> struct strips {
     }
 };
 
-// rows fetched ahead (the loop is unrolled by as many); 8 where a short strip has many halo rows (11x15, 8 planes of 256^2: 15.1 -> 13.0 us)
+// rows fetched ahead (the loop is unrolled by as many); 8 where a short strip has many halo rows (11x15, 8 planes of 256^2: 15.1 -> 13.0 us,
+// under MTA_CONV_FORCE_VALU=1)
 template <int R, int M> constexpr int rows_ahead() { return M == 4 && R > 7 ? 8 : 4; }
 
 // y = conv(x) (BWD: the gradient with respect to x: kernel reversed in both axes, row halo below); M rows per strip

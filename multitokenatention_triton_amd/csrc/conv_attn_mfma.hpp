@@ -42,8 +42,9 @@ typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 // grids: NW = 8 with one block of 16 rows each, see launch_mfma.  (The scores-only kernel on eight, with the fragments of K read twice as
 // often: 6x11 B2 H16 S512 D64 12.5 -> 17.4 us, B4 H16 S1024 D128 38.4 -> 43.2.)
 // What bounds the attention kernel: matrix products (896 flops executed per score at 6x11, D = 128: Q K^T and P V 256 each, the
-// conv as Toeplitz products 384) beside the vector ALU (the exponentials) and the LDS, which would each take 40 to 60 % of its
-// time alone.  So the vector work is kept small (one maximum, one multiply-add, one exponential and half a conversion and a sum
+// conv as Toeplitz products 384) beside the vector ALU (the exponentials) and the LDS, which would each take 35 to 50 % of its
+// time alone (6x11 B1 H32 S8192 D128, by counters: the matrix cores are busy 47 % of the cycles at about 2.1 GHz, the LDS 42 %, the vector ALU
+// 37 %): what is left is how far the two wavefronts of a SIMD overlap them between two barriers per key block.  So the vector work is kept small (one maximum, one multiply-add, one exponential and half a conversion and a sum
 // per score: no rounding between the conv and the probabilities) and is written between the products of the same wavefront:
 // the first row block's probabilities among the second one's conv products, half of the second one's among those of P V.
 // The loop has one body: K, V and the buffer the next block goes to are offsets into one LDS array (all reads of it are issued
@@ -979,8 +980,7 @@ int dispatch_mfma(const void *q, const void *k, const void *v, const void *w, vo
         MTA_FUSED_CASE(6, 11)
         MTA_FUSED_CASE(7, 7)
         MTA_FUSED_CASE(7, 9)
-        // (the 44 registers of its Toeplitz fragments leave the scores kernel two workgroups per CU and the attention
-        // kernel, at the limit of two with 7 kernel rows, one)
+        // (the 44 registers of its Toeplitz fragments leave both kernels two workgroups per CU)
         MTA_FUSED_CASE(11, 15)
 #undef MTA_FUSED_CASE
     }

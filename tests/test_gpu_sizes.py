@@ -606,8 +606,8 @@ def test_sums_by_number_of_partial_results(pkg, parts):
 @pytest.mark.parametrize("r,k", [(3, 3), (5, 5), (6, 11), (7, 7), (11, 15)])
 @pytest.mark.parametrize("d", [64, 128])
 def test_fp16_attention_by_grid(pkg, d, r, k):
-    """fp16 attention of 600 workgroups and, of the same heads, 2 x 300, which the chip holds at once: other instances for 5 to 7 kernel
-    rows, the same sums in the same order."""
+    """fp16 attention of 600 workgroups, four wavefronts of 32 rows each, and, of the same heads, of 2 x 300, few enough for eight of 16: the
+    same sums in the same order."""
     g = torch.Generator(device="cuda").manual_seed(59)
     q, kk, v = (torch.randn(1, 300, 136, d, generator=g, device="cuda").half() for _ in range(3))
     w = (0.1 * torch.randn(300, r, k, generator=g, device="cuda")).half()
