@@ -93,11 +93,16 @@ def test_conv_attention_fp32_scratch(pkg, b, h, s):
         assert s * s * 4 < beside <= 516 << 20
         del got
         torch.cuda.empty_cache()
-        total = torch.cuda.get_device_properties(0).total_memory
+        total, room, fill = torch.cuda.get_device_properties(0).total_memory, torch.cuda.memory_reserved(), []
         try:
-            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 6 * q.numel() * 4 + (24 << 20)) / total)
+            torch.cuda.set_per_process_memory_fraction(room / total)
+            with pytest.raises(torch.OutOfMemoryError):   # (what is left free in the pool's segments)
+                while len(fill) < 4096:
+                    fill.append(torch.empty(16 << 20, dtype=torch.uint8, device="cuda"))
+            torch.cuda.set_per_process_memory_fraction((room + 6 * q.numel() * 4 + (24 << 20)) / total)
             got = module(q, k, v, True, None)[0]
         finally:
+            fill.clear()
             torch.cuda.set_per_process_memory_fraction(1.0)
     want, _ = pkg.ops.conv_attn_fwd(q, k, v, module.weight.detach(), True, None, return_lse=True)
     assert torch.equal(got, want)
