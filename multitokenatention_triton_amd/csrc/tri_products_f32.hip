@@ -593,7 +593,7 @@ int check(const void *a, const void *b, const void *c, int64_t B, int64_t H, int
 
 // Scores on tiles of 128 x 128 in LDS slabs from half a workgroup per CU on, on the bf16 matrix cores (tri_products_split.hip) from 300 tiles on, and
 // at D = 128 instead of the slabs: us, direct | slabs | split: D64 B1 H8 S512 (80 tiles) 6.2 | 9.4 | 8.5, B1 H16 S512 (160) 14.8 | 9.4 | 9.1, B2 H16
-// S512 (320) - | 15.1 | 12.7, B1 H16 S1024 (576) 24.7 | 22.2 | 17.6; D128 (80) 8.4 | 13.2 | 11.1, (160) 17.5 | 14.7 | 11.7, (576) 39.5 | 34.4 | 26.2.
+// S512 (320) - | 15.1 | 13.2, B1 H16 S1024 (576) 24.7 | 22.2 | 18.3; D128 (80) 8.4 | 13.2 | 11.1, (160) 17.5 | 14.7 | 12.1, (576) 39.5 | 34.4 | 26.2.
 
 // resident: workgroups that a CU holds at once
 template <typename K, typename... ARGS>

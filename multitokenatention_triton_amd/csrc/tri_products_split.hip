@@ -7,13 +7,13 @@
 // products of the step before (rows of bf16, 16-byte chunks XOR-swizzled by the key), and serve all four wavefronts.
 // What bounds it is the CU's path to the L2, which the scores (out) and the keys (in, half as much at D = 64, as much at 128) pass: 4.6
 // TB/s together at B1 H16 S2048 D64.  On v_mfma_f32_16x16x4f32, in slabs of 16 dims of both operands, it was the matrix rate and the
-// loads of two operands per tile.  us, those -> this: D64 B2 H16 S512 15.1 -> 12.6, B1 H12 S800 13.9 -> 12.0, B1 H16 S1024 22.2 -> 17.6, B1
-// H32 S1024 36.6 -> 28.8, B1 H16 S2048 61.5 -> 42.1; D128 B1 H16 S512 14.7 -> 11.7, B1 H32 S1024 64.5 -> 42.6, B1 H16 S2048 102 -> 63.8.  Error
+// loads of two operands per tile.  us, those -> this: D64 B2 H16 S512 15.1 -> 13.2, B1 H12 S800 13.9 -> 12.4, B1 H16 S1024 22.2 -> 18.3, B1
+// H32 S1024 36.6 -> 27.3, B1 H16 S2048 61.5 -> 41.9; D128 B1 H16 S512 14.7 -> 12.1, B1 H32 S1024 64.5 -> 40.9, B1 H16 S2048 102 -> 62.7.  Error
 // against 64 bits (2-norm): D64 1.4e-7 -> 0.5e-7, D128 2.0e-7 -> 0.65e-7.
 // Runs of 1 | 2 | 4 steps: D64 B1 H16 S1024 (1152 steps) 18.7 | 17.6 | 20.4, B1 H32 S1024 (2304) 34.4 | 31.9 | 28.8, B1 H16 S2048 (4352) 56.3 | 46.3
 // | 42.1; D128, twice as many, B2 H16 S512 17.5 | 17.3 | 18.2, B1 H16 S2048 88.0 | 70.8 | 63.8.
 // Operands are split 2^24 times as large (split.hpp); a wavefront with a sum that is not finite then forms its step again with fp32
-// products.  (Unscaled, with a look at the sums, which cannot tell small operands against large ones: 1 to 4 % faster, and up to 12000
+// products.  (Unscaled, with a look at the sums, which cannot tell small operands against large ones: up to 5 % faster, and up to 12000
 // times the error of 32-bit sums.  us with nothing in the caches, that -> this: D64 B1 H16 S512 9.8 -> 9.8, S1024 19.3 -> 20.2, S2048 54.0 -> 53.8;
 // D128 11.6 -> 12.1, 27.1 -> 27.4, 68.3 -> 69.1.)
 // (P V and P^T X in this form, with a V block per 64 rows: as fast as on the fp32 instructions - B1 H32 S1024 D64 26.1 | 28.3, B1 H32 S2048 D128 155 |
