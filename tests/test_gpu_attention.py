@@ -250,6 +250,63 @@ def test_qk_conv_parity(pkg, case, fill):
             assert (got[..., 0, s - 64:].float() == torch.tensor(sentinel).to(dtype).float()).all()
 
 
+PAIR_CASES = [(3, 3, 64), (3, 5, 128), (5, 5, 128), (5, 7, 64), (6, 11, 64), (6, 11, 128), (7, 7, 128), (7, 9, 64), (11, 15, 128)]
+
+
+def _non_finite_inputs(h, s, d, dtype):
+    """Q, K, V of three heads: one row of Q NaN, one infinite, at an odd and an even row; one key infinite."""
+    q, k, v = O.seeded_qkv(1, h, s, d, dtype, seed=17)
+    clean = q.clone(), k.clone()
+    q[0, 0, 101] = float("nan")
+    q[0, 1, 60] = float("inf")
+    k[0, 2, 150] = float("inf")
+    return q, k, v, clean
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", PAIR_CASES)
+def test_qk_conv_non_finite_scores_stay_local(pkg, case, dtype):
+    """The conv's products take two query rows and eight keys at a time, with zero taps where a row of the window belongs to the
+    other row only: a score that is not finite makes the R x S outputs that take it non-finite, and no others."""
+    r, sk, d = case
+    h, s = 3, 200
+    print(f"qk_conv non-finite {case} {dtype}", flush=True)
+    q, k, _, (cq, ck) = _non_finite_inputs(h, s, d, dtype)
+    w = O.seeded_conv_weight(h, r, sk, 0.05, dtype)
+    w[w == 0] = 0.01
+    scale = float(torch.rsqrt(torch.tensor(float(d))))
+    low = torch.tril(torch.ones(s, s, dtype=torch.bool))
+    scores = torch.matmul(q.float(), k.float().transpose(2, 3)).masked_fill(~low, 0.0)
+    foot = O.depthwise_conv((~torch.isfinite(scores)).float(), torch.ones(h, r, sk), True) > 0.5
+    got = pkg.ops.qk_conv(q.cuda(), k.cuda(), w.cuda(), True, scale).cpu().float()
+    clean = pkg.ops.qk_conv(cq.cuda(), ck.cuda(), w.cuda(), True, scale).cpu().float()
+    assert torch.equal(~torch.isfinite(got), foot & low)
+    ok = low & ~foot          # (formed again tap by tap where a neighbour was NaN: another order of the sum, one rounding)
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    torch.testing.assert_close(got[ok], clean[ok], rtol=ulp, atol=1e-5)
+
+
+@pytest.mark.parametrize("planes", [1, 80])   # workgroups of eight wavefronts with a row block each, of four with two
+@pytest.mark.parametrize("case", PAIR_CASES)
+def test_conv_attention_non_finite_rows_stay_local(pkg, case, planes):
+    """A query row that is not finite reaches the R rows from it on, an infinite key every row that attends a score of it."""
+    r, sk, d = case
+    h, s, dtype = 3 * planes, 200, torch.bfloat16
+    print(f"conv_attn non-finite {case} planes={planes}", flush=True)
+    q, k, v, (cq, ck) = _non_finite_inputs(3, s, d, dtype)
+    w = O.seeded_conv_weight(3, r, sk, 0.05, dtype)
+    many = lambda t: t.repeat(*((1, planes) if t.dim() == 4 else (planes,)), *(1,) * 2).cuda()  # noqa: E731
+    got = pkg.ops.conv_attn_fwd(many(q), many(k), many(v), many(w), True, None).cpu().float()
+    clean = pkg.ops.conv_attn_fwd(many(cq), many(ck), many(v), many(w), True, None).cpu().float()
+    bad = torch.zeros(3, s, dtype=torch.bool)
+    bad[0, 101:101 + r] = True
+    bad[1, 60:60 + r] = True
+    bad[2, 150:] = True       # (rows ahead of the key never see it)
+    bad = bad.repeat(planes, 1)
+    assert not torch.isfinite(got[0][bad]).any()
+    torch.testing.assert_close(got[0][~bad], clean[0][~bad], **tol(dtype))
+
+
 def _band_first(kind, b, s, seed=3):
     """int32 (B,S) first visible key per row: a sliding window, packed documents (per batch entry), or ragged."""
     rows = torch.arange(s)
