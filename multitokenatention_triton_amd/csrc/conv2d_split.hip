@@ -5,23 +5,29 @@
 // Every fp32 value is the sum of three bf16 values (8 + 8 + 8 bits of its significand; each one the rounded remainder of those
 // before it), exactly: x = x0 + x1 + x2, w = w0 + w1 + w2 (fp16: two parts, bf16: one).  Of the products of parts the six (bf16 data with
 // fp32 weights: three) with i + j <= 2 are formed; each is exact in fp32, what is left out is below 2^-26 |x w|, a quarter of the last place that one fp32
-// multiply-add rounds away.  A kernel row is applied as in conv2d_causal.hip, as a banded Toeplitz product (one 32-key window
-// holds the taps of 16 outputs), once per pair of parts: w0 x0 adds into one accumulator, the small ones into two others, and a
-// result is their sum.  So an output takes R roundings of its own size where multiply-adds took R*S: the error against 64 bits
-// (2-norm) is 0.55e-7 forward and 1.0e-7 for the input gradient, where they left 1.3e-7 and 2.9e-7 (scores, 333^2 and 512^2).
+// multiply-add rounds away.  A product takes the outputs of two rows and eight keys
+// of sixteen pairs of rows; its 32 slots are four rows of the pair's window, eight columns each, and three such chunks hold the taps of eight keys:
+// an operand from LDS serves the three groups of keys whose windows it is part of.  Once per pair of parts: w0 x0 adds into two accumulators
+// (16-bit data: one), the small ones into another, and a result is their sum.  So an output takes 9 roundings of its own size or less (11x15) where
+// multiply-adds took R*S: the error against 64 bits
+// (2-norm) is 0.48e-7 forward and 0.73e-7 for the input gradient, where they left 1.3e-7 and 2.9e-7 (scores, 333^2 and 512^2; random taps
+// 0.58e-7 and 0.59e-7; with one accumulator for w0 x0 1.0e-7 and 1.1e-7).
 //
 // Why: R*S multiply-adds on the vector units (0.079 PFLOP/s without packed fp32 forms) bound the row-sliding kernels from about 50
-// taps on.  The Toeplitz form executes 6 * 64 * R flops for the 2*R*S of an output, at 2.5 PFLOP/s: 2.5 times the vector rate.
-// us, conv2d_rows -> this, fp32: lower triangle 16 planes of 512^2 23 -> 18.5, 12 of 801^2 32 -> 28.5, 16 of 1024^2 58 -> 38, 32 of
+// taps on.  This form executes 6 * 64 * 9 flops for the 2 * 165 of an output of 11x15, at 2.5 PFLOP/s.
+// One kernel row and sixteen keys per product (11 products and as many operands per 256 outputs, 9 and 4 now) -> this, fp32 11x15, whole
+// rows: 16 planes of 512^2 19.9 -> 18.9, 12 of 801^2 31.1 -> 28.8, 16 of 1024^2 41.3 -> 37.9, 32 of 1024^2 66.6 -> 60.5, 16 of 2048^2 142 either way;
+// 16-bit data, with as many workgroups per CU as their registers allow (split_occ) where two ran: bf16 16 of 1001^2 7x7 21.7 -> 20.6, 11x15 23.3 -> 21.7,
+// fp16 6x11 27.4 -> 23.8, with fp32 weights 16 of 1024^2 bf16 6x11 23.0 -> 20.6, 7x9 23.8 -> 20.1, fp16 6x11 27.7 -> 29.0, 7x9 29.1 -> 28.9 (177 registers: two).
+// us, conv2d_rows -> the former, fp32: lower triangle 16 planes of 512^2 23 -> 18.5, 12 of 801^2 32 -> 28.5, 16 of 1024^2 58 -> 38, 32 of
 // 1024^2 105 -> 68, 16 of 2048^2 177 -> 128; whole rows 31 -> 20, 34 -> 31, 86 -> 43, 152 -> 80, 260 -> 151.  Smaller kernels stay
 // there, lower triangle | whole rows: 7x9 16 of 1024^2 29.7 | 39.4 against 29.4 | 34.5 here, 16 of 512^2 13.9 | 16.4 against 15.3 |
 // 16.5, 16 of 2048^2 92 | 128 against 98 | 140; 6x11 and 5x7 alike or slower.
 // 16-bit data with fp32 weights, lower triangle of 16 planes of 1024^2, bf16 | fp16: 5x7 22.2 -> 18.6 | 22.2 -> 22.7, 7x7 26.0 -> 20.6 | (kept) 26.4,
 // 6x11 29.4 -> 19.5 | 29.6 -> 24.6, 7x9 28.9 -> 20.8 | 29.4 -> 25.8; bf16 16 of 512^2 6x11 13.0 -> 10.8, 32 of 2048^2 6x11 152 -> 115, 7x7 121 -> 117 (5x7
 // 109 -> 114: kept); weights of the data's type, whole rows of 16 planes of 1001^2: bf16 7x7 34.6 -> 23.3, 6x11 40.4 -> 22.9, fp16 6x11 40.8 -> 28.1.
-// What bounds it: half of the time the matrix cores are busy (16 of 2048^2: 62 of 128 us); without the loads, stores and
-// the splitting the products take 95 us - their operands' LDS reads, the barrier of a strip and the blocks beside the
-// triangle - and the CU's path to the L2 (1.5 times the strip in, the strip out) the rest.
+// What bounds it (16 of 1024^2, 40 us): without products 24, without loads and splitting 35, without stores 39; 16 of 2048^2, 145 us: 137, 96, 111 -
+// the CU's path to the L2 (1.5 times the strip in, the strip out), and at 1024^2 five rounds of strips with the products' 17 us in them.
 // Values that have three parts are split 2^24 times as large, results taken back: every fp32 value below 2^104 then has parts that are normal
 // numbers (the smallest denormal's only bit is 2^-125), however small it is and whatever lies beside it, and the products of parts of
 // small values stay above the denormals as well.  Results that are not finite then - an operand was not, or is larger, or a sum of
@@ -33,9 +39,8 @@
 //
 // Shape.  A workgroup of four wavefronts takes strips of 32 rows x 128 keys of one plane, one after the other, two workgroups per
 // CU.  A strip and its halo are loaded four keys per lane, two strips ahead, into registers; split and written to one of two LDS
-// buffers (a plane of bf16 per part with rows of 288 bytes, for which a fragment read - 16 rows x 64 bytes - is free of bank
-// conflicts) a vector at a time between the products of the strip before.  The Toeplitz fragments of the plane's kernel stay in
-// registers (3 * R * 4 of them); they come out of a table of all windows of every kernel row.
+// buffers (a plane of bf16 per part) a vector at a time between the products of the strip before.  The fragments of the plane's kernel stay in
+// registers (11x15: 3 parts * 3 quads * 3 chunks * 4 of them); they come out of a table of all windows of every kernel row.
 #include "conv2d_rows.hpp"
 #include "split.hpp"
 
@@ -45,6 +50,7 @@ using namespace mta;
 constexpr int P_TM = 32, P_TN = 128;       // strip
 constexpr int P_HL = 8;                    // keys staged left (and right) of it
 constexpr int P_LD = P_TN + 2 * P_HL;      // keys of a staged row
+constexpr int P_RS = P_LD + 8;             // its length in LDS, an odd number of 16-byte chunks: operand reads free of bank conflicts (two rows between lanes)
 constexpr int P_QUADS = P_LD / 4;
 
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
@@ -61,14 +67,20 @@ inline int64_t p_count(int64_t H, int64_t W, int tri)
 
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
+// Workgroups per CU: a strip is a chain of loads, splitting, products and stores between two barriers, and what hides it is the other
+// workgroups.  The fewer parts, the fewer registers and the less LDS a workgroup takes.
+template <typename T, int WP, int R> constexpr int split_occ() { return parts_of<T>() == 1 && WP == 1 ? 4 : parts_of<T>() * WP <= 4 && R <= 7 ? 3 : 2; }
+
 template <typename T, int WP, int R, int S, bool BWD>
-__global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
+__global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
                                                        int W, int causal, float in_scale, int use_scale, int w_dtype, int planes, int total, int per_plane)
 {
-    constexpr int PAD = BWD ? S - 1 - (S - 1) / 2 : (S - 1) / 2, SHIFT = P_HL - PAD;   // first tap's slot in a 32-key window
-    static_assert(SHIFT >= 0 && SHIFT + 16 + S - 1 <= 32 && S - 1 - PAD <= P_HL, "the taps of 16 outputs in a window of 32 keys");
+    constexpr int PAD = BWD ? S - 1 - (S - 1) / 2 : (S - 1) / 2, SHIFT = P_HL - PAD;   // first tap's column in a window of 24
+    static_assert(SHIFT >= 0 && SHIFT + 8 + S - 1 <= 24, "the taps of 8 outputs in three chunks of 8 columns");
+    constexpr int NQ = (R + 4) / 4;                    // quads of rows in the window of a pair of rows
+    constexpr bool OVER = 4 * NQ > R + 1;              // ... whose last one reaches beyond it
     constexpr int ROWS = P_TM + R - 1, RPI = 256 / P_QUADS, IT = (ROWS + RPI - 1) / RPI;   // a round of loads: RPI rows, four threads idle
-    constexpr int PLANE = ROWS * P_LD;                 // bf16 values of one part
+    constexpr int PLANE = ROWS * P_RS;                 // bf16 values of one part
     constexpr int NE = S + 7;                          // windows of a kernel row that hold a tap: first slot - SHIFT - ln = -7 .. S-1
     constexpr int XP = parts_of<T>();                  // parts of a value (WP: of a tap)
     __shared__ __align__(16) uint16_t xs[2][XP * PLANE];
@@ -142,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
         split2<XP>(v[2], v[3], b);
         if (lr < RPI && ((it + 1) * RPI <= ROWS || r < ROWS)) {
 #pragma unroll
-            for (int s = 0; s < XP; ++s) *reinterpret_cast<uint2 *>(to + s * PLANE + r * P_LD + lk) = make_uint2(a[s], b[s]);
+            for (int s = 0; s < XP; ++s) *reinterpret_cast<uint2 *>(to + s * PLANE + r * P_RS + lk) = make_uint2(a[s], b[s]);
         }
     };
     strip t{0, 0}, next{0, 0};
@@ -152,8 +164,9 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
         for (int it = 0; it < IT; ++it) fetch(t, it);     // in flight while the kernel is prepared
     }
 
-    // ---- the kernel's fragments: lane (ln, kg), slot t holds tap 8*kg + t - SHIFT - ln ----
-    frag8<bf16_t> tz[WP][R];
+    // ---- the kernel's fragments, quad q, chunk c: lane (ln, kg) is output row ln/8 of a pair and key ln%8 of a group, slot t the window's row
+    // 4q + kg and column 8c + t: tap (4q + kg - ln/8, 8c + t - SHIFT - ln%8) ----
+    frag8<bf16_t> tz[WP][NQ * 3];
     {
         constexpr int NT = (R * (S + 16) + 255) / 256;
         uint16_t *const table = xs[0], *const taps = table + WP * R * (NE + 1) * 8;   // [part][row][8 zeros, S taps, 8 zeros]
@@ -182,12 +195,16 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
             *reinterpret_cast<u16x8 *>(table + e * 8) = win;
         }
         __syncthreads();
-        const int from = 8 * kg - SHIFT - ln + 7;
 #pragma unroll
         for (int s = 0; s < WP; ++s)
 #pragma unroll
-            for (int i = 0; i < R; ++i)
-                tz[s][i] = *reinterpret_cast<const frag8<bf16_t> *>(table + ((s * R + i) * (NE + 1) + (from >= 0 && from < NE ? from : NE)) * 8);
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const int i = 4 * q + kg - (ln >> 3), from = 8 * c - SHIFT - (ln & 7) + 7;
+                    const bool some = i >= 0 && i < R && from >= 0 && from < NE;
+                    tz[s][q * 3 + c] = *reinterpret_cast<const frag8<bf16_t> *>(table + ((s * R + (some ? i : 0)) * (NE + 1) + (some ? from : NE)) * 8);
+                }
         __syncthreads();
     }
     if (first < total) {
@@ -206,76 +223,99 @@ __global__ __launch_bounds__(256, 2) void conv2d_split(const T *__restrict__ x, 
         const bool more = id + per_plane < total, more2 = id + 2 * per_plane < total;
         const strip after = more2 ? next_strip() : t;   // (asked for either way: behind a branch around the loads their waits would be waits for all)
         const bool plain = inside(next);
-        // ---- four blocks of 16 x 16 per wavefront (16 rows x 64 keys), in halves of the kernel rows.  The operands of a kernel row are read
-        // while the row before is multiplied (the order is pinned).  Between the halves the next strip's vectors go to the other
-        // buffer, one by one, and those of the strip behind it are asked for ----
-        const uint16_t *xw = xs[n] + ((wave & 1) * 16 + ln) * P_LD + (wave >> 1) * 64 + kg * 8;
+        // ---- 32 rows x 32 keys per wavefront: four groups of 8 keys of 16 pairs of rows.  Chunk by chunk and quad by quad, each an operand of the
+        // three groups whose windows hold the chunk, read while the one before is multiplied (the order is pinned).  In between the next
+        // strip's vectors go to the other buffer, one by one, and those of the strip behind it are asked for ----
+        constexpr int NG = 4, NX = NG + 2, NSTEP = NX * NQ;
+        const uint16_t *const xw = xs[n] + (2 * ln + kg) * P_RS + wave * 32;
+        const int over = OVER ? (2 * ln + 4 * (NQ - 1) + kg < ROWS ? 0 : ROWS - 1 - (2 * ln + 4 * (NQ - 1) + kg)) * P_RS : 0;   // (rows that were not staged: one that was)
         frag8<bf16_t> f[2][XP];
         auto read = [&](int m) __attribute__((always_inline)) {
+            const int q = m % NQ;
 #pragma unroll
-            for (int s = 0; s < XP; ++s) f[m & 1][s] = *reinterpret_cast<const frag8<bf16_t> *>(xw + s * PLANE + m % R * P_LD + m / R * 16);
+            for (int s = 0; s < XP; ++s)
+                f[m & 1][s] = *reinterpret_cast<const frag8<bf16_t> *>(xw + s * PLANE + 4 * q * P_RS + m / NQ * 8 + (OVER && q == NQ - 1 ? over : 0));
         };
-        const int lower = causal ? (t.p0 + (wave & 1) * 16 + 15 - t.q0 - (wave >> 1) * 64) >> 4 : 3;   // last block that touches the triangle
+        const int lower = causal ? (t.p0 + P_TM - 1 - t.q0 - wave * 32) >> 3 : NG - 1;   // last group that touches the triangle
         // (address of a lane's results: a uniform base and a byte offset within the strip)
-        const int pl = (wave & 1) * 16 + ln, ql = (wave >> 1) * 64 + kg * 4;
+        const int pl = 2 * ln, ql = wave * 32 + kg * 4;
         char *const ybase = reinterpret_cast<char *>(yp + (int64_t)t.p0 * W + t.q0);
         const unsigned yoff = (unsigned)(pl * W + ql) * (unsigned)sizeof(T);
         const bool whole = t.p0 + P_TM <= H && t.q0 + P_TN <= W && (!causal || t.q0 + P_TN - 1 <= t.p0);
         float bad = 0.0f;   // not 0: a result that is not finite
+        // sums of the large products, fp32 data: of the middle chunk, which holds the taps next to the output's own position, and of the other two,
+        // so that a sum is rounded fewer times and that of a kernel near the identity once or twice; and of the small ones
+        constexpr bool TWO = XP == 3;
+        f32x4 big[NG], small[NG], rim_[TWO ? NG : 1], *const rim = TWO ? rim_ : big;
         read(0);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            f32x4 big{0.0f, 0.0f, 0.0f, 0.0f}, small0 = big, small1 = big;
+        for (int x = 0; x < NX; ++x) {
+            if (x < NG) big[x] = small[x] = rim[x] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                if (b <= lower) {
+            for (int q = 0; q < NQ; ++q) {
+                const int m = x * NQ + q;
+                if (x - 2 <= lower) {
+                    if (m + 1 < NSTEP) read(m + 1);
+                    // part ws of the taps times part s of the values, for the groups that take this chunk
+                    auto products = [&](f32x4 *acc, int ws, int s) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int i = half ? R / 2 : 0; i < (half ? R : R / 2); ++i) {
-                        const int m = b * R + i;
-                        if (m + 1 < 4 * R) read(m + 1);
-                        if constexpr (XP > 2) mma16(small0, tz[0][i], f[m & 1][2]);
-                        if constexpr (WP > 1) mma16(small1, tz[WP > 1 ? 1 : 0][i], f[m & 1][0]);
-                        if constexpr (XP > 1 && WP > 1) mma16(small0, tz[WP > 1 ? 1 : 0][i], f[m & 1][1]);
-                        if constexpr (XP > 1) mma16(small1, tz[0][i], f[m & 1][1]);
-                        if constexpr (WP > 2) mma16(small0, tz[WP > 2 ? 2 : 0][i], f[m & 1][0]);
-                        mma16(big, tz[0][i], f[m & 1][0]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-                constexpr int LEAD = 8 - IT;     // (not ahead of the last strip's stores: loads and stores complete on one counter)
-                const int it = b * 2 + half - LEAD;
-                if (it >= 0) {
-                    if (more) stage(next, plain, it, xs[n ^ 1]);
-                    fetch(after, it);
+                        for (int c = 2; c >= 0; --c)
+                            if (x - c >= 0 && x - c < NG) mma16(acc[x - c], tz[ws][q * 3 + c], f[m & 1][s]);
+                    };
+                    if constexpr (XP > 2) products(small, 0, 2);
+                    if constexpr (WP > 2) products(small, 2, 0);
+                    if constexpr (XP > 1 && WP > 1) products(small, 1, 1);
+#pragma unroll
+                    for (int c = 2; c >= 0; --c)
+                        if (x - c >= 0 && x - c < NG) mma16(c == 1 ? big[x - c] : rim[x - c], tz[0][q * 3 + c], f[m & 1][0]);
+                    if constexpr (WP > 1) products(small, 1, 0);
+                    if constexpr (XP > 1) products(small, 0, 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                constexpr int LEAD = NSTEP / 4;  // (not ahead of the last strip's stores: loads and stores complete on one counter)
+#pragma unroll
+                for (int it = 0; it < IT; ++it)
+                    if (m == LEAD + it * (NSTEP - LEAD) / IT) {
+                        if (more) stage(next, plain, it, xs[n ^ 1]);
+                        fetch(after, it);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
             }
-            // (stores of 16 rows x 64 bytes; the second half of a 128-byte line follows with the next block)
-            float v[4];
+            if (x == 3 || x == 5) {   // two groups are complete: a lane gets four keys of each row of its pair, stores of 16 rows x 64 bytes
+                const int w = x - 3;
+                float v[2][4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                v[u] = (big[u] + (small0[u] + small1[u])) * DOWN;
-                bad = fmaf(v[u], 0.0f, bad);
-            }
-            if (whole) {
-                asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));   // (one store, not one shared in part with the other branch)
-                quad4<T> o;
+                for (int g = 0; g < 2; ++g)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[u]);
-                __builtin_memcpy(ybase + yoff + b * 16 * (int)sizeof(T), &o, sizeof(o));
-            } else {
-                const int p = t.p0 + pl, q = t.q0 + ql + b * 16;
-                if (p < H && q < W && !(causal == 2 && q > p)) {
+                    for (int u = 0; u < 4; ++u) {
+                        v[g][u] = (big[w + g][u] + (TWO ? rim[w + g][u] + small[w + g][u] : small[w + g][u])) * DOWN;
+                        bad = fmaf(v[g][u], 0.0f, bad);
+                    }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) v[u] = causal && q + u > p ? 0.0f : v[u];
-                    store_quad<T>(yp + (int64_t)p * W, q, W, v);
+                for (int u = 0; u < 4; ++u) swap32(v[0][u], v[1][u]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (whole) {
+                        asm volatile("" : "+v"(v[h][0]), "+v"(v[h][1]), "+v"(v[h][2]), "+v"(v[h][3]));   // (one store, not one shared in part with the other branch)
+                        quad4<T> o;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[h][u]);
+                        __builtin_memcpy(ybase + (yoff + (unsigned)(h * W + w * 8) * (unsigned)sizeof(T)), &o, sizeof(o));
+                    } else {
+                        const int p = t.p0 + pl + h, q = t.q0 + ql + w * 8;
+                        if (p < H && q < W && !(causal == 2 && q > p)) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) v[h][u] = causal && q + u > p ? 0.0f : v[h][u];
+                            store_quad<T>(yp + (int64_t)p * W, q, W, v[h]);
+                        }
+                    }
                 }
             }
         }
         if (__builtin_amdgcn_ballot_w64(bad != 0.0f) != 0) {   // this lane's results that are not finite: multiply-adds, tap by tap
 #pragma unroll 1
             for (int e = opaque(0); e < 16; ++e) {
-                const int pe = t.p0 + pl, q = t.q0 + ql + (e >> 2) * 16 + (e & 3);
+                const int pe = t.p0 + pl + (e >> 2 & 1), q = t.q0 + ql + (e >> 3) * 16 + (e & 3);
                 if (pe >= H || q >= W || (causal && q > pe)) continue;
                 T *const at = yp + (int64_t)pe * W + q;
                 if (__builtin_isfinite(to_float(*at))) continue;
@@ -326,7 +366,7 @@ int launch_split(const void *x, const void *w, void *y, int64_t planes, int64_t 
 {
     const int64_t total = p_count(H, W, causal != 0);
     if (total > 0x3fffffffLL) return MTA_ERR_SHAPE;
-    int64_t per_plane = (2 * device_cu_count() + planes - 1) / planes;   // one round of resident workgroups
+    int64_t per_plane = (split_occ<T, WP, R>() * device_cu_count() + planes - 1) / planes;   // one round of resident workgroups
     if (per_plane > total) per_plane = total;
     hipLaunchKernelGGL((conv2d_split<T, WP, R, S, BWD>), dim3((unsigned)(planes * per_plane)), dim3(256), 0, st, (const T *)x, w, (T *)y, (int)C, (int)H,
                        (int)W, causal, in_scale, use_scale, w_dtype, (int)planes, (int)total, (int)per_plane);

@@ -155,24 +155,6 @@ template <typename T> __device__ __forceinline__ float dot2_io(uint32_t a, uint3
     }
 }
 
-// An exchange between whole rows of 16 lanes on the vector ALU (no LDS permute, so the LDS counter stays ours to count): 16: the odd
-// rows of a and the even rows of b change places; 32: the upper half of a and the lower half of b.
-__device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b)
-{
-    const u32x2_t r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0], b = r[1];
-}
-__device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b)
-{
-    const u32x2_t r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0], b = r[1];
-}
-__device__ __forceinline__ void swap32(float &a, float &b)
-{
-    uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
-    swap32(x, y);
-    a = __uint_as_float(x), b = __uint_as_float(y);
-}
 // Bit 3 of the lane index changes places with the choice between a and b: lanes 8-15 of every 16 get from b what lanes 0-7 hold there,
 // and lanes 0-7 from a what lanes 8-15 do.
 __device__ __forceinline__ void swap8(uint32_t &a, uint32_t &b)

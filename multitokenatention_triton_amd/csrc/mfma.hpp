@@ -44,6 +44,25 @@ __device__ __forceinline__ void mma16(f32x4 &c, const frag8<f16_t> &a, const fra
     c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
 
+typedef unsigned int lane_u2 __attribute__((ext_vector_type(2)));
+// An exchange between whole rows of 16 lanes on the vector ALU (no LDS permute, so the LDS counter stays ours to count): 16: the odd
+// rows of a and the even rows of b change places; 32: the upper half of a and the lower half of b.
+__device__ __forceinline__ void swap16(uint32_t &a, uint32_t &b)
+{
+    const lane_u2 r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void swap32(uint32_t &a, uint32_t &b)
+{
+    const lane_u2 r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void swap32(float &a, float &b)
+{
+    uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    swap32(x, y);
+    a = __uint_as_float(x), b = __uint_as_float(y);
+}
 template <typename T> __device__ __forceinline__ frag8<T> zero_frag()
 {
     frag8<T> f;
