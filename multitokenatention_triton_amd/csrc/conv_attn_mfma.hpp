@@ -273,8 +273,8 @@ template <int R, int SK> struct fused_geom {
 // long items all start early and the short ones fill the end of the grid.  Built on the host for every launch (a
 // counting sort over at most ITEM_TABLE_MAX items) and passed by value as a kernel argument; n = 0: no table, the kernel
 // cuts every query block's key range into chunks of jc_len blocks and walks the query blocks from the last to the first.
-// The chunks need not be equal: the first part of a query block's key range goes into long items (one extra key block
-// per item rebuilds the retained score columns, and an item costs a few microseconds to set up), the rest into short
+// The chunks need not be equal: the first part of a query block's key range goes into long items (an item costs a few
+// microseconds to set up), the rest into short
 // ones, which are started last and even out the end of the grid.
 struct item_table {
     int n;
@@ -339,8 +339,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
     // B1 H20 S2048 D128 53.2 -> 45.8 | 106 -> 88.6; without a conv B1 H12 S2048 D64 16.9 -> 14.4, S2560 23.8 -> 20.1.  per_xcd: the old deal, see
     // launch_mfma.
     // Work item = (batch*head, query block, chunk of jc_len key blocks).  The scores-only kernel splits the key
-    // range of a query block (its output columns are independent; a chunk starts one key block early to rebuild
-    // the retained halo columns), so that items are short and equal and the grid runs in several even rounds;
+    // range of a query block (its output columns are independent; a chunk starts with the 16 keys ahead of it, for
+    // the kept columns), so that items are short and equal and the grid runs in several even rounds;
     // the attention kernel accumulates over all keys and gets jc_len = all of them.
     // (a 32-bit division: the 64-bit ones that this took were half a microsecond of a workgroup's start)
     unsigned id = blockIdx.x;
@@ -449,8 +449,6 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         if (j_first > j_lo) j_lo = j_first;
         if (j_lo > j_end) return;
     }
-    // one key block earlier only fills the retained score columns (before the first one: the right pad, if any)
-    const int j_start = RAW ? j_lo : j_lo > 0 ? j_lo - 1 : (G::PWR > 0 ? -1 : 0);
     // What the start waits for is asked for at once, this wavefront's rows of Q and the kernel's taps ahead of the first blocks of K and V:
     // behind them, the taps waited for the blocks and Q was asked for when those had come.  With the 32-bit divisions above, scores
     // kernel, us: bf16 6x11 B2 H16 S1008 D64 22.3 -> 21.1, B4 H16 S1024 D128 40.6 -> 40.1, 7x7 B1 H16 S1024 D64 18.6 -> 17.7, B1 H16 S2048 D128 42.1 ->
@@ -475,8 +473,21 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         }
     }
     asm volatile("" : : : "memory");
-    issue_k(j_start, SCORES_ONLY ? B0 : KV);
-    if (!SCORES_ONLY) issue_v(j_start, KV + TILE);
+    // The score columns kept from the key block ahead of the first one are the last of its 16 keys: those rows of K go to their place in
+    // the buffer that the block behind the first gets (the zero-padded taps lie at its other end).  They used to be the by-product of a whole
+    // key block with a copy and barriers of its own: us, scores bf16 6x11 D128, in a loop, B1 H4 S200 8.1 -> 7.0, B1 H8 S512 8.8 -> 7.6, B2 H16
+    // S1008 26.7 -> 24.7, B1 H16 S2048 43.7 -> 41.9, B4 H16 S1024 44.9 -> 44.0, B2 H16 S4096 224 -> 221; shorter or longer items: no gain.
+    if constexpr (!RAW) {
+        static_assert((R + 2) * G::WZ_LD <= (F_BK - 16) * D && 64 / CPR <= 16 && F_NT / CPR >= 16, "16 rows of K beside the taps; whole wavefronts copy them");
+        const int first = (j_lo - 1) * F_BK + G::PWR, row = kv_row0 + (ROUNDS - 1) * (F_NT / CPR);
+        if (__builtin_amdgcn_readfirstlane(row) >= F_BK - 16) {
+            const int key = first + row < 0 ? 0 : (first + row >= S ? S - 1 : first + row);
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(Kp + (kv_off0 + (key - kv_row0) * D)),
+                                             (lds_void_t *)(wz + ((ROUNDS - 1) * F_NT + wave * 64) * 8), 16, 0, 0);
+        }
+    }
+    issue_k(j_lo, SCORES_ONLY ? B0 : KV);
+    if (!SCORES_ONLY) issue_v(j_lo, KV + TILE);
 
     if constexpr (!RAW) {
     // zero the score tile once (the columns kept from the key block before the first one; 15 taps: columns nobody writes)
@@ -514,6 +525,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         }
         fmax_w = __builtin_amdgcn_readfirstlane(m);
     }
+    __builtin_amdgcn_s_waitcnt(0);   // this wavefront's 16 rows of K, the first blocks
     __syncthreads();
 
     // The conv's taps as operands: product row m = ln is the output of row m/8 of the pair and key m%8 of the group; a slot that holds column
@@ -586,6 +598,46 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
     }
     const int crow = q0 - G::HR + pair_row + (kg >> 1);   // this lane's row of the sequence, from the conv to the probabilities
 
+    // four scores of row block rb, keys col .. col + 3, as the tile holds them
+    auto score4 = [&](int rb, f32x4 a, int col, bool masked, uint32_t &lo, uint32_t &hi) __attribute__((always_inline)) {
+        lo = pack2<T>(a[0], a[1]), hi = pack2<T>(a[2], a[3]);
+        if (SCORES_ONLY) {  // MTA scales the scores before the conv, in the I/O dtype: round, scale, round again
+            float a0, a1, a2, a3;
+            unpack2<T>(lo, a0, a1);
+            unpack2<T>(hi, a2, a3);
+            lo = pack2<T>(a0 * scale, a1 * scale);
+            hi = pack2<T>(a2 * scale, a3 * scale);
+        }
+        if (masked) {
+            MTA_KEEP_BRANCH();
+            const int lim = causal ? (prow[rb] < S - 1 ? prow[rb] : S - 1) : S - 1;  // last key kept
+            const int first = BAND ? (flo[rb] > 0 ? flo[rb] : 0) : 0;  // first key kept
+            if (col < first || col > lim) lo &= 0xffff0000u;
+            if (col + 1 < first || col + 1 > lim) lo &= 0x0000ffffu;
+            if (col + 2 < first || col + 2 > lim) hi &= 0xffff0000u;
+            if (col + 3 < first || col + 3 > lim) hi &= 0x0000ffffu;
+        }
+    };
+    if constexpr (!RAW) {   // the kept columns: scores of the last 16 keys of the block ahead of the first
+        f32x4 sacc[RB];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const frag8<T> kf = *reinterpret_cast<const frag8<T> *>(wz + (F_BK - 16 + ln) * D + (((ks * 4 + kg) ^ (ln & (CPR - 1))) * 8));
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                if (ks == 0) sacc[rb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                mma16(sacc[rb], kf, qf[rb][ks]);
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            uint32_t lo, hi;
+            score4(rb, sacc[rb], (j_lo - 1) * F_BK + G::PWR + F_BK - 16 + kg * 4, true, lo, hi);
+            *reinterpret_cast<uint2 *>(tile + trow[rb] * G::SLD + G::KEPT + F_BK - 16 + kg * 4) = make_uint2(lo, hi);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+
     auto plain = [&](int j) {
         const int cbase = j * F_BK + G::PWR;
         return j >= 0 && cbase + F_BK <= S && (!causal || cbase + F_BK - 1 <= pmin) && (!BAND || cbase >= fmax_w);
@@ -644,24 +696,8 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) {
                     const f32x4 a = sacc[cb & 1][rb];
-                    uint32_t lo = pack2<T>(a[0], a[1]), hi = pack2<T>(a[2], a[3]);
-                    if (SCORES_ONLY) {  // MTA scales the scores before the conv, in the I/O dtype: round, scale, round again
-                        float a0, a1, a2, a3;
-                        unpack2<T>(lo, a0, a1);
-                        unpack2<T>(hi, a2, a3);
-                        lo = pack2<T>(a0 * scale, a1 * scale);
-                        hi = pack2<T>(a2 * scale, a3 * scale);
-                    }
-                    if (!s_plain) {
-                        MTA_KEEP_BRANCH();
-                        const int col = cbase + cb * 16 + kg * 4;
-                        const int lim = causal ? (prow[rb] < S - 1 ? prow[rb] : S - 1) : S - 1;  // last key kept
-                        const int first = BAND ? (flo[rb] > 0 ? flo[rb] : 0) : 0;  // first key kept
-                        if (col < first || col > lim) lo &= 0xffff0000u;
-                        if (col + 1 < first || col + 1 > lim) lo &= 0x0000ffffu;
-                        if (col + 2 < first || col + 2 > lim) hi &= 0xffff0000u;
-                        if (col + 3 < first || col + 3 > lim) hi &= 0x0000ffffu;
-                    }
+                    uint32_t lo, hi;
+                    score4(rb, a, cbase + cb * 16 + kg * 4, !s_plain, lo, hi);
                     // Two 16-key blocks go to the tile together.  A lane holds keys 4kg..4kg+3 of each; after the
                     // exchange between neighbouring lane groups (even groups give their second block's part and take
                     // the neighbour's first block's part) it holds 8 consecutive keys of one block: one 16-byte write
@@ -710,7 +746,6 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         // (attention kernel: nobody reads K(j) any more, the next V block may land in its buffer)
         if (!SCORES_ONLY && j < j_end) issue_v(j + 1, Vn);
-        if (j < j_lo) return;
 
         // ---- conv (products over the score tile) -> global (scores only) / -> online softmax ----
         // A product needs taps from registers and an operand from LDS, and a wavefront that waits for each operand where it is used
@@ -1035,7 +1070,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         }
     };
     if constexpr (SCORES_ONLY) {
-        for (int j = j_start;;) {  // block(tag, j, K(j), V(j), where K(j+1) goes, where V(j+1) goes)
+        for (int j = j_lo;;) {  // block(tag, j, K(j), V(j), where K(j+1) goes, where V(j+1) goes)
             if (plain(j)) block(std::true_type{}, j, B0, B0, B1, B1);
             else block(std::false_type{}, j, B0, B0, B1, B1);
             if (++j > j_end) break;
@@ -1045,7 +1080,7 @@ __global__ __launch_bounds__(64 * NW, SCORES_ONLY && R <= 7 ? QK_OCC : 2) void c
         }
     } else {
         int kb = 0, vb = TILE, nb = 2 * TILE;   // where K(j) and V(j) are, and the third buffer
-        for (int j = j_start; j <= j_end; ++j) {
+        for (int j = j_lo; j <= j_end; ++j) {
             block(std::false_type{}, j, KV + kb, KV + vb, KV + nb, KV + kb);
             const int k_next = nb;
             nb = vb;
@@ -1162,8 +1197,7 @@ int launch_mfma(const void *q, const void *k, const void *v, const void *w, void
             for (int j0 = 0; j0 < nk && ok;) {
                 const int len = j0 < nlong ? std::min(big, nlong - j0) : std::min(small, nk - j0);
                 if (n >= ITEM_TABLE_MAX) { ok = false; break; }
-                // what the kernel visits: one key block earlier rebuilds the retained columns (ahead of the first: the right pad)
-                lens[n] = len + (!RAW && (j0 > 0 || G::PWR > 0) ? 1 : 0);
+                lens[n] = len;
                 items[n++] = (uint32_t)qb | ((uint32_t)j0 << 11) | ((uint32_t)len << 22);
                 j0 += len;
             }
