@@ -7,12 +7,19 @@
 // What the operator-by-operator pipeline writes to memory and reads back between the two stages - c, a whole
 // (N,C,H,W) tensor - stays in registers here.
 //
-// A workgroup of four wavefronts owns a 32 x 64 tile of positions for all 16 heads of a mixing group; wavefront w owns
-// row block w & 1 (16 rows) and key half w >> 1 (32 keys = two 16 x 16 blocks).  Head by head, the tile's window
+// A workgroup of eight wavefronts owns a 32 x 64 tile of positions for all 16 heads of a mixing group; wavefront w owns
+// row block w & 1 (16 rows) and key quarter w >> 1 (16 keys).  Head by head, the tile's window
 // ((32+R-1) rows x 80 keys) is copied global -> LDS asynchronously one head ahead (two buffers, one barrier per head)
 // and convolved as in conv2d_mfma: per block and kernel row one v_mfma_f32_16x16x32 of a Toeplitz fragment with 16
 // contiguous bytes of a staged row per lane.  The rounded results of all 16 heads stay in the lane that computed them
-// (64 registers).
+// (32 registers).
+// What bounds it is the chain of steps that a tile is - per head a wait, a barrier, fragments, operands, products: without any products it
+// takes 150 us of 160 (fp16 7x7 B1 H16 S4096) - and then memory.  So a step is split over eight wavefronts where four took two blocks each:
+// 16 wavefronts per CU of 128 registers, which takes the addresses of rare work (the table, the weights) formed where it is done, the
+// mixing's products four at a time and two operands in flight at 7x7.  And the results are stored as ordinary data: tensors of which the
+// lower triangle fits the caches are read there by the next kernel, larger ones do not mind.  us of the forward (D64, D128 at S4096),
+// four wavefronts | eight | ordinary stores: fp16 7x7 B1 H16 S2048 160 | 139 | 132, B3 H16 S1024 129 | 116 | 114, S4096 488 | 461 | 459, 5x5 S2048 151 |
+// 132 | 125, bf16 3x3 groups of 4 B1 H32 S2048 244 | 230 | 218, groups of 2 B1 H16 S3000 286 | 277 | 239, fp16 7x7 B2 H16 S4096 889 | 889 (last two).
 //
 // Toeplitz fragments change with every head.  A lane's fragment of kernel row i is eight consecutive taps starting at
 // an offset that depends on the lane only through e = 8*(lane/16) - lane%16, and is non-zero for S+7 values of e: the
@@ -43,15 +50,15 @@ using namespace mta;
 // diagonal (never written)
 __device__ __align__(16) unsigned int xm_zero16[4];
 
-constexpr int X_NW = 4;            // wavefronts per workgroup
+constexpr int X_NW = 8;            // wavefronts per workgroup
 constexpr int X_WT = 64 * X_NW;    // threads per workgroup
 constexpr int X_TM = 32;           // tile rows
 constexpr int X_TN = 64;           // tile keys
-constexpr int X_HALF = X_TN / 2;   // keys per wavefront
+constexpr int X_HALF = X_TN / (X_NW / 2); // keys per wavefront
 constexpr int X_NCB = X_HALF / 16; // 16 x 16 blocks per wavefront
 constexpr int X_HG = 16;           // heads mixed together
 constexpr int X_RPB = X_TN / X_TM; // tile rows per X_TN x X_TN block of the lower triangle
-static_assert(X_RPB == 2 && X_NCB == 2, "tile geometry");
+static_assert(X_RPB == 2 && X_NCB == 1, "tile geometry");
 
 template <int R, int S> struct xgeom {
     static constexpr int PADW = (S - 1) / 2;
@@ -117,7 +124,7 @@ constexpr int X_ROT = 19;  // by how many workgroups the dealing of an XCD's ite
 template <int R> constexpr int x_occ() { return 2; }  // persistent workgroups per CU
 
 template <typename T, int R, int S, int GROUP>
-__global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__restrict__ x, const T *__restrict__ wc,
+__global__ __launch_bounds__(X_WT, (x_occ<R>() * X_NW / 4)) void conv_mix16_mfma(const T *__restrict__ x, const T *__restrict__ wc,
                                                                    const T *__restrict__ wm, T *__restrict__ y, int C, int H,
                                                                    int W, int causal, int fill_upper, int tiles_n, int ipp,
                                                                    xm_split split, int nw, int tri)
@@ -143,7 +150,7 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
     static_assert(RAW_BYTES % 16 == 0 && NRAW <= X_WT, "the kernels of a group are whole 16-byte vectors, one per thread");
     constexpr unsigned RAW_OFF = 16;                             // where the raw kernels lie in the staging area while the table is built
     static_assert(RAW_BYTES + 32 <= STG_BYTES, "the raw kernels and what is read around them lie in the staging area");
-    constexpr int NST = 16;                                      // store instructions per wavefront and item
+    constexpr int NST = 64 / X_NW;                               // store instructions per wavefront and item
     static_assert((NBUF - 2) * STAGE_IT + NST <= 63, "vmcnt field");
     __shared__ __align__(16) T tiles[NBUF * BUF];
     __shared__ __align__(16) u32x4 table[TAB_VECS + 1];          // (+ one vector of zeros)
@@ -246,11 +253,13 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
     auto build_table = [&](int g) {
         wg_barrier();  // every wavefront is done with the staging area and with the previous group's table
         u32x4 rawv = {0u, 0u, 0u, 0u};
-        if (tid < NRAW) rawv = *reinterpret_cast<const u32x4 *>(wc + (int64_t)g * X_HG * (R * S) + tid * VEC);
-        if (tid < NRAW) lds_store16(stage_lds + RAW_OFF + 16u * (unsigned)tid, rawv);
+        const int tid_ = opaque(tid);   // (rare: nothing of it is to be kept in registers outside)
+        if (tid_ < NRAW) rawv = *reinterpret_cast<const u32x4 *>(wc + (int64_t)g * X_HG * (R * S) + tid_ * VEC);
+        if (tid_ < NRAW) lds_store16(stage_lds + RAW_OFF + 16u * (unsigned)tid_, rawv);
         lds_wait();
         wg_barrier();
-        for (int v = tid; v < TAB_VECS; v += X_WT) {
+#pragma unroll 1
+        for (int v = tid_; v < TAB_VECS; v += X_WT) {
             const int hi = v / G::NVEC, ve = v - hi * G::NVEC;
             // (taps ve-7 .. ve of the row, read where they would lie: the 16 bytes ahead of the kernels and what follows
             // them are part of the staging area, and what is read outside the row is not used)
@@ -270,7 +279,7 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
             }
             lds_store16(table_lds + 16u * (unsigned)v, u32x4{pk[0], pk[1], pk[2], pk[3]});
         }
-        if (tid == 0) lds_store16(table_lds + 16u * (unsigned)TAB_VECS, u32x4{0u, 0u, 0u, 0u});
+        if (tid_ == 0) lds_store16(table_lds + 16u * (unsigned)TAB_VECS, u32x4{0u, 0u, 0u, 0u});
         lds_wait();
         wg_barrier();  // the table is complete; the staging area is free again
     };
@@ -303,10 +312,10 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
         if (c_kind != 0) {  // wholly above the diagonal: +0 on request, for all 16 heads
             if (c_kind == 1) {
                 const u4 z = {0u, 0u, 0u, 0u};
-                const int r = tid >> 3, cv = (tid & 7) * VEC;
+                const int tid = opaque((int)threadIdx.x), r = (tid >> 3) & (X_TM - 1), cv = (tid & 7) * VEC;
                 if (p0 + r < H && q0 + cv < W) {
 #pragma unroll
-                    for (int h = 0; h < X_HG; ++h) __builtin_nontemporal_store(z, reinterpret_cast<u4 *>(yg + h * HW + (int64_t)(p0 + r) * W + q0 + cv));
+                    for (int h = tid / (8 * X_TM); h < X_HG; h += X_WT / (8 * X_TM)) __builtin_nontemporal_store(z, reinterpret_cast<u4 *>(yg + h * HW + (int64_t)(p0 + r) * W + q0 + cv));
                 }
                 prev_st = -1;
             }
@@ -324,10 +333,11 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
             build_table(cur_g);
             // weight fragment of the mixing: lane (output head ln, group kg) holds wm[o][4kg .. 4kg+3]; of groups within a lane: wm[4kg+v]
             // [4kg .. 4kg+3], what lies outside the groups unused
+            const int lane_ = opaque(lane), kg_ = lane_ >> 4;
 #pragma unroll
             for (int v = 0; v < NWF; ++v) {
-                const int o = GROUP == X_HG ? ln : kg * 4 + v;
-                wf[v] = *reinterpret_cast<const xm_u2 *>(wm + (int64_t)(cur_g * X_HG + o) * C + cur_g * X_HG + kg * 4);
+                const int o = GROUP == X_HG ? lane_ & 15 : kg_ * 4 + v;
+                wf[v] = *reinterpret_cast<const xm_u2 *>(wm + (int64_t)(cur_g * X_HG + o) * C + cur_g * X_HG + kg_ * 4);
             }
 #pragma unroll
             for (int v = 0; v < NWF; ++v) asm volatile("s_waitcnt vmcnt(0)" : "+v"(wf[v]) : : "memory");  // (rare: everything in flight is waited for here)
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
 
             f32x4 acc[X_NCB];
             const unsigned xa = tile_lds + (unsigned)((rb0 + ln) * LD + kh * X_HALF + kg * 8) * sizeof(T);
-            constexpr int NPROD = X_NCB * R, NLD = (NPROD - 1) < 8 ? (NPROD - 1) : 8, NSLOT = NLD + 1;
+            constexpr int NPROD = X_NCB * R, NLD = R >= 7 ? 2 : R - 1 < 4 ? R - 1 : 4, NSLOT = NLD + 1;   // (what the registers leave room for)
             u32x4 ring[NSLOT];
             auto issue = [&](auto ic) __attribute__((always_inline)) {
                 constexpr int nn = decltype(ic)::value;
@@ -467,43 +477,47 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
                 cres[8 + v][cb][part] = s[0]; cres[12 + v][cb][part] = s[1];
             }
             // cres[4kq + v][cb][part] now: head 4kg + v, keys 4kq + 2 part, +1 of the block
-            f32x4 macc[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int kq = j >> 2, t = j & 3, part = t >> 1;
-                const unsigned sel = (t & 1) ? 0x07060302u : 0x05040100u;
-                const xm_u2 col = {__builtin_amdgcn_perm(cres[4 * kq + 1][cb][part], cres[4 * kq + 0][cb][part], sel),
-                                   __builtin_amdgcn_perm(cres[4 * kq + 3][cb][part], cres[4 * kq + 2][cb][part], sel)};
-                if constexpr (GROUP == X_HG) {
-                    macc[j] = xm_mma16(T{}, wf[0], col);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        if constexpr (GROUP == 4) macc[j][v] = xm_dot2(T{}, wf[v][1], col[1], xm_dot2(T{}, wf[v][0], col[0], 0.0f));
-                        else macc[j][v] = xm_dot2(T{}, wf[v][v / 2], col[v / 2], 0.0f);
-                    }
-                }
-            }
             const int qb = q0 + kh * X_HALF + cb * 16;
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
+            for (int u = 0; u < 8; ++u) {   // keys 2u, 2u + 1 of the block
+                f32x4 macc[2];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    uint32_t o = pack2<T>(macc[2 * u][v], macc[2 * u + 1][v]);
+                for (int t2 = 0; t2 < 2; ++t2) {
+                    const int kq = u >> 1, part = u & 1;
+                    const unsigned sel = t2 ? 0x07060302u : 0x05040100u;
+                    const xm_u2 col = {__builtin_amdgcn_perm(cres[4 * kq + 1][cb][part], cres[4 * kq + 0][cb][part], sel),
+                                       __builtin_amdgcn_perm(cres[4 * kq + 3][cb][part], cres[4 * kq + 2][cb][part], sel)};
+                    if constexpr (GROUP == X_HG) {
+                        macc[t2] = xm_mma16(T{}, wf[0], col);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            if constexpr (GROUP == 4) macc[t2][v] = xm_dot2(T{}, wf[v][1], col[1], xm_dot2(T{}, wf[v][0], col[0], 0.0f));
+                            else macc[t2][v] = xm_dot2(T{}, wf[v][v / 2], col[v / 2], 0.0f);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    uint32_t o = pack2<T>(macc[0][v], macc[1][v]);
                     if (cross) {
                         if (qb + 2 * u > prow) o &= 0xffff0000u;
                         if (qb + 2 * u + 1 > prow) o &= 0x0000ffffu;
                     }
                     outp[cb][v][u] = o;
                 }
+                if (u & 1) __builtin_amdgcn_sched_barrier(0);   // (all products first would take 64 registers)
+            }
         }
 
         // ---- stores through LDS: round v carries output head 4*og + v of every lane group og ----
         // staging: [og][row 0..31][8 slots of 16 bytes], slot index XOR ((row >> 1) & 7)
+        const int lane = opaque((int)threadIdx.x & 63), ln = lane & 15, kg = lane >> 4;
         const int srow = rb0 + ln;
         const unsigned wbase = stage_lds + (unsigned)((kg * X_TM + srow) * (X_TN * (int)sizeof(T)));
         const int wsw = (srow >> 1) & 7;
-        const int r_l = lane >> 3, c_l = lane & 7;  // reader: row r_l + 8k, slot c_l, lane group `wave`
+        const int r_l = (wave >> 2) * (X_TM * 4 / X_NW) + (lane >> 3), c_l = lane & 7, og = wave & 3;  // reader: row r_l + 8k, slot c_l, lane group og
+        constexpr int NK = NST / 4;
         // the tile's outputs all lie inside the plane and are all wanted: unconditional stores, NST per wavefront
         const bool full_out = p0 + X_TM <= H && q0 + X_TN <= W && (!cross || fill_upper);
 #pragma unroll
@@ -513,31 +527,32 @@ __global__ __launch_bounds__(X_WT, x_occ<R>()) void conv_mix16_mfma(const T *__r
             for (int cb = 0; cb < X_NCB; ++cb)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
-                    const int slot = kh * 4 + cb * 2 + k;
+                    const int slot = kh * (X_HALF / 8) + cb * 2 + k;
                     lds_store16(wbase + 16u * (unsigned)(slot ^ wsw),
                                 u32x4{outp[cb][v][4 * k], outp[cb][v][4 * k + 1], outp[cb][v][4 * k + 2], outp[cb][v][4 * k + 3]});
                 }
             lds_wait();
             wg_barrier();
-            u32x4 val[4];
+            u32x4 val[NK];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < NK; ++k) {
                 const int row = k * 8 + r_l;
-                val[k] = lds_load16(stage_lds + (unsigned)((wave * X_TM + row) * (X_TN * (int)sizeof(T))) +
+                val[k] = lds_load16(stage_lds + (unsigned)((og * X_TM + row) * (X_TN * (int)sizeof(T))) +
                                     16u * (unsigned)(c_l ^ ((row >> 1) & 7)));
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(val[0]), "+v"(val[1]), "+v"(val[2]), "+v"(val[3]) : : "memory");
-            T *yh = yg + (int64_t)(wave * 4 + v) * HW;
+#pragma unroll
+            for (int k = 0; k < NK; ++k) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(val[k]) : : "memory");
+            T *yh = yg + (int64_t)(og * 4 + v) * HW;
             if (full_out) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    __builtin_nontemporal_store(val[k], reinterpret_cast<u32x4 *>(yh + (int64_t)(p0 + k * 8 + r_l) * W + q0 + c_l * VEC));
+                for (int k = 0; k < NK; ++k)
+                    *reinterpret_cast<u32x4 *>(yh + (int64_t)(p0 + k * 8 + r_l) * W + q0 + c_l * VEC) = val[k];
             } else {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
+                for (int k = 0; k < NK; ++k) {
                     const int row = p0 + k * 8 + r_l, col = q0 + c_l * VEC;
                     if (row < H && col < W && (!causal || fill_upper || col <= row))
-                        __builtin_nontemporal_store(val[k], reinterpret_cast<u32x4 *>(yh + (int64_t)row * W + col));
+                        *reinterpret_cast<u32x4 *>(yh + (int64_t)row * W + col) = val[k];
                 }
             }
         }

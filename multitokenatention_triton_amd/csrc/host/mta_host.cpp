@@ -43,21 +43,18 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 }
 
 // Whether conv + mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
-// heads at about 20 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other.
-// us of the forward (H16 D64 fp16, the post-softmax conv 3x3 / 7x7), one kernel | two: 272 tiles (B1 S1024) 68.7 | 60.2 / 72.8 | 64.5,
-// 544 (B2 S1008) 101.0 | 88.3 / 106.4 | 95.6, 600 (B1 S1536) 109.9 | 91.9 / 115.9 | 98.3, 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3,
-// 840 (B2 S1280) 126.1 | 123.9 / 131.8 | 133.3, 1056 (B1 S2048) 155.0 | 164.5 / 161.5 | 175.5, 1088 (B4 S1024) 149.8 | 171.4 /
-// 156.9 | 182.6; the runs of one side differ by up to 2.
-// Groups of 2 or 4 heads: 1056 tiles 57 | 60 / 64 | 62, 2112 (B2 S2048) 92 | 120 / 98 | 125, 4160 (B1 S4096) 148 | 232 / 163 | 238.
-// Tiles for one round that is nearly full and surely fits are as good for them (what is left to spare takes up an uneven deal over the
-// XCDs; the whole forward, B H16 D64, bf16 groups of 4 / fp16 groups of 2, 3x3): 420 tiles (B1 S1280) 79.2 | 77.3 / 78.1 | 77.4, (B2 S896)
-// 81.9 | 81.6 / 81.1 | 82.5, 440 (B4 S640) 84.5 | 84.9 / 84.5 | 89.1, 448 (B8 S448) 87.9 | 92.4 / 89.3 | 99.8, 480 (B2 S960) 83.6 | 84.7 /
-// 83.2 | 86.1, but 506 (B1 S1408) 93.9 | 83.5 / 92.1 | 83.4.  The dense 16 heads gain nothing there: 420 (B1 S1280) 80.0 | 77.5, 440 85.1 | 81.1,
-// 448 85.9 | 85.2, 480 81.9 | 80.5, 506 95.2 | 86.1, 7x7 at 506 100.9 | 90.4.
+// heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or one
+// round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs).
+// us of the forward (H16 D64, the pre-softmax conv 6x11), two kernels | one, fp16 dense 3x3 / 7x7 after the softmax / bf16 groups of 4, 3x3:
+// 72 tiles (B1 S512) 37.8 | 44.2 / 38.6 | 46.3 / 36.1 | 36.2, 272 (B1 S1024) 61.6 | 62.1 / 63.6 | 65.7 / 65.7 | 70.6, 342 (B1 S1152) 66.6 | 67.0 / 69.4 |
+// 70.6 / 69.8 | 70.6, 420 (B1 S1280) 74.8 | 72.8 / 78.0 | 76.6 / 74.9 | 77.0, 420 (B2 S896) 74.7 | 74.5 / 78.1 | 78.1 / 78.8 | 79.2, 440 (B4 S640)
+// 78.7 | 75.0 / 82.8 | 79.0 / 81.5 | 78.0, 506 (B1 S1408) 83.3 | 85.1 / 87.3 | 90.8 / 81.5 | 87.6, 544 (B2 S1008) 79.9 | 80.4 / 84.1 | 86.4 /
+// 85.0 | 84.7, 600 (B1 S1536) 90.1 | 94.9 / 94.3 | 100 / 89.9 | 98.2, 630 (B3 S896) 91.4 | 95.8 / 96.0 | 101 / 92.9 | 98.7.  Beyond, with the kernel as
+// it was at 20 us a tile: 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3 one | two, 1056 (B1 S2048) 155 | 165 / 162 | 176; now 816 7x7 114, 1056 132.
 bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only, bool dense)
 {
     const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64, tiles = planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk);
-    return tiles >= 800 || (!dense && tiles >= 430 && tiles <= 490);
+    return tiles >= 800 || (tiles >= (dense ? 410 : 430) && tiles <= 490);
 }
 
 int64_t lcm(int64_t a, int64_t b)
