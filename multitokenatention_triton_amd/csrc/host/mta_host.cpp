@@ -43,8 +43,9 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 }
 
 // Whether conv + mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
-// heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or one
-// round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs).
+// heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or, for
+// groups of 2 or 4 heads, one round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs); the dense 16
+// heads gain little there.
 // us of the forward (H16 D64, the pre-softmax conv 6x11), two kernels | one, fp16 dense 3x3 / 7x7 after the softmax / bf16 groups of 4, 3x3:
 // 72 tiles (B1 S512) 37.8 | 44.2 / 38.6 | 46.3 / 36.1 | 36.2, 272 (B1 S1024) 61.6 | 62.1 / 63.6 | 65.7 / 65.7 | 70.6, 342 (B1 S1152) 66.6 | 67.0 / 69.4 |
 // 70.6 / 69.8 | 70.6, 420 (B1 S1280) 74.8 | 72.8 / 78.0 | 76.6 / 74.9 | 77.0, 420 (B2 S896) 74.7 | 74.5 / 78.1 | 78.1 / 78.8 | 79.2, 440 (B4 S640)
@@ -54,7 +55,7 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only, bool dense)
 {
     const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64, tiles = planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk);
-    return tiles >= 800 || (tiles >= (dense ? 410 : 430) && tiles <= 490);
+    return tiles >= 800 || (!dense && tiles >= 430 && tiles <= 490);
 }
 
 int64_t lcm(int64_t a, int64_t b)
