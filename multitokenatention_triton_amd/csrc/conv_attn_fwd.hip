@@ -412,7 +412,7 @@ extern "C" int mta_conv_attn_fwd(const void *q, const void *k, const void *v, co
     return mta_conv_attn_fwd_lse(q, k, v, w, o, nullptr, B, H, S, D, R, Sk, causal, scale, io_dtype, w_dtype, stream);
 }
 
-// kernel sizes with a scores-only instance (the cases of dispatch_mfma<.., true>)
+// kernel sizes that the 16-bit scores kernel has an instance for (the cases of dispatch_scores)
 static bool scores_instance(int R, int Sk)
 {
     return (R == 3 && (Sk == 3 || Sk == 5)) || (R == 5 && (Sk == 5 || Sk == 7)) || (R == 6 && Sk == 11) ||

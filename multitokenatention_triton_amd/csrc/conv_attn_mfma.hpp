@@ -39,6 +39,10 @@ namespace {
 // D128 1067 -> 990 (executed 1.0 PFLOP/s; an 8192^3 library product reaches 1.08), 3x3 B1 H32 S4096 D128 276 -> 246, 7x7 B1 H16
 // S2048 D128 98.9 -> 87.0, 6x11 B1 H8 S2048 D64 78.8 -> 66.7, 5x5 B2 H32 S4096 D64 378 -> 341; fp16 7x9 B4 H12 S2048 D64 120 -> 93,
 // 11x15 B1 H32 S4096 D128 595 -> 360.
+// A launch without the scores kernel's table of work items (3 KB of kernel arguments) and an item that is its query block, of which the table's
+// search found the number by walking: B1 H32 S8192 D128 970 -> 957, 7x7 B1 H24 S2048 D128 80.9 -> 76.3, 3x3 B1 H32 S1024 D64 28.2 -> 27.0, B1 H4 S100
+// 7.8 -> 7.1.  The columns ahead of the first key block from 16 keys instead of a key block (as the scores kernel does): 26.5, 77.9, and on large
+// grids 1 % slower (3x3 B1 H32 S4096 D128 238 | 239): not kept.
 constexpr int F_SLD = 80;  // score-tile row stride (elements): exactly the retained columns + one key block.  With this one a fragment
                            // read (16 consecutive rows x 64 bytes) is free of bank conflicts as it is: the LDS serves
                            // lanes 0-7 together with lanes 24-31 (8-15 with 16-23, ...), and rows 160 bytes apart put
