@@ -18,7 +18,8 @@
 // One kernel row and sixteen keys per product (11 products and as many operands per 256 outputs, 9 and 4 now) -> this, fp32 11x15, whole
 // rows: 16 planes of 512^2 19.9 -> 18.9, 12 of 801^2 31.1 -> 28.8, 16 of 1024^2 41.3 -> 37.9, 32 of 1024^2 66.6 -> 60.5, 16 of 2048^2 142 either way;
 // 16-bit data, with as many workgroups per CU as their registers allow (split_occ) where two ran: bf16 16 of 1001^2 7x7 21.7 -> 20.6, 11x15 23.3 -> 21.7,
-// fp16 6x11 27.4 -> 23.8, with fp32 weights 16 of 1024^2 bf16 6x11 23.0 -> 20.6, 7x9 23.8 -> 20.1, fp16 6x11 27.7 -> 29.0, 7x9 29.1 -> 28.9 (177 registers: two).
+// fp16 6x11 27.4 -> 23.8, with fp32 weights 16 of 1024^2 bf16 6x11 23.0 -> 20.6, 7x9 23.8 -> 20.1, fp16 6x11 29.9 -> 27.1,
+// 7x9 30.1 -> 25.8, 16 of 2048^2 76.5 -> 74, 80.3 -> 70.
 // us, conv2d_rows -> the former, fp32: lower triangle 16 planes of 512^2 23 -> 18.5, 12 of 801^2 32 -> 28.5, 16 of 1024^2 58 -> 38, 32 of
 // 1024^2 105 -> 68, 16 of 2048^2 177 -> 128; whole rows 31 -> 20, 34 -> 31, 86 -> 43, 152 -> 80, 260 -> 151.  Smaller kernels stay
 // there, lower triangle | whole rows: 7x9 16 of 1024^2 29.7 | 39.4 against 29.4 | 34.5 here, 16 of 512^2 13.9 | 16.4 against 15.3 |
@@ -68,8 +69,9 @@ inline int64_t p_count(int64_t H, int64_t W, int tri)
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
 // Workgroups per CU: a strip is a chain of loads, splitting, products and stores between two barriers, and what hides it is the other
-// workgroups.  The fewer parts, the fewer registers and the less LDS a workgroup takes.
-template <typename T, int WP, int R> constexpr int split_occ() { return parts_of<T>() == 1 && WP == 1 ? 4 : parts_of<T>() * WP <= 4 && R <= 7 ? 3 : 2; }
+// workgroups.  The fewer parts, the fewer registers and the less LDS a workgroup takes.  (fp16 data with three parts of a tap: 177 registers, of
+// which the third workgroup takes 9 - five values go to scratch memory and back - and gives 7 to 11 %, figures above: 29.0 and 28.9 with two.)
+template <typename T, int WP, int R> constexpr int split_occ() { return parts_of<T>() == 1 && WP == 1 ? 4 : parts_of<T>() * WP <= 6 && R <= 7 ? 3 : 2; }
 
 template <typename T, int WP, int R, int S, bool BWD>
 __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
