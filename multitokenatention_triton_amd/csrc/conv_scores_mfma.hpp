@@ -69,9 +69,6 @@ __device__ __forceinline__ uint32_t upper_half_of(uint32_t a, uint32_t b)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0xe4, 0xc, 0xf, false);   // (0xe4: every lane its own)
 }
-// NaN if one of them is
-__device__ __forceinline__ float max3_nan(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
-
 // The conv on the matrix cores.  A product (16x16x32) takes two query rows x eight keys of output (its 16 rows) for sixteen pairs of
 // query rows (its 16 columns): the pair's window has R + 1 rows, the eight keys' SK + 7 columns, and the 32 slots of the contraction
 // hold 8-column chunks of the window's rows, 8 slots a lane group.  6x11 needs 7 x 18 = 126 slots for 256 outputs, four products;
@@ -475,6 +472,7 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         const int cbase = j * F_BK + G::PWR;
         return j >= 0 && cbase + F_BK <= S && (!causal || cbase + F_BK - 1 <= pmin) && (!BAND || cbase >= fmax_w);
     };
+    float nan = 0.0f;   // NaN once a product of the key block has met a value that is not finite
     // PLAIN: the key block (its scores and its conv outputs) lies inside the sequence and on or below the diagonal
     // for all 32 rows of this wavefront: no masks and no per-sub-block tests (most blocks of a long sequence)
     auto block = [&](auto plain_tag, int j, const T *Kb, T *Kn) __attribute__((always_inline)) {
@@ -616,15 +614,8 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
                 }
             }
         };
-        float nan = 0.0f;           // NaN once one of this lane's results is
+        nan = 0.0f;
         uint32_t held[4][2];        // four groups, packed
-        // Rows of the conv's window that one row of a pair does not take meet taps 0, which an infinity or a NaN there turns into NaN: results
-        // that are NaN are formed again, tap by tap.  The value of the tile that tap (i, t) of the output in row `row` of the tile and key
-        // `q` of the block takes:
-        auto tile_value = [&](int row, int q, int i, int t) __attribute__((always_inline)) {
-            const int r_ = row - (R - 1) + i, col = q + t + G::SHIFT - G::C0;
-            return to_float(col >= 0 ? tile[r_ * G::SLD + col] : reinterpret_cast<const T *>(side)[r_ * 2 + col + 2]);
-        };
         // what happens to group w (rows crow, keys j*64 + 8w ..) once it is complete
         auto finish = [&](auto wc) __attribute__((always_inline)) {
             constexpr int w = decltype(wc)::value;
@@ -635,7 +626,9 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
             // merges them.  Marked non-temporal, each 64-byte half went to memory on its own and the write counter
             // read 1.38 times the bytes; the price of the merge is that the scores displace some of the head's K blocks
             // from the L2 - fetches 79 -> 196 MB per launch at the benchmark shape, 825 -> 736 MB in total, 4 % faster.)
-            nan = max3_nan(max3_nan(nan, a[0], a[1]), a[2], a[3]);
+            // (a value that is not finite reaches all results of its products, and each chunk the products of two groups, the last one those of
+            // the last group: one of four results of every other group tells)
+            if constexpr (w % 2 == 0 || w == NWIN - 1) nan = fmaf(a[0], 0.0f, nan);
             uint32_t lo = pack2<T>(a[0], a[1]), hi = pack2<T>(a[2], a[3]);
             if (!PLAIN && causal && j * F_BK + w * 8 + 7 > pmin) {  // the group touches the diagonal for some row
                 const int col = j * F_BK + w * 8 + (kg & 1) * 4;
@@ -708,28 +701,74 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         static_for<NWIN>([&](auto wc) __attribute__((always_inline)) {
             if constexpr (plan.last[decltype(wc)::value] + LAG >= NREAD) finish(wc);
         });
-        if (__builtin_amdgcn_ballot_w64(nan != nan) != 0) {
-            MTA_KEEP_BRANCH();
-            __builtin_amdgcn_s_waitcnt(0);   // the stores above come first
-            const int key = j * F_BK + opaque_lane(lane), row0_ = __builtin_amdgcn_readfirstlane(pair_row);
-#pragma unroll 1
-            for (int r_ = 0; r_ < 32; ++r_) {
-                const int tr_ = row0_ + r_, p_ = q0 - G::HR + tr_;
-                if (tr_ < G::HR || tr_ >= (wave + 1) * 32 || p_ >= S) continue;
-                float acc = 0.0f;
-#pragma unroll 1
-                for (int it = 0; it < R * SK; ++it) acc = fmaf(to_float(Wt[head * R * SK + it]), tile_value(tr_, key - j * F_BK, it / SK, it % SK), acc);
-                if (key < S && (!causal || key <= p_)) *reinterpret_cast<T *>(o_at + (o_offset(p_) + (unsigned)(key * (int)sizeof(T)))) = from_float<T>(acc);
+        }
+    };
+    // A row of a pair meets taps 0 in the window row that only the other one takes, a key of a group in the columns that only others take,
+    // and an infinity or a NaN there turns those into NaN.  Results that are NaN are formed again, tap by tap, all others stay the products'
+    // own.  A lane reads back the vectors that it has stored and takes eight keys of one row at a time, a window row after the other,
+    // until none of its wavefront's sums can become a number any more.  us, all values finite | one row of Q NaN | all of Q (in brackets with
+    // all 32 rows of such a block formed again, a key per lane): bf16 6x11 B2 H16 S4096 D128 254 | 527 | 789 (4608 | 14361), fp16 7x7 B1 H16
+    // S4096 102 | 464 | 468 (3123 | 6370), bf16 11x15 B1 H16 S2048 D64 39 | 296 | 158 (3417 | 6939), 3x3 B2 H16 S1024 D64 18 | 40 | 63 (65 | 199).
+    // Keeping the groups' NaN masks instead of reading back: all of Q 395, 189, 128, 36, but every launch 2 % slower.
+    auto form_again = [&](int j) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);   // the stores come first
+        const int lane_ = opaque_lane(lane), key0 = (lane_ >> 4) * 8, first = wave * (16 * RB) + cshift + 2 * (lane_ & 15);   // (rare: nothing of it is kept in registers outside)
+        char *const o_block = o_at + (int64_t)j * F_BK * (int)sizeof(T);
+        unsigned wanted = 0;             // bit 8n + u: NaN in row n/2 of the pair, key 32 (n%2) + key0 + u
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int col = j * F_BK + (n & 1) * 32 + key0;
+            u32x4_t back = {0, 0, 0, 0};
+            if (stored[n >> 1] && col < S && (!causal || fill_upper || col <= q0 - G::HR + first + (n >> 1)))
+                back = *reinterpret_cast<const u32x4_t *>(o_block + o_off[n >> 1] + (n & 1) * 32 * (int)sizeof(T));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float a, b;
+                unpack2<T>(back[u], a, b);
+                wanted |= (a != a ? 1u : 0u) << (8 * n + 2 * u) | (b != b ? 2u : 0u) << (8 * n + 2 * u);
             }
         }
+#pragma unroll 1
+        for (int n = 0; n < 4; ++n) {
+            const unsigned want = wanted >> (8 * n) & 255u;
+            if (__builtin_amdgcn_ballot_w64(want != 0) == 0) continue;
+            const int q = (n & 1) * 32 + key0, row = first + (n >> 1) - (R - 1);
+            float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+            for (int i = 0; i < R; ++i) {
+                const T *const from = tile + (row + i) * G::SLD + q + G::SHIFT - G::C0, *const ahead = reinterpret_cast<const T *>(side) + (row + i) * 2;
+                float x[SK + 7];
+#pragma unroll
+                for (int e = 0; e < SK + 7; ++e) x[e] = to_float(e < G::C0 - G::SHIFT && q == 0 ? ahead[e] : from[e]);   // (LEFT: two columns of the first group)
+#pragma unroll
+                for (int t = 0; t < SK; ++t) {
+                    const float tap = to_float(Wt[(head * R + i) * SK + t]);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc[u] = fmaf(tap, x[t + u], acc[u]);
+                }
+                unsigned open = 0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) open |= (acc[u] == acc[u] ? 1u : 0u) << u;
+                if (__builtin_amdgcn_ballot_w64((open & want) != 0) == 0) break;
+            }
+            T *const at = reinterpret_cast<T *>(o_block + (n >> 1 ? o_off[1] : o_off[0])) + (n & 1) * 32;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (want >> u & 1) at[u] = from_float<T>(acc[u]);
         }
+    };
+    auto check = [&](int j) __attribute__((always_inline)) {
+        if constexpr (!RAW)
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan != nan) != 0, 0)) form_again(j);
     };
     for (int j = j_lo;;) {  // block(tag, j, K(j), where K(j+1) goes)
         if (plain(j)) block(std::true_type{}, j, B0, B1);
         else block(std::false_type{}, j, B0, B1);
+        check(j);
         if (++j > j_end) break;
         if (plain(j)) block(std::true_type{}, j, B1, B0);
         else block(std::false_type{}, j, B1, B0);
+        check(j);
         if (++j > j_end) break;
     }
 

@@ -281,9 +281,57 @@ def test_qk_conv_non_finite_scores_stay_local(pkg, case, dtype):
     got = pkg.ops.qk_conv(q.cuda(), k.cuda(), w.cuda(), True, scale).cpu().float()
     clean = pkg.ops.qk_conv(cq.cuda(), ck.cuda(), w.cuda(), True, scale).cpu().float()
     assert torch.equal(~torch.isfinite(got), foot & low)
-    ok = low & ~foot          # (formed again tap by tap where a neighbour was NaN: another order of the sum, one rounding)
+    ok = low & ~foot          # (formed again tap by tap where the products made NaN of them: another order of the sum, one rounding)
     ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
     torch.testing.assert_close(got[ok], clean[ok], rtol=ulp, atol=1e-5)
+
+
+@pytest.mark.parametrize("form", ["planes", "triangular", "band"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", PAIR_CASES)
+def test_qk_conv_non_finite_scores_leave_the_others_their_bits(pkg, case, dtype, form):
+    """Work items of several key blocks (28 heads of 1160 rows), both layouts of the scores and a band mask; in each head a query row that
+    is NaN, a query row with one infinity or a key with one, at rows that belong to all four wavefronts, their first and last rows
+    among them, and to all places of a key block.  Non-finite are the outputs that take such a score and no others; an output whose products
+    met no such value keeps the bits that it has without them, and one that is formed again is off by another order of its sum."""
+    r, sk, d = case
+    h, s, group = 28, 1160, 4
+    print(f"qk_conv non-finite, long items {case} {dtype} {form}", flush=True)
+    q, k, _ = (t.cuda() for t in O.seeded_qkv(1, h, s, d, dtype, seed=19))
+    w = O.seeded_conv_weight(h, r, sk, 0.05, dtype)
+    w[w == 0] = 0.01
+    w = w.cuda()
+    scale = float(torch.rsqrt(torch.tensor(float(d))))
+    rows = torch.arange(s, device="cuda")
+    seen = (rows[None, :] <= rows[:, None])[None].expand(h, s, s)
+    first = (rows - 299).clamp(min=0).to(torch.int32)[None] if form == "band" else None
+    if form == "band":
+        seen = seen & (rows[None, None, :] >= first[0][None, :, None])
+
+    def run(q, k):
+        if form == "triangular":
+            return pkg.ops.tri_unpack(pkg.ops.qk_conv_tri(q, k, w, scale, group), 1, h, s, group)[0]
+        return pkg.ops.qk_conv(q, k, w, True, scale, fill_upper=False, first_visible=first)[0]
+
+    clean = run(q, k)
+    bq, bk = q.clone(), k.clone()
+    for i in range(h):
+        if i % 4 < 2:
+            bq[0, i, (5, 127, 128, 40, 71, 360, 481, 602, 723, 844, 965, 1086, 1120, 1159)[i // 4 * 2 + i % 4]] = float("nan")
+        elif i % 4 == 2:
+            bq[0, i, (0, 118, 239, 370, 511, 702, 933)[i // 4], i] = float("inf")
+        else:
+            bk[0, i, (0, 63, 64, 130, 317, 571, 1022)[i // 4], i] = float("inf")
+    got = run(bq, bk)
+    off = (~torch.isfinite(torch.matmul(bq.float(), bk.float().transpose(2, 3))[0]) & seen).float()
+    left = (sk - 1) // 2
+    takes = F.max_pool2d(F.pad(off, (left, sk - 1 - left, r - 1, 0)), (r, sk), stride=1) > 0
+    assert torch.equal(~torch.isfinite(got[seen]), takes[seen])
+    met = F.max_pool2d(F.pad(off, (32, 32, r, 1)), (r + 2, 65), stride=1) > 0   # (a pair's other row, a group's other keys)
+    assert torch.equal(got[seen & ~met], clean[seen & ~met])
+    near = seen & ~takes
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    torch.testing.assert_close(got[near].float(), clean[near].float(), rtol=ulp, atol=1e-5)
 
 
 @pytest.mark.parametrize("planes", [1, 80])   # workgroups of eight wavefronts with a row block each, of four with two
