@@ -16,10 +16,16 @@
 // Why: R*S multiply-adds on the vector units (0.079 PFLOP/s without packed fp32 forms) bound the row-sliding kernels from about 50
 // taps on.  This form executes 6 * 64 * 9 flops for the 2 * 165 of an output of 11x15, at 2.5 PFLOP/s.
 // One kernel row and sixteen keys per product (11 products and as many operands per 256 outputs, 9 and 4 now) -> this, fp32 11x15, whole
-// rows: 16 planes of 512^2 19.9 -> 18.9, 12 of 801^2 31.1 -> 28.8, 16 of 1024^2 41.3 -> 37.9, 32 of 1024^2 66.6 -> 60.5, 16 of 2048^2 142 either way;
-// 16-bit data, with as many workgroups per CU as their registers allow (split_occ) where two ran: bf16 16 of 1001^2 7x7 21.7 -> 20.6, 11x15 23.3 -> 21.7,
-// fp16 6x11 27.4 -> 23.8, with fp32 weights 16 of 1024^2 bf16 6x11 23.0 -> 20.6, 7x9 23.8 -> 20.1, fp16 6x11 29.9 -> 27.1,
-// 7x9 30.1 -> 25.8, 16 of 2048^2 76.5 -> 74, 80.3 -> 70.
+// rows: 16 planes of 512^2 19.9 -> 18.9, 16 of 1024^2 41.3 -> 37.9, 32 of 1024^2 66.6 -> 60.5, 16 of 2048^2 142 either way.
+// 16-bit data gains by that only if it is also stored well: two groups at a time, four keys a lane, stores are 16 rows x 32 bytes and two wavefronts
+// complete a line; without stores this form was the faster one everywhere, with them the slower one up to 333^2.  So all four groups leave together,
+// eight keys a lane: 16 rows x 64 bytes in half the instructions and fewer registers.  One row and sixteen keys, two workgroups per CU | two rows,
+// 32 bytes, three and four workgroups | 64 bytes, at most three (split_occ), lower triangle (input gradient), us: bf16 6x11 16 of 333^2 6.0 | 6.9 | 6.3
+// (6.9 | 7.8 | 7.0), 12 of 801^2 12.4 | 14.4 | 12.1 (15.9 | 18.4 | 15.1), 16 of 1023^2 17.9 | 17.2 | 16.0 (23.4 | 21.6 | 20.6), 32 of 1023^2 28.0 | 30.6 |
+// 25.9 (36.4 | 38.8 | 32.9), 16 of 2047^2 51.0 | 47.3 | 42.8 (65.8 | 55.7 | 52.3); with fp32 weights 7x7 12 of 801^2 14.5 | 15.2 | 13.6 (17.4 | 18.2 |
+// 16.3), 16 of 1023^2 20.3 | 19.0 | 17.7 (25.5 | 23.3 | 22.2); fp16 7x9 16 of 333^2 7.6 | 7.9 | 7.3, 16 of 1023^2 23.4 | 21.6 | 20.0 (28.7 | 24.5 |
+// 23.9), with fp32 weights 6x11 16 of 2047^2 74.6 | 74.0 | 67.2 (84.1 | 83.9 | 81.3).  Left behind the first by 0.2 to 0.5 us: 5x7 and 6x11 of planes up to
+// 333^2, of a strip or two per CU.
 // us, conv2d_rows -> the former, fp32: lower triangle 16 planes of 512^2 23 -> 18.5, 12 of 801^2 32 -> 28.5, 16 of 1024^2 58 -> 38, 32 of
 // 1024^2 105 -> 68, 16 of 2048^2 177 -> 128; whole rows 31 -> 20, 34 -> 31, 86 -> 43, 152 -> 80, 260 -> 151.  Smaller kernels stay
 // there, lower triangle | whole rows: 7x9 16 of 1024^2 29.7 | 39.4 against 29.4 | 34.5 here, 16 of 512^2 13.9 | 16.4 against 15.3 |
@@ -38,10 +44,12 @@
 // not see small values beside ordinary ones: lower triangle of 16 planes, fp32 512^2 19.2 -> 18.5 us, 2048^2 130.9 -> 127.9, bf16 with fp32
 // weights 1024^2 6x11 20.6 -> 19.5, fp16 7x9 26.4 -> 25.1.)
 //
-// Shape.  A workgroup of four wavefronts takes strips of 32 rows x 128 keys of one plane, one after the other, two workgroups per
-// CU.  A strip and its halo are loaded four keys per lane, two strips ahead, into registers; split and written to one of two LDS
+// Shape.  A workgroup of four wavefronts takes strips of 32 rows x 128 keys of one plane, one after the other, two or three workgroups per
+// CU (split_occ).  A strip and its halo are loaded four keys per lane, two strips ahead, into registers; split and written to one of two LDS
 // buffers (a plane of bf16 per part) a vector at a time between the products of the strip before.  The fragments of the plane's kernel stay in
 // registers (11x15: 3 parts * 3 quads * 3 chunks * 4 of them); they come out of a table of all windows of every kernel row.
+#include <algorithm>
+
 #include "conv2d_rows.hpp"
 #include "split.hpp"
 
@@ -69,9 +77,11 @@ inline int64_t p_count(int64_t H, int64_t W, int tri)
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
 // Workgroups per CU: a strip is a chain of loads, splitting, products and stores between two barriers, and what hides it is the other
-// workgroups.  The fewer parts, the fewer registers and the less LDS a workgroup takes.  (fp16 data with three parts of a tap: 177 registers, of
-// which the third workgroup takes 9 - five values go to scratch memory and back - and gives 7 to 11 %, figures above: 29.0 and 28.9 with two.)
-template <typename T, int WP, int R> constexpr int split_occ() { return parts_of<T>() == 1 && WP == 1 ? 4 : parts_of<T>() * WP <= 6 && R <= 7 ? 3 : 2; }
+// workgroups; as many as registers and LDS hold (fp16 data with three parts of a tap gives five values to scratch memory for the third), but
+// three.  bf16 data and taps leave room for four, whose strips come in fewer and emptier rounds.  us, 6x11, two | three | four, lower triangle
+// (whole planes): 12 of 801^2 12.3 | 11.8 | 13.4 (16.2 | 15.2 | 17.1), 32 of 511^2 12.6 | 11.0 | 13.2 (15.7 | 14.5 | 14.2), 4 of 2047^2 16.2 | 15.5 | 18.4
+// (25.8 | 23.4 | 22.3), 16 of 2047^2 39.6 | 40.0 | 38.6 (74.8 | 66.9 | 71.9); the other way only 8 of 801^2 9.1 | 8.8 | 8.1 (11.9 | 12.1 | 10.9).
+template <typename T, int WP, int R> constexpr int split_occ() { return parts_of<T>() * WP == 1 || (parts_of<T>() * WP <= 6 && R <= 7) ? 3 : 2; }
 
 template <typename T, int WP, int R, int S, bool BWD>
 __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(const T *__restrict__ x, const void *__restrict__ w, T *__restrict__ y, int C, int H,
@@ -240,11 +250,13 @@ __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(con
         };
         const int lower = causal ? (t.p0 + P_TM - 1 - t.q0 - wave * 32) >> 3 : NG - 1;   // last group that touches the triangle
         // (address of a lane's results: a uniform base and a byte offset within the strip)
-        const int pl = 2 * ln, ql = wave * 32 + kg * 4;
+        constexpr int LK = sizeof(T) == 2 ? 8 : 4;   // keys of a row that a lane stores at a time
+        const int pl = 2 * ln, ql = wave * 32 + kg * LK;
         char *const ybase = reinterpret_cast<char *>(yp + (int64_t)t.p0 * W + t.q0);
         const unsigned yoff = (unsigned)(pl * W + ql) * (unsigned)sizeof(T);
         const bool whole = t.p0 + P_TM <= H && t.q0 + P_TN <= W && (!causal || t.q0 + P_TN - 1 <= t.p0);
         float bad = 0.0f;   // not 0: a result that is not finite
+        uint32_t out[sizeof(T) == 2 ? NG : 1][2];   // 16-bit data: the groups' results, packed
         // sums of the large products, fp32 data: of the middle chunk, which holds the taps next to the output's own position, and of the other two,
         // so that a sum is rounded fewer times and that of a kernel near the identity once or twice; and of the small ones
         constexpr bool TWO = XP == 3;
@@ -283,7 +295,7 @@ __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(con
                         __builtin_amdgcn_sched_barrier(0);
                     }
             }
-            if (x == 3 || x == 5) {   // two groups are complete: a lane gets four keys of each row of its pair, stores of 16 rows x 64 bytes
+            if (x == 3 || x == 5) {   // two groups are complete
                 const int w = x - 3;
                 float v[2][4];
 #pragma unroll
@@ -293,22 +305,59 @@ __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(con
                         v[g][u] = (big[w + g][u] + (TWO ? rim[w + g][u] + small[w + g][u] : small[w + g][u])) * DOWN;
                         bad = fmaf(v[g][u], 0.0f, bad);
                     }
+                if constexpr (sizeof(T) == 2) {
+                    // all four groups leave together: a lane gets the eight keys of group kg in each row of its pair, stores of 16 rows x 64 bytes
 #pragma unroll
-                for (int u = 0; u < 4; ++u) swap32(v[0][u], v[1][u]);
+                    for (int g = 0; g < 2; ++g)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (whole) {
-                        asm volatile("" : "+v"(v[h][0]), "+v"(v[h][1]), "+v"(v[h][2]), "+v"(v[h][3]));   // (one store, not one shared in part with the other branch)
-                        quad4<T> o;
+                        for (int n = 0; n < 2; ++n) out[w + g][n] = pack2<T>(v[g][2 * n], v[g][2 * n + 1]);
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) o.v[u] = from_float<T>(v[h][u]);
-                        __builtin_memcpy(ybase + (yoff + (unsigned)(h * W + w * 8) * (unsigned)sizeof(T)), &o, sizeof(o));
-                    } else {
-                        const int p = t.p0 + pl + h, q = t.q0 + ql + w * 8;
-                        if (p < H && q < W && !(causal == 2 && q > p)) {
+                    for (int n = 0; n < 2; ++n) swap16(out[w][n], out[w + 1][n]);   // (afterwards: [w] keys 0-3, [w + 1] keys 4-7 of group w + kg%2)
+                    if (w == 0) continue;
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) v[h][u] = causal && q + u > p ? 0.0f : v[h][u];
-                            store_quad<T>(yp + (int64_t)p * W, q, W, v[h]);
+                    for (int n = 0; n < 4; ++n) swap32(out[n >> 1][n & 1], out[2 + (n >> 1)][n & 1]);   // ([0], [1] the pair's first row, [2], [3] the second)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        mta_u32x4 o = {out[2 * h][0], out[2 * h][1], out[2 * h + 1][0], out[2 * h + 1][1]};
+                        if (whole) {
+                            asm volatile("" : "+v"(o));   // (one store, not one shared in part with the other branch)
+                            __builtin_memcpy(ybase + (yoff + (unsigned)(h * W) * (unsigned)sizeof(T)), &o, sizeof(o));
+                        } else {
+                            const int p = t.p0 + pl + h, q = t.q0 + ql;
+#pragma unroll
+                            for (int n = 0; n < 4; ++n) {
+                                if (causal && q + 2 * n > p) o[n] &= 0xffff0000u;
+                                if (causal && q + 2 * n + 1 > p) o[n] &= 0x0000ffffu;
+                            }
+                            // (asked for by quads; mostly both)
+                            const bool one = p < H && q < W && !(causal == 2 && q > p), two = p < H && q + 4 < W && !(causal == 2 && q + 4 > p);
+                            if (two && q + 8 <= W) {
+                                __builtin_memcpy(yp + (int64_t)p * W + q, &o, sizeof(o));
+                            } else {
+#pragma unroll
+                                for (int g = 0; g < 2; ++g) {
+                                    unpack2<T>(o[2 * g], v[g][0], v[g][1]);
+                                    unpack2<T>(o[2 * g + 1], v[g][2], v[g][3]);
+                                    if (g ? two : one) store_quad<T>(yp + (int64_t)p * W, q + 4 * g, W, v[g]);
+                                }
+                            }
+                        }
+                    }
+                } else {   // a lane gets four keys of each row of its pair, stores of 16 rows x 64 bytes
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) swap32(v[0][u], v[1][u]);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        if (whole) {
+                            asm volatile("" : "+v"(v[h][0]), "+v"(v[h][1]), "+v"(v[h][2]), "+v"(v[h][3]));
+                            __builtin_memcpy(ybase + (yoff + (unsigned)(h * W + w * 8) * (unsigned)sizeof(T)), v[h], sizeof(v[h]));
+                        } else {
+                            const int p = t.p0 + pl + h, q = t.q0 + ql + w * 8;
+                            if (p < H && q < W && !(causal == 2 && q > p)) {
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) v[h][u] = causal && q + u > p ? 0.0f : v[h][u];
+                                store_quad<T>(yp + (int64_t)p * W, q, W, v[h]);
+                            }
                         }
                     }
                 }
@@ -317,7 +366,7 @@ __global__ __launch_bounds__(256, (split_occ<T, WP, R>())) void conv2d_split(con
         if (__builtin_amdgcn_ballot_w64(bad != 0.0f) != 0) {   // this lane's results that are not finite: multiply-adds, tap by tap
 #pragma unroll 1
             for (int e = opaque(0); e < 16; ++e) {
-                const int pe = t.p0 + pl + (e >> 2 & 1), q = t.q0 + ql + (e >> 3) * 16 + (e & 3);
+                const int pe = t.p0 + pl + (LK == 8 ? e >> 3 : e >> 2 & 1), q = t.q0 + ql + (LK == 8 ? e & 7 : (e >> 3) * 16 + (e & 3));
                 if (pe >= H || q >= W || (causal && q > pe)) continue;
                 T *const at = yp + (int64_t)pe * W + q;
                 if (__builtin_isfinite(to_float(*at))) continue;
@@ -368,7 +417,9 @@ int launch_split(const void *x, const void *w, void *y, int64_t planes, int64_t 
 {
     const int64_t total = p_count(H, W, causal != 0);
     if (total > 0x3fffffffLL) return MTA_ERR_SHAPE;
-    int64_t per_plane = (split_occ<T, WP, R>() * device_cu_count() + planes - 1) / planes;   // one round of resident workgroups
+    // One round of resident workgroups, rounded down: those beyond it would start when the others end.  fp32 11x15, lower triangle, us, rounded up ->
+    // down: 12 planes of 801^2 26.0 -> 23.7, 24 of 1023^2 62.0 -> 49.0, 12 of 1501^2 68.8 -> 55.9.
+    int64_t per_plane = std::max<int64_t>(split_occ<T, WP, R>() * device_cu_count() / planes, 1);
     if (per_plane > total) per_plane = total;
     hipLaunchKernelGGL((conv2d_split<T, WP, R, S, BWD>), dim3((unsigned)(planes * per_plane)), dim3(256), 0, st, (const T *)x, w, (T *)y, (int)C, (int)H,
                        (int)W, causal, in_scale, use_scale, w_dtype, (int)planes, (int)total, (int)per_plane);

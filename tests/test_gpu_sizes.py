@@ -1152,12 +1152,14 @@ def test_conv_11x15_split_range(pkg, bwd):
         assert ((got.double() - want).abs() <= 167 * (2.0 ** -24 * size + 2.0 ** -149)).all()
 
 
-@pytest.mark.parametrize("n,c,h,w", [(2, 8, 1000, 1001), (1, 16, 777, 777), (3, 7, 700, 801)])
-@pytest.mark.parametrize("dtype,wdtype,r,k", [(torch.float32, torch.float32, 11, 15), (torch.bfloat16, torch.float32, 6, 11), (torch.float16, torch.float16, 7, 9)])
+@pytest.mark.parametrize("n,c,h,w", [(2, 8, 1000, 1001), (1, 16, 777, 777), (3, 7, 700, 801), (1, 5, 261, 331), (1, 5, 300, 269), (2, 8, 200, 335)])
+@pytest.mark.parametrize("dtype,wdtype,r,k", [(torch.float32, torch.float32, 11, 15), (torch.bfloat16, torch.float32, 6, 11), (torch.float16, torch.float16, 7, 9),
+                                                (torch.bfloat16, torch.bfloat16, 6, 11), (torch.float16, torch.float32, 6, 11)])
 def test_conv_split_strips_in_turns(pkg, dtype, wdtype, r, k, n, c, h, w):
-    """Convs on the parts of the values where a workgroup walks several strips (two workgroups per CU: 32 or 25 per plane here), planes dealt to the XCDs
-    and not: forward, lower triangle only, input gradient, causal or not; in the middle of a walk an infinite value, whose
-    results come from multiply-adds, and in fp32 a stretch of tiny ones.  Bounds as for planes of few strips."""
+    """Convs on the parts of the values where a workgroup walks several strips (two workgroups per CU with fp32 data, three with the others: 24 to 48
+    per plane here), planes dealt to the XCDs and not, and planes of few strips whose rows end at all places of the eight keys that are
+    stored together: forward, lower triangle only, input gradient, causal or not; in the middle of a walk an infinite value, whose results
+    come from multiply-adds, and in fp32 a stretch of tiny ones.  Bounds as for planes of few strips."""
     g = torch.Generator(device="cuda").manual_seed(79)
     x, weight = torch.randn(n, c, h, w, generator=g, device="cuda").to(dtype), (0.1 * torch.randn(c, r, k, generator=g, device="cuda")).to(wdtype)
     hit = (n - 1, c // 2, h // 2, w // 4)
