@@ -334,12 +334,15 @@ def test_qk_conv_non_finite_scores_leave_the_others_their_bits(pkg, case, dtype,
     torch.testing.assert_close(got[near].float(), clean[near].float(), rtol=ulp, atol=1e-5)
 
 
-@pytest.mark.parametrize("planes", [1, 80])   # workgroups of eight wavefronts with a row block each, of four with two
+@pytest.mark.parametrize("wavefronts", [8, 4])   # with one block of 16 rows each, with two
 @pytest.mark.parametrize("case", PAIR_CASES)
-def test_conv_attention_non_finite_rows_stay_local(pkg, case, planes):
+def test_conv_attention_non_finite_rows_stay_local(pkg, case, wavefronts):
     """A query row that is not finite reaches the R rows from it on, an infinite key every row that attends a score of it."""
     r, sk, d = case
-    h, s, dtype = 3 * planes, 200, torch.bfloat16
+    s, dtype = 200, torch.bfloat16
+    # two query blocks a head; four wavefronts from more than 2 1/4 (D = 64) or 1 3/4 (128) workgroups per CU on
+    planes = 1 if wavefronts == 8 else (9 if d == 64 else 7) * torch.cuda.get_device_properties(0).multi_processor_count // (4 * 3 * 2) + 1
+    h = 3 * planes
     print(f"conv_attn non-finite {case} planes={planes}", flush=True)
     q, k, v, (cq, ck) = _non_finite_inputs(3, s, d, dtype)
     w = O.seeded_conv_weight(3, r, sk, 0.05, dtype)
