@@ -77,7 +77,7 @@ inline int64_t p_count(int64_t H, int64_t W, int tri)
 template <typename T> constexpr int parts_of() { return __is_same(T, float) ? 3 : __is_same(T, f16_t) ? 2 : 1; }
 
 // Workgroups per CU: a strip is a chain of loads, splitting, products and stores between two barriers, and what hides it is the other
-// workgroups; as many as registers and LDS hold (fp16 data with three parts of a tap gives five values to scratch memory for the third), but
+// workgroups; as many as registers and LDS hold (fp16 data with three parts of a tap: with some values in scratch memory), at most
 // three.  bf16 data and taps leave room for four, whose strips come in fewer and emptier rounds.  us, 6x11, two | three | four, lower triangle
 // (whole planes): 12 of 801^2 12.3 | 11.8 | 13.4 (16.2 | 15.2 | 17.1), 32 of 511^2 12.6 | 11.0 | 13.2 (15.7 | 14.5 | 14.2), 4 of 2047^2 16.2 | 15.5 | 18.4
 // (25.8 | 23.4 | 22.3), 16 of 2047^2 39.6 | 40.0 | 38.6 (74.8 | 66.9 | 71.9); the other way only 8 of 801^2 9.1 | 8.8 | 8.1 (11.9 | 12.1 | 10.9).

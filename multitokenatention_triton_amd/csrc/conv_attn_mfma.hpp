@@ -418,7 +418,7 @@ __global__ __launch_bounds__(64 * NW, 2) void conv_attn_fwd_mfma(const T *__rest
         auto finish = [&](auto bc) __attribute__((always_inline)) {
             constexpr int b = decltype(bc)::value;
             constexpr int rb = b / NCB, cb = b % NCB;
-            const f32x4 a = cacc[b % (2)];
+            const f32x4 a = cacc[b % 2];
             const int p_ = cprow[rb];
             // (fp32 from here to the probabilities: the factor goes into the exponential's multiply-add)
             float v4[4] = {a[0], a[1], a[2], a[3]};
@@ -472,8 +472,8 @@ __global__ __launch_bounds__(64 * NW, 2) void conv_attn_fwd_mfma(const T *__rest
             // LDS operations younger than read n: exactly the reads issued after it
             constexpr int younger = (n + NLD < NREAD ? n + NLD : NREAD - 1) - n;
             lds_wait_upto<younger>(ring[n % NSLOT]);
-            if constexpr (i == 0) cacc[blk % (2)] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            mma16(cacc[blk % (2)], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
+            if constexpr (i == 0) cacc[blk % 2] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            mma16(cacc[blk % 2], tz[i], __builtin_bit_cast(frag8<T>, ring[n % NSLOT]));
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (blk >= 1 && i == LAG - 1) {
                 finish(std::integral_constant<int, blk - 1>{});

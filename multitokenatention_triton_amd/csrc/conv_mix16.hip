@@ -136,7 +136,7 @@ __global__ __launch_bounds__(X_WT, (x_occ<R>() * X_NW / 4)) void conv_mix16_mfma
     constexpr int STAGE_IT = (SLOTS + X_WT - 1) / X_WT;
     constexpr int BUF = ((SLOTS + 3) & ~3) * VEC;                // elements per window buffer
     // The slots of a window are copied in STAGE_IT rounds: full rounds of one slot per thread, then the remainder spread
-    // evenly over the four wavefronts (their first REM_W lanes), so that every wavefront issues the same number of copy
+    // evenly over the eight wavefronts (their first REM_W lanes), so that every wavefront issues the same number of copy
     // instructions per window - the number the waits below count.
     constexpr int REM = SLOTS - (STAGE_IT - 1) * X_WT;           // slots of the last round
     constexpr int REM_W = (REM + X_NW - 1) / X_NW;               // ... per wavefront
@@ -630,8 +630,10 @@ int launch_x(const void *x, const void *wc, const void *wm, void *y, int64_t N, 
     if (ipp64 > (1 << 24)) return MTA_ERR_SHAPE;
     const int64_t npg = N * (C / X_HG);
     // Groups within a lane: below 400 tiles of 16 heads, less than a round of the persistent workgroups, the kernel that computes on the
-    // vector units is as fast (this | that, us, bf16, 3x3, groups of 4: 272 tiles (B1 H16 S1024) 27.6 | 25, 440 (B4 S640) 28.8 | 34, 1056
-    // (B1 S2048) 57 | 108, 4160 (B1 S4096) 148 | 329).
+    // vector units is as fast with the smallest kernels (this | that, us, bf16 3x3 groups of 4 / fp16 3x3 groups of 2 / bf16 7x7 groups of 4: 72 tiles (B1
+    // H16 S512) 20.8 | 10.9 / 20.3 | 8.8 / 23.7 | 15.4, 272 (B1 S1024) 27.7 | 30.1 / 26.9 | 28.3 / 31.5 | 46.4, 342 (B1 S1152) 27.9 | 25.1 / 27.1 | 24.5 / 32.1 |
+    // 39.6, 380 (B1 S1216) 28.7 | 29.3 / 28.1 | 26.2 / 32.5 | 44.7, 440 (B4 S640) 28.8 | 33.4 / 28.2 | 30.6 / 33.5 | 51.6, 1056 (B1 S2048) 49.3 | 105 / 48.0 |
+    // 96.5 / 58.5 | 161); 7x7 in between is left to the module's two kernels, which take less than either.
     if (GROUP < X_HG && npg * ipp64 < 400) return MTA_ERR_UNSUPPORTED;
     const xm_split sp = make_split<R, S>(npg, tiles_m, tiles_n, causal, fill_upper, tri, ipp64);
     int64_t longest = 0;

@@ -34,18 +34,15 @@ constexpr int QK_SHORT_PERCENT = 50;
 constexpr int ITEM_TABLE_MAX = 768;
 struct qk_chunks { int big, small; };
 // How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 16000 on the grid
-// runs in several rounds whatever the length and 48/24 keeps the rebuilt columns few; below, items as short as it takes to
-// have two or three per CU, down to one key block, win although each rebuilds one key block's worth of columns: the grid is
-// otherwise a fraction of the chip, each workgroup walking its keys alone.  us, 48/24 | as short as the rule makes them:
-// B1 H8 S256 D64 3x3 (80 blocks) 13.3 | 7.6; B1 H16 S512 D128 5x5 (448) 23.3 | 11.5; B2 H16 S512 D64 6x11 (896) 22.6 | 13.4;
-// B4 H16 S512 (1792) 26.3 | 22.0; B1 H8 S2048 D64 (2450) 48.9 | 23.9.
-// Where the line lies, the kernel alone (in brackets the forward with groups of 4 heads / with all weights dense; three processes
-// a side, which differ by up to 3 on the kernel and 2 on a forward), 48/24 | 16/8: B1 H16 S2048 D128 7x7 (5216) 62 | 51 (117 | 108 /
-// 184 | 171); B1 H32 S2048 D64 5x5 (10432) 58 | 56 (158 | 156 / 394 | 392); B2 H16 S2048 D128 6x11 (10432) 68 | 69 (165 | 166 /
-// 298 | 293); B1 H16 S3072 D128 3x3 (10688) 65 | 63 (199 | 190 / 309 | 297); B1 H16 S3712 D64 7x9 (15088) 82 | 81 (236 | 235 /
-// 386 | 383); B3 H16 S2048 D128 7x7 (15648) 99 | 103 (241 | 245 / 395 | 396); B1 H16 S4096 D128 7x7 (19104) 121 | 126 (300 | 299 /
-// 485 | 490); B4 H16 S2048 D64 3x3 (20864) 87 | 90 (242 | 246 / 462 | 471); B2 H16 S3072 D128 6x11 (21376) 133 | 136 (332 | 331 /
-// 536 | 545); B2 H16 S4096 D128 6x11 (38208) 225 | 236 (538 | 546 / 887 | 898).
+// runs in several rounds whatever the length and 48/24 keeps the starts few; below, items as short as it takes to
+// have two or three per CU, down to one key block, win although each forms the 16 columns ahead of it again: the grid is
+// otherwise a fraction of the chip, each workgroup walking its keys alone.  us, the kernel in a loop, bf16, 48/24 | as short as the rule makes them:
+// B1 H8 S256 D64 3x3 (80 blocks) 10.9 | 6.0; B1 H16 S512 D128 5x5 (448) 19.4 | 9.2; B2 H16 S512 D64 6x11 (896) 20.4 | 12.1;
+// B4 H16 S512 (1792) 22.1 | 17.9; B1 H8 S2048 D64 (2450) 46.1 | 22.9.
+// Where the line lies, 48/24 | 16/8 (two processes a side, which differ by up to 4, at S3712 by 12): B1 H16 S2048 D128 7x7 (5216) 50.4 | 40.0; B1 H32 S2048
+// D64 5x5 (10432) 51.0 | 46.8; B2 H16 S2048 D128 6x11 (10432) 70.5 | 71.0; B1 H16 S3072 D128 3x3 (10688) 62.6 | 62.8; B1 H16 S3712 D64 7x9 (15088)
+// 79.0 | 75.4; B3 H16 S2048 D128 7x7 (15648) 94.8 | 98.5; B1 H16 S4096 D128 7x7 (19104) 116.5 | 117.2; B4 H16 S2048 D64 3x3 (20864) 85.0 | 89.8; B2 H16
+// S3072 D128 6x11 (21376) 144 | 143; B2 H16 S4096 D128 6x11 (38208) 238 | 250.
 inline qk_chunks qk_chunk_rule(int64_t blocks, int64_t head_blocks, int nqb)
 {
     if (blocks >= 16000) return {48, 24};
@@ -625,7 +622,7 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
             // (Ordinary stores: a 128-byte line is completed by two instructions a few hundred cycles apart, and the L2
             // merges them.  Marked non-temporal, each 64-byte half went to memory on its own and the write counter
             // read 1.38 times the bytes; the price of the merge is that the scores displace some of the head's K blocks
-            // from the L2 - fetches 79 -> 196 MB per launch at the benchmark shape, 825 -> 736 MB in total, 4 % faster.)
+            // from the L2 - at the benchmark shape 541 MB are written and 294 fetched per launch, for 68 MB of Q and K.)
             // (a value that is not finite reaches all results of its products, and each chunk the products of two groups, the last one those of
             // the last group: one of four results of every other group tells)
             if constexpr (w % 2 == 0 || w == NWIN - 1) nan = fmaf(a[0], 0.0f, nan);
@@ -813,7 +810,7 @@ int launch_scores(const conv_attn_args &a)
         static thread_local int count[MAXLEN + 2];
         static thread_local uint32_t items[ITEM_TABLE_MAX];
         static thread_local int lens[ITEM_TABLE_MAX];
-        // long chunks for the first part of a query block's key range, short ones for the last QK_SHORT_SHARE of it
+        // long chunks for the first part of a query block's key range, short ones for the last QK_SHORT_PERCENT of it
         static const int env_big = [] { const char *e = getenv("MTA_QK_CHUNK_LONG"); return e ? atoi(e) : 0; }();
         static const int env_small = [] { const char *e = getenv("MTA_QK_CHUNK_SHORT"); return e ? atoi(e) : 0; }();
         static const int share = [] { const char *e = getenv("MTA_QK_SHORT_PERCENT"); return e ? atoi(e) : QK_SHORT_PERCENT; }();
@@ -883,7 +880,7 @@ template <typename T, int D, bool BAND> int dispatch_scores(const conv_attn_args
     MTA_SCORES_CASE(6, 11)
     MTA_SCORES_CASE(7, 7)
     MTA_SCORES_CASE(7, 9)
-    // (the 36 registers of its taps' operands leave two workgroups per CU)
+    // (the 36 registers of its taps' operands leave three workgroups per CU at D = 64, two at 128)
     MTA_SCORES_CASE(11, 15)
 #undef MTA_SCORES_CASE
     return 1;

@@ -43,15 +43,16 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 }
 
 // Whether conv + mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
-// heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or, for
-// groups of 2 or 4 heads, one round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs); the dense 16
-// heads gain little there.
-// us of the forward (H16 D64, the pre-softmax conv 6x11), two kernels | one, fp16 dense 3x3 / 7x7 after the softmax / bf16 groups of 4, 3x3:
-// 72 tiles (B1 S512) 37.8 | 44.2 / 38.6 | 46.3 / 36.1 | 36.2, 272 (B1 S1024) 61.6 | 62.1 / 63.6 | 65.7 / 65.7 | 70.6, 342 (B1 S1152) 66.6 | 67.0 / 69.4 |
-// 70.6 / 69.8 | 70.6, 420 (B1 S1280) 74.8 | 72.8 / 78.0 | 76.6 / 74.9 | 77.0, 420 (B2 S896) 74.7 | 74.5 / 78.1 | 78.1 / 78.8 | 79.2, 440 (B4 S640)
-// 78.7 | 75.0 / 82.8 | 79.0 / 81.5 | 78.0, 506 (B1 S1408) 83.3 | 85.1 / 87.3 | 90.8 / 81.5 | 87.6, 544 (B2 S1008) 79.9 | 80.4 / 84.1 | 86.4 /
-// 85.0 | 84.7, 600 (B1 S1536) 90.1 | 94.9 / 94.3 | 100 / 89.9 | 98.2, 630 (B3 S896) 91.4 | 95.8 / 96.0 | 101 / 92.9 | 98.7.  Beyond, with the kernel as
-// it was at 20 us a tile: 816 (B3 S1024) 126.6 | 127.1 / 132.4 | 140.3 one | two, 1056 (B1 S2048) 155 | 165 / 162 | 176; now 816 7x7 114, 1056 132.
+// heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or
+// one round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs).  Groups of 2 or 4 heads take that
+// round; dense weights gain there too, 4 to 6 %, and are left on the two kernels.
+// us of the forward (H16 D64, the pre-softmax conv 6x11), two kernels | one, fp16 dense 3x3 / 7x7 after the softmax / bf16 groups of 4, 3x3 / fp16 groups
+// of 2, 3x3: 272 tiles (B1 S1024) 62.5 | 63.3 / 63.5 | 65.9 / 65.1 | 71.8 / 63.9 | 68.1, 380 (B1 S1216) 73.5 | 72.2 / 76.6 | 75.9 / 73.8 | 77.5 / 73.7 | 73.6,
+// 420 (B1 S1280) 74.9 | 73.2 / 78.2 | 76.9 / 75.7 | 77.1 / 75.6 | 75.6, 440 (B4 S640) 79.2 | 75.2 / 83.0 | 79.2 / 81.6 | 78.1 / 83.8 | 76.3, 448 (B8 S448) 81.9 |
+// 78.3 / 85.8 | 82.3 / 82.3 | 77.9 / 87.2 | 75.7, 480 (B2 S960) 79.1 | 74.8 / 83.5 | 78.8 / 81.7 | 78.9 / 82.3 | 76.9, 506 (B1 S1408) 83.8 | 85.7 / 87.8 | 91.7 /
+// 81.6 | 88.2 / 81.8 | 86.2, 544 (B2 S1008) 80.3 | 81.3 / 84.4 | 87.2 / 85.6 | 85.0 / 86.0 | 83.3, 600 (B1 S1536) 90.5 | 95.3 / 94.8 | 101 / 89.8 | 98.4 / 90.5 |
+// 96.8, 702 (B1 S1664) 96.4 | 95.7 / 101 | 101 / 95.9 | 97.8 / 95.5 | 95.9, 756 (B1 S1728) 106 | 106 / 110 | 111 / 103 | 105 / 103 | 103, 816 (B3 S1024) 119 |
+// 113 / 126 | 118 / 109 | 109 / 110 | 107, 840 (B2 S1280) 114 | 109 / 120 | 115 / 112 | 114 / 113 | 113, 1056 (B1 S2048) 133 | 126 / 136 | 135 / 134 | 133 / 131 | 130.
 bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_only, bool dense)
 {
     const int64_t tr = (rows + 31) / 32, tk = (keys + 63) / 64, tiles = planes * (lower_only && rows == keys ? tk * (tk + 1) : tr * tk);
