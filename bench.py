@@ -52,6 +52,7 @@ def stage_model(name, b, h, s, d, r=6, sk=11, esize=2):
       qk_conv          reads q,k; writes the lower triangle of the scores (QK^T, scale and conv fused)
       mix_softmax_mix  reads the lower triangle, writes the lower triangle (P V below never reads above it)
       pv               reads the lower triangle of P and V, writes O
+      softmax_mix_pv   the two in one kernel, announced as the two stages at once: reads the lower triangle of the scores and V, writes O
       conv_pre / mix_* / softmax / conv_post (unfused route) read the triangle and write the full tensor
       qk, pv_gemm      library GEMMs over the full square
     """
@@ -60,7 +61,7 @@ def stage_model(name, b, h, s, d, r=6, sk=11, esize=2):
         return 2 * qkv + t, 2 * b * h * tri(s) * d + 2 * r * sk * b * h * tri(s)
     if name == "mix_softmax_mix":
         return 2 * t, 0
-    if name == "pv":
+    if name in ("pv", "softmax_mix_pv"):
         return t + 2 * qkv, 2 * b * h * tri(s) * d
     if name in ("qk", "pv_gemm"):
         return 2 * qkv + full, 2 * b * h * s * s * d
@@ -68,9 +69,8 @@ def stage_model(name, b, h, s, d, r=6, sk=11, esize=2):
 
 
 # Which kernel runs a stage of the headline forward, as rocprofv3 names it in profiles/mta_forward_c4_hbm_traffic.txt
-STAGE_KERNEL = {"qk_conv": "conv_scores_mfma<bf16_t, 128, 6, 11, false>",
-                "mix_softmax_mix": "mix_softmax_mix_packed<bf16_t, 4, 1, false, true, 512, 8, false, false>",
-                "pv": "causal_pv_mid_kernel<bf16_t, 128, 8, 1, 1>"}
+STAGE_KERNEL = {"qk_conv": "conv_scores_mfma<bf16_t, 128, 6, 11, false, true>",
+                "softmax_mix_pv": "softmax_mix_pv<bf16_t, 128, 4, 4, 4, 2, 2, false>"}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "mta_forward_c4_hbm_traffic.txt")
 
 
@@ -538,6 +538,7 @@ def main():
     with torch.no_grad():
         ms = time_steps(torch, lambda i: mod(*sets[i], None, None), len(sets), args.warmup, args.steps)
         stages = stage_breakdown(torch, mod, sets, max(3, min(args.steps, 10)))
+        stages["softmax_mix_pv"] = stages.pop("mix_softmax_mix") + stages.pop("pv")   # (one kernel in this configuration)
         ran_own_pv = "qk" not in stages  # the fused route ends in mta_causal_pv_fwd, the unfused one in a library GEMM
         hip_stages = {k: v for k, v in stages.items() if k != "qk" and (k != "pv" or ran_own_pv)}
         dom = max(hip_stages, key=hip_stages.get)

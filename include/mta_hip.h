@@ -292,6 +292,24 @@ int mta_headmix_softmax_tri_fwd(const void *x, const void *w1, const void *w2, c
                                 int w_dtype, void *stream);
 int mta_causal_pv_tri_fwd(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H, int64_t S,
                           int64_t D, int group, int io_dtype, void *stream);
+/* ---- The causal forward in two stages, where nothing stands between the first conv and the softmax (an identity head weight ahead of the softmax,
+ * no post-softmax conv): the probabilities never reach memory.  16-bit I/O.
+ *   mta_qk_conv_stats_fwd:  mta_qk_conv_tri_fwd (group > 0) or, with group = 0, mta_qk_conv_fwd / mta_qk_conv_band_fwd over (B,H,S,S) planes
+ *                           (causal, nothing written above the diagonal), that also leaves the rows' statistics in `stats`: B*H*slots*S pairs of
+ *                           floats (8-byte aligned), slots = mta_qk_conv_stats_slots(B, H, S, R): of each of the pieces that the row's keys are worked on in a
+ *                           reference r and the sum of exp2(score log2(e) - r) over the scores as stored.  key_bias (fp32, (B,S), or NULL): -inf for a
+ *                           key that no row sees (left out of the statistics), 0 for the others; no other values.
+ *   mta_softmax_mix_pv_fwd: O = (W2 softmax(x)) V (mta_headmix_softmax_*_fwd with w1 = NULL, then mta_causal_pv_*_fwd, the probabilities rounded as
+ *                           these store them) from such scores and their statistics, of a call with the same B, H, S, R (the conv's rows),
+ *                           key_bias and first_visible; tri: x in the triangular layout, its group = `group`; w2 (H,H) block diagonal by
+ *                           groups of `group` heads (2 or 4), of the I/O dtype.
+ * The _supported question: 1 when there is a kernel, nothing is launched. */
+int mta_qk_conv_stats_slots(int64_t B, int64_t H, int64_t S, int R);
+int mta_qk_conv_stats_fwd(const void *q, const void *k, const void *w, const void *key_bias, const void *first_visible, void *s_out, void *stats,
+                          int64_t B, int64_t H, int64_t S, int64_t D, int R, int Sk, float scale, int group, int io_dtype, int w_dtype, void *stream);
+int mta_softmax_mix_pv_supported(int64_t H, int64_t S, int64_t D, int group, int io_dtype, int w_dtype, int key_bias);
+int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
+                           int64_t B, int64_t H, int64_t S, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream);
 /* 1 when mta_headmix_softmax_tri_fwd has a kernel for these sizes and dtypes (has_w1 / has_w2: which weights are given;
  * band: with first_visible; key_bias: with a key bias), else 0.  A host-side question: nothing is launched. */
 int mta_headmix_softmax_tri_supported(int64_t C, int64_t S, int group_size, int out_planes, int io_dtype, int w_dtype,

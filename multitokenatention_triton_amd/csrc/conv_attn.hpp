@@ -3,7 +3,7 @@
 // fill_upper belong to it), else the attention output (lse may be NULL).
 #pragma once
 
-#include "common.hpp"
+#include "scores_cut.hpp"
 
 namespace mta {
 struct conv_attn_args {
@@ -19,11 +19,19 @@ struct conv_attn_args {
     bool scores_only;
     hipStream_t st;
     row_strides qs = {0, 0, 0};   // a 1x1 kernel's q where its rows do not follow one another
+    scores_stats stats = {nullptr, nullptr, 0, {1, 1, 0}};   // scores only, conv_scores_stats_dispatch: the rows' statistics
 };
 int conv_attn_mfma_bf16(const conv_attn_args &a);
 int conv_attn_mfma_f16(const conv_attn_args &a);
 inline int conv_attn_mfma_dispatch(int io_dtype, const conv_attn_args &a)
 {
     return io_dtype == MTA_BF16 ? conv_attn_mfma_bf16(a) : io_dtype == MTA_F16 ? conv_attn_mfma_f16(a) : 1;
+}
+// the scores kernel with the statistics of its rows (causal)
+int conv_scores_stats_bf16(const conv_attn_args &a);
+int conv_scores_stats_f16(const conv_attn_args &a);
+inline int conv_scores_stats_dispatch(int io_dtype, const conv_attn_args &a)
+{
+    return io_dtype == MTA_BF16 ? conv_scores_stats_bf16(a) : io_dtype == MTA_F16 ? conv_scores_stats_f16(a) : 1;
 }
 }  // namespace mta

@@ -520,6 +520,38 @@ extern "C" int mta_qk_conv_tri_fwd(const void *q, const void *k, const void *w, 
     return rc == 1 ? MTA_ERR_UNSUPPORTED : rc;
 }
 
+extern "C" int mta_qk_conv_stats_slots(int64_t B, int64_t H, int64_t S, int R)
+{
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535 || R < 1 || R > MTA_MAX_FUSED_KERNEL_R) return 0;
+    bool table;
+    return scores_slots(S, R, scores_cut_of(B * H, S, R, true, table));
+}
+
+// mta_qk_conv_tri_fwd (group > 0) or mta_qk_conv_fwd / mta_qk_conv_band_fwd without a fill (group = 0), causal, that also leaves the maximum and the
+// sum of exponentials of every row's scores item by item
+extern "C" int mta_qk_conv_stats_fwd(const void *q, const void *k, const void *w, const void *key_bias, const void *first_visible, void *s_out, void *stats,
+                                     int64_t B, int64_t H, int64_t S, int64_t D, int R, int Sk, float scale, int group, int io_dtype, int w_dtype, void *stream)
+{
+    if (!q || !k || !w || !s_out || !stats) return MTA_ERR_NULL;
+    if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535) return MTA_ERR_SHAPE;
+    if (group < 0 || (group > 0 && H % group != 0)) return MTA_ERR_GROUP;
+    if (R < 1 || Sk < 1 || R > MTA_MAX_FUSED_KERNEL_R || Sk > MTA_MAX_FUSED_KERNEL_S) return MTA_ERR_KERNEL_SIZE;
+    if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
+    if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(s_out, 16) || !aligned_to(w, dtype_size(w_dtype)) || !aligned_to(stats, 8) ||
+        (key_bias && !aligned_to(key_bias, 4)) || (first_visible && !aligned_to(first_visible, 4)))
+        return MTA_ERR_ALIGN;
+    if (io_dtype == MTA_F32 || w_dtype != io_dtype || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
+    if (group > 0 && (int64_t)group * tri_rowoff((int)S) > 0x7fffffffLL) return MTA_ERR_UNSUPPORTED;  // (32-bit offsets inside a group)
+    bool table;
+    const scores_cut cut = scores_cut_of(B * H, S, R, true, table);
+    conv_attn_args a = {q, k, nullptr, w, s_out, nullptr, B, H, S, D, R, Sk, 1, scale, 0, (const int *)first_visible, group, true, (hipStream_t)stream};
+    a.stats = {(float2 *)stats, (const float *)key_bias, scores_slots(S, R, cut), cut};
+    const int rc = conv_scores_stats_dispatch(io_dtype, a);
+    if (rc == 1 && scores_instance(R, Sk)) return MTA_ERR_KERNEL_SIZE;
+    return rc == 1 ? MTA_ERR_UNSUPPORTED : rc;
+}
+
 // mta_qk_conv_fwd under a band mask: key k of query row p of batch entry b is visible iff first_visible[b, p] <= k <= p
 // (int32, (B, S)); the scores of hidden keys enter the conv as 0.  Causal by construction.
 extern "C" int mta_qk_conv_band_fwd(const void *q, const void *k, const void *w, const void *first_visible, void *s_out,

@@ -7,6 +7,7 @@
 #include <stdlib.h>
 
 #include "conv_attn_lds.hpp"
+#include "scores_cut.hpp"
 
 namespace {
 
@@ -26,31 +27,6 @@ namespace {
 // on long grids, B1 H32 S8192 D128 1004 -> 953, and lost where a workgroup's chain of steps counts, 6x11 B1 H8 S2048 D64 52 -> 70, B1 H32
 // S1300 43 -> 56.
 constexpr int QK_OCC = 3;     // wavefronts per SIMD the kernel is compiled for (three workgroups per CU)
-constexpr int QK_CHUNK = 32;  // key blocks per work item of the kernel when no item table is built
-// with an item table: long and short items (key blocks), and the share of a query block's key range that goes into short
-// ones (MTA_QK_CHUNK_LONG / MTA_QK_CHUNK_SHORT / MTA_QK_SHORT_PERCENT in the environment override them, for comparisons)
-// (long items measured at B2 H16 S4096 D128: 32/32/0 237 us, 16/16/0 231, 64/16/50 238, 48/24/50 228, 52/26/50 227, 48/24/35 243)
-constexpr int QK_SHORT_PERCENT = 50;
-constexpr int ITEM_TABLE_MAX = 768;
-struct qk_chunks { int big, small; };
-// How long the items are, from the launch's key blocks over all heads (768 workgroups are resident).  From 16000 on the grid
-// runs in several rounds whatever the length and 48/24 keeps the starts few; below, items as short as it takes to
-// have two or three per CU, down to one key block, win although each forms the 16 columns ahead of it again: the grid is
-// otherwise a fraction of the chip, each workgroup walking its keys alone.  us, the kernel in a loop, bf16, 48/24 | as short as the rule makes them:
-// B1 H8 S256 D64 3x3 (80 blocks) 10.9 | 6.0; B1 H16 S512 D128 5x5 (448) 19.4 | 9.2; B2 H16 S512 D64 6x11 (896) 20.4 | 12.1;
-// B4 H16 S512 (1792) 22.1 | 17.9; B1 H8 S2048 D64 (2450) 46.1 | 22.9.
-// Where the line lies, 48/24 | 16/8 (two processes a side, which differ by up to 4, at S3712 by 12): B1 H16 S2048 D128 7x7 (5216) 50.4 | 40.0; B1 H32 S2048
-// D64 5x5 (10432) 51.0 | 46.8; B2 H16 S2048 D128 6x11 (10432) 70.5 | 71.0; B1 H16 S3072 D128 3x3 (10688) 62.6 | 62.8; B1 H16 S3712 D64 7x9 (15088)
-// 79.0 | 75.4; B3 H16 S2048 D128 7x7 (15648) 94.8 | 98.5; B1 H16 S4096 D128 7x7 (19104) 116.5 | 117.2; B4 H16 S2048 D64 3x3 (20864) 85.0 | 89.8; B2 H16
-// S3072 D128 6x11 (21376) 144 | 143; B2 H16 S4096 D128 6x11 (38208) 238 | 250.
-inline qk_chunks qk_chunk_rule(int64_t blocks, int64_t head_blocks, int nqb)
-{
-    if (blocks >= 16000) return {48, 24};
-    if (blocks < 600) return {1, 1};
-    int small = (int)std::min<int64_t>(std::max<int64_t>((blocks + 400) / 800, 1), 8);
-    while (head_blocks / small + 2 * nqb > ITEM_TABLE_MAX && small < 24) small *= 2;   // (the table holds one head's items)
-    return {2 * small, small};
-}
 __device__ __forceinline__ uint32_t lds_read4_at(unsigned addr, int off)
 {
     uint32_t v;
@@ -146,14 +122,18 @@ struct item_table {
 // BAND: a mask of the form "key k of query row p is visible iff band_lo[b, p] <= k <= p" - the
 // scores of the hidden keys enter the conv as 0, as the reference's masked_fill ahead of its conv leaves them
 // (mta_attention_triton.py:70-73).
-template <typename T, int D, int R, int SK, bool BAND>
-__global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ Wt,
+// STATS (causal): the statistics of each row's scores of the item, as they are stored (scores_stats): 32 more vector instructions and eight exponentials per
+// eight scores of a lane, us without | with them: bf16 6x11 B2 H16 S4096 D128 248 | 253 (in a loop: the clock), B4 H16 S1024 36.6 | 45.5, B1 H16 S2048 38.2 |
+// 47.6, 7x7 B2 H16 S4096 D64 181 | 209.  With the maximum so far taken at every eight, and a factor for the sum, B2 H16 S4096 took 22 us more.
+template <typename T, int D, int R, int SK, bool BAND, bool STATS>
+__global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 128) ? QK_OCC : 2) void conv_scores_mfma(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ Wt,
                                                            T *__restrict__ O, int S, int causal, float scale, int H, int nqb, int fill_upper,
                                                            unsigned total_wg, unsigned heads, unsigned per_xcd, int jc_len,
-                                                           item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs)
+                                                           item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs, scores_stats st)
 {
     using G = scores_geom<R, SK>;
     constexpr bool RAW = R == 1 && SK == 1;
+    static_assert(!RAW || !STATS, "raw scores have no statistics");
     constexpr int NW = 4, F_NT = 64 * NW, F_SR = 128, RB = F_SR / (16 * NW);   // (RB: blocks of 16 rows per wavefront)
     constexpr int CPR = D / 8;                     // 16-byte chunks per K row
     constexpr int TILE = F_BK * D;                 // elements per K block
@@ -266,6 +246,7 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
     int j_lo = tbl_lo >= 0 ? tbl_lo : jc * jc_len;                // first key block whose outputs this item produces
     const int j_len = tbl_lo >= 0 ? tbl_len : jc_len;
     const int j_end = (j_lo + j_len - 1 < j_last) ? j_lo + j_len - 1 : j_last;
+    float2 *const stats_at = STATS ? st.at + ((int64_t)bh * st.slots + st.cut.index(j_last + 1, j_lo)) * S : nullptr;   // the item's, row 0
     if constexpr (BAND) {
         // Key blocks that lie wholly ahead of the first key any row of this query block sees are skipped: no visible
         // position takes a tap from them, and what they would hold is hidden from every row (left unwritten).  Every
@@ -287,7 +268,13 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         fmin = __builtin_amdgcn_readfirstlane(fmin);
         const int j_first = (fmin > 0 ? fmin : 0) / F_BK;
         if (j_first > j_lo) j_lo = j_first;
-        if (j_lo > j_end) return;
+        if (j_lo > j_end) {
+            if constexpr (STATS) {
+                for (int r = tid; r < G::BQ; r += F_NT)
+                    if (q0 + r < S) stats_at[q0 + r] = make_float2(NO_SCORE, 0.0f);
+            }
+            return;
+        }
     }
     // What the start waits for is asked for at once, this wavefront's rows of Q and the kernel's taps ahead of the first block of K:
     // behind it, the taps waited for the block and Q was asked for when that had come.  With the 32-bit divisions above, scores
@@ -424,7 +411,6 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         stored[h] = tr_ >= G::HR && tr_ < (wave + 1) * 32 && p_ < S;
         o_off[h] = o_offset(p_) + (unsigned)(o_col * (int)sizeof(T));
     }
-    const int crow = q0 - G::HR + pair_row + (kg >> 1);   // this lane's row of the sequence, from the conv on
 
     // four scores of row block rb, keys col .. col + 3, as the tile holds them
     auto score4 = [&](int rb, f32x4 a, int col, bool masked, uint32_t &lo, uint32_t &hi) __attribute__((always_inline)) {
@@ -437,7 +423,8 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         hi = pack2<T>(a2 * scale, a3 * scale);
         if (masked) {
             MTA_KEEP_BRANCH();
-            const int lim = causal ? (prow[rb] < S - 1 ? prow[rb] : S - 1) : S - 1;  // last key kept
+            const int prow_ = STATS ? q0 - G::HR + wave * (16 * RB) + rb * 16 + (opaque_lane(lane) & 15) : prow[rb];   // (formed here: registers)
+            const int lim = causal ? (prow_ < S - 1 ? prow_ : S - 1) : S - 1;  // last key kept
             const int first = BAND ? (flo[rb] > 0 ? flo[rb] : 0) : 0;  // first key kept
             if (col < first || col > lim) lo &= 0xffff0000u;
             if (col + 1 < first || col + 1 > lim) lo &= 0x0000ffffu;
@@ -469,6 +456,68 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         const int cbase = j * F_BK + G::PWR;
         return j >= 0 && cbase + F_BK <= S && (!causal || cbase + F_BK - 1 <= pmin) && (!BAND || cbase >= fmax_w);
     };
+    // STATS, of this lane's keys of the rows of its pair: minus a reference, in powers of two, and the sum of exponentials relative to it
+    float row_neg[2] = {-NO_SCORE, -NO_SCORE}, row_sum[2] = {0.0f, 0.0f};
+    int row_lo[2] = {0, 0};
+    uint64_t hidden = 0;                                              // keys of the block that the key bias hides
+    const float *const kb = STATS && st.key_bias ? st.key_bias + (int64_t)(bh / H) * S : nullptr;
+    float kb_next = 0.0f;
+    auto load_bias = [&](int j) __attribute__((always_inline)) {
+        const int key = j * F_BK + lane;
+        kb_next = kb[key < S ? key : S - 1];
+    };
+    if constexpr (STATS) {
+        if (kb) load_bias(j_lo);
+        if constexpr (BAND) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int p_ = q0 - G::HR + pair_row + h;
+                row_lo[h] = p_ >= 0 && p_ < S ? band_lo[(bh / H) * (int64_t)S + p_] : 0;
+            }
+        }
+    }
+    // Eight scores of the row h of the pair, keys col .., into the row's statistics.  The reference is the maximum of the lane's first eight
+    // (FIRST) and stays: exponentials of what follows may be large, and where they are too large for 32 bits (the sum is infinite or NaN) all of
+    // it is done again with the maximum so far (EVERY), as it is under a band mask, whose rows' first scores may be hidden.
+    constexpr float LOG2E = 1.4426950408889634f;
+    const std::integral_constant<int, 0> rest{};
+    const std::integral_constant<int, 1> first_ones{};
+    const std::integral_constant<int, 2> every{};
+    auto take = [&](auto mode, auto plain_tag, int h, u32x4_t v, int col, uint64_t hide, int shift) __attribute__((always_inline)) {
+        constexpr int MODE = BAND ? 2 : decltype(mode)::value;
+        if (!decltype(plain_tag)::value || BAND || hide != 0) {
+            MTA_KEEP_BRANCH();
+            const uint32_t gone = (uint32_t)(hide >> shift) >> ((opaque_lane(lane) >> 4) * 8) & 255u;
+            const int last = q0 - G::HR + wave * (16 * RB) + cshift + 2 * (opaque_lane(lane) & 15) + h - col, first = BAND ? row_lo[h] - col : 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                constexpr uint32_t NINF = std::is_same<T, bf16_t>::value ? 0xff80u : 0xfc00u;
+                if (2 * u > last || 2 * u < first || (gone >> (2 * u) & 1u)) v[u] = (v[u] & 0xffff0000u) | NINF;
+                if (2 * u + 1 > last || 2 * u + 1 < first || (gone >> (2 * u + 1) & 1u)) v[u] = (v[u] & 0x0000ffffu) | NINF << 16;
+            }
+        }
+        if constexpr (MODE != 0) {
+            float m = -3.402823466e38f;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float x0, x1;
+                unpack2<T>(v[u], x0, x1);
+                asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(m), "v"(x0), "v"(x1));
+            }
+            const float neg = fminf(-m * LOG2E, row_neg[h]);   // (no score yet: NO_SCORE stays)
+            if constexpr (MODE == 2) row_sum[h] *= __builtin_amdgcn_exp2f(neg - row_neg[h]);
+            row_neg[h] = neg;
+        }
+        float sum = row_sum[h];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float x0, x1;
+            unpack2<T>(v[u], x0, x1);
+            sum += __builtin_amdgcn_exp2f(fmaf(x0, LOG2E, row_neg[h]));
+            sum += __builtin_amdgcn_exp2f(fmaf(x1, LOG2E, row_neg[h]));
+        }
+        row_sum[h] = sum;
+    };
     float nan = 0.0f;   // NaN once a product of the key block has met a value that is not finite
     // PLAIN: the key block (its scores and its conv outputs) lies inside the sequence and on or below the diagonal
     // for all 32 rows of this wavefront: no masks and no per-sub-block tests (most blocks of a long sequence)
@@ -495,13 +544,17 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
             }
         }
         if (j < j_end) issue_k(j + 1, Kn);  // lands while this block is being worked on
+        if (STATS && kb) {
+            hidden = __builtin_amdgcn_ballot_w64(kb_next == -INFINITY);
+            if (j < j_end) load_bias(j + 1);
+        }
 
         // ---- S^T = K Q^T, zero above the diagonal / outside the sequence, to the score tile ----
         {
             // Pipelined like the conv phase below: K fragments are read from assembly KLD steps (two 16-key
             // blocks) ahead into a ring of registers, a step being one fragment and the two products it feeds (both row
             // blocks); a block's scores are rounded, scaled, masked and written LAG steps into the next block.
-            constexpr int NSTEP = NCB * KS, KLD = 2 * KS, KSLOT = KLD + 1, LAG = 2;
+            constexpr int NSTEP = NCB * KS, KLD = STATS && D == 128 && (R == 6 || BAND) ? 5 : 2 * KS, KSLOT = KLD + 1, LAG = 2;
             static_assert(NSTEP > KLD && KS >= LAG && NCB % 2 == 0, "pipeline deeper than the work; blocks are written in pairs");
             unsigned ka[KS];
 #pragma unroll
@@ -581,7 +634,7 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         constexpr int NWIN = F_BK / 8;   // groups of eight keys
         constexpr conv_reads plan = G::reads(NWIN);
         constexpr int NREAD = plan.n;
-        constexpr int NLD = 6, NSLOT = NLD + 3, LAG = 2, NACC = 4;   // (LAST takes dwords of the two operands before it)
+        constexpr int NLD = STATS && D == 128 && R == 6 && !BAND ? 3 : 6, NSLOT = NLD + 3, LAG = 2, NACC = 4;   // (LAST takes dwords of the two operands before it)
         static_assert(NREAD > NLD, "pipeline deeper than the work");
         static_assert(G::LEFT || G::NP + (LAG + G::NQ + G::PAIR - 1) / (G::NQ + G::PAIR) <= NACC, "groups in flight share registers");
         const unsigned row0 = lds_addr(tile) + (unsigned)((pair_row - (R - 1)) * G::SLD * (int)sizeof(T));
@@ -628,7 +681,8 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
             if constexpr (w % 2 == 0 || w == NWIN - 1) nan = fmaf(a[0], 0.0f, nan);
             uint32_t lo = pack2<T>(a[0], a[1]), hi = pack2<T>(a[2], a[3]);
             if (!PLAIN && causal && j * F_BK + w * 8 + 7 > pmin) {  // the group touches the diagonal for some row
-                const int col = j * F_BK + w * 8 + (kg & 1) * 4;
+                const int lane_ = STATS ? opaque_lane(lane) : lane;
+                const int col = j * F_BK + w * 8 + (lane_ >> 4 & 1) * 4, crow = q0 - G::HR + wave * (16 * RB) + cshift + 2 * (lane_ & 15) + (lane_ >> 5);   // this lane's row
                 if (col > crow) lo &= 0xffff0000u;
                 if (col + 1 > crow) lo &= 0x0000ffffu;
                 if (col + 2 > crow) hi &= 0xffff0000u;
@@ -646,8 +700,17 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int p_ = q0 - G::HR + pair_row + h, col = j * F_BK + (w - 3) * 8 + o_col;
+                    const u32x4_t eight = {held[2 * h][0], held[2 * h][1], held[2 * h + 1][0], held[2 * h + 1][1]};
                     if (stored[h] && (PLAIN || (col < S && (!causal || fill_upper || col <= p_))))
-                        *reinterpret_cast<u32x4_t *>(o_block + o_off[h] + (w - 3) * 8 * (int)sizeof(T)) = u32x4_t{held[2 * h][0], held[2 * h][1], held[2 * h + 1][0], held[2 * h + 1][1]};
+                        *reinterpret_cast<u32x4_t *>(o_block + o_off[h] + (w - 3) * 8 * (int)sizeof(T)) = eight;
+                    if constexpr (STATS) {
+                        if (w == 3 && j == j_lo) {
+                            MTA_KEEP_BRANCH();
+                            take(first_ones, plain_tag, h, eight, col, hidden, 0);
+                        } else {
+                            take(rest, plain_tag, h, eight, col, hidden, (w - 3) * 8);
+                        }
+                    }
                 }
             }
         };
@@ -754,9 +817,10 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
                 if (want >> u & 1) at[u] = from_float<T>(acc[u]);
         }
     };
+    bool again = false;   // STATS: results have been formed again, the statistics are those of what they were
     auto check = [&](int j) __attribute__((always_inline)) {
         if constexpr (!RAW)
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan != nan) != 0, 0)) form_again(j);
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan != nan) != 0, 0)) form_again(j), again = true;
     };
     for (int j = j_lo;;) {  // block(tag, j, K(j), where K(j+1) goes)
         if (plain(j)) block(std::true_type{}, j, B0, B1);
@@ -767,6 +831,38 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
         else block(std::false_type{}, j, B1, B0);
         check(j);
         if (++j > j_end) break;
+    }
+
+    if constexpr (STATS) {
+        const int lane_ = opaque_lane(lane), kg_ = lane_ >> 4, pair = wave * (16 * RB) + cshift + 2 * (lane_ & 15);   // (nothing of it is kept in registers)
+        if (!BAND) again = again || __builtin_amdgcn_ballot_w64(!(row_sum[0] < 1e30f) || !(row_sum[1] < 1e30f)) != 0;
+        if (__builtin_expect(again, 0)) {   // the statistics of what is stored now, read back
+            __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) row_neg[h] = -NO_SCORE, row_sum[h] = 0.0f;
+#pragma unroll 1
+            for (int j = j_lo; j <= j_end; ++j) {
+                const int key = j * F_BK + lane_;
+                const uint64_t gone = kb ? __builtin_amdgcn_ballot_w64(kb[key < S ? key : S - 1] == -INFINITY) : 0;
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    const int h = n >> 1, col = j * F_BK + (n & 1) * 32 + kg_ * 8;
+                    if (stored[h] && col < S && col <= q0 - G::HR + pair + h)
+                        take(every, std::false_type{}, h, *reinterpret_cast<const u32x4_t *>(o_at + (int64_t)j * F_BK * (int)sizeof(T) + o_off[h] + (n & 1) * 32 * (int)sizeof(T)), col, gone, (n & 1) * 32);
+                }
+            }
+        }
+        // the keys of a row lie with four lanes, 16 apart
+#pragma unroll
+        for (int off = 16; off < 64; off *= 2)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float neg = __shfl_xor(row_neg[h], off), sum = __shfl_xor(row_sum[h], off), least = fminf(neg, row_neg[h]);
+                row_sum[h] = row_sum[h] * __builtin_amdgcn_exp2f(least - row_neg[h]) + sum * __builtin_amdgcn_exp2f(least - neg);
+                row_neg[h] = least;
+            }
+        if (kg_ < 2 && (kg_ == 0 ? stored[0] : stored[1]))
+            stats_at[q0 - G::HR + pair + kg_] = kg_ == 0 ? make_float2(-row_neg[0], row_sum[0]) : make_float2(-row_neg[1], row_sum[1]);
     }
 
     // +0 for the key blocks to the right of the last one visited (all above the diagonal)
@@ -787,7 +883,7 @@ __global__ __launch_bounds__(256, R <= 7 ? QK_OCC : 2) void conv_scores_mfma(con
     }
 }
 
-template <typename T, int D, int R, int SK, bool BAND>
+template <typename T, int D, int R, int SK, bool BAND, bool STATS>
 int launch_scores(const conv_attn_args &a)
 {
     using G = scores_geom<R, SK>;
@@ -796,59 +892,42 @@ int launch_scores(const conv_attn_args &a)
     const int64_t B = a.B, H = a.H, S = a.S;
     const int causal = BAND ? 1 : a.causal, tri_gl = RAW ? 0 : a.tri_gl;
     const int nqb = (int)((S + G::BQ - 1) / G::BQ);
+    static_assert(G::BQ == scores_rows(R), "rows of a query block");
     constexpr int jc_len = QK_CHUNK;
+    bool table;
+    const scores_cut cut = scores_cut_of(B * H, S, R, causal, table);
     int64_t items_per_bh = 0;
-    for (int qb = 0; qb < nqb; ++qb) {
-        const int64_t ql = std::min<int64_t>((int64_t)qb * G::BQ + G::BQ - 1, S - 1);
-        items_per_bh += ((causal ? ql / F_BK : (S - 1) / F_BK) + jc_len) / jc_len;
-    }
-    // the items of a head, longest first (the number of key blocks an item visits, as the kernel computes it)
+    // the items of a head, longest first (the number of key blocks an item visits, as the kernel computes it): long chunks for the first part
+    // of a query block's key range, short ones for the rest
     item_table tbl;
     tbl.n = 0;
-    if (nqb <= 2047 && (S + F_BK - 1) / F_BK <= 2047) {
-        constexpr int MAXLEN = 1023;
-        static thread_local int count[MAXLEN + 2];
-        static thread_local uint32_t items[ITEM_TABLE_MAX];
-        static thread_local int lens[ITEM_TABLE_MAX];
-        // long chunks for the first part of a query block's key range, short ones for the last QK_SHORT_PERCENT of it
-        static const int env_big = [] { const char *e = getenv("MTA_QK_CHUNK_LONG"); return e ? atoi(e) : 0; }();
-        static const int env_small = [] { const char *e = getenv("MTA_QK_CHUNK_SHORT"); return e ? atoi(e) : 0; }();
-        static const int share = [] { const char *e = getenv("MTA_QK_SHORT_PERCENT"); return e ? atoi(e) : QK_SHORT_PERCENT; }();
-        int64_t head_blocks = 0;
-        for (int qb = 0; qb < nqb; ++qb) {
-            const int64_t ql = std::min<int64_t>((int64_t)qb * G::BQ + G::BQ - 1, S - 1);
-            head_blocks += (causal ? ql / F_BK : (S - 1) / F_BK) + 1;
+    constexpr int MAXLEN = 1023;
+    static thread_local int count[MAXLEN + 2];
+    static thread_local uint32_t items[ITEM_TABLE_MAX];
+    static thread_local int lens[ITEM_TABLE_MAX];
+    int n = 0;
+    for (int qb = 0; qb < nqb; ++qb) {
+        const int nk = causal ? scores_key_blocks(qb, G::BQ, (int)S) : (int)((S - 1) / F_BK) + 1, nlong = cut.longs(nk);
+        items_per_bh += cut.items(nk);
+        if (!table) continue;
+        for (int j0 = 0; j0 < nk;) {
+            const int len = j0 < nlong ? std::min(cut.big, nlong - j0) : std::min(cut.small, nk - j0);
+            lens[n] = len;
+            items[n++] = (uint32_t)qb | ((uint32_t)j0 << 11) | ((uint32_t)len << 22);
+            j0 += len;
         }
-        const qk_chunks cut = qk_chunk_rule(B * H * head_blocks, head_blocks, nqb);
-        const int big = env_big ? env_big : cut.big, small = env_small ? env_small : cut.small;
-        int n = 0;
-        bool ok = big >= 1 && small >= 1 && big <= MAXLEN && small <= MAXLEN && share >= 0 && share <= 100;
-        for (int qb = 0; qb < nqb && ok; ++qb) {
-            const int64_t ql = std::min<int64_t>((int64_t)qb * G::BQ + G::BQ - 1, S - 1);
-            const int nk = (int)(causal ? ql / F_BK : (S - 1) / F_BK) + 1;  // key blocks 0 .. j_last
-            const int nshort = std::min(nk, (nk * share / 100 + small / 2) / small * small);
-            const int nlong = nk - nshort;
-            for (int j0 = 0; j0 < nk && ok;) {
-                const int len = j0 < nlong ? std::min(big, nlong - j0) : std::min(small, nk - j0);
-                if (n >= ITEM_TABLE_MAX) { ok = false; break; }
-                lens[n] = len;
-                items[n++] = (uint32_t)qb | ((uint32_t)j0 << 11) | ((uint32_t)len << 22);
-                j0 += len;
-            }
+    }
+    if (n > 1) {
+        std::fill(count, count + MAXLEN + 2, 0);
+        for (int i = 0; i < n; ++i) ++count[lens[i]];
+        int pos = 0;
+        for (int len = MAXLEN + 1; len >= 0; --len) {  // positions: longer items first
+            const int c = count[len];
+            count[len] = pos;
+            pos += c;
         }
-        if (ok && n > 1) {
-            std::fill(count, count + MAXLEN + 2, 0);
-            for (int i = 0; i < n; ++i) ++count[lens[i]];
-            int pos = 0;
-            for (int len = MAXLEN + 1; len >= 0; --len) {  // positions: longer items first
-                const int c = count[len];
-                count[len] = pos;
-                pos += c;
-            }
-            for (int i = n - 1; i >= 0; --i) tbl.e[count[lens[i]]++] = items[i];  // among equal lengths later query blocks first
-            tbl.n = n;
-            items_per_bh = n;
-        }
+        for (int i = n - 1; i >= 0; --i) tbl.e[count[lens[i]]++] = items[i];  // among equal lengths later query blocks first
+        tbl.n = n;
     }
     const int64_t total_wg = B * H * items_per_bh;
     if (total_wg > 0x7ffffff0LL) return MTA_ERR_SHAPE;
@@ -861,18 +940,19 @@ int launch_scores(const conv_attn_args &a)
     const bool by_head = RAW && S % 64 != 0 && S > 3072 && S <= 4096 && (B * H) % 8 != 0 && B * H > 8;
     const int64_t per_xcd = by_head ? (total_wg + 7) / 8 : 0;
     dim3 grid((unsigned)(by_head ? per_xcd * 8 : total_wg));
-    hipLaunchKernelGGL((conv_scores_mfma<T, D, R, SK, BAND>), grid, dim3(256), 0, a.st, (const T *)a.q, (const T *)a.k, (const T *)a.w, (T *)a.o,
+    hipLaunchKernelGGL((conv_scores_mfma<T, D, R, SK, BAND, STATS>), grid, dim3(256), 0, a.st, (const T *)a.q, (const T *)a.k, (const T *)a.w, (T *)a.o,
                        (int)S, causal, a.scale, (int)H, nqb, a.fill_upper, (unsigned)total_wg, (unsigned)(B * H), (unsigned)per_xcd, jc_len, tbl, a.band_lo, tri_gl,
-                       RAW ? a.qs : row_strides{0, 0, 0});
+                       RAW ? a.qs : row_strides{0, 0, 0}, a.stats);
     return launch_status();
 }
 
 // returns 1 when no instantiation covers the kernel size (the caller then uses the general kernel)
-template <typename T, int D, bool BAND> int dispatch_scores(const conv_attn_args &a)
+template <typename T, int D, bool BAND, bool STATS> int dispatch_scores(const conv_attn_args &a)
 {
-    if (a.R == 1 && a.Sk == 1) return launch_scores<T, D, 1, 1, BAND>(a);   // no conv (weights are not read)
+    if constexpr (!STATS)
+        if (a.R == 1 && a.Sk == 1) return launch_scores<T, D, 1, 1, BAND, false>(a);   // no conv (weights are not read)
 #define MTA_SCORES_CASE(r, s) \
-    if (a.R == r && a.Sk == s) return launch_scores<T, D, r, s, BAND>(a);
+    if (a.R == r && a.Sk == s) return launch_scores<T, D, r, s, BAND, STATS>(a);
     MTA_SCORES_CASE(3, 3)
     MTA_SCORES_CASE(3, 5)
     MTA_SCORES_CASE(5, 5)

@@ -59,6 +59,20 @@ bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_onl
     return tiles >= 800 || (!dense && tiles >= 430 && tiles <= 490);
 }
 
+// Whether softmax, mixing and P V in one kernel (softmax_mix_pv.hip) beat softmax + mixing, then P V: its workgroups walk a row's keys, a chain
+// that only a grid of enough blocks of 64 rows (over the groups of heads) hides.  Groups of 2: everywhere.  us of the forward, three kernels | two, bf16 6x11
+// without a mask, groups of 4, D128: 1 block (B1 H4 S64) 16.4 | 17.4, 40 (B2 H16 S296) 24.2 | 23.9, 48 (B2 H8 S768) 35.4 | 39.0, (B1 H4 S3072) 61.6 | 87.0, 56
+// (B2 H16 S448) 29.8 | 28.9, 80 (B1 H16 S1280) 50.9 | 55.2, 96 (B4 H32 S136) 29.0 | 22.5, (B2 H16 S768) 46.9 | 45.1, (B1 H16 S1536) 63.3 | 66.0, 116 (B1 H16
+// S1856) 77.0 | 77.2, 126 (B1 H12 S2688) 114 | 104, 160 (B1 H16 S2500) 138 | 122, 192 (B4 H12 S1024) 74.3 | 74.1, 240 (B4 H16 S900) 94.5 | 88.5, 512 (B2 H16
+// S4096) 521 | 437; D64: 1 (B1 H4 S64) 15.4 | 14.5, 5 (B1 H4 S296) 16.1 | 16.8, 16 (B1 H8 S512) 17.7 | 19.0, 20 (B1 H16 S296) 17.9 | 17.2, 48 (B2 H8 S768) 33.7 |
+// 31.4, (B1 H8 S1536) 41.4 | 43.0, 64 (B1 H16 S1008) 40.3 | 38.8, 80 (B1 H16 S1280) 47.2 | 47.2, 128 (B1 H8 S4096) 147 | 123, 216 (B1 H16 S3400) 186 | 143.
+bool softmax_pv_pays(int64_t planes, int64_t keys, int64_t head_dim, int64_t group)
+{
+    if (group == 2) return true;
+    const int64_t blocks = planes / group * ((keys + 63) / 64);
+    return head_dim == 64 ? blocks >= 80 || keys <= 16 * blocks || keys <= 256 : blocks >= 120 || keys <= 8 * blocks;
+}
+
 int64_t lcm(int64_t a, int64_t b)
 {
     int64_t x = a, y = b;
@@ -202,7 +216,7 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 // ---- inference -------------------------------------------------------------------------------------------------------
 // The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
 // hides (-inf) are zeroed, so that their scores enter the pre-softmax conv as 0, and their V rows too where a post-softmax
-// conv that is not the identity writes into their columns.  `first`: int32 (B,S), a band mask (row p sees the keys
+// conv that is not the identity writes into their columns (`key_bias_hides`: its values are 0 and -inf).  `first`: int32 (B,S), a band mask (row p sees the keys
 // first[p] .. p), applied to the scores inside the first kernel (where the first stage is two: between them) and as -inf inside the softmax kernel, and behind a
 // post-softmax conv that is not the identity the hidden stretch of every row is zeroed again; the caller has checked that
 // the first stage exists.  `empty_rows`: bool (B,S), the rows of the band that see no key (first[p] = p + 1): the softmax
@@ -211,7 +225,7 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
 // the identity, and their rows of the output, where nothing else would, at the end.
 Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &conv_w, const Tensor &w_pre, const Tensor &post_conv_w,
                          const Tensor &w_post, bool causal, bool pre_identity, int64_t pre_group, bool post_conv_identity, bool post_identity,
-                         int64_t post_group, const OptTensor &key_bias_, const OptTensor &first_, const OptTensor &empty_rows_, bool planes,
+                         int64_t post_group, const OptTensor &key_bias_, bool key_bias_hides, const OptTensor &first_, const OptTensor &empty_rows_, bool planes,
                          double dropout, const py::object &hook)
 {
     at::NoGradGuard no_grad;
@@ -253,6 +267,21 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && !has_tangent(v) && dtype == v.scalar_type() &&
                         (as_is || dtype != at::kFloat) && lower_products_supported(dtype, v.sizes(), causal);
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
+
+    // Two kernels: the scores with the statistics of their rows, and softmax, mixing and P V in one, the probabilities in registers only (which
+    // is why the hook hears of the two stages at once).
+    if (causal && pre_identity && post_conv_identity && w2 && qk_kernel && own_pv && dropout <= 0 && !(key_bias && (first || !key_bias_hides)) &&
+        softmax_pv_pays(planes_of[0] * heads, n_keys, v.size(-1), g_post) && stats_route_supported(q, k, conv_w, g_post, *w2, key_bias.has_value())) {
+        const bool tri = !planes && g_post * tri_row_offset(n_keys) < (int64_t(1) << 31);
+        mark("qk_conv");
+        const auto [scores, stats] = qk_conv_stats(q, k, conv_w, scale, g_post, tri, key_bias, first);
+        mark("mix_softmax_mix");
+        mark("pv");
+        Tensor out = softmax_mix_pv(scores, stats, *w2, v, conv_w.size(1), g_post, tri, key_bias, first);
+        if (empty_rows) out.masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
+        mark("end");
+        return result(out);
+    }
 
     // Three kernels with nothing elementwise between them: the two score tensors are nobody else's business, and they travel
     // in the triangular layout (what lies on and below the diagonal only, the rows a workgroup of the softmax stage reads

@@ -451,6 +451,41 @@ inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, co
     return o;
 }
 
+// scores with the statistics of their rows, and what follows from the two: see mta_qk_conv_stats_fwd.  key_bias: 0 and -inf only
+inline bool stats_route_supported(const Tensor &q, const Tensor &k, const Tensor &conv_w, int64_t group, const Tensor &w2, bool key_bias)
+{
+    if (!qk_conv_supported(q, k, conv_w) || w2.scalar_type() != q.scalar_type() || reinterpret_cast<uintptr_t>(ptr(w2)) % 4) return false;
+    const int c = code(q, "Q");
+    return mta_softmax_mix_pv_supported(q.size(1), q.size(2), q.size(3), (int)group, c, c, key_bias) != 0;
+}
+
+// (scores, statistics); tri: in the triangular layout
+inline std::pair<Tensor, Tensor> qk_conv_stats(const Tensor &q_, const Tensor &k_, const Tensor &w_, double scale, int64_t group, bool tri,
+                                               const OptTensor &key_bias, const OptTensor &first)
+{
+    const Tensor q = on_gpu_vectors(q_, "Q"), k = on_gpu_vectors(k_, "K"), w = on_gpu(w_, "W");
+    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3), r = w.size(1);
+    check_conv_weight(w, h);
+    Tensor y = tri ? at::empty({b * h * tri_row_offset(s)}, q.options()) : at::empty({b, h, s, s}, q.options());
+    Tensor stats = at::empty({b * h, mta_qk_conv_stats_slots(b, h, s, (int)r), s, 2}, q.options().dtype(at::kFloat));
+    check(mta_qk_conv_stats_fwd(ptr(q), ptr(k), ptr(w), ptr(key_bias), ptr(first), out_ptr(y), out_ptr(stats), b, h, s, d, (int)r, (int)w.size(2), (float)scale,
+                                tri ? (int)group : 0, code(q, "Q"), code(w, "W"), stream_of(q)),
+          "mta_qk_conv_stats_fwd");
+    return {y, stats};
+}
+
+inline Tensor softmax_mix_pv(const Tensor &x, const Tensor &stats, const Tensor &w2_, const Tensor &v_, int64_t r, int64_t group, bool tri,
+                             const OptTensor &key_bias, const OptTensor &first)
+{
+    const Tensor v = on_gpu_vectors(v_, "V"), w2 = on_gpu(w2_, "weight");
+    check_head_weight(w2, v.size(1));
+    Tensor o = at::empty(v.sizes(), v.options());
+    check(mta_softmax_mix_pv_fwd(ptr(x), ptr(stats), ptr(w2), ptr(key_bias), ptr(first), ptr(v), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), (int)r,
+                                 (int)group, tri, code(x, "scores"), code(w2, "weight"), stream_of(x)),
+          "mta_softmax_mix_pv_fwd");
+    return o;
+}
+
 // Rows of up to three (B,H,S,D) tensors, of any strides, into dense ones of S_out rows, one launch (mta_rows_copy).
 class RowsCopy {
   public:

@@ -1,0 +1,422 @@
+// O = (W2 softmax(x)) V in one pass over the scores:  x is the score tensor behind the conv (16 bits, planes or the triangular layout), the row
+// statistics come from the kernel that wrote it (conv_scores_mfma.hpp), the probabilities exist in registers only.
+//
+// A wavefront owns 16 query rows of a mixing group of G heads and the results of GO of them (GO * D / 16 accumulators).  A step is 32 keys: a
+// lane (row ln, eight keys kg) loads the G heads' scores of its keys, turns them into probabilities - a multiply-add and an exponential
+// each, the row's factor being in the exponent -, rounds them, mixes the G heads key by key on 4x4x4 matrix products, whose contraction
+// lies within a lane, and rounds the result: what the softmax stage would have stored is then in the lane that supplies it as operand of O^T
+// += V^T P^T.  V comes in blocks of 32 keys of GO heads, copied global -> LDS asynchronously a step ahead, read by transpose reads.  The
+// probabilities of the next step are formed between the products of this one.
+// What it saves is writing and reading the probabilities, half of what the three kernels of this route move: bf16 B2 H16 S4096 D128 groups of 4,
+// softmax + mixing 184 us, P V 144 -> 189 (the scores kernel pays 5 to 9 for the statistics); B4 H16 S1024 33 + 23 -> 38; D64 B2 H16 S4096 184 + 135
+// -> 156.  What bounds it: at B2 H16 S4096 D128 108 us without loads, 97 for the scores alone as tiles of 16 rows, 69 for V and the products - they overlap
+// in part only, a barrier a step holding eight wavefronts to the slowest load.  Not better there (us): scores non-temporal 218, blocks of
+// V asked for three steps ahead and one wavefront per SIMD 232, 128 rows 254, results of two of the four heads per workgroup 237 to 273 (twice
+// the exponentials; where the grid is short they win, form_of), packed dot products in place of the 4x4x4 ones (as fast, more vector instructions).
+#include <type_traits>
+
+#include <stdlib.h>
+
+#include "mfma.hpp"
+#include "scores_cut.hpp"
+#include "strip_common.hpp"
+
+namespace {
+using namespace mta;
+
+constexpr int BK = 32;               // keys per step
+constexpr int MOST_KEYS = 1 << 15;   // under a key bias
+
+// 16 independent 4 x 4 x 4 products: a lane's four values of b (one position's) times the matrix whose row l % 4 lane l holds in a
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+template <typename T> __device__ __forceinline__ f32x4 mix4(u32x2 a, u32x2 b)
+{
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (std::is_same<T, bf16_t>::value)
+        return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4_t, a), __builtin_bit_cast(s16x4_t, b), zero, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4_t, a), __builtin_bit_cast(f16x4_t, b), zero, 0, 0, 0);
+}
+template <int N> __device__ __forceinline__ void copies_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+template <int N> __device__ __forceinline__ void lds_wait_upto(u32x2 &a, u32x2 &b) { asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N) : "memory"); }
+// what is asked for behind this is asked for after what is ahead of it: the waits count
+__device__ __forceinline__ void in_order()
+{
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ unsigned lds_at(const void *p) { return (unsigned)(uintptr_t)(lds_void_t *)p; }
+
+// 16 bytes a lane from a buffer of `bytes` bytes, at `at` (past its end: zeros), to LDS.  From a buffer, not from an address: copies
+// from addresses make the compiler wait for everything in flight ahead of any use of a loaded register, these it counts.
+__device__ __forceinline__ void copy_to_lds(const void *from, int bytes, void *to, int at)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(from), 0, bytes, 0x00027000), (lds_void_t *)to, 16, at, 0, 0, 0);
+}
+
+struct pv_args {
+    const void *x, *w2, *v;
+    const float2 *stats;     // [batch * head][slot][row]: scores_stats
+    const float *key_bias;   // (B,S) or NULL
+    const int *band_lo;      // (B,S) or NULL
+    void *o;
+    int S, H, groups, nrb, cus, tri, slots, rows;
+    scores_cut cut;
+    float per_gph, per_rows, per_big, per_small;   // reciprocals of H / G, rows, cut.big, cut.small
+};
+// x / n by the reciprocal of n: exact for x below 2^20 and n below 2^11 (x + 1/2 keeps 1 / 2n away from every multiple, the product is off by 2^-22 of it)
+__device__ __forceinline__ int quotient(int x, float per_n) { return (int)(((float)x + 0.5f) * per_n); }
+
+template <typename T, int D, int G, int GO, int RW, int GR, int OCC, bool KB>
+__global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_args a)
+{
+    constexpr int CPR = D / 8, HEAD = BK * D, TILE = GO * HEAD, GT = 64 * RW, ROUNDS = TILE / 8 / GT, RPH = HEAD / 8 / GT, DB = D / 16, ROWS = 16 * RW;
+    static_assert(RPH >= 1, "whole copy rounds");
+    __shared__ __align__(16) T lds[GR * 2 * TILE];
+    __shared__ uint32_t hidden[KB ? MOST_KEYS / BK : 1];   // a bit per key that the bias hides
+    const int S = a.S, tid = threadIdx.x % GT, grp = GR == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    int bg, rank;
+    if (!longest_first(a.groups * (G / GO), a.nrb, a.cus, bg, rank)) return;
+    const int h0 = bg % (G / GO) * GO;   // the first of the group's heads whose results are formed here
+    bg /= G / GO;
+    const int q0 = (a.nrb - 1 - rank) * ROWS, w0 = q0 + wave * 16, prow = w0 + ln, pc = prow < S ? prow : S - 1;
+    const int b = quotient(bg, a.per_gph), g = bg - b * (a.H / G);   // batch entry, group of its
+    T *const mine = lds + grp * 2 * TILE;
+
+    // the group's scores: a row of head i lies i * between elements behind the first head's (the same distance for the 16 rows of a wavefront)
+    const T *const xg = static_cast<const T *>(a.x) + (a.tri ? (int64_t)bg * (G * tri_rowoff(S)) + G * tri_rowoff(w0 < S ? w0 : S - 1) : ((int64_t)bg * G * S + (w0 < S ? w0 : S - 1)) * S);
+    const int64_t between = a.tri ? tri_rowlen(w0 < S ? w0 : S - 1) : (int64_t)S * S;
+    const unsigned row_at = (unsigned)(pc - (w0 < S ? w0 : S - 1)) * (unsigned)(a.tri ? G * (int)between : S) + kg * 8;
+    const T *const Vg = static_cast<const T *>(a.v) + (int64_t)(bg * G + h0) * S * D;
+
+    // The mixing weights, row lane % 4: of four heads; of two heads twice on the diagonal, for two keys at a time
+    u32x2 wm = {0u, 0u};
+    {
+        const T *const w2 = static_cast<const T *>(a.w2) + (int64_t)(g * G + h0 + lane % GO) * a.H + g * G;
+        if constexpr (G == 4) wm = u32x2{*reinterpret_cast<const uint32_t *>(w2), *reinterpret_cast<const uint32_t *>(w2 + 2)};
+        else wm = lane & 2 ? u32x2{0u, *reinterpret_cast<const uint32_t *>(w2)} : u32x2{*reinterpret_cast<const uint32_t *>(w2), 0u};
+    }
+
+    const int q_last = (q0 + ROWS - 1 < S - 1) ? q0 + ROWS - 1 : S - 1;
+    int j_end = q_last / BK, j0 = 0;
+    int lo = 0, lo_max = 0;
+    if (a.band_lo) {   // the steps ahead of the first key any of these rows sees are not visited (their scores may be undefined)
+        int f = S;
+        for (int r = lane; r < ROWS; r += 64)
+            if (q0 + r < S) f = min(f, a.band_lo[(int64_t)b * S + q0 + r]);
+        lo = first_key(a.band_lo, (int64_t)b * S + pc, pc);
+        int m = lo;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            f = min(f, __shfl_xor(f, off));
+            m = max(m, __shfl_xor(m, off));
+        }
+        f = __builtin_amdgcn_readfirstlane(f);
+        lo_max = __builtin_amdgcn_readfirstlane(m);
+        j0 = min((f > 0 ? f : 0) / BK, j_end);
+    }
+    const int jg = j0 + ((grp - j0) & (GR - 1)), n = jg <= j_end ? (j_end - jg) / GR + 1 : 0, nall = (j_end - j0) / GR + 1;
+
+    const int row0 = tid / CPR;
+    int voff[RPH];
+#pragma unroll
+    for (int r = 0; r < RPH; ++r) {
+        const int row = row0 + r * (GT / CPR);
+        voff[r] = (row * D + ((tid % CPR) ^ v_swizzle<D>(row)) * 8) * (int)sizeof(T);
+    }
+    auto issue_v = [&](int j, int buf) __attribute__((always_inline)) {
+        T *const dst = mine + buf * TILE;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r)
+            copy_to_lds(Vg + (int64_t)(r / RPH) * S * D, S * D * (int)sizeof(T), dst + (r * GT + wave * 64) * 8, voff[r % RPH] + j * HEAD * (int)sizeof(T));
+    };
+    auto load_x = [&](int j, u32x4 (&x)[G]) __attribute__((always_inline)) {   // beyond the row: its start
+        const unsigned at = (j * BK + kg * 8 <= pc ? (unsigned)(j * BK) : 0u - kg * 8) + row_at;
+#pragma unroll
+        for (int i = 0; i < G; ++i) x[i] = *reinterpret_cast<const u32x4 *>(xg + i * between + at);
+    };
+    // Every step asks for the same number of things, behind the last one again for its own: the waits count them.
+    u32x4 x[2][G];   // scores of two steps
+    auto block = [&](int i) { return min(jg + i * GR, j_end); };
+    load_x(block(0), x[0]);
+    in_order();
+    issue_v(block(0), 0);
+    in_order();
+    load_x(block(1), x[1]);
+    in_order();
+
+    // the rows' factors: p = exp2(x log2(e) - c), c = reference + log2(sum), head kg (kg % G) of row ln here, all heads of it in every lane below
+    constexpr float LOG2E = 1.4426950408889634f;
+    float c[G];
+    {
+        const int qb = quotient(pc, a.per_rows), nk = scores_key_blocks(qb, a.rows, S);
+        const int nshort = min(nk, quotient(quotient(nk * a.cut.share, 0.01f) + a.cut.small / 2, a.per_small) * a.cut.small), nlong = nk - nshort;
+        const int items = quotient(nlong + a.cut.big - 1, a.per_big) + quotient(nshort + a.cut.small - 1, a.per_small);   // (scores_cut::items)
+        const float2 *const at = a.stats + ((int64_t)(bg * G + kg % G) * a.slots) * S + pc;
+        float m = NO_SCORE, l = 0.0f;
+        constexpr int AT_ONCE = 8;
+        for (int i = 0; i < items; i += AT_ONCE) {
+            float2 s[AT_ONCE];
+#pragma unroll
+            for (int k = 0; k < AT_ONCE; ++k) s[k] = at[(int64_t)min(i + k, items - 1) * S];
+            float most = m;
+#pragma unroll
+            for (int k = 0; k < AT_ONCE; ++k) most = fmaxf(most, s[k].x);
+            l *= __builtin_amdgcn_exp2f(m - most);
+#pragma unroll
+            for (int k = 0; k < AT_ONCE; ++k) l += i + k < items ? s[k].y * __builtin_amdgcn_exp2f(s[k].x - most) : 0.0f;
+            m = most;
+        }
+        // (a row that sees no key: NaN, as the softmax of -inf alone gives)
+        const float cv = l == 0.0f ? __builtin_nanf("") : m + __builtin_amdgcn_logf(l);
+#pragma unroll
+        for (int i = 0; i < G; ++i) c[i] = __shfl(cv, (i << 4) + ln);
+    }
+    if constexpr (KB) {   // a bit per key that the bias hides
+        const float *const kb = a.key_bias + (int64_t)b * S;
+        for (int w = (int)(threadIdx.x >> 6); w < (j_end + 2) / 2; w += RW * GR) {
+            const uint64_t h = __builtin_amdgcn_ballot_w64(kb[min(w * 64 + lane, S - 1)] == -INFINITY);
+            if (lane == 0) reinterpret_cast<uint2 *>(hidden)[w] = make_uint2((uint32_t)h, (uint32_t)(h >> 32));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    f32x4 oacc[GO][DB];
+#pragma unroll
+    for (int i = 0; i < GO; ++i)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[i][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int vrow = kg * 8 + (ln >> 2), vat = vrow * D + ((((ln & 3) >> 1) ^ v_swizzle<D>(vrow)) * 8) + (ln & 1) * 4;
+    unsigned va[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) va[db] = lds_at(mine + (vat ^ (db * 16)));
+    constexpr uint32_t NINF = std::is_same<T, bf16_t>::value ? 0xff80ff80u : 0xfc00fc00u;
+    auto hide = [&](u32x4 (&xs)[G], const uint32_t (&keep)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) xs[i][d] = (xs[i][d] & keep[d]) | (NINF & ~keep[d]);
+    };
+    // what a mask hides among the scores of step j becomes -inf
+    auto masks = [&](int j, u32x4 (&xs)[G]) __attribute__((always_inline)) {
+        if (j * BK + BK - 1 > w0 || j * BK < lo_max) {   // keys beyond the row, or ahead of its first one
+            asm volatile("" ::: "memory");
+            const int key = j * BK + kg * 8;
+            uint32_t keep[4];
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                keep[d] = (key + 2 * d <= pc && key + 2 * d >= lo ? 0xffffu : 0u) | (key + 2 * d + 1 <= pc && key + 2 * d + 1 >= lo ? 0xffff0000u : 0u);
+            hide(xs, keep);
+        }
+        if constexpr (KB) {
+            const uint32_t all = __builtin_amdgcn_readfirstlane(hidden[j]);
+            if (all != 0) {
+                asm volatile("" ::: "memory");
+                const uint32_t bits = all >> (kg * 8);
+                uint32_t keep[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) keep[d] = (bits >> (2 * d) & 1u ? 0u : 0xffffu) | (bits >> (2 * d + 1) & 1u ? 0u : 0xffff0000u);
+                hide(xs, keep);
+            }
+        }
+    };
+    // Scores -> mixed probabilities as operands, in 32 pieces of a few instructions, four for a key: the probabilities of half the heads, of the
+    // others, rounded and packed; mixed; rounded and packed key by key.
+    float e[4];
+    u32x2 pk;
+    f32x4 mx[2];
+    auto piece = [&](auto kc, const u32x4 (&xs)[G], u32x4 (&p)[G]) __attribute__((always_inline)) {
+        constexpr int t = decltype(kc)::value / 4, s = decltype(kc)::value % 4, d = t / 2, u = t % 2;   // (two heads: keys t and t + 1 at an even t)
+        auto prob = [&](int h, int hi) {
+            float x0, x1;
+            unpack2<T>(xs[h][d], x0, x1);
+            return __builtin_amdgcn_exp2f(fmaf(hi ? x1 : x0, LOG2E, -c[h]));
+        };
+        if constexpr (G == 4) {
+            if constexpr (s < 2) e[2 * s] = prob(2 * s, u), e[2 * s + 1] = prob(2 * s + 1, u);
+            else if constexpr (s == 2) pk = u32x2{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3])};
+            else mx[u] = mix4<T>(wm, pk);
+            if constexpr (s == 3 && u == 1) {
+#pragma unroll
+                for (int o = 0; o < GO; ++o) p[o][d] = pack2<T>(mx[0][o], mx[1][o]);
+            }
+        } else if constexpr (u == 0) {
+            if constexpr (s < 2) e[2 * s] = prob(0, s), e[2 * s + 1] = prob(1, s);
+            else if constexpr (s == 2) pk = u32x2{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3])};
+            else mx[0] = mix4<T>(wm, pk);
+        } else if constexpr (s == 3) {
+#pragma unroll
+            for (int o = 0; o < GO; ++o) p[o][d] = pack2<T>(mx[0][o], mx[0][2 + o]);
+        }
+    };
+    // The products of a step and, between them, the probabilities of the next one: matrix cores, LDS and vector units side by side.
+    auto product = [&](auto bufc, const u32x4 (&p)[G], const u32x4 (&xs)[G], u32x4 (&pn)[G]) __attribute__((always_inline)) {
+        constexpr int buf = decltype(bufc)::value, N = GO * DB, AHEAD = (GO * D > 256 && OCC == 2) || OCC == 3 ? 2 : 4;
+        u32x2 fa[AHEAD + 1], fb[AHEAD + 1];
+        auto read = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, off = (buf * TILE + i / DB * HEAD) * (int)sizeof(T);
+            fa[i % (AHEAD + 1)] = lds_load_tr8_at(va[i % DB], off);
+            fb[i % (AHEAD + 1)] = lds_load_tr8_at(va[i % DB], off + 4 * D * (int)sizeof(T));
+        };
+        static_for<AHEAD>(read);
+        static_for<N>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            if constexpr (i + AHEAD < N) read(std::integral_constant<int, i + AHEAD>{});
+            constexpr int younger = 2 * ((i + AHEAD < N ? i + AHEAD : N - 1) - i);
+            lds_wait_upto<younger>(fa[i % (AHEAD + 1)], fb[i % (AHEAD + 1)]);
+            struct { u32x2 a, b; } both = {fa[i % (AHEAD + 1)], fb[i % (AHEAD + 1)]};
+            mma16(oacc[i / DB][i % DB], __builtin_bit_cast(frag8<T>, both), __builtin_bit_cast(frag8<T>, p[i / DB]));
+            static_for<32 / N>([&](auto kc) __attribute__((always_inline)) { piece(std::integral_constant<int, i * (32 / N) + decltype(kc)::value>{}, xs, pn); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // Step i: key block jg + i GR; its probabilities are formed, its block of V was asked for a step ago, the scores of the next one one and a
+    // half.  Behind the barrier nobody reads the other buffer any more; registers whose scores have become probabilities get those of the
+    // step after the next two.
+    u32x4 p[2][G];
+    auto live = [&](int i) { return i < n && (jg + i * GR) * BK <= w0 + 15; };
+    auto step = [&](auto nowc, auto full, int i) __attribute__((always_inline)) {
+        constexpr int now = decltype(nowc)::value;
+        constexpr bool FULL = decltype(full)::value;   // three more steps follow, and no row of this wavefront ends before the next one
+        copies_wait<G>();                              // V of this step has come (behind it only G loads of scores)
+        wg_barrier();
+        const int j = jg + i * GR;
+        issue_v(FULL ? j + GR : block(i + 1), now ^ 1);
+        in_order();
+        if (FULL || live(i)) {   // (behind the last step of a row: probabilities of scores that nobody wants)
+            if (FULL || live(i + 1)) masks(j + GR, x[now ^ 1]);
+            product(nowc, p[now], x[now ^ 1], p[now ^ 1]);
+        }
+        load_x(FULL ? j + 3 * GR : block(i + 3), x[now ^ 1]);
+        in_order();
+    };
+    if (live(0)) {
+        masks(jg, x[0]);
+        static_for<32>([&](auto kc) __attribute__((always_inline)) { piece(kc, x[0], p[0]); });
+    }
+    in_order();
+    load_x(block(2), x[0]);
+    in_order();
+    const std::integral_constant<int, 0> b0{};
+    const std::integral_constant<int, 1> b1{};
+    const int full = n - 4 - (ROWS / BK + GR) / GR;   // (the first wavefront's rows end ROWS / BK key blocks before the last one's)
+    int i = 0;
+    for (; i + 2 <= full; i += 2) {
+        step(b0, std::true_type{}, i);
+        step(b1, std::true_type{}, i + 1);
+    }
+    for (; i < nall; i += 2) {
+        step(b0, std::false_type{}, i);
+        if (i + 1 < nall) step(b1, std::false_type{}, i + 1);
+    }
+    copies_wait<0>();   // (nothing may come into LDS that is no longer this workgroup's)
+    if constexpr (GR > 1) {   // the groups' sums, the upper half's to the lower half by way of the buffers until one is left
+        static_assert(GR * 2 * TILE * sizeof(T) >= (size_t)GR / 2 * GT * GO * DB * 16, "half the groups' sums fit the buffers");
+        __syncthreads();
+        f32x4 *const part = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+        for (int h = GR / 2; h > 0; h /= 2) {
+            if (grp >= h && grp < 2 * h) {
+#pragma unroll
+                for (int k = 0; k < GO * DB; ++k) part[((grp - h) * GO * DB + k) * GT + tid] = oacc[k / DB][k % DB];
+            }
+            __syncthreads();
+            if (grp < h) {
+#pragma unroll
+                for (int k = 0; k < GO * DB; ++k) oacc[k / DB][k % DB] += part[(grp * GO * DB + k) * GT + tid];
+            }
+            if (h > 1) __syncthreads();
+        }
+        if (grp > 0) return;
+    }
+    if (prow >= S) return;
+#pragma unroll
+    for (int h = 0; h < GO; ++h)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[h][db][v]);
+            *reinterpret_cast<quad *>(static_cast<T *>(a.o) + ((int64_t)(bg * G + h0 + h) * S + prow) * D + db * 16 + kg * 4) = out;
+        }
+}
+
+// ---- which form --------------------------------------------------------------------------------------------------------
+// Of how many heads a workgroup forms the results, of how many rows, and how many groups of wavefronts share the keys: WHOLE all, 64, two; HALF_LONG half of them,
+// 64, one (groups of 4 at D64: all, 32, two); HALF_SHORT half, 32, two; HALF_SPLIT half, 16, four.  With half of the heads the exponentials
+// are formed twice, but there are twice the workgroups and a step is shorter; more groups of wavefronts shorten the chain of steps.  The
+// line runs by n, the 64-row blocks over the groups of heads.  us of the forward, bf16 6x11, the four in this order:
+//   groups of 4, D128  n 8 (B1 H4 S512) 34.9 | 30.0 | 24.1 | 22.4, 36 (B1 H16 S576) 42.5 | 38.5 | 31.4 | 31.3, 48 (B2 H16 S384) 37.7 | 32.9 | 28.4 | 33.0, 128 (B2 H16 S1024) 70.9 |
+//     65.0 | 54.4 | 79.6, 192 (B4 H12 S1001) 91.6 | 88.5 | 88.7 | 127, 256 (B4 H16 S1024) 86.6 | 82.2 | 87.5 | 144, 464 (B4 H16 S1856) 203 | 222 | 242 | 388, 512 (B2 H16 S4096) 437 | 485 | 516 | 781
+//   groups of 4, D64   n 8 27.9 | 23.3 | 20.9 | 18.3, 64 (B1 H16 S1008) 54.0 | 47.1 | 42.7 | 39.5, 128 59.3 | 52.4 | 47.9 | 53.8, 192 75.6 | 70.4 | 69.9 | 81.5, 256 73.6 | 67.2 | 75.6 | 90.6, 464 167 | 173 | 190 | 229
+//   groups of 2, D128  n 16 (B1 H4 S512) 23.1 | 22.2 | 18.3 | 17.5, 64 (B1 H4 S2048) 56.1 | 56.7 | 42.7 | 40.4, 72 (B1 H16 S576) 29.7 | 28.7 | 25.0 | 27.9, 128 (B1 H16 S1008) 46.5 | 45.6 | 39.8 |
+//     46.3, 256 (B1 H16 S2048) 83.1 | 85.3 | 85.1 | 101, 512 (B1 H32 S2048) 118 | 130 | 136 | 176;  D64  64 47.7 | 53.0 | 39.6 | 34.3, 72 25.8 | 25.9 | 22.5 | 22.0, 128 40.4 | 42.2 | 36.4 | 38.5, 256 72.7 | 78.3 | 74.8 | 80.5
+enum pv_form { WHOLE = 1, HALF_LONG, HALF_SHORT, HALF_SPLIT };
+
+pv_form form_of(int64_t groups, int64_t S, int D, int G)
+{
+    static const int force = [] { const char *e = getenv("MTA_SOFTMAX_PV_FORM"); return e ? atoi(e) : 0; }();   // (comparison switch: always that form)
+    if (force >= WHOLE && force <= HALF_SPLIT) return (pv_form)force;
+    const int64_t n = groups * ((S + 63) / 64);
+    if (G == 2) return n >= 200 ? WHOLE : n > 64 ? HALF_SHORT : HALF_SPLIT;
+    if (n >= 400) return WHOLE;
+    if (D == 64) return n >= 190 ? HALF_LONG : n > 64 ? HALF_SHORT : HALF_SPLIT;
+    return n >= 240 ? HALF_LONG : n > 36 ? HALF_SHORT : HALF_SPLIT;
+}
+
+template <typename T, int D, int G, int GO, int RW, int GR, int OCC> int go(pv_args a, int64_t groups, int resident, hipStream_t st)
+{
+    const int64_t blocks = (a.S + 16 * RW - 1) / (16 * RW), wg = (groups * (G / GO) * blocks + 7) / 8 * 8;
+    if (wg > 0x7fffffffLL) return MTA_ERR_SHAPE;
+    a.groups = (int)groups, a.nrb = (int)blocks;
+    a.cus = wg <= (int64_t)resident * device_cu_count() ? device_cu_count() / 8 : 0;
+    if (a.key_bias) hipLaunchKernelGGL((softmax_mix_pv<T, D, G, GO, RW, GR, OCC, true>), dim3((unsigned)wg), dim3(64 * RW * GR), 0, st, a);
+    else hipLaunchKernelGGL((softmax_mix_pv<T, D, G, GO, RW, GR, OCC, false>), dim3((unsigned)wg), dim3(64 * RW * GR), 0, st, a);
+    return launch_status();
+}
+
+template <typename T, int D, int G> int launch(const pv_args &a, int64_t groups, hipStream_t st)
+{
+    switch (form_of(groups, a.S, D, G)) {
+    case WHOLE: return go<T, D, G, G, 4, 2, 2>(a, groups, 1, st);
+    case HALF_LONG:
+        if constexpr (G == 4 && D == 64) return go<T, D, G, G, 2, 2, 2>(a, groups, 2, st);
+        else return go<T, D, G, G / 2, 4, 1, 3>(a, groups, 3, st);
+    case HALF_SHORT: return go<T, D, G, G / 2, 2, 2, D == 64 ? 3 : 2>(a, groups, D == 64 ? 3 : 2, st);
+    default: return go<T, D, G, G / 2, 1, 4, D == 64 ? 2 : 1>(a, groups, D == 64 ? 2 : 1, st);
+    }
+}
+template <typename T> int launch_type(const pv_args &a, int64_t groups, int64_t D, int group, hipStream_t st)
+{
+    if (D == 64) return group == 2 ? launch<T, 64, 2>(a, groups, st) : launch<T, 64, 4>(a, groups, st);
+    return group == 2 ? launch<T, 128, 2>(a, groups, st) : launch<T, 128, 4>(a, groups, st);
+}
+}  // namespace
+
+extern "C" int mta_softmax_mix_pv_supported(int64_t H, int64_t S, int64_t D, int group, int io_dtype, int w_dtype, int key_bias)
+{
+    return (io_dtype == MTA_BF16 || io_dtype == MTA_F16) && w_dtype == io_dtype && (group == 2 || group == 4) && H > 0 && H % group == 0 && S > 0 && S % 8 == 0 &&
+           S <= (key_bias ? MOST_KEYS : 1 << 19) && (D == 64 || D == 128);
+}
+
+extern "C" int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
+                                      int64_t B, int64_t H, int64_t S, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream)
+{
+    if (!x || !stats || !w2 || !v || !o) return MTA_ERR_NULL;
+    if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535) return MTA_ERR_SHAPE;
+    if (R < 1 || R > MTA_MAX_FUSED_KERNEL_R) return MTA_ERR_KERNEL_SIZE;
+    if (group <= 0 || H % group != 0) return MTA_ERR_GROUP;
+    if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
+    if (!aligned_to(x, 16) || !aligned_to(v, 16) || !aligned_to(o, 16) || !aligned_to(stats, 8) || !aligned_to(w2, 4) || (key_bias && !aligned_to(key_bias, 4)) ||
+        (first_visible && !aligned_to(first_visible, 4)))
+        return MTA_ERR_ALIGN;
+    if (!mta_softmax_mix_pv_supported(H, S, D, group, io_dtype, w_dtype, key_bias != nullptr)) return MTA_ERR_UNSUPPORTED;
+    bool table;
+    const scores_cut cut = scores_cut_of(B * H, S, R, true, table);
+    const int rows = scores_rows(R);
+    const pv_args a{x, w2, v, (const float2 *)stats, (const float *)key_bias, (const int *)first_visible, o, (int)S, (int)H, 0, 0, 0, tri != 0,
+                    scores_slots(S, R, cut), rows, cut, (float)group / (float)H, 1.0f / (float)rows, 1.0f / (float)cut.big, 1.0f / (float)cut.small};
+    const int64_t groups = B * (H / group);
+    return io_dtype == MTA_BF16 ? launch_type<bf16_t>(a, groups, D, group, (hipStream_t)stream) : launch_type<f16_t>(a, groups, D, group, (hipStream_t)stream);
+}

@@ -342,9 +342,10 @@ class MTAAttentionTriton(nn.Module):
         return (_weight_of(modules["mta_conv_triton"]), _weight_of(modules["wpsm_triton"]),
                 _weight_of(modules["mta_conv_after_sm_triton"]), _weight_of(modules["wposm_triton"]))
 
-    def _forward_native(self, xq, xk, xv, key_bias=None, first_visible=None, empty_rows=None):
+    def _forward_native(self, xq, xk, xv, key_bias=None, first_visible=None, empty_rows=None, key_bias_hides=True):
         """Both routes of the module docstring in native code (csrc/host/mta_host.cpp).  ``key_bias``: fp32 (B,Sk), added to
-        the mixed scores ahead of the softmax; the K and V rows of the keys it hides count as zeros.  ``first_visible``:
+        the mixed scores ahead of the softmax; the K and V rows of the keys it hides count as zeros.  ``key_bias_hides``: its
+        values are 0 and -inf.  ``first_visible``:
         int32 (B,S), a band mask (row p sees the keys first_visible[p] .. p); the caller has checked that the first kernel
         exists.  ``empty_rows``: bool (B,S) or None, the rows of the band that see no key (first_visible[p] = p + 1)."""
         weights = self._weights()
@@ -357,7 +358,7 @@ class MTAAttentionTriton(nn.Module):
                                          self._stage_hook)
         st = self._current_structure()
         return host.forward_inference(xq, xk, xv, *weights, self.causal, st.pre_head_identity, st.pre_head_group or 0, st.post_conv_identity,
-                                      st.post_head_identity, st.post_head_group or 0, key_bias, first_visible, empty_rows,
+                                      st.post_head_identity, st.post_head_group or 0, key_bias, key_bias_hides, first_visible, empty_rows,
                                       self.score_layout == "planes", dropout, self._stage_hook)
 
     def _forward_stagewise_planes(self, xq, xk, xv, mask_planes, mask_additive=None, mask_empty_rows=False):
@@ -472,7 +473,7 @@ class MTAAttentionTriton(nn.Module):
                     bias = torch.where(mask, 0.0, float("-inf")).to(torch.float32)
                 else:
                     bias = mask.type(xq.dtype).to(torch.float32)   # the reference adds it in the I/O dtype
-                return self._forward_native(xq, xk, xv, key_bias=_pad_rows(bias, 0.0).contiguous())
+                return self._forward_native(xq, xk, xv, key_bias=_pad_rows(bias, 0.0).contiguous(), key_bias_hides=mask.dtype == torch.bool)
             # a 4-D mask, the same for all heads, of one of two forms goes into the kernels without a (B,H,S,S) tensor:
             # "causal rule + hidden keys" per batch entry (key padding: a key bias and zeroed K and V rows, as for the
             # 2-D mask above) and "row p sees the keys first[p] .. p" (sliding windows, packed documents: one int32 per

@@ -467,6 +467,15 @@ def _band_arg(first_visible, b, s):
     return first_visible
 
 
+def _bias_arg(key_bias, n, s):
+    if key_bias is None:
+        return None
+    key_bias = _device_tensor(key_bias, "key_bias")
+    if key_bias.dtype != torch.float32 or tuple(key_bias.shape) != (n, s) or not key_bias.is_contiguous():
+        raise ValueError(f"key_bias must be a contiguous fp32 tensor of shape ({n},{s})")
+    return key_bias
+
+
 def tri_route_supported(q: torch.Tensor, k: torch.Tensor, conv_weight: torch.Tensor, group: int, w1, w2, band: bool,
                         out_planes: bool = False, key_bias: bool = False) -> bool:
     """Whether the triangular-layout kernels exist for these tensors (host-side questions to the library);
@@ -525,10 +534,7 @@ def headmix_softmax_tri(x: torch.Tensor, w1: Optional[torch.Tensor], w2: Optiona
     if not present or any(w.dtype != present[0].dtype for w in present):
         raise TypeError("one or two weights of one dtype")
     first_visible = _band_arg(first_visible, n, s)
-    if key_bias is not None:
-        key_bias = _device_tensor(key_bias, "key_bias")
-        if key_bias.dtype != torch.float32 or tuple(key_bias.shape) != (n, s) or not key_bias.is_contiguous():
-            raise ValueError(f"key_bias must be a contiguous fp32 tensor of shape ({n},{s})")
+    key_bias = _bias_arg(key_bias, n, s)
     y = torch.empty((n, c, s, s), dtype=x.dtype, device=x.device) if out_planes else torch.empty_like(x)
     with torch.cuda.device(x.device):
         rc = _lib.load().mta_headmix_softmax_tri_fwd(
@@ -554,6 +560,53 @@ def causal_pv_tri(p: torch.Tensor, v: torch.Tensor, group: int, first_visible: O
                                                first_visible.data_ptr() if first_visible is not None else None,
                                                out.data_ptr(), b, h, s, d, int(group), _code(p, "P"), _stream(p))
     _lib.check(rc, "mta_causal_pv_tri_fwd")
+    return out
+
+
+def qk_conv_stats(q: torch.Tensor, k: torch.Tensor, weight: torch.Tensor, scale: float, group: int, tri: bool = True,
+                  key_bias: Optional[torch.Tensor] = None, first_visible: Optional[torch.Tensor] = None):
+    """``qk_conv_tri`` (or with ``tri=False`` the causal ``qk_conv`` without a fill), and the statistics of the rows for
+    ``softmax_mix_pv``; ``key_bias``: fp32 (B,S) of 0 and -inf; see mta_qk_conv_stats_fwd."""
+    q, k, weight = _device_tensor(q, "Q"), _device_tensor(k, "K"), _device_tensor(weight.detach(), "W")
+    if q.dim() != 4 or q.shape != k.shape or q.dtype != k.dtype:
+        raise ValueError(f"Q and K must share a (B,H,S,D) shape and dtype, got {tuple(q.shape)}, {tuple(k.shape)}")
+    b, h, s, d = q.shape
+    assert weight.dim() == 3 and weight.shape[0] == h, "conv weight must be (H,R,S)"
+    first_visible = _band_arg(first_visible, b, s)
+    key_bias = _bias_arg(key_bias, b, s)
+    out = torch.empty((b * h * tri_row_offset(s),) if tri else (b, h, s, s), dtype=q.dtype, device=q.device)
+    lib = _lib.load()
+    stats = torch.empty((b * h, lib.mta_qk_conv_stats_slots(b, h, s, weight.shape[1]), s, 2), dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        rc = lib.mta_qk_conv_stats_fwd(q.data_ptr(), k.data_ptr(), weight.data_ptr(), key_bias.data_ptr() if key_bias is not None else None,
+                                       first_visible.data_ptr() if first_visible is not None else None, out.data_ptr(), stats.data_ptr(),
+                                       b, h, s, d, weight.shape[1], weight.shape[2], float(scale), int(group) if tri else 0,
+                                       _code(q, "Q"), _code(weight, "W"), _stream(q))
+    _lib.check(rc, "mta_qk_conv_stats_fwd")
+    return out, stats
+
+
+def softmax_mix_pv(x: torch.Tensor, stats: torch.Tensor, w2: torch.Tensor, v: torch.Tensor, rows: int, group: int,
+                   key_bias: Optional[torch.Tensor] = None, first_visible: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """(W2 softmax(x)) V from the scores and statistics of ``qk_conv_stats`` (the same mask, ``rows``: of its conv kernel), V
+    (B,H,S,D); see mta_softmax_mix_pv_fwd."""
+    x, v, w2 = _device_tensor(x, "scores"), _device_tensor(v, "V"), _device_tensor(w2.detach(), "weight")
+    b, h, s, d = v.shape
+    tri = x.dim() == 1
+    lib = _lib.load()
+    if x.dtype != v.dtype or tuple(x.shape) != ((b * h * tri_row_offset(s),) if tri else (b, h, s, s)):
+        raise ValueError(f"scores {tuple(x.shape)} do not belong to a V of shape {tuple(v.shape)}")
+    if stats.dtype != torch.float32 or not stats.is_contiguous() or tuple(stats.shape) != (b * h, lib.mta_qk_conv_stats_slots(b, h, s, rows), s, 2):
+        raise ValueError(f"statistics {tuple(stats.shape)} do not belong to a V of shape {tuple(v.shape)}")
+    assert tuple(w2.shape) == (h, h), f"Weight must be ({h},{h}), got {tuple(w2.shape)}"
+    first_visible = _band_arg(first_visible, b, s)
+    key_bias = _bias_arg(key_bias, b, s)
+    out = torch.empty_like(v)
+    with torch.cuda.device(v.device):
+        rc = lib.mta_softmax_mix_pv_fwd(x.data_ptr(), stats.data_ptr(), w2.data_ptr(), key_bias.data_ptr() if key_bias is not None else None,
+                                        first_visible.data_ptr() if first_visible is not None else None, v.data_ptr(), out.data_ptr(),
+                                        b, h, s, d, int(rows), int(group), int(tri), _code(x, "scores"), _code(w2, "weight"), _stream(v))
+    _lib.check(rc, "mta_softmax_mix_pv_fwd")
     return out
 
 

@@ -617,6 +617,105 @@ def test_triangular_layout_stages_equal_the_plane_layout(pkg, case):
                                          first_visible=first), o_plane)
 
 
+# B, H, S, D, R, Sk, group, dtype, mask: every form of the kernel (by the number of 64-row blocks over the groups), the shortest rows, edges of its
+# 16 rows x 32 keys and of the scores kernel's pieces
+STATS_CASES = [
+    (1, 4, 8, 128, 3, 3, 4, torch.bfloat16, None), (1, 2, 40, 64, 5, 5, 2, torch.float16, None), (2, 4, 72, 64, 3, 5, 4, torch.bfloat16, "keys"),
+    (1, 4, 520, 128, 6, 11, 4, torch.float16, None), (2, 4, 1160, 128, 6, 11, 4, torch.bfloat16, "documents"), (1, 8, 1032, 64, 7, 9, 4, torch.float16, "keys"),
+    (4, 32, 136, 128, 6, 11, 4, torch.bfloat16, None), (4, 64, 264, 128, 3, 3, 4, torch.float16, "keys"), (4, 64, 456, 128, 5, 7, 4, torch.bfloat16, "window"),
+    (4, 32, 328, 64, 11, 15, 4, torch.bfloat16, "ragged"), (4, 64, 424, 64, 6, 11, 4, torch.float16, None), (2, 64, 200, 128, 7, 7, 2, torch.bfloat16, "keys"),
+    (2, 32, 136, 128, 3, 3, 2, torch.float16, "window"), (4, 64, 136, 64, 5, 5, 2, torch.bfloat16, None), (2, 32, 232, 64, 6, 11, 2, torch.float16, "documents"),
+    (1, 4, 4168, 64, 7, 7, 4, torch.bfloat16, None),
+]
+
+
+@pytest.mark.parametrize("case", STATS_CASES)
+def test_softmax_mix_pv(pkg, case):
+    """Softmax, mixing and P V in one kernel over the scores kernel's rows and statistics, in both layouts.  Against 64 bits from the same
+    stored scores.  A probability and a mixed probability are rounded once each (u of their size, half a step of the smallest number at least), so
+    is a result; the exponents, below 64, are formed in fp32 and the sums are fp32 sums of s terms: 2^-17 of the sum of sizes covers both."""
+    b, h, s, d, r, sk, group, dtype, kind = case
+    print(f"softmax mix pv case={case}", flush=True)
+    ops = pkg.ops
+    g = torch.Generator().manual_seed(91)
+    q, k, v = (t.cuda() for t in O.seeded_qkv(b, h, s, d, dtype, seed=92))
+    q = q * 2
+    w = (torch.randn(h, r, sk, generator=g) * 0.2).to(dtype).cuda()
+    w2 = O.block_diag_head_weight(h, group, 0.3, g, dtype).cuda()
+    at = torch.arange(s, device="cuda")
+    seen = (at[None, :] <= at[:, None])[None].expand(b, s, s)
+    first = key_bias = None
+    if kind == "keys":          # padding on the right, holes, and in the last entry keys hidden from the start on: rows that see no key
+        keep = at[None, :] < torch.tensor([s - 3 * i for i in range(b)], device="cuda")[:, None]
+        keep[0, 5::7] = False
+        keep[-1, :min(s // 3, 40)] = False
+        key_bias = torch.where(keep, 0.0, float("-inf"))
+        seen = seen & keep[:, None, :]
+    elif kind:
+        first = _band_first(kind, b, s).cuda()
+        first[-1, s // 2:s // 2 + 3] = at[s // 2:s // 2 + 3].int() + 1   # rows that see no key
+        seen = seen & (at[None, None, :] >= first[:, :, None])
+    some = slice(0, group) if h <= 8 else slice(h - group, h)
+    u, least = (2.0 ** -8, 0.0) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -25)
+    got = {}
+    for tri in (True, False):
+        x, stats = ops.qk_conv_stats(q, k, w, d ** -0.5, group, tri, key_bias, first)
+        got[tri] = ops.softmax_mix_pv(x, stats, w2, v, r, group, key_bias, first)
+    assert torch.equal(got[True].nan_to_num(7.0), got[False].nan_to_num(7.0))
+    plane = ops.qk_conv(q, k, w, True, d ** -0.5, fill_upper=False, first_visible=first)
+    assert torch.equal(x[seen[:, None].expand_as(x)], plane[seen[:, None].expand_as(x)])
+    for i in range(b):
+        xs = x[i, some].double().masked_fill(~seen[i], float("-inf"))
+        p = torch.softmax(xs, -1)
+        vd, w2d = v[i, some].double(), w2[some, some].double()
+        mixed = torch.einsum("oi,ipq->opq", w2d, p.nan_to_num(0.0))
+        size = torch.einsum("oi,ipq->opq", w2d.abs(), p.nan_to_num(0.0))
+        empty = ~seen[i].any(-1)
+        want = mixed @ vd
+        bound = (2.02 * u + 2.0 ** -17) * (size @ vd.abs()) + u * want.abs() + least * (w2d.abs().sum(1)[:, None, None] + 2) * vd.abs().sum(-2, keepdim=True)
+        out = got[True][i, some].double()
+        assert out[:, empty].isnan().all()
+        assert ((out - want).abs() <= bound)[:, ~empty].all(), ((out - want).abs() / bound)[:, ~empty].max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_softmax_mix_pv_scores_that_are_not_finite_or_far_apart(pkg, dtype):
+    """A NaN row of Q spoils the rows whose conv window holds it and no other (the others keep their bits); scores that rise along the keys by
+    more than 32 bits hold as exponentials, relative to the row's first, give the softmax all the same."""
+    ops = pkg.ops
+    b, h, s, d, group = 1, 4, 392, 64, 4
+    print(f"softmax mix pv, not finite {dtype}", flush=True)
+    g = torch.Generator().manual_seed(93)
+    q, k, v = (torch.randn(b, h, s, d, generator=g).to(dtype).cuda() for _ in range(3))
+    w = (torch.randn(h, 6, 11, generator=g) * 0.1).to(dtype).cuda()
+    w2 = O.block_diag_head_weight(h, group, 0.3, g, dtype).cuda()
+
+    def run(q_):
+        x, stats = ops.qk_conv_stats(q_, k, w, d ** -0.5, group)
+        return ops.softmax_mix_pv(x, stats, w2, v, 6, group)
+    clean = run(q)
+    for value in (float("nan"), float("inf")):
+        bad = q.clone()
+        bad[0, 1, 200] = value
+        got = run(bad)
+        hit = torch.zeros(s, dtype=torch.bool, device="cuda")
+        hit[200:206] = True
+        assert got[:, :, hit].isnan().all() and torch.equal(got[:, :, ~hit], clean[:, :, ~hit])
+    w1 = torch.zeros_like(w)
+    w1[:, -1, 5] = 1.0
+    rise = torch.linspace(-40, 40, s).to(dtype)[None, None, :, None].expand(b, h, s, d).contiguous().cuda()
+    one = torch.full_like(q, 0.5)
+    x, stats = ops.qk_conv_stats(one, rise, w1, d ** -0.5, group)
+    got = ops.softmax_mix_pv(x, stats, w2, v, 6, group).double()
+    xs = ops.tri_unpack(x, b, h, s, group).double().masked_fill(torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    assert xs[0, 0, -1].max() - xs[0, 0, -1].min() > 200
+    p = torch.softmax(xs, -1)
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    size = torch.einsum("oi,bipq->bopq", w2.double().abs(), p) @ v.double().abs()
+    want = torch.einsum("oi,bipq->bopq", w2.double(), p) @ v.double()
+    assert ((got - want).abs() <= (2.02 * u + 2.0 ** -15) * size + u * want.abs() + 2.0 ** -24 * s).all()   # (exponents below 256: 2^-15)
+
+
 def test_mta_score_layouts_agree_general_route(pkg):
     """Dense 16-head weights and a post-softmax conv: the first score tensor in the triangular layout (the default) or in
     planes, the same stages and the same output bit for bit."""
