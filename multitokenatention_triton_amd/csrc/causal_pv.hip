@@ -405,8 +405,7 @@ template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mi
 // every form (two workgroups of 8 or one of 16).  A wavefront of 16 rows instead of 32 reads its V fragments from LDS for one
 // product each instead of two, which the LDS has room for, and leaves the registers (95 instead of 180) for twice the
 // wavefronts: the reads of P and V that one waits for fly beside the others' products.
-// SUMS = 2: a group adds its even and its odd steps up apart, so that two groups leave a row's sum in the order in which four do.
-template <typename T, int D, int RW, int GR, int SUMS = 1>
+template <typename T, int D, int RW, int GR>
 __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1)) void causal_pv_mid_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
     const int *__restrict__ band_lo, int H, int tri_gl, float scale)
@@ -471,18 +470,16 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
     }
     // this group's blocks, by the block's own number (what a band mask skips leaves every sum as it is)
     const int jg = j0 + ((grp - j0) & (GR - 1)), nsteps = (j_end - j0) / GR + 1;
-    f32x4 sums[SUMS][DB];
+    f32x4 oacc[DB];
 #pragma unroll
-    for (int i = 0; i < SUMS; ++i)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) sums[i][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     frag8<T> p_a[P_KS], p_b[P_KS];
     if (jg <= j_end) issue_v(jg, v_a);
     load_p(jg, p_a);
     // lane's place in a block of V for the transpose reads: rows kg*8 + ln/4 (+4), whose swizzle no other part of the row
     // number touches; head-dim block db is an exclusive or away
     const int vrow = kg * 8 + (ln >> 2), vat = vrow * D + ((((ln & 3) >> 1) ^ v_swizzle<D>(vrow)) * 8) + (ln & 1) * 4;
-    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pf)[P_KS], frag8<T> (&pn)[P_KS], f32x4 (&oacc)[DB]) __attribute__((always_inline)) {
+    auto step = [&](int j, const T *Vb, T *Vn, frag8<T> (&pf)[P_KS], frag8<T> (&pn)[P_KS]) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0);   // V block j and the P fragments have arrived
         __syncthreads();                 // for every wavefront; reads of the other buffer are finished
         if (j > j_end) return;
@@ -520,17 +517,12 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
         }
     };
     for (int i = 0, j = jg;;) {
-        step(j, v_a, v_b, p_a, p_b, sums[0]);
+        step(j, v_a, v_b, p_a, p_b);
         if (++i >= nsteps) break;
         j += GR;
-        step(j, v_b, v_a, p_b, p_a, sums[SUMS - 1]);
+        step(j, v_b, v_a, p_b, p_a);
         if (++i >= nsteps) break;
         j += GR;
-    }
-    f32x4 (&oacc)[DB] = sums[0];
-    if constexpr (SUMS == 2) {
-#pragma unroll
-        for (int db = 0; db < DB; ++db) oacc[db] += sums[1][db];
     }
     if constexpr (GR > 1) {
         if (!mid_sums<T, DB, GT, GR>(v_a_all, v_b_all, oacc, grp, tid)) return;
@@ -799,54 +791,322 @@ __global__ __launch_bounds__(64 * RW * GR, 4) void causal_ptx_mid_kernel(const T
     }
 }
 
-// ---- which kernel ------------------------------------------------------------------------------------------------------
-// What bounds both products is the bytes a CU can pull through the L2 (about 9 TB/s over the chip): the scores once, and the other
-// operand (V, X) once for every block of output rows.  Larger blocks need less of it, smaller ones fill the chip: the line
-// runs by the number of 64-row blocks.  us, narrow | 64 rows, four groups | 64 rows, two groups | 128 rows, two groups | 128 rows, one
-// group | the wide kernel (P V; P^T X had pairs of 128 keys per workgroup there), rotating P tensors:
-//   P V    B2 H4 S2048 D128 (256 blocks)  15.6 | 18.8 | 21.5 | 28.8 | 32.7 | 48.0      B1 H16 S1024 D128 (256)   11.4 | 12.2 | 12.9 | 17.4 | 18.6 | 29.6
-//          B1 H12 S1536 D64 (288)         11.6 | 13.1 | 16.2 | 20.4 | 23.5 | 37.9      B1 H12 S1536 D128 (288)   16.1 | 16.1
-//          B1 H8 S3072 D128 (384)         36.2 | 33.2 | 39.2 | 50.2 | 59.4 | 72.4      B2 H16 S1008 D64 (512)    16.3 | 11.9 | 11.6 | 13.7 | 15.3 | 28.8
-//          B1 H16 S2048 D128 (512)        34.2 | 29.8 | 28.6 | 36.3 | 41.9 | 51.7      B2 H12 S2048 D128 (768)   58.4 | 53.3 | 40.7 | 45.3 | 51.4 | 55.2
-//          B1 H16 S4096 D128 (1024)       118  | 113  | 91.7 | 84.6 | 101  | 95.7      B4 H16 S1024 D128 (1024)  45.1 | 36.2 | 28.0 | 28.1 | 26.2 | 31.8
-//          B2 H16 S3072 D64 (1536)        105  | 88.6 | 76.9 | 85.3 | 86.3 | 97.3      B2 H16 S3072 D128 (1536)  137  | 114  | 98.6 | 98.0 | 89.9 | 111
-//          B4 H32 S2048 D64 (2048)        181  | 164  | 131  | 146  | 126  | 140       B2 H16 S4096 D64 (2048)   177  | 156  | 135  | 150  | 135  | 126
-//          in the triangular layout B2 H16 S4096 D128 (2048) 236 | 194 | 167 | 160 | 145 | 152, B4 H16 S4096 D128 465 | 388 | 331 | 318 | 282 | 305
-//   P^T X  B1 H12 S1000 D64 (192)         10.3 | 11.2 | 11.4 | 11.5 | 12.7 | 19.5      B1 H16 S1536 D128 (384)   17.3 | 16.2 | 18.5 | 21.7 | 24.7 | 34.1
-//          B1 H32 S1024 D128 (512)        19.6 | 16.2 | 14.1 | 17.2 | 18.6 | 26.7      B1 H16 S2048 D64 (512)    25.8 | 21.7 | 26.1 | 24.9 | 29.7 | 34.9
-//          B1 H16 S3072 D128 (768)        66.7 | 61.2 | 53.2 | 48.8 | 56.2 | 59.0      B1 H16 S4096 D64 (1024)   85.2 | 67.7 | 82.0 | 69.6 | 73.3 | 72.0
-//          B4 H16 S1024 D64 (1024)        27.2 | 20.1 | 18.6 | 21.2 | 19.5 | 23.3      B2 H16 S2048 D128 (1024)  64.8 | 69.0 | 49.9 | 51.1 | 50.4 | 53.6
-//          B3 H16 S2048 D128 (1536)       94.1 | 91.2 | 68.3 | 68.1 | 60.8 | 70.0      B4 H32 S2048 D64 (2048)   171  | 129  | 118  | 137  | 122  | 141
-// The fp32 sums of a row have three orders: block by block (the wide kernel, 128 rows with one group), the even and the odd blocks apart
-// (two groups), every fourth block apart (four groups, also as two with two sums each; the narrow kernel's four wavefronts).  So a head's last bit may differ
-// between batch sizes that take different kernels.
-enum product_kernel { WIDE = 1, R64_2, NARROW, R64_4, R128_2, R128_1 };
-
-product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bool tri)
+// ---- rings ------------------------------------------------------------------------------------------------------------
+// The two products with NB buffers instead of two: NB - 1 blocks are in flight at every time, where the kernels above wait for all they
+// asked for at each step and have one.  What a step waits for is counted, so every step asks for the same number of things, also past
+// the last block (then at the end of the buffer the copies come from, where nothing is read), and the copies come from buffers:
+// beside copies from addresses the compiler waits for everything in flight ahead of each use of a loaded register.  Few wavefronts per CU
+// are enough for that, so that a short grid gets by without groups; a long one has the wavefronts anyway (product_form()).
+// The sums of GR groups of GT threads added up in the first group (true there), the upper half's handed to the lower half through LDS
+template <int DB, int GT, int GR> __device__ __forceinline__ bool ring_sums(void *lds, f32x4 (&oacc)[DB], int grp, int tid)
 {
-    // MTA_PV_SPLIT in the environment: 1 .. 6 = always that kernel of the list above (comparison switch; P^T X has no wide one)
+    f32x4 *const part = static_cast<f32x4 *>(lds);
+    __syncthreads();   // nobody reads operands any more
+#pragma unroll
+    for (int h = GR / 2; h > 0; h /= 2) {
+        if (grp >= h && grp < 2 * h) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) part[((grp - h) * DB + db) * GT + tid] = oacc[db];
+        }
+        __syncthreads();
+        if (grp < h) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) oacc[db] += part[(grp * DB + db) * GT + tid];
+        }
+        if (h > 1) __syncthreads();
+    }
+    return grp == 0;
+}
+
+template <typename T, int D, int RW, int GR, int NB, int OCC>
+__global__ __launch_bounds__(64 * RW * GR, OCC) void causal_pv_ring_kernel(
+    const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
+    const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+{
+    constexpr int CPR = D / 8, TILE = P_BK * D, GT = 64 * RW, ROUNDS = TILE / 8 / GT, DB = D / 16, ROWS = 16 * RW, L = ROUNDS + P_KS;
+    static_assert(TILE / 8 % GT == 0 && (GT / CPR) % 16 == 0, "whole copy rounds that keep the swizzle phase");
+    static_assert(GR * NB * TILE * (int)sizeof(T) >= GR / 2 * DB * GT * 16, "half the groups' sums fit the buffers");
+    __shared__ __align__(16) T lds[GR * NB * TILE];
+    const int tid = threadIdx.x % GT, grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    int bh, rank;
+    if (!longest_first(heads, nrb, cus, bh, rank)) return;
+    const int q0 = (nrb - 1 - rank) * ROWS;
+    const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
+    const T *Vp = V + bh * (int64_t)S * D;
+    T *Op = O + bh * (int64_t)S * D;
+    T *const mine = lds + grp * NB * TILE;
+
+    const int row0 = tid / CPR, voff = (row0 * D + ((tid % CPR) ^ v_swizzle<D>(row0)) * 8) * (int)sizeof(T);
+    const int w0 = q0 + wave * 16, prow = w0 + ln;
+    const int pc = prow < S ? prow : S - 1;
+    const T *prow_ptr = tri_gl > 0 ? Pp + tri_gl * tri_rowoff(pc) + (int)(bh % tri_gl) * tri_rowlen(pc) : Pp + (int64_t)pc * S;
+    const int lim = causal ? pc : S - 1;   // last key of this lane's row
+    const int q_last = (q0 + ROWS - 1 < S - 1) ? q0 + ROWS - 1 : S - 1;
+    const int j_end = causal ? q_last / P_BK : (S - 1) / P_BK;
+    int j0 = 0;
+    if (band_lo) {   // the blocks ahead of the first key any of these rows sees hold zeros
+        int f = S;
+        for (int r = lane; r < ROWS; r += 64)
+            if (q0 + r < S) {
+                const int b = band_lo[(bh / H) * (int64_t)S + q0 + r];
+                f = b < f ? b : f;
+            }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const int o = __shfl_xor(f, off);
+            f = o < f ? o : f;
+        }
+        f = __builtin_amdgcn_readfirstlane(f);
+        j0 = (f > 0 ? f : 0) / P_BK;
+        if (j0 > j_end) j0 = j_end;
+    }
+    // this group's blocks, by the block's own number (what a band mask skips leaves every sum as it is)
+    const int jg = j0 + ((grp - j0) & (GR - 1)), nsteps = (j_end - j0) / GR + 1;
+    frag8<T> p[NB][P_KS];
+    // block j, to buffer b: the same number of loads whatever j is, so that the waits can count; rows past the sequence are zeros,
+    // a block past the last one is all of it past the end of the buffer (nothing is read), and so are the rows' vectors (their start again)
+    auto fetch = [&](int j, auto bc) __attribute__((always_inline)) {
+        constexpr int b = decltype(bc)::value;
+        const int left = j <= j_end ? S - j * P_BK : 0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r)
+            copy_to_lds(Vp + (int64_t)j * TILE, left * D * (int)sizeof(T), mine + b * TILE + (r * GT + wave * 64) * 8, voff + r * (GT / CPR) * D * (int)sizeof(T));
+        in_order();
+#pragma unroll
+        for (int ks = 0; ks < P_KS; ++ks) {
+            const int key = j * P_BK + ks * 32 + kg * 8;
+            p[b][ks] = *reinterpret_cast<const frag8<T> *>(prow_ptr + (key <= lim ? key : 0));
+        }
+        in_order();
+    };
+    f32x4 oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // lane's place in a block of V for the transpose reads: rows kg*8 + ln/4 (+4), whose swizzle no other part of the row
+    // number touches; head-dim block db is an exclusive or away
+    const int vrow = kg * 8 + (ln >> 2), vat = vrow * D + ((((ln & 3) >> 1) ^ v_swizzle<D>(vrow)) * 8) + (ln & 1) * 4;
+    unsigned va[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) va[db] = lds_at(mine + (vat ^ (db * 16)));
+    static_for<NB - 1>([&](auto bc) __attribute__((always_inline)) { fetch(jg + decltype(bc)::value * GR, bc); });
+    auto step = [&](int j, auto bc) __attribute__((always_inline)) {
+        constexpr int b = decltype(bc)::value, N = P_KS * DB, AHEAD = DB == 8 ? 6 : 4;
+        copies_wait<(NB - 2) * L>();   // V block j and the rows' vectors have arrived
+        wg_barrier();                  // for every wavefront; reads of the buffer ahead of it are finished
+        fetch(j + (NB - 1) * GR, std::integral_constant<int, (b + NB - 1) % NB>{});
+        if (j > j_end || (causal && j * P_BK > w0 + 15)) return;   // wholly above the diagonal for these rows
+        if (j * P_BK + P_BK - 1 > (causal ? w0 : S - 1)) {
+#pragma unroll
+            for (int ks = 0; ks < P_KS; ++ks) {
+                const int left = lim - (j * P_BK + ks * 32 + kg * 8);
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    if (t > left) p[b][ks].v[t] = from_float<T>(0.0f);
+            }
+        }
+        u32x2 ta[AHEAD + 1], tb[AHEAD + 1];
+        auto read = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, off = (b * TILE + i / DB * 32 * D) * (int)sizeof(T);
+            ta[i % (AHEAD + 1)] = lds_load_tr8_at(va[i % DB], off);
+            tb[i % (AHEAD + 1)] = lds_load_tr8_at(va[i % DB], off + 4 * D * (int)sizeof(T));
+        };
+        static_for<AHEAD>(read);
+        static_for<N>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, younger = 2 * ((i + AHEAD < N ? i + AHEAD : N - 1) - i);
+            if constexpr (i + AHEAD < N) read(std::integral_constant<int, i + AHEAD>{});
+            lds_wait_upto<younger>(ta[i % (AHEAD + 1)], tb[i % (AHEAD + 1)]);
+            const struct { u32x2 a, b; } both = {ta[i % (AHEAD + 1)], tb[i % (AHEAD + 1)]};
+            mma16(oacc[i % DB], __builtin_bit_cast(frag8<T>, both), p[b][i / DB]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    for (int i = 0; i < nsteps; i += NB)
+        static_for<NB>([&](auto bc) __attribute__((always_inline)) { step(jg + (i + decltype(bc)::value) * GR, bc); });
+    copies_wait<0>();   // (nothing may come into LDS that is no longer this workgroup's)
+    if constexpr (GR > 1) {
+        if (!ring_sums<DB, GT, GR>(lds, oacc, grp, tid)) return;
+    }
+    if (prow >= S) return;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[db][v] * scale);
+        *reinterpret_cast<quad *>(Op + (int64_t)prow * D + db * 16 + kg * 4) = out;
+    }
+}
+
+template <typename T, int D, int RW, int GR, int PB, int NB, int OCC>
+__global__ __launch_bounds__(64 * RW * GR, OCC) void causal_ptx_ring_kernel(const T *__restrict__ P, const T *__restrict__ X, T *__restrict__ O, int S,
+                                                                          int causal, int heads, int nkb, int cus, float scale, int H, row_strides xs)
+{
+    constexpr int XC = D / 8, KB = 16 * RW, PC = KB / 8, XT = PB * D, PT = PB * KB, GT = 64 * RW, XR = XT / 8 / GT, PR = PT / 8 / GT, DB = D / 16,
+                  KS = PB / 32, BUF = XT + PT, L = XR + PR;
+    static_assert(XT / 8 % GT == 0 && PT / 8 % GT == 0 && GT / XC % 16 == 0 && GT / PC % 16 == 0, "whole copy rounds that keep the swizzle phase");
+    static_assert(GR * NB * BUF * (int)sizeof(T) >= GR / 2 * DB * GT * 16, "half the groups' sums fit the buffers");
+    __shared__ __align__(16) T lds[GR * NB * BUF];
+    const int tid = threadIdx.x % GT, grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    T *const mine = lds + grp * NB * BUF;
+    int bh, kb;
+    if (!longest_first(heads, nkb, cus, bh, kb)) return;
+    const int k0 = kb * KB;   // (the first keys have the most query rows)
+    const T *Pp = P + bh * (int64_t)S * S + k0;
+    const T *Xp = X + bh / H * xs.batch + bh % H * xs.head;
+    const int xrow = (int)xs.row;
+    T *Op = O + bh * (int64_t)S * D;
+
+    const int xrow0 = tid / XC, xoff = (xrow0 * xrow + ((tid % XC) ^ v_swizzle<D>(xrow0)) * 8) * (int)sizeof(T);
+    const int prow0 = tid / PC;
+    int pchunk = (tid % PC) ^ v_swizzle<KB>(prow0);
+    if (k0 + pchunk * 8 >= S) pchunk = 0;   // (keys past the sequence: rows of the result that nobody stores)
+    const int poff = (prow0 * S + pchunk * 8) * (int)sizeof(T);
+    const int j_start = causal ? k0 / PB : 0, j_end = (S - 1) / PB;
+    // block j of X and P to buffer b, the same number of copies whatever j is; rows past the sequence are zeros
+    auto fetch = [&](int j, int b) __attribute__((always_inline)) {
+        const int left = j <= j_end ? (S - j * PB < PB ? S - j * PB : PB) : 0;
+        const int xbytes = left > 0 ? ((left - 1) * xrow + D) * (int)sizeof(T) : 0, pbytes = left > 0 ? (left * S - k0) * (int)sizeof(T) : 0;
+#pragma unroll
+        for (int r = 0; r < XR; ++r)
+            copy_to_lds(Xp + (int64_t)j * PB * xrow, xbytes, mine + b * BUF + (r * GT + wave * 64) * 8, xoff + r * (GT / XC) * xrow * (int)sizeof(T));
+#pragma unroll
+        for (int r = 0; r < PR; ++r)
+            copy_to_lds(Pp + (int64_t)j * PB * S, pbytes, mine + b * BUF + XT + (r * GT + wave * 64) * 8, poff + r * (GT / PC) * S * (int)sizeof(T));
+        in_order();
+    };
+    // a lane's place in a block for the transpose reads: rows kg*8 + ln/4 (+4; 32 further per step), whose swizzle no other part
+    // of the row number touches; 16-wide column block c is an exclusive or away
+    const int trow = kg * 8 + (ln >> 2), half = (ln & 3) >> 1, sub = (ln & 1) * 4;
+    const int xat = trow * D + ((half ^ v_swizzle<D>(trow)) * 8) + sub, pat = trow * KB + (((wave * 2 + half) ^ v_swizzle<KB>(trow)) * 8) + sub;
+    unsigned xa[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) xa[db] = lds_at(mine + (xat ^ (db * 16)));
+    const unsigned pa = lds_at(mine + XT + pat);
+    const int w0 = k0 + wave * 16, krow = w0 + ln;
+    const int jg = j_start + ((grp - j_start) & (GR - 1)), nsteps = (j_end - j_start) / GR + 1;
+    f32x4 oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    static_for<NB - 1>([&](auto bc) __attribute__((always_inline)) { fetch(jg + decltype(bc)::value * GR, decltype(bc)::value); });
+    auto step = [&](int j, auto bc) __attribute__((always_inline)) {
+        constexpr int b = decltype(bc)::value, N = KS * DB, AHEAD = 4;
+        copies_wait<(NB - 2) * L>();   // block j has arrived
+        wg_barrier();                  // for every wavefront; reads of the buffer ahead of it are finished
+        fetch(j + (NB - 1) * GR, (b + NB - 1) % NB);
+        const int pbase = j * PB;
+        if (j > j_end || (causal && pbase + PB - 1 < w0)) return;   // every row of the block lies above these keys
+        const bool edge = pbase + PB > S || (causal && pbase < w0 + 15);
+        u32x2 qa[KS], qb[KS], ta[AHEAD + 1], tb[AHEAD + 1];
+        static_for<KS>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int ks = decltype(kc)::value, off = (b * BUF + ks * 32 * KB) * (int)sizeof(T);
+            qa[ks] = lds_load_tr8_at(pa, off);
+            qb[ks] = lds_load_tr8_at(pa, off + 4 * KB * (int)sizeof(T));
+        });
+        auto read = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, off = (b * BUF + i / DB * 32 * D) * (int)sizeof(T);
+            ta[i % (AHEAD + 1)] = lds_load_tr8_at(xa[i % DB], off);
+            tb[i % (AHEAD + 1)] = lds_load_tr8_at(xa[i % DB], off + 4 * D * (int)sizeof(T));
+        };
+        static_for<AHEAD>(read);
+        frag8<T> pf[KS];
+        static_for<KS>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int ks = decltype(kc)::value;
+            lds_wait_upto<2 * AHEAD + 2 * (KS - 1 - ks)>(qa[ks], qb[ks]);
+            const struct { u32x2 a, b; } both = {qa[ks], qb[ks]};
+            pf[ks] = __builtin_bit_cast(frag8<T>, both);
+            if (edge) {   // query rows above the key (causal: P is undefined there) or past the sequence count as 0
+                const int first = (causal ? krow : 0) - (pbase + ks * 32 + kg * 8), end = S - (pbase + ks * 32 + kg * 8);
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    if (t < first || t >= end) pf[ks].v[t] = from_float<T>(0.0f);
+            }
+        });
+        static_for<N>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, younger = 2 * ((i + AHEAD < N ? i + AHEAD : N - 1) - i);
+            if constexpr (i + AHEAD < N) read(std::integral_constant<int, i + AHEAD>{});
+            lds_wait_upto<younger>(ta[i % (AHEAD + 1)], tb[i % (AHEAD + 1)]);
+            const struct { u32x2 a, b; } both = {ta[i % (AHEAD + 1)], tb[i % (AHEAD + 1)]};
+            mma16(oacc[i % DB], __builtin_bit_cast(frag8<T>, both), pf[i / DB]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    for (int i = 0; i < nsteps; i += NB)
+        static_for<NB>([&](auto bc) __attribute__((always_inline)) { step(jg + (i + decltype(bc)::value) * GR, bc); });
+    copies_wait<0>();   // (nothing may come into LDS that is no longer this workgroup's)
+    if constexpr (GR > 1) {
+        if (!ring_sums<DB, GT, GR>(lds, oacc, grp, tid)) return;
+    }
+    if (krow >= S) return;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        struct alignas(8) quad { T v[4]; } out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out.v[v] = from_float<T>(oacc[db][v] * scale);
+        *reinterpret_cast<quad *>(Op + (int64_t)krow * D + db * 16 + kg * 4) = out;
+    }
+}
+
+// ---- which kernel ------------------------------------------------------------------------------------------------------
+// What bounds both products is the latency and the bytes of a CU's path to the L2 (about 9 TB/s over the chip): the scores once, and the
+// other operand (V, X) once for every block of output rows.  Larger blocks need less of it, smaller ones fill the chip: the line
+// runs by the number n of 64-row blocks.  RING kernels are the rings of three (P^T X of 128 rows: four) buffers with 64 or 128 rows, _2 with
+// two groups; R kernels have two buffers.  us, rotating P tensors; P V, narrow | R64_2 | R128_1 | RING64 | RING64_2 | RING128 (R figures of
+// grids beyond 512 blocks: the kernel taken there):
+//   n  256  B1 H8 S2048 D128   15.8 | -- | -- | 16.0 | 18.2 | 23.2         320  B1 H5 S4096 D128   -- | -- | -- | 35.4 | 32.0 | 45.6  (four groups 37.4)
+//      288  B1 H12 S1536 D128  16.1 | -- | -- | 15.4 | 14.4 | 18.7             384  B1 H8 S3072 D64    -- | -- | -- | 22.5 | 23.2 | 29.4 (four groups 24.1)
+//      512  B1 H16 S2048 D128  34.2 | 23.1 | 41.9 | 19.5 | 23.6 | 24.3         512  B1 H16 S2048 D64   -- | 19.2 | -- | 15.3 | 18.4 | 21.3
+//      512  B2 H16 S1008 D64   16.3 | 10.6 | 15.3 | 9.8 | 11.9 | 11.5          512  B4 H16 S512 D128   -- | 10.1 | -- | 10.8 | 15.6 | 11.3
+//      768  B1 H16 S3072 D64   -- | 47.4 | -- | 39.7 | 41.7 | 41.6             768  B1 H16 S3072 D128  -- | 50.6 | -- | 51.9 | 53.9 | 51.8
+//     1024  B1 H16 S4096 D128  118 | 91.7 | 101 | 97.8 | 108 | 77.0            1024 B4 H16 S1024 D128  45.1 | 28.0 | 23.8 | 26.3 | 35.6 | 23.8
+//     1536  B2 H16 S3072 D64   105 | 76.4 | 86.3 | 75.9 | 79.5 | 70.4          2048 B1 H32 S4096 D128  -- | -- | 137 | 163 | 176 | 144
+//          in the triangular layout B2 H16 S4096 D128 (2048) narrow 236, R64_2 167, R128_1 145, wide 152
+//   P^T X, narrow | R64_2 | R128_1 | RING64_2 (D64: RING64, four buffers of 64 rows) | RING128 | RING128_2
+//   n  256  B1 H8 S2048 D128   16.4 | -- | -- | 18.3 | 30.8 | 26.3             384  B1 H8 S3072 D64    -- | -- | -- | 20.3 (four groups 25.8)
+//      512  B1 H16 S2048 D128  -- | 25 | -- | 20.5 | 31.4 | 26.8               512  B4 H16 S512 D128   -- | 10.5 | -- | 10.6 | 12.3 | 12.6
+//      512  B1 H16 S2048 D64   25.8 | 26.1 | 29.7 | 15.5                       768  B1 H16 S3072 D128  66.7 | 53.2 | 56.2 | 46.8 | 49.1 | 42.9
+//     1024  B1 H16 S4096 D128  -- | -- | 78.4 | 79.9 | 73.4 | 71.4             1024 B2 H16 S2048 D128  64.8 | 49.9 | 50.4 | 49.0 | 46.4 | 49.8
+//     1024  B4 H16 S1024 D64   27.2 | 16.5 | 19.5 | 18.4                       2048 B4 H32 S1024 D128  -- | -- | 43.9 | 51.4 | 43.3 | 54.1
+// Over 120 random grids of 257 to 2500 blocks these lines give 0.935 (P V) and 0.914 (P^T X) of the time that kernels of two buffers took.
+// The fp32 sums of a row have three orders: block by block (one group), the even and the odd blocks apart (two groups), every fourth
+// block apart (the narrow kernel's four wavefronts).  So a head's last bit may differ between batch sizes that take different kernels.
+enum product_kernel { WIDE = 1, R64_2, NARROW, RING64_2, RING128, R128_1, RING64, RING128_2 };
+
+product_kernel product_form(int64_t heads, int64_t S, int D, bool transposed, bool tri, bool band)
+{
+    // MTA_PV_SPLIT in the environment: 1 .. 8 = always that kernel of the list above (comparison switch), or the next to it where a product
+    // has no such form
     static const int force = [] { const char *e = getenv("MTA_PV_SPLIT"); return e ? atoi(e) : 0; }();
-    if (force >= WIDE && force <= R128_1) return force == WIDE && transposed ? R128_1 : (product_kernel)force;
+    if (force >= WIDE && force <= RING128_2) return force == WIDE && transposed ? R128_1 : (product_kernel)force;
     const int64_t n = heads * ((S + 63) / 64);
     if (n <= 256) return NARROW;   // (resident at once: a CU gets a long and a short block)
-    if (n < 450) return R64_4;
+    // Many short sequences end their rings soon after they have filled them: P V of B4 H16 S832 D64 (832 blocks) 13.0 on two groups, 15.7 as
+    // a ring; P^T X of B4 H16 S640 D128 (640) 13.0 | 15.2.
+    const bool longer = S > (D == 64 ? 2 : 3) * (n - 256);
     if (transposed) {
-        if (D == 64) return n < 2048 && S > 1024 ? R64_4 : R64_2;
-        if (n < 1024) return S <= 1024 ? R64_2 : n <= 512 ? R64_4 : R128_2;
-        return n < 1536 && S > 2048 ? R128_2 : R128_1;
+        if (D == 64) return n < 2048 && (S > 1024 || (n < 1024 && longer)) ? RING64 : R64_2;
+        if (n < 704) return longer ? RING64_2 : R64_2;
+        if (n < 1024) return S > 1024 ? RING128_2 : R64_2;
+        return n <= 1536 && S > 768 ? RING128 : R128_1;
     }
-    if (n >= 2048) return S >= 4096 && !tri ? WIDE : R128_1;
-    if (D == 64 || n < 1024) return R64_2;
-    return n < 1536 && S >= 2048 ? R128_2 : R128_1;
+    // (Under a band mask a block of rows has few key blocks: two workgroups of two groups per CU in place of one whose ring is deeper, with the
+    // same sums.  Window of S/4, B1 H12 S2256 D128 (432): 15.5 | 18.9.)
+    if (n < 450 && D == 128) return S > 4 * n ? (band ? R64_2 : RING64_2) : S > 1000 ? RING64 : R64_2;
+    if (n < 640 && D == 128) return longer ? RING64 : R64_2;
+    if (n < 1024) return D == 64 && (n < 544 ? longer : 2 * S > 5 * n) ? RING64 : R64_2;
+    if (D == 64 ? n < 2048 && S >= 2304 : n < 1600 && S >= 2048) return RING128;
+    return n >= 2048 ? S >= 4096 && !tri ? WIDE : R128_1 : D == 64 ? R64_2 : R128_1;
 }
 
 // A kernel's grid: a workgroup per block of `rows` output rows, `resident` of them on a CU at once; f(grid, blocks per head, cus as
-// longest_first() takes it).  False where the grid is too large.
+// longest_first() takes it).  A grid that is resident at once but for one more round, which then comes longest first again, pairs
+// long and short blocks as well: P V | P^T X of B2 H12 S2784 D128 (528 workgroups of two per CU) 66.8 | 60.2 -> 58.2 | 55.0 us, B2 H16
+// S2072 54.9 | 50.1 -> 47.3 | 43.8; two more rounds, or one on top of a reversed round: up to 11 % slower.  False where the grid is too large.
 template <typename F> bool product_grid(int64_t heads, int64_t S, int rows, int resident, int causal, F &&f)
 {
     const int64_t blocks = (S + rows - 1) / rows, wg = (heads * blocks + 7) / 8 * 8;
     if (wg > 0x7fffffffLL) return false;
-    f(dim3((unsigned)wg), (int)blocks, causal && wg <= (int64_t)resident * device_cu_count() ? device_cu_count() / 8 : 0);
+    f(dim3((unsigned)wg), (int)blocks, causal && wg <= (int64_t)(resident + (resident % 2 == 0)) * device_cu_count() ? device_cu_count() / 8 : 0);
     return true;
 }
 
@@ -860,13 +1120,18 @@ int launch_t(const void *p, const void *x, row_strides xs, void *o, int64_t B, i
         });
         return fits ? launch_status() : MTA_ERR_SHAPE;
     };
-    switch (product_form(B * H, S, D, true, false)) {
-    case NARROW: return go(causal_ptx_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 3 : 2);
-    case R64_4: return go(causal_ptx_mid_kernel<T, D, 4, 4, 32>, 64, 1024, 1);
-    case R64_2: return go(causal_ptx_mid_kernel<T, D, 4, 2, 32>, 64, 512, 2);
-    case R128_2: return go(causal_ptx_mid_kernel<T, D, 8, 2, 64>, 128, 1024, 1);
-    default: return go(causal_ptx_mid_kernel<T, D, 8, 1, 64>, 128, 512, 2);
-    }
+    const product_kernel form = product_form(B * H, S, D, true, false, false);
+    if constexpr (D == 128) {
+        switch (form) {
+        case RING64:
+        case RING64_2: return go(causal_ptx_ring_kernel<T, D, 4, 2, 32, 3, 4>, 64, 512, 2);
+        case RING128: return go(causal_ptx_ring_kernel<T, D, 8, 1, 32, 4, 4>, 128, 512, 2);
+        case RING128_2: return go(causal_ptx_ring_kernel<T, D, 8, 2, 32, 3, 4>, 128, 1024, 1);
+        case R128_1: return go(causal_ptx_mid_kernel<T, D, 8, 1, 64>, 128, 512, 2);
+        default: break;
+        }
+    } else if (form >= RING64_2) return go(causal_ptx_ring_kernel<T, D, 4, 1, 64, 4, 2>, 64, 256, 2);
+    return form == NARROW ? go(causal_ptx_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 3 : 2) : go(causal_ptx_mid_kernel<T, D, 4, 2, 32>, 64, 512, 2);
 }
 
 template <typename T, int D>
@@ -880,18 +1145,17 @@ int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t 
         });
         return fits ? launch_status() : MTA_ERR_SHAPE;
     };
-    switch (product_form(B * H, S, D, false, tri_gl > 0)) {
+    switch (product_form(B * H, S, D, false, tri_gl > 0, band_lo != nullptr)) {
     case NARROW: return go(causal_pv_narrow_kernel<T, D>, N_ROWS, 256, D == 64 ? 4 : 2);
-    // (Under a band mask a block of rows has few key blocks: two workgroups per CU, two groups in each, that add in the same order.  P V,
-    // narrow | four groups | two, us: window of S/4, B1 H16 S1440 (368 blocks) D64 11.4 | 12.5 | 11.0, D128 16.1 | 16.3 | 12.8; B1 H8 S3584 (448)
-    // 16.0 | 19.2 | 14.6, 24.8 | 23.6 | 18.9, with S/2 22.7 | 27.5 | 21.2, 37.0 | 33.8 | 28.0.  Few blocks beyond one for every CU are left to four
-    // groups, which are ahead there where the window is long: B1 H4 S4992 (312) S/4 15.0 | 20.8 | 15.8, 24.8 | 25.6 | 19.9, S/2 19.7 | 21.8 | 24.1,
-    // 28.1 | 26.2 | 28.8; S4352 (272) S/4 12.1 | 13.5 | 13.3, 17.4 | 17.8 | 16.5, S/2 19.7 | 19.6 | 23.0, 28.2 | 24.4 | 27.5.)
-    case R64_4: return band_lo && B * H * ((S + 63) / 64) >= 300 ? go(causal_pv_mid_kernel<T, D, 4, 2, 2>, 64, 512, 2) : go(causal_pv_mid_kernel<T, D, 4, 4>, 64, 1024, 1);
+    case RING64_2:
+        if constexpr (D == 128) return go(causal_pv_ring_kernel<T, D, 4, 2, 3, 2>, 64, 512, 1);
+        [[fallthrough]];
+    case RING64: return go(causal_pv_ring_kernel<T, D, 4, 1, 3, 3>, 64, 256, D == 64 ? 6 : 3);
+    case RING128:
+    case RING128_2: return go(causal_pv_ring_kernel<T, D, 8, 1, 3, 4>, 128, 512, D == 64 ? 3 : 2);
     case R64_2: return go(causal_pv_mid_kernel<T, D, 4, 2>, 64, 512, 2);
-    case R128_2: return go(causal_pv_mid_kernel<T, D, 8, 2>, 128, 1024, 1);
     case R128_1: return go(causal_pv_mid_kernel<T, D, 8, 1>, 128, 512, 2);
-    default: break;
+    case WIDE: break;
     }
     const int nqb = (int)((S + P_BQ - 1) / P_BQ);
     const int64_t total_wg = B * H * ((nqb + 1) / 2), per_xcd = (total_wg + 7) / 8;
@@ -996,7 +1260,7 @@ extern "C" int mta_causal_products(const void *p, const void *v, const void *x, 
     if (!p || !v || !x || !o || !ot) return MTA_ERR_NULL;
     const bool one = io_dtype != MTA_F32 && dtype_size(io_dtype) && B > 0 && H > 0 && S > 0 && S <= (1 << 24) && B * H <= 65535 && (D == 64 || D == 128) &&
                      S % 8 == 0 && aligned_to(p, 16) && aligned_to(v, 16) && aligned_to(x, 16) && aligned_to(o, 16) && aligned_to(ot, 16) &&
-                     product_form(B * H, S, (int)D, false, false) == NARROW && product_form(B * H, S, (int)D, true, false) == NARROW;
+                     product_form(B * H, S, (int)D, false, false, false) == NARROW && product_form(B * H, S, (int)D, true, false, false) == NARROW;
     if (!one) {
         const int rc = mta_causal_pv_scaled_fwd(p, v, o, B, H, S, D, causal, scale, io_dtype, stream);
         return rc != MTA_OK ? rc : mta_causal_ptx_scaled_fwd(p, x, ot, B, H, S, D, causal, scale, io_dtype, stream);

@@ -89,6 +89,23 @@ __device__ __forceinline__ void lds_wait(u32x4 &a) { asm volatile("s_waitcnt lgk
 // workgroup barrier without the memory fence __syncthreads() carries (which would wait for the copy in flight)
 __device__ __forceinline__ void wg_barrier() { asm volatile("s_barrier" : : : "memory"); }
 
+template <int N> __device__ __forceinline__ void copies_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+template <int N> __device__ __forceinline__ void lds_wait_upto(u32x2 &a, u32x2 &b) { asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(N) : "memory"); }
+// what is asked for behind this is asked for after what is ahead of it: the waits count
+__device__ __forceinline__ void in_order()
+{
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ unsigned lds_at(const void *p) { return (unsigned)(uintptr_t)(lds_void_t *)p; }
+
+// 16 bytes a lane from a buffer of `bytes` bytes, at `at` (past its end: zeros), to LDS.  From a buffer, not from an address: copies
+// from addresses make the compiler wait for everything in flight ahead of any use of a loaded register, these it counts.
+__device__ __forceinline__ void copy_to_lds(const void *from, int bytes, void *to, int at)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(from), 0, bytes, 0x00027000), (lds_void_t *)to, 16, at, 0, 0, 0);
+}
+
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>), in order
 template <int... I, typename F> __device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F &&f)
 {

@@ -953,6 +953,25 @@ def test_products_by_grid_size(pkg, heads, s, d, dtype):
     assert torch.equal(pkg.ops.causal_pv(banded, x, True, first_visible=first), pkg.ops.causal_pv(banded, x, True))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,s,d", [(258, 8, 64), (258, 8, 128), (70, 200, 64), (17, 1008, 128), (9, 1800, 128), (10, 3080, 128), (79, 776, 128),
+                                       (44, 1032, 128), (33, 2056, 128), (30, 2312, 64), (24, 2784, 128)])
+def test_products_on_rings(pkg, heads, s, d, dtype):
+    """The products of grids whose blocks come through rings of buffers: fewer blocks than a ring holds, as many as it holds and one more,
+    last blocks of 8 and of all rows, 64 and 128 output rows, one and two groups, a grid of one round more than is resident at once; as
+    test_products_by_grid_size compares them.  P^T X of rows that lie apart is that of the same rows side by side."""
+    test_products_by_grid_size(pkg, heads, s, d, dtype)
+    lib, st, code = pkg._lib.load(), torch.cuda.current_stream().cuda_stream, 1 if dtype == torch.bfloat16 else 2
+    g = torch.Generator(device="cuda").manual_seed(59)
+    p = torch.rand((1, heads, s, s), generator=g, device="cuda").to(dtype)
+    x = torch.randn((1, s, heads, d), generator=g, device="cuda").to(dtype).transpose(1, 2)
+    got, want = (torch.full((heads, s, d), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    assert lib.mta_causal_ptx_rows_fwd(p.data_ptr(), x.data_ptr(), *x.stride()[:3], got.data_ptr(), 1, heads, s, d, 1, 0.5, code, st) == 0
+    y = x.contiguous()
+    assert lib.mta_causal_ptx_scaled_fwd(p.data_ptr(), y.data_ptr(), want.data_ptr(), 1, heads, s, d, 1, 0.5, code, st) == 0
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("heads,s,d", [(288, 4, 64), (160, 68, 128), (256, 36, 64), (512, 36, 64), (260, 128, 128), (768, 36, 64), (400, 100, 128)])
 def test_fp32_products_by_grid_size(pkg, heads, s, d):
     """P V and P^T X in fp32 on the kernels that share V (X) in LDS, which the number of row blocks chooses: one block, edges of the
