@@ -268,13 +268,13 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G < 8 && G * NV == 8) ? RS
         if (lane == 0) red[0][wave * G + o] = v;
     }
     __syncthreads();
+    constexpr int STEP = NW <= 4 ? NW : 1;   // (16 wavefronts unrolled: 128 reads at once, which spilled)
 #pragma unroll
-    for (int o = 0; o < G; ++o) {
-        float v = red[0][o];
+    for (int o = 0; o < G; ++o) m[o] = red[0][o];
+#pragma unroll STEP
+    for (int i = 1; i < NW; ++i)
 #pragma unroll
-        for (int i = 1; i < NW; ++i) v = fmaxf(v, red[0][i * G + o]);
-        m[o] = v;
-    }
+        for (int o = 0; o < G; ++o) m[o] = fmaxf(m[o], red[0][i * G + o]);
 #pragma unroll
     for (int o = 0; o < G; ++o) {
         float sum = 0.0f;
@@ -299,12 +299,13 @@ __global__ __launch_bounds__(NT, (!KB && NT == 256 && G < 8 && G * NV == 8) ? RS
     }
     __syncthreads();
 #pragma unroll
-    for (int o = 0; o < G; ++o) {
-        float v = red[1][o];
+    for (int o = 0; o < G; ++o) inv[o] = red[1][o];
+#pragma unroll STEP
+    for (int i = 1; i < NW; ++i)
 #pragma unroll
-        for (int i = 1; i < NW; ++i) v += red[1][i * G + o];
-        inv[o] = 1.0f / v;
-    }
+        for (int o = 0; o < G; ++o) inv[o] += red[1][i * G + o];
+#pragma unroll
+    for (int o = 0; o < G; ++o) inv[o] = 1.0f / inv[o];
 #pragma unroll
     for (int o = 0; o < G; ++o)
 #pragma unroll
@@ -968,6 +969,9 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         // 12.6 / 12.9, with a key bias 23.4 / 25.0 / 17.4 -> 12.3 / 12.8 / 13.2, a band 17.8 / 24.0 / 16.8 -> 12.1 / 12.9 / 13.1; B4 H16 S1024 36.4 / 44.4 /
         // 39.3 -> 30.0 / 32.8 / 32.0, key bias 50.1 / 53.8 / 41.0 -> 31.6 / 34.7 / 33.5; key bias B2 H16 S1536 41.8 / 45.1 / 36.6 -> 33.2 / 38.6 / 36.6.
         // The partial results of the wavefronts that are left out were neutral: the bits stay.
+        // Groups of 8 beyond 2048 keys, and with a band of 2, take 8 wavefronts of one pass too: the general kernel's fp32 FMAs and unpacked scores
+        // bound those (us, first weight | second | both: 8 x 3392^2 fp16 116 | 90 | 117 -> 42 | 41 | 48, key bias 121 -> 50, band 95 -> 36; 8 x
+        // 4096^2 142 -> 62; 32 x 2560^2 292 -> 91: 3.8 to 4.8 TB/s).
         // key bias without a band mask: the packed kernel's KBIAS instances
         if (packed_ok && kb && !row_lo && aligned_to(kb, 16)) {
 #define MTA_RSK_LAUNCH(g, v, h1, h2, nt, occ)                                                                          \
@@ -987,7 +991,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
             MTA_RSK_CASE(4, 1, 64, 1) MTA_RSK_CASE(4, 1, 128, 1) MTA_RSK_CASE(4, 1, 256, 1)
             if (!(w1 && w2)) MTA_RSK_CASE(4, 1, 512, 8)
             MTA_RSK_CASE(4, 2, 256, RS_OCC)
-            MTA_RSK_CASE(8, 1, 64, 1) MTA_RSK_CASE(8, 1, 128, 1) MTA_RSK_CASE(8, 1, 256, 4)  // (8 heads: a register budget without spills)
+            MTA_RSK_CASE(8, 1, 64, 1) MTA_RSK_CASE(8, 1, 128, 1) MTA_RSK_CASE(8, 1, 256, 4) MTA_RSK_CASE(8, 1, 512, 4)  // (8 heads: a register budget without spills)
 #undef MTA_RSK_CASE
 #undef MTA_RSK_LAUNCH
         }
@@ -1007,7 +1011,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         MTA_RSB_LAUNCH(g, false, true, nt, occ)                                                                        \
     }
             MTA_RSB_CASE(2, 64, 1) MTA_RSB_CASE(2, 128, 1) MTA_RSB_CASE(4, 64, 1) MTA_RSB_CASE(4, 128, 1) MTA_RSB_CASE(8, 64, 1) MTA_RSB_CASE(8, 128, 1)
-            MTA_RSB_CASE(2, 256, 1) MTA_RSB_CASE(4, 256, 1) MTA_RSB_CASE(4, 512, 8) MTA_RSB_CASE(8, 256, RS_OCC)
+            MTA_RSB_CASE(2, 256, 1) MTA_RSB_CASE(2, 512, 8) MTA_RSB_CASE(4, 256, 1) MTA_RSB_CASE(4, 512, 8) MTA_RSB_CASE(8, 256, RS_OCC) MTA_RSB_CASE(8, 512, RS_OCC)
 #undef MTA_RSB_CASE
 #undef MTA_RSB_LAUNCH
         }
@@ -1030,7 +1034,7 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
             // 4 heads x up to 4096 keys: with one weight, 8 wavefronts of one pass each (63 registers: 8 wavefronts per
             // SIMD; measured 2 % faster than 4 wavefronts of two passes); with both weights the latter is 4 % faster
             if (!(w1 && w2)) MTA_RSP_CASE(4, 1, 512, 8)
-            MTA_RSP_CASE(4, 2, 256, RS_OCC) MTA_RSP_CASE(8, 1, 256, RS_OCC)
+            MTA_RSP_CASE(4, 2, 256, RS_OCC) MTA_RSP_CASE(8, 1, 256, RS_OCC) MTA_RSP_CASE(8, 1, 512, RS_OCC)
 #undef MTA_RSP_CASE
 #undef MTA_RSP_LAUNCH
         }
@@ -1065,7 +1069,15 @@ int dispatch(const void *x, const void *w1, const void *w2, const float *kb_in, 
         MTA_RS_CASE(1, 1) MTA_RS_CASE(1, 2) MTA_RS_CASE(1, 4) MTA_RS_CASE(1, 8)
         MTA_RS_CASE(2, 1) MTA_RS_CASE(2, 2) MTA_RS_CASE(2, 4)
         MTA_RS_CASE(4, 1) MTA_RS_CASE(4, 2) MTA_RS_CASE(4, 4)
-        MTA_RS_CASE(8, 1) MTA_RS_CASE(8, 2)
+        MTA_RS_CASE(8, 1)
+        MTA_RS_CASE(8, 2)
+        // 8 heads in fp32 beyond 2048 keys: three passes (140 registers, three workgroups per CU), then twice the wavefronts (two of 8).
+        // us, three sweeps that read the row 24 times -> this | the other one: 8 x 2304^2 660 -> 52 | 65, 2880^2 1049 -> 72 | 84, 4096^2 -> 132
+        // (four passes 151, one pass of 16 wavefronts 230); up to 2048 keys 8 wavefronts lose: 2048^2 47 against 40.
+        if constexpr (sizeof(T) == 4) {
+            MTA_RS_CASE(8, 3)
+            if (G == 8 && Q <= 512 * VEC * 2) return launch_fixed<T, 8, 2, 512>(x, w1, w2, kb, row_lo, y, N, C, P, Q, causal, w_dtype, fill_upper, st);
+        }
 #undef MTA_RS_CASE
     }
     constexpr int NT = 256;
@@ -1136,7 +1148,7 @@ extern "C" int mta_headmix_softmax_tri_supported(int64_t C, int64_t S, int group
     if (out_planes || (band && key_bias)) return 0;
     if (band && has_w1 && has_w2) return 0;
     const int g = group_size;
-    const int64_t cap = band ? (g == 4 ? 4096 : (g == 2 || g == 8) ? 2048 : 0) : (g == 2 ? 8192 : g == 4 ? 4096 : g == 8 ? 2048 : 0);
+    const int64_t cap = g == 2 && !band ? 8192 : g == 2 || g == 4 || g == 8 ? 4096 : 0;
     return S <= cap ? 1 : 0;
 }
 

@@ -122,7 +122,7 @@ def test_triangular_layout_entry_points_validate_and_answer_on_the_host():
     # which combinations the softmax stage has a kernel for: (C, S, group, out_planes, io, w, has_w1, has_w2, band, key_bias)
     q = lib.mta_headmix_softmax_tri_supported
     assert q(16, 4096, 4, 0, 1, 1, 1, 1, 0, 0) == 1 and q(16, 4104, 4, 0, 1, 1, 1, 1, 0, 0) == 0   # packed kernel: up to 4096 keys
-    assert q(16, 8192, 2, 0, 2, 2, 1, 0, 0, 0) == 1 and q(16, 2048, 8, 0, 1, 1, 0, 1, 0, 0) == 1 and q(16, 2056, 8, 0, 1, 1, 0, 1, 0, 0) == 0
+    assert q(16, 8192, 2, 0, 2, 2, 1, 0, 0, 0) == 1 and q(16, 4096, 8, 0, 1, 1, 0, 1, 0, 0) == 1 and q(16, 4104, 8, 0, 1, 1, 0, 1, 0, 0) == 0
     assert q(16, 4096, 4, 0, 1, 1, 1, 0, 1, 0) == 1 and q(16, 4096, 4, 0, 1, 1, 1, 1, 1, 0) == 0   # band: one weight only
     assert q(16, 4096, 4, 0, 0, 0, 1, 1, 0, 0) == 0 and q(16, 4096, 4, 0, 1, 0, 1, 1, 0, 0) == 0   # fp32 data / fp32 weights
     assert q(16, 4096, 4, 1, 1, 1, 1, 1, 0, 0) == 0 and q(16, 4096, 16, 1, 1, 1, 1, 0, 0, 0) == 1   # planes out: groups of 16 only

@@ -500,6 +500,49 @@ def test_fp32_dense_mix_softmax_mix(pkg, h, masked):
             torch.testing.assert_close(got.double().cpu(), s, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("masked", ["", "bias", "band"])
+def test_softmax_of_8_heads_long_rows(pkg, masked, dtype):
+    """Groups of 8 beyond 2048 keys (16 bits: one pass of 8 wavefronts, up to 4096; fp32: three passes, up to 3072, or 8 wavefronts), and what lies
+    beyond; 16 bits also groups of 2 with a band.  Whole numbers in x and the first weight: their mixed scores are exact in every type.
+    What is left, in halves of an ulp (2^-8 in bf16, 2^-11 in fp16): two where a probability near a tie is rounded the other way, and one for the
+    result, of sum |w2| p each; fp32: exp2 of an argument of up to 64 log2(e), 92 ulp of 2^-24 of it, and the sums."""
+    g = torch.Generator().manual_seed(61)
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -18}[dtype]
+    lengths = {torch.float32: (2052, 3072, 3076)}.get(dtype, (2056,))
+    shapes = [(s, s, True) for s in lengths[:2]] + ([] if masked == "band" else [(2, s, False) for s in (*lengths, 4096, 4104)])
+    for group in (8, 2) if dtype != torch.float32 and masked == "band" else (8,):
+        for p, q, causal in shapes:
+            print(f"softmax of {group} heads {p}x{q} causal={causal} {masked} {dtype}", flush=True)
+            x = torch.randint(-2, 3, (1, group, p, q), generator=g).cuda()
+            at = torch.arange(q, device="cuda")
+            keep = (at <= torch.arange(p, device="cuda")[:, None] if causal else torch.ones(p, q, dtype=torch.bool, device="cuda"))[None, None]
+            first = bias = None
+            if masked == "band":
+                first = (torch.arange(p, device="cuda") - 700).clamp(min=0)[None].to(torch.int32)
+                first[0, 2050:] = 2049 - 5   # a visible stretch that starts in the last of the slices of 512 keys
+                keep = keep & (at >= first[:, None, :, None])
+            if masked == "bias":
+                bias = torch.randint(-3, 2, (1, q), generator=g).float().cuda()
+                bias[0, 1:q // 2] = float("-inf")
+            w1 = torch.randint(-1, 2, (group, group), generator=g).cuda()
+            w2 = (torch.eye(group) + 0.1 * torch.randn(group, group, generator=g)).to(dtype).cuda()
+            below = at <= torch.arange(p, device="cuda")[:, None] if causal else torch.ones(p, q, dtype=torch.bool, device="cuda")
+            xd = x.to(dtype).masked_fill(~below, float("nan"))
+            for one, two in ((True, False), (False, True), (True, True)):
+                s = torch.einsum("oi,nipq->nopq", w1.double(), x.double()) if one else x.double()
+                if bias is not None:
+                    s = s + bias.double()[:, None, None, :]
+                want = torch.softmax(s.masked_fill(~keep, float("-inf")), -1).to(dtype).double()
+                size = want
+                if two:
+                    size = torch.einsum("oi,nipq->nopq", w2.double().abs(), want)
+                    want = torch.einsum("oi,nipq->nopq", w2.double(), want)
+                got = pkg.ops.headmix_softmax(xd, w1.to(dtype) if one else None, w2 if two else None, causal, group_size=group, key_bias=bias, first_visible=first)
+                least = 2.0 ** -23 if dtype == torch.float16 else 1e-30   # (probabilities that are subnormal in fp16)
+                assert ((got.double() - want).abs() <= 3 * half * size + group * least).all(), (one, two)
+
+
 def test_fp32_softmax_gradient_sizes(pkg):
     """fp32 rows in registers (up to 8192 keys of whole vectors) and in two sweeps: edges of the instances, NaN above the
     diagonal.  Against float64: the order of the row's sum of p * dp, sum of |p * dp| at most about 4."""
