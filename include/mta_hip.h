@@ -266,6 +266,17 @@ int mta_mask_fill_fwd(const void *x, const void *visible, void *y, int64_t N, in
 int mta_mask_add_fwd(const void *x, const void *mask, void *y, int64_t N, int64_t C, int64_t P, int64_t Q,
                      int mask_batch, int mask_heads, int causal, int io_dtype, void *stream);
 
+/* What a mask (N,H,S,S) amounts to, in one read of it.  stride_*: elements; mask_dtype: a dtype code (additive: +-0 attends, -inf does
+ * not) or -1 for booleans (a byte each, non-zero attends).  flags (one int32, 0 before the call) becomes the sum of
+ *    1  some row does not see exactly what the reference row - the last one, without `causal` the first - sees (causal: up to itself)
+ *    2  the reference row does not see key 0 (without `causal`: sees no key)
+ *    4  some row that sees a key does not see exactly the keys from its first visible one up to itself
+ *    8  some row sees no key          16  some value is neither 0 nor -inf          32  the heads' planes differ
+ * first (int32 (N,S_out)): a row's first visible key, p + 1 if it sees none; bias (fp32 (N,S_out)): 0 where the reference row sees the key,
+ * else -inf; S <= S_out <= S + 64, the columns beyond S hold their own index and 0.  With `causal` only keys q <= p count for 1, 4 and 8. */
+int mta_mask_classify(const void *mask, int64_t stride_b, int64_t stride_h, int64_t stride_row, int64_t stride_key, int64_t N, int64_t H,
+                      int64_t S, int64_t S_out, int causal, int mask_dtype, void *flags, void *first, void *bias, void *stream);
+
 /* ---- The three stages of the causal forward (mta_attention_triton.py:68-89 without a post-softmax conv) over
  * score tensors in a TRIANGULAR LAYOUT.  The (B,H,S,S) tensors between the three kernels never leave the library's
  * caller, so their layout is free; this one stores what lies on and below the diagonal only and puts the rows that one

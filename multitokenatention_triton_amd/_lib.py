@@ -44,6 +44,7 @@ SIGNATURES = {
     "mta_band_zero_f32": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "mta_band_zero_fwd": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "mta_mask_fill_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _int, _vp]),
+    "mta_mask_classify": (_int, [_vp] + [_i64] * 8 + [_int, _int, _vp, _vp, _vp, _vp]),
     "mta_mask_add_fwd": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
     "mta_qk_conv_tri_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _f32, _int, _int, _int, _vp]),
     "mta_headmix_softmax_tri_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _int, _int, _vp]),

@@ -601,14 +601,33 @@ class MTAAttentionTriton(nn.Module):
           (None, None)     anything else (per-head planes, holes that differ between rows, other finite values, a row
                            that sees nothing).
         With the causal rule the arrays are padded to a multiple of 8 columns, as the native routes pad the rows.
-        A few reductions over the mask and one read back; the answer for the last mask object seen is kept while its
-        version does not change."""
+        One read of the mask (``mta_mask_classify``; other dtypes: elementwise operations) and one read back; the answer for the last
+        mask object seen is kept while its version does not change."""
         if mask.size(0) not in (1, bsz) or mask.size(-2) != s or mask.size(-1) != s or mask.size(1) not in (1, self.n_heads):
             return None, None
         key = (mask._version, bsz)
         cached = getattr(self, "_mask_cache", None)   # (the mask object itself is kept: its identity cannot be reused)
         if cached is not None and cached[0] is mask and cached[1] == key:
             return cached[2]
+        answer, empty_rows = (None, None), None
+        if mask.is_cuda and mask.dtype in (torch.bool, torch.float32, torch.float16, torch.bfloat16) and not mask.is_neg():
+            found, first, bias = ops.mask_classify(mask.detach(), self.causal, s + -s % 8 if self.causal else s)
+            if found & (ops.MASK_OTHER_VALUE | ops.MASK_HEADS_DIFFER):
+                pass
+            elif not found & (ops.MASK_NOT_KEYS | ops.MASK_FIRST_HIDDEN):
+                answer = ("keys", bias if bias.size(0) == bsz else bias.expand(bsz, -1).contiguous())
+            elif self.causal and not found & ops.MASK_NOT_BAND:
+                first = first if first.size(0) == bsz else first.expand(bsz, -1).contiguous()
+                answer = ("band", first)
+                if found & ops.MASK_EMPTY_ROW:
+                    empty_rows = first > torch.arange(first.size(1), device=mask.device)
+        else:
+            answer, empty_rows = self._structured_mask_elementwise(mask, bsz, s)
+        self._mask_cache = (mask, key, answer, empty_rows)
+        return answer
+
+    def _structured_mask_elementwise(self, mask, bsz: int, s: int):
+        """(answer of ``_structured_mask``, empty rows) for masks that the kernel does not read (other dtypes, host memory)."""
         answer, empty_rows = (None, None), None
         plane = mask[:, 0]
         same_heads = mask.size(1) == 1 or bool((mask == mask[:, :1]).all())
@@ -643,8 +662,7 @@ class MTAAttentionTriton(nn.Module):
                     answer = ("band", first.contiguous())
                     if bool(empty.any()):
                         empty_rows = _pad_rows(empty.expand(bsz, s), False).contiguous()
-        self._mask_cache = (mask, key, answer, empty_rows)
-        return answer
+        return answer, empty_rows
 
     def _band_empty_rows(self, mask):
         """bool (B, S rounded up to a multiple of 8): the query rows of the band mask last classified that see no key at all, or None if every row sees

@@ -658,6 +658,25 @@ def band_zero_(x: torch.Tensor, first_visible: torch.Tensor) -> Optional[torch.T
     return x
 
 
+# what mta_mask_classify finds
+MASK_NOT_KEYS, MASK_FIRST_HIDDEN, MASK_NOT_BAND, MASK_EMPTY_ROW, MASK_OTHER_VALUE, MASK_HEADS_DIFFER = 1, 2, 4, 8, 16, 32
+
+
+def mask_classify(mask: torch.Tensor, causal: bool, s_out: int):
+    """What a mask (N,H,S,S), boolean or additive, of any strides, amounts to: (the sum of the MASK_ bits that hold, int32 (N,s_out) first visible
+    keys, fp32 (N,s_out) key bias); see mta_mask_classify.  One kernel and one read back."""
+    n, h, s, _ = mask.shape
+    buf = torch.zeros(8 + 2 * n * s_out, dtype=torch.int32, device=mask.device)   # (the bias on a 16-byte boundary)
+    bias, first = buf[8:8 + n * s_out].view(torch.float32).view(n, s_out), buf[8 + n * s_out:].view(n, s_out)
+    sb, sh, sr, sk = (stride if size > 1 else 0 for stride, size in zip(mask.stride(), mask.shape))
+    with torch.cuda.device(mask.device):
+        rc = _lib.load().mta_mask_classify(mask.data_ptr(), sb, sh, sr, sk if s > 1 else 1, n, h, s, s_out, int(bool(causal)),
+                                           -1 if mask.dtype == torch.bool else _code(mask, "mask"), buf.data_ptr(), first.data_ptr(),
+                                           bias.data_ptr(), _stream(mask))
+    _lib.check(rc, "mta_mask_classify")
+    return int(buf[0]), first, bias
+
+
 def mask_fill(x: torch.Tensor, visible: torch.Tensor, neg_inf: bool, causal: bool,
               out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``visible ? x : (-inf if neg_inf else 0)`` for a mask tensor of arbitrary content: ``visible`` is uint8 (or bool),

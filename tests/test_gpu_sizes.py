@@ -1484,3 +1484,50 @@ def test_conv_split_of_16_bit_data(pkg, dtype, wd, r, k):
     assert not torch.isfinite(got[0, 0][touched.tril()]).any()
     torch.testing.assert_close(got[0, 0][~touched].float(), plain[0, 0][~touched].float(), rtol=2 * ulp, atol=2.0 ** -20)
     assert torch.equal(got[0, 1], plain[0, 1])
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_mask_kinds_in_one_read(pkg, causal):
+    """mta_mask_classify against the elementwise operations that other dtypes take: every kind of mask, booleans and additive ones, one plane or one
+    per batch entry or head, strides that vectors fit and others, lengths around vectors and a wavefront's step; exact."""
+    g = torch.Generator().manual_seed(71)
+    mod = pkg.MTAAttentionTriton(2, pkg.MTAConfig(), dropout=0.0, causal=causal, use_mask=True).cuda()
+    kinds = {}
+    for s in (1, 7, 16, 17, 250, 256, 1025, 1040, 2100):
+        at = torch.arange(s)
+        lower = at[None, :] <= at[:, None]
+        n = max(1, s // 3)
+        forms = {"all": torch.ones(2, 1, s, s, dtype=torch.bool), "causal": lower.expand(2, 1, s, s),
+                 "padded": (at < torch.tensor([[n], [s]])[:, None])[:, None].expand(2, 1, s, s), "first hidden": (at >= min(n, s - 1)).expand(1, 1, s, s),
+                 "window": (lower & (at[None, :] > at[:, None] - n))[None, None], "nothing": torch.zeros(1, 1, s, s, dtype=torch.bool),
+                 "left": (lower & (at[None, :] >= torch.tensor([n, 0])[:, None, None]))[:, None], "holes": (torch.rand(1, 1, s, s, generator=g) < 0.9) | (at == 0),
+                 "upper only": lower[None, None] | (torch.rand(1, 1, s, s, generator=g) < 0.5)}
+        for where in {(s - 1, 0), (s - 1, s - 1), (s // 2, s // 4), (0, 0), (0, s - 1)}:   # one position off
+            off = forms["padded"].clone()
+            off[-1, 0][where] ^= True
+            forms[f"off {where}"] = off
+        for name, m in forms.items():
+            heads = m.expand(m.size(0), 2, s, s).clone()
+            other = heads.clone()
+            other[0, 1, s // 2, s - 1] ^= True
+            for what, plane in (("one", m), ("heads", heads), ("differ", other)):
+                add = torch.where(plane, 0.0, float("-inf"))
+                odd, minus, nan = add.clone(), add.clone(), add.clone()
+                odd[-1, -1, s // 2, 0], nan[0, 0, 0, s - 1] = -1e9, float("nan")
+                minus[plane] = -0.0
+                made = [("bool", plane), ("fp32", add), ("bf16", add.bfloat16()), ("fp16", add.half()), ("value", odd), ("value bf16", odd.bfloat16()),
+                        ("nan", nan), ("-0", minus.half())]
+                if what == "one":
+                    wide = torch.zeros(*m.shape[:3], s + 3, dtype=torch.bool)
+                    wide[..., 1:s + 1] = m
+                    made += [("stride", wide.cuda()[..., 1:s + 1]), ("transposed", m.cuda().transpose(2, 3).contiguous().transpose(2, 3)), ("expanded", m[:1].cuda().expand(2, 1, s, s))]
+                for kind, mask in made:
+                    mask = mask.cuda()
+                    mod._mask_cache = None
+                    got, empty = mod._structured_mask(mask, 2, s), mod._band_empty_rows(mask)
+                    want, want_empty = mod._structured_mask_elementwise(mask, 2, s)
+                    assert got[0] == want[0], (s, name, what, kind, got[0], want[0])
+                    kinds[got[0]] = kinds.get(got[0], 0) + 1
+                    for a, b in ((got[1], want[1]), (empty, want_empty)):
+                        assert (a is None) == (b is None) and (a is None or (a.dtype == b.dtype and a.is_contiguous() and torch.equal(a, b))), (s, name, what, kind)
+    assert set(kinds) == ({"keys", "band", None} if causal else {"keys", None})
