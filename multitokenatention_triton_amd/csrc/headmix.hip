@@ -9,6 +9,7 @@
 // Causal: vectors wholly above the diagonal are never read and receive the fill
 // value; the vector that straddles the diagonal is masked per element.
 #include <stdlib.h>
+#include <type_traits>
 
 #include "common.hpp"
 #include "mfma.hpp"
@@ -499,6 +500,14 @@ int launch(const void *x, const void *w, void *y, int64_t N, int64_t C, int64_t 
                                    (const T *)w, (T *)y, (int)C, (int)P, (int)Q, causal, fill, wt, qch);
             return launch_status();
         }
+    }
+    if constexpr (VEC == 8) {
+        // 16-bit data that no kernel above takes (fp32 weights): 32 heads x 8 keys are 256 sums, with bf16's unpacking all registers and one
+        // wavefront per SIMD; 4 keys per lane halve them.  us, 8 | 4 keys, fp32 weights, forward: bf16 32 x 256^2 42 | 14, 1024^2 137 | 28, 64 x
+        // 2048^2 542 | 200; fp16, which converts as it multiplies, 1024^2 43 | 35 but 1504^2, two workgroups a row, 76 | 81; 16 heads 1024^2 bf16 13.7 | 11.4,
+        // fp16 15.2 | 12.8, 2048^2 32 | 38.  12 and 8 heads alike.
+        if ((G == 32 && (std::is_same<T, bf16_t>::value || Q <= NT * 4)) || (G == 16 && Q <= NT * 4))
+            return launch<T, 4>(x, w, y, N, C, P, Q, G, causal, fill, w_dtype, wt, w_same_dtype, st);
     }
     if constexpr (VEC == 4 && sizeof(T) == 4) {
         // 32 heads, rows that a workgroup covers with half vectors as well: twice the wavefronts, of half the registers, each half as long a chain

@@ -1531,3 +1531,26 @@ def test_mask_kinds_in_one_read(pkg, causal):
                     for a, b in ((got[1], want[1]), (empty, want_empty)):
                         assert (a is None) == (b is None) and (a is None or (a.dtype == b.dtype and a.is_contiguous() and torch.equal(a, b))), (s, name, what, kind)
     assert set(kinds) == ({"keys", "band", None} if causal else {"keys", None})
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", [16, 32])
+def test_headmix_wide_groups_with_fp32_weights(pkg, group, dtype):
+    """16-bit data with fp32 weights: four keys per lane up to 1024 keys (32 heads in bf16: any length), eight beyond, and ragged lengths one.  Against
+    float64: half an ulp of the result and fp32 sums of `group` terms."""
+    g = torch.Generator().manual_seed(81)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for n, c, p, q in ((1, group, 3, 8), (2, 2 * group, 70, 70), (1, group, 136, 136), (1, group, 2, 1024), (1, group, 3, 1028), (1, group, 2, 1032), (1, group, 2, 2056)):
+        x = torch.randn(n, c, p, q, generator=g).to(dtype).cuda()
+        w = torch.block_diag(*[torch.eye(group) + 0.2 * torch.randn(group, group, generator=g) for _ in range(c // group)]).cuda()
+        keep = torch.ones(p, q, dtype=torch.bool, device="cuda")
+        for causal in (True, False):
+            low = keep.tril() if causal else keep
+            xd = x.masked_fill(~low, float("nan"))
+            for name, m, fn in (("forward", w, lambda: pkg.ops.headmix(xd, w, causal, 0.0, group_size=group)),
+                                ("input gradient", w.t(), lambda: pkg.ops.headmix_bwd_input(xd, w, causal, group))):
+                want = torch.einsum("oi,nipq->nopq", m.double(), x.double()) * low
+                size = torch.einsum("oi,nipq->nopq", m.double().abs(), x.double().abs())
+                got = fn()
+                assert ((got.double() - want).abs() <= half * want.abs() + group * 2.0 ** -23 * size + 2.0 ** -24).all(), (name, n, c, p, q, causal)
+                assert (got[..., ~low] == 0).all()
