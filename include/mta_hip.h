@@ -321,6 +321,19 @@ int mta_qk_conv_stats_fwd(const void *q, const void *k, const void *w, const voi
 int mta_softmax_mix_pv_supported(int64_t H, int64_t S, int64_t D, int group, int io_dtype, int w_dtype, int key_bias);
 int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
                            int64_t B, int64_t H, int64_t S, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream);
+/* The causal forward of lengths that are not a multiple of 8 without padded copies: Q, K and V have `rows` rows, S - 7 <= rows <= S, everything else has
+ * S, a multiple of 8.  Rows of the results beyond `rows` are not defined; no row up to there depends on them.  16-bit I/O.
+ *   mta_qk_conv_ragged_fwd:        mta_qk_conv_tri_fwd (group > 0) or mta_qk_conv_fwd / mta_qk_conv_band_fwd without a fill (group = 0); with
+ *                                  `stats` mta_qk_conv_stats_fwd without a key bias
+ *   mta_causal_pv_ragged_fwd:      mta_causal_pv_tri_fwd (group > 0) or mta_causal_pv_band_fwd (group = 0), causal
+ *   mta_softmax_mix_pv_ragged_fwd: mta_softmax_mix_pv_fwd */
+int mta_qk_conv_ragged_fwd(const void *q, const void *k, const void *w, const void *first_visible, void *s_out, void *stats, int64_t B, int64_t H,
+                           int64_t S, int64_t rows, int64_t D, int R, int Sk, float scale, int group, int io_dtype, int w_dtype, void *stream);
+int mta_causal_pv_ragged_fwd(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H, int64_t S, int64_t rows,
+                             int64_t D, int group, int io_dtype, void *stream);
+int mta_softmax_mix_pv_ragged_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
+                                  int64_t B, int64_t H, int64_t S, int64_t rows, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype,
+                                  void *stream);
 /* 1 when mta_headmix_softmax_tri_fwd has a kernel for these sizes and dtypes (has_w1 / has_w2: which weights are given;
  * band: with first_visible; key_bias: with a key bias), else 0.  A host-side question: nothing is launched. */
 int mta_headmix_softmax_tri_supported(int64_t C, int64_t S, int group_size, int out_planes, int io_dtype, int w_dtype,

@@ -51,6 +51,9 @@ SIGNATURES = {
     "mta_causal_pv_tri_fwd": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
     "mta_headmix_softmax_tri_supported": (_int, [_i64, _i64, _int, _int, _int, _int, _int, _int, _int, _int]),
     "mta_qk_conv_stats_slots": (_int, [_i64, _i64, _i64, _int]),
+    "mta_qk_conv_ragged_fwd": (_int, [_vp] * 6 + [_i64] * 5 + [_int, _int, _f32, _int, _int, _int, _vp]),
+    "mta_causal_pv_ragged_fwd": (_int, [_vp] * 4 + [_i64] * 5 + [_int, _int, _vp]),
+    "mta_softmax_mix_pv_ragged_fwd": (_int, [_vp] * 7 + [_i64] * 5 + [_int] * 5 + [_vp]),
     "mta_qk_conv_stats_fwd": (_int, [_vp] * 7 + [_i64] * 4 + [_int, _int, _f32, _int, _int, _int, _vp]),
     "mta_softmax_mix_pv_supported": (_int, [_i64] * 3 + [_int] * 4),
     "mta_softmax_mix_pv_fwd": (_int, [_vp] * 7 + [_i64] * 4 + [_int] * 5 + [_vp]),

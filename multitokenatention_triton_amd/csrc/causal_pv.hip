@@ -38,7 +38,7 @@ constexpr int P_KS = P_BK / 32;  // 32-key contraction steps per iteration
 template <typename T, int D>
 __global__ __launch_bounds__(P_NT, P_OCC) void causal_pv_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int nqb, int64_t total_wg,
-    int64_t per_xcd, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+    int64_t per_xcd, const int *__restrict__ band_lo, int H, int tri_gl, float scale, int SV)
 {
     constexpr int CPR = D / 8;               // 16-byte chunks per V row
     constexpr int TILE = P_BK * D;           // elements per V block
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(P_NT, P_OCC) void causal_pv_kernel(
     const int64_t bh = lid / npairs;
     // (tri_gl > 0: P in the triangular layout, groups of tri_gl heads interleaved by rows)
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
-    const T *Vp = V + bh * (int64_t)S * D;
+    const T *Vp = V + bh * (int64_t)SV * D;   // (SV: rows that V has, at most S)
     T *Op = O + bh * (int64_t)S * D;
   for (int half = 0; half < 2; ++half) {
     const int qb = half == 0 ? nqb - 1 - pi : pi;
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(P_NT, P_OCC) void causal_pv_kernel(
             if (TILE / 8 % P_NT != 0 && slot >= TILE / 8) break;
             const int row = slot / CPR, c = (slot % CPR) ^ v_swizzle<D>(row);
             int vr = j * P_BK + row;
-            vr = vr >= S ? S - 1 : vr;
+            vr = vr >= SV ? SV - 1 : vr;
             __builtin_amdgcn_global_load_lds((glb_void_t *)(Vp + (int64_t)vr * D + c * 8),
                                              (lds_void_t *)(dst + (r * P_NT + wave * 64) * 8), 16, 0, 0);
         }
@@ -245,7 +245,7 @@ __device__ __forceinline__ void narrow_reduce(T *a, T *b, const f32x4 (&oacc)[RB
 
 template <typename T, int D>
 __device__ __forceinline__ void pv_narrow(T *lds, unsigned wg, const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal,
-                                          int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+                                          int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl, float scale, int SV)
 {
     constexpr int CPR = D / 8, TILE = N_STEP * D, ROUNDS = TILE / 8 / 64, DB = D / 16;
     T *const v_a_all = lds, *const v_b_all = lds + 4 * TILE;
@@ -257,7 +257,7 @@ __device__ __forceinline__ void pv_narrow(T *lds, unsigned wg, const T *__restri
     if (!longest_first(wg, heads, nrb, cus, bh, rank)) return;
     const int q0 = (nrb - 1 - rank) * N_ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
-    const T *Vp = V + bh * (int64_t)S * D;
+    const T *Vp = V + bh * (int64_t)SV * D;   // (SV: rows that V has, at most S)
     T *Op = O + bh * (int64_t)S * D;
 
     auto issue_v = [&](int j, T *dst) {   // keys past the sequence re-read the last one: their probabilities are masked
@@ -265,7 +265,7 @@ __device__ __forceinline__ void pv_narrow(T *lds, unsigned wg, const T *__restri
         for (int r = 0; r < ROUNDS; ++r) {
             const int slot = r * 64 + lane, row = slot / CPR, c = (slot % CPR) ^ v_swizzle<D>(row);
             int vr = j * N_STEP + row;
-            vr = vr >= S ? S - 1 : vr;
+            vr = vr >= SV ? SV - 1 : vr;
             __builtin_amdgcn_global_load_lds((glb_void_t *)(Vp + (int64_t)vr * D + c * 8), (lds_void_t *)(dst + r * 64 * 8), 16, 0, 0);
         }
     };
@@ -369,10 +369,10 @@ __device__ __forceinline__ void pv_narrow(T *lds, unsigned wg, const T *__restri
 template <typename T, int D>
 __global__ __launch_bounds__(256, 2) void causal_pv_narrow_kernel(const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S,
                                                                   int causal, int heads, int nrb, int cus, const int *__restrict__ band_lo, int H, int tri_gl,
-                                                                  float scale)
+                                                                  float scale, int SV)
 {
     __shared__ __align__(16) T lds[8 * N_STEP * D];
-    pv_narrow<T, D>(lds, blockIdx.x, P, V, O, S, causal, heads, nrb, cus, band_lo, H, tri_gl, scale);
+    pv_narrow<T, D>(lds, blockIdx.x, P, V, O, S, causal, heads, nrb, cus, band_lo, H, tri_gl, scale, SV);
 }
 
 // The sums of GR groups of GT threads added up in the first group (true there): the upper half of the groups hand theirs to the
@@ -408,7 +408,7 @@ template <typename T, int DB, int GT, int GR> __device__ __forceinline__ bool mi
 template <typename T, int D, int RW, int GR>
 __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1)) void causal_pv_mid_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
-    const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+    const int *__restrict__ band_lo, int H, int tri_gl, float scale, int SV)
 {
     constexpr int CPR = D / 8, TILE = P_BK * D, GT = 64 * RW, ROUNDS = TILE / 8 / GT, DB = D / 16, ROWS = 16 * RW;
     static_assert(TILE / 8 % GT == 0 && (GT / CPR) % 16 == 0, "whole copy rounds that keep the swizzle phase");
@@ -422,18 +422,18 @@ __global__ __launch_bounds__(64 * RW * GR, RW * GR / 4 * (RW * GR <= 8 ? 2 : 1))
     if (!longest_first(heads, nrb, cus, bh, rank)) return;
     const int q0 = (nrb - 1 - rank) * ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
-    const T *Vp = V + bh * (int64_t)S * D;
+    const T *Vp = V + bh * (int64_t)SV * D;   // (SV: rows that V has, at most S)
     T *Op = O + bh * (int64_t)S * D;
 
     const int row0 = tid / CPR, voff0 = row0 * D + ((tid % CPR) ^ v_swizzle<D>(row0)) * 8;
     auto issue_v = [&](int j, T *dst) {   // keys past the sequence re-read the last one: their probabilities are masked
-        const bool inside = (j + 1) * P_BK <= S;
+        const bool inside = (j + 1) * P_BK <= SV;
 #pragma unroll
         for (int r = 0; r < ROUNDS; ++r) {
             int off = j * TILE + voff0 + r * (GT / CPR) * D;
             if (!inside) {
                 const int key = j * P_BK + row0 + r * (GT / CPR);
-                off -= (key >= S ? key - (S - 1) : 0) * D;
+                off -= (key >= SV ? key - (SV - 1) : 0) * D;
             }
             __builtin_amdgcn_global_load_lds((glb_void_t *)(Vp + off), (lds_void_t *)(dst + (r * GT + wave * 64) * 8), 16, 0, 0);
         }
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void causal_products_narrow_kernel(const T 
     __shared__ __align__(16) T lds[ptx_narrow_lds<T, D>()];
     const unsigned wg = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
     if (blockIdx.x & 8) ptx_narrow<T, D>(lds, wg, P, X, Ot, S, causal, heads, blocks, cus, scale, heads, row_strides{0, (int64_t)S * D, D});
-    else pv_narrow<T, D>(lds, wg, P, V, O, S, causal, heads, blocks, cus, nullptr, 1, 0, scale);
+    else pv_narrow<T, D>(lds, wg, P, V, O, S, causal, heads, blocks, cus, nullptr, 1, 0, scale, S);
 }
 
 // ---- the transposed product --------------------------------------------------------------------------------------
@@ -821,7 +821,7 @@ template <int DB, int GT, int GR> __device__ __forceinline__ bool ring_sums(void
 template <typename T, int D, int RW, int GR, int NB, int OCC>
 __global__ __launch_bounds__(64 * RW * GR, OCC) void causal_pv_ring_kernel(
     const T *__restrict__ P, const T *__restrict__ V, T *__restrict__ O, int S, int causal, int heads, int nrb, int cus,
-    const int *__restrict__ band_lo, int H, int tri_gl, float scale)
+    const int *__restrict__ band_lo, int H, int tri_gl, float scale, int SV)
 {
     constexpr int CPR = D / 8, TILE = P_BK * D, GT = 64 * RW, ROUNDS = TILE / 8 / GT, DB = D / 16, ROWS = 16 * RW, L = ROUNDS + P_KS;
     static_assert(TILE / 8 % GT == 0 && (GT / CPR) % 16 == 0, "whole copy rounds that keep the swizzle phase");
@@ -833,7 +833,7 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void causal_pv_ring_kernel(
     if (!longest_first(heads, nrb, cus, bh, rank)) return;
     const int q0 = (nrb - 1 - rank) * ROWS;
     const T *Pp = tri_gl > 0 ? P + (bh / tri_gl) * (tri_gl * tri_rowoff(S)) : P + bh * (int64_t)S * S;
-    const T *Vp = V + bh * (int64_t)S * D;
+    const T *Vp = V + bh * (int64_t)SV * D;   // (SV: rows that V has, at most S)
     T *Op = O + bh * (int64_t)S * D;
     T *const mine = lds + grp * NB * TILE;
 
@@ -868,7 +868,7 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void causal_pv_ring_kernel(
     // a block past the last one is all of it past the end of the buffer (nothing is read), and so are the rows' vectors (their start again)
     auto fetch = [&](int j, auto bc) __attribute__((always_inline)) {
         constexpr int b = decltype(bc)::value;
-        const int left = j <= j_end ? S - j * P_BK : 0;
+        const int left = j <= j_end ? SV - j * P_BK : 0;
 #pragma unroll
         for (int r = 0; r < ROUNDS; ++r)
             copy_to_lds(Vp + (int64_t)j * TILE, left * D * (int)sizeof(T), mine + b * TILE + (r * GT + wave * 64) * 8, voff + r * (GT / CPR) * D * (int)sizeof(T));
@@ -1136,12 +1136,12 @@ int launch_t(const void *p, const void *x, row_strides xs, void *o, int64_t B, i
 
 template <typename T, int D>
 int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int causal, hipStream_t st,
-           const int *band_lo = nullptr, int tri_gl = 0, float scale = 1.0f)
+           const int *band_lo = nullptr, int tri_gl = 0, float scale = 1.0f, int64_t v_rows = 0)
 {
     auto go = [&](auto kern, int rows, int threads, int resident) {
         const bool fits = product_grid(B * H, S, rows, resident, causal, [&](dim3 grid, int blocks, int cus) {
             hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, (int)(B * H), blocks, cus, band_lo, (int)H,
-                               tri_gl, scale);
+                               tri_gl, scale, (int)(v_rows ? v_rows : S));
         });
         return fits ? launch_status() : MTA_ERR_SHAPE;
     };
@@ -1161,7 +1161,7 @@ int launch(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t 
     const int64_t total_wg = B * H * ((nqb + 1) / 2), per_xcd = (total_wg + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffLL) return MTA_ERR_SHAPE;
     hipLaunchKernelGGL((causal_pv_kernel<T, D>), dim3((unsigned)(per_xcd * 8)), dim3(P_NT), 0, st, (const T *)p, (const T *)v, (T *)o, (int)S, causal, nqb,
-                       total_wg, per_xcd, band_lo, (int)H, tri_gl, scale);
+                       total_wg, per_xcd, band_lo, (int)H, tri_gl, scale, (int)(v_rows ? v_rows : S));
     return launch_status();
 }
 }  // namespace
@@ -1216,6 +1216,26 @@ extern "C" int mta_causal_pv_tri_fwd(const void *p, const void *v, const void *f
     if (io_dtype == MTA_BF16)
         return D == 64 ? launch<bf16_t, 64>(p, v, o, B, H, S, 1, st, lo, group) : launch<bf16_t, 128>(p, v, o, B, H, S, 1, st, lo, group);
     return D == 64 ? launch<f16_t, 64>(p, v, o, B, H, S, 1, st, lo, group) : launch<f16_t, 128>(p, v, o, B, H, S, 1, st, lo, group);
+}
+
+// V of `rows` rows, S - 7 <= rows <= S, whose probabilities beyond them are not read by the rows up to there (causal): group > 0 P in the
+// triangular layout, 0 planes.  O has S rows; what those beyond `rows` hold is not defined.
+extern "C" int mta_causal_pv_ragged_fwd(const void *p, const void *v, const void *first_visible, void *o, int64_t B, int64_t H, int64_t S, int64_t rows,
+                                        int64_t D, int group, int io_dtype, void *stream)
+{
+    if (!p || !v || !o) return MTA_ERR_NULL;
+    if (!dtype_size(io_dtype)) return MTA_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535 || rows <= 0 || rows > S || rows < S - 7) return MTA_ERR_SHAPE;
+    if (group < 0 || (group > 0 && H % group != 0)) return MTA_ERR_GROUP;
+    if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
+    if (!aligned_to(p, 16) || !aligned_to(v, 16) || !aligned_to(o, 16) || (first_visible && !aligned_to(first_visible, 4)))
+        return MTA_ERR_ALIGN;
+    if (io_dtype == MTA_F32 || S % 8 != 0) return MTA_ERR_UNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    const int *lo = (const int *)first_visible;
+    if (io_dtype == MTA_BF16)
+        return D == 64 ? launch<bf16_t, 64>(p, v, o, B, H, S, 1, st, lo, group, 1.0f, rows) : launch<bf16_t, 128>(p, v, o, B, H, S, 1, st, lo, group, 1.0f, rows);
+    return D == 64 ? launch<f16_t, 64>(p, v, o, B, H, S, 1, st, lo, group, 1.0f, rows) : launch<f16_t, 128>(p, v, o, B, H, S, 1, st, lo, group, 1.0f, rows);
 }
 
 extern "C" int mta_causal_pv_fwd(const void *p, const void *v, void *o, int64_t B, int64_t H, int64_t S, int64_t D,

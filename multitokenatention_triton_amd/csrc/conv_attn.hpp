@@ -19,6 +19,7 @@ struct conv_attn_args {
     bool scores_only;
     hipStream_t st;
     row_strides qs = {0, 0, 0};   // a 1x1 kernel's q where its rows do not follow one another
+    int64_t rows = 0;             // scores only: rows of q and k where they have fewer than S (0: S)
     scores_stats stats = {nullptr, nullptr, 0, {1, 1, 0}};   // scores only, conv_scores_stats_dispatch: the rows' statistics
 };
 int conv_attn_mfma_bf16(const conv_attn_args &a);

@@ -552,6 +552,32 @@ extern "C" int mta_qk_conv_stats_fwd(const void *q, const void *k, const void *w
     return rc == 1 ? MTA_ERR_UNSUPPORTED : rc;
 }
 
+// The causal entry points above for q and k of `rows` rows, S - 7 <= rows <= S: group > 0 the triangular layout, 0 planes without a fill; stats or NULL
+extern "C" int mta_qk_conv_ragged_fwd(const void *q, const void *k, const void *w, const void *first_visible, void *s_out, void *stats, int64_t B, int64_t H,
+                                      int64_t S, int64_t rows, int64_t D, int R, int Sk, float scale, int group, int io_dtype, int w_dtype, void *stream)
+{
+    if (!q || !k || !w || !s_out) return MTA_ERR_NULL;
+    if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535 || rows <= 0 || rows > S || rows < S - 7) return MTA_ERR_SHAPE;
+    if (group < 0 || (group > 0 && H % group != 0)) return MTA_ERR_GROUP;
+    if (R < 1 || Sk < 1 || R > MTA_MAX_FUSED_KERNEL_R || Sk > MTA_MAX_FUSED_KERNEL_S) return MTA_ERR_KERNEL_SIZE;
+    if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
+    if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(s_out, 16) || !aligned_to(w, dtype_size(w_dtype)) || (stats && !aligned_to(stats, 8)) ||
+        (first_visible && !aligned_to(first_visible, 4)))
+        return MTA_ERR_ALIGN;
+    if (io_dtype == MTA_F32 || w_dtype != io_dtype || S % 8 != 0 || !scores_instance(R, Sk)) return MTA_ERR_UNSUPPORTED;
+    if (group > 0 && (int64_t)group * tri_rowoff((int)S) > 0x7fffffffLL) return MTA_ERR_UNSUPPORTED;  // (32-bit offsets inside a group)
+    conv_attn_args a = {q, k, nullptr, w, s_out, nullptr, B, H, S, D, R, Sk, 1, scale, 0, (const int *)first_visible, group, true, (hipStream_t)stream};
+    a.rows = rows;
+    if (stats) {
+        bool table;
+        const scores_cut cut = scores_cut_of(B * H, S, R, true, table);
+        a.stats = {(float2 *)stats, nullptr, scores_slots(S, R, cut), cut};
+    }
+    const int rc = stats ? conv_scores_stats_dispatch(io_dtype, a) : conv_attn_mfma_dispatch(io_dtype, a);
+    return rc == 1 ? MTA_ERR_KERNEL_SIZE : rc;
+}
+
 // mta_qk_conv_fwd under a band mask: key k of query row p of batch entry b is visible iff first_visible[b, p] <= k <= p
 // (int32, (B, S)); the scores of hidden keys enter the conv as 0.  Causal by construction.
 extern "C" int mta_qk_conv_band_fwd(const void *q, const void *k, const void *w, const void *first_visible, void *s_out,

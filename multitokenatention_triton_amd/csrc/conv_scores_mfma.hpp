@@ -127,7 +127,7 @@ struct item_table {
 // 47.6, 7x7 B2 H16 S4096 D64 181 | 209.  With the maximum so far taken at every eight, and a factor for the sum, B2 H16 S4096 took 22 us more.
 template <typename T, int D, int R, int SK, bool BAND, bool STATS>
 __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 128) ? QK_OCC : 2) void conv_scores_mfma(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ Wt,
-                                                           T *__restrict__ O, int S, int causal, float scale, int H, int nqb, int fill_upper,
+                                                           T *__restrict__ O, int S, int SR, int causal, float scale, int H, int nqb, int fill_upper,
                                                            unsigned total_wg, unsigned heads, unsigned per_xcd, int jc_len,
                                                            item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs, scores_stats st)
 {
@@ -198,9 +198,9 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     const int head = (int)((unsigned)bh % (unsigned)H);
     const int q0 = qb * G::BQ;
     const bool q_strided = RAW && qs.row != 0;
-    const T *Qp = Q + (q_strided ? (int64_t)(bh / H) * qs.batch + head * qs.head : (int64_t)bh * S * D);
+    const T *Qp = Q + (q_strided ? (int64_t)(bh / H) * qs.batch + head * qs.head : (int64_t)bh * SR * D);
     const int64_t q_row = q_strided ? qs.row : D;
-    const T *Kp = K + (int64_t)bh * S * D;
+    const T *Kp = K + (int64_t)bh * SR * D;   // (SR: rows that q and k have, at most S; those beyond re-read the last one)
     // (tri_gl > 0: the scores go out in the triangular layout, groups of tri_gl heads interleaved by rows;
     // nothing above the diagonal is stored then)
     const bool tri = tri_gl > 0;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     // (a block inside the sequence: a uniform address and this lane's offset, which the copy adds by itself)
     auto issue_k = [&](int j, T *dst) __attribute__((always_inline)) {
         const int first = j * F_BK + G::PWR;
-        if (first >= 0 && first + F_BK <= S) {
+        if (first >= 0 && first + F_BK <= SR) {
             const char *at = reinterpret_cast<const char *>(Kp + (int64_t)first * D);
 #pragma unroll
             for (int r = 0; r < ROUNDS; ++r)
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
 #pragma unroll
             for (int r = 0; r < ROUNDS; ++r) {
                 int row = first + kv_row0 + r * (F_NT / CPR);
-                row = row < 0 ? 0 : (row >= S ? S - 1 : row);
+                row = row < 0 ? 0 : (row >= SR ? SR - 1 : row);
                 __builtin_amdgcn_global_load_lds((glb_void_t *)(Kp + (kv_off0 + (row - kv_row0) * D)),
                                                  (lds_void_t *)(dst + (r * F_NT + wave * 64) * 8), 16, 0, 0);
             }
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     for (int rb = 0; rb < RB; ++rb) {
         trow[rb] = wave * (16 * RB) + rb * 16 + ln;
         prow[rb] = q0 - G::HR + trow[rb];
-        const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= S ? S - 1 : prow[rb]);
+        const int pc = prow[rb] < 0 ? 0 : (prow[rb] >= SR ? SR - 1 : prow[rb]);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) qf[rb][ks] = *reinterpret_cast<const frag8<T> *>(Qp + pc * q_row + ks * 32 + kg * 8);
     }
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
         static_assert((R + 2) * G::WZ_LD <= (F_BK - 16) * D && 64 / CPR <= 16 && F_NT / CPR >= 16, "16 rows of K beside the taps; whole wavefronts copy them");
         const int first = (j_lo - 1) * F_BK + G::PWR, row = kv_row0 + (ROUNDS - 1) * (F_NT / CPR);
         if (__builtin_amdgcn_readfirstlane(row) >= F_BK - 16) {
-            const int key = first + row < 0 ? 0 : (first + row >= S ? S - 1 : first + row);
+            const int key = first + row < 0 ? 0 : (first + row >= SR ? SR - 1 : first + row);
             __builtin_amdgcn_global_load_lds((glb_void_t *)(Kp + (kv_off0 + (key - kv_row0) * D)),
                                              (lds_void_t *)(wz + ((ROUNDS - 1) * F_NT + wave * 64) * 8), 16, 0, 0);
         }
@@ -941,7 +941,7 @@ int launch_scores(const conv_attn_args &a)
     const int64_t per_xcd = by_head ? (total_wg + 7) / 8 : 0;
     dim3 grid((unsigned)(by_head ? per_xcd * 8 : total_wg));
     hipLaunchKernelGGL((conv_scores_mfma<T, D, R, SK, BAND, STATS>), grid, dim3(256), 0, a.st, (const T *)a.q, (const T *)a.k, (const T *)a.w, (T *)a.o,
-                       (int)S, causal, a.scale, (int)H, nqb, a.fill_upper, (unsigned)total_wg, (unsigned)(B * H), (unsigned)per_xcd, jc_len, tbl, a.band_lo, tri_gl,
+                       (int)S, (int)(a.rows ? a.rows : S), causal, a.scale, (int)H, nqb, a.fill_upper, (unsigned)total_wg, (unsigned)(B * H), (unsigned)per_xcd, jc_len, tbl, a.band_lo, tri_gl,
                        RAW ? a.qs : row_strides{0, 0, 0}, a.stats);
     return launch_status();
 }

@@ -213,6 +213,14 @@ OptTensor lower_scores(const Tensor &a, const Tensor &b, const OptTensor &first)
     return out;
 }
 
+// whether the first and the last kernel of the 16-bit causal route take Q, K and V of fewer rows than the scores have where they lie
+bool reads_ragged(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &conv_w, int64_t s_pad)
+{
+    for (const Tensor *x : {&q, &k, &v})
+        if (!x->is_cuda() || !x->is_contiguous() || x->numel() == 0 || x->is_neg() || reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16) return false;
+    return alike(q, k, v) && !has_tangent(v) && qk_conv_supported(q, k, conv_w, s_pad) && causal_pv_supported(v.scalar_type(), s_pad, v.size(3));
+}
+
 // ---- inference -------------------------------------------------------------------------------------------------------
 // The fused route.  `key_bias`: fp32 (B,Sk), added to the mixed scores ahead of the softmax; the K rows of the keys it
 // hides (-inf) are zeroed, so that their scores enter the pre-softmax conv as 0, and their V rows too where a post-softmax
@@ -242,10 +250,14 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
                     first = mask_row(first_, at::kInt, "the band mask", planes_of, causal, columns, q_),
                     empty_rows = mask_row(empty_rows_, at::kBool, "the empty rows", planes_of, causal, columns, q_);
     Tensor q = q_, k = k_, v = v_;
+    // A length that is not a multiple of 8, in 16 bits: the kernels at both ends read Q, K and V where they lie (`ragged`: the length of the scores).
+    // The padded copies cost a launch and 3 to 13 us.  Forwards, us: bf16 6x11 / 3x3 B2 H16 S1001 D64 85.8 -> 79.8, 7x9 / 7x9 B1 H16 S283 32.7 -> 29.8, fp16
+    // groups of 8 B1 H16 S1001 D64 41.2 -> 38.8.  Key masks keep the copies, which zero the hidden rows on the way.
+    const int64_t ragged = s_pad != s_real && !key_bias && reads_ragged(q_, k_, v_, conv_w, s_pad) ? s_pad : 0;
     if (key_bias && !alike(q_, k_, v_)) {
         k = zero_hidden(k_, *key_bias);
         if (!post_conv_identity) v = zero_hidden(v_, *key_bias);
-    } else if (s_pad != s_real || key_bias) {
+    } else if ((s_pad != s_real && !ragged) || key_bias) {
         RowsCopy rows(s_pad, key_bias);
         if (s_pad != s_real) q = rows.add(q_, false, 1.0);
         k = rows.add(k_, true, 1.0);
@@ -255,29 +267,29 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     // (what the padding rows hold is nobody's business)
     auto result = [&](const Tensor &out) { return (s_pad == s_real ? out : out.narrow(2, 0, s_real)).transpose(1, 2); };
     const double scale = score_scale(q);
-    const int64_t heads = planes_of[1], n_keys = k.size(-2);
+    const int64_t heads = planes_of[1], n_keys = ragged ? ragged : k.size(-2);
     const OptTensor w1 = pre_identity ? OptTensor() : OptTensor(w_pre), w2 = post_identity ? OptTensor() : OptTensor(w_post);
     const int64_t g_pre = pre_identity ? 1 : pre_group ? pre_group : heads, g_post = post_identity ? 1 : post_group ? post_group : heads;
     const int64_t g_both = lcm(g_pre, g_post);
     const bool masked = key_bias || first;
-    const bool qk_kernel = qk_conv_supported(q, k, conv_w), as_is = product_type(q.scalar_type()) == q.scalar_type();
+    const bool qk_kernel = qk_conv_supported(q, k, conv_w, ragged), as_is = product_type(q.scalar_type()) == q.scalar_type();
     const auto dtype = qk_kernel ? q.scalar_type() : product_type(q.scalar_type());   // (of the scores)
     const bool one_pass = post_conv_identity && one_pass_group(g_both, dtype, n_keys, w1, w2) && masks_ok(g_both, dtype, masked);
     // the last stage may leave the upper triangle unwritten only if our own P V kernel consumes it
     const bool own_pv = (s_pad != s_real || score_planes_of(planes_of, v.sizes())) && !has_tangent(v) && dtype == v.scalar_type() &&
-                        (as_is || dtype != at::kFloat) && lower_products_supported(dtype, v.sizes(), causal);
+                        (as_is || dtype != at::kFloat) && (ragged || lower_products_supported(dtype, v.sizes(), causal));
     const bool bias_vectors = !key_bias || reinterpret_cast<uintptr_t>(ptr(*key_bias)) % 16 == 0;
 
     // Two kernels: the scores with the statistics of their rows, and softmax, mixing and P V in one, the probabilities in registers only (which
     // is why the hook hears of the two stages at once).
     if (causal && pre_identity && post_conv_identity && w2 && qk_kernel && own_pv && dropout <= 0 && !(key_bias && (first || !key_bias_hides)) &&
-        softmax_pv_pays(planes_of[0] * heads, n_keys, v.size(-1), g_post) && stats_route_supported(q, k, conv_w, g_post, *w2, key_bias.has_value())) {
+        softmax_pv_pays(planes_of[0] * heads, n_keys, v.size(-1), g_post) && stats_route_supported(q, k, conv_w, g_post, *w2, key_bias.has_value(), ragged)) {
         const bool tri = !planes && g_post * tri_row_offset(n_keys) < (int64_t(1) << 31);
         mark("qk_conv");
-        const auto [scores, stats] = qk_conv_stats(q, k, conv_w, scale, g_post, tri, key_bias, first);
+        const auto [scores, stats] = qk_conv_stats(q, k, conv_w, scale, g_post, tri, key_bias, first, ragged);
         mark("mix_softmax_mix");
         mark("pv");
-        Tensor out = softmax_mix_pv(scores, stats, *w2, v, conv_w.size(1), g_post, tri, key_bias, first);
+        Tensor out = softmax_mix_pv(scores, stats, *w2, v, conv_w.size(1), g_post, tri, key_bias, first, ragged);
         if (empty_rows) out.masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
         mark("end");
         return result(out);
@@ -287,13 +299,13 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     // in the triangular layout (what lies on and below the diagonal only, the rows a workgroup of the softmax stage reads
     // side by side): half the footprint, and every stage streams memory in longer runs.
     if (!planes && causal && one_pass && own_pv && dropout <= 0 && (g_both == 2 || g_both == 4 || g_both == 8 || g_both == 16) && bias_vectors &&
-        tri_route_supported(q, k, conv_w, g_both, w1, w2, first.has_value(), false, key_bias.has_value())) {
+        tri_route_supported(q, k, conv_w, g_both, w1, w2, first.has_value(), false, key_bias.has_value(), ragged)) {
         mark("qk_conv");
-        Tensor scores = qk_conv_tri(q, k, conv_w, scale, g_both, first);
+        Tensor scores = qk_conv_tri(q, k, conv_w, scale, g_both, first, ragged);
         mark("mix_softmax_mix");
         scores = headmix_softmax_tri(scores, w1, w2, q.size(0), heads, n_keys, g_both, first, false, key_bias);
         mark("pv");
-        Tensor out = causal_pv_tri(scores, v, g_both, first);
+        Tensor out = causal_pv_tri(scores, v, g_both, first, ragged);
         if (empty_rows) out.masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
         mark("end");
         return result(out);
@@ -304,13 +316,13 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     // the softmax stage hands the conv (B,H,S,S) planes)
     const bool tri_first = !planes && causal && !one_pass && g_pre == 16 && masks_ok(16, dtype, masked) && w1 &&
                            !(post_conv_identity && !w2 && !own_pv) &&
-                           tri_route_supported(q, k, conv_w, 16, w1, OptTensor(), first.has_value(), true, key_bias.has_value());
+                           tri_route_supported(q, k, conv_w, 16, w1, OptTensor(), first.has_value(), true, key_bias.has_value(), ragged);
     if (tri_first) {
         mark("qk_conv");
-        scores = qk_conv_tri(q, k, conv_w, scale, 16, first);
+        scores = qk_conv_tri(q, k, conv_w, scale, 16, first, ragged);
     } else if (qk_kernel) {
         mark("qk_conv");
-        scores = qk_conv(q, k, conv_w, causal, scale, false, first);
+        scores = qk_conv(q, k, conv_w, causal, scale, false, first, ragged);
     } else {
         mark("qk");
         const OptTensor raw = causal && as_is ? lower_scores(q, k, first) : OptTensor();
@@ -374,7 +386,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     }
     if (dropout > 0) scores = at::dropout(scores, dropout, true);
     mark("pv");
-    OptTensor out = own_pv ? causal_pv(scores, v, causal, first, 1.0) : OptTensor();
+    OptTensor out = own_pv ? causal_pv(scores, v, causal, first, 1.0, ragged) : OptTensor();
     if (!out) out = at::matmul(scores, v);
     if (empty_rows) out->masked_fill_(empty_rows->unsqueeze(1).unsqueeze(-1), 0);
     mark("end");

@@ -282,12 +282,13 @@ inline OptTensor conv2d_headmix(const Tensor &x_, const Tensor &wc_, const Tenso
     return y;
 }
 
-inline bool qk_conv_supported(const Tensor &q, const Tensor &k, const Tensor &w)
+// (here and below: `s_pad` > 0 is the length of the scores where Q, K and V are rows of a shorter one, at most 7 fewer, that are read where they lie)
+inline bool qk_conv_supported(const Tensor &q, const Tensor &k, const Tensor &w, int64_t s_pad = 0)
 {
     if (q.dim() != 4 || q.sizes() != k.sizes() || q.scalar_type() != k.scalar_type() || w.dim() != 3 || !is16(q) ||
         w.scalar_type() != q.scalar_type())
         return false;
-    return mta_qk_conv_supported(q.size(2), q.size(3), (int)w.size(1), (int)w.size(2), code(q, "Q"), code(w, "W")) != 0;
+    return mta_qk_conv_supported(s_pad ? s_pad : q.size(2), q.size(3), (int)w.size(1), (int)w.size(2), code(q, "Q"), code(w, "W")) != 0;
 }
 
 inline bool causal_pv_supported(at::ScalarType t, int64_t s, int64_t d)
@@ -296,15 +297,16 @@ inline bool causal_pv_supported(at::ScalarType t, int64_t s, int64_t d)
 }
 
 // scale * conv(mask0(Q K^T)) as a (B,H,S,S) tensor; the caller has asked qk_conv_supported
-inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool causal, double scale, bool fill_upper, const OptTensor &first)
+inline Tensor qk_conv(const Tensor &q_, const Tensor &k_, const Tensor &w_, bool causal, double scale, bool fill_upper, const OptTensor &first, int64_t s_pad = 0)
 {
     const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
-    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    const int64_t b = q.size(0), h = q.size(1), s = s_pad ? s_pad : q.size(2), d = q.size(3);
     check_conv_weight(w, h);
     Tensor y = at::empty({b, h, s, s}, q.options());
     const int r = (int)w.size(1), sk = (int)w.size(2), ic = code(q, "Q"), wc = code(w, "W");
-    const int rc = first ? mta_qk_conv_band_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, r, sk, (float)scale, fill_upper, ic, wc, stream_of(q))
-                         : mta_qk_conv_fwd(ptr(q), ptr(k), ptr(w), out_ptr(y), b, h, s, d, r, sk, causal, (float)scale, fill_upper, ic, wc, stream_of(q));
+    const int rc = s_pad ? mta_qk_conv_ragged_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), nullptr, b, h, s, q.size(2), d, r, sk, (float)scale, 0, ic, wc, stream_of(q))
+                 : first ? mta_qk_conv_band_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, r, sk, (float)scale, fill_upper, ic, wc, stream_of(q))
+                 : mta_qk_conv_fwd(ptr(q), ptr(k), ptr(w), out_ptr(y), b, h, s, d, r, sk, causal, (float)scale, fill_upper, ic, wc, stream_of(q));
     check(rc, "mta_qk_conv_fwd");
     return y;
 }
@@ -325,8 +327,16 @@ inline bool score_planes_of(c10::IntArrayRef p, c10::IntArrayRef x)
     return p.size() == 4 && x.size() == 4 && p[0] == x[0] && p[1] == x[1] && p[2] == x[2] && p[3] == x[2];
 }
 
-inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first, double scale)
+inline OptTensor causal_pv(const Tensor &p_, const Tensor &v_, bool causal, const OptTensor &first, double scale, int64_t s_pad = 0)
 {
+    if (s_pad) {   // (16-bit and causal: the caller has checked)
+        const Tensor p = on_gpu(p_, "P"), v = on_gpu(v_, "V");
+        const int64_t b = v.size(0), h = v.size(1), d = v.size(3);
+        TORCH_CHECK(causal && scale == 1.0 && p.scalar_type() == v.scalar_type() && p.sizes() == c10::IntArrayRef({b, h, s_pad, s_pad}));
+        Tensor o = at::empty({b, h, s_pad, d}, v.options());
+        check(mta_causal_pv_ragged_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), b, h, s_pad, v.size(2), d, 0, code(p, "P"), stream_of(p)), "mta_causal_pv_fwd");
+        return o;
+    }
     if (p_.scalar_type() != v_.scalar_type() || !score_planes_of(p_.sizes(), v_.sizes()) ||
         !lower_products_supported(p_.scalar_type(), v_.sizes(), causal))
         return std::nullopt;
@@ -399,25 +409,27 @@ inline void band_zero_(const Tensor &x, const Tensor &first)
 
 // whether the triangular-layout kernels exist (host-side questions to the library)
 inline bool tri_route_supported(const Tensor &q, const Tensor &k, const Tensor &conv_w, int64_t group, const OptTensor &w1, const OptTensor &w2,
-                                bool band, bool out_planes, bool key_bias)
+                                bool band, bool out_planes, bool key_bias, int64_t s_pad = 0)
 {
-    if (!qk_conv_supported(q, k, conv_w) || (!w1 && !w2)) return false;
+    if (!qk_conv_supported(q, k, conv_w, s_pad) || (!w1 && !w2)) return false;
     for (const OptTensor *w : {&w1, &w2})
         if (*w && ((*w)->scalar_type() != q.scalar_type() || reinterpret_cast<uintptr_t>(ptr(*w)) % 4)) return false;
-    const int64_t h = q.size(1), s = q.size(2);
+    const int64_t h = q.size(1), s = s_pad ? s_pad : q.size(2);
     if (h % group || group * tri_row_offset(s) >= (int64_t(1) << 31) || !causal_pv_supported(q.scalar_type(), s, q.size(3))) return false;
     const int c = code(q, "Q");
     return mta_headmix_softmax_tri_supported(h, s, (int)group, out_planes, c, c, w1.has_value(), w2.has_value(), band, key_bias) != 0;
 }
 
-inline Tensor qk_conv_tri(const Tensor &q_, const Tensor &k_, const Tensor &w_, double scale, int64_t group, const OptTensor &first)
+inline Tensor qk_conv_tri(const Tensor &q_, const Tensor &k_, const Tensor &w_, double scale, int64_t group, const OptTensor &first, int64_t s_pad = 0)
 {
     const Tensor q = on_gpu(q_, "Q"), k = on_gpu(k_, "K"), w = on_gpu(w_, "W");
-    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3);
+    const int64_t b = q.size(0), h = q.size(1), s = s_pad ? s_pad : q.size(2), d = q.size(3);
     check_conv_weight(w, h);
     Tensor y = at::empty({b * h * tri_row_offset(s)}, q.options());
-    check(mta_qk_conv_tri_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, (int)w.size(1), (int)w.size(2), (float)scale, (int)group,
-                              code(q, "Q"), code(w, "W"), stream_of(q)),
+    check(s_pad ? mta_qk_conv_ragged_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), nullptr, b, h, s, q.size(2), d, (int)w.size(1), (int)w.size(2),
+                                         (float)scale, (int)group, code(q, "Q"), code(w, "W"), stream_of(q))
+                : mta_qk_conv_tri_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), b, h, s, d, (int)w.size(1), (int)w.size(2), (float)scale, (int)group,
+                                      code(q, "Q"), code(w, "W"), stream_of(q)),
           "mta_qk_conv_tri_fwd");
     return y;
 }
@@ -439,48 +451,54 @@ inline Tensor headmix_softmax_tri(const Tensor &x, const OptTensor &w1, const Op
     return y;
 }
 
-inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, const OptTensor &first)
+inline Tensor causal_pv_tri(const Tensor &p, const Tensor &v_, int64_t group, const OptTensor &first, int64_t s_pad = 0)
 {
     const Tensor v = on_gpu(v_, "V");
-    TORCH_CHECK_VALUE(v.dim() == 4 && p.numel() == v.size(0) * v.size(1) * tri_row_offset(v.size(2)) && p.scalar_type() == v.scalar_type(),
+    const int64_t s = s_pad ? s_pad : v.size(2);
+    TORCH_CHECK_VALUE(v.dim() == 4 && p.numel() == v.size(0) * v.size(1) * tri_row_offset(s) && p.scalar_type() == v.scalar_type(),
                       "P in the triangular layout does not belong to a V of shape ", v.sizes());
-    Tensor o = at::empty(v.sizes(), v.options());
-    check(mta_causal_pv_tri_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), (int)group, code(p, "P"),
-                                stream_of(p)),
+    Tensor o = at::empty({v.size(0), v.size(1), s, v.size(3)}, v.options());
+    check(s_pad ? mta_causal_pv_ragged_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), s, v.size(2), v.size(3), (int)group, code(p, "P"),
+                                           stream_of(p))
+                : mta_causal_pv_tri_fwd(ptr(p), ptr(v), ptr(first), out_ptr(o), v.size(0), v.size(1), s, v.size(3), (int)group, code(p, "P"), stream_of(p)),
           "mta_causal_pv_tri_fwd");
     return o;
 }
 
 // scores with the statistics of their rows, and what follows from the two: see mta_qk_conv_stats_fwd.  key_bias: 0 and -inf only
-inline bool stats_route_supported(const Tensor &q, const Tensor &k, const Tensor &conv_w, int64_t group, const Tensor &w2, bool key_bias)
+inline bool stats_route_supported(const Tensor &q, const Tensor &k, const Tensor &conv_w, int64_t group, const Tensor &w2, bool key_bias, int64_t s_pad = 0)
 {
-    if (!qk_conv_supported(q, k, conv_w) || w2.scalar_type() != q.scalar_type() || reinterpret_cast<uintptr_t>(ptr(w2)) % 4) return false;
+    if (!qk_conv_supported(q, k, conv_w, s_pad) || w2.scalar_type() != q.scalar_type() || reinterpret_cast<uintptr_t>(ptr(w2)) % 4) return false;
     const int c = code(q, "Q");
-    return mta_softmax_mix_pv_supported(q.size(1), q.size(2), q.size(3), (int)group, c, c, key_bias) != 0;
+    return mta_softmax_mix_pv_supported(q.size(1), s_pad ? s_pad : q.size(2), q.size(3), (int)group, c, c, key_bias) != 0;
 }
 
 // (scores, statistics); tri: in the triangular layout
 inline std::pair<Tensor, Tensor> qk_conv_stats(const Tensor &q_, const Tensor &k_, const Tensor &w_, double scale, int64_t group, bool tri,
-                                               const OptTensor &key_bias, const OptTensor &first)
+                                               const OptTensor &key_bias, const OptTensor &first, int64_t s_pad = 0)
 {
     const Tensor q = on_gpu_vectors(q_, "Q"), k = on_gpu_vectors(k_, "K"), w = on_gpu(w_, "W");
-    const int64_t b = q.size(0), h = q.size(1), s = q.size(2), d = q.size(3), r = w.size(1);
+    const int64_t b = q.size(0), h = q.size(1), s = s_pad ? s_pad : q.size(2), d = q.size(3), r = w.size(1);
     check_conv_weight(w, h);
     Tensor y = tri ? at::empty({b * h * tri_row_offset(s)}, q.options()) : at::empty({b, h, s, s}, q.options());
     Tensor stats = at::empty({b * h, mta_qk_conv_stats_slots(b, h, s, (int)r), s, 2}, q.options().dtype(at::kFloat));
-    check(mta_qk_conv_stats_fwd(ptr(q), ptr(k), ptr(w), ptr(key_bias), ptr(first), out_ptr(y), out_ptr(stats), b, h, s, d, (int)r, (int)w.size(2), (float)scale,
+    TORCH_CHECK(!s_pad || !key_bias);
+    check(s_pad ? mta_qk_conv_ragged_fwd(ptr(q), ptr(k), ptr(w), ptr(first), out_ptr(y), out_ptr(stats), b, h, s, q.size(2), d, (int)r, (int)w.size(2), (float)scale,
+                                         tri ? (int)group : 0, code(q, "Q"), code(w, "W"), stream_of(q))
+                : mta_qk_conv_stats_fwd(ptr(q), ptr(k), ptr(w), ptr(key_bias), ptr(first), out_ptr(y), out_ptr(stats), b, h, s, d, (int)r, (int)w.size(2), (float)scale,
                                 tri ? (int)group : 0, code(q, "Q"), code(w, "W"), stream_of(q)),
           "mta_qk_conv_stats_fwd");
     return {y, stats};
 }
 
 inline Tensor softmax_mix_pv(const Tensor &x, const Tensor &stats, const Tensor &w2_, const Tensor &v_, int64_t r, int64_t group, bool tri,
-                             const OptTensor &key_bias, const OptTensor &first)
+                             const OptTensor &key_bias, const OptTensor &first, int64_t s_pad = 0)
 {
     const Tensor v = on_gpu_vectors(v_, "V"), w2 = on_gpu(w2_, "weight");
     check_head_weight(w2, v.size(1));
-    Tensor o = at::empty(v.sizes(), v.options());
-    check(mta_softmax_mix_pv_fwd(ptr(x), ptr(stats), ptr(w2), ptr(key_bias), ptr(first), ptr(v), out_ptr(o), v.size(0), v.size(1), v.size(2), v.size(3), (int)r,
+    const int64_t s = s_pad ? s_pad : v.size(2);
+    Tensor o = at::empty({v.size(0), v.size(1), s, v.size(3)}, v.options());
+    check(mta_softmax_mix_pv_ragged_fwd(ptr(x), ptr(stats), ptr(w2), ptr(key_bias), ptr(first), ptr(v), out_ptr(o), v.size(0), v.size(1), s, v.size(2), v.size(3), (int)r,
                                  (int)group, tri, code(x, "scores"), code(w2, "weight"), stream_of(x)),
           "mta_softmax_mix_pv_fwd");
     return o;

@@ -44,7 +44,7 @@ struct pv_args {
     const float *key_bias;   // (B,S) or NULL
     const int *band_lo;      // (B,S) or NULL
     void *o;
-    int S, H, groups, nrb, cus, tri, slots, rows;
+    int S, SV, H, groups, nrb, cus, tri, slots, rows;   // SV: rows that v has, at most S
     scores_cut cut;
     float per_gph, per_rows, per_big, per_small;   // reciprocals of H / G, rows, cut.big, cut.small
 };
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_arg
     const T *const xg = static_cast<const T *>(a.x) + (a.tri ? (int64_t)bg * (G * tri_rowoff(S)) + G * tri_rowoff(w0 < S ? w0 : S - 1) : ((int64_t)bg * G * S + (w0 < S ? w0 : S - 1)) * S);
     const int64_t between = a.tri ? tri_rowlen(w0 < S ? w0 : S - 1) : (int64_t)S * S;
     const unsigned row_at = (unsigned)(pc - (w0 < S ? w0 : S - 1)) * (unsigned)(a.tri ? G * (int)between : S) + kg * 8;
-    const T *const Vg = static_cast<const T *>(a.v) + (int64_t)(bg * G + h0) * S * D;
+    const T *const Vg = static_cast<const T *>(a.v) + (int64_t)(bg * G + h0) * a.SV * D;
 
     // The mixing weights, row lane % 4: of four heads; of two heads twice on the diagonal, for two keys at a time
     u32x2 wm = {0u, 0u};
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_arg
         T *const dst = mine + buf * TILE;
 #pragma unroll
         for (int r = 0; r < ROUNDS; ++r)
-            copy_to_lds(Vg + (int64_t)(r / RPH) * S * D, S * D * (int)sizeof(T), dst + (r * GT + wave * 64) * 8, voff[r % RPH] + j * HEAD * (int)sizeof(T));
+            copy_to_lds(Vg + (int64_t)(r / RPH) * a.SV * D, a.SV * D * (int)sizeof(T), dst + (r * GT + wave * 64) * 8, voff[r % RPH] + j * HEAD * (int)sizeof(T));
     };
     auto load_x = [&](int j, u32x4 (&x)[G]) __attribute__((always_inline)) {   // beyond the row: its start
         const unsigned at = (j * BK + kg * 8 <= pc ? (unsigned)(j * BK) : 0u - kg * 8) + row_at;
@@ -383,12 +383,13 @@ extern "C" int mta_softmax_mix_pv_supported(int64_t H, int64_t S, int64_t D, int
            S <= (key_bias ? MOST_KEYS : 1 << 19) && (D == 64 || D == 128);
 }
 
-extern "C" int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
-                                      int64_t B, int64_t H, int64_t S, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream)
+// v of v_rows rows, S - 7 <= v_rows <= S (o has S; what those beyond v_rows hold is not defined)
+extern "C" int mta_softmax_mix_pv_ragged_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
+                                      int64_t B, int64_t H, int64_t S, int64_t v_rows, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream)
 {
     if (!x || !stats || !w2 || !v || !o) return MTA_ERR_NULL;
     if (!dtype_size(io_dtype) || !dtype_size(w_dtype)) return MTA_ERR_DTYPE;
-    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535) return MTA_ERR_SHAPE;
+    if (B <= 0 || H <= 0 || S <= 0 || S > (1 << 24) || B * H > 65535 || v_rows <= 0 || v_rows > S || v_rows < S - 7) return MTA_ERR_SHAPE;
     if (R < 1 || R > MTA_MAX_FUSED_KERNEL_R) return MTA_ERR_KERNEL_SIZE;
     if (group <= 0 || H % group != 0) return MTA_ERR_GROUP;
     if (D != 64 && D != 128) return MTA_ERR_HEAD_DIM;
@@ -399,8 +400,14 @@ extern "C" int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const vo
     bool table;
     const scores_cut cut = scores_cut_of(B * H, S, R, true, table);
     const int rows = scores_rows(R);
-    const pv_args a{x, w2, v, (const float2 *)stats, (const float *)key_bias, (const int *)first_visible, o, (int)S, (int)H, 0, 0, 0, tri != 0,
+    const pv_args a{x, w2, v, (const float2 *)stats, (const float *)key_bias, (const int *)first_visible, o, (int)S, (int)v_rows, (int)H, 0, 0, 0, tri != 0,
                     scores_slots(S, R, cut), rows, cut, (float)group / (float)H, 1.0f / (float)rows, 1.0f / (float)cut.big, 1.0f / (float)cut.small};
     const int64_t groups = B * (H / group);
     return io_dtype == MTA_BF16 ? launch_type<bf16_t>(a, groups, D, group, (hipStream_t)stream) : launch_type<f16_t>(a, groups, D, group, (hipStream_t)stream);
+}
+
+extern "C" int mta_softmax_mix_pv_fwd(const void *x, const void *stats, const void *w2, const void *key_bias, const void *first_visible, const void *v, void *o,
+                                      int64_t B, int64_t H, int64_t S, int64_t D, int R, int group, int tri, int io_dtype, int w_dtype, void *stream)
+{
+    return mta_softmax_mix_pv_ragged_fwd(x, stats, w2, key_bias, first_visible, v, o, B, H, S, S, D, R, group, tri, io_dtype, w_dtype, stream);
 }

@@ -119,6 +119,19 @@ def test_triangular_layout_entry_points_validate_and_answer_on_the_host():
     assert lib.mta_mask_fill_fwd(p, p, p, 1, 1, 8, 12, 1, 1, 0, 1, 1, None) == -9
     assert lib.mta_mask_add_fwd(None, p, p, 1, 1, 8, 8, 1, 1, 1, 1, None) == -1
     assert lib.mta_mask_add_fwd(p, p, p, 2, 4, 8, 8, 3, 1, 1, 1, None) == -3 and lib.mta_mask_add_fwd(p, p, p, 1, 1, 8, 12, 1, 1, 1, 1, None) == -9
+    # lengths that are not a multiple of 8: rows of Q, K and V within 7 of the scores' length
+    for rows, rc in ((0, -3), (56, -3), (65, -3)):
+        assert lib.mta_qk_conv_ragged_fwd(p, p, p, None, p, None, 1, 4, 64, rows, 64, 3, 3, 0.1, 4, 1, 1, None) == rc
+        assert lib.mta_causal_pv_ragged_fwd(p, p, None, p, 1, 4, 64, rows, 64, 4, 1, None) == rc
+        assert lib.mta_softmax_mix_pv_ragged_fwd(p, p, p, None, None, p, p, 1, 4, 64, rows, 64, 3, 4, 1, 1, 1, None) == rc
+    assert lib.mta_qk_conv_ragged_fwd(p, p, p, None, p, None, 1, 4, 64, 61, 64, 3, 3, 0.1, 4, 0, 0, None) == -9      # fp32
+    assert lib.mta_qk_conv_ragged_fwd(p, p, p, None, p, None, 1, 4, 60, 57, 64, 3, 3, 0.1, 4, 1, 1, None) == -9
+    assert lib.mta_qk_conv_ragged_fwd(p + 2, p, p, None, p, None, 1, 4, 64, 61, 64, 3, 3, 0.1, 4, 1, 1, None) == -6
+    assert lib.mta_causal_pv_ragged_fwd(p, p, None, p, 1, 6, 64, 61, 64, 4, 1, None) == -5
+    # the mask's kinds: null pointers, sizes, dtypes
+    assert lib.mta_mask_classify(None, 64, 64, 8, 1, 1, 1, 8, 8, 1, -1, p, p, p, None) == -1
+    assert lib.mta_mask_classify(p, 64, 64, 8, 1, 1, 1, 8, 7, 1, -1, p, p, p, None) == -3
+    assert lib.mta_mask_classify(p, 64, 64, 8, 1, 1, 1, 8, 8, 1, 7, p, p, p, None) != 0
     # which combinations the softmax stage has a kernel for: (C, S, group, out_planes, io, w, has_w1, has_w2, band, key_bias)
     q = lib.mta_headmix_softmax_tri_supported
     assert q(16, 4096, 4, 0, 1, 1, 1, 1, 0, 0) == 1 and q(16, 4104, 4, 0, 1, 1, 1, 1, 0, 0) == 0   # packed kernel: up to 4096 keys

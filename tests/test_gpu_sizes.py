@@ -1554,3 +1554,53 @@ def test_headmix_wide_groups_with_fp32_weights(pkg, group, dtype):
                 got = fn()
                 assert ((got.double() - want).abs() <= half * want.abs() + group * 2.0 ** -23 * size + 2.0 ** -24).all(), (name, n, c, p, q, causal)
                 assert (got[..., ~low] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("kind", ["groups of 2", "groups of 4", "groups of 8", "dense", "post conv"])
+def test_ragged_lengths_are_read_where_they_lie(pkg, kind, masked, dtype):
+    """16-bit forwards of lengths that are not a multiple of 8 against the same rows with zero rows behind them, bit for bit: the same kernels in the
+    same form, and what lies behind a head's rows - the next head's, or NaN behind the last - is not read.  All forms of P V, the triangular layout
+    and planes, scores with statistics, windows; head groups of NaN beside the compared ones."""
+    g = torch.Generator(device="cuda").manual_seed(91)
+    group = int(kind[-1]) if "groups" in kind else 0
+    for b, h, s, d in ((1, 8, 1, 64), (2, 8, 7, 128), (1, 8, 65, 64), (2, 16, 129, 128), (2, 16, 1001, 64), (1, 16, 2045, 128), (4, 16, 1531, 64), (1, 32, 4093, 64)):
+        if s > 4000 and kind not in ("post conv", "groups of 4"):
+            continue
+        print(f"ragged {kind} masked={masked} {dtype} {(b, h, s, d)}", flush=True)
+        mod = pkg.MTAAttentionTriton(h, pkg.MTAConfig(query_kernel_size=3, key_kernel_size=5), dropout=0.0, causal=True, use_mask=masked).cuda().to(dtype)
+        with torch.no_grad():
+            mod.mta_conv_triton.weight.copy_(0.2 * torch.randn(h, 3, 5, generator=g, device="cuda"))
+            post = mod.mta_conv_after_sm_triton.weight
+            post.zero_()[:, -1, 1] = 1.0
+            if kind == "post conv":
+                post.add_(0.1 * torch.randn(post.shape, generator=g, device="cuda"))
+            block = torch.arange(h, device="cuda") // (group or h)
+            for w in (mod.wpsm_triton.weight, mod.wposm_triton.weight):
+                w.copy_((torch.eye(h, device="cuda") + 0.2 * torch.randn(h, h, generator=g, device="cuda")) * (block[:, None] == block[None, :]))
+            if group in (2, 4):
+                mod.wpsm_triton.weight.copy_(torch.eye(h))
+        mod.eval().requires_grad_(False)
+        mod.infer_weight_structure()
+        pad = -s % 8
+        at = torch.arange(s + pad, device="cuda")
+        window = (at[None, :] <= at[:, None]) & (at[None, :] > at[:, None] - max(1, s // 3))
+        mask = window[None, None] if masked else None
+        rows = [torch.randn(b, h, s, d, generator=g, device="cuda").to(dtype) for _ in range(3)]
+        clean = h
+        if group and group < h:   # the last groups NaN
+            clean = h - group
+            for x in rows:
+                x[:, clean:] = float("nan")
+        ragged = []
+        for x in rows:
+            room = torch.full((x.numel() + 64 * d,), float("nan"), dtype=dtype, device="cuda")
+            room[:x.numel()] = x.flatten()
+            ragged.append(room[:x.numel()].view(x.shape))
+        padded = [torch.nn.functional.pad(x, (0, 0, 0, pad)) for x in rows]
+        with torch.no_grad():
+            got = mod(*ragged, mask[..., :s, :s] if masked else None, None)
+            want = mod(*padded, mask, None)[:, :s]
+        assert got.shape == (b, s, h, d)
+        assert torch.equal(got[:, :, :clean], want[:, :, :clean]) and not got[:, :, :clean].isnan().any()
