@@ -610,7 +610,9 @@ class MTAAttentionTriton(nn.Module):
         if cached is not None and cached[0] is mask and cached[1] == key:
             return cached[2]
         answer, empty_rows = (None, None), None
-        if mask.is_cuda and mask.dtype in (torch.bool, torch.float32, torch.float16, torch.bfloat16) and not mask.is_neg():
+        # (the kernel's range: a grid row per batch entry, and no empty masks)
+        in_range = 0 < mask.size(0) <= 65535 and 0 < mask.size(1) <= 4096 and 0 < s
+        if in_range and mask.is_cuda and mask.dtype in (torch.bool, torch.float32, torch.float16, torch.bfloat16) and not mask.is_neg():
             found, first, bias = ops.mask_classify(mask.detach(), self.causal, s + -s % 8 if self.causal else s)
             if found & (ops.MASK_OTHER_VALUE | ops.MASK_HEADS_DIFFER):
                 pass
@@ -627,7 +629,7 @@ class MTAAttentionTriton(nn.Module):
         return answer
 
     def _structured_mask_elementwise(self, mask, bsz: int, s: int):
-        """(answer of ``_structured_mask``, empty rows) for masks that the kernel does not read (other dtypes, host memory)."""
+        """(answer of ``_structured_mask``, empty rows) for masks that the kernel does not read (other dtypes, host memory, more than 65535 batch entries)."""
         answer, empty_rows = (None, None), None
         plane = mask[:, 0]
         same_heads = mask.size(1) == 1 or bool((mask == mask[:, :1]).all())

@@ -1533,6 +1533,16 @@ def test_mask_kinds_in_one_read(pkg, causal):
     assert set(kinds) == ({"keys", "band", None} if causal else {"keys", None})
 
 
+@pytest.mark.parametrize("n", [65535, 65536])
+def test_mask_of_many_batch_entries(pkg, n):
+    """One entry per grid row: more of them than a grid has are classified by the elementwise operations, with the same answer."""
+    mod = pkg.MTAAttentionTriton(2, pkg.MTAConfig(), dropout=0.0, causal=True, use_mask=True).cuda()
+    mask = torch.ones(n, 1, 4, 4, dtype=torch.bool, device="cuda")
+    mask[:, :, :, 3] = torch.arange(n, device="cuda")[:, None, None] % 2 == 0
+    got, want = mod._structured_mask(mask, n, 4), mod._structured_mask_elementwise(mask, n, 4)[0]
+    assert got[0] == want[0] == "keys" and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("group", [16, 32])
 def test_headmix_wide_groups_with_fp32_weights(pkg, group, dtype):
