@@ -633,7 +633,8 @@ STATS_CASES = [
 def test_softmax_mix_pv(pkg, case):
     """Softmax, mixing and P V in one kernel over the scores kernel's rows and statistics, in both layouts.  Against 64 bits from the same
     stored scores.  A probability and a mixed probability are rounded once each (u of their size, half a step of the smallest number at least), so
-    is a result; the exponents, below 64, are formed in fp32 and the sums are fp32 sums of s terms: 2^-17 of the sum of sizes covers both."""
+    is a result; the exponents relative to the row's reference, below 64, are formed in fp32 and the sums are fp32 sums of s terms: 2^-17 of the sum of sizes
+    covers both."""
     b, h, s, d, r, sk, group, dtype, kind = case
     print(f"softmax mix pv case={case}", flush=True)
     ops = pkg.ops
@@ -713,7 +714,36 @@ def test_softmax_mix_pv_scores_that_are_not_finite_or_far_apart(pkg, dtype):
     u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     size = torch.einsum("oi,bipq->bopq", w2.double().abs(), p) @ v.double().abs()
     want = torch.einsum("oi,bipq->bopq", w2.double(), p) @ v.double()
-    assert ((got - want).abs() <= (2.02 * u + 2.0 ** -15) * size + u * want.abs() + 2.0 ** -24 * s).all()   # (exponents below 256: 2^-15)
+    # (an exponent relative to the reference is below 128 - beyond, the statistics take another reference -, so off by 2^-18, here and in the sum: 2^-17)
+    assert ((got - want).abs() <= (2.02 * u + 2.0 ** -17) * size + u * want.abs() + 2.0 ** -24 * s).all()
+
+
+@pytest.mark.parametrize("seen", ["one key", "tied keys"])
+@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1e3), (torch.bfloat16, 1e6), (torch.bfloat16, 1e8), (torch.float16, 1e3), (torch.float16, 4e4)])
+@pytest.mark.parametrize("case", [(2, 8, 136, 64, 4), (2, 8, 520, 64, 2), (2, 8, 1032, 64, 4), (8, 16, 264, 128, 4)])
+def test_mta_probabilities_do_not_depend_on_the_size_of_the_scores(pkg, case, dtype, size, seen):
+    """All scores have one value (a tap of 8 behind products that 16 bits hold), so that a row that sees n keys has the probabilities 1 / n, whatever the value.  A probability, a mixed one and a
+    result are rounded once each (u of their size, half a step of the smallest number at least); the fp32 sums and the exponential add 2^-18: n terms of V, whose
+    roundings, 2^-24 each, add up to sqrt(n) of it."""
+    b, h, s, d, group = case
+    print(f"mta size of the scores {case, dtype, size, seen}", flush=True)
+    g = torch.Generator().manual_seed(94)
+    w2 = O.block_diag_head_weight(h, group, 0.3, g, dtype)
+    one = O.identity_conv_kernel(h, 3, 3, dtype)
+    mod = _mta_module(pkg, h, 3, 3, 3, 3, 8 * one, torch.eye(h, dtype=dtype), one, w2, dtype, use_mask=seen == "one key")
+    q = torch.full((b, h, s, d), (size / 8 / d ** 0.5) ** 0.5, dtype=dtype, device="cuda")
+    v = torch.randn(b, h, s, d, generator=g).to(dtype).cuda()
+    p = torch.eye(s, dtype=torch.float64, device="cuda")
+    if seen == "tied keys":
+        p = torch.ones_like(p).tril() / torch.arange(1, s + 1, device="cuda")[:, None]
+    got = mod(q, q, v, (p > 0)[None, None] if seen == "one key" else None, None).transpose(1, 2).double()
+    w2, v = w2.double().cuda(), v.double()
+    want = w2.sum(1)[:, None, None] * (p @ v)          # (all heads' probabilities are the same)
+    size_ = w2.abs().sum(1)[:, None, None] * (p @ v.abs())
+    u, least = (2.0 ** -8, 0.0) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -25)
+    tiny = least * ((w2.abs().sum(1)[:, None, None] + 1) * ((p > 0).double() @ v.abs()) + 1)
+    off, bound = (got - want).abs(), (2.02 * u + 2.0 ** -18) * size_ + 1.01 * u * want.abs() + tiny
+    assert (off <= bound).all(), (off / bound).max()
 
 
 def test_mta_score_layouts_agree_general_route(pkg):
