@@ -69,7 +69,7 @@ def stage_model(name, b, h, s, d, r=6, sk=11, esize=2):
 
 
 # Which kernel runs a stage of the headline forward, as rocprofv3 names it in profiles/mta_forward_c4_hbm_traffic.txt
-STAGE_KERNEL = {"qk_conv": "conv_scores_mfma<bf16_t, 128, 6, 11, false, true>",
+STAGE_KERNEL = {"qk_conv": "conv_scores_mfma<bf16_t, 128, 6, 11, false, 1>",
                 "softmax_mix_pv": "softmax_mix_pv<bf16_t, 128, 4, 4, 4, 2, 2, false>"}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "mta_forward_c4_hbm_traffic.txt")
 

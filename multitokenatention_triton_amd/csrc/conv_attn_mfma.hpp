@@ -596,7 +596,7 @@ template <typename T, int D> int dispatch_attn(const conv_attn_args &a)
 template <typename T, int D> int dispatch_mfma_d(const conv_attn_args &a)
 {
     if (!a.scores_only) return dispatch_attn<T, D>(a);
-    return a.band_lo ? dispatch_scores<T, D, true, false>(a) : dispatch_scores<T, D, false, false>(a);
+    return a.band_lo ? dispatch_scores<T, D, true, 0>(a) : dispatch_scores<T, D, false, 0>(a);
 }
 template <typename T> int dispatch_mfma_type(const conv_attn_args &a) { return a.D == 64 ? dispatch_mfma_d<T, 64>(a) : dispatch_mfma_d<T, 128>(a); }
 }  // namespace

@@ -125,14 +125,15 @@ struct item_table {
 // STATS (causal): the statistics of each row's scores of the item, as they are stored (scores_stats): 32 more vector instructions and eight exponentials per
 // eight scores of a lane, us without | with them: bf16 6x11 B2 H16 S4096 D128 248 | 253 (in a loop: the clock), B4 H16 S1024 36.6 | 45.5, B1 H16 S2048 38.2 |
 // 47.6, 7x7 B2 H16 S4096 D64 181 | 209.  With the maximum so far taken at every eight, and a factor for the sum, B2 H16 S4096 took 22 us more.
-template <typename T, int D, int R, int SK, bool BAND, bool STATS>
+// STATS 2: with a key bias, which an instance of its own has to look for.
+template <typename T, int D, int R, int SK, bool BAND, int STATS>
 __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 128) ? QK_OCC : 2) void conv_scores_mfma(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ Wt,
                                                            T *__restrict__ O, int S, int SR, int causal, float scale, int H, int nqb, int fill_upper,
                                                            unsigned total_wg, unsigned heads, unsigned per_xcd, int jc_len,
                                                            item_table tbl, const int *__restrict__ band_lo, int tri_gl, row_strides qs, scores_stats st)
 {
     using G = scores_geom<R, SK>;
-    constexpr bool RAW = R == 1 && SK == 1;
+    constexpr bool RAW = R == 1 && SK == 1, KB = STATS == 2;
     static_assert(!RAW || !STATS, "raw scores have no statistics");
     constexpr int NW = 4, F_NT = 64 * NW, F_SR = 128, RB = F_SR / (16 * NW);   // (RB: blocks of 16 rows per wavefront)
     constexpr int CPR = D / 8;                     // 16-byte chunks per K row
@@ -460,14 +461,14 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     float row_neg[2] = {-NO_SCORE, -NO_SCORE}, row_sum[2] = {0.0f, 0.0f};
     int row_lo[2] = {0, 0};
     uint64_t hidden = 0;                                              // keys of the block that the key bias hides
-    const float *const kb = STATS && st.key_bias ? st.key_bias + (int64_t)(bh / H) * S : nullptr;
+    const float *const kb = KB && st.key_bias ? st.key_bias + (int64_t)(bh / H) * S : nullptr;
     float kb_next = 0.0f;
     auto load_bias = [&](int j) __attribute__((always_inline)) {
         const int key = j * F_BK + lane;
         kb_next = kb[key < S ? key : S - 1];
     };
     if constexpr (STATS) {
-        if (kb) load_bias(j_lo);
+        if (KB && kb) load_bias(j_lo);
         if constexpr (BAND) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -478,14 +479,17 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     }
     // Eight scores of the row h of the pair, keys col .., into the row's statistics.  The reference is the maximum of the lane's first eight
     // (FIRST) and stays: exponentials of what follows may be large, and where they are too large for 32 bits (the sum is infinite or NaN) all of
-    // it is done again with the maximum so far (EVERY), as it is under a band mask, whose rows' first scores may be hidden.
+    // it is done again with the maximum so far (EVERY), as it is under a band mask, whose rows' first scores may be hidden.  Where a key bias hides all
+    // of a lane's eight, the next ones are its first (`fresh`: some lane of the wavefront has none yet): the items that start within the padding of a left-padded
+    // sequence were all done again, forward of B1 H12 S1808 D64 bf16 7x7 83.7 -> 77.0 us.
+    bool fresh = true;
     constexpr float LOG2E = 1.4426950408889634f;
     const std::integral_constant<int, 0> rest{};
     const std::integral_constant<int, 1> first_ones{};
     const std::integral_constant<int, 2> every{};
     auto take = [&](auto mode, auto plain_tag, int h, u32x4_t v, int col, uint64_t hide, int shift) __attribute__((always_inline)) {
         constexpr int MODE = BAND ? 2 : decltype(mode)::value;
-        if (!decltype(plain_tag)::value || BAND || hide != 0) {
+        if (!decltype(plain_tag)::value || BAND || (KB && hide != 0)) {
             MTA_KEEP_BRANCH();
             const uint32_t gone = (uint32_t)(hide >> shift) >> ((opaque_lane(lane) >> 4) * 8) & 255u;
             const int last = q0 - G::HR + wave * (16 * RB) + cshift + 2 * (opaque_lane(lane) & 15) + h - col, first = BAND ? row_lo[h] - col : 0;
@@ -506,7 +510,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
             }
             const float neg = fminf(-m * LOG2E, row_neg[h]);   // (no score yet: NO_SCORE stays)
             if constexpr (MODE == 2) row_sum[h] *= __builtin_amdgcn_exp2f(neg - row_neg[h]);
-            row_neg[h] = neg;
+            if (MODE == 2 || !KB || row_neg[h] == -NO_SCORE) row_neg[h] = neg;
         }
         float sum = row_sum[h];
 #pragma unroll
@@ -544,7 +548,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
             }
         }
         if (j < j_end) issue_k(j + 1, Kn);  // lands while this block is being worked on
-        if (STATS && kb) {
+        if (KB && kb) {
             hidden = __builtin_amdgcn_ballot_w64(kb_next == -INFINITY);
             if (j < j_end) load_bias(j + 1);
         }
@@ -704,14 +708,15 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
                     if (stored[h] && (PLAIN || (col < S && (!causal || fill_upper || col <= p_))))
                         *reinterpret_cast<u32x4_t *>(o_block + o_off[h] + (w - 3) * 8 * (int)sizeof(T)) = eight;
                     if constexpr (STATS) {
-                        if (w == 3 && j == j_lo) {
+                        if (KB && !BAND ? fresh : w == 3 && j == j_lo) {
                             MTA_KEEP_BRANCH();
-                            take(first_ones, plain_tag, h, eight, col, hidden, 0);
+                            take(first_ones, plain_tag, h, eight, col, hidden, (w - 3) * 8);
                         } else {
                             take(rest, plain_tag, h, eight, col, hidden, (w - 3) * 8);
                         }
                     }
                 }
+                if (KB && !BAND && fresh) fresh = __builtin_amdgcn_ballot_w64(row_neg[0] == -NO_SCORE || row_neg[1] == -NO_SCORE) != 0;
             }
         };
         static_for<NLD>(issue);
@@ -843,7 +848,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
 #pragma unroll 1
             for (int j = j_lo; j <= j_end; ++j) {
                 const int key = j * F_BK + lane_;
-                const uint64_t gone = kb ? __builtin_amdgcn_ballot_w64(kb[key < S ? key : S - 1] == -INFINITY) : 0;
+                const uint64_t gone = KB && kb ? __builtin_amdgcn_ballot_w64(kb[key < S ? key : S - 1] == -INFINITY) : 0;
 #pragma unroll
                 for (int n = 0; n < 4; ++n) {
                     const int h = n >> 1, col = j * F_BK + (n & 1) * 32 + kg_ * 8;
@@ -883,7 +888,7 @@ __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 12
     }
 }
 
-template <typename T, int D, int R, int SK, bool BAND, bool STATS>
+template <typename T, int D, int R, int SK, bool BAND, int STATS>
 int launch_scores(const conv_attn_args &a)
 {
     using G = scores_geom<R, SK>;
@@ -947,10 +952,10 @@ int launch_scores(const conv_attn_args &a)
 }
 
 // returns 1 when no instantiation covers the kernel size (the caller then uses the general kernel)
-template <typename T, int D, bool BAND, bool STATS> int dispatch_scores(const conv_attn_args &a)
+template <typename T, int D, bool BAND, int STATS> int dispatch_scores(const conv_attn_args &a)
 {
     if constexpr (!STATS)
-        if (a.R == 1 && a.Sk == 1) return launch_scores<T, D, 1, 1, BAND, false>(a);   // no conv (weights are not read)
+        if (a.R == 1 && a.Sk == 1) return launch_scores<T, D, 1, 1, BAND, 0>(a);   // no conv (weights are not read)
 #define MTA_SCORES_CASE(r, s) \
     if (a.R == r && a.Sk == s) return launch_scores<T, D, r, s, BAND, STATS>(a);
     MTA_SCORES_CASE(3, 3)

@@ -4,7 +4,8 @@
 namespace {
 template <int D> int with_stats(const mta::conv_attn_args &a)
 {
-    return a.band_lo ? dispatch_scores<mta::f16_t, D, true, true>(a) : dispatch_scores<mta::f16_t, D, false, true>(a);
+    if (a.band_lo) return dispatch_scores<mta::f16_t, D, true, 2>(a);
+    return a.stats.key_bias ? dispatch_scores<mta::f16_t, D, false, 2>(a) : dispatch_scores<mta::f16_t, D, false, 1>(a);
 }
 }  // namespace
 

@@ -626,6 +626,8 @@ STATS_CASES = [
     (4, 32, 328, 64, 11, 15, 4, torch.bfloat16, "ragged"), (4, 64, 424, 64, 6, 11, 4, torch.float16, None), (2, 64, 200, 128, 7, 7, 2, torch.bfloat16, "keys"),
     (2, 32, 136, 128, 3, 3, 2, torch.float16, "window"), (4, 64, 136, 64, 5, 5, 2, torch.bfloat16, None), (2, 32, 232, 64, 6, 11, 2, torch.float16, "documents"),
     (1, 4, 4168, 64, 7, 7, 4, torch.bfloat16, None),
+    # padding on the left, up to and beyond the eight keys of a lane, its next eight, a block, a work item
+    (6, 4, 328, 64, 6, 11, 4, torch.bfloat16, "left"), (6, 4, 648, 128, 3, 3, 2, torch.float16, "left"), (2, 8, 2056, 64, 7, 7, 4, torch.float16, "left"),
 ]
 
 
@@ -650,6 +652,11 @@ def test_softmax_mix_pv(pkg, case):
         keep = at[None, :] < torch.tensor([s - 3 * i for i in range(b)], device="cuda")[:, None]
         keep[0, 5::7] = False
         keep[-1, :min(s // 3, 40)] = False
+        key_bias = torch.where(keep, 0.0, float("-inf"))
+        seen = seen & keep[:, None, :]
+    elif kind == "left":
+        keep = at[None, :] >= torch.tensor([7, s - 9, 32, 40, 129, 64], device="cuda")[:b, None]
+        keep[0, 3] = True
         key_bias = torch.where(keep, 0.0, float("-inf"))
         seen = seen & keep[:, None, :]
     elif kind:
