@@ -332,12 +332,17 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_arg
 // Of how many heads a workgroup forms the results, of how many rows, and how many groups of wavefronts share the keys: WHOLE all, 64, two; HALF_LONG half of them,
 // 64, one (groups of 4 at D64: all, 32, two); HALF_SHORT half, 32, two; HALF_SPLIT half, 16, four.  With half of the heads the exponentials
 // are formed twice, but there are twice the workgroups and a step is shorter; more groups of wavefronts shorten the chain of steps.  The
-// line runs by n, the 64-row blocks over the groups of heads.  us of the forward, bf16 6x11, the four in this order:
-//   groups of 4, D128  n 8 (B1 H4 S512) 34.9 | 30.0 | 24.1 | 22.4, 36 (B1 H16 S576) 42.5 | 38.5 | 31.4 | 31.3, 48 (B2 H16 S384) 37.7 | 32.9 | 28.4 | 33.0, 128 (B2 H16 S1024) 70.9 |
-//     65.0 | 54.4 | 79.6, 192 (B4 H12 S1001) 91.6 | 88.5 | 88.7 | 127, 256 (B4 H16 S1024) 86.6 | 82.2 | 87.5 | 144, 464 (B4 H16 S1856) 203 | 222 | 242 | 388, 512 (B2 H16 S4096) 437 | 485 | 516 | 781
-//   groups of 4, D64   n 8 27.9 | 23.3 | 20.9 | 18.3, 64 (B1 H16 S1008) 54.0 | 47.1 | 42.7 | 39.5, 128 59.3 | 52.4 | 47.9 | 53.8, 192 75.6 | 70.4 | 69.9 | 81.5, 256 73.6 | 67.2 | 75.6 | 90.6, 464 167 | 173 | 190 | 229
-//   groups of 2, D128  n 16 (B1 H4 S512) 23.1 | 22.2 | 18.3 | 17.5, 64 (B1 H4 S2048) 56.1 | 56.7 | 42.7 | 40.4, 72 (B1 H16 S576) 29.7 | 28.7 | 25.0 | 27.9, 128 (B1 H16 S1008) 46.5 | 45.6 | 39.8 |
-//     46.3, 256 (B1 H16 S2048) 83.1 | 85.3 | 85.1 | 101, 512 (B1 H32 S2048) 118 | 130 | 136 | 176;  D64  64 47.7 | 53.0 | 39.6 | 34.3, 72 25.8 | 25.9 | 22.5 | 22.0, 128 40.4 | 42.2 | 36.4 | 38.5, 256 72.7 | 78.3 | 74.8 | 80.5
+// line runs by n, the 64-row blocks over the groups of heads.  us of the forward, bf16 or fp16, several kernel sizes, the four in this order:
+//   groups of 4, D128  n 24 (B4 H12 S72) 21.2 | 16.3 | 15.8, 36 (B2 H12 S352) 32.3 | 27.8 | 24.6, 96 (B2 H32 S360) 38.7 | 34.2 | 32.2, 168 (B2 H16 S1296) 84.5 |
+//     82.1 | 69.7, 200 (B4 H8 S1600) 104 | 99.6 | 95.5, 240 (B2 H16 S1864) 121 | 116 | 119, 320 (B2 H16 S2552) 198 | 195 | 208, 408 (B2 H16 S3256) 275 | 312 | 322,
+//     504 (B2 H16 S3976) 408 | 454 | 487.  HALF_SPLIT has one workgroup per CU there: from 257 on (n 36, B4 H12 S184 18.4 against 24.6) a second round, and
+//     where it wins (few long rows, n 28, B1 H16 S440 26.1 against 25.4) three kernels are faster than two.
+//   groups of 4, D64   n 8 (B1 H16 S72) 17.4 | 14.9 | 14.1 | 14.0, 32 (B4 H16 S128) 19.3 | 16.4 | 15.1 | 14.8, 64 (B1 H32 S464) 31.6 | 27.1 | 24.7 | 23.7, 104 (B1 H32 S800)
+//     51.3 | 45.7 | 42.3 | 46.2, 168 (B2 H16 S1296) 67.7 | 59.8 | 56.5 | 67.1, 208 (B2 H16 S1608) 93.0 | 83.4 | 85.0 | 99.4, 256 (B1 H16 S4048) 224 | 194 | 215 | 239, 400 (B4 H16
+//     S1560) 116 | 120 | 130 | 163
+//   groups of 2, D128  n 26 (B1 H4 S816) 28.6 | 27.6 | 22.3 | 20.5, 64 (B1 H4 S2032) 56.8 | 56.9 | 43.8 | 41.4, 88 (B1 H16 S664) 29.9 | 28.8 | 24.6 | 28.6, 188 (B1 H8 S2952)
+//     85.6 | 88.9 | 78.6 | 91.4, 256 (B1 H16 S2032) 73.1 | 74.5 | 74.9 | 91.7, 416 (B4 H4 S3328) 148 | 166 | 167 | 203;  D64  24 (B1 H8 S336) 17.3 | 17.6 | 15.2 | 14.0, 72 (B1
+//     H16 S560) 23.7 | 24.4 | 21.5 | 20.8, 144 (B2 H16 S544) 27.2 | 27.8 | 25.5 | 27.9, 228 (B1 H12 S2432) 67.6 | 76.8 | 70.9 | 74.5, 456 (B2 H8 S3600) 139 | 159 | 157 | 173
 enum pv_form { WHOLE = 1, HALF_LONG, HALF_SHORT, HALF_SPLIT };
 
 pv_form form_of(int64_t groups, int64_t S, int D, int G)
@@ -348,7 +353,7 @@ pv_form form_of(int64_t groups, int64_t S, int D, int G)
     if (G == 2) return n >= 200 ? WHOLE : n > 64 ? HALF_SHORT : HALF_SPLIT;
     if (n >= 400) return WHOLE;
     if (D == 64) return n >= 190 ? HALF_LONG : n > 64 ? HALF_SHORT : HALF_SPLIT;
-    return n >= 240 ? HALF_LONG : n > 36 ? HALF_SHORT : HALF_SPLIT;
+    return n >= 240 ? HALF_LONG : HALF_SHORT;
 }
 
 template <typename T, int D, int G, int GO, int RW, int GR, int OCC> int go(pv_args a, int64_t groups, int resident, hipStream_t st)
@@ -369,8 +374,10 @@ template <typename T, int D, int G> int launch(const pv_args &a, int64_t groups,
     case HALF_LONG:
         if constexpr (G == 4 && D == 64) return go<T, D, G, G, 2, 2, 2>(a, groups, 2, st);
         else return go<T, D, G, G / 2, 4, 1, 3>(a, groups, 3, st);
-    case HALF_SHORT: return go<T, D, G, G / 2, 2, 2, D == 64 ? 3 : 2>(a, groups, D == 64 ? 3 : 2, st);
-    default: return go<T, D, G, G / 2, 1, 4, D == 64 ? 2 : 1>(a, groups, D == 64 ? 2 : 1, st);
+    case HALF_SPLIT:
+        if constexpr (G == 2 || D == 64) return go<T, D, G, G / 2, 1, 4, D == 64 ? 2 : 1>(a, groups, D == 64 ? 2 : 1, st);
+        [[fallthrough]];
+    default: return go<T, D, G, G / 2, 2, 2, D == 64 ? 3 : 2>(a, groups, D == 64 ? 3 : 2, st);
     }
 }
 template <typename T> int launch_type(const pv_args &a, int64_t groups, int64_t D, int group, hipStream_t st)
