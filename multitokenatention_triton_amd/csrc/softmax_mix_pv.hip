@@ -342,7 +342,9 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_arg
 //     S1560) 116 | 120 | 130 | 163
 //   groups of 2, D128  n 26 (B1 H4 S816) 28.6 | 27.6 | 22.3 | 20.5, 64 (B1 H4 S2032) 56.8 | 56.9 | 43.8 | 41.4, 88 (B1 H16 S664) 29.9 | 28.8 | 24.6 | 28.6, 188 (B1 H8 S2952)
 //     85.6 | 88.9 | 78.6 | 91.4, 256 (B1 H16 S2032) 73.1 | 74.5 | 74.9 | 91.7, 416 (B4 H4 S3328) 148 | 166 | 167 | 203;  D64  24 (B1 H8 S336) 17.3 | 17.6 | 15.2 | 14.0, 72 (B1
-//     H16 S560) 23.7 | 24.4 | 21.5 | 20.8, 144 (B2 H16 S544) 27.2 | 27.8 | 25.5 | 27.9, 228 (B1 H12 S2432) 67.6 | 76.8 | 70.9 | 74.5, 456 (B2 H8 S3600) 139 | 159 | 157 | 173
+//     H16 S560) 23.7 | 24.4 | 21.5 | 20.8, 80 (B2 H16 S264) 18.9 | 18.9 | 16.8 | 17.6, 144 (B2 H16 S544) 27.2 | 27.8 | 25.5 | 27.9, 228 (B1 H12 S2432) 67.6 | 76.8 | 70.9 | 74.5, 456 (B2 H8 S3600) 139 | 159 | 157 | 173
+//     Few heads with long rows: HALF_SPLIT beyond n 64 too, HALF_SHORT | HALF_SPLIT, B1 H4: D128 S2112 (66) 42.0 | 38.9, S2752 (86) 53.4 | 53.1, S3000 (94) 55.8 | 58.5;
+//     D64 S2112 39.7 | 35.0 (right-padded 46.2 | 40.9, three kernels 42.2), S3712 (116) 63.1 | 61.8, S4096 (128) 68.3 | 69.4, B1 H12 S768 (72) 24.2 | 22.5
 enum pv_form { WHOLE = 1, HALF_LONG, HALF_SHORT, HALF_SPLIT };
 
 pv_form form_of(int64_t groups, int64_t S, int D, int G)
@@ -350,7 +352,7 @@ pv_form form_of(int64_t groups, int64_t S, int D, int G)
     static const int force = [] { const char *e = getenv("MTA_SOFTMAX_PV_FORM"); return e ? atoi(e) : 0; }();   // (comparison switch: always that form)
     if (force >= WHOLE && force <= HALF_SPLIT) return (pv_form)force;
     const int64_t n = groups * ((S + 63) / 64);
-    if (G == 2) return n >= 200 ? WHOLE : n > 64 ? HALF_SHORT : HALF_SPLIT;
+    if (G == 2) return n >= 200 ? WHOLE : n <= 64 || (D == 64 ? n <= 116 && S >= 512 : n <= 86 && S > 24 * n) ? HALF_SPLIT : HALF_SHORT;
     if (n >= 400) return WHOLE;
     if (D == 64) return n >= 190 ? HALF_LONG : n > 64 ? HALF_SHORT : HALF_SPLIT;
     return n >= 240 ? HALF_LONG : HALF_SHORT;
