@@ -59,17 +59,25 @@ bool conv_mix16_fills(int64_t planes, int64_t rows, int64_t keys, bool lower_onl
     return tiles >= 800 || (!dense && tiles >= 430 && tiles <= 490);
 }
 
-// Whether softmax, mixing and P V in one kernel (softmax_mix_pv.hip) beat softmax + mixing, then P V: its workgroups walk a row's keys, a chain
-// that only a grid of enough blocks of 64 rows (over the groups of heads) hides.  Groups of 2: everywhere.  us of the forward, three kernels | two, bf16 6x11
-// without a mask, groups of 4, D128: 1 block (B1 H4 S64) 16.4 | 17.4, 40 (B2 H16 S296) 24.2 | 23.9, 48 (B2 H8 S768) 35.4 | 39.0, (B1 H4 S3072) 61.6 | 87.0, 56
-// (B2 H16 S448) 29.8 | 28.9, 80 (B1 H16 S1280) 50.9 | 55.2, 96 (B4 H32 S136) 29.0 | 22.5, (B2 H16 S768) 46.9 | 45.1, (B1 H16 S1536) 63.3 | 66.0, 116 (B1 H16
-// S1856) 77.0 | 77.2, 126 (B1 H12 S2688) 114 | 104, 160 (B1 H16 S2500) 138 | 122, 192 (B4 H12 S1024) 74.3 | 74.1, 240 (B4 H16 S900) 94.5 | 88.5, 512 (B2 H16
-// S4096) 521 | 437; D64: 1 (B1 H4 S64) 15.4 | 14.5, 5 (B1 H4 S296) 16.1 | 16.8, 16 (B1 H8 S512) 17.7 | 19.0, 20 (B1 H16 S296) 17.9 | 17.2, 48 (B2 H8 S768) 33.7 |
-// 31.4, (B1 H8 S1536) 41.4 | 43.0, 64 (B1 H16 S1008) 40.3 | 38.8, 80 (B1 H16 S1280) 47.2 | 47.2, 128 (B1 H8 S4096) 147 | 123, 216 (B1 H16 S3400) 186 | 143.
-bool softmax_pv_pays(int64_t planes, int64_t keys, int64_t head_dim, int64_t group)
+// Whether softmax, mixing and P V in one kernel (softmax_mix_pv.hip) beat softmax + mixing, then P V: its workgroups walk a row's keys, a chain that only a
+// grid of enough blocks of 64 rows (over the groups of heads) hides, or short rows.  `padded`: a key bias, or rows that see no key - both kernels look for
+// hidden keys at every step, and rows that start late are as long as any -, so the line lies higher; under windows and documents the chains are
+// short and it lies where it does without a mask.  us of the forward, three kernels | two, several kernel sizes, 16 bits:
+//   no mask, groups of 4    D128: 24 blocks (B1 H32 S184) 17.7 | 18.0, 36 (B4 H12 S184) 20.0 | 18.4, (B1 H8 S1152) 37.2 | 44.0, 96 (B4 H16 S376) 36.5 | 35.2, 104 (B4 H8 S832)
+//     44.9 | 44.9, 160 (B1 H32 S1256) 74.2 | 70.9, 256 (B2 H16 S2000) 148 | 131;  D64: 12 (B1 H16 S136) 14.7 | 14.1, 32 (B2 H16 S208) 17.2 | 16.5, 36 (B1 H12 S752)
+//     25.9 | 27.0, 64 (B1 H32 S464) 27.2 | 23.7, 84 (B4 H4 S1336) 46.9 | 48.3, 136 (B1 H16 S2176) 85.4 | 76.8, 256 (B1 H16 S4048) 236 | 194
+//   windows and documents, groups of 4    D128: 36 (B4 H12 S184) 20.9 | 19.3, 64 (B1 H32 S464) 29.7 | 26.7, 132 (B1 H16 S2112) 73.0 | 62.1;  D64: 60 (B2 H12 S584) 27.7 |
+//     26.0, 116 (B1 H16 S1856) 55.5 | 53.5, 138 (B1 H12 S2904) 75.1 | 62.2
+//   padded, groups of 4    D128, right: 24 (B2 H16 S184) 20.8 | 22.2, 48 (B1 H32 S144) 6 % faster, 72 (B2 H16 S536) 38.1 | 41.1, 96 (B4 H16 S376) 40.7 | 42.6, 128 (B1 H16 S2000)
+//     88.0 | 96.6, 160 (B2 H32 S264) 3 % faster, 208 (B1 H16 S3288) 210 | 195; left: 96 (B1 H32 S712) 8 % slower, 136 (B2 H16 S1088) even, 176 (B1 H16 S2760)
+//     124 | 109;  D64, right: 72 (B4 H8 S568) 36.3 | 35.6, 76 (B1 H16 S1184) 45.7 | 51.0, 96 (B4 H16 S368) 35.2 | 34.0, 140 (B1 H16 S2200) 99.8 | 94.2, 256 (B1 H16 S4040) 240 |
+//     199; left: 81 (B1 H12 S1672) 58.1 | 66.9, 171 (B1 H12 S3616) 163 | 145; up to 24 blocks of up to 256 keys 10 % faster or even (a launch less)
+//   groups of 2: everywhere, B1 H4 S2112 D64 38.0 | 34.8, but for padded rows of few heads: B1 H4 D128 S3328 (104) 69.3 | 74.4, left 75.8 | 82.5
+bool softmax_pv_pays(int64_t planes, int64_t keys, int64_t head_dim, int64_t group, bool padded)
 {
-    if (group == 2) return true;
     const int64_t blocks = planes / group * ((keys + 63) / 64);
+    if (group == 2) return !padded || keys <= 20 * blocks || blocks > 130 || blocks < (head_dim == 64 ? 117 : 82);
+    if (padded) return head_dim == 64 ? blocks >= 130 || keys <= 5 * blocks || (keys <= 256 && blocks <= 24) : blocks >= 140 || 2 * keys <= 7 * blocks;
     return head_dim == 64 ? blocks >= 80 || keys <= 16 * blocks || keys <= 256 : blocks >= 120 || keys <= 8 * blocks;
 }
 
@@ -283,7 +291,7 @@ Tensor forward_inference(const Tensor &q_, const Tensor &k_, const Tensor &v_, c
     // Two kernels: the scores with the statistics of their rows, and softmax, mixing and P V in one, the probabilities in registers only (which
     // is why the hook hears of the two stages at once).
     if (causal && pre_identity && post_conv_identity && w2 && qk_kernel && own_pv && dropout <= 0 && !(key_bias && (first || !key_bias_hides)) &&
-        softmax_pv_pays(planes_of[0] * heads, n_keys, v.size(-1), g_post) && stats_route_supported(q, k, conv_w, g_post, *w2, key_bias.has_value(), ragged)) {
+        softmax_pv_pays(planes_of[0] * heads, n_keys, v.size(-1), g_post, key_bias || empty_rows) && stats_route_supported(q, k, conv_w, g_post, *w2, key_bias.has_value(), ragged)) {
         const bool tri = !planes && g_post * tri_row_offset(n_keys) < (int64_t(1) << 31);
         mark("qk_conv");
         const auto [scores, stats] = qk_conv_stats(q, k, conv_w, scale, g_post, tri, key_bias, first, ragged);
