@@ -211,6 +211,14 @@ def stage_breakdown(torch, mod, sets, steps):
     return {k: sum(v) / len(v) for k, v in acc.items()}
 
 
+def join_stages(stages):
+    """Stage times with softmax + mixing and P V as one where one kernel does both: it is announced as the two stages at once, so that the
+    first of them takes next to no time (as two kernels they take 0.18 and 0.14 ms at the headline configuration)."""
+    if 10 * stages.get("mix_softmax_mix", 1e9) < stages.get("pv", 0.0):
+        stages["softmax_mix_pv"] = stages.pop("mix_softmax_mix") + stages.pop("pv")
+    return stages
+
+
 def _record(torch):
     ev = torch.cuda.Event(enable_timing=True)
     ev.record()  # on the current stream, the one ops.py hands to the library
@@ -537,8 +545,7 @@ def main():
 
     with torch.no_grad():
         ms = time_steps(torch, lambda i: mod(*sets[i], None, None), len(sets), args.warmup, args.steps)
-        stages = stage_breakdown(torch, mod, sets, max(3, min(args.steps, 10)))
-        stages["softmax_mix_pv"] = stages.pop("mix_softmax_mix") + stages.pop("pv")   # (one kernel in this configuration)
+        stages = join_stages(stage_breakdown(torch, mod, sets, max(3, min(args.steps, 10))))
         ran_own_pv = "qk" not in stages  # the fused route ends in mta_causal_pv_fwd, the unfused one in a library GEMM
         hip_stages = {k: v for k, v in stages.items() if k != "qk" and (k != "pv" or ran_own_pv)}
         dom = max(hip_stages, key=hip_stages.get)
