@@ -42,6 +42,21 @@ __host__ __device__ inline int scores_key_blocks(int qb, int rows, int S)
     return (last < S - 1 ? last : S - 1) / QK_BK + 1;
 }
 
+// x / n by the reciprocal of n: exact for x below 2^20 (x + 1/2 keeps 1 / 2n away from every multiple, the product is off by 2^-22 of it)
+__host__ __device__ inline int quotient(int x, float per_n) { return (int)(((float)x + 0.5f) * per_n); }
+// The same numbers where dividing by what is only known at run time costs too much: a row's items, by reciprocals
+struct scores_items {
+    scores_cut cut;
+    int rows;                           // of a query block
+    float per_rows, per_big, per_small; // reciprocals of rows, cut.big, cut.small
+    scores_items(const scores_cut &c, int r) : cut(c), rows(r), per_rows(1.0f / (float)r), per_big(1.0f / (float)c.big), per_small(1.0f / (float)c.small) {}
+    __host__ __device__ int of_row(int p, int S) const   // = cut.items(scores_key_blocks(p / rows, rows, S))
+    {
+        const int nk = scores_key_blocks(quotient(p, per_rows), rows, S), want = quotient(quotient(nk * cut.share, 0.01f) + cut.small / 2, per_small) * cut.small;
+        const int nshort = want < nk ? want : nk;
+        return quotient(nk - nshort + cut.big - 1, per_big) + quotient(nshort + cut.small - 1, per_small);
+    }
+};
 
 constexpr int QK_CHUNK = 32;  // key blocks per work item of the kernel when no item table is built
 // with an item table: long and short items (key blocks), and the share of a query block's key range that goes into short

@@ -44,12 +44,10 @@ struct pv_args {
     const float *key_bias;   // (B,S) or NULL
     const int *band_lo;      // (B,S) or NULL
     void *o;
-    int S, SV, H, groups, nrb, cus, tri, slots, rows;   // SV: rows that v has, at most S
-    scores_cut cut;
-    float per_gph, per_rows, per_big, per_small;   // reciprocals of H / G, rows, cut.big, cut.small
+    int S, SV, H, groups, nrb, cus, tri, slots;   // SV: rows that v has, at most S
+    scores_items items;
+    float per_gph;           // reciprocal of H / G
 };
-// x / n by the reciprocal of n: exact for x below 2^20 and n below 2^11 (x + 1/2 keeps 1 / 2n away from every multiple, the product is off by 2^-22 of it)
-__device__ __forceinline__ int quotient(int x, float per_n) { return (int)(((float)x + 0.5f) * per_n); }
 
 template <typename T, int D, int G, int GO, int RW, int GR, int OCC, bool KB>
 __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_args a)
@@ -137,9 +135,7 @@ __global__ __launch_bounds__(64 * RW * GR, OCC) void softmax_mix_pv(const pv_arg
     constexpr float LOG2E = 1.4426950408889634f;
     float ref[G], inv[G];
     {
-        const int qb = quotient(pc, a.per_rows), nk = scores_key_blocks(qb, a.rows, S);
-        const int nshort = min(nk, quotient(quotient(nk * a.cut.share, 0.01f) + a.cut.small / 2, a.per_small) * a.cut.small), nlong = nk - nshort;
-        const int items = quotient(nlong + a.cut.big - 1, a.per_big) + quotient(nshort + a.cut.small - 1, a.per_small);   // (scores_cut::items)
+        const int items = a.items.of_row(pc, S);
         const float2 *const at = a.stats + ((int64_t)(bg * G + kg % G) * a.slots) * S + pc;
         float m = NO_SCORE, l = 0.0f;
         constexpr int AT_ONCE = 8;
@@ -411,9 +407,8 @@ extern "C" int mta_softmax_mix_pv_ragged_fwd(const void *x, const void *stats, c
     if (!mta_softmax_mix_pv_supported(H, S, D, group, io_dtype, w_dtype, key_bias != nullptr)) return MTA_ERR_UNSUPPORTED;
     bool table;
     const scores_cut cut = scores_cut_of(B * H, S, R, true, table);
-    const int rows = scores_rows(R);
     const pv_args a{x, w2, v, (const float2 *)stats, (const float *)key_bias, (const int *)first_visible, o, (int)S, (int)v_rows, (int)H, 0, 0, 0, tri != 0,
-                    scores_slots(S, R, cut), rows, cut, (float)group / (float)H, 1.0f / (float)rows, 1.0f / (float)cut.big, 1.0f / (float)cut.small};
+                    scores_slots(S, R, cut), scores_items(cut, scores_rows(R)), (float)group / (float)H};
     const int64_t groups = B * (H / group);
     return io_dtype == MTA_BF16 ? launch_type<bf16_t>(a, groups, D, group, (hipStream_t)stream) : launch_type<f16_t>(a, groups, D, group, (hipStream_t)stream);
 }

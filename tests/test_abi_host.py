@@ -4,6 +4,7 @@ surface mirrors the reference's names, parameters and error behaviour."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -338,3 +339,46 @@ def test_dropin_shims_resolve():
         assert importlib.import_module("triton_linear_head").TritonLinearHead is mta.TritonLinearHead
     finally:
         sys.path.pop(0)
+
+
+CUT_PROGRAM = r"""
+#include <cstdio>
+#include "scores_cut.hpp"
+using namespace mta;
+int main()
+{
+    long long rows = 0, wrong = 0, tables = 0, none = 0;
+    for (int R : {3, 5, 6, 7, 11})
+        for (int64_t heads : {1, 2, 12, 64, 1024, 65535})
+            for (int64_t S = 8; S <= (1 << 19); S = S < 2048 ? S + 8 : S < 40000 ? S + 1048 : S + 52424) {
+                bool table;
+                const scores_cut cut = scores_cut_of(heads, S, R, true, table);
+                ++(table ? tables : none);
+                const scores_items items(cut, scores_rows(R));
+                const int slots = scores_slots(S, R, cut);
+                for (int64_t p = 0; p < S; p = S <= 2048 || p % items.rows == items.rows - 1 || p + items.rows > S ? p + 1 : p + items.rows - 1 - p % items.rows, ++rows) {
+                    const int nk = scores_key_blocks((int)(p / items.rows), items.rows, (int)S), n = cut.items(nk);
+                    // an item starts where the kernel that writes the statistics starts it, and has the place it gives it
+                    int j = 0, at = 0;
+                    for (const int nlong = cut.longs(nk); j < nk; ++at) {
+                        wrong += cut.index(nk, j) != at;
+                        j += j < nlong ? (cut.big < nlong - j ? cut.big : nlong - j) : (cut.small < nk - j ? cut.small : nk - j);
+                        if (S > 2048 && p % 997) { at = n - 1; j = nk; }
+                    }
+                    wrong += at != n || items.of_row((int)p, (int)S) != n || n > slots;
+                }
+            }
+    printf("%lld %lld %lld %lld\n", rows, wrong, tables, none);
+}
+"""
+
+
+def test_items_of_a_row_by_reciprocals(tmp_path):
+    """The work items of a row as the scores kernel cuts them, and as the kernel behind it counts them, by reciprocals: the same for all lengths up to
+    2^19, with a table of the items and without one."""
+    (tmp_path / "cut.hip").write_text(CUT_PROGRAM)
+    exe = str(tmp_path / "cut")
+    subprocess.run(["hipcc", "-x", "hip", "--cuda-host-only", "-O2", "-std=c++17", "-I", os.path.join(os.path.dirname(mta.__file__), "csrc"),
+                    str(tmp_path / "cut.hip"), "-o", exe], check=True, capture_output=True, timeout=300)
+    rows, wrong, tables, none = map(int, subprocess.run([exe], check=True, capture_output=True, text=True, timeout=300).stdout.split())
+    assert wrong == 0 and rows > 10 ** 6 and tables > 1000 and none > 100
