@@ -617,15 +617,15 @@ def test_triangular_layout_stages_equal_the_plane_layout(pkg, case):
                                          first_visible=first), o_plane)
 
 
-# B, H, S, D, R, Sk, group, dtype, mask: every form of the kernel (by the number of 64-row blocks over the groups), the shortest rows, edges of its
-# 16 rows x 32 keys and of the scores kernel's pieces
+# B, H, S, D, R, Sk, group, dtype, mask: every form of the kernel (by the number of 64-row blocks over the groups; those with a key bias where the
+# switches of test_gpu_switches.py choose them), the shortest rows, edges of its 16 rows x 32 keys and of the scores kernel's pieces
 STATS_CASES = [
     (1, 4, 8, 128, 3, 3, 4, torch.bfloat16, None), (1, 2, 40, 64, 5, 5, 2, torch.float16, None), (2, 4, 72, 64, 3, 5, 4, torch.bfloat16, "keys"),
     (1, 4, 520, 128, 6, 11, 4, torch.float16, None), (2, 4, 1160, 128, 6, 11, 4, torch.bfloat16, "documents"), (1, 8, 1032, 64, 7, 9, 4, torch.float16, "keys"),
     (4, 32, 136, 128, 6, 11, 4, torch.bfloat16, None), (4, 64, 264, 128, 3, 3, 4, torch.float16, "keys"), (4, 64, 456, 128, 5, 7, 4, torch.bfloat16, "window"),
     (4, 32, 328, 64, 11, 15, 4, torch.bfloat16, "ragged"), (4, 64, 424, 64, 6, 11, 4, torch.float16, None), (2, 64, 200, 128, 7, 7, 2, torch.bfloat16, "keys"),
     (2, 32, 136, 128, 3, 3, 2, torch.float16, "window"), (4, 64, 136, 64, 5, 5, 2, torch.bfloat16, None), (2, 32, 232, 64, 6, 11, 2, torch.float16, "documents"),
-    (1, 4, 4168, 64, 7, 7, 4, torch.bfloat16, None),
+    (1, 4, 4168, 64, 7, 7, 4, torch.bfloat16, None), (1, 4, 200, 128, 5, 5, 2, torch.bfloat16, None), (2, 8, 328, 64, 3, 5, 2, torch.float16, "keys"),
     # padding on the left, up to and beyond the eight keys of a lane, its next eight, a block, a work item
     (6, 4, 328, 64, 6, 11, 4, torch.bfloat16, "left"), (6, 4, 648, 128, 3, 3, 2, torch.float16, "left"), (2, 8, 2056, 64, 7, 7, 4, torch.float16, "left"),
 ]
@@ -723,6 +723,30 @@ def test_softmax_mix_pv_scores_that_are_not_finite_or_far_apart(pkg, dtype):
     want = torch.einsum("oi,bipq->bopq", w2.double(), p) @ v.double()
     # (an exponent relative to the reference is below 128 - beyond, the statistics take another reference -, so off by 2^-18, here and in the sum: 2^-17)
     assert ((got - want).abs() <= (2.02 * u + 2.0 ** -17) * size + u * want.abs() + 2.0 ** -24 * s).all()
+
+
+@pytest.mark.parametrize("d,rows", [(64, 3), (128, 6)])
+def test_softmax_mix_pv_beyond_the_item_table(pkg, d, rows):
+    """A row so long that a head's work items do not fit the scores kernel's table: items of one length.  Rows of all parts of the sequence against 64 bits
+    from the same stored scores; the bound of test_softmax_mix_pv, 2^-16 for four times the terms."""
+    ops = pkg.ops
+    b, h, s, group, dtype = 1, 2, 18440, 2, torch.float16
+    print(f"softmax mix pv, long rows {d, rows}", flush=True)
+    g = torch.Generator().manual_seed(95)
+    q, k, v = (t.cuda() for t in O.seeded_qkv(b, h, s, d, dtype, seed=96))
+    w = (torch.randn(h, rows, 3 if rows == 3 else 11, generator=g) * 0.2).to(dtype).cuda()
+    w2 = O.block_diag_head_weight(h, group, 0.3, g, dtype).cuda()
+    x, stats = ops.qk_conv_stats(q, k, w, d ** -0.5, group, tri=False)
+    assert stats.shape[1] == -(-s // 64 // 32)   # (items of 32 key blocks)
+    got = ops.softmax_mix_pv(x, stats, w2, v, rows, group)[0].double()
+    u = 2.0 ** -11
+    for p in (0, 1, 63, 64, 127, 128, 2047, 2048, 2111, 8191, 8192, 12345, s - 65, s - 2, s - 1):
+        probs = torch.softmax(x[0, :, p, :p + 1].double(), -1)
+        vd, w2d = v[0, :, :p + 1].double(), w2.double()
+        want = torch.einsum("oq,oqd->od", w2d @ probs, vd)
+        size = torch.einsum("oq,oqd->od", w2d.abs() @ probs, vd.abs())
+        bound = (2.02 * u + 2.0 ** -16) * size + u * want.abs() + 2.0 ** -25 * (w2d.abs().sum(1)[:, None] + 2) * vd.abs().sum(1)
+        assert ((got[:, p] - want).abs() <= bound).all(), (p, ((got[:, p] - want).abs() / bound).max())
 
 
 @pytest.mark.parametrize("seen", ["one key", "tied keys"])

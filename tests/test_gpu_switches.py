@@ -26,11 +26,19 @@ GROUPS = [
      "test_conv_parity or test_conv_identity_tap or test_conv_backward_parity"),
     # dense groups of 16 heads in the one-pass conv + mixing entry point on the vector-ALU kernel
     ({"MTA_CONV_MIX16_OFF": "1"}, ["tests/test_gpu_ops.py"], "test_conv_headmix_parity"),
-    # P V of small grids on the one-group kernel that large grids run (by default they split the key blocks between two
-    # groups of wavefronts)
-    ({"MTA_PV_SPLIT": "1"}, ["tests/test_gpu_attention.py"], "test_causal_pv"),
-    # ... and on 128-row blocks whose key blocks two groups share
-    ({"MTA_PV_SPLIT": "5"}, ["tests/test_gpu_attention.py"], "test_causal_pv"),
+    # P V and P^T X on one kernel whatever the grid: the wide one (P^T X: 128 rows), 64 rows in two groups, the rings of 64 rows (in two groups, in
+    # one), of 128 rows (in one group; P^T X also in two)
+    ({"MTA_PV_SPLIT": "1"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    ({"MTA_PV_SPLIT": "2"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    ({"MTA_PV_SPLIT": "4"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    ({"MTA_PV_SPLIT": "5"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    ({"MTA_PV_SPLIT": "7"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    ({"MTA_PV_SPLIT": "8"}, ["tests/test_gpu_attention.py"], "test_causal_pv or test_causal_ptx"),
+    # softmax, mixing and P V in one kernel in each of its forms, with and without a key bias
+    ({"MTA_SOFTMAX_PV_FORM": "1"}, ["tests/test_gpu_attention.py"], "test_softmax_mix_pv and not beyond"),
+    ({"MTA_SOFTMAX_PV_FORM": "2"}, ["tests/test_gpu_attention.py"], "test_softmax_mix_pv and not beyond"),
+    ({"MTA_SOFTMAX_PV_FORM": "3"}, ["tests/test_gpu_attention.py"], "test_softmax_mix_pv and not beyond"),
+    ({"MTA_SOFTMAX_PV_FORM": "4"}, ["tests/test_gpu_attention.py"], "test_softmax_mix_pv and not beyond"),
     # mix -> softmax -> mix for groups of 16 heads with a workgroup per row (by default workgroups take lists of rows)
     # the inference route with its score tensors as (B,H,S,S) planes (by default: the triangular layout)
     ({"MTA_SCORE_LAYOUT": "planes"}, ["tests/test_gpu_attention.py"],
