@@ -123,8 +123,8 @@ struct item_table {
 // scores of the hidden keys enter the conv as 0, as the reference's masked_fill ahead of its conv leaves them
 // (mta_attention_triton.py:70-73).
 // STATS (causal): the statistics of each row's scores of the item, as they are stored (scores_stats): 32 more vector instructions and eight exponentials per
-// eight scores of a lane, us without | with them: bf16 6x11 B2 H16 S4096 D128 248 | 253 (in a loop: the clock), B4 H16 S1024 36.6 | 45.5, B1 H16 S2048 38.2 |
-// 47.6, 7x7 B2 H16 S4096 D64 181 | 209.  With the maximum so far taken at every eight, and a factor for the sum, B2 H16 S4096 took 22 us more.
+// eight scores of a lane, us without | with them | and a key bias: bf16 6x11 B2 H16 S4096 D128 226 | 247 | 255 (in a loop: the clock), B4 H16 S1024
+// 37.6 | 44.2 | 46.0, B1 H16 S2048 37.7 | 46.1 | 47.4, 7x7 B2 H16 S4096 D64 180 | 195 | 203.  With the maximum so far taken at every eight, and a factor for the sum, B2 H16 S4096 took 22 us more.
 // STATS 2: with a key bias, which an instance of its own has to look for.
 template <typename T, int D, int R, int SK, bool BAND, int STATS>
 __global__ __launch_bounds__(256, R <= 7 && !(STATS && BAND && R >= 6 && D == 128) ? QK_OCC : 2) void conv_scores_mfma(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ Wt,

@@ -45,7 +45,7 @@ bool masks_ok(int64_t group, at::ScalarType t, bool masked)
 // Whether conv + mixing of 16 heads in one kernel is worth it: its 512 persistent workgroups walk 32 x 64 tiles of all 16
 // heads at 16 to 18 us each, so that it takes more than one and a half rounds of tiles to meet the two kernels one after the other, or
 // one round that is nearly full and surely fits (what is left to spare takes up an uneven deal over the XCDs).  Groups of 2 or 4 heads take that
-// round; dense weights gain there too, 4 to 6 %, and are left on the two kernels.
+// round; dense weights are left on the two kernels: they gain 3 to 6 % from 440 to 490 tiles, nothing at 420, and lose 2 to 4 % at 506.
 // us of the forward (H16 D64, the pre-softmax conv 6x11), two kernels | one, fp16 dense 3x3 / 7x7 after the softmax / bf16 groups of 4, 3x3 / fp16 groups
 // of 2, 3x3: 272 tiles (B1 S1024) 62.5 | 63.3 / 63.5 | 65.9 / 65.1 | 71.8 / 63.9 | 68.1, 380 (B1 S1216) 73.5 | 72.2 / 76.6 | 75.9 / 73.8 | 77.5 / 73.7 | 73.6,
 // 420 (B1 S1280) 74.9 | 73.2 / 78.2 | 76.9 / 75.7 | 77.1 / 75.6 | 75.6, 440 (B4 S640) 79.2 | 75.2 / 83.0 | 79.2 / 81.6 | 78.1 / 83.8 | 76.3, 448 (B8 S448) 81.9 |

@@ -7,12 +7,13 @@
 // lies within a lane, and rounds the result: what the softmax stage would have stored is then in the lane that supplies it as operand of O^T
 // += V^T P^T.  V comes in blocks of 32 keys of GO heads, copied global -> LDS asynchronously a step ahead, read by transpose reads.  The
 // probabilities of the next step are formed between the products of this one.
-// What it saves is writing and reading the probabilities, half of what the three kernels of this route move: bf16 B2 H16 S4096 D128 groups of 4,
-// softmax + mixing 184 us, P V 144 -> 189 (the scores kernel pays 5 to 9 for the statistics); B4 H16 S1024 33 + 23 -> 38; D64 B2 H16 S4096 184 + 135
-// -> 156.  What bounds it: at B2 H16 S4096 D128 108 us without loads, 97 for the scores alone as tiles of 16 rows, 69 for V and the products - they overlap
-// in part only, a barrier a step holding eight wavefronts to the slowest load.  Not better there (us): scores non-temporal 218, blocks of
-// V asked for three steps ahead and one wavefront per SIMD 232, 128 rows 254, results of two of the four heads per workgroup 237 to 273 (twice
-// the exponentials; where the grid is short they win, form_of), packed dot products in place of the 4x4x4 ones (as fast, more vector instructions).
+// What it saves is writing and reading the probabilities, half of what the three kernels of this route move: bf16 6x11 B2 H16 S4096 D128 groups of 4,
+// softmax + mixing 183 us, P V 148 -> 196 (with a key bias 197; the scores kernel pays 7 to 21 for the statistics); B4 H16 S1024 30 + 22 -> 39; D64 B2 H16 S4096
+// 177 + 134 -> 161.  What bounds it: at B2 H16 S4096 D128, where it took 189 with the sum in the exponent, 108 us without loads, 97 for the scores alone as tiles of 16
+// rows, 69 for V and the products - they overlap in part only, a barrier a step holding eight wavefronts to the slowest load.  Not better there (us, against
+// those 189): scores non-temporal 218, blocks of V asked for three steps ahead and one wavefront per SIMD 232, 128 rows 254, results of two of the four heads per
+// workgroup 237 to 273 (twice the exponentials; where the grid is short they win, form_of), packed dot products in place of the 4x4x4 ones (as fast, more vector
+// instructions).
 #include <type_traits>
 
 #include <stdlib.h>
